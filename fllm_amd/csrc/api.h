@@ -99,7 +99,8 @@ int fllm_linear_add_normed(const void *x, int ldx, const void *w, const float *b
 // the separate norm, rotary and SwiGLU kernels.
 //   fllm_weight_tiles_supported  1 where the kernels take tiles: N >= 16, K a multiple of 1,024
 //   fllm_weight_tiles_elements   bfloat16 elements of the copy: N rounded up to 16, times K
-//   fllm_tile_weights            writes the copy: [tile of 16 rows][block of 128 columns][k-step of 32][lane][8]
+//   fllm_tile_weights            writes the copy: [tile of 16 rows][k-step of 32][lane][8] (any K in steps of 32; only those that
+//                                are supported serve the products here, the others fllm_experts_stream)
 //   fllm_linear_add_tiled        out += x w^T (+ bias), float32 out, 1..128 rows (beyond 64: w_tiles required, K in steps of 256)
 //   fllm_linear_f32_tiled        out = x w^T (+ bias), float32 out, 1..64 rows (the vocabulary projection); with w_tiles where it can
 //   fllm_tile_weights_gate_up    the copy of [gate; up] ([2 inter][K]) for the SwiGLU epilogue of 17 to 64 rows: tile T holds
@@ -443,6 +444,14 @@ int fllm_experts_up(const void *h, int ldh, const int32_t *ids, int rows, int to
 int fllm_experts_grouped_ungated(const void *h, int ldh, const int32_t *ids, int rows, int top, const void *w_up, const void *w_down,
                                  int E, int inter, int K, int N, void *act, float *out, int32_t *work, float *planes,
                                  hipStream_t stream);
+
+// The same for steps of few pairs (decode): the picked experts' matrices stream once, no scratch but act (bfloat16 [rows * top, inter]).
+// gated 1: w_up the tile-major copy (fllm_tile_weights) of [E * 2 inter][K], gate rows then up rows of an expert; gated 0: that of
+// [E * inter][K], relu(.)^2, weights null.  w_down that of [E * N][inter]; out float32 [rows * top, N].  1: shape declined (more than
+// 16 pairs an expert on average or 512 in all, widths that are no multiples of 32, N no multiple of 16).
+int fllm_experts_stream(const void *h, int ldh, const int32_t *ids, const float *weights, int rows, int top, const void *w_up,
+                        const void *w_down, int E, int inter, int K, int N, int gated, void *act, float *out, float limit, float alpha,
+                        float up_offset, hipStream_t stream);
 
 // ---- layer norms and the small passes around them (layer_norms.hip) ----
 // out1[i] = (x[r] - mean) * rsqrt(mean (x[r] - mean)^2 + eps1) * w1, r = rows ? rows[i] : i, and with w2 the same with w2 and eps2 in out2.

@@ -1214,19 +1214,18 @@ int launch_resident_plan(SkinnyArgs a, const ResidentPlan &p, int ntiles, const 
 // Tile-major weights serve matrices whose eight waves' K ranges are whole blocks of 128 columns.
 bool tiles_fit(int N, int K) { return N >= 16 && K >= 1024 && K % 1024 == 0; }
 
-// tiles[T][B][u][lane][8] = w[16 T + lane % 16][128 B + 32 u + 8 (lane / 16) ...]: tile T of 16 rows, block B of 128 columns,
-// k-step u of 32, and inside it the 16 bytes of each of the 64 lanes of a wave in lane order; rows past N are zeros
+// tiles[T][s][lane][8] = w[16 T + lane % 16][32 s + 8 (lane / 16) ...]: tile T of 16 rows, k-step s of 32, and inside it the 16 bytes
+// of each of the 64 lanes of a wave in lane order (four steps are a block of 128 columns); rows past N are zeros
 // `half_rows` > 0: w is a gate matrix on top of an up matrix of `half_rows` rows each, and tile T is rows 8 T .. 8 T + 7 of
 // the one followed by the same rows of the other, as the SwiGLU epilogue wants them
 __global__ void __launch_bounds__(256) tile_weights_kernel(const bf16_t *__restrict__ w, bf16_t *__restrict__ tiles, int N, int K, size_t pieces,
                                                            int half_rows) {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
-    const int blocks = K / 128;
+    const int steps = K / 32;
     for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < pieces; v += stride) {
-        const int lane = (int)(v & 63), u = (int)((v >> 6) & 3);
-        const size_t tb = v >> 8;
-        const int B = (int)(tb % blocks);
-        const size_t T = tb / blocks;
+        const int lane = (int)(v & 63);
+        const size_t step = v >> 6;
+        const size_t T = step / steps;
         const int r = lane & 15;
         size_t n = T * 16 + r;
         bool there = n < (size_t)N;
@@ -1235,7 +1234,7 @@ __global__ void __launch_bounds__(256) tile_weights_kernel(const bf16_t *__restr
             there = o < (size_t)half_rows;
             n = o + (size_t)(r >> 3) * half_rows;
         }
-        const int k = B * 128 + u * 32 + (lane >> 4) * 8;
+        const int k = (int)(step % steps) * 32 + (lane >> 4) * 8;
         *(bf16x8_t *)(tiles + v * 8) = there ? *(const bf16x8_t *)(w + n * K + k) : zero8();
     }
 }
@@ -1620,7 +1619,7 @@ extern "C" int fllm_weight_tiles_supported(int N, int K) { return tiles_fit(N, K
 extern "C" size_t fllm_weight_tiles_elements(int N, int K) { return (size_t)((N + 15) / 16) * 16 * (size_t)K; }
 
 extern "C" int fllm_tile_weights(const void *w, void *tiles, int N, int K, hipStream_t stream) {
-    FLLM_REQUIRE(tiles_fit(N, K), "tile_weights: takes matrices of at least 16 rows whose width is a multiple of 1,024 (N=%d K=%d)", N, K);
+    FLLM_REQUIRE(N >= 16 && K >= 32 && K % 32 == 0, "tile_weights: takes matrices of at least 16 rows whose width is a multiple of 32 (N=%d K=%d)", N, K);
     FLLM_REQUIRE(w != nullptr && tiles != nullptr && aligned16(w) && aligned16(tiles), "tile_weights: operands must be there and 16-byte aligned");
     const size_t pieces = fllm_weight_tiles_elements(N, K) / 8;
     const size_t want = (pieces + 255) / 256;

@@ -1,0 +1,195 @@
+// Routed experts of decode steps (bfloat16, few (row, pick) pairs): the picked experts' matrices stream once from their
+// tile-major copies straight into matrix-core operands.
+//
+// What bounds it is the bytes of the picked experts' weights, so everything else is kept out of their way: no list of
+// pairs is made by a kernel of its own (a workgroup finds its expert's pairs in `ids` itself), no scaled copies of the rows are
+// made (an operand is scaled where it is loaded, rounded to bfloat16 as a stored copy would be), and the down product is not cut
+// into planes that a further kernel adds.  A workgroup takes 16 output columns (of gate and of up) or 32 of one expert, its eight waves
+// cut K between them with 6 to 12 KiB asked for at a time each, and they meet in LDS once.  A load of the tile-major copy is
+// 1 KiB in a row, whole cache lines that carry the non-temporal hint; the same kernel reading the rows as the checkpoint has them
+// (64 bytes of each of 16) runs at 4.4 instead of 5.9 TB/s, and through LDS in whole rows, a tile at a time, at 4.0.
+// An expert's weights serve up to 64 pairs from registers.
+//
+// MFMA operand layout (v_mfma_f32_16x16x32_bf16): A lane l holds A[m = l%16][k = 8*(l/16) .. +7]; B likewise with n = l%16;
+// D lane l holds D[m = 4*(l/16) + i][n = l%16], i = 0..3.
+#include <type_traits>
+
+#include "api.h"
+#include "common.h"
+
+namespace {
+
+constexpr int kThreads = 512, kWaves = kThreads / kWave;
+constexpr int kMostPairs = 512;
+
+// MODE 0: act[pair, c] = a(g) * (u + up_offset), x = h[pair / top] times the pick's weight (weights null: as it is), w [E][2 N][K]
+// MODE 1: out[pair, c] = w[e][c] . x[pair], float32, w [E][N][K]
+// MODE 2: act[pair, c] = relu(w[e][c] . h[pair / top])^2, w [E][N][K]
+// w is tile-major: [16 rows][K / 32] blocks of 64 lanes x 8 values (fllm_tile_weights' order; rows and K whole tiles).
+// G: groups of 16 pairs that share a load of the weights.
+template <int MODE, int G>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
+expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__restrict__ ids, const float *__restrict__ weights, int pairs,
+                     int top, const bf16_t *__restrict__ w, int E, int N, int K, int k_per, int by_pair, bf16_t *__restrict__ act,
+                     float *__restrict__ out, float limit, float alpha, float up_offset) {
+    constexpr int RT = MODE == 1 ? 1 : 2;                  // 16-row weight tiles a workgroup
+    constexpr int COLS = MODE == 2 ? 32 : 16;              // output columns a workgroup
+    constexpr int U = MODE == 0 && G > 1 ? 3 : 6;          // products a wave asks for at a time (two tiles, two groups: 128 registers)
+    __shared__ __attribute__((aligned(16))) f32x4_t red[kWaves][RT][kWave];
+    __shared__ short s_pair[kMostPairs];
+    __shared__ int s_count;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int l16 = lane & 15, lg = lane >> 4;
+    const int c0 = blockIdx.x * COLS;
+    auto expert_of = [&](int p) {
+        const int e = ids[p];
+        return e < 0 ? 0 : (e >= E ? E - 1 : e);           // never outside the stack of experts
+    };
+    // blockIdx.y names an expert, or (by_pair) a pair: then the first pair of an expert stands for it
+    const int e = by_pair ? expert_of(blockIdx.y) : (int)blockIdx.y;
+    if (wave == 0) {
+        int count = 0;
+        for (int p0 = 0; p0 < pairs; p0 += kWave) {
+            const int p = p0 + lane;
+            const bool mine = p < pairs && expert_of(p) == e;
+            const unsigned long long mask = __ballot(mine);
+            if (mine) s_pair[count + __popcll(mask & ((1ull << lane) - 1))] = (short)p;
+            count += __popcll(mask);
+        }
+        if (lane == 0) s_count = count;
+    }
+    __syncthreads();
+    const int count = s_count;
+    if (count == 0 || (by_pair && s_pair[0] != (int)blockIdx.y)) return;
+
+    const bf16_t *tiles[RT];
+#pragma unroll
+    for (int t = 0; t < RT; t++) {
+        const int c = min(c0 + (MODE == 2 ? 16 * t : 0), N - 16);      // a tile beyond the matrix reads its last one again
+        tiles[t] = w + ((size_t)e * (MODE == 0 ? 2 : 1) * N + (MODE == 0 && t == 1 ? N : 0) + c) * K + lane * 8;
+    }
+    const int k_begin = wave * k_per, k_end = min(K, k_begin + k_per);
+    for (int g0 = 0; g0 < count; g0 += 16 * G) {
+        const bf16_t *src[G];
+        float scale[G];
+        f32x4_t acc[G][RT];
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            const int pair = s_pair[min(g0 + 16 * g + l16, count - 1)];
+            src[g] = x + (size_t)(MODE == 1 ? pair : pair / top) * ldx + 8 * lg;
+            scale[g] = MODE == 0 && weights != nullptr ? weights[pair] : 1.0f;
+#pragma unroll
+            for (int t = 0; t < RT; t++) acc[g][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+        // U products, all of their loads asked for before the first product; a wave's last ones masked where they are fewer
+        auto block = [&](int k0, auto whole) {
+            bf16x8_t a[RT][U], b[G][U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int k = decltype(whole)::value ? k0 + 32 * u : min(k0 + 32 * u, k_end - 32);
+#pragma unroll
+                for (int t = 0; t < RT; t++) a[t][u] = __builtin_nontemporal_load((const bf16x8_t *)(tiles[t] + (size_t)k * 16));
+#pragma unroll
+                for (int g = 0; g < G; g++) b[g][u] = *(const bf16x8_t *)(src[g] + k);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (!decltype(whole)::value && k0 + 32 * u >= k_end) break;
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+                    if (MODE == 0 && weights != nullptr) {
+#pragma unroll
+                        for (int i = 0; i < 8; i++) b[g][u][i] = (bf16_t)((float)b[g][u][i] * scale[g]);
+                    }
+#pragma unroll
+                    for (int t = 0; t < RT; t++) acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][u], b[g][u], acc[g][t], 0, 0, 0);
+                }
+            }
+        };
+        int k0 = k_begin;
+        for (; k0 + 32 * U <= k_end; k0 += 32 * U) block(k0, std::true_type{});
+        if (k0 < k_end) block(k0, std::false_type{});
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            if (g0 + 16 * g >= count) break;
+            if (g0 + g > 0) __syncthreads();               // the sums of the pairs before have been read
+#pragma unroll
+            for (int t = 0; t < RT; t++) red[wave][t][lane] = acc[g][t];
+            __syncthreads();
+            // a thread an output: neighbours are neighbouring columns of one pair; the waves' sums in wave order
+            for (int o = threadIdx.x; o < 16 * COLS; o += kThreads) {
+                const int m = o % COLS, n = o / COLS, tile = m / 16, mm = m % 16;
+                if (g0 + 16 * g + n >= count || c0 + m >= N) continue;
+                const int from = n + 16 * (mm / 4), at = mm % 4;
+                float v = 0.f, u = 0.f;
+#pragma unroll
+                for (int s = 0; s < kWaves; s++) {
+                    v += red[s][MODE == 2 ? tile : 0][from][at];
+                    if (MODE == 0) u += red[s][RT - 1][from][at];
+                }
+                const size_t to = (size_t)s_pair[g0 + 16 * g + n] * N + c0 + m;
+                if (MODE == 0) {
+                    if (limit > 0.f) {
+                        v = fminf(v, limit);
+                        u = fminf(fmaxf(u, -limit), limit);
+                    }
+                    act[to] = (bf16_t)(v / (1.0f + expf(-alpha * v)) * (u + up_offset));
+                } else if (MODE == 2) {
+                    v = fmaxf(v, 0.f);
+                    act[to] = (bf16_t)(v * v);
+                } else {
+                    out[to] = v;
+                }
+            }
+        }
+    }
+}
+
+template <int MODE, int G>
+void launch_groups(const void *x, int ldx, const int32_t *ids, const float *weights, long pairs, int top, const void *w, int E, int N, int K,
+            void *act, float *out, float limit, float alpha, float up_offset, hipStream_t stream) {
+    const int by_pair = pairs < E;
+    const int cols = MODE == 2 ? 32 : 16;
+    const int k_per = ((K + kWaves - 1) / kWaves + 31) / 32 * 32;
+    hipLaunchKernelGGL((expert_stream_kernel<MODE, G>), dim3((N + cols - 1) / cols, by_pair ? (unsigned)pairs : (unsigned)E), dim3(kThreads), 0,
+                       stream, (const bf16_t *)x, ldx, ids, weights, (int)pairs, top, (const bf16_t *)w, E, N, K, k_per, by_pair,
+                       (bf16_t *)act, out, limit, alpha, up_offset);
+}
+
+template <int MODE>
+void launch(int groups, const void *x, int ldx, const int32_t *ids, const float *weights, long pairs, int top, const void *w, int E, int N,
+            int K, void *act, float *out, float limit, float alpha, float up_offset, hipStream_t stream) {
+    if (groups == 1) launch_groups<MODE, 1>(x, ldx, ids, weights, pairs, top, w, E, N, K, act, out, limit, alpha, up_offset, stream);
+    else launch_groups<MODE, 2>(x, ldx, ids, weights, pairs, top, w, E, N, K, act, out, limit, alpha, up_offset, stream);
+}
+
+}  // namespace
+
+// 0: launched, negative: error, 1: shape declined.  h bfloat16 [rows, K] (row stride ldh); ids / weights [rows, top] (weights null: all
+// 1); w_up the tile-major copy of [E * 2 inter, K] (gate rows, then up rows of an expert), or with gated 0 of [E * inter, K] and a
+// relu(.)^2 activation (weights must be null); w_down that of [E * N, inter]; act bfloat16 [rows * top, inter] (scratch); out float32
+// [rows * top, N].
+extern "C" int fllm_experts_stream(const void *h, int ldh, const int32_t *ids, const float *weights, int rows, int top, const void *w_up,
+                                   const void *w_down, int E, int inter, int K, int N, int gated, void *act, float *out, float limit,
+                                   float alpha, float up_offset, hipStream_t stream) {
+    FLLM_REQUIRE(rows >= 0 && top > 0 && E > 0 && inter > 0 && K > 0 && N > 0 && ldh >= K, "experts_stream: bad sizes");
+    FLLM_REQUIRE(h && ids && w_up && w_down && act && out, "experts_stream: operands missing");
+    FLLM_REQUIRE(gated || !weights, "experts_stream: experts without a gate carry their weights on the outputs");
+    if (!fllm_fast_kernels_enabled()) return 1;
+    // every wave has a product at least
+    if (K % 32 != 0 || inter % 32 != 0 || K < 32 * kWaves || inter < 32 * kWaves || N % 16 != 0 || ldh % 8 != 0 || E > 4096) return 1;
+    if ((((uintptr_t)h | (uintptr_t)w_up | (uintptr_t)w_down | (uintptr_t)act) & 15) != 0) return 1;
+    const long pairs = (long)rows * top;
+    if (pairs == 0) return 0;
+    if (pairs > kMostPairs || pairs > 16L * E) return 1;      // more pairs an expert: tiles of 64 and 128 pairs are faster (below)
+    // Measured, microseconds of both products (grouped_tiles_kernel with what it needs around it -> this kernel with one, with two groups),
+    // weights from memory, 8 experts of 4,480 lanes at a width of 1,536, two picks a row:
+    //   1 row (one pair at a time -> this) 25 -> 22;  4 rows 55 -> 39;  8 rows 70 -> 51, 54;  16 rows 75 -> 57, 59;
+    //   32 rows 77 -> 61, 62;  48 rows 77 -> 80, 70;  64 rows 78 -> 92, 75;  96 rows 83 -> 123, 92
+    // (165 of 330 MB at one row's share; 5.8 TB/s at 16 rows); 8 experts of 2,048 lanes at 1,024: 8 rows 37 -> 19, 64 rows 42 -> 38, 32.
+    const int groups = pairs <= 8L * E ? 1 : 2;
+    if (gated) launch<0>(groups, h, ldh, ids, weights, pairs, top, w_up, E, inter, K, act, nullptr, limit, alpha, up_offset, stream);
+    else launch<2>(groups, h, ldh, ids, nullptr, pairs, top, w_up, E, inter, K, act, nullptr, 0.f, 0.f, 0.f, stream);
+    launch<1>(groups, act, inter, ids, nullptr, pairs, 1, w_down, E, N, inter, nullptr, out, 0.f, 0.f, 0.f, stream);
+    return fllm_check_launch("experts_stream");
+}

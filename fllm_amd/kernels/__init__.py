@@ -182,6 +182,8 @@ def load_library(build_if_missing: bool = True):
         "fllm_relu_squared": [c_void, c_void, c_size, c_int, c_void],
         "fllm_route_grouped": [c_void, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_int, c_void, c_void, c_float, c_int,
                                c_void],
+        "fllm_experts_stream": [c_void, c_int, c_void, c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_void,
+                                c_void, c_float, c_float, c_float, c_void],
         "fllm_experts_grouped_ungated": [c_void, c_int, c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_void, c_void,
                                          c_void, c_void, c_void],
         "fllm_experts_up": [c_void, c_int, c_void, c_int, c_int, c_void, c_int, c_int, c_int, c_void, c_int, c_void],
@@ -959,6 +961,60 @@ class Ops:
         code = self.lib.fllm_experts_grouped(_ptr(h), h.stride(0), _ptr(ids), _ptr(weights), rows, top, _ptr(w_gate_up), _ptr(w_down), E,
                                              two_i // 2, K, N, _ptr(act), _ptr(xs), _ptr(out), _ptr(work), _ptr(planes), float(limit), float(alpha),
                                              float(up_offset), self._stream())
+        if code == 1:
+            return False
+        self._check(code)
+        return True
+
+    def tile_experts(self, w: torch.Tensor) -> bool:
+        """Keeps beside a stack of experts' matrices (bfloat16 [experts, N, K] on the GPU, N in steps of 16, K in steps of 32 from 256 on) a copy in
+        the order `experts_stream` reads it, as `tile_for_decode` does for single matrices; given up with `w`."""
+        if not (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 3 and w.is_contiguous()):
+            return False
+        E, N, K = w.shape
+        if N % 16 != 0 or K % 32 != 0 or K < 256 or E * N >= 1 << 31:
+            return False
+        key, kind = w.data_ptr(), ("experts", E, N, K)
+        if key in Ops._tiles and Ops._tiles[key][0] == kind:
+            return True
+        with torch.cuda.device(w.device):
+            tiles = torch.empty(E * N * K, dtype=torch.bfloat16, device=w.device)
+            self._check(self.lib.fllm_tile_weights(_ptr(w), _ptr(tiles), E * N, K, self._stream()))
+        Ops._tiles[key] = (kind, tiles)
+        weakref.finalize(w, Ops._tiles.pop, key, None)
+        return True
+
+    def _expert_tiles_of(self, w: torch.Tensor) -> Optional[torch.Tensor]:
+        held = Ops._tiles.get(w.data_ptr())
+        return held[1] if held is not None and held[0] == ("experts",) + tuple(w.shape) else None
+
+    def experts_stream(self, h: torch.Tensor, ids: torch.Tensor, weights: Optional[torch.Tensor], w_up: torch.Tensor, w_down: torch.Tensor,
+                       out: torch.Tensor, gated: bool = True, limit: float = 0.0, alpha: float = 1.0, up_offset: float = 0.0) -> bool:
+        """`experts_gate_up` (gated; weights None: all 1) or `experts_up` and then `experts_down` for steps of few pairs (bfloat16): the
+        picked experts' matrices stream once, from their tile-major copies (`tile_experts`).  out float32 [rows * top, width].  False: not
+        taken (no copies, more than 16 pairs an expert, float32, other sizes), nothing was written."""
+        if h.dtype != torch.bfloat16 or not h.is_cuda or not Ops._tiles:
+            return False
+        up_tiles, down_tiles = self._expert_tiles_of(w_up), self._expert_tiles_of(w_down)
+        if up_tiles is None or down_tiles is None:
+            return False
+        rows, K = h.shape
+        top = ids.shape[1]
+        E, inter, N = w_up.shape[0], w_up.shape[1] // (2 if gated else 1), w_down.shape[1]
+        if rows * top > 16 * E or rows * top > 512:
+            return False
+        _need(h.dim() == 2 and h.stride(1) == 1, "h must be a row-major matrix")
+        _need(gated or weights is None, "experts without a gate carry their weights on the outputs")
+        _dense(w_up, "w_up", h.dtype, (E, inter * (2 if gated else 1), K))
+        _dense(w_down, "w_down", h.dtype, (E, N, inter))
+        _dense(ids, "ids", torch.int32, (rows, top))
+        if weights is not None:
+            _dense(weights, "weights", torch.float32, (rows, top))
+        _dense(out, "out", torch.float32, (rows * top, N))
+        act = torch.empty((rows * top, inter), dtype=h.dtype, device=h.device)
+        code = self.lib.fllm_experts_stream(_ptr(h), h.stride(0) if rows > 1 else K, _ptr(ids), _ptr(weights), rows, top, _ptr(up_tiles),
+                                            _ptr(down_tiles), E, inter, K, N, 1 if gated else 0, _ptr(act), _ptr(out), float(limit),
+                                            float(alpha), float(up_offset), self._stream())
         if code == 1:
             return False
         self._check(code)

@@ -87,6 +87,8 @@ class RoutedExperts(FeedForward):
                 raise ValueError("experts without a gate carry their weight on the output and clamp nothing")
             self.w_up = torch.stack([rt.matrix(weights[f"up_{e}"]) for e in range(n)]).contiguous()
         self.w_down = torch.stack([rt.matrix(weights[f"down_{e}"]) for e in range(n)]).contiguous()
+        rt.tile_experts(self.w_gate_up if self.gated else self.w_up)
+        rt.tile_experts(self.w_down)
         self.shared = int(spec.get("shared") or 0)
         if self.shared:
             if self.gated:
@@ -122,7 +124,11 @@ class RoutedExperts(FeedForward):
             on_output, weights = weights, None
         parts = branch if branch is not None else rt.empty((rows * self.top, self.hidden), torch.float32)
         grouped = getattr(ops, "experts_grouped", None)
-        if not self.gated:
+        stream = getattr(ops, "experts_stream", None)        # decode steps
+        if stream is not None and stream(h, ids, weights, self.w_gate_up if self.gated else self.w_up, self.w_down, parts, self.gated, self.limit,
+                                         self.alpha, self.up_offset):
+            pass
+        elif not self.gated:
             ungrouped = getattr(ops, "experts_grouped_ungated", None)
             if ungrouped is None or not ungrouped(h, ids, self.w_up, self.w_down, parts):
                 act = rt.empty((rows * self.top, self.inter))

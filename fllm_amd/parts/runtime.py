@@ -51,17 +51,27 @@ class Runtime:
         `priority`: while a model is being built the copies are only asked for, and made when it is whole
         (`tiles_for_model`), the lower numbers first: 0 for copies that every decode step reads (output and down
         projections), 1 for the layers' other matrices, 2 for the vocabulary projection (once a step)."""
-        make = getattr(self.ops, "tile_for_decode", None)
-        if not self.decode_weight_tiles or make is None or self.dtype != torch.bfloat16 or not w.is_cuda:
+        tile = getattr(self.ops, "tile_for_decode", None)
+        if tile is not None:
+            self._ask_for_copy(w, (lambda t: tile(t, gate_up=True)) if gate_up else tile, priority)
+
+    def tile_experts(self, w: torch.Tensor, priority: int = 1) -> None:
+        """The same for a stack of experts' matrices [experts, N, K] (`Ops.tile_experts`)."""
+        tile = getattr(self.ops, "tile_experts", None)
+        if tile is not None:
+            self._ask_for_copy(w, tile, priority)
+
+    def _ask_for_copy(self, w: torch.Tensor, make, priority: int) -> None:
+        if not self.decode_weight_tiles or self.dtype != torch.bfloat16 or not w.is_cuda:
             return
         if self._tile_requests is not None:
-            self._tile_requests.append((priority, len(self._tile_requests), w, gate_up))
+            self._tile_requests.append((priority, len(self._tile_requests), w, make))
             return
         if self.decode_weight_tiles == "auto":
             free, _ = torch.cuda.mem_get_info(self.device)
             if w.numel() * w.element_size() > free // 20:
                 return                                    # the device is filling up
-        make(w, gate_up=True) if gate_up else make(w)
+        make(w)
 
     def collect_tile_requests(self) -> None:
         """From here on `tile_for_decode` only notes what is asked for, until `tiles_for_model`."""
@@ -73,8 +83,7 @@ class Runtime:
         cache's).  A copy that does not fit is left out and smaller ones behind it may still be made, so a model too
         large for all copies keeps those that every step reads.  Returns the bytes copied."""
         requests, self._tile_requests = sorted(self._tile_requests or [], key=lambda r: r[:2]), None
-        make = getattr(self.ops, "tile_for_decode", None)
-        if not requests or make is None:
+        if not requests:
             return 0
         budget = None
         if self.decode_weight_tiles == "auto":
@@ -82,11 +91,11 @@ class Runtime:
             free, _ = torch.cuda.mem_get_info(self.device)
             budget = free // 2
         made = 0
-        for _, _, w, gate_up in requests:
+        for _, _, w, make in requests:
             size = w.numel() * w.element_size()
             if budget is not None and size > budget:
                 continue
-            if make(w, gate_up=True) if gate_up else make(w):
+            if make(w):
                 made += size
                 if budget is not None:
                     budget -= size
