@@ -993,48 +993,67 @@ __device__ __forceinline__ float penalised(float v, const FllmAdjustRow &a, int 
     return v - (a.presence_penalty + a.frequency_penalty * (float)count);
 }
 
+// grid (rows, parts): a workgroup has kAdjustSpan neighbouring tokens of a row and applies of every list what falls on them, so that the
+// workgroups of a row never meet.  An allow list blocks nearly the whole vocabulary; with one workgroup a row that looked every token up in
+// the list it took 122 us of a step of 16 rows at a vocabulary of 128,256, and takes 8 like this.
+constexpr int kAdjustSpan = 8192;
+
+__device__ __forceinline__ int first_at_least(const int32_t *__restrict__ rising, int n, int value) {
+    int lo = 0, hi = n;                            // the first entry >= value lies in [lo, hi]
+    while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        if (rising[mid] < value) lo = mid + 1; else hi = mid;
+    }
+    return lo;
+}
+
 __global__ void __launch_bounds__(kAdjustBlock)
 adjust_logits_kernel(float *__restrict__ logits, int vocab, const FllmAdjustRow *__restrict__ rows, const FllmAdjustLists lists,
                      const int32_t *__restrict__ last_tokens) {
     __shared__ int last_was_listed;
+    __shared__ unsigned int allowed_bits[kAdjustSpan / 32];
     const FllmAdjustRow a = rows[blockIdx.x];
+    const int begin = blockIdx.y * kAdjustSpan, end = min(vocab, begin + kAdjustSpan);
+    const auto mine = [&](int id) { return id >= begin && id < end; };
     float *w = logits + (size_t)blockIdx.x * vocab;
     const int last = a.last_row >= 0 ? last_tokens[a.last_row] : -1;
     if (threadIdx.x == 0) last_was_listed = 0;
     __syncthreads();
     for (int j = threadIdx.x; j < a.seen_len; j += kAdjustBlock) {        // ids of a row are distinct: no two threads meet
         const int id = lists.seen_ids[a.seen_off + j];
-        if (id < 0 || id >= vocab) continue;
+        if (!mine(id)) continue;
         int count = lists.seen_counts[a.seen_off + j];
         if (id == last) count++, last_was_listed = 1;
         w[id] = penalised(w[id], a, count);
     }
     __syncthreads();
-    if (threadIdx.x == 0 && last >= 0 && last < vocab && !last_was_listed) w[last] = penalised(w[last], a, 1);
+    if (threadIdx.x == 0 && mine(last) && !last_was_listed) w[last] = penalised(w[last], a, 1);
     __syncthreads();
     for (int j = threadIdx.x; j < a.bias_len; j += kAdjustBlock) {
         const int id = lists.bias_ids[a.bias_off + j];
-        if (id >= 0 && id < vocab) w[id] += lists.bias_values[a.bias_off + j];
+        if (mine(id)) w[id] += lists.bias_values[a.bias_off + j];
     }
     __syncthreads();
     for (int j = threadIdx.x; j < a.blocked_len; j += kAdjustBlock) {
         const int id = lists.blocked_ids[a.blocked_off + j];
-        if (id >= 0 && id < vocab) w[id] = -INFINITY;
+        if (mine(id)) w[id] = -INFINITY;
     }
     for (int j = threadIdx.x; j < a.pairs_len; j += kAdjustBlock) {
         const int id = lists.then_blocked[a.pairs_off + j];
-        if (lists.if_last[a.pairs_off + j] == last && id >= 0 && id < vocab) w[id] = -INFINITY;
+        if (lists.if_last[a.pairs_off + j] == last && mine(id)) w[id] = -INFINITY;
     }
     if (a.allowed_len > 0) {                       // every token that is not on the rising list
         const int32_t *allowed = lists.allowed_ids + a.allowed_off;
-        for (int i = threadIdx.x; i < vocab; i += kAdjustBlock) {
-            int lo = 0, hi = a.allowed_len;        // the first entry >= i lies in [lo, hi]
-            while (lo < hi) {
-                const int mid = (lo + hi) / 2;
-                if (allowed[mid] < i) lo = mid + 1; else hi = mid;
-            }
-            if (lo == a.allowed_len || allowed[lo] != i) w[i] = -INFINITY;
+        const int from = first_at_least(allowed, a.allowed_len, begin), to = first_at_least(allowed, a.allowed_len, end);
+        for (int i = threadIdx.x; i < kAdjustSpan / 32; i += kAdjustBlock) allowed_bits[i] = 0;
+        __syncthreads();
+        for (int j = from + threadIdx.x; j < to; j += kAdjustBlock) {
+            const int at = allowed[j] - begin;
+            atomicOr(&allowed_bits[at / 32], 1u << (at % 32));
         }
+        __syncthreads();
+        for (int i = begin + threadIdx.x; i < end; i += kAdjustBlock)
+            if (!(allowed_bits[(i - begin) / 32] >> ((i - begin) % 32) & 1u)) w[i] = -INFINITY;
     }
 }
 
@@ -1250,7 +1269,7 @@ extern "C" int fllm_adjust_logits(float *logits, int rows, int vocab, const Fllm
     FLLM_REQUIRE(rows >= 0 && vocab > 0, "adjust_logits: bad sizes rows=%d vocab=%d", rows, vocab);
     if (rows == 0) return 0;
     FLLM_REQUIRE(logits != nullptr && row_records != nullptr && lists != nullptr, "adjust_logits: logits, row records and lists are required");
-    hipLaunchKernelGGL(adjust_logits_kernel, dim3(rows), dim3(kAdjustBlock), 0, stream, logits, vocab, row_records, *lists, last_tokens);
+    hipLaunchKernelGGL(adjust_logits_kernel, dim3(rows, (vocab + kAdjustSpan - 1) / kAdjustSpan), dim3(kAdjustBlock), 0, stream, logits, vocab, row_records, *lists, last_tokens);
     return fllm_check_launch("adjust_logits");
 }
 
