@@ -619,41 +619,96 @@ __global__ void __launch_bounds__(kBlock) relu_squared_vec_kernel(const bf16_t *
     *(bf16x8_t *)(out + i * 8) = v;
 }
 
-// normed_rope_store for heads normed over their own lanes, no rotation, keys in chunks of 8: a thread takes eight lanes, `lanes` threads
-// (a power of two of at least k_dim / 8, at most a wave) a head; then the values, eight lanes a thread.
+// normed_rope_store for bfloat16 rows, eight neighbouring lanes a thread: everything the row needs (the lanes, the ones they turn with,
+// weights, angles, the other layer's values) is asked for at once, so that a row waits for memory once behind its position.  One workgroup a
+// row; a head's `lanes` threads (a power of two) lie side by side.  Lane by lane, with a wait a step, a row of 12 + 2 heads of 128 took
+// 13.0 us in a decode step of two rows; like this 5.5.
+// norm_mode as in normed_rope_store_kernel; rope_dims / 2 a multiple of 8.
 __global__ void __launch_bounds__(kBlock)
-normed_store_vec_kernel(const bf16_t *__restrict__ qkv, int ld, const float *__restrict__ q_weight, const float *__restrict__ k_weight, float eps,
-                        bf16_t *__restrict__ q_out, const int32_t *__restrict__ row_pos, const int32_t *__restrict__ row_seg,
-                        const int32_t *__restrict__ tables, int table_stride, bf16_t *__restrict__ k_pages, bf16_t *__restrict__ v_pages, int heads,
-                        int kv_heads, int k_dim, int v_dim, int page_size, int store_kv, const bf16_t *__restrict__ blend, int blend_ld,
-                        const float *__restrict__ blend_amount, int lanes) {
+normed_rope_store_vec_kernel(const bf16_t *__restrict__ qkv, int ld, int norm_mode, const float *__restrict__ q_weight,
+                             const float *__restrict__ k_weight, float eps, bf16_t *__restrict__ q_out, const int32_t *__restrict__ row_pos,
+                             const int32_t *__restrict__ row_seg, const int32_t *__restrict__ tables, int table_stride,
+                             const float *__restrict__ cos_table, const float *__restrict__ sin_table, bf16_t *__restrict__ k_pages,
+                             bf16_t *__restrict__ v_pages, int heads, int kv_heads, int k_dim, int v_dim, int rope_dims, int page_size,
+                             int store_kv, int values_from_keys, const bf16_t *__restrict__ blend, int blend_ld,
+                             const float *__restrict__ blend_amount, int lanes) {
+    __shared__ float scratch[2 * kWaves];
     const size_t r = blockIdx.x;
-    const int seg = row_seg[r];
-    if (seg < 0) return;
-    const int pos = row_pos[r], off = pos % page_size;
+    const int seg = row_seg[r], pos = row_pos[r];
     const bf16_t *row = qkv + r * ld;
-    const int page = store_kv ? tables[(size_t)seg * table_stride + pos / page_size] : 0;
-    const int all = heads + (store_kv ? kv_heads : 0), each = kBlock / lanes, c = (threadIdx.x % lanes) * 8;
-    for (int h = threadIdx.x / lanes; h < all; h += each) {      // the lanes of a head stay together: shuffles below reach active lanes
-        bf16x8_t v;
-        float ss = 0.f;
-        if (c < k_dim) {
-            v = *(const bf16x8_t *)(row + (size_t)h * k_dim + c);
+    const int each = kBlock / lanes, c = (threadIdx.x % lanes) * 8, half = rope_dims / 2;
+    const bool turns = c < rope_dims;
+    const int pc = c < half ? c + half : c - half;              // the lanes that these turn with
+    const int all = heads + kv_heads;
+    float inv_q = 1.f, inv_k = 1.f;
+    if (norm_mode == 2) {                                       // one norm over all of q, one over all of k
+        float sq = 0.f, sk = 0.f;
+        for (int e0 = threadIdx.x * 8; e0 < all * k_dim; e0 += kBlock * 8) {
+            const bf16x8_t v = *(const bf16x8_t *)(row + e0);
+            float ss = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; e++) ss = fmaf((float)v[e], (float)v[e], ss);
+            if (e0 < heads * k_dim) sq += ss;
+            else sk += ss;
         }
-        for (int o = lanes / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, kWave);
-        if (c >= k_dim) continue;
-        const float inv = 1.0f / sqrtf(ss / (float)k_dim + eps);
-        const float *w = (h < heads ? q_weight : k_weight) + c;
-        const f32x4_t w0 = *(const f32x4_t *)w, w1 = *(const f32x4_t *)(w + 4);
+        sq = wave_sum(sq);
+        sk = wave_sum(sk);
+        if ((threadIdx.x & (kWave - 1)) == 0) scratch[threadIdx.x / kWave] = sq, scratch[kWaves + threadIdx.x / kWave] = sk;
+        __syncthreads();
+        sq = sk = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = (bf16_t)((float)v[e] * inv * (e < 4 ? w0[e & 3] : w1[e & 3]));
-        if (h < heads) *(bf16x8_t *)(q_out + (r * heads + h) * k_dim + c) = v;
-        else *(bf16x8_t *)(k_pages + key_offset(page, kv_heads, h - heads, page_size, k_dim, off, c)) = v;
+        for (int i = 0; i < kWaves; i++) sq += scratch[i], sk += scratch[kWaves + i];
+        inv_q = 1.0f / sqrtf(sq / (float)(heads * k_dim) + eps);
+        inv_k = 1.0f / sqrtf(sk / (float)(kv_heads * k_dim) + eps);
+    }
+    if (seg < 0) return;                                        // padding row: its queries are never read
+    const int off = pos % page_size;
+    const int page = store_kv ? tables[(size_t)seg * table_stride + pos / page_size] : 0;
+    const float *cs = cos_table + (size_t)pos * half, *sn = sin_table + (size_t)pos * half;
+    // the lanes of a head stay together: the shuffles below reach active lanes
+    for (int h = threadIdx.x / lanes; h < (store_kv ? all : heads); h += each) {
+        const bool is_q = h < heads, there = c < k_dim;
+        bf16x8_t v = {}, p = {};
+        f32x4_t w[2], wp[2], cv[2], sv[2];
+        if (there) {
+            const bf16_t *head = row + (size_t)h * k_dim;
+            const float *weight = (is_q ? q_weight : k_weight) + (norm_mode == 2 ? (size_t)(is_q ? h : h - heads) * k_dim : 0);
+            v = *(const bf16x8_t *)(head + c);
+            if (turns) p = *(const bf16x8_t *)(head + pc);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                if (norm_mode != 0) w[j] = *(const f32x4_t *)(weight + c + 4 * j);
+                if (!turns) continue;
+                if (norm_mode != 0) wp[j] = *(const f32x4_t *)(weight + pc + 4 * j);
+                cv[j] = *(const f32x4_t *)(cs + (c < half ? c : pc) + 4 * j);
+                sv[j] = *(const f32x4_t *)(sn + (c < half ? c : pc) + 4 * j);
+            }
+        }
+        float inv = is_q ? inv_q : inv_k;
+        if (norm_mode == 1) {
+            float ss = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) ss = fmaf((float)v[e], (float)v[e], ss);
+            for (int o = lanes / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, kWave);
+            inv = 1.0f / sqrtf(ss / (float)k_dim + eps);
+        }
+        if (!there) continue;
+        bf16x8_t o8;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            float val = (float)v[e] * inv * (norm_mode != 0 ? w[e / 4][e % 4] : 1.f);
+            if (turns) {
+                const float other = (float)p[e] * inv * (norm_mode != 0 ? wp[e / 4][e % 4] : 1.f);
+                const float cc = cv[e / 4][e % 4], ss = sv[e / 4][e % 4];
+                val = c < half ? val * cc - other * ss : val * cc + other * ss;
+            }
+            o8[e] = (bf16_t)val;
+        }
+        if (is_q) *(bf16x8_t *)(q_out + (r * heads + h) * k_dim + c) = o8;
+        else *(bf16x8_t *)(k_pages + key_offset(page, kv_heads, h - heads, page_size, k_dim, off, c)) = o8;
     }
     if (!store_kv) return;
-    const bf16_t *values = row + (size_t)(heads + kv_heads) * k_dim;
+    const bf16_t *values = row + (size_t)(values_from_keys ? heads : all) * k_dim;
     const float a = blend != nullptr ? blend_amount[0] : 0.f;
     for (int e0 = threadIdx.x * 8; e0 < kv_heads * v_dim; e0 += kBlock * 8) {
         bf16x8_t v = *(const bf16x8_t *)(values + e0);
@@ -680,6 +735,43 @@ int small_grid(size_t total) {
 
 }  // namespace
 
+// What fllm_normed_rope_store launches, its operands checked by the caller (fllm_qk_norm_rope_store is the other one).
+int fllm_launch_normed_rope_store(const void *qkv, int ld, int norm_mode, const float *q_weight, const float *k_weight, float eps,
+                                  void *q_out, const int32_t *row_pos, const int32_t *row_seg, const int32_t *tables,
+                                  int table_stride, const float *cos_table, const float *sin_table, int table_positions,
+                                  void *k_pages, void *v_pages, int rows, int heads, int kv_heads, int k_dim, int v_dim,
+                                  int rope_dims, int page_size, int key_chunk, int dtype, int store_kv, int values_from_keys,
+                                  const void *blend, int blend_ld, const float *blend_amount, hipStream_t stream) {
+    if (rows == 0) return 0;
+    const size_t smem = (size_t)(heads + kv_heads) * sizeof(float);
+    const uintptr_t bases = (uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)blend | (uintptr_t)q_weight | (uintptr_t)k_weight |
+                            (rope_dims > 0 ? (uintptr_t)cos_table | (uintptr_t)sin_table : 0);
+    // whole pieces of 8 lanes everywhere, on 16 bytes; a head's threads in one wave
+    if (dtype == FLLM_BF16 && rope_dims % 16 == 0 && key_chunk == 8 && k_dim % 8 == 0 && k_dim <= 8 * kWave && v_dim % 8 == 0 && ld % 8 == 0 &&
+        blend_ld % 8 == 0 && (bases & 15) == 0) {
+        int lanes = 1;
+        while (lanes < k_dim / 8) lanes *= 2;
+        hipLaunchKernelGGL(normed_rope_store_vec_kernel, dim3(rows), dim3(kBlock), 0, stream, (const bf16_t *)qkv, ld, norm_mode, q_weight, k_weight,
+                           eps, (bf16_t *)q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table, (bf16_t *)k_pages,
+                           (bf16_t *)v_pages, heads, kv_heads, k_dim, v_dim, rope_dims, page_size, store_kv, values_from_keys,
+                           (const bf16_t *)blend, blend_ld, blend_amount, lanes);
+        return fllm_check_launch("normed_rope_store");
+    }
+    if (dtype == FLLM_F32)
+        hipLaunchKernelGGL(normed_rope_store_kernel<float>, dim3(rows), dim3(kBlock), smem, stream, (const float *)qkv, ld, norm_mode,
+                           q_weight, k_weight, eps, (float *)q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table,
+                           (float *)k_pages, (float *)v_pages, heads, kv_heads, k_dim, v_dim, rope_dims, page_size, key_chunk, store_kv,
+                           values_from_keys, (const float *)blend, blend_ld, blend_amount);
+    else if (dtype == FLLM_BF16)
+        hipLaunchKernelGGL(normed_rope_store_kernel<bf16_t>, dim3(rows), dim3(kBlock), smem, stream, (const bf16_t *)qkv, ld, norm_mode,
+                           q_weight, k_weight, eps, (bf16_t *)q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table,
+                           (bf16_t *)k_pages, (bf16_t *)v_pages, heads, kv_heads, k_dim, v_dim, rope_dims, page_size, key_chunk,
+                           store_kv, values_from_keys, (const bf16_t *)blend, blend_ld, blend_amount);
+    else
+        FLLM_REQUIRE(false, "normed_rope_store: unknown dtype %d", dtype);
+    return fllm_check_launch("normed_rope_store");
+}
+
 extern "C" int fllm_normed_rope_store(const void *qkv, int ld, int norm_mode, const float *q_weight, const float *k_weight, float eps,
                                       void *q_out, const int32_t *row_pos, const int32_t *row_seg, const int32_t *tables,
                                       int table_stride, const float *cos_table, const float *sin_table, int table_positions,
@@ -701,31 +793,10 @@ extern "C" int fllm_normed_rope_store(const void *qkv, int ld, int norm_mode, co
                  "normed_rope_store: operands missing");
     FLLM_REQUIRE(blend == nullptr || (blend_amount != nullptr && blend_ld >= kv_heads * v_dim && !values_from_keys),
                  "normed_rope_store: values that are mixed in need rows of %d and an amount", kv_heads * v_dim);
-    if (rows == 0) return 0;
-    const size_t smem = (size_t)(heads + kv_heads) * sizeof(float);
-    const uintptr_t bases = (uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)blend | (uintptr_t)q_weight | (uintptr_t)k_weight;
-    if (dtype == FLLM_BF16 && norm_mode == 1 && rope_dims == 0 && !values_from_keys && key_chunk == 8 && k_dim % 8 == 0 && k_dim <= 8 * kWave &&
-        v_dim % 8 == 0 && ld % 8 == 0 && blend_ld % 8 == 0 && (bases & 15) == 0) {
-        int lanes = 1;
-        while (lanes < k_dim / 8) lanes *= 2;
-        hipLaunchKernelGGL(normed_store_vec_kernel, dim3(rows), dim3(kBlock), 0, stream, (const bf16_t *)qkv, ld, q_weight, k_weight, eps,
-                           (bf16_t *)q_out, row_pos, row_seg, tables, table_stride, (bf16_t *)k_pages, (bf16_t *)v_pages, heads, kv_heads, k_dim,
-                           v_dim, page_size, store_kv, (const bf16_t *)blend, blend_ld, blend_amount, lanes);
-        return fllm_check_launch("normed_rope_store");
-    }
-    if (dtype == FLLM_F32)
-        hipLaunchKernelGGL(normed_rope_store_kernel<float>, dim3(rows), dim3(kBlock), smem, stream, (const float *)qkv, ld, norm_mode,
-                           q_weight, k_weight, eps, (float *)q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table,
-                           (float *)k_pages, (float *)v_pages, heads, kv_heads, k_dim, v_dim, rope_dims, page_size, key_chunk, store_kv,
-                           values_from_keys, (const float *)blend, blend_ld, blend_amount);
-    else if (dtype == FLLM_BF16)
-        hipLaunchKernelGGL(normed_rope_store_kernel<bf16_t>, dim3(rows), dim3(kBlock), smem, stream, (const bf16_t *)qkv, ld, norm_mode,
-                           q_weight, k_weight, eps, (bf16_t *)q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table,
-                           (bf16_t *)k_pages, (bf16_t *)v_pages, heads, kv_heads, k_dim, v_dim, rope_dims, page_size, key_chunk,
-                           store_kv, values_from_keys, (const bf16_t *)blend, blend_ld, blend_amount);
-    else
-        FLLM_REQUIRE(false, "normed_rope_store: unknown dtype %d", dtype);
-    return fllm_check_launch("normed_rope_store");
+    return fllm_launch_normed_rope_store(qkv, ld, norm_mode, q_weight, k_weight, eps, q_out, row_pos, row_seg, tables, table_stride,
+                                         cos_table, sin_table, table_positions, k_pages, v_pages, rows, heads, kv_heads, k_dim, v_dim,
+                                         rope_dims, page_size, key_chunk, dtype, store_kv, values_from_keys, blend, blend_ld,
+                                         blend_amount, stream);
 }
 
 extern "C" int fllm_pool_blocks(const void *k_pages, const void *v_pages, float *pool_k, float *pool_v, const int32_t *tables,

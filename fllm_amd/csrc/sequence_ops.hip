@@ -309,6 +309,59 @@ gated_norm_kernel(const X *__restrict__ x, const float *__restrict__ w, float ep
     }
 }
 
+// The same for bfloat16 rows out, widths in steps of 4 and everything on 16 (rows in float32) or 8 bytes: a thread holds NV pieces of four
+// lanes of the row, the weight and the gate, asked for at once (1,536 lanes at 4 rows: 7.4 us in two rounds lane by lane, 4.7 like this).
+template <int NV, typename X>
+__global__ void __launch_bounds__(kBlock)
+gated_norm_vec_kernel(const X *__restrict__ x, const float *__restrict__ w, float eps, const bf16_t *__restrict__ gate, int gate_ld,
+                      bf16_t *__restrict__ out, int width) {
+    __shared__ float scratch[kWaves];
+    const size_t r = blockIdx.x;
+    float v[NV][4];
+    f32x4_t weight[NV];
+    bf16x4_t g[NV];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int c = (i * kBlock + threadIdx.x) * 4;
+        if (c >= width) break;
+        if constexpr (sizeof(X) == 4) {
+            const f32x4_t a = *(const f32x4_t *)(x + r * width + c);
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[i][e] = a[e];
+        } else {
+            const bf16x4_t a = *(const bf16x4_t *)(x + r * width + c);
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[i][e] = (float)a[e];
+        }
+        g[i] = *(const bf16x4_t *)(gate + r * gate_ld + c);
+        if (w != nullptr) weight[i] = *(const f32x4_t *)(w + c);
+    }
+    float inv = 1.0f;
+    if (w != nullptr) {
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            if ((i * kBlock + threadIdx.x) * 4 >= width) break;
+#pragma unroll
+            for (int e = 0; e < 4; e++) ss = fmaf(v[i][e], v[i][e], ss);
+        }
+        inv = 1.0f / sqrtf(block_sum<kWaves>(ss, scratch) / (float)width + eps);
+    }
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int c = (i * kBlock + threadIdx.x) * 4;
+        if (c >= width) break;
+        bf16x4_t o;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            float a = v[i][e] * inv;
+            if (w != nullptr) a *= weight[i][e];
+            o[e] = (bf16_t)(a * sigmoid_f((float)g[i][e]));
+        }
+        *(bf16x4_t *)(out + r * width + c) = o;
+    }
+}
+
 // ---- polynomial activation with normed powers -----------------------------------------------------------------------------------
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
@@ -334,6 +387,57 @@ polynorm_kernel(const T *__restrict__ z, int ld, const float *__restrict__ coeff
     for (int c = threadIdx.x; c < width; c += kBlock) {
         const float a = to_f32<T>(src[c]);
         out[r * width + c] = from_f32<T>(fmaf(a, fmaf(a, fmaf(a, c3, c2), c1), c0));
+    }
+}
+
+// The same for bfloat16 rows in pieces of 8 on 16 bytes: a workgroup of 1,024 threads keeps the row in registers, NV pieces a thread, and
+// adds up the three sums in one meeting (8,960 lanes at 4 rows: 8.0 us with 256 threads that read the row twice, 5.9 like this).
+constexpr int kPolyBlock = 1024;
+template <int NV>
+__global__ void __launch_bounds__(kPolyBlock)
+polynorm_vec_kernel(const bf16_t *__restrict__ z, int ld, const float *__restrict__ coeffs, float eps, bf16_t *__restrict__ out, int width) {
+    __shared__ float scratch[3][kPolyBlock / kWave];
+    const size_t r = blockIdx.x;
+    bf16x8_t v[NV];
+    const float k0 = coeffs[0], k1 = coeffs[1], k2 = coeffs[2], c0 = coeffs[3];
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int c = (i * kPolyBlock + threadIdx.x) * 8;
+        if (c < width) v[i] = *(const bf16x8_t *)(z + r * ld + c);
+    }
+    float s2 = 0.f, s4 = 0.f, s6 = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        if ((i * kPolyBlock + threadIdx.x) * 8 >= width) break;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float a = (float)v[i][e], a2 = a * a, a3 = a2 * a;
+            s2 += a2;
+            s4 = fmaf(a2, a2, s4);
+            s6 = fmaf(a3, a3, s6);
+        }
+    }
+    s2 = wave_sum(s2);
+    s4 = wave_sum(s4);
+    s6 = wave_sum(s6);
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    if (lane == 0) scratch[0][wave] = s2, scratch[1][wave] = s4, scratch[2][wave] = s6;
+    __syncthreads();
+    s2 = s4 = s6 = 0.f;
+#pragma unroll
+    for (int i = 0; i < kPolyBlock / kWave; i++) s2 += scratch[0][i], s4 += scratch[1][i], s6 += scratch[2][i];
+    const float n = (float)width;
+    const float c1 = k0 / sqrtf(s2 / n + eps), c2 = k1 / sqrtf(s4 / n + eps), c3 = k2 / sqrtf(s6 / n + eps);
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int c = (i * kPolyBlock + threadIdx.x) * 8;
+        if (c >= width) break;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float a = (float)v[i][e];
+            v[i][e] = (bf16_t)fmaf(a, fmaf(a, fmaf(a, c3, c2), c1), c0);
+        }
+        *(bf16x8_t *)(out + r * width + c) = v[i];
     }
 }
 
@@ -486,6 +590,26 @@ extern "C" int fllm_gated_norm(const void *x, int x_dtype, const float *w, float
     FLLM_REQUIRE(rows >= 0 && width > 0 && gate_ld >= width, "gated_norm: bad sizes");
     FLLM_REQUIRE(x && gate && out, "gated_norm: operands missing");
     if (rows == 0) return 0;
+    const uintptr_t bases = (uintptr_t)x | (uintptr_t)w;
+    if (dtype == FLLM_BF16 && width % 4 == 0 && width <= 8 * 4 * kBlock && gate_ld % 4 == 0 && (bases & 15) == 0 &&
+        (((uintptr_t)gate | (uintptr_t)out) & 7) == 0) {
+#define FLLM_GATED_VEC(NV, X)                                                                                                          \
+    hipLaunchKernelGGL((gated_norm_vec_kernel<NV, X>), dim3(rows), dim3(kBlock), 0, stream, (const X *)x, w, eps, (const bf16_t *)gate, gate_ld, \
+                       (bf16_t *)out, width)
+#define FLLM_GATED_ROW(X)                              \
+    do {                                               \
+        if (pieces <= 2) FLLM_GATED_VEC(2, X);         \
+        else if (pieces <= 4) FLLM_GATED_VEC(4, X);    \
+        else FLLM_GATED_VEC(8, X);                     \
+    } while (0)
+        const int pieces = (width / 4 + kBlock - 1) / kBlock;
+        if (x_dtype == FLLM_F32) FLLM_GATED_ROW(float);
+        else if (x_dtype == FLLM_BF16) FLLM_GATED_ROW(bf16_t);
+        else FLLM_REQUIRE(false, "gated_norm: unknown dtypes %d, %d", x_dtype, dtype);
+#undef FLLM_GATED_ROW
+#undef FLLM_GATED_VEC
+        return fllm_check_launch("gated_norm");
+    }
 #define FLLM_GATED(X, T) hipLaunchKernelGGL((gated_norm_kernel<X, T>), dim3(rows), dim3(kBlock), 0, stream, (const X *)x, w, eps, \
                                             (const T *)gate, gate_ld, (T *)out, width)
     if (x_dtype == FLLM_F32 && dtype == FLLM_F32) FLLM_GATED(float, float);
@@ -501,6 +625,14 @@ extern "C" int fllm_polynorm(const void *z, int ld, const float *coeffs, float e
     FLLM_REQUIRE(rows >= 0 && width > 0 && ld >= width, "polynorm: bad sizes");
     FLLM_REQUIRE(z && coeffs && out, "polynorm: operands missing");
     if (rows == 0) return 0;
+    if (dtype == FLLM_BF16 && width % 8 == 0 && ld % 8 == 0 && width <= 4 * 8 * kPolyBlock && (((uintptr_t)z | (uintptr_t)out) & 15) == 0) {
+#define FLLM_POLY(NV) hipLaunchKernelGGL((polynorm_vec_kernel<NV>), dim3(rows), dim3(kPolyBlock), 0, stream, (const bf16_t *)z, ld, coeffs, eps, \
+                                         (bf16_t *)out, width)
+        if (width <= 2 * 8 * kPolyBlock) FLLM_POLY(2);
+        else FLLM_POLY(4);
+#undef FLLM_POLY
+        return fllm_check_launch("polynorm");
+    }
     if (dtype == FLLM_F32)
         hipLaunchKernelGGL(polynorm_kernel<float>, dim3(rows), dim3(kBlock), 0, stream, (const float *)z, ld, coeffs, eps, (float *)out, width);
     else if (dtype == FLLM_BF16)

@@ -23,6 +23,13 @@ int fllm_talking_attention_bf16_fast(const void *q, const void *gate, int gate_s
                                      int key_chunk, int max_context, int splits, float *ws, size_t ws_floats, int single_rows,
                                      hipStream_t stream);   // talking_attention_mfma.hip; 1: declined
 
+int fllm_launch_normed_rope_store(const void *qkv, int ld, int norm_mode, const float *q_weight, const float *k_weight, float eps,
+                                  void *q_out, const int32_t *row_pos, const int32_t *row_seg, const int32_t *tables,
+                                  int table_stride, const float *cos_table, const float *sin_table, int table_positions,
+                                  void *k_pages, void *v_pages, int rows, int heads, int kv_heads, int k_dim, int v_dim,
+                                  int rope_dims, int page_size, int key_chunk, int dtype, int store_kv, int values_from_keys,
+                                  const void *blend, int blend_ld, const float *blend_amount, hipStream_t stream);   // mixer_variants.hip
+
 namespace {
 
 constexpr int kBlock = 256;
@@ -32,54 +39,6 @@ constexpr int kMaxOut = 16;   // heads * v_dim <= kBlock * kMaxOut
 // [page][kv_head][k_dim / c][token][c]: c = 8 is key_offset() of common.h, c = 1 keys transposed like the values
 __device__ __forceinline__ size_t key_at(size_t page, int kv_heads, int kvh, int page_size, int k_dim, int token, int d, int c) {
     return ((((size_t)page * kv_heads + kvh) * (k_dim / c) + d / c) * page_size + token) * c + d % c;
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock)
-qk_norm_rope_store_kernel(const T *__restrict__ qkv, int ld, const float *__restrict__ q_weight, const float *__restrict__ k_weight,
-                          float eps, T *__restrict__ q_out, const int32_t *__restrict__ row_pos, const int32_t *__restrict__ row_seg,
-                          const int32_t *__restrict__ tables, int table_stride, const float *__restrict__ cos_table,
-                          const float *__restrict__ sin_table, T *__restrict__ k_pages, T *__restrict__ v_pages, int heads,
-                          int kv_heads, int k_dim, int v_dim, int rope_dims, int page_size, int key_chunk, int store_kv) {
-    __shared__ float scratch[kWaves];
-    const size_t r = blockIdx.x;
-    const int seg = row_seg[r];
-    if (seg < 0) return;   // padding row: its queries are never read
-    const int pos = row_pos[r];
-    const int nq = heads * k_dim, nk = kv_heads * k_dim, nv = kv_heads * v_dim;
-    const T *q = qkv + r * ld, *k = q + nq, *v = k + nk;
-    // asked for before the sums, so that the lookup waits beside them and not behind them
-    const int page = store_kv ? tables[(size_t)seg * table_stride + pos / page_size] : 0, off = pos % page_size;
-    float sq = 0.f, sk = 0.f;
-    for (int c = threadIdx.x; c < nq; c += kBlock) { const float a = to_f32<T>(q[c]); sq += a * a; }
-    for (int c = threadIdx.x; c < nk; c += kBlock) { const float a = to_f32<T>(k[c]); sk += a * a; }
-    sq = block_sum<kWaves>(sq, scratch);
-    sk = block_sum<kWaves>(sk, scratch);
-    const float inv_q = 1.0f / sqrtf(sq / (float)nq + eps), inv_k = 1.0f / sqrtf(sk / (float)nk + eps);
-    const int half = rope_dims / 2;
-    const float *cs = cos_table + (size_t)pos * half, *sn = sin_table + (size_t)pos * half;
-    for (int idx = threadIdx.x; idx < nq + (store_kv ? nk : 0); idx += kBlock) {
-        const bool is_q = idx < nq;
-        const int e = is_q ? idx : idx - nq;
-        const T *src = is_q ? q : k;
-        const float *w = is_q ? q_weight : k_weight;
-        const float inv = is_q ? inv_q : inv_k;
-        const int h = e / k_dim, c = e - h * k_dim;
-        float val = to_f32<T>(src[e]) * inv * w[e];
-        if (c < rope_dims) {
-            const int i = c < half ? c : c - half;
-            const int pe = c < half ? e + half : e - half;
-            const float other = to_f32<T>(src[pe]) * inv * w[pe];
-            val = c < half ? val * cs[i] - other * sn[i] : val * cs[i] + other * sn[i];
-        }
-        if (is_q) q_out[r * nq + e] = from_f32<T>(val);
-        else k_pages[key_at(page, kv_heads, h, page_size, k_dim, off, c, key_chunk)] = from_f32<T>(val);
-    }
-    if (!store_kv) return;
-    for (int e = threadIdx.x; e < nv; e += kBlock) {
-        const int h = e / v_dim, c = e - h * v_dim;
-        v_pages[(((size_t)page * kv_heads + h) * v_dim + c) * page_size + off] = v[e];
-    }
 }
 
 template <typename T>
@@ -213,19 +172,10 @@ extern "C" int fllm_qk_norm_rope_store(const void *qkv, int ld, const float *q_w
     FLLM_REQUIRE(key_chunk > 0 && k_dim % key_chunk == 0, "qk_norm_rope_store: keys of %d values in chunks of %d", k_dim, key_chunk);
     FLLM_REQUIRE(!store_kv || (k_pages && v_pages), "qk_norm_rope_store: pages missing");
     FLLM_REQUIRE(q_weight && k_weight && q_out, "qk_norm_rope_store: operands missing");
-    if (rows == 0) return 0;
-    if (dtype == FLLM_F32)
-        hipLaunchKernelGGL(qk_norm_rope_store_kernel<float>, dim3(rows), dim3(kBlock), 0, stream, (const float *)qkv, ld, q_weight,
-                           k_weight, eps, (float *)q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table,
-                           (float *)k_pages, (float *)v_pages, heads, kv_heads, k_dim, v_dim, rope_dims, page_size, key_chunk, store_kv);
-    else if (dtype == FLLM_BF16)
-        hipLaunchKernelGGL(qk_norm_rope_store_kernel<bf16_t>, dim3(rows), dim3(kBlock), 0, stream, (const bf16_t *)qkv, ld, q_weight,
-                           k_weight, eps, (bf16_t *)q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table,
-                           (bf16_t *)k_pages, (bf16_t *)v_pages, heads, kv_heads, k_dim, v_dim, rope_dims, page_size, key_chunk,
-                           store_kv);
-    else
-        FLLM_REQUIRE(false, "qk_norm_rope_store: unknown dtype %d", dtype);
-    return fllm_check_launch("qk_norm_rope_store");
+    // the norms over whole projections, the rotation and the store are those of normed_rope_store
+    return fllm_launch_normed_rope_store(qkv, ld, 2, q_weight, k_weight, eps, q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table,
+                                  table_positions, k_pages, v_pages, rows, heads, kv_heads, k_dim, v_dim, rope_dims, page_size, key_chunk,
+                                  dtype, store_kv, 0, nullptr, 0, nullptr, stream);
 }
 
 extern "C" int fllm_talking_attention(const void *q, const void *gate, int gate_stride, const void *k_pages, const void *v_pages,
