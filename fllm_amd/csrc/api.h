@@ -445,6 +445,13 @@ int fllm_experts_grouped_ungated(const void *h, int ldh, const int32_t *ids, int
                                  int E, int inter, int K, int N, void *act, float *out, int32_t *work, float *planes,
                                  hipStream_t stream);
 
+// Products of many bfloat16 rows on 256- and 128-row tiles (gemm_tiles.h).  0: launched, 1: declined (sizes that are no multiples of the
+// tiles' pieces, or with `force` 0 shapes that the general path is faster at).
+int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up, void *out, int M, int inter, int K, float limit, float alpha,
+                       float up_offset, int force, hipStream_t stream);
+int fllm_linear_tiles(const void *x, int ldx, const void *w, const float *bias, void *out, int ldo, int M, int N, int K, int mode, int force,
+                      hipStream_t stream);
+
 // The same for steps of few pairs (decode): the picked experts' matrices stream once, no scratch but act (bfloat16 [rows * top, inter]).
 // gated 1: w_up the tile-major copy (fllm_tile_weights) of [E * 2 inter][K], gate rows then up rows of an expert; gated 0: that of
 // [E * inter][K], relu(.)^2, weights null.  w_down that of [E * N][inter]; out float32 [rows * top, N].  1: shape declined (more than

@@ -1,7 +1,8 @@
 // bfloat16 matrix products y = x w^T on the MFMA units of gfx950, float32 accumulation.
 //
 // Calls of up to 64 rows (decode steps) go to the weight-streaming kernel of linear_skinny.hip.
-// `tiled` (M > 64, prompt portions) is a 128x128x64 LDS-tiled kernel, four waves of 64x64 each on
+// Stored products of more rows whose sizes fit go to linear_tiles.hip.
+// `tiled` (the others, M > 64) is a 128x128x64 LDS-tiled kernel, four waves of 64x64 each on
 // v_mfma_f32_32x32x16_bf16, with register prefetch of the next tile.
 //
 // MFMA operand layouts used here (wave64):
@@ -130,6 +131,10 @@ int fllm_linear_bf16_fast(const void *x, int ldx, const void *w, const float *bi
     const bf16_t *xb = (const bf16_t *)x, *wb = (const bf16_t *)w;
     if (M <= 64) {
         const int rc = fllm_linear_bf16_skinny(x, ldx, w, bias, out, ldo, M, N, K, out_mode, stream);
+        if (rc != 1) return rc;
+    }
+    if (out_mode == 0) {      // whole pieces of the larger tiles (2,048 rows, 2,048 x 1,536 with a bias: 34 -> 24 us)
+        const int rc = fllm_linear_tiles(x, ldx, w, bias, out, ldo, M, N, K, 0, 1, stream);
         if (rc != 1) return rc;
     }
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;

@@ -1,0 +1,69 @@
+// Products of many bfloat16 rows on the tiles of gemm_tiles.h: gate and up with the activation in the epilogue, the squared ReLU, and plain
+// products (with a bias, or where their tiles fill the device).
+#include "api.h"
+#include "gemm_tiles.h"
+
+using namespace fllm_tiles;
+
+namespace {
+
+bool operands_fit(const void *x, int ldx, const void *w, const void *out, int ldo, int M, long w_rows, int N, int K) {
+    return ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0) && ldx % 8 == 0 && ldo % 8 == 0 && N % 8 == 0 &&
+           (uint64_t)M * ldx * 2 < (1ull << 32) && (uint64_t)w_rows * K * 2 < (1ull << 32);      // byte offsets of 32 bits
+}
+
+TileArgs tile_args(const void *x, int ldx, const void *w, void *out, int ldo, int M, int N, int K) {
+    TileArgs a = {};
+    a.x = (const bf16_t *)x, a.w = (const bf16_t *)w, a.out = out;
+    a.ldx = ldx, a.ldo = ldo, a.M = M, a.N = N, a.K = K;
+    return a;
+}
+long tiles_of(long M, int bm, int N, int cols) { return (M + bm - 1) / bm * ((N + cols - 1) / cols); }
+
+}  // namespace
+
+// 0: launched, negative: error, 1: declined (the shape, or with `force` 0 a shape that the general path is faster at; 256 or 128 forces
+// that row tile).
+//
+// The fused product against the library's product and an activation kernel, microseconds at 136 / 512 / 1,024 / 2,048 rows: 2 x 14,336 x
+// 4,096 62 -> 65 / 106 -> 95 / 203 -> 183 / 378 -> 356; 2 x 8,192 x 2,048 26 -> 27 / 41 -> 32 / 65 -> 54 / 120 -> 106; 2 x 8,960 x 1,536
+// 26 -> 23 / 42 -> 36 / 75 -> 67 / 132 -> 115; 2 x 4,096 x 1,024 26 -> 17 / 26 -> 17 / 29 -> 20 / 42 -> 35.
+extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up, void *out, int M, int inter, int K, float limit, float alpha,
+                                  float up_offset, int force, hipStream_t stream) {
+    FLLM_REQUIRE(M >= 0 && inter > 0 && K > 0 && ldx >= K && x && w_gate_up && out, "gate_up_tiles: bad sizes or operands missing");
+    if (!fllm_fast_kernels_enabled() || !operands_fit(x, ldx, w_gate_up, out, inter, M, 2L * inter, inter, K)) return 1;
+    if (M == 0) return 0;
+    const long t256 = tiles_of(M, 256, inter, 128), t128 = tiles_of(M, 128, inter, 128);
+    int bm = row_tile(t256, t128, K);
+    if (force > 1) bm = force;
+    if (bm == 0) return 1;
+    TileArgs a = tile_args(x, ldx, w_gate_up, out, inter, M, inter, K);
+    a.limit = limit, a.alpha = alpha, a.up_offset = up_offset;
+    return launch_tiles<EPI_GLU, false>(a, bm, bm == 256 ? t256 : t128, stream);
+}
+
+// mode 0: out bfloat16 = x w^T (+ bias); 1: out float32 = x w^T; 2: out bfloat16 = relu(x w^T)^2.
+//
+// The squared ReLU against the library's product and a kernel of its own (13,312 x 1,536): 26 -> 20 us at 136 rows, 31 -> 23 at 512, 87 -> 68
+// at 2,048.  A bias (2,048 x 1,536; the general path is linear_tiled_mfma_kernel): 32 -> 23 us at 136 rows, 34 -> 24 at 2,048.  Without either
+// the library has kernels for every tile of the device's time, and these tiles are ahead only where they fill whole rounds over the compute
+// units: 4,096 x 14,336 at 2,048 rows (256 tiles) 207 -> 188 us, at 1,900 (240) 191 -> 182, at 1,536 (192) 167 -> 177; 4,096 x 4,096 at
+// 2,048 rows 59 -> 55; 6,144 x 4,096 at 2,048 rows (192 of 256 rows) 80 -> 77, at 1,900 76 -> 78.  Hence nine tenths of the last round.
+extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const float *bias, void *out, int ldo, int M, int N, int K, int mode,
+                                 int force, hipStream_t stream) {
+    FLLM_REQUIRE(M >= 0 && N > 0 && K > 0 && ldx >= K && ldo >= N && x && w && out && mode >= 0 && mode <= 2,
+                 "linear_tiles: bad sizes or operands missing");
+    if (!fllm_fast_kernels_enabled() || (bias && mode != 0) || !operands_fit(x, ldx, w, out, ldo, M, N, N, K)) return 1;
+    if (M == 0) return 0;
+    const long t256 = tiles_of(M, 256, N, 256), t128 = tiles_of(M, 128, N, 256);
+    int bm = row_tile(t256, t128, K);
+    if (force > 1) bm = force;
+    if (bm == 0) return 1;
+    TileArgs a = tile_args(x, ldx, w, out, ldo, M, N, K);
+    a.bias = bias;
+    const long tiles = bm == 256 ? t256 : t128, slots = (tiles + 255) / 256 * 256;
+    if (!force && mode != 2 && !bias && (K < 2048 || 10 * tiles < 9 * slots)) return 1;
+    if (mode == 0) return launch_tiles<EPI_STORE, false>(a, bm, tiles, stream);
+    if (mode == 1) return launch_tiles<EPI_F32, false>(a, bm, tiles, stream);
+    return launch_tiles<EPI_RELU2, false>(a, bm, tiles, stream);
+}

@@ -1,6 +1,6 @@
 // Routed experts on the matrix cores (bfloat16, prompt portions): the (row, pick) pairs of a step are grouped by expert on
-// the device, and every expert multiplies the rows that picked it as tiles of 64 or 128 rows, so that its matrices are read
-// once a row tile instead of once a row.  Three launches: grouping, gate/up with the activation, down.  A pair's result does not
+// the device, and every expert multiplies the rows that picked it as tiles of 64 or 128 rows (steps of many pairs an expert: of 128 or
+// 256, gemm_tiles.h), so that its matrices are read once a row tile instead of once a row.  Three launches: grouping, gate/up with the activation, down.  A pair's result does not
 // depend on which rows share its tile (a row of a matrix-core product is a sum over K in an order of its own).
 //
 // MFMA operand layout used here (wave64, v_mfma_f32_32x32x16_bf16): A lane l holds A[m = l%32][k = 8*(l/32) .. +7]; B
@@ -9,11 +9,17 @@
 
 #include "api.h"
 #include "common.h"
+#include "gemm_tiles.h"
 
 namespace {
 
 constexpr int GK = 64, LDT = GK + 8;
 constexpr int kThreads = 256;
+// Pairs an expert on average from which the tiles of gemm_tiles.h serve.  Microseconds of both products with what they need around them, 8
+// experts of 4,480 lanes at a width of 1,536 (tiles here -> those), two picks a row: 200 rows 111 -> 132, 256 rows 138 -> 135, 384 rows 152 ->
+// 144, 512 rows 186 -> 147, 1,024 rows 239 -> 170, 2,048 rows 332 -> 245; without a gate 384 rows 128 -> 103, 2,048 rows 223 -> 157; 2,048
+// lanes at 1,024: 256 rows 50 -> 59, 384 rows 76 -> 65, 2,048 rows 137 -> 106.
+constexpr int kLargeTilePairs = 96;
 
 __device__ __forceinline__ bf16x8_t zero8() {
     bf16x8_t z;
@@ -235,6 +241,42 @@ int down_slices(long pairs, int E, int N, int inter) {
     return (int)std::max(1L, std::min(16L, std::min(want, most)));
 }
 
+// The row tile of gemm_tiles.h for both products of a step's pairs, 0 where the tiles above serve: steps of few pairs an expert, sizes that are
+// no whole pieces.  Of 256 and 128 the one whose two products take fewer rounds over the compute units, weighted with their K; how many
+// row tiles the experts fill is known on the device alone, so half a tile an expert is assumed on top of the pairs.
+int large_row_tile(long pairs, int E, int inter, int K, int N, int up_columns, const void *x, int ldx, long x_rows, const void *out) {
+    using namespace fllm_tiles;
+    if (pairs / E < kLargeTilePairs || K % 128 != 0 || inter % 128 != 0 || K < 256 || inter < 256 || N % 8 != 0) return 0;
+    if ((((uintptr_t)x | (uintptr_t)out) & 15) != 0 || ldx % 8 != 0) return 0;
+    const uint64_t most = 1ull << 32;      // byte offsets of 32 bits
+    if ((uint64_t)x_rows * ldx * 2 >= most || (uint64_t)pairs * inter * 2 >= most || (uint64_t)2 * inter * K * 2 >= most || (uint64_t)N * inter * 2 >= most)
+        return 0;
+    auto cost = [&](int bm) {
+        const long rows = (pairs + (long)E * bm / 2) / bm;
+        const long up = (rows * ((inter + up_columns - 1) / up_columns) + 255) / 256, down = (rows * ((N + 255) / 256) + 255) / 256;
+        return (double)up * K + (double)down * inter;
+    };
+    return cost(256) <= kShortRound * cost(128) ? 256 : 128;
+}
+
+// Both products on those tiles, behind group_pairs_kernel and (where the picks' weights scale the rows) scaled_rows_kernel.
+template <int UP>
+int launch_large(int bm, const void *x, int ldx, int top, const void *w_up, const void *w_down, int E, int inter, int K, int N, long pairs, void *act,
+                 float *out, const int32_t *work, long max_tiles, float limit, float alpha, float up_offset, hipStream_t stream) {
+    using namespace fllm_tiles;
+    TileArgs a = {};
+    a.x = (const bf16_t *)x, a.w = (const bf16_t *)w_up, a.out = act;
+    a.ldx = ldx, a.ldo = inter, a.M = (int)pairs, a.N = inter, a.K = K;
+    a.limit = limit, a.alpha = alpha, a.up_offset = up_offset;
+    a.work = work, a.max_tiles = (int)max_tiles, a.top = top;
+    const int columns = UP == EPI_GLU ? 128 : 256;
+    int rc = launch_tiles<UP, true>(a, bm, max_tiles * ((inter + columns - 1) / columns), stream);
+    if (rc != 0) return rc;
+    a.x = (const bf16_t *)act, a.w = (const bf16_t *)w_down, a.out = out;
+    a.ldx = inter, a.ldo = N, a.N = N, a.K = inter, a.top = -1;
+    return launch_tiles<EPI_F32, true>(a, bm, max_tiles * ((N + 255) / 256), stream);
+}
+
 }  // namespace
 
 // floats of scratch that fllm_experts_grouped needs for the planes of a down product cut along K (0: it is not cut)
@@ -262,8 +304,10 @@ extern "C" int fllm_experts_grouped(const void *h, int ldh, const int32_t *ids, 
     if ((((uintptr_t)h | (uintptr_t)w_gate_up | (uintptr_t)w_down | (uintptr_t)act | (uintptr_t)xs) & 15) != 0) return 1;
     const long pairs = (long)rows * top;
     if (pairs == 0) return 0;
+    const bool scaled = weights != nullptr;
+    const int large = large_row_tile(pairs, E, inter, K, N, 128, scaled ? xs : h, scaled ? K : ldh, scaled ? pairs : rows, out);
     // row tiles of 128 pairs where the experts' shares are large enough to fill them
-    const int GM = pairs / E >= 96 ? 128 : 64;
+    const int GM = large ? large : (pairs / E >= 96 ? 128 : 64);
     const long max_tiles = (pairs + GM - 1) / GM + E;
     // column tiles of 64 for the down product where 128 would give the device fewer workgroups than compute units, and
     // K slices where that is still too few (decode steps)
@@ -274,12 +318,14 @@ extern "C" int fllm_experts_grouped(const void *h, int ldh, const int32_t *ids, 
     const long up_tiles = (inter + 63) / 64, down_tiles = (N + GN_DOWN - 1) / GN_DOWN;
     if (pairs > (1L << 24) || max_tiles * up_tiles > 0x7fffffffL || max_tiles * down_tiles > 0x7fffffffL) return 1;
     hipLaunchKernelGGL(group_pairs_kernel, dim3(1), dim3(1024), (size_t)3 * E * sizeof(int), stream, ids, (int)pairs, E, (int)max_tiles, GM, work);
-    const bool scaled = weights != nullptr;
     if (scaled)
         hipLaunchKernelGGL(scaled_rows_kernel, dim3((unsigned)pairs), dim3(256), 0, stream, (const bf16_t *)h, ldh, weights, top,
                            work + 1 + 3 * max_tiles, (bf16_t *)xs, K);
     const void *up_in = scaled ? xs : h;
     const int up_ld = scaled ? K : ldh;
+    if (large)
+        return launch_large<fllm_tiles::EPI_GLU>(large, up_in, up_ld, scaled ? 0 : top, w_gate_up, w_down, E, inter, K, N, pairs, act, out, work,
+                                                 max_tiles, limit, alpha, up_offset, stream);
     float *down_out = slices > 1 ? planes : out;
 #define FLLM_GROUPED(MODE, ROWS, COLS, X, LDX, W, NN, KK)                                                                                  \
     hipLaunchKernelGGL((grouped_tiles_kernel<MODE, ROWS, COLS>),                                                                           \
@@ -312,7 +358,8 @@ extern "C" int fllm_experts_grouped_ungated(const void *h, int ldh, const int32_
     if ((((uintptr_t)h | (uintptr_t)w_up | (uintptr_t)w_down | (uintptr_t)act) & 15) != 0) return 1;
     const long pairs = (long)rows * top;
     if (pairs == 0) return 0;
-    const int GM = pairs / E >= 96 ? 128 : 64;
+    const int large = large_row_tile(pairs, E, inter, K, N, 256, h, ldh, rows, out);
+    const int GM = large ? large : (pairs / E >= 96 ? 128 : 64);
     const long max_tiles = (pairs + GM - 1) / GM + E;
     const int GN_UP = max_tiles * ((inter + 127) / 128) < 256 ? 64 : 128;
     const int GN_DOWN = max_tiles * ((N + 127) / 128) < 256 ? 64 : 128;
@@ -322,6 +369,9 @@ extern "C" int fllm_experts_grouped_ungated(const void *h, int ldh, const int32_
     const long up_tiles = (inter + GN_UP - 1) / GN_UP, down_tiles = (N + GN_DOWN - 1) / GN_DOWN;
     if (pairs > (1L << 24) || max_tiles * up_tiles > 0x7fffffffL || max_tiles * down_tiles > 0x7fffffffL) return 1;
     hipLaunchKernelGGL(group_pairs_kernel, dim3(1), dim3(1024), (size_t)3 * E * sizeof(int), stream, ids, (int)pairs, E, (int)max_tiles, GM, work);
+    if (large)
+        return launch_large<fllm_tiles::EPI_RELU2>(large, h, ldh, top, w_up, w_down, E, inter, K, N, pairs, act, out, work, max_tiles, 0.f, 0.f, 0.f,
+                                                   stream);
     float *down_out = slices > 1 ? planes : out;
 #define FLLM_UNGATED(MODE, ROWS, COLS, X, LDX, W, NN, KK, TILES, SLICES, KPER)                                                          \
     hipLaunchKernelGGL((grouped_tiles_kernel<MODE, ROWS, COLS>), dim3((unsigned)(max_tiles * (TILES)), SLICES), dim3(kThreads), 0, stream, \

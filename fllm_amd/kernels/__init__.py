@@ -182,6 +182,8 @@ def load_library(build_if_missing: bool = True):
         "fllm_relu_squared": [c_void, c_void, c_size, c_int, c_void],
         "fllm_route_grouped": [c_void, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_int, c_void, c_void, c_float, c_int,
                                c_void],
+        "fllm_gate_up_tiles": [c_void, c_int, c_void, c_void, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_void],
+        "fllm_linear_tiles": [c_void, c_int, c_void, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_int, c_void],
         "fllm_experts_stream": [c_void, c_int, c_void, c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_void,
                                 c_void, c_float, c_float, c_float, c_void],
         "fllm_experts_grouped_ungated": [c_void, c_int, c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_void, c_void,
@@ -443,6 +445,9 @@ class Ops:
             return out
         if (self.library_gemm_from is not None and M >= self.library_gemm_from and x.dtype == torch.bfloat16
                 and bias is None):
+            if mode == OUT_STORE and M > 64 and self._tiles_take(self.lib.fllm_linear_tiles(
+                    _ptr(x), ldx, _ptr(w), None, _ptr(out), ldo, M, N, K, 0, 0, self._stream())):
+                return out
             if mode == OUT_STORE:
                 torch.matmul(x, w.t(), out=out)
             elif mode == OUT_STORE_F32:
@@ -453,6 +458,39 @@ class Ops:
         self._check(self.lib.fllm_linear(_ptr(x), ldx, _ptr(w), _ptr(bias), _ptr(out), ldo, M, N, K, _DTYPE_CODE[x.dtype],
                                          mode, self._stream()))
         return out
+
+    # ---- products of many rows with the activation in the epilogue ---------------------------------
+    def _tiles_take(self, code: int) -> bool:
+        if code == 1:
+            return False
+        self._check(code)
+        return True
+
+    def gate_up_tiles(self, x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, limit: float = 0.0, alpha: float = 1.0,
+                      up_offset: float = 0.0) -> bool:
+        """out = a(g) * (u + up_offset), g and u the two halves of x @ w_gate_up.T, the activation as in `glu_clamped` (the defaults are
+        SwiGLU), for steps of more than 64 bfloat16 rows; out bfloat16 [M, I].  False: not taken (few rows, the GEMM library switched off,
+        sizes that are no multiples of the tiles' pieces), nothing was written."""
+        M, K = x.shape
+        two_i = w_gate_up.shape[0]
+        if M <= 64 or x.dtype != torch.bfloat16 or not x.is_cuda or self.library_gemm_from is None or M < self.library_gemm_from:
+            return False
+        _need(x.stride(1) == 1 and two_i % 2 == 0, "x must be row-major and w_gate_up have an even number of rows")
+        _dense(w_gate_up, "w_gate_up", torch.bfloat16, (two_i, K))
+        _dense(out, "out", torch.bfloat16, (M, two_i // 2))
+        return self._tiles_take(self.lib.fllm_gate_up_tiles(_ptr(x), x.stride(0), _ptr(w_gate_up), _ptr(out), M, two_i // 2, K, float(limit),
+                                                            float(alpha), float(up_offset), 0, self._stream()))
+
+    def relu_squared_tiles(self, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+        """out = relu(x @ w.T)^2 likewise."""
+        M, K = x.shape
+        N = w.shape[0]
+        if M <= 64 or x.dtype != torch.bfloat16 or not x.is_cuda or self.library_gemm_from is None or M < self.library_gemm_from:
+            return False
+        _need(x.stride(1) == 1, "x must be row-major")
+        _dense(w, "w", torch.bfloat16, (N, K))
+        _dense(out, "out", torch.bfloat16, (M, N))
+        return self._tiles_take(self.lib.fllm_linear_tiles(_ptr(x), x.stride(0), _ptr(w), None, _ptr(out), N, M, N, K, 2, 0, self._stream()))
 
     # ---- fused forms of decode steps (bfloat16, at most 64 rows) ---------------------------------
     def fused_decode_supported(self, rows: int, width: int) -> bool:

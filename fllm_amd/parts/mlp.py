@@ -9,6 +9,12 @@ from ..registry import register_part
 from .base import INIT_BIAS, INIT_MATRIX, INIT_NORM, FeedForward, add_and_prepare, fused_form, take_prepared
 
 
+def activated_tiles(ops, form: str, bias, *operands) -> bool:
+    """Prompt-sized steps: the kernel library's product with the activation in its epilogue, where it has one that takes these rows."""
+    take = getattr(ops, form, None) if bias is None else None
+    return take is not None and take(*operands)
+
+
 class GatedMLP(FeedForward):
     graph_safe = True      # forward launches kernels only: no per-step decision on the host
 
@@ -77,7 +83,7 @@ class GatedMLP(FeedForward):
         if (getattr(ops, "prefers_own_gate_up", None) is not None and ops.prefers_own_gate_up(rows, self.w_gate_up)
                 and self.hidden % 8 == 0 and h.stride(0) % 8 == 0):
             ops.gate_up_swiglu(h, self.w_gate_up, act, bias=self.b_gate_up)     # the activation as the product's epilogue
-        else:
+        elif not activated_tiles(ops, "gate_up_tiles", self.b_gate_up, h, self.w_gate_up, act):
             gate_up = rt.empty((rows, 2 * self.inter))
             ops.linear(h, self.w_gate_up, gate_up, bias=self.b_gate_up)
             ops.swiglu(gate_up, act)
@@ -96,10 +102,11 @@ class GatedMLP(FeedForward):
             ops.gate_up_swiglu(h, self.w_gate_up, act, bias=self.b_gate_up)
             ops.linear(act, self.w_down, residual, bias=self.b_down, accumulate=True)
             return
-        gate_up = rt.empty((rows, 2 * self.inter))
-        ops.linear(h, self.w_gate_up, gate_up, bias=self.b_gate_up)
         act = rt.empty((rows, self.inter))
-        ops.swiglu(gate_up, act)
+        if not activated_tiles(ops, "gate_up_tiles", self.b_gate_up, h, self.w_gate_up, act):
+            gate_up = rt.empty((rows, 2 * self.inter))
+            ops.linear(h, self.w_gate_up, gate_up, bias=self.b_gate_up)
+            ops.swiglu(gate_up, act)
         ops.linear(act, self.w_down, residual, bias=self.b_down, accumulate=True)
 
 
@@ -165,7 +172,7 @@ class ClampedGLU(FeedForward):
                      or (rows <= getattr(ops, "GATE_UP_SWIGLU_ROWS", 0) and (start is None or rows < start)))):
             # steps that the hand-written products serve: the activation is the epilogue of the gate/up product
             ops.gate_up_glu(h, self.w_gate_up, act, self.limit, self.alpha, self.up_offset)
-        else:
+        elif not activated_tiles(ops, "gate_up_tiles", None, h, self.w_gate_up, act, self.limit, self.alpha, self.up_offset):
             gate_up = rt.empty((rows, 2 * self.inter))
             ops.linear(h, self.w_gate_up, gate_up)
             ops.glu_clamped(gate_up, act, self.limit, self.alpha, self.up_offset)
@@ -248,7 +255,7 @@ class SquaredReLUMLP(FeedForward):
         rt, ops = self.rt, self.rt.ops
         act = rt.empty((h.shape[0], self.inter))
         fused = getattr(ops, "linear_relu_squared", None)          # the activation as the product's epilogue: decode-sized steps
-        if fused is None or not fused(h, self.w_up, act):
+        if (fused is None or not fused(h, self.w_up, act)) and not activated_tiles(ops, "relu_squared_tiles", None, h, self.w_up, act):
             ops.linear(h, self.w_up, act)
             ops.activation(act, act, "relu2")
         if branch is not None:
