@@ -612,18 +612,59 @@ attn_tile32_kernel(AttnArgs p) {
 // ---------------------------------------------------------------------------------------------
 // decode kernel
 // ---------------------------------------------------------------------------------------------
-// A decode step reads the keys and values of a request once, so these loads carry the non-temporal hint (a step of
-// the 8B sizes at batch 8: 4.75 -> 4.62 ms at contexts of 8,192, 8.88 -> 8.34 ms at 32,768; 6.20 -> 6.02 ms at batch 64).
+// A decode step reads the keys of a request once and a load takes whole lines of them, so it carries the non-temporal hint.
+// So do the values in pages of up to 16 tokens, whose rows follow each other.  In larger pages they go without: a load takes
+// 64 bytes of each of 16 rows and the next one the other half of the same lines, and with the hint the second asks memory
+// again (64 rows of 1,024 keys at the 8B sizes in pages of 64: both with the hint 62 us, both without 54, keys alone 45.5).
 #ifdef FLLM_CACHE_TEMPORAL
 #define FLLM_CACHE_LOAD(ptr) (*(ptr))
 #else
 #define FLLM_CACHE_LOAD(ptr) __builtin_nontemporal_load(ptr)
 #endif
-template <int D, int WAVES>
-__global__ void __launch_bounds__(WAVES * kWave)
+typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
+
+// P^T as the second product takes it.  A lane (c, g) has the scores of keys 16 j + 4 g + i of two tiles j and wants those of
+// keys 8 g .. 8 g + 7, so that the values it meets are eight neighbouring tokens, one 16-byte load: rows of 16 lanes change
+// places between the tiles (halves of the wave first, then the odd rows of the one with the even rows of the other).
+__device__ __forceinline__ bf16x8_t neighbours(bf16x8_t p) {
+    u32x4_t w = __builtin_bit_cast(u32x4_t, p);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const auto h = __builtin_amdgcn_permlane32_swap(w[i], w[2 + i], false, false);
+        const auto q = __builtin_amdgcn_permlane16_swap(h[0], h[1], false, false);
+        w[i] = q[0];
+        w[2 + i] = q[1];
+    }
+    return __builtin_bit_cast(bf16x8_t, w);
+}
+
+// Two neighbouring floats that pass between workgroups of a launch, as one 8-byte access at the device's point of coherence.
+typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+__device__ __forceinline__ void put2(float *to, float a, float b) {
+    const f32x2_t v = {a, b};
+    __hip_atomic_store((unsigned long long *)to, __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ f32x2_t get2(const float *from) {
+    return __builtin_bit_cast(f32x2_t, __hip_atomic_load((const unsigned long long *)from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+__device__ __forceinline__ void store2(bf16_t *to, float a, float b) {
+    to[0] = (bf16_t)a;
+    to[1] = (bf16_t)b;
+}
+
+// PM, what a page holds: 0: 8 tokens; 1: 16, a tile of keys; 2: 32 or more.
+// What bounds it: the bytes of keys and values, and in short contexts the trips to memory that follow each other.  A wave
+// has 64 keys and their values on their way at all times, asked for ahead of the softmax of the 64 before, page numbers
+// are scalar loads, and a value load is 16 bytes a lane.  At the 8B sizes in pages of 16 (of 64), against blocks of 32 keys
+// that were asked for and waited for in turn: eight rows of 1,024 keys 11.6 -> 11.0 us (14.4 -> 12.0), 40 rows of 48 to 800
+// 21.0 -> 18.6 (31.9 -> 22.5), four of 8,000 28.7 -> 24.5 (42.9 -> 25.9), 64 of 1,024 46.8 -> 43.8, 6.1 TB/s (70 -> 45.7).
+// Four waves of 64 keys (heads of 128: 227 registers) and not eight of 32: a second set of registers for the next block
+// spilled at 128, and 133 left a compute unit one workgroup of eight waves.
+template <int D, int WAVES, int PM>
+__global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(D >= 128 ? 2 : 3)))
 attn_decode_kernel(AttnArgs p, int qtiles) {
     constexpr int KD = D / 32, DT = D / 16;
-    constexpr int OP = D + 1;
+    constexpr int OP = D + 2;
     extern __shared__ float dsm[];   // sm_m[WAVES][16], sm_l[WAVES][16], sm_o[WAVES][gq][OP]
     const int row = blockIdx.x;
     const int qtile = blockIdx.y % qtiles, kvh = blockIdx.y / qtiles;
@@ -631,12 +672,11 @@ attn_decode_kernel(AttnArgs p, int qtiles) {
     const int G = p.heads / p.kv_heads;
     const int gq = min(G - qtile * 16, 16);   // query heads of this workgroup
     float *sm_m = dsm, *sm_l = dsm + WAVES * 16, *sm_o = dsm + 2 * WAVES * 16;
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int c = lane & 15, g = lane >> 4;
     const int hg = qtile * 16 + c;
     const int seg = p.row_seg[row];
-    const bool qvalid = hg < G && seg >= 0;
-    const int head = kvh * G + (hg < G ? hg : 0);
+    const int head = kvh * G + (hg < G ? hg : 0);        // lanes without a head of their own: computed, never stored
     const int n = seg >= 0 ? p.row_pos[row] + 1 : 0;
     const int lo = first_key(n - 1, p.window, p.chunk);
     const int ps = p.page_size, psh = p.ps_shift, pmask = ps - 1, nkv = p.kv_heads;
@@ -648,89 +688,134 @@ attn_decode_kernel(AttnArgs p, int qtiles) {
     if (p.counters && split >= live_splits) return;
     const int32_t *tbl = p.tables + (size_t)(seg >= 0 ? seg : 0) * p.table_stride;
 
-    bf16x8_t qf[KD];
+    // A wave takes 64 neighbouring keys at a time, two blocks of 32, each two score tiles of 16.  Row c of a tile at key t is
+    // key t + c, so that a load of the tile's keys (chunks 4 kk + g of 16 neighbouring tokens) is 1 KiB in a row where a page
+    // holds 16 tokens or more.  The values of a block are rows of V^T, eight neighbouring tokens a lane (`neighbours`): the
+    // two blocks together read whole lines where a page holds 64 tokens.
+    // The keys of the wave's next 64 are asked for as soon as these are multiplied, the values likewise, into the same
+    // registers.  Every lane loads, so that no load sits behind a branch: a block without keys loads its neighbour's again,
+    // a lane without a key of its own reads page 0.
+    typedef const __attribute__((address_space(4))) int32_t *constant_t;
+    const constant_t ctbl = (constant_t)(uintptr_t)tbl;      // a page that is the same for every lane: a scalar load
+    struct Pages {
+        int k[4], v[2];       // pages of 16 tokens or more: k for the values as well
+    };
+    auto tile_at = [&](int kb, int t) { return (kb + 32 * (t >> 1) < end ? kb + 32 * (t >> 1) : kb) + 16 * (t & 1); };
+    auto block_pages = [&](int kb) {      // kb may lie behind the last key: nothing is asked for there
+        Pages pg;
 #pragma unroll
-    for (int kk = 0; kk < KD; kk++)
-        qf[kk] = qvalid ? *(const bf16x8_t *)(p.q + (size_t)row * p.q_stride + (size_t)head * D + kk * 32 + g * 8) : zero8();
+        for (int t = 0; t < 4; t++) {
+            const int at = tile_at(kb, t);
+            if (PM == 2) {
+                pg.k[t] = at - 16 * (t & 1) < end ? ctbl[at >> psh] : 0;        // the block's: its values may be seen where this tile's keys are not
+            } else if (PM == 1) {
+                pg.k[t] = at < end && at + 16 > lo ? ctbl[at >> psh] : 0;
+            } else {
+                pg.k[t] = at + c >= lo && at + c < end ? tbl[(at + c) >> psh] : 0;
+                if ((t & 1) == 0) pg.v[t >> 1] = at + 8 * g < end && at + 8 * g + 8 > lo ? tbl[(at + 8 * g) >> psh] : 0;
+            }
+        }
+        return pg;
+    };
+    bf16x8_t kf[4][KD], vf[2][DT];
+    const size_t head_bytes = (size_t)(2 * D) * ps;         // of a page
+    auto load_keys = [&](int kb, const Pages &pg) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int at = tile_at(kb, t);
+            const char *page = (const char *)p.kp + ((size_t)pg.k[t] * nkv + kvh) * head_bytes + (PM > 0 ? (size_t)((at & pmask) * 16) : 0);
+            const unsigned int off = (unsigned int)((g * ps + (PM > 0 ? c : (at + c) & pmask)) * 16);
+#pragma unroll
+            for (int kk = 0; kk < KD; kk++) kf[t][kk] = FLLM_CACHE_LOAD((const bf16x8_t *)(page + (size_t)(kk * 64 * ps) + off));
+        }
+    };
+    auto load_values = [&](int kb, const Pages &pg) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int at = tile_at(kb, 2 * h);
+            const char *page = (const char *)p.vp + (size_t)kvh * head_bytes;
+            const size_t step = (size_t)nkv * head_bytes;
+            if (PM == 0) page += (size_t)pg.v[h] * step;
+            else if (PM == 1) page += g < 2 ? (size_t)pg.k[2 * h] * step : (size_t)pg.k[2 * h + 1] * step;
+            else page += (size_t)pg.k[2 * h] * step + (size_t)((at & pmask) * 2);
+            const unsigned int off = (unsigned int)((c * ps + (PM == 2 ? 8 * g : (at + 8 * g) & pmask)) * 2);
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++) {
+                const bf16x8_t *from = (const bf16x8_t *)(page + (size_t)(dt * 32 * ps) + off);
+                vf[h][dt] = PM == 2 ? *from : FLLM_CACHE_LOAD(from);
+            }
+        }
+    };
 
     f32x4_t o[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) o[dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
-
-    // A block is 32 keys: two score tiles of 16.  Row c of tile j is key kb + 16 j + c, so that a load of the tile's keys
-    // (chunks 4 kk + g of 16 neighbouring tokens) is 1 KiB in a row where a page holds 16 tokens or more.  Lane (c, g) then
-    // holds the scores of keys kb + 16 j + 4 g + i, i = 0..3, and takes exactly those eight keys' values as its operand
-    // of the second product: two runs of four neighbouring tokens of V^T, 8 bytes each.
-    // The page numbers of a block are asked for one block ahead, so that a block waits for one memory latency
-    // (its keys and values), not for two in a row.
-    auto block_pages = [&](int kb, int (&kpage)[2], int (&vpage)[2]) {
+    int kb = begin + wave * 64;
+    if (kb < end) {
+        bf16x8_t qf[KD];
+        Pages pg = block_pages(kb);
+        load_keys(kb, pg);
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int key = kb + 16 * j + c, vkey = kb + 16 * j + 4 * g;
-            kpage[j] = (kb < end && key < n && key >= lo) ? tbl[key >> psh] : 0;
-            vpage[j] = (kb < end && vkey < n && vkey + 4 > lo) ? tbl[vkey >> psh] : 0;
-        }
-    };
-    int kpage_next[2], vpage_next[2];
-    block_pages(begin + wave * 32, kpage_next, vpage_next);
-    for (int kb = begin + wave * 32; kb < end; kb += WAVES * 32) {
-        int kpage[2], vpage[2];
+        for (int kk = 0; kk < KD; kk++) qf[kk] = *(const bf16x8_t *)(p.q + (size_t)row * p.q_stride + (size_t)head * D + kk * 32 + g * 8);
+        __builtin_amdgcn_sched_barrier(0);       // loads come back in order: the scores do not wait for the values
+        load_values(kb, pg);
+        __builtin_amdgcn_sched_barrier(0);
+        pg = block_pages(kb + WAVES * 64);
+        f32x4_t s[4];
+        auto scores = [&]() {
 #pragma unroll
-        for (int j = 0; j < 2; j++) kpage[j] = kpage_next[j], vpage[j] = vpage_next[j];
-        block_pages(kb + WAVES * 32, kpage_next, vpage_next);
-        // All loads of the block are issued before the first product: one memory latency per block.
-        bf16x8_t kf[2][KD];
-        bf16x4_t vf[2][DT];
-        bool vtail[2];
+            for (int t = 0; t < 4; t++) {
+                s[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int key = kb + 16 * j + c;
-            const bool valid = key >= lo && key < n;
-            const bf16_t *kr = p.kp + key_offset(kpage[j], nkv, kvh, ps, D, key & pmask, g * 8);
-#pragma unroll
-            for (int kk = 0; kk < KD; kk++) kf[j][kk] = valid ? FLLM_CACHE_LOAD((const bf16x8_t *)(kr + (size_t)kk * 4 * ps * 8)) : zero8();
-            const int vkey = kb + 16 * j + 4 * g;
-            const bool vload = vkey < n && vkey + 4 > lo;
-            vtail[j] = vload && vkey + 4 > n;
-            const bf16_t *vr = p.vp + (((size_t)vpage[j] * nkv + kvh) * D + c) * ps + (vkey & pmask);
-#pragma unroll
-            for (int dt = 0; dt < DT; dt++) vf[j][dt] = vload ? FLLM_CACHE_LOAD((const bf16x4_t *)(vr + (size_t)dt * 16 * ps)) : (bf16x4_t){(bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f};
-        }
-
-        f32x4_t s[2];
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            s[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kk = 0; kk < KD; kk++) s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[j][kk], qf[kk], s[j], 0, 0, 0);
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int key = kb + 16 * j + 4 * g + i;
-                const bool vis = key >= lo && key < n;
-                s[j][i] = vis ? s[j][i] * p.scale_log2 : -INFINITY;
+                for (int kk = 0; kk < KD; kk++) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][kk], qf[kk], s[t], 0, 0, 0);
             }
-        float alpha;
-        softmax_step<2>(s, m_run, l_run, alpha);
-        const bf16x8_t pf = pack_p(s[0], s[1]);
+        };
+        auto add_values = [&]() {
+            if (kb >= lo && kb + 64 <= n && kb + 32 < end) {        // every key of both blocks is seen
 #pragma unroll
-        for (int dt = 0; dt < DT; dt++) {
-            bf16x8_t a;
+                for (int t = 0; t < 4; t++) s[t] *= p.scale_log2;
+            } else {
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+                for (int t = 0; t < 4; t++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    // slots past the last token hold whatever an earlier request left
-                    const bool past = vtail[j] && kb + 16 * j + 4 * g + e >= n;
-                    a[4 * j + e] = past ? (bf16_t)0.0f : vf[j][dt][e];
+                    for (int i = 0; i < 4; i++) {
+                        const int key = kb + 16 * t + 4 * g + i;
+                        s[t][i] = key >= lo && key < end ? s[t][i] * p.scale_log2 : -INFINITY;
+                    }
+                // slots past the last token and pages never asked for hold whatever an earlier request left
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int from = lo - (kb + 32 * h + 8 * g), to = end - (kb + 32 * h + 8 * g);      // the lane's tokens from .. to - 1 are seen
+                    u32x4_t keep;
+#pragma unroll
+                    for (int w = 0; w < 4; w++)
+                        keep[w] = (2 * w >= from && 2 * w < to ? 0x0000ffffu : 0u) | (2 * w + 1 >= from && 2 * w + 1 < to ? 0xffff0000u : 0u);
+#pragma unroll
+                    for (int dt = 0; dt < DT; dt++) vf[h][dt] = __builtin_bit_cast(bf16x8_t, __builtin_bit_cast(u32x4_t, vf[h][dt]) & keep);
                 }
-            o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pf, o[dt] * alpha, 0, 0, 0);
+            }
+            float alpha;
+            softmax_step<4>(s, m_run, l_run, alpha);
+            const bf16x8_t pf[2] = {neighbours(pack_p(s[0], s[1])), neighbours(pack_p(s[2], s[3]))};
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++) {
+                o[dt] *= alpha;
+#pragma unroll
+                for (int h = 0; h < 2; h++) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[h][dt], pf[h], o[dt], 0, 0, 0);
+            }
+        };
+        for (; kb + WAVES * 64 < end; kb += WAVES * 64) {
+            scores();
+            load_keys(kb + WAVES * 64, pg);
+            add_values();
+            load_values(kb + WAVES * 64, pg);
+            pg = block_pages(kb + 2 * WAVES * 64);
         }
+        scores();
+        add_values();
     }
-    // the waves saw different keys: merge their statistics and outputs
+    // the waves saw different keys: merge their statistics and outputs, two neighbouring outputs a thread
     if (g == 0) {
         sm_m[wave * 16 + c] = m_run;
         sm_l[wave * 16 + c] = l_run;
@@ -742,31 +827,32 @@ attn_decode_kernel(AttnArgs p, int qtiles) {
             for (int i = 0; i < 4; i++) sm_o[(wave * gq + c) * OP + dt * 16 + g * 4 + i] = o[dt][i];
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < gq * D; idx += WAVES * kWave) {
-        const int qi = idx / D, d = idx - qi * D;
+    for (int idx = threadIdx.x; idx < gq * (D / 2); idx += WAVES * kWave) {
+        const int qi = idx / (D / 2), d = 2 * (idx - qi * (D / 2));
         const int h = qtile * 16 + qi;
         float m = -INFINITY;
 #pragma unroll
         for (int w = 0; w < WAVES; w++) m = fmaxf(m, sm_m[w * 16 + qi]);
-        float l = 0.f, acc = 0.f;
+        float l = 0.f;
+        f32x2_t acc = {0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < WAVES; w++) {
             const float f = sm_m[w * 16 + qi] == -INFINITY ? 0.f : fast_exp2(sm_m[w * 16 + qi] - m);
             l += sm_l[w * 16 + qi] * f;
-            acc += sm_o[(w * gq + qi) * OP + d] * f;
+            const f32x2_t part = *(const f32x2_t *)(sm_o + (w * gq + qi) * OP + d);
+            acc[0] += part[0] * f;
+            acc[1] += part[1] * f;
         }
         const size_t hrow = (size_t)row * p.heads + kvh * G + h;
         if (live_splits == 1) {
             l = with_sink(l, m, p.sinks, kvh * G + h);
-            p.out[hrow * D + d] = (bf16_t)(l > 0.f ? acc / l : 0.f);
+            store2(p.out + hrow * D + d, l > 0.f ? acc[0] / l : 0.f, l > 0.f ? acc[1] / l : 0.f);
         } else if (p.counters) {   // read by another workgroup of this launch: straight to the device's point of coherence
-            __hip_atomic_store(p.ws_o + (hrow * p.splits + split) * D + d, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (d == 0) {
-                __hip_atomic_store(p.ws_ml + (hrow * p.splits + split) * 2, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(p.ws_ml + (hrow * p.splits + split) * 2 + 1, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+            put2(p.ws_o + (hrow * p.splits + split) * D + d, acc[0], acc[1]);
+            if (d == 0) put2(p.ws_ml + (hrow * p.splits + split) * 2, m, l);
         } else {
-            p.ws_o[(hrow * p.splits + split) * D + d] = acc;
+            p.ws_o[(hrow * p.splits + split) * D + d] = acc[0];
+            p.ws_o[(hrow * p.splits + split) * D + d + 1] = acc[1];
             if (d == 0) {
                 p.ws_ml[(hrow * p.splits + split) * 2] = m;
                 p.ws_ml[(hrow * p.splits + split) * 2 + 1] = l;
@@ -785,38 +871,39 @@ attn_decode_kernel(AttnArgs p, int qtiles) {
     if (s_seen != live_splits - 1) return;
     parts_visible();
     if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
-    // The parts are read eight at a time, all loads of a group asked for before the first is used.  The first group's
-    // values are kept: up to eight parts (the usual case) cost one round trip to memory, not one for the largest
+    // The parts are read sixteen at a time, all loads of a group asked for before the first is used.  The first group's
+    // values are kept: up to sixteen parts (the usual case) cost one round trip to memory, not one for the largest
     // maximum and another for the sums.
-    constexpr int GRP = 8;
-    for (int idx = threadIdx.x; idx < gq * D; idx += WAVES * kWave) {
-        const int qi = idx / D, d = idx - qi * D;
+    constexpr int GRP = 16;
+    for (int idx = threadIdx.x; idx < gq * (D / 2); idx += WAVES * kWave) {
+        const int qi = idx / (D / 2), d = 2 * (idx - qi * (D / 2));
         const size_t hrow = (size_t)row * p.heads + kvh * G + qtile * 16 + qi;
         const float *ml = p.ws_ml + hrow * p.splits * 2;
         const float *po = p.ws_o + hrow * p.splits * D + d;
-        auto load_group = [&](int s0, float (&ms)[GRP], float (&ls)[GRP], float (&os)[GRP]) {
+        auto load_group = [&](int s0, f32x2_t (&mls)[GRP], f32x2_t (&os)[GRP]) {
 #pragma unroll
             for (int i = 0; i < GRP; i++) {
                 const bool live = s0 + i < live_splits;
-                ms[i] = live ? __hip_atomic_load(ml + (s0 + i) * 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -INFINITY;
-                ls[i] = live ? __hip_atomic_load(ml + (s0 + i) * 2 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
-                os[i] = live ? __hip_atomic_load(po + (size_t)(s0 + i) * D, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
+                mls[i] = live ? get2(ml + (s0 + i) * 2) : (f32x2_t){-INFINITY, 0.f};
+                os[i] = live ? get2(po + (size_t)(s0 + i) * D) : (f32x2_t){0.f, 0.f};
             }
         };
-        float l = 0.f, acc = 0.f;
-        auto add_group = [&](float m, const float (&ms)[GRP], const float (&ls)[GRP], const float (&os)[GRP]) {
+        float l = 0.f;
+        f32x2_t acc = {0.f, 0.f};
+        auto add_group = [&](float m, const f32x2_t (&mls)[GRP], const f32x2_t (&os)[GRP]) {
 #pragma unroll
             for (int i = 0; i < GRP; i++) {       // in the order of the parts
-                const float f = ms[i] == -INFINITY ? 0.f : fast_exp2(ms[i] - m);
-                l += ls[i] * f;
-                acc += os[i] * f;
+                const float f = mls[i][0] == -INFINITY ? 0.f : fast_exp2(mls[i][0] - m);
+                l += mls[i][1] * f;
+                acc[0] += os[i][0] * f;
+                acc[1] += os[i][1] * f;
             }
         };
-        float ms0[GRP], ls0[GRP], os0[GRP];
-        load_group(0, ms0, ls0, os0);
+        f32x2_t ml0[GRP], os0[GRP];
+        load_group(0, ml0, os0);
         float m = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < GRP; i++) m = fmaxf(m, ms0[i]);
+        for (int i = 0; i < GRP; i++) m = fmaxf(m, ml0[i][0]);
         for (int s0 = GRP; s0 < live_splits; s0 += GRP) {
             float ms[GRP];
 #pragma unroll
@@ -825,14 +912,14 @@ attn_decode_kernel(AttnArgs p, int qtiles) {
 #pragma unroll
             for (int i = 0; i < GRP; i++) m = fmaxf(m, ms[i]);
         }
-        add_group(m, ms0, ls0, os0);
+        add_group(m, ml0, os0);
         for (int s0 = GRP; s0 < live_splits; s0 += GRP) {
-            float ms[GRP], ls[GRP], os[GRP];
-            load_group(s0, ms, ls, os);
-            add_group(m, ms, ls, os);
+            f32x2_t mls[GRP], os[GRP];
+            load_group(s0, mls, os);
+            add_group(m, mls, os);
         }
         l = with_sink(l, m, p.sinks, kvh * G + qtile * 16 + qi);      // once, where the parts meet
-        p.out[hrow * D + d] = (bf16_t)(l > 0.f ? acc / l : 0.f);
+        store2(p.out + hrow * D + d, l > 0.f ? acc[0] / l : 0.f, l > 0.f ? acc[1] / l : 0.f);
     }
 }
 
@@ -918,12 +1005,13 @@ int launch(const AttnArgs &a, int uniform_rows, int max_context, void *workspace
     if (uniform_rows) {
         const int qtiles = (G + 15) / 16;
         AttnArgs p = a;
-        constexpr int WAVES = D >= 128 ? 8 : 16;   // wide heads: fewer waves, so that the operands of a block fit the registers
+        constexpr int WAVES = D >= 128 ? 4 : 8;   // of 64 keys each; wide heads: fewer waves, so that their operands fit the registers
         void *dev_ws = nullptr;
         size_t dev_ws_bytes = 0;
         const bool fused = fllm_device_workspace(&dev_ws, &dev_ws_bytes) &&
-                           (size_t)a.rows * a.kv_heads * qtiles * sizeof(int) <= kWorkspaceCounterBytes && fllm_option_fused_merge();
-        decode_split_plan(a.rows, a.kv_heads, qtiles, max_context, WAVES * 32, fused, &p.splits, &p.keys_per_split);
+                           (size_t)a.rows * a.kv_heads * qtiles * sizeof(int) <= kWorkspaceCounterBytes && fllm_option_fused_merge() &&
+                           ((uintptr_t)workspace & 7) == 0;      // the parts pass in pieces of 8 bytes
+        decode_split_plan(a.rows, a.kv_heads, qtiles, max_context, fllm_plan::decode_unit(D), fused, &p.splits, &p.keys_per_split);
         p.counters = fused && p.splits > 1 ? (int *)dev_ws : nullptr;
         if (p.splits > 1) {
             const size_t need = fllm_plan::decode_workspace_need(a.rows, a.heads, D, p.splits);
@@ -935,16 +1023,20 @@ int launch(const AttnArgs &a, int uniform_rows, int max_context, void *workspace
         FLLM_REQUIRE(a.kv_heads * qtiles <= 65535 && p.splits <= 65535, "attention: grid too large");
         const int gq = G < 16 ? G : 16;
         const size_t smem = fllm_plan::decode_lds_bytes(D, G);
-        static_assert(WAVES == (D >= 128 ? 8 : 16), "the plan's wave count is the kernel's");
+        static_assert(WAVES == (D >= 128 ? 4 : 8), "the plan's wave count is the kernel's");
         static bool attribute_set = false;   // more than the default 64 KiB of dynamic LDS has to be asked for once
         if (!attribute_set) {
-            const hipError_t e = hipFuncSetAttribute((const void *)attn_decode_kernel<D, WAVES>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);   // a few static bytes come on top
+            hipError_t e = hipFuncSetAttribute((const void *)attn_decode_kernel<D, WAVES, 2>,
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);   // a few static bytes come on top
+            if (e == hipSuccess) e = hipFuncSetAttribute((const void *)attn_decode_kernel<D, WAVES, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);
+            if (e == hipSuccess) e = hipFuncSetAttribute((const void *)attn_decode_kernel<D, WAVES, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);
             FLLM_REQUIRE(e == hipSuccess, "attention: cannot raise the LDS limit: %s", hipGetErrorString(e));
             attribute_set = true;
         }
-        hipLaunchKernelGGL((attn_decode_kernel<D, WAVES>), dim3(a.rows, a.kv_heads * qtiles, p.splits), dim3(WAVES * kWave),
-                           smem, stream, p, qtiles);
+        const dim3 grid(a.rows, a.kv_heads * qtiles, p.splits);
+        if (a.page_size >= 32) hipLaunchKernelGGL((attn_decode_kernel<D, WAVES, 2>), grid, dim3(WAVES * kWave), smem, stream, p, qtiles);
+        else if (a.page_size == 16) hipLaunchKernelGGL((attn_decode_kernel<D, WAVES, 1>), grid, dim3(WAVES * kWave), smem, stream, p, qtiles);
+        else hipLaunchKernelGGL((attn_decode_kernel<D, WAVES, 0>), grid, dim3(WAVES * kWave), smem, stream, p, qtiles);
         if (p.splits > 1 && !p.counters)
             hipLaunchKernelGGL(attn_merge_kernel<D>, dim3(a.rows, a.heads), dim3(kWave), 0, stream, p.ws_ml, p.ws_o, a.out,
                                a.heads, p.splits, p.sinks);
@@ -973,7 +1065,7 @@ size_t fllm_attention_bf16_workspace_bytes(int rows, int heads, int kv_heads, in
     // the larger of the two plans (with and without the device workspace): which one runs is decided at the launch
     size_t most = 0;
     for (int fused = 0; fused < 2; fused++) {
-        decode_split_plan(rows, kv_heads, qtiles, max_context, (head_dim >= 128 ? 8 : 16) * 32, fused != 0, &splits, &per);
+        decode_split_plan(rows, kv_heads, qtiles, max_context, fllm_plan::decode_unit(head_dim), fused != 0, &splits, &per);
         most = std::max(most, fllm_plan::decode_workspace_need(rows, heads, head_dim, splits));
     }
     return most;
