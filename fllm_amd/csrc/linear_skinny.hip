@@ -639,13 +639,18 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
 // ---------------------------------------------------------------------------------------------
 // Every wave owns one 16-row weight tile (8 gate + 8 up rows for the SwiGLU form) for the whole K
 // slice of its workgroup, so no sums cross waves.  The activations of the slice pass through LDS in
-// chunks of 256 columns, shared by the four waves, the next chunk on its way from global memory
+// chunks of 256 columns, shared by the four waves, the next chunk (up to 48 rows: the next two, which
+// leaves two chunks of weights on their way where a chunk is waited for) on its way from global memory
 // while the current one is multiplied (two buffers, one barrier per chunk).  The weights go from
 // global memory straight into MFMA A operands, two chunks (16 KiB a wave) in flight ahead of the
 // products, across chunk, tile and item borders.  Workgroup b owns slice b % S and the row groups
 // b / S, b / S + G / S, ...  With S > 1 a wave leaves its tile's sums in the workspace and counts
 // the tile; the wave that counts the last slice adds the S partial sums in slice order and runs
-// the epilogue (as in the resident kernel).
+// the epilogue (as in the resident kernel), up to 48 rows with the parts and the operands of all row
+// tiles in one trip to memory.  What bounds it: the weights' bytes in large matrices, the trips that
+// follow each other in small ones.  At 40 rows, against one chunk ahead, a trip a row tile and slices
+// for two workgroups a compute unit: 4,096 x 4,096 17.8 -> 14.3 us, 4,096 x 14,336 29.3 -> 26.1 (4.5 TB/s),
+// 6,144 x 4,096 23.2 -> 22.0, gate/up of 2 x 14,336 x 4,096 44.9 -> 41.7, of 2 x 8,192 x 2,048 23.9 -> 17.1.
 // WT: the weights come from their tile-major copy (fllm_tile_weights, fllm_tile_weights_gate_up), K a multiple of 256.
 // PRO_SCALED: the rows are what the product before prepared for an RMSNorm (fllm_linear_add_normed); the row's scale,
 // from the parts of its sum of squares, multiplies the finished sums.
@@ -662,6 +667,7 @@ skinny_wide_kernel(SkinnyArgs a) {
     constexpr int XL = (XPIECES + THREADS - 1) / THREADS;   // loads per thread and chunk
     constexpr int NT = EPI == EPI_SWIGLU ? 8 : 16; // outputs per row and tile
     constexpr int RT = EPI == EPI_SWIGLU ? 2 : 1;
+    constexpr bool DEEP = MT <= 3;                 // registers for a second chunk of activations and all row tiles' operands
     __shared__ __attribute__((aligned(16))) bf16_t xs[2][ROWS * XP];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int r = lane & 15, g = lane >> 4;
@@ -705,8 +711,7 @@ skinny_wide_kernel(SkinnyArgs a) {
         if (++w_chunk == nchunks) w_chunk = 0, w_item++;
     };
     // activations: the chunk index within the slice is all that matters (every item walks the same slice)
-    bf16x8_t xr[XL];
-    auto load_x = [&](int chunk) {
+    auto load_x = [&](bf16x8_t (&xr)[XL], int chunk) {
 #pragma unroll
         for (int i = 0; i < XL; i++) {
             const int idx = threadIdx.x + i * THREADS;
@@ -714,7 +719,7 @@ skinny_wide_kernel(SkinnyArgs a) {
             xr[i] = *(const bf16x8_t *)((m < M && c < kcn && idx < XPIECES) ? x + (size_t)m * a.ldx + ks0 + c : zeros);
         }
     };
-    auto store_x = [&](int buffer) {
+    auto store_x = [&](const bf16x8_t (&xr)[XL], int buffer) {
 #pragma unroll
         for (int i = 0; i < XL; i++) {
             const int idx = threadIdx.x + i * THREADS;
@@ -723,56 +728,79 @@ skinny_wide_kernel(SkinnyArgs a) {
         }
     };
 
-    bf16x8_t wa[KS], wb[KS];
+    // Loads come back in the order they were asked for, so what is waited for first is asked for first: the parts of the
+    // sums of squares, two chunks of activations, two of weights.
+    __shared__ float ssq_rows[PRO == PRO_SCALED ? ROWS : 1];
+    constexpr int SQ = 16;                       // pieces of four parts asked for in one go
+    f32x4_t sq[PRO == PRO_SCALED ? SQ : 1];
+    const int sq_m = threadIdx.x >> 2, sq_q = threadIdx.x & 3;
+    const int per = (a.ssq_count + 3) / 4;
+    const int sq0 = min(sq_q * per, a.ssq_count), sq1 = min(sq0 + per, a.ssq_count);
+    const float *sq_parts = PRO == PRO_SCALED ? a.ssq_in + (size_t)min(sq_m, M - 1) * a.ssq_count : nullptr;
+    const bool sq_pieces = (per & 3) == 0 && (a.ssq_count & 3) == 0 && ((uintptr_t)a.ssq_in & 15) == 0;
+    if (PRO == PRO_SCALED && sq_pieces) {
+#pragma unroll
+        for (int i = 0; i < SQ; i++) sq[PRO == PRO_SCALED ? i : 0] = *(const f32x4_t *)(sq0 + 4 * i < sq1 ? sq_parts + sq0 + 4 * i : (const float *)zeros);
+    }
+    bf16x8_t wa[KS], wb[KS], xa[XL], xb[XL];
+    const int second = nchunks > 1 ? 1 : 0;
+    load_x(xa, 0);
+    if (DEEP) load_x(xb, second);
+    __builtin_amdgcn_sched_barrier(0);
     issue_w(wa);
     issue_w(wb);
-    __shared__ float ssq_rows[PRO == PRO_SCALED ? ROWS : 1];
+    __builtin_amdgcn_sched_barrier(0);
     if (PRO == PRO_SCALED) {
         // A row's sum of squares arrives in parts (up to a few hundred).  Four neighbouring threads share a row: each adds
-        // a quarter of the parts in index order, all its loads asked for together, and the quarters are added in order:
-        // the same sum for a row whatever the batch and the workgroup, and one trip to memory for all rows at once.
+        // a quarter of the parts in index order, and the quarters are added in order: the same sum for a row whatever the
+        // batch and the workgroup, and one trip to memory for all rows at once.
         static_assert(THREADS >= 4 * ROWS, "four threads a row");
-        const int m = threadIdx.x >> 2, q = threadIdx.x & 3;
         float t = 0.f;
         if (threadIdx.x < 4 * ROWS) {      // whole waves: ROWS is a multiple of 16
-            const int per = (a.ssq_count + 3) / 4;
-            const int i0 = min(q * per, a.ssq_count), i1 = min(i0 + per, a.ssq_count);
-            if (m < M) {
-                const float *parts = a.ssq_in + (size_t)m * a.ssq_count;
-                if ((per & 3) == 0 && (a.ssq_count & 3) == 0 && ((uintptr_t)a.ssq_in & 15) == 0) {
-#pragma unroll 4
-                    for (int i = i0; i < i1; i += 4) {
-                        const f32x4_t v = *(const f32x4_t *)(parts + i);
-                        t += v[0];
-                        t += v[1];
-                        t += v[2];
-                        t += v[3];
-                    }
-                } else {
-                    for (int i = i0; i < i1; i++) t += parts[i];
+            if (sq_pieces) {
+#pragma unroll
+                for (int i = 0; i < SQ; i++) {
+                    const f32x4_t v = sq[PRO == PRO_SCALED ? i : 0];      // zeros behind the last part
+                    t += v[0];
+                    t += v[1];
+                    t += v[2];
+                    t += v[3];
                 }
+                for (int i = sq0 + 4 * SQ; i < sq1; i += 4) {
+                    const f32x4_t v = *(const f32x4_t *)(sq_parts + i);
+                    t += v[0];
+                    t += v[1];
+                    t += v[2];
+                    t += v[3];
+                }
+            } else {
+                for (int i = sq0; i < sq1; i++) t += sq_parts[i];
             }
             const float t1 = __shfl_xor(t, 1, kWave);
-            const float pair = (q & 1) ? t1 + t : t + t1;          // quarter 2 k, then quarter 2 k + 1
+            const float pair = (sq_q & 1) ? t1 + t : t + t1;          // quarter 2 k, then quarter 2 k + 1
             const float other = __shfl_xor(pair, 2, kWave);
-            const float sum = (q & 2) ? other + pair : pair + other;
-            if (q == 0 && m < M) ssq_rows[m] = sum;
+            const float sum = (sq_q & 2) ? other + pair : pair + other;
+            if (sq_q == 0 && sq_m < M) ssq_rows[sq_m] = sum;
         }
     }
-    if (total > 0) {
-        load_x(0);
-        store_x(0);
-    }
+    store_x(xa, 0);
     __syncthreads();
 
+    EpilogueOperands rows[DEEP ? MT : 1];       // segment, position and page of this lane's rows: the same for every item
+    if (DEEP) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) load_row_operands<EPI>(a, mt * 16 + r, rows[mt]);
+    }
     f32x4_t acc[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) acc[mt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     int item = 0, chunk = 0;
 
-    auto step = [&](bf16x8_t (&buf)[KS], int q) {
+    // `now`: free; the activations of the chunk two ahead take it.  `next`: those of the next chunk, on their way since the
+    // step before, ahead of the weights that were asked for there: waiting for them leaves two chunks of weights on their way
+    auto step = [&](bf16x8_t (&buf)[KS], bf16x8_t (&now)[XL], bf16x8_t (&next)[XL], int q) {
         const int next_chunk = chunk + 1 == nchunks ? 0 : chunk + 1;
-        load_x(next_chunk);      // on its way while this chunk is multiplied (once more than needed at the very end)
+        if (!DEEP) load_x(now, next_chunk);      // on its way while this chunk is multiplied
         const bf16_t *xb = &xs[q & 1][r * XP + g * 8];
 #pragma unroll
         for (int u = 0; u < KS; u++) {
@@ -782,83 +810,117 @@ skinny_wide_kernel(SkinnyArgs a) {
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(buf[u], xf[mt], acc[mt], 0, 0, 0);
         }
+        if (DEEP) {
+            load_x(now, next_chunk + 1 == nchunks ? 0 : next_chunk + 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         issue_w(buf);      // the chunk two ahead takes this one's registers
-        store_x((q + 1) & 1);
+        store_x(DEEP ? next : now, (q + 1) & 1);
         __syncthreads();   // the next chunk is in LDS; everybody has read the one before it
         chunk = next_chunk;
         if (chunk != 0 || item >= my_items) return;      // (a step behind the last item multiplies zeros and ends nothing)
         // the item is complete: this wave's tile has its sums over the slice
         const int tile = (rg0 + item * rstride) * WAVES + wave;
         item++;
+        if (tile >= ntiles) {       // (the sums of a tile that is not there: dropped)
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) acc[mt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            return;
+        }
         const bool owner = EPI == EPI_SWIGLU ? g < 2 : true;      // 8-output tiles: lanes g < 2 hold gate rows, g >= 2 the up rows
         const int nb = tile * NT + g * 4;
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            f32x4_t s[RT];
-            s[0] = acc[mt];
+        auto take_sums = [&](int mt, f32x4_t (&sums)[RT]) {
+            sums[0] = acc[mt];
             if (EPI == EPI_SWIGLU) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) s[RT - 1][i] = __shfl(acc[mt][i], (lane + 32) & 63, kWave);
+                for (int i = 0; i < 4; i++) sums[RT - 1][i] = __shfl(acc[mt][i], (lane + 32) & 63, kWave);
             }
             acc[mt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-            const int m = mt * 16 + r;
-            bool finish = tile < ntiles;
-            if (S > 1 && tile < ntiles) {       // wave-uniform: the whole wave takes part in the hand-over
-                const __amdgpu_buffer_rsrc_t wsb = workspace_buffer(a.ws);
-                const unsigned int part = (unsigned int)(((((size_t)tile * S + sl) * MT + mt) * RT * kWave + lane) * 16);
-                if (owner && m < M) {
+        };
+        // What the epilogues read is asked for in one go, ahead of the wait for the parts of the sums: an epilogue's stores
+        // keep the compiler from moving the next one's loads up.
+        EpilogueOperands eo[DEEP ? MT : 1];
+        auto ask = [&]() {
+            if (DEEP) {
 #pragma unroll
-                    for (int t = 0; t < RT; t++) hand_over(wsb, part + t * kWave * 16, s[t]);
+                for (int mt = 0; mt < MT; mt++) {
+                    eo[mt].seg = rows[mt].seg, eo[mt].pos = rows[mt].pos, eo[mt].page = rows[mt].page;
+                    if (owner) load_item_operands<EPI>(a, mt * 16 + r, nb, n_out, eo[mt]);
                 }
-                if (mt == MT - 1) {
-                    // the pieces pass by the caches on both ways: it is enough that the wave's own have arrived in
-                    // memory before the tile is counted
-                    parts_published();
-                    int seen = 0;
-                    if (lane == 0) seen = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    seen = __shfl(seen, 0, kWave);
-                    if (seen == S - 1) {        // the last slice of this tile: add the parts in slice order
-                        parts_visible();
-                        if (lane == 0) __hip_atomic_store(a.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        };
+        auto finish = [&](int mt, f32x4_t (&sums)[RT]) {
+            const int m = mt * 16 + r;
+            if (!owner || m >= M || nb >= n_out) return;
+            EpilogueOperands own;
+            if (!DEEP) load_row_operands<EPI>(a, m, own);
+            epilogue<PRO, EPI, RT>(a, sums, PRO == PRO_SCALED ? ssq_rows[m] : 0.f, m, nb, n_out, DEEP ? eo[DEEP ? mt : 0] : own);
+        };
+        if (S == 1) {
+            ask();
 #pragma unroll
-                        for (int mt2 = 0; mt2 < MT; mt2++) {
-                            const int m2 = mt2 * 16 + r;
-                            const bool mine = owner && m2 < M && nb < n_out;
-                            f32x4_t t2[RT];
+            for (int mt = 0; mt < MT; mt++) {
+                f32x4_t s[RT];
+                take_sums(mt, s);
+                finish(mt, s);
+            }
+            return;
+        }
+        const __amdgpu_buffer_rsrc_t wsb = workspace_buffer(a.ws);
 #pragma unroll
-                            for (int t = 0; t < RT; t++) t2[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-                            // the parts of up to eight slices are asked for together (one trip to memory, not one a
-                            // slice) and added in slice order; every lane loads, so that no load sits behind a branch
-                            constexpr int GRP = MT > 4 ? 4 : 8;      // (with more row tiles the registers are needed elsewhere)
-                            for (int s0 = 0; s0 < S; s0 += GRP) {
-                                f32x4_t pv[GRP][RT];
+        for (int mt = 0; mt < MT; mt++) {
+            const unsigned int part = (unsigned int)(((((size_t)tile * S + sl) * MT + mt) * RT * kWave + lane) * 16);
+            f32x4_t s[RT];
+            take_sums(mt, s);
+            if (owner && mt * 16 + r < M) {
 #pragma unroll
-                                for (int j = 0; j < GRP; j++) {
-                                    const int s2 = s0 + j < S ? s0 + j : s0;
-                                    const unsigned int src = (unsigned int)(((((size_t)tile * S + s2) * MT + mt2) * RT * kWave + lane) * 16);
+                for (int t = 0; t < RT; t++) hand_over(wsb, part + t * kWave * 16, s[t]);
+            }
+        }
+        ask();
+        // the pieces pass by the caches on both ways: it is enough that the wave's own have arrived in memory before the
+        // tile is counted
+        parts_published();
+        int seen = 0;
+        if (lane == 0) seen = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        seen = __shfl(seen, 0, kWave);
+        if (seen != S - 1) return;
+        // the last slice of this tile: add the parts in slice order
+        parts_visible();
+        if (lane == 0) __hip_atomic_store(a.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // the parts of several slices (and of all row tiles, where there are registers) are asked for together, one trip to
+        // memory; every lane loads, so that no load sits behind a branch
+        constexpr int MB = DEEP ? MT : 1;
+        constexpr int GRP = DEEP ? (MB * RT <= 2 ? 8 : MB * RT <= 4 ? 4 : 2) : MT > 4 ? 4 : 8;
 #pragma unroll
-                                    for (int t = 0; t < RT; t++) pv[j][t] = take_over(wsb, src + t * kWave * 16);
-                                }
+        for (int mt0 = 0; mt0 < MT; mt0 += MB) {
+            f32x4_t sum[MB][RT];
 #pragma unroll
-                                for (int j = 0; j < GRP; j++)
+            for (int mt = 0; mt < MB; mt++)
 #pragma unroll
-                                    for (int t = 0; t < RT; t++)
-                                        if (s0 + j < S) t2[t] += pv[j][t];
-                            }
-                            if (!mine) continue;
-                            EpilogueOperands eo;
-                            load_row_operands<EPI>(a, m2, eo);
-                            epilogue<PRO, EPI, RT>(a, t2, PRO == PRO_SCALED ? ssq_rows[m2] : 0.f, m2, nb, n_out, eo);
-                        }
+                for (int t = 0; t < RT; t++) sum[mt][t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            for (int s0 = 0; s0 < S; s0 += GRP) {
+                f32x4_t pv[GRP][MB][RT];
+#pragma unroll
+                for (int j = 0; j < GRP; j++) {
+                    const int s2 = s0 + j < S ? s0 + j : s0;
+#pragma unroll
+                    for (int mt = 0; mt < MB; mt++) {
+                        const unsigned int src = (unsigned int)(((((size_t)tile * S + s2) * MT + mt0 + mt) * RT * kWave + lane) * 16);
+#pragma unroll
+                        for (int t = 0; t < RT; t++) pv[j][mt][t] = take_over(wsb, src + t * kWave * 16);
                     }
                 }
-                finish = false;
+#pragma unroll
+                for (int j = 0; j < GRP; j++)
+#pragma unroll
+                    for (int mt = 0; mt < MB; mt++)
+#pragma unroll
+                        for (int t = 0; t < RT; t++)
+                            if (s0 + j < S) sum[mt][t] += pv[j][mt][t];
             }
-            if (finish && owner && m < M && nb < n_out) {
-                EpilogueOperands eo;
-                load_row_operands<EPI>(a, m, eo);
-                epilogue<PRO, EPI, RT>(a, s, PRO == PRO_SCALED ? ssq_rows[m] : 0.f, m, nb, n_out, eo);
-            }
+#pragma unroll
+            for (int mt = 0; mt < MB; mt++) finish(mt0 + mt, sum[mt]);
         }
     };
 
@@ -866,8 +928,8 @@ skinny_wide_kernel(SkinnyArgs a) {
     // multiplies zeros): only then does the compiler see that the loads of one buffer always lie behind those of
     // the other, and lets them stay in flight.
     for (int q = 0; q < total; q += 2) {
-        step(wa, q);
-        step(wb, q + 1);
+        step(wa, xa, xb, q);
+        step(wb, DEEP ? xb : xa, xa, q + 1);
     }
 }
 

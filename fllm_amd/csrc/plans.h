@@ -90,9 +90,13 @@ inline size_t chunk_workspace_need(int ntiles, int S, int mt, int rt) {
 inline ChunkPlan plan_chunks(int K, int ntiles, int mt, int rt, size_t ws_bytes, bool have_ws, int cus, int forced, int waves = 4) {
     const int ngroups = (ntiles + waves - 1) / waves;
     const int slots = 8 / waves * cus;
-    // K slices: as many as fill the chip with the row groups there are, each at least two chunks long
+    // K slices: as many as fill the chip with the row groups there are, each at least two chunks long.  Up to 48 rows a
+    // workgroup has enough on its way for a compute unit of its own, and more slices only cost their sums' way through
+    // memory (40 rows, with one workgroup a unit and with two: 4,096 x 4,096 14.4 and 17.5 us, 4,096 x 14,336 26.4 and
+    // 29.3; with 49 to 64 rows two are no slower).
+    const int fill = mt <= 3 ? cus : slots;
     int S = 1;
-    while (S < 8 && ngroups * S * 2 <= slots && (K + 2 * S - 1) / (2 * S) >= 512) S *= 2;
+    while (S < 8 && ngroups * S * 2 <= fill && (K + 2 * S - 1) / (2 * S) >= 512) S *= 2;
     if (forced > 0) S = forced;
     while (S > 1) {
         const size_t need = chunk_workspace_need(ntiles, S, mt, rt);      // the kernel's offsets into it are 32 bits
@@ -114,11 +118,12 @@ inline ChunkPlan plan_chunks(int K, int ntiles, int mt, int rt, size_t ws_bytes,
 }
 // What the busiest compute unit streams under a plan, in weight rows x columns: its workgroups' row tiles over their
 // slices, as often as the row groups of a slice come round.
-inline long chunk_plan_cost(const ChunkPlan &p, int ntiles) {
+inline long chunk_plan_cost(const ChunkPlan &p, int ntiles, int cus) {
     const int ngroups = (ntiles + p.waves - 1) / p.waves;
     const int per_slice = p.grid / p.S;
     const long rounds = (ngroups + per_slice - 1) / per_slice;
-    return rounds * (8 / p.waves) * p.waves * (long)p.slice;
+    const long together = p.grid <= cus ? 1 : 8 / p.waves;       // workgroups of a compute unit
+    return rounds * together * p.waves * (long)p.slice;
 }
 // The number of waves (four, seven or eight) whose plan leaves the least to the busiest compute unit; on a tie four,
 // but see below.
@@ -129,10 +134,10 @@ inline ChunkPlan plan_chunks_balanced(int K, int ntiles, int mt, int rt, size_t 
     if (forced_waves == 4 || forced_waves == 7 || forced_waves == 8)
         return plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, forced_waves);
     ChunkPlan best = plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, 4);
-    long best_cost = chunk_plan_cost(best, ntiles);
+    long best_cost = chunk_plan_cost(best, ntiles, cus);
     for (int waves = 7; waves <= 8; waves++) {
         const ChunkPlan p = plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, waves);
-        const long cost = chunk_plan_cost(p, ntiles);
+        const long cost = chunk_plan_cost(p, ntiles, cus);
         // a tie between four and eight waves, no slices either way, three or four row tiles of activations: eight waves
         // share one copy of a chunk in LDS where two workgroups of four hold one each (the vocabulary projection at
         // 64 rows: 207 -> 194 us)
