@@ -166,7 +166,7 @@ __device__ __forceinline__ void multiply(f32x4_t (&c)[4][2], const bf16x8_t (&x)
 // reads x half 1, asks for W half 1; quarter 3 reads W half 0 of k + 1 and asks for x half 1 of k + 2.  Every quarter ends its reading side
 // by waiting until at most 12 loads (six half tiles) are outstanding: then what the next quarter reads has arrived.
 template <int EPI, bool GROUPED>
-__global__ void __launch_bounds__(kThreads, 2) tiles256_kernel(const TileArgs a) {
+__device__ __forceinline__ void tiles256(const TileArgs &a) {
     extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int wm = w >> 2, wn = w & 3, l16 = lane & 15, lg = lane >> 4;
@@ -299,7 +299,7 @@ __global__ void __launch_bounds__(kThreads, 2) tiles256_kernel(const TileArgs a)
 // the products, so LDS and the matrix cores are busy alike.  LDS: three buffers of [x][W half 0][W half 1].  K step k: half 0 reads x of k
 // and asks for W half 1 of k + 2 and W half 0 of k + 3; half 1 reads W half 1 of k and W half 0 of k + 1 and asks for x of k + 3.
 template <int EPI, bool GROUPED>
-__global__ void __launch_bounds__(kThreads, 2) tiles128_kernel(const TileArgs a) {
+__device__ __forceinline__ void tiles128(const TileArgs &a) {
     extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int wm = w >> 2, wn = w & 3, l16 = lane & 15, lg = lane >> 4;
@@ -428,20 +428,39 @@ __global__ void __launch_bounds__(kThreads, 2) tiles128_kernel(const TileArgs a)
     }
 }
 
+// The kernels, products of their own and grouped ones under names of their own in a trace; the modes of the grouped ones are those of
+// the small grouped tiles: 0 gate and up with the activation, 1 float32 sums, 2 the squared ReLU.
+template <int EPI, int ROWS>
+__global__ void __launch_bounds__(kThreads, 2) tiles_kernel(const TileArgs a) {
+    if constexpr (ROWS == 256) tiles256<EPI, false>(a);
+    else tiles128<EPI, false>(a);
+}
+template <int MODE, int ROWS>
+__global__ void __launch_bounds__(kThreads, 2) large_grouped_tiles_kernel(const TileArgs a) {
+    constexpr int EPI = MODE == 0 ? EPI_GLU : MODE == 1 ? EPI_F32 : EPI_RELU2;
+    if constexpr (ROWS == 256) tiles256<EPI, true>(a);
+    else tiles128<EPI, true>(a);
+}
+template <int EPI, bool GROUPED, int ROWS>
+auto tiles_entry() -> void (*)(TileArgs) {
+    if constexpr (GROUPED) return large_grouped_tiles_kernel<EPI == EPI_GLU ? 0 : EPI == EPI_F32 ? 1 : 2, ROWS>;
+    else return tiles_kernel<EPI, ROWS>;
+}
+
 // Launches one of the two on `blocks` workgroups (one a compute unit at most; grouped: as many tiles as there may be).
 template <int EPI, bool GROUPED>
 int launch_tiles(const TileArgs &a, int bm, long tiles, hipStream_t stream) {
     static bool raised = false;      // more than 64 KiB of LDS has to be asked for once
     if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void *)tiles256_kernel<EPI, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds256);
+        hipError_t e = hipFuncSetAttribute((const void *)tiles_entry<EPI, GROUPED, 256>(), hipFuncAttributeMaxDynamicSharedMemorySize, kLds256);
         if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)tiles128_kernel<EPI, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds128);
+            e = hipFuncSetAttribute((const void *)tiles_entry<EPI, GROUPED, 128>(), hipFuncAttributeMaxDynamicSharedMemorySize, kLds128);
         FLLM_REQUIRE(e == hipSuccess, "gemm tiles: cannot raise the LDS limit: %s", hipGetErrorString(e));
         raised = true;
     }
     const unsigned blocks = (unsigned)(tiles < 256 ? tiles : 256);
-    if (bm == 256) hipLaunchKernelGGL((tiles256_kernel<EPI, GROUPED>), dim3(blocks), dim3(kThreads), kLds256, stream, a);
-    else hipLaunchKernelGGL((tiles128_kernel<EPI, GROUPED>), dim3(blocks), dim3(kThreads), kLds128, stream, a);
+    if (bm == 256) hipLaunchKernelGGL((tiles_entry<EPI, GROUPED, 256>()), dim3(blocks), dim3(kThreads), kLds256, stream, a);
+    else hipLaunchKernelGGL((tiles_entry<EPI, GROUPED, 128>()), dim3(blocks), dim3(kThreads), kLds128, stream, a);
     return fllm_check_launch("gemm tiles");
 }
 
