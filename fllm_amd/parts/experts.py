@@ -23,6 +23,7 @@ import torch
 
 from ..registry import register_part
 from .base import INIT_BIAS, INIT_MATRIX, FeedForward
+from .mlp import activated_tiles
 
 
 class RoutedExperts(FeedForward):
@@ -58,8 +59,9 @@ class RoutedExperts(FeedForward):
         if self.weight_on not in ("input", "output"):
             raise ValueError(f"a pick's weight goes on the expert's input or output, not on {self.weight_on!r}")
         # forward(..., branch=t) stores the picks' outputs in t; with the weights on the outputs the sum needs the weights,
-        # so this part then adds to the stream itself (an arrangement hands it a stand-in)
-        self.stores_branch = self.weight_on == "input"
+        # so this part then adds to the stream itself (an arrangement hands it a stand-in), unless a shared expert's
+        # product stores there first
+        self.stores_branch = self.weight_on == "input" or bool(spec.get("shared"))
         self.limit = float(spec.get("limit") or 0.0)          # 0: nothing is clamped
         self.alpha = float(spec.get("alpha", 1.0))
         self.up_offset = float(spec.get("up_offset", 0.0))
@@ -101,10 +103,11 @@ class RoutedExperts(FeedForward):
     def branch_parts(self) -> int:
         """Rows of a stored branch that make up one token's output: a token's picks leave their outputs one after the
         other, and whoever adds the branch to the stream sums them in pick order."""
-        return self.top
+        return self.top if self.weight_on == "input" else 1
 
     def forward(self, ctx, h, residual, branch=None):
-        """`branch`: float32 [rows * top, width], row r's picks at r * top ..; None: the sum goes into `residual`."""
+        """`branch`: float32 [rows * branch_parts, width], row r's picks at r * top .. or its finished sum at r; None: the sum
+        goes into `residual`."""
         rt, ops = self.rt, self.rt.ops
         rows = h.shape[0]
         ids = rt.empty((rows, self.top), torch.int32)
@@ -117,11 +120,14 @@ class RoutedExperts(FeedForward):
         else:
             ops.route_topk(h, self.w_router, self.top, ids, weights, score=self.score, renormalize=self.renormalize,
                            route_scale=self.route_scale)
-        on_output = None
-        if self.weight_on == "output" and branch is not None:
+        on_output, stored = None, branch is not None
+        if self.weight_on == "output" and branch is not None and not self.shared:
             raise ValueError("experts whose weights lie on their outputs add to the stream themselves: no stored branch")
         if self.weight_on == "output":          # the experts read the rows as they are; the weights wait for the sum
             on_output, weights = weights, None
+            if branch is not None:              # the shared expert's product stores, the picks' sum is added to it
+                self._shared(h, branch, accumulate=False)
+                residual, branch = branch, None
         parts = branch if branch is not None else rt.empty((rows * self.top, self.hidden), torch.float32)
         grouped = getattr(ops, "experts_grouped", None)
         stream = getattr(ops, "experts_stream", None)        # decode steps
@@ -146,11 +152,18 @@ class RoutedExperts(FeedForward):
                 ops.postnorm_add(residual, parts, ones, None, parts=self.top, part_weights=on_output)
             else:
                 ops.postnorm_add(residual, parts, ones, None, parts=self.top)
-        if self.shared:          # one more expert that every row uses, its weight 1: its sum joins the picks' in the stream
-            wide = rt.empty((rows, self.shared))
+        if self.shared and not stored:
+            self._shared(h, residual, accumulate=True)
+
+    def _shared(self, h, out, accumulate):
+        """One more expert that every row uses, its weight 1: its output in `out`, or added to it."""
+        rt, ops = self.rt, self.rt.ops
+        wide = rt.empty((h.shape[0], self.shared))
+        fused = getattr(ops, "linear_relu_squared", None)          # the activation as the product's epilogue: decode-sized steps
+        if (fused is None or not fused(h, self.w_shared_up, wide)) and not activated_tiles(ops, "relu_squared_tiles", None, h, self.w_shared_up, wide):
             ops.linear(h, self.w_shared_up, wide)
             ops.activation(wide, wide, "relu2")
-            ops.linear(wide, self.w_shared_down, residual, accumulate=True)
+        ops.linear(wide, self.w_shared_down, out, accumulate=accumulate)
 
     def _ones(self, key, shape):
         ones = self.rt.shared.get(key)
