@@ -5,7 +5,8 @@
 // that go straight there (global_load_lds, 16 bytes a lane, seven half tiles ahead of their use) and waited for by count, never all.  Eight
 // waves, two a SIMD, work in two groups that are half a step apart: while one group issues the 16 products of a quarter tile, the other
 // reads its next operands from LDS and asks for a half tile of a later step; a barrier swaps them.  A half tile's place is filled again one
-// step after it was read, behind the barrier that follows the read's own wait.  16-byte chunk c of row r lies at place c ^ (r % 8) of the row:
+// step after it was read, behind a barrier that follows the read's own wait (a tile's first read of W, which lies ahead of the two
+// groups' first step, has a barrier of its own).  16-byte chunk c of row r lies at place c ^ (r % 8) of the row:
 // the lanes of an operand then meet every bank once.  Rows of W are dealt to LDS so that a lane ends up with 8 neighbouring columns (a
 // 16-byte store); a workgroup asks for its next tile's first steps before it stores the last one.
 //
@@ -257,6 +258,7 @@ __device__ __forceinline__ void tiles256(const TileArgs &a) {
         FLLM_SWAP;
         read_w(0, 0, wx);
         FLLM_LGKM0;
+        FLLM_SWAP;                          // step 0 asks for what takes that half tile's place: every wave has read it
         if (wm == 1) FLLM_SWAP;             // the second group runs half a quarter behind the first
         int k = 0;
         for (; k + 4 <= T; k += 2) {
@@ -374,6 +376,7 @@ __device__ __forceinline__ void tiles128(const TileArgs &a) {
         FLLM_SWAP;
         read_w(0, 0, w0);
         FLLM_LGKM0;
+        FLLM_SWAP;                          // as above
         if (wm == 1) FLLM_SWAP;
         uint32_t s0 = 0, s1 = kSlot, s2 = 2 * kSlot;      // where steps k, k + 1 and k + 2 lie
         int k = 0;
