@@ -467,15 +467,4 @@ int launch_tiles(const TileArgs &a, int bm, long tiles, hipStream_t stream) {
     return fllm_check_launch("gemm tiles");
 }
 
-// 256 or 128: the row tile whose rounds over the 256 compute units take less; 0: shapes they do not take.  A round of 128-row tiles takes
-// kShortRound of one of 256-row tiles (measured 0.54 to 0.64: 28,672 columns of 4,096 57 against 89 us, 16,384 of 2,048 30 against 53).
-constexpr double kShortRound = 0.62;
-inline int row_tile(long tiles256, long tiles128, int K) {
-    const bool wide = K % 128 == 0 && K >= 256, tall = K % 64 == 0 && K >= 192;
-    if (!wide && !tall) return 0;
-    if (!wide) return 128;
-    const double a = (double)((tiles256 + 255) / 256), b = kShortRound * (double)((tiles128 + 255) / 256);
-    return a <= b ? 256 : 128;
-}
-
 }  // namespace fllm_tiles

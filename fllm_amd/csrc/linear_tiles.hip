@@ -2,6 +2,7 @@
 // products (with a bias, or where their tiles fill the device).
 #include "api.h"
 #include "gemm_tiles.h"
+#include "plans.h"
 
 using namespace fllm_tiles;
 
@@ -22,8 +23,8 @@ long tiles_of(long M, int bm, int N, int cols) { return (M + bm - 1) / bm * ((N 
 
 }  // namespace
 
-// 0: launched, negative: error, 1: declined (the shape, or with `force` 0 a shape that the general path is faster at; 256 or 128 forces
-// that row tile).
+// 0: launched, negative: error, 1: declined (the shape, or with `force` 0 a shape that the general path is faster at; `force` 256 or 128
+// asks for that row tile and is declined where K is too short for it or no whole steps, as is any value but 0, 1 and these).
 //
 // The fused product against the library's product and an activation kernel, microseconds at 136 / 512 / 1,024 / 2,048 rows: 2 x 14,336 x
 // 4,096 62 -> 65 / 106 -> 95 / 203 -> 183 / 378 -> 356; 2 x 8,192 x 2,048 26 -> 27 / 41 -> 32 / 65 -> 54 / 120 -> 106; 2 x 8,960 x 1,536
@@ -34,8 +35,7 @@ extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up,
     if (!fllm_fast_kernels_enabled() || !operands_fit(x, ldx, w_gate_up, out, inter, M, 2L * inter, inter, K)) return 1;
     if (M == 0) return 0;
     const long t256 = tiles_of(M, 256, inter, 128), t128 = tiles_of(M, 128, inter, 128);
-    int bm = row_tile(t256, t128, K);
-    if (force > 1) bm = force;
+    const int bm = fllm_plan::row_tile(t256, t128, K, force);
     if (bm == 0) return 1;
     TileArgs a = tile_args(x, ldx, w_gate_up, out, inter, M, inter, K);
     a.limit = limit, a.alpha = alpha, a.up_offset = up_offset;
@@ -56,8 +56,7 @@ extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const fl
     if (!fllm_fast_kernels_enabled() || (bias && mode != 0) || !operands_fit(x, ldx, w, out, ldo, M, N, N, K)) return 1;
     if (M == 0) return 0;
     const long t256 = tiles_of(M, 256, N, 256), t128 = tiles_of(M, 128, N, 256);
-    int bm = row_tile(t256, t128, K);
-    if (force > 1) bm = force;
+    const int bm = fllm_plan::row_tile(t256, t128, K, force);
     if (bm == 0) return 1;
     TileArgs a = tile_args(x, ldx, w, out, ldo, M, N, K);
     a.bias = bias;

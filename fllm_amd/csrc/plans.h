@@ -198,6 +198,20 @@ inline SlabPlan plan_slab(int M, int n_tiles, int K, int mt, int rt, bool norm, 
     return best;
 }
 
+// ---- products of many rows on tiles of 256 or 128 rows (gemm_tiles.h) ----
+// K that the tiles can walk: in steps of 64, two steps a trip and four at least (256 rows), three at least (128 rows).
+inline bool row_tile_takes(int bm, int K) { return bm == 256 ? K % 128 == 0 && K >= 256 : bm == 128 && K % 64 == 0 && K >= 192; }
+// 256 or 128: the row tile whose rounds over the 256 compute units take less; 0: shapes they do not take.  A round of 128-row tiles takes
+// kShortRound of one of 256-row tiles (measured 0.54 to 0.64: 28,672 columns of 4,096 57 against 89 us, 16,384 of 2,048 30 against 53).
+// `asked`: 256 or 128 where a caller wants that one, 0 or 1 where it leaves the choice here.
+constexpr double kShortRound = 0.62;
+inline int row_tile(long tiles256, long tiles128, int K, int asked = 0) {
+    if (asked != 0 && asked != 1) return row_tile_takes(asked, K) ? asked : 0;
+    if (!row_tile_takes(256, K)) return row_tile_takes(128, K) ? 128 : 0;
+    const double a = (double)((tiles256 + 255) / 256), b = kShortRound * (double)((tiles128 + 255) / 256);
+    return a <= b ? 256 : 128;
+}
+
 // ---- decode attention: contexts split over workgroups ----
 // How a decode step of `rows` rows is split over the context.  A workgroup takes `unit` keys per round (64 a
 // wave).  Contexts are split when the rows alone do not fill the machine: down to one round per workgroup when

@@ -10,6 +10,7 @@
 #include "api.h"
 #include "common.h"
 #include "gemm_tiles.h"
+#include "plans.h"
 
 namespace {
 
@@ -256,7 +257,7 @@ int large_row_tile(long pairs, int E, int inter, int K, int N, int up_columns, c
         const long up = (rows * ((inter + up_columns - 1) / up_columns) + 255) / 256, down = (rows * ((N + 255) / 256) + 255) / 256;
         return (double)up * K + (double)down * inter;
     };
-    return cost(256) <= kShortRound * cost(128) ? 256 : 128;
+    return cost(256) <= fllm_plan::kShortRound * cost(128) ? 256 : 128;
 }
 
 // Both products on those tiles, behind group_pairs_kernel and (where the picks' weights scale the rows) scaled_rows_kernel.

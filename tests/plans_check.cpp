@@ -134,6 +134,19 @@ int main() {
                                 }
                             }
                 }
+    // ---- products of many rows on tiles ----
+    // What a tile walks: 256 rows steps 0 1 .. in pairs, the last four apart, 128 rows the last three apart; a K that is not taken
+    // would be cut short or read past its end, also where a caller asks for the tile.
+    for (int K = 1; K <= 1024; K++)
+        for (int asked : {0, 1, 2, 64, 128, 192, 256, 512, -1})
+            for (long rows : {1, 129, 300, 4096}) {
+                const int bm = row_tile((rows + 255) / 256 * 40, (rows + 127) / 128 * 40, K, asked);
+                REQUIRE(bm == 0 || bm == 128 || bm == 256, "row tile %d", bm);
+                REQUIRE(bm != 256 || (K % 128 == 0 && K / 64 >= 4), "256 rows at K %d (asked %d)", K, asked);
+                REQUIRE(bm != 128 || (K % 64 == 0 && K / 64 >= 3), "128 rows at K %d (asked %d)", K, asked);
+                REQUIRE(asked == 0 || asked == 1 || bm == 0 || bm == asked, "asked for %d, got %d", asked, bm);
+                if (asked == 0 || asked == 1) REQUIRE((bm != 0) == (K % 64 == 0 && K >= 192), "K %d declined", K);
+            }
     // ---- decode attention ----
     for (int rows : {1, 2, 8, 24, 64, 256})
         for (int kv_heads : {1, 2, 8, 64})

@@ -72,6 +72,9 @@ def test_what_is_declined(ops):
     assert linear(ptr(x), 256, ptr(x), None, ptr(out), 256, 256, 128, 224, 0, 1) == 1      # whole steps
     assert linear(ptr(x) + 2, 256, ptr(x), None, ptr(out), 256, 200, 128, 192, 0, 1) == 1  # operands on 16 bytes
     assert linear(ptr(x), 256, ptr(x), None, ptr(out), 256, 256, 256, 256, 0, 0) == 1      # a quarter of a round: left to the library
+    for width, asked in ((192, 256), (128, 128), (256, 2), (256, 192), (256, -1)):         # a row tile that cannot walk this K; no row tile
+        assert linear(ptr(x), 256, ptr(x), None, ptr(out), 256, 200, 128, width, 0, asked) == 1
+        assert ops.lib.fllm_gate_up_tiles(ptr(x), 256, ptr(x), ptr(out), 200, 128, width, 0.0, 1.0, 0.0, asked, ops._stream()) == 1
     assert not ops.gate_up_tiles(x[:64], x, out[:64, :128].contiguous())
     assert ops.gate_up_tiles(x[:65], x, out[:65, :128].contiguous())
 
