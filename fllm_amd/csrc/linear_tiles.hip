@@ -26,9 +26,9 @@ long tiles_of(long M, int bm, int N, int cols) { return (M + bm - 1) / bm * ((N 
 // 0: launched, negative: error, 1: declined (the shape, or with `force` 0 a shape that the general path is faster at; `force` 256 or 128
 // asks for that row tile and is declined where K is too short for it or no whole steps, as is any value but 0, 1 and these).
 //
-// The fused product against the library's product and an activation kernel, microseconds at 136 / 512 / 1,024 / 2,048 rows: 2 x 14,336 x
-// 4,096 62 -> 65 / 106 -> 95 / 203 -> 183 / 378 -> 356; 2 x 8,192 x 2,048 26 -> 27 / 41 -> 32 / 65 -> 54 / 120 -> 106; 2 x 8,960 x 1,536
-// 26 -> 23 / 42 -> 36 / 75 -> 67 / 132 -> 115; 2 x 4,096 x 1,024 26 -> 17 / 26 -> 17 / 29 -> 20 / 42 -> 35.
+// The fused product against the library's product and an activation kernel, microseconds at 512 / 1,024 / 2,048 rows: 2 x 14,336 x 4,096
+// 106 -> 95 / 203 -> 183 / 378 -> 356; 2 x 8,192 x 2,048 41 -> 32 / 65 -> 54 / 120 -> 106; 2 x 8,960 x 1,536 42 -> 36 / 75 -> 67 / 132 -> 115;
+// 2 x 4,096 x 1,024 26 -> 17 / 29 -> 20 / 42 -> 35.  Where few rows or half-empty rounds make it slower: activation_joins in plans.h.
 extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up, void *out, int M, int inter, int K, float limit, float alpha,
                                   float up_offset, int force, hipStream_t stream) {
     FLLM_REQUIRE(M >= 0 && inter > 0 && K > 0 && ldx >= K && x && w_gate_up && out, "gate_up_tiles: bad sizes or operands missing");
@@ -36,16 +36,17 @@ extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up,
     if (M == 0) return 0;
     const long t256 = tiles_of(M, 256, inter, 128), t128 = tiles_of(M, 128, inter, 128);
     const int bm = fllm_plan::row_tile(t256, t128, K, force);
-    if (bm == 0) return 1;
+    const long tiles = bm == 256 ? t256 : t128;
+    if (bm == 0 || (!force && !fllm_plan::activation_joins(M, 2L * inter, K, bm, tiles))) return 1;
     TileArgs a = tile_args(x, ldx, w_gate_up, out, inter, M, inter, K);
     a.limit = limit, a.alpha = alpha, a.up_offset = up_offset;
-    return launch_tiles<EPI_GLU, false>(a, bm, bm == 256 ? t256 : t128, stream);
+    return launch_tiles<EPI_GLU, false>(a, bm, tiles, stream);
 }
 
 // mode 0: out bfloat16 = x w^T (+ bias); 1: out float32 = x w^T; 2: out bfloat16 = relu(x w^T)^2.
 //
-// The squared ReLU against the library's product and a kernel of its own (13,312 x 1,536): 26 -> 20 us at 136 rows, 31 -> 23 at 512, 87 -> 68
-// at 2,048.  A bias (2,048 x 1,536; the general path is linear_tiled_mfma_kernel): 32 -> 23 us at 136 rows, 34 -> 24 at 2,048.  Without either
+// The squared ReLU against the library's product and a kernel of its own (13,312 x 1,536): 31 -> 23 us at 512 rows, 87 -> 68 at 2,048; fewer rows
+// as above.  A bias (2,048 x 1,536; the general path is linear_tiled_mfma_kernel): 32 -> 23 us at 136 rows, 34 -> 24 at 2,048.  Without either
 // the library has kernels for every tile of the device's time, and these tiles are ahead only where they fill whole rounds over the compute
 // units: 4,096 x 14,336 at 2,048 rows (256 tiles) 207 -> 188 us, at 1,900 (240) 191 -> 182, at 1,536 (192) 167 -> 177; 4,096 x 4,096 at
 // 2,048 rows 59 -> 55; 6,144 x 4,096 at 2,048 rows (192 of 256 rows) 80 -> 77, at 1,900 76 -> 78.  Hence nine tenths of the last round.
@@ -61,6 +62,7 @@ extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const fl
     TileArgs a = tile_args(x, ldx, w, out, ldo, M, N, K);
     a.bias = bias;
     const long tiles = bm == 256 ? t256 : t128, slots = (tiles + 255) / 256 * 256;
+    if (!force && mode == 2 && !fllm_plan::activation_joins(M, N, K, bm, tiles)) return 1;
     if (!force && mode != 2 && !bias && (K < 2048 || 10 * tiles < 9 * slots)) return 1;
     if (mode == 0) return launch_tiles<EPI_STORE, false>(a, bm, tiles, stream);
     if (mode == 1) return launch_tiles<EPI_F32, false>(a, bm, tiles, stream);

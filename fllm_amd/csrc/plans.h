@@ -212,6 +212,23 @@ inline int row_tile(long tiles256, long tiles128, int K, int asked = 0) {
     return a <= b ? 256 : 128;
 }
 
+// Whether a product with its activation in the epilogue (gate and up: `columns` counts both; the squared ReLU) goes to the tiles, or to the GEMM
+// library and a kernel for the activation.  A tile costs the same however few of its rows and columns are there and however few of the
+// compute units have one, where the library has smaller tiles and cuts K; against that stands one pass over the product, which
+// weighs less the longer K is.  share: what the rounds of the tiles do for this product, 1 where every compute unit has whole 256-row
+// tiles all the time.  Measured inside a graph, weights from memory, microseconds library and kernel -> tiles at rows: 28,672 columns of
+// 4,096 65 60 -> 67, 160 65 -> 68, 320 85 -> 97, 640 0.92x, then 420 1.08x, 512 114 -> 100, 900 1.10x (line at 0.65); 16,384 of 2,048 128 24 -> 34, 256 33 -> 34,
+// 513 0.92x, 1,030 0.94x, then 420 1.18x, 512 43 -> 38, 768 1.08x (line at 0.57); 17,920 of 1,536 128 25.5 -> 29.6, then 192 29.3 -> 27.5, 320 34 -> 28;
+// the squared ReLU of 4,480 of 1,536 128 19 -> 26, 512 22.9 -> 24.8, then 900 1.21x, of 13,312 of 1,536 128 22 -> 28, then 320 31 -> 26, 512 35 -> 28 (line at
+// 0.29).  Up to K 1,024 the two sides are a few microseconds apart on the device (8,192 of 1,024 128 15.8 -> 20.3, 320 19.5 -> 19.2, 512 21.5 -> 19.9) and a
+// prompt step of such a model waits for the host's launches, of which the tiles save one: 24 -> 18 to 20 at 65 to 512 rows launched one by one.
+inline bool activation_joins(long M, long columns, int K, int bm, long tiles) {
+    if (K <= 1024) return true;
+    const double rounds = (double)((tiles + 255) / 256) * (bm == 256 ? 1.0 : kShortRound);
+    const double share = (double)M * (double)columns / (rounds * 256.0 * 65536.0), line = (K - 1024) / 1792.0;
+    return share >= (line < 0.65 ? line : 0.65);
+}
+
 // ---- decode attention: contexts split over workgroups ----
 // How a decode step of `rows` rows is split over the context.  A workgroup takes `unit` keys per round (64 a
 // wave).  Contexts are split when the rows alone do not fill the machine: down to one round per workgroup when
