@@ -49,7 +49,7 @@ assert SAMPLE_ROW_BYTES == 32
 _lib = None
 
 
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 
 def load_library(build_if_missing: bool = True):
