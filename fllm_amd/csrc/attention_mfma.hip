@@ -665,7 +665,8 @@ __global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per
 attn_decode_kernel(AttnArgs p, int qtiles) {
     constexpr int KD = D / 32, DT = D / 16;
     constexpr int OP = D + 2;
-    extern __shared__ float dsm[];   // sm_m[WAVES][16], sm_l[WAVES][16], sm_o[WAVES][gq][OP]
+    // sm_m[WAVES][16], sm_l[WAVES][16], sm_o[WAVES][gq][OP]; outputs are read in pairs, so the area begins on 16 bytes behind the kernel's own
+    extern __shared__ __attribute__((aligned(16))) float dsm[];
     const int row = blockIdx.x;
     const int qtile = blockIdx.y % qtiles, kvh = blockIdx.y / qtiles;
     const int split = blockIdx.z;
