@@ -1082,7 +1082,7 @@ int fllm_attention_bf16_fast(const void *q, int q_stride, const void *k_pages, c
     if (v_dim != head_dim) return 1;     // these kernels read keys and values of one width
     (void)num_pages;
     if (!fast_shape(heads, kv_heads, head_dim, page_size)) return 1;
-    if (q_stride % 8 != 0 || ((uintptr_t)q & 15) != 0) return 1;
+    if (q_stride % 8 != 0 || (((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages) & 15) != 0) return 1;      // 16-byte loads
     const int singles = num_segs - single_from;       // segments of one row each, at the end of the batch
     if (single_from == 0 && rows != num_segs) return 1;
     if (singles > rows) return 1;

@@ -745,8 +745,8 @@ int fllm_launch_normed_rope_store(const void *qkv, int ld, int norm_mode, const 
     if (rows == 0) return 0;
     const size_t smem = (size_t)(heads + kv_heads) * sizeof(float);
     const uintptr_t bases = (uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)blend | (uintptr_t)q_weight | (uintptr_t)k_weight |
-                            (rope_dims > 0 ? (uintptr_t)cos_table | (uintptr_t)sin_table : 0);
-    // whole pieces of 8 lanes everywhere, on 16 bytes; a head's threads in one wave
+                            (rope_dims > 0 ? (uintptr_t)cos_table | (uintptr_t)sin_table : 0) | (store_kv ? (uintptr_t)k_pages : 0);
+    // whole pieces of 8 lanes everywhere, on 16 bytes (values are stored one by one); a head's threads in one wave
     if (dtype == FLLM_BF16 && rope_dims % 16 == 0 && key_chunk == 8 && k_dim % 8 == 0 && k_dim <= 8 * kWave && v_dim % 8 == 0 && ld % 8 == 0 &&
         blend_ld % 8 == 0 && (bases & 15) == 0) {
         int lanes = 1;

@@ -77,3 +77,33 @@ def test_decode_attention_at_its_edges(d, heads, kv_heads, ps, window, chunk, si
             error = (got - exact).abs().max() / exact.abs().max()
             assert error <= 2 ** -7, (offset, batch, float(error))
     assert torch.isfinite(torch.cat(results)).all()
+
+
+@pytest.mark.parametrize("moved", ["keys", "values"])
+def test_pages_that_begin_off_16_bytes_go_to_the_plain_kernel(moved):
+    """The matrix-core kernels read 16 bytes of keys and of values at a time; pages that begin elsewhere give the plain kernel's bits."""
+    from fllm_amd.kernels import Ops
+    ops = Ops()
+    gen = torch.Generator().manual_seed(9)
+    heads, kv_heads, d, ps, contexts = 8, 2, 64, 16, [1, 40, 100]
+    pages, rows = 24, len(contexts)
+    rnd = lambda *s: torch.randn(*s, generator=gen).to(torch.bfloat16).cuda()
+    q, kp, vp = rnd(rows, heads * d), rnd(pages, kv_heads, d // 8, ps, 8), rnd(pages, kv_heads, d, ps)
+    tables = torch.randperm(pages, generator=gen)[:rows * 7].view(rows, 7).to(torch.int32).cuda()
+    pos = torch.tensor([n - 1 for n in contexts], dtype=torch.int32, device="cuda")
+    seg, start = (torch.arange(n, dtype=torch.int32, device="cuda") for n in (rows, rows + 1))
+    off = lambda t: torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape).copy_(t)
+
+    def run(k, v):
+        out = torch.empty((rows, heads * d), dtype=torch.bfloat16, device="cuda")
+        space = torch.empty(ops.attention_workspace_bytes(rows, heads, kv_heads, d, 100) + 16, dtype=torch.uint8, device="cuda")
+        ops.attention(q, k, v, tables, pos, seg, start, out, heads, kv_heads, d, ps, d ** -0.5, None, 100, uniform_rows=1, workspace=space)
+        return out
+
+    got = run(off(kp) if moved == "keys" else kp, off(vp) if moved == "values" else vp)
+    ops.set_fast_kernels(False)
+    try:
+        want = run(kp, vp)
+    finally:
+        ops.set_fast_kernels(True)
+    assert torch.equal(got, want)

@@ -96,6 +96,31 @@ def test_normed_and_rotated_heads(ops, mode, heads, kv_heads, k_dim, v_dim, rope
     assert torch.equal(outs[0][2], outs[1][2])          # values are stored, or blended in float32, alike
 
 
+@pytest.mark.parametrize("form", ["heads", "projections"])
+def test_keys_that_begin_off_16_bytes_are_stored_by_the_plain_form(ops, form):
+    """Pieces of 16 bytes go to pages that begin on 16 bytes only: the same bits as the plain form, which operands off that boundary select."""
+    g = torch.Generator().manual_seed(3)
+    rows, page, pages, heads, kv_heads, dim = 5, 16, 4, 12, 2, 128
+    qkv = torch.randn(rows, (heads + 2 * kv_heads) * dim, generator=g).to(torch.bfloat16).to(DEV)
+    qw, kw = (1.0 + 0.1 * torch.randn(dim if form == "heads" else n * dim, generator=g).to(DEV) for n in (heads, kv_heads))
+    angles = torch.rand(64, dim // 2, generator=g) * 6.0
+    cos, sin = torch.cos(angles).contiguous().to(DEV), torch.sin(angles).contiguous().to(DEV)
+    pos = torch.tensor([0, 15, 16, 37, 5], dtype=torch.int32, device=DEV)
+    seg = torch.tensor([0, 0, 1, 1, -1], dtype=torch.int32, device=DEV)
+    tables = torch.tensor([[3, 1, 0], [2, 0, 1]], dtype=torch.int32, device=DEV)
+    outs = []
+    for rows_as, pages_as in ((off, lambda t: t), (lambda t: t, off)):
+        q = torch.zeros(rows, heads * dim, dtype=torch.bfloat16, device=DEV)
+        k = pages_as(torch.zeros(pages, kv_heads, dim // 8, page, 8, dtype=torch.bfloat16, device=DEV))
+        v = torch.zeros(pages, kv_heads, dim, page, dtype=torch.bfloat16, device=DEV)
+        if form == "heads":
+            ops.normed_rope_store(rows_as(qkv), 1, qw, kw, 1e-5, q, pos, seg, tables, cos, sin, k, v, heads, kv_heads, dim, dim, dim, page, 8)
+        else:
+            ops.qk_norm_rope_store(rows_as(qkv), qw, kw, 1e-5, q, pos, seg, tables, cos, sin, k, v, heads, kv_heads, dim, dim, dim, page, 8)
+        outs.append((q[:4], k, v))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
 @pytest.mark.parametrize("x_type", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rows,width,weighted", [(1, 4, True), (3, 1536, True), (2, 2052, False), (2, 8192, True)])
 def test_gated_norms(ops, rows, width, weighted, x_type):
