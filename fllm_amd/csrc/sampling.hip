@@ -1048,8 +1048,8 @@ adjust_logits_kernel(float *__restrict__ logits, int vocab, const FllmAdjustRow 
         for (int i = threadIdx.x; i < kAdjustSpan / 32; i += kAdjustBlock) allowed_bits[i] = 0;
         __syncthreads();
         for (int j = from + threadIdx.x; j < to; j += kAdjustBlock) {
-            const int at = allowed[j] - begin;
-            atomicOr(&allowed_bits[at / 32], 1u << (at % 32));
+            const unsigned int at = (unsigned int)(allowed[j] - begin);
+            if (at < kAdjustSpan) atomicOr(&allowed_bits[at / 32], 1u << (at % 32));      // a list that does not rise stays inside the span's bits
         }
         __syncthreads();
         for (int i = begin + threadIdx.x; i < end; i += kAdjustBlock)

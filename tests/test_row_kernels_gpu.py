@@ -162,3 +162,21 @@ def test_adjusted_logits_over_spans(ops, vocab):
     want = ReferenceOps().adjust_logits(logits.clone(), packed, sections, last)
     got = ops.adjust_logits(logits.clone().to(DEV), packed.to(DEV), sections, last.to(DEV)).cpu()
     torch.testing.assert_close(got, want.float(), rtol=1e-6, atol=1e-6)
+
+
+def test_allow_lists_that_do_not_rise_stay_inside_their_row(ops):
+    """The lists are the caller's word to rise; one that does not may block more than it says, and nothing outside of its row."""
+    from fllm_amd.sampling import SamplingParams
+    from fllm_amd.sampling.adjust import AdjustRow, pack
+    vocab, listed = 20000, (3, 700, 8191, 8192, 12000, 19999)
+    packed, sections = pack([None, AdjustRow(SamplingParams(allowed_token_ids=listed), {}, allowed=listed), None])
+    words = packed.tolist()
+    at = next(i for i in range(len(words)) if tuple(words[i:i + len(listed)]) == listed)
+    logits = torch.randn(3, vocab, generator=torch.Generator().manual_seed(1))
+    blocked = [t for t in range(vocab) if t not in listed]
+    for order in ((19999, 12000, 8192, 8191, 700, 3), (8192, 3, 19999, 700, 12000, 8191), (12000, 19999, 3, 8191, 8192, 700)):
+        packed[at:at + len(listed)] = torch.tensor(order, dtype=torch.int32)
+        got = ops.adjust_logits(logits.clone().to(DEV), packed.to(DEV), sections).cpu()
+        assert torch.equal(got[0], logits[0]) and torch.equal(got[2], logits[2])
+        assert (got[1, blocked] == float("-inf")).all()
+        assert all(got[1, t] in (logits[1, t], float("-inf")) for t in listed)
