@@ -93,7 +93,8 @@ class Engine:
         token (end of sequence, stop id) has one more row in flight by then; that row is dropped.
 
         `decode_weight_tiles` (True, False, "auto": within half of the memory that is free once the weights are placed):
-        second copies of the layers' matrices in the order decode steps read them (`Runtime.tile_for_decode`).
+        second copies of the layers' matrices in the order decode steps read them (`Runtime.tile_for_decode`), routed
+        experts' last and within an eighth; the cache has the fewer pages.
 
         `check_layers`: the first so many steps run every layer also with the plain kernels and print, layer by
         layer, how far the two are apart, the largest value, a checksum and NaN/Inf counts (`runner.check_layers`)."""

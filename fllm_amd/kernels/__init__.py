@@ -1004,14 +1004,18 @@ class Ops:
         self._check(code)
         return True
 
+    @staticmethod
+    def tile_experts_supported(w: torch.Tensor) -> bool:
+        """Whether `tile_experts` can keep a copy of this stack."""
+        return (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 3 and w.is_contiguous() and w.shape[1] % 16 == 0 and w.shape[2] % 32 == 0
+                and w.shape[2] >= 256 and w.shape[0] * w.shape[1] < 1 << 31)
+
     def tile_experts(self, w: torch.Tensor) -> bool:
         """Keeps beside a stack of experts' matrices (bfloat16 [experts, N, K] on the GPU, N in steps of 16, K in steps of 32 from 256 on) a copy in
         the order `experts_stream` reads it, as `tile_for_decode` does for single matrices; given up with `w`."""
-        if not (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 3 and w.is_contiguous()):
+        if not self.tile_experts_supported(w):
             return False
         E, N, K = w.shape
-        if N % 16 != 0 or K % 32 != 0 or K < 256 or E * N >= 1 << 31:
-            return False
         key, kind = w.data_ptr(), ("experts", E, N, K)
         if key in Ops._tiles and Ops._tiles[key][0] == kind:
             return True

@@ -89,8 +89,7 @@ class RoutedExperts(FeedForward):
                 raise ValueError("experts without a gate carry their weight on the output and clamp nothing")
             self.w_up = torch.stack([rt.matrix(weights[f"up_{e}"]) for e in range(n)]).contiguous()
         self.w_down = torch.stack([rt.matrix(weights[f"down_{e}"]) for e in range(n)]).contiguous()
-        rt.tile_experts(self.w_gate_up if self.gated else self.w_up)
-        rt.tile_experts(self.w_down)
+        rt.tile_experts(self.w_gate_up if self.gated else self.w_up, self.w_down)
         self.shared = int(spec.get("shared") or 0)
         if self.shared:
             if self.gated:

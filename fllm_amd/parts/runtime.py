@@ -6,6 +6,8 @@ from typing import Any, Dict
 
 import torch
 
+EXPERTS = 3       # the priority of routed experts' copies, behind every other
+
 
 class Runtime:
     """`dtype` is the compute precision: float32 (everything in true 32-bit) or bfloat16
@@ -20,7 +22,7 @@ class Runtime:
         self.ops = ops
         self.max_context = int(max_context)
         # second copies of some weight matrices in the order decode steps read them (`tile_for_decode`): True, False, or
-        # "auto": as long as they leave half of the free memory to the cache
+        # "auto": as long as they leave half of the free memory to the cache (routed experts: seven eighths)
         self.decode_weight_tiles = decode_weight_tiles
         self._tile_requests = None            # a list while a model is being built
         # weak: a placed tensor lives as long as a part holds it (pieces of a concatenated matrix are freed)
@@ -50,28 +52,32 @@ class Runtime:
         bytes again and takes a fifth off such a product at 8 rows).  `gate_up`: w is [gate; up], see the library.
         `priority`: while a model is being built the copies are only asked for, and made when it is whole
         (`tiles_for_model`), the lower numbers first: 0 for copies that every decode step reads (output and down
-        projections), 1 for the layers' other matrices, 2 for the vocabulary projection (once a step)."""
+        projections), 1 for the layers' other matrices, 2 for the vocabulary projection (once a step), 3 for routed
+        experts (`tile_experts`)."""
         tile = getattr(self.ops, "tile_for_decode", None)
         if tile is not None:
-            self._ask_for_copy(w, (lambda t: tile(t, gate_up=True)) if gate_up else tile, priority)
+            self._ask_for_copy((w,), lambda: tile(w, gate_up=True) if gate_up else tile(w), priority)
 
-    def tile_experts(self, w: torch.Tensor, priority: int = 1) -> None:
-        """The same for a stack of experts' matrices [experts, N, K] (`Ops.tile_experts`)."""
-        tile = getattr(self.ops, "tile_experts", None)
-        if tile is not None:
-            self._ask_for_copy(w, tile, priority)
+    def tile_experts(self, *stacks: torch.Tensor) -> None:
+        """The same for the stacks of experts' matrices [experts, N, K] that a step reads together (`Ops.tile_experts`): all of
+        them or none, since the kernel that reads the copies takes both products.  They come last (a step reads the
+        picked experts of them only) and have a share of their own (`tiles_for_model`)."""
+        tile, supported = getattr(self.ops, "tile_experts", None), getattr(self.ops, "tile_experts_supported", None)
+        if tile is not None and all(supported(w) for w in stacks):
+            self._ask_for_copy(stacks, lambda: all([tile(w) for w in stacks]), EXPERTS)
 
-    def _ask_for_copy(self, w: torch.Tensor, make, priority: int) -> None:
-        if not self.decode_weight_tiles or self.dtype != torch.bfloat16 or not w.is_cuda:
+    def _ask_for_copy(self, matrices, make, priority: int) -> None:
+        if not self.decode_weight_tiles or self.dtype != torch.bfloat16 or not all(w.is_cuda for w in matrices):
             return
+        size = sum(w.numel() * w.element_size() for w in matrices)
         if self._tile_requests is not None:
-            self._tile_requests.append((priority, len(self._tile_requests), w, make))
+            self._tile_requests.append((priority, len(self._tile_requests), size, make))
             return
         if self.decode_weight_tiles == "auto":
             free, _ = torch.cuda.mem_get_info(self.device)
-            if w.numel() * w.element_size() > free // 20:
+            if size > free // 20:
                 return                                    # the device is filling up
-        make(w)
+        make()
 
     def collect_tile_requests(self) -> None:
         """From here on `tile_for_decode` only notes what is asked for, until `tiles_for_model`."""
@@ -80,25 +86,28 @@ class Runtime:
     def tiles_for_model(self) -> int:
         """Makes the copies that the parts of a model asked for, now that all its weights are on the device: in the order
         of their priorities, and under "auto" within half of the memory that is free now (the other half is the
-        cache's).  A copy that does not fit is left out and smaller ones behind it may still be made, so a model too
-        large for all copies keeps those that every step reads.  Returns the bytes copied."""
+        cache's), routed experts within an eighth: their stacks are most of a large routed model, and every byte of a
+        copy is one that the cache has no pages for.  A copy that does not fit is left out and smaller ones behind it
+        may still be made, so a model too large for all copies keeps those that every step reads.  Returns the bytes
+        copied."""
         requests, self._tile_requests = sorted(self._tile_requests or [], key=lambda r: r[:2]), None
         if not requests:
             return 0
-        budget = None
+        budget = experts_budget = None
         if self.decode_weight_tiles == "auto":
             torch.cuda.empty_cache()          # what placing the weights left in the allocator's hands counts as free
             free, _ = torch.cuda.mem_get_info(self.device)
-            budget = free // 2
+            budget, experts_budget = free // 2, free // 8
         made = 0
-        for _, _, w, make in requests:
-            size = w.numel() * w.element_size()
-            if budget is not None and size > budget:
+        for priority, _, size, make in requests:
+            if budget is not None and size > (min(budget, experts_budget) if priority == EXPERTS else budget):
                 continue
-            if make(w):
+            if make():
                 made += size
                 if budget is not None:
                     budget -= size
+                    if priority == EXPERTS:
+                        experts_budget -= size
         return made
 
     def forget_host_tensors(self) -> None:

@@ -67,3 +67,49 @@ def test_outside_a_model_a_copy_is_made_at_once(monkeypatch):
     rt.tile_for_decode(Matrix("large", 16))             # more than a twentieth of what is free
     rt.tile_for_decode(Matrix("pair", 2), gate_up=True)
     assert lib.made == [("small", False), ("pair", True)]
+
+
+class LibraryWithExperts(Library):
+    def tile_experts_supported(self, w):
+        return not w.name.startswith("odd")
+
+    def tile_experts(self, w):
+        self.made.append(w.name)
+        return True
+
+
+def build_routed(rt, layers=3, kind=""):
+    rt.collect_tile_requests()
+    for layer in range(layers):
+        rt.tile_experts(Matrix(f"up{layer}", 200), Matrix(f"{kind}down{layer}", 100))
+        rt.tile_for_decode(Matrix(f"o{layer}", 32))
+        rt.tile_for_decode(Matrix(f"qkv{layer}", 48), priority=1)
+    rt.tile_for_decode(Matrix("vocabulary", 300), priority=2)
+    return rt.tiles_for_model()
+
+
+def test_experts_copies_come_last_in_pairs_and_within_an_eighth(monkeypatch):
+    dense = [(f"{kind}{layer}", False) for kind in ("o", "qkv") for layer in range(3)] + [("vocabulary", False)]       # 540 MiB
+    pairs = [name for layer in range(3) for name in (f"up{layer}", f"down{layer}")]                                    # 300 MiB a layer
+    for free_mib, want in ((1 << 20, dense + pairs),
+                           (8 * 650, dense + pairs[:4]),            # an eighth holds two layers' pairs
+                           (8 * 290, dense),                        # and not one, though a single stack would fit
+                           (2 * 560, dense),                        # what every step reads is not pushed out
+                           (2 * 100, [("o0", False), ("o1", False), ("o2", False)])):
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device=None: (free_mib << 20, 1 << 40))
+        lib = LibraryWithExperts()
+        made = build_routed(Runtime(torch.device("cpu"), torch.bfloat16, lib, 128, decode_weight_tiles="auto"))
+        assert lib.made == want, (free_mib, lib.made)
+        assert made == sum((540 if want[:7] == dense else 32 * len(want), 300 * sum(n in ("up0", "up1", "up2") for n in want))) << 20
+    lib = LibraryWithExperts()
+    build_routed(Runtime(torch.device("cpu"), torch.bfloat16, lib, 128, decode_weight_tiles=True))
+    assert lib.made == dense + pairs
+    lib = LibraryWithExperts()                                      # a stack that has no copy: neither has the other
+    build_routed(Runtime(torch.device("cpu"), torch.bfloat16, lib, 128, decode_weight_tiles=True), kind="odd")
+    assert lib.made == dense
+    lib = LibraryWithExperts()                                      # outside of a model: at once, within a twentieth together
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device=None: (100 << 20, 1 << 40))
+    rt = Runtime(torch.device("cpu"), torch.bfloat16, lib, 128)
+    rt.tile_experts(Matrix("a", 3), Matrix("b", 3))
+    rt.tile_experts(Matrix("c", 3), Matrix("d", 2))
+    assert lib.made == ["c", "d"]
