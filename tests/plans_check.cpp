@@ -163,18 +163,29 @@ int main() {
         REQUIRE(activation_joins(m.rows, m.columns, m.K, bm, bm == 256 ? t256 : t128) == m.joins, "%d columns of %d, %ld rows", m.columns, m.K, m.rows);
     }
     // ---- decode attention ----
+    for (int head_dim : {32, 64, 128}) {      // a wave's 64 keys; one row of one head group, and the part that tips the choice
+        const int unit = decode_unit(head_dim), last = 16 * unit - 31;
+        REQUIRE(unit == decode_waves(head_dim) * 64, "unit %d", unit);
+        int splits = 0, per = 0;
+        decode_split_plan(1, 1, 1, last, unit, true, &splits, &per);
+        REQUIRE(splits == 16 && per == unit, "%d parts of %d", splits, per);
+        decode_split_plan(1, 1, 1, last + 1, unit, true, &splits, &per);
+        REQUIRE(splits == 9 && per == 2 * unit, "%d parts of %d", splits, per);
+    }
     for (int rows : {1, 2, 8, 24, 64, 256})
         for (int kv_heads : {1, 2, 8, 64})
             for (int group : {1, 4, 7, 16, 40})
                 for (int head_dim : {32, 64, 128})
-                    for (int context : {1, 31, 256, 1000, 4096, 40000, 131072})
+                    // around sixteen and thirty-two parts of one round (256 and 512 keys)
+                    for (int context : {1, 31, 256, 1000, 4065, 4066, 4096, 8161, 8162, 16353, 16354, 40000, 131072})
                         for (int fused = 0; fused < 2; fused++) {
-                            const int qtiles = (group + 15) / 16, unit = decode_waves(head_dim) * 32;
+                            const int qtiles = (group + 15) / 16, unit = decode_unit(head_dim);
                             int splits = 0, per = 0;
                             decode_split_plan(rows, kv_heads, qtiles, context, unit, fused != 0, &splits, &per);
                             const long span = (long)context + 31;
                             REQUIRE(splits >= 1 && splits <= 64 && per % unit == 0, "decode splits %d per %d", splits, per);
                             REQUIRE((long)splits * per >= span && (long)(splits - 1) * per < span, "decode: %d splits of %d keys for %d", splits, per, context);
+                            REQUIRE(!fused || per > unit || splits <= 16, "decode: %d parts of one round, the merge reads sixteen a trip", splits);
                             REQUIRE(decode_lds_bytes(head_dim, group) + 1024 <= kLdsBytes, "decode LDS");
                             const size_t need = decode_workspace_need(rows, kv_heads * group, head_dim, splits);
                             if (splits > 1) {

@@ -1,6 +1,6 @@
 """Products of many rows on 256- and 128-row tiles (gemm_tiles.h) against float64: tiles of one row, rows and columns that no tile divides,
-the shortest K, K of an odd number of steps (128-row tiles), several tiles a workgroup, every epilogue, and grouped by expert with experts
-of no pair, one pair and several tiles.  Tolerance: operands are exact in float64, so an output may be off by the float32 sum (K * 2^-24 of the
+the shortest K, K of an odd number of steps (128-row tiles), more tiles than workgroups for each row tile and epilogue, and grouped by expert
+with experts of no pair, one pair and several tiles, and with more tiles than workgroups in both products.  Tolerance: operands are exact in float64, so an output may be off by the float32 sum (K * 2^-24 of the
 sum of the products' sizes, which random signs keep far below) and one rounding to bfloat16, 2^-9; twice that, of the value and of a
 hundredth of the largest."""
 import pytest
@@ -51,6 +51,29 @@ def test_every_epilogue(ops, M, N, K, bm):
     assert ops.lib.fllm_linear_tiles(ptr(x), K + 8, ptr(w), None, ptr(sums), N + 16, M, N, K, 1, bm, stream) == 0
     close(sums[:, :N], first, 1e-4)
     assert sums[:, N:].isnan().all()
+
+
+@pytest.mark.parametrize("bm,K", [(256, 256), (256, 640), (128, 192), (128, 448)])
+def test_workgroups_that_take_several_tiles(ops, bm, K):
+    """A launch has 256 workgroups at most.  2,100 rows x 8,200 columns are 297 tiles of 256 rows (gate and up 585), 561 of 128 (1,105): a workgroup
+    asks for its next tile's first steps before it stores the one that it has, and the last row and column tiles are ragged."""
+    M, N = 2100, 8200
+    g = torch.Generator().manual_seed(K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(2 * N, K, generator=g) * K ** -0.5).to(torch.bfloat16).to(DEV)
+    bias = torch.randn(N, generator=g).to(DEV)
+    y = x.double() @ w.double().T
+    gate, up = y[:, :N], y[:, N:]
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    assert ops.lib.fllm_gate_up_tiles(ptr(x), K, ptr(w), ptr(out), M, N, K, 0.0, 1.0, 0.0, bm, ops._stream()) == 0
+    close(out, gate * torch.sigmoid(gate) * up, 2 * BF16_EPS)
+    for mode, b, want in ((0, None, gate), (0, bias, gate + bias.double()), (2, None, gate.clamp(min=0) ** 2)):
+        out.fill_(float("nan"))
+        assert ops.lib.fllm_linear_tiles(ptr(x), K, ptr(w), ptr(b), ptr(out), N, M, N, K, mode, bm, ops._stream()) == 0
+        close(out, want, BF16_EPS)
+    sums = torch.full((M, N), float("nan"), device=DEV)
+    assert ops.lib.fllm_linear_tiles(ptr(x), K, ptr(w), None, ptr(sums), N, M, N, K, 1, bm, ops._stream()) == 0
+    close(sums, gate, 1e-4)
 
 
 @pytest.mark.parametrize("M,N,K", [(200, 264, 192), (140, 1032, 320)])
@@ -114,3 +137,32 @@ def test_experts_on_large_tiles(ops, rows, width, inter, experts, top, spread, g
     # two steps of the largest output (the largest activation times the largest weight is below twice that output)
     off = (out.cpu().double() - want).abs()
     assert (off <= 2 * BF16_EPS * (want.abs() + want.abs().max())).all() and off.norm() <= 1e-3 * want.norm()
+
+
+@pytest.mark.parametrize("gated,inter", [(True, 2048), (False, 4096)])
+@pytest.mark.parametrize("rows", [3000, 3840])      # tiles of 128 rows and of 256 take fewer rounds
+def test_experts_with_more_tiles_than_workgroups(ops, rows, gated, inter):
+    """6,000 and 7,680 pairs of four experts: 300 to 800 tiles in either product, the last of an expert ragged."""
+    g = torch.Generator().manual_seed(rows)
+    bf, experts, top, width = torch.bfloat16, 4, 2, 3072
+    h = torch.randn(rows, width, generator=g).to(bf).to(DEV)
+    w_up = (torch.randn(experts, (2 if gated else 1) * inter, width, generator=g) * 2 * width ** -0.5).to(bf).to(DEV)
+    w_down = (torch.randn(experts, width, inter, generator=g) * inter ** -0.5).to(bf).to(DEV)
+    ids = torch.stack([torch.randperm(experts, generator=g)[:top] for _ in range(rows)]).to(torch.int32).to(DEV)
+    weights = torch.rand(rows, top, generator=g).to(DEV)
+    out = torch.full((rows * top, width), float("nan"), device=DEV)
+    if gated:
+        assert ops.experts_grouped(h, ids, weights, w_up, w_down, out)
+    else:
+        assert ops.experts_grouped_ungated(h, ids, w_up, w_down, out)
+    flat = ids.reshape(-1).long()
+    for e in range(experts):
+        at = torch.nonzero(flat == e).flatten()
+        x = h[at // top]
+        if gated:
+            x = (x.float() * weights.reshape(-1)[at][:, None]).to(bf)
+        y = x.double() @ w_up[e].double().T
+        act = torch.nn.functional.silu(y[:, :inter]) * y[:, inter:] if gated else y.clamp(min=0) ** 2
+        want = act.to(bf).double() @ w_down[e].double().T
+        off = (out[at].double() - want).abs()               # the bound of the test above
+        assert (off <= 2 * BF16_EPS * (want.abs() + want.abs().max())).all() and off.norm() <= 1e-3 * want.norm()

@@ -139,3 +139,44 @@ def test_embedding_and_head_parts(rt):
     logits = head.forward(None, h.to(DEV))
     assert logits.dtype == torch.float32
     compare(logits, h.double().numpy() @ w["weight"].double().numpy().T, rt, "head")
+
+
+@pytest.mark.parametrize("rows", [1, 20, 70, 400])
+def test_a_shared_expert_stores_the_branch_and_the_picks_join_it(rt, rows):
+    """Experts with their weights on the outputs beside a shared one: a stored branch (whatever it held) is the shared expert's output plus the
+    weighted sum of the picks, the same as what is added to a stream; without a shared expert there is nothing to store."""
+    from reference_ops import ReferenceOps
+    hidden, inter, shared, experts, top = 256, 288, 512, 6, 2
+    params = {"hidden_size": hidden, "intermediate_size": inter, "experts": experts, "top": top, "score": "sigmoid", "renormalize": True, "route_scale": 1.5,
+              "weight_on": "output", "gated": False, "groups": 3, "groups_kept": 2, "shared": shared}
+    names = {"router": "r", "correction": "c", "shared_up": "su", "shared_down": "sd"}
+    names.update({f"{kind}_{e}": f"{kind}{e}" for kind in ("up", "down") for e in range(experts)})
+    spec = PartSpec("routed_experts", params, names)
+    w = weights_for("feed_forward", spec, 5, rt.dtype)
+    part = part_class("feed_forward", "routed_experts")(spec, w, rt)
+    assert part.stores_branch and part.branch_parts == 1
+    h = torch.randn(rows, hidden, generator=torch.Generator().manual_seed(rows)).to(rt.dtype)
+    branch = torch.full((rows, hidden), float("nan"), device=DEV)
+    part.forward(None, h.to(DEV), None, branch=branch)
+    stream = torch.zeros((rows, hidden), device=DEV)
+    part.forward(None, h.to(DEV), stream)
+
+    double = {name: t.to(rt.dtype).double() if name != "correction" else t for name, t in w.items()}
+    ids, weights = torch.empty((rows, top), dtype=torch.int32), torch.empty((rows, top))
+    ReferenceOps().route_grouped(h, double["router"], w["correction"], top, 3, 2, ids, weights, route_scale=1.5)
+    x = h.double()
+    want = (torch.clamp(x @ double["shared_up"].T, min=0.0) ** 2) @ double["shared_down"].T
+    for r in range(rows):
+        for k in range(top):
+            e = int(ids[r, k])
+            want[r] += weights[r, k].double() * (double[f"down_{e}"] @ torch.clamp(double[f"up_{e}"] @ x[r], min=0.0) ** 2)
+    # the activations are rounded once (2^-9 each, signs at random), in prompts a product that is added is rounded once more
+    scale = want.abs().max()
+    limit = 3e-5 if rt.dtype == torch.float32 else 2.0 ** -7
+    for got in (branch, stream):
+        assert (got.double().cpu() - want).abs().max() <= limit * scale
+    bare = dict(params, shared=0)
+    alone = part_class("feed_forward", "routed_experts")(PartSpec("routed_experts", bare, {n: v for n, v in names.items() if "shared" not in n}), w, rt)
+    assert not alone.stores_branch
+    with pytest.raises(ValueError, match="no stored branch"):
+        alone.forward(None, h.to(DEV), None, branch=branch)

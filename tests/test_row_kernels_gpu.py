@@ -1,6 +1,6 @@
 """The forms of the row kernels that read everything a row needs in one round of loads (bfloat16, pieces of 4 and 8 lanes), against the
-plain forms of the same entry points, which an operand that begins off a 16-byte boundary selects: widths of one piece, of a whole
-round of the workgroup and one more, heads whose threads fill no power of two, every norm, rotations of part of a head, padding rows."""
+plain forms of the same entry points, which an operand that begins off a 16-byte boundary selects, and against float64: widths of one piece, of
+a whole round of the workgroup and one more, heads whose threads fill no power of two, every norm, rotations of part of a head, padding rows."""
 import pytest
 import torch
 
@@ -180,3 +180,104 @@ def test_allow_lists_that_do_not_rise_stay_inside_their_row(ops):
         assert torch.equal(got[0], logits[0]) and torch.equal(got[2], logits[2])
         assert (got[1, blocked] == float("-inf")).all()
         assert all(got[1, t] in (logits[1, t], float("-inf")) for t in listed)
+
+
+def near(got, exact):
+    """Against float64: one rounding to bfloat16 (at most 2^-8 of the value; a float32 result has none that counts) behind sums of up to 32,768
+    float32 terms, whose errors stay below 2^-18 of the largest value."""
+    eps = 2.0 ** -8 if got.dtype == torch.bfloat16 else 0.0
+    got, exact = got.double().cpu(), exact.double()
+    assert ((got - exact).abs() <= eps * exact.abs() + 2.0 ** -18 * exact.abs().max()).all(), ((got - exact).abs() / exact.abs().max()).max()
+
+
+@pytest.mark.parametrize("rows,width,experts,top,score", [(1, 8, 8, 2, "sigmoid"), (5, 1536, 8, 2, "softmax"), (3, 2056, 70, 5, "sigmoid"), (2, 512, 3, 3, "softmax")])
+def test_routers_against_float64(ops, rows, width, experts, top, score):
+    from reference_ops import ReferenceOps
+    g = torch.Generator().manual_seed(width + 1)
+    h = torch.randn(rows, width, generator=g).to(torch.bfloat16)
+    w = (torch.randn(experts, width, generator=g) * width ** -0.5 * 2).to(torch.bfloat16)
+    correction = torch.rand(experts, generator=g)
+    groups = 2 if experts % 2 == 0 else 1
+    new = lambda d: (torch.empty(rows, top, dtype=torch.int32, device=d), torch.empty(rows, top, device=d))
+    for call in (lambda o, d, out: o.route_topk(h.to(d), w.to(d), top, *out, score=score, renormalize=True, route_scale=2.5),
+                 lambda o, d, out: o.route_grouped(h.to(d), w.to(d), correction.to(d), top, groups, groups, *out, route_scale=2.5)):
+        got, want = new(DEV), new("cpu")
+        call(ops, DEV, got)
+        call(ReferenceOps(), "cpu", want)
+        assert torch.equal(got[0].cpu(), want[0])
+        torch.testing.assert_close(got[1].cpu(), want[1], rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("rows,width", [(3, 4), (2, 1024), (1, 1028), (5, 1536), (2, 4096), (2, 4100)])
+@pytest.mark.parametrize("weighted,normed,nexts", [(True, True, torch.bfloat16), (False, False, torch.float32), (True, False, None)])
+def test_sums_of_normed_branches_against_float64(ops, rows, width, parts, weighted, normed, nexts):
+    from reference_ops import ReferenceOps
+    g = torch.Generator().manual_seed(parts * 11 + width)
+    x, branch, gain, pw, nw = (torch.randn(*s, generator=g) for s in ((rows, width), (rows * parts, width), (width,), (rows, parts), (width,)))
+    results = []
+    for o, d, of in ((ops, DEV, lambda t: t), (ReferenceOps(), "cpu", lambda t: t.double())):
+        y = of(x.to(d, copy=True))
+        nxt = None if nexts is None else torch.empty(rows, width, dtype=nexts if d == DEV else torch.float64, device=d)
+        o.postnorm_add(y, of(branch.to(d)), of(gain.to(d)), 1e-5 if normed else None, parts=parts, part_weights=of(pw.to(d)) if weighted else None,
+                       next_weight=None if nexts is None else of(nw.to(d)), next_eps=1e-6, next_out=nxt)
+        results.append((y, nxt))
+    near(results[0][0], results[1][0])
+    if nexts is not None:
+        near(results[0][1], results[1][1])
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("heads,kv_heads,k_dim,v_dim,rope,keys_are_values", [(12, 2, 128, 128, 128, False), (3, 1, 24, 40, 16, False), (5, 5, 512, 512, 256, True),
+                                                                             (20, 4, 64, 32, 0, False)])
+def test_normed_and_rotated_heads_against_float64(ops, mode, heads, kv_heads, k_dim, v_dim, rope, keys_are_values):
+    from reference_ops import ReferenceOps
+    g = torch.Generator().manual_seed(heads * k_dim + mode + 1)
+    rows, page, pages = 5, 16, 4
+    wide = heads * k_dim + kv_heads * (k_dim + (0 if keys_are_values else v_dim))
+    qkv = torch.randn(rows, wide + 8, generator=g).to(torch.bfloat16)
+    qw, kw = (1.0 + 0.1 * torch.randn(n * k_dim if mode == 2 else k_dim, generator=g) for n in (heads, kv_heads))
+    angles = torch.rand(64, rope // 2, generator=g) * 6.0
+    cos, sin = torch.cos(angles).contiguous(), torch.sin(angles).contiguous()
+    pos, seg = torch.tensor([0, 15, 16, 37, 5], dtype=torch.int32), torch.tensor([0, 0, 1, 1, -1], dtype=torch.int32)
+    tables = torch.tensor([[3, 1, 0], [2, 0, 1]], dtype=torch.int32)
+    blend = None if keys_are_values else torch.randn(rows, kv_heads * v_dim, generator=g).to(torch.bfloat16)
+    amount = torch.tensor([0.3])
+    results = []
+    for o, d, kind in ((ops, DEV, torch.bfloat16), (ReferenceOps(), "cpu", torch.float64)):
+        at = lambda t: None if t is None else t.to(d)
+        q = torch.zeros(rows, heads * k_dim, dtype=kind, device=d)
+        k = torch.zeros(pages, kv_heads, k_dim // 8, page, 8, dtype=kind, device=d)
+        v = torch.zeros(pages, kv_heads, v_dim, page, dtype=kind, device=d)
+        o.normed_rope_store(at(qkv if d == DEV else qkv.double()), mode, at(qw) if mode else None, at(kw) if mode else None, 1e-5, q, at(pos), at(seg), at(tables),
+                            at(cos), at(sin), k, v, heads, kv_heads, k_dim, v_dim, rope, page, 8, values_from_keys=keys_are_values,
+                            blend=at(blend), blend_amount=at(amount) if blend is not None else None)
+        results.append((q[:4], k, v))
+    for a, b in zip(*results):
+        near(a, b)
+
+
+@pytest.mark.parametrize("x_type", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,width,weighted", [(1, 4, True), (3, 1536, True), (2, 2052, False), (2, 8192, True)])
+def test_gated_norms_against_float64(ops, rows, width, weighted, x_type):
+    from reference_ops import ReferenceOps
+    g = torch.Generator().manual_seed(width + 1)
+    x, w = torch.randn(rows, width, generator=g).to(x_type), torch.randn(width, generator=g) if weighted else None
+    gate = torch.randn(rows, width + 12, generator=g).to(torch.bfloat16)[:, 12:]
+    got, want = torch.empty(rows, width, dtype=torch.bfloat16, device=DEV), torch.empty(rows, width, dtype=torch.float64)
+    wide = torch.zeros(rows, width + 12, dtype=torch.bfloat16, device=DEV)
+    wide[:, 12:] = gate.to(DEV)
+    ops.gated_norm(x.to(DEV), w.to(DEV) if weighted else None, 1e-5, wide[:, 12:], got)
+    ReferenceOps().gated_norm(x, w, 1e-5, gate, want)
+    near(got, want)
+
+
+@pytest.mark.parametrize("rows,width", [(1, 8), (3, 8960), (2, 16392), (1, 32768)])
+def test_polynomial_activation_against_float64(ops, rows, width):
+    from reference_ops import ReferenceOps
+    z = torch.randn(rows, width, generator=torch.Generator().manual_seed(width + 1)).to(torch.bfloat16)
+    coeffs = torch.tensor([0.7, -0.4, 0.2, 0.1])
+    got, want = torch.empty(rows, width, dtype=torch.bfloat16, device=DEV), torch.empty(rows, width, dtype=torch.float64)
+    ops.polynorm(z.to(DEV), coeffs.to(DEV), 1e-5, got)
+    ReferenceOps().polynorm(z, coeffs, 1e-5, want)
+    near(got, want)
