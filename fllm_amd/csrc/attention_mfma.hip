@@ -18,9 +18,10 @@
 //                  while the current one is multiplied (described at the kernel); faster than the tile kernel
 //                  for portions of any length.  Few rows over long contexts: several workgroups share a row
 //                  tile's keys and the one that arrives last adds their parts up.
-//   decode kernel  one row per segment: a workgroup takes (row, key/value head, context split), its
-//                  sixteen waves stride over 32-key blocks loading K and V^T straight into MFMA
-//                  operands; long contexts of small batches are split and merged by a second kernel.
+//   decode kernel  one row per segment: a workgroup takes (row, key/value head, context split), its four
+//                  waves (heads narrower than 128: eight) stride over blocks of 64 keys, K and V^T
+//                  straight into MFMA operands; contexts that are split are merged by the split that
+//                  arrives last, or by a second kernel where there is no device workspace.
 #include <algorithm>
 #include "api.h"
 #include "common.h"

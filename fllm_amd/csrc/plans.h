@@ -117,7 +117,11 @@ inline ChunkPlan plan_chunks(int K, int ntiles, int mt, int rt, size_t ws_bytes,
     return p;
 }
 // What the busiest compute unit streams under a plan, in weight rows x columns: its workgroups' row tiles over their
-// slices, as often as the row groups of a slice come round.
+// slices, as often as the row groups of a slice come round.  Workgroups that are no more than the compute units have one
+// each, also where two of four waves would fit: their tiles then spread over more units than those of seven waves would
+// (microseconds of seven waves and of four, with the same slices, weights from memory, at 49 / 64 rows: 2,048 x 8,192
+// 21.3 -> 18.7 / 21.9 -> 19.6, 2,048 x 14,336 28.3 -> 23.6 / 28.8 -> 24.1, 4,096 x 2,048 15.4 -> 14.1 / 15.9 -> 14.8, 6,144 x 1,024 13.8 ->
+// 12.6 / 14.3 -> 13.0; gate/up of 2 x 4,096 x 1,024 15.8 -> 13.9 / 16.0 -> 14.0, of 2 x 2,048 x 2,048 17.4 -> 15.6 / 17.6 -> 15.8).
 inline long chunk_plan_cost(const ChunkPlan &p, int ntiles, int cus) {
     const int ngroups = (ntiles + p.waves - 1) / p.waves;
     const int per_slice = p.grid / p.S;

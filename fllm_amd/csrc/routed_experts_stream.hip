@@ -8,7 +8,7 @@
 // cut K between them with 6 to 12 KiB asked for at a time each, and they meet in LDS once.  A load of the tile-major copy is
 // 1 KiB in a row, whole cache lines that carry the non-temporal hint; the same kernel reading the rows as the checkpoint has them
 // (64 bytes of each of 16) runs at 4.4 instead of 5.9 TB/s, and through LDS in whole rows, a tile at a time, at 4.0.
-// An expert's weights serve up to 64 pairs from registers.
+// A load of an expert's weights serves up to 32 pairs from registers.
 //
 // MFMA operand layout (v_mfma_f32_16x16x32_bf16): A lane l holds A[m = l%16][k = 8*(l/16) .. +7]; B likewise with n = l%16;
 // D lane l holds D[m = 4*(l/16) + i][n = l%16], i = 0..3.
