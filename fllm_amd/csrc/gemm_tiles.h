@@ -21,7 +21,7 @@
 
 namespace fllm_tiles {
 
-enum { EPI_STORE = 0, EPI_GLU = 1, EPI_RELU2 = 2, EPI_F32 = 3 };
+enum { EPI_STORE = 0, EPI_GLU = 1, EPI_RELU2 = 2, EPI_F32 = 3 };      // EPI_F32: grouped products alone
 
 struct TileArgs {
     const bf16_t *x;        // rows, row stride ldx (a multiple of 8)

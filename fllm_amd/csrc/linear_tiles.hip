@@ -43,7 +43,7 @@ extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up,
     return launch_tiles<EPI_GLU, false>(a, bm, tiles, stream);
 }
 
-// mode 0: out bfloat16 = x w^T (+ bias); 1: out float32 = x w^T; 2: out bfloat16 = relu(x w^T)^2.
+// mode 0: out = x w^T (+ bias); 2: out = relu(x w^T)^2; bfloat16.
 //
 // The squared ReLU against the library's product and a kernel of its own (13,312 x 1,536): 31 -> 23 us at 512 rows, 87 -> 68 at 2,048; fewer rows
 // as above.  A bias (2,048 x 1,536; the general path is linear_tiled_mfma_kernel): 32 -> 23 us at 136 rows, 34 -> 24 at 2,048.  Without either
@@ -52,7 +52,7 @@ extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up,
 // 2,048 rows 59 -> 55; 6,144 x 4,096 at 2,048 rows (192 of 256 rows) 80 -> 77, at 1,900 76 -> 78.  Hence nine tenths of the last round.
 extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const float *bias, void *out, int ldo, int M, int N, int K, int mode,
                                  int force, hipStream_t stream) {
-    FLLM_REQUIRE(M >= 0 && N > 0 && K > 0 && ldx >= K && ldo >= N && x && w && out && mode >= 0 && mode <= 2,
+    FLLM_REQUIRE(M >= 0 && N > 0 && K > 0 && ldx >= K && ldo >= N && x && w && out && (mode == 0 || mode == 2),
                  "linear_tiles: bad sizes or operands missing");
     if (!fllm_fast_kernels_enabled() || (bias && mode != 0) || !operands_fit(x, ldx, w, out, ldo, M, N, N, K)) return 1;
     if (M == 0) return 0;
@@ -63,8 +63,7 @@ extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const fl
     a.bias = bias;
     const long tiles = bm == 256 ? t256 : t128, slots = (tiles + 255) / 256 * 256;
     if (!force && mode == 2 && !fllm_plan::activation_joins(M, N, K, bm, tiles)) return 1;
-    if (!force && mode != 2 && !bias && (K < 2048 || 10 * tiles < 9 * slots)) return 1;
+    if (!force && mode == 0 && !bias && (K < 2048 || 10 * tiles < 9 * slots)) return 1;
     if (mode == 0) return launch_tiles<EPI_STORE, false>(a, bm, tiles, stream);
-    if (mode == 1) return launch_tiles<EPI_F32, false>(a, bm, tiles, stream);
     return launch_tiles<EPI_RELU2, false>(a, bm, tiles, stream);
 }
