@@ -648,9 +648,11 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
 // the tile; the wave that counts the last slice adds the S partial sums in slice order and runs
 // the epilogue (as in the resident kernel), up to 48 rows with the parts and the operands of all row
 // tiles in one trip to memory.  What bounds it: the weights' bytes in large matrices, the trips that
-// follow each other in small ones.  At 40 rows, against one chunk ahead, a trip a row tile and slices
-// for two workgroups a compute unit: 4,096 x 4,096 17.8 -> 14.3 us, 4,096 x 14,336 29.3 -> 26.1 (4.5 TB/s),
-// 6,144 x 4,096 23.2 -> 22.0, gate/up of 2 x 14,336 x 4,096 44.9 -> 41.7, of 2 x 8,192 x 2,048 23.9 -> 17.1.
+// follow each other in small ones.  At 40 rows, against one chunk ahead, a trip a row tile and slices for two workgroups a
+// compute unit: 4,096 x 4,096 16.6 -> 13.3 us, 4,096 x 14,336 29.9 -> 27.4 (4.3 TB/s), 6,144 x 4,096 19.2 -> 17.1, gate/up of
+// 2 x 14,336 x 4,096 47.7 -> 44.6, of 2 x 8,192 x 2,048 22.8 -> 16.5.  The parts of a group of slices have to be asked for ahead of a
+// barrier for the compiler, which otherwise fetches and awaits them two at a time: 4,096 x 4,096 at 40 / 64 / 128 rows 13.6 -> 13.3 / 20.3 ->
+// 18.3 / 30.7 -> 28.5, 2,048 x 8,192 15.5 -> 15.0 / 19.5 -> 17.3 / 35.7 -> 32.0.
 // WT: the weights come from their tile-major copy (fllm_tile_weights, fllm_tile_weights_gate_up), K a multiple of 256.
 // PRO_SCALED: the rows are what the product before prepared for an RMSNorm (fllm_linear_add_normed); the row's scale,
 // from the parts of its sum of squares, multiplies the finished sums.
@@ -911,6 +913,7 @@ skinny_wide_kernel(SkinnyArgs a) {
                         for (int t = 0; t < RT; t++) pv[j][mt][t] = take_over(wsb, src + t * kWave * 16);
                     }
                 }
+                __builtin_amdgcn_sched_barrier(0);      // left alone, the compiler fetches two at a time and waits in between
 #pragma unroll
                 for (int j = 0; j < GRP; j++)
 #pragma unroll

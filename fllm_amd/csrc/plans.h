@@ -92,8 +92,9 @@ inline ChunkPlan plan_chunks(int K, int ntiles, int mt, int rt, size_t ws_bytes,
     const int slots = 8 / waves * cus;
     // K slices: as many as fill the chip with the row groups there are, each at least two chunks long.  Up to 48 rows a
     // workgroup has enough on its way for a compute unit of its own, and more slices only cost their sums' way through
-    // memory (40 rows, with one workgroup a unit and with two: 4,096 x 4,096 14.4 and 17.5 us, 4,096 x 14,336 26.4 and
-    // 29.3; with 49 to 64 rows two are no slower).
+    // memory (40 rows, with one workgroup a unit and with two: 4,096 x 4,096 13.3 and 16.2 us, 4,096 x 14,336 28.0 and
+    // 29.6).  49 to 64 rows keep two; one is faster for sums into the stream (64 rows: 16.1 and 18.4, 30.3 and 32.7), their
+    // other epilogues were not measured with it.
     const int fill = mt <= 3 ? cus : slots;
     int S = 1;
     while (S < 8 && ngroups * S * 2 <= fill && (K + 2 * S - 1) / (2 * S) >= 512) S *= 2;
@@ -120,8 +121,8 @@ inline ChunkPlan plan_chunks(int K, int ntiles, int mt, int rt, size_t ws_bytes,
 // slices, as often as the row groups of a slice come round.  Workgroups that are no more than the compute units have one
 // each, also where two of four waves would fit: their tiles then spread over more units than those of seven waves would
 // (microseconds of seven waves and of four, with the same slices, weights from memory, at 49 / 64 rows: 2,048 x 8,192
-// 21.3 -> 18.7 / 21.9 -> 19.6, 2,048 x 14,336 28.3 -> 23.6 / 28.8 -> 24.1, 4,096 x 2,048 15.4 -> 14.1 / 15.9 -> 14.8, 6,144 x 1,024 13.8 ->
-// 12.6 / 14.3 -> 13.0; gate/up of 2 x 4,096 x 1,024 15.8 -> 13.9 / 16.0 -> 14.0, of 2 x 2,048 x 2,048 17.4 -> 15.6 / 17.6 -> 15.8).
+// 19.1 -> 16.5 / 19.6 -> 17.3, 2,048 x 14,336 26.2 -> 21.3 / 26.5 -> 21.7, 4,096 x 2,048 14.3 -> 12.9 / 14.7 -> 13.5, 6,144 x 1,024 13.2 ->
+// 11.9 / 13.6 -> 12.3; gate/up of 2 x 4,096 x 1,024 14.7 -> 12.6 / 14.8 -> 12.8, of 2 x 2,048 x 2,048 15.3 -> 13.2 / 15.4 -> 13.7).
 inline long chunk_plan_cost(const ChunkPlan &p, int ntiles, int cus) {
     const int ngroups = (ntiles + p.waves - 1) / p.waves;
     const int per_slice = p.grid / p.S;
