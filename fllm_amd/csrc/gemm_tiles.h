@@ -10,9 +10,10 @@
 // the lanes of an operand then meet every bank once.  Rows of W are dealt to LDS so that a lane ends up with 8 neighbouring columns (a
 // 16-byte store); a workgroup asks for its next tile's first steps before it stores the last one.
 //
-// Measured (one MI355X, random operands, weights from memory, beside the GEMM library's best): 8,192 x 8,192 x 8,192 705 us (1.56 PFLOP/s,
-// library 690); 2,048 x 28,672 x 4,096 with the SwiGLU in the epilogue 345 us (1.40; library 345 and a SwiGLU kernel of 22 to 29);
-// 2,048 x 4,096 x 14,336 as 128-row tiles 188 us (1.28; library 206), as 256-row tiles 255 (half of the compute units).
+// Measured (one MI355X, random operands, weights from memory, launches that follow one another, beside the GEMM library; boxes differ by
+// 5 %): 8,192 x 8,192 x 8,192 720 us (1.53 PFLOP/s, library 703); 2,048 x 28,672 x 4,096 with the SwiGLU in the epilogue 361 to 382 us (1.33 to
+// 1.26; library and a SwiGLU kernel 382 to 422), in a model's prompt step 362; 2,048 x 4,096 x 14,336 as 128-row tiles 197 us (1.22; library
+// 217), as 256-row tiles 257 (half of the compute units).
 //
 // MFMA operand layout (v_mfma_f32_16x16x32_bf16): A lane l holds A[m = l%16][k = 8*(l/16) .. +7]; B likewise with n = l%16; D lane l holds
 // D[m = 4*(l/16) + i][n = l%16], i = 0..3.  A is W here, B the rows of x.

@@ -26,9 +26,9 @@ long tiles_of(long M, int bm, int N, int cols) { return (M + bm - 1) / bm * ((N 
 // 0: launched, negative: error, 1: declined (the shape, or with `force` 0 a shape that the general path is faster at; `force` 256 or 128
 // asks for that row tile and is declined where K is too short for it or no whole steps, as is any value but 0, 1 and these).
 //
-// The fused product against the library's product and an activation kernel, microseconds at 512 / 1,024 / 2,048 rows: 2 x 14,336 x 4,096
-// 106 -> 95 / 203 -> 183 / 378 -> 356; 2 x 8,192 x 2,048 41 -> 32 / 65 -> 54 / 120 -> 106; 2 x 8,960 x 1,536 42 -> 36 / 75 -> 67 / 132 -> 115;
-// 2 x 4,096 x 1,024 26 -> 17 / 29 -> 20 / 42 -> 35.  Where few rows or half-empty rounds make it slower: activation_joins in plans.h.
+// The fused product against the library's product and an activation kernel, inside a graph, weights from memory, microseconds at 512 /
+// 1,024 / 2,048 rows: 2 x 14,336 x 4,096 116 -> 104 / 212 -> 191 / 382 -> 361; 2 x 8,192 x 2,048 43 -> 37 / 69 -> 59 / 121 -> 111; 2 x 8,960 x 1,536
+// 45 -> 43 / 79 -> 72 / 137 -> 118; 2 x 4,096 x 1,024 20 -> 18 / 27 -> 21 / 42 -> 35.  Where few rows or half-empty rounds make it slower: activation_joins in plans.h.
 extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up, void *out, int M, int inter, int K, float limit, float alpha,
                                   float up_offset, int force, hipStream_t stream) {
     FLLM_REQUIRE(M >= 0 && inter > 0 && K > 0 && ldx >= K && x && w_gate_up && out, "gate_up_tiles: bad sizes or operands missing");
@@ -45,7 +45,7 @@ extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up,
 
 // mode 0: out = x w^T (+ bias); 2: out = relu(x w^T)^2; bfloat16.
 //
-// The squared ReLU against the library's product and a kernel of its own (13,312 x 1,536): 31 -> 23 us at 512 rows, 87 -> 68 at 2,048; fewer rows
+// The squared ReLU against the library's product and a kernel of its own (13,312 x 1,536): 37 -> 28 us at 512 rows, 95 -> 79 at 2,048; fewer rows
 // as above.  A bias (2,048 x 1,536; the general path is linear_tiled_mfma_kernel): 32 -> 23 us at 136 rows, 34 -> 24 at 2,048.  Without either
 // the library has kernels for every tile of the device's time, and these tiles are ahead only where they fill whole rounds over the compute
 // units: 4,096 x 14,336 at 2,048 rows (256 tiles) 207 -> 188 us, at 1,900 (240) 191 -> 182, at 1,536 (192) 167 -> 177; 4,096 x 4,096 at
