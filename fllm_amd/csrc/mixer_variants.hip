@@ -622,8 +622,10 @@ __global__ void __launch_bounds__(kBlock) relu_squared_vec_kernel(const bf16_t *
 // normed_rope_store for bfloat16 rows, eight neighbouring lanes a thread: everything the row needs (the lanes, the ones they turn with,
 // weights, angles, the other layer's values) is asked for at once, so that a row waits for memory once behind its position.  One workgroup a
 // row; a head's `lanes` threads (a power of two) lie side by side.  Lane by lane, with a wait a step, a row of 12 + 2 heads of 128 took
-// 13.0 us in a decode step of two rows; like this 5.5.
+// 13.0 us in a decode step of two rows; like this 5.5.  TURNS false, no rotation: a kernel of its own, so that a row neither waits for nor
+// holds what a rotation needs (a step of one row of 12 + 2 heads of 128 6.1 us with the question asked in the kernel, 4.8 like this).
 // norm_mode as in normed_rope_store_kernel; rope_dims / 2 a multiple of 8.
+template <bool TURNS>
 __global__ void __launch_bounds__(kBlock)
 normed_rope_store_vec_kernel(const bf16_t *__restrict__ qkv, int ld, int norm_mode, const float *__restrict__ q_weight,
                              const float *__restrict__ k_weight, float eps, bf16_t *__restrict__ q_out, const int32_t *__restrict__ row_pos,
@@ -637,7 +639,7 @@ normed_rope_store_vec_kernel(const bf16_t *__restrict__ qkv, int ld, int norm_mo
     const int seg = row_seg[r], pos = row_pos[r];
     const bf16_t *row = qkv + r * ld;
     const int each = kBlock / lanes, c = (threadIdx.x % lanes) * 8, half = rope_dims / 2;
-    const bool turns = c < rope_dims;
+    const bool turns = TURNS && c < rope_dims;
     const int pc = c < half ? c + half : c - half;              // the lanes that these turn with
     const int all = heads + kv_heads;
     float inv_q = 1.f, inv_k = 1.f;
@@ -751,8 +753,9 @@ int fllm_launch_normed_rope_store(const void *qkv, int ld, int norm_mode, const 
         blend_ld % 8 == 0 && (bases & 15) == 0) {
         int lanes = 1;
         while (lanes < k_dim / 8) lanes *= 2;
-        hipLaunchKernelGGL(normed_rope_store_vec_kernel, dim3(rows), dim3(kBlock), 0, stream, (const bf16_t *)qkv, ld, norm_mode, q_weight, k_weight,
-                           eps, (bf16_t *)q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table, (bf16_t *)k_pages,
+        const auto kernel = rope_dims > 0 ? normed_rope_store_vec_kernel<true> : normed_rope_store_vec_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3(rows), dim3(kBlock), 0, stream, (const bf16_t *)qkv, ld, norm_mode, q_weight, k_weight, eps,
+                           (bf16_t *)q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table, (bf16_t *)k_pages,
                            (bf16_t *)v_pages, heads, kv_heads, k_dim, v_dim, rope_dims, page_size, store_kv, values_from_keys,
                            (const bf16_t *)blend, blend_ld, blend_amount, lanes);
         return fllm_check_launch("normed_rope_store");
