@@ -1,29 +1,36 @@
 // Matrix-core form of the attention whose heads talk to each other (talking_attention.hip says what is computed),
 // bfloat16 operands, float32 scores, statistics and sums.
 //
-// A workgroup of four waves takes 16 consecutive rows of one request (a prompt portion's row tile, or a decode step's
-// single row) with ALL heads, because a mixed score needs every head's raw score of the same (row, key).  It walks the
-// keys the tile sees in blocks of 64; with `splits` > 1 the blocks of a tile are dealt out to that many workgroups,
-// which leave their running maxima, sums and unnormalised outputs in a workspace that a second kernel merges (few row
-// tiles would otherwise leave most of the 256 compute units idle: a decode step has one tile a request).
+// A workgroup of eight waves takes 16 consecutive rows of one request (a prompt portion's row tile) with ALL heads, because a
+// mixed score needs every head's raw score of the same (row, key).  It walks the keys the tile sees in blocks of 128; the
+// blocks of a tile are dealt out in runs of `share_blocks` to several workgroups where a launch has few tiles, which leave
+// their running maxima, sums and unnormalised outputs in a workspace that a second kernel merges.  (Decode steps, one row a
+// request, have a kernel of their own further down.)
 //
-// Keys and values pass through LDS, one key/value head at a time (a "stage": 64 keys x k_dim, then 64 keys x v_dim):
-// all threads load the stage after the next one into registers while the waves multiply from the stage in LDS, so the
-// latency of the pages is hidden behind the products and LDS holds one head's block however many heads there are.
-// The products are the transposed ones, v_mfma_f32_16x16x32_bf16 with D[m = 4 (l / 16) + i][n = l % 16], so that a
+// Keys and values go straight from the pages into operands: a wave's 16 keys and a wave's 16 value lanes serve that wave
+// alone, so a pass through LDS would share nothing.  What the waves share lies in LDS: the tile's queries, a block's maxima and
+// its weights.  The products are the transposed ones, v_mfma_f32_16x16x32_bf16 with D[m = 4 (l / 16) + i][n = l % 16], so that a
 // lane keeps one row throughout:
 //
 //   1. wave w takes the block's keys 16 w .. 16 w + 15: for every head  raw_g^T[key][row] = K_{g / group} Q_g^T
-//      (A = 16 keys x 32 lanes from the stage, B = the rows' queries from LDS).  A lane then holds, for its four
-//      (key, row) pairs, the raw scores of all heads: the mix  s_h = sum_g talk'[h, g] raw_g  is lane-local
-//      (talk'[h, g] = talk[h, g] * scale * temp[g], prepared in LDS once).
-//   2. the block's largest score a (head, row) goes through LDS (four waves hold different keys); every wave computes
+//      (A = 16 keys x 32 lanes, B = the rows' queries from LDS).  A lane then holds, for its four (key, row) pairs, the raw
+//      scores of all heads: the mix  s_h = sum_g talk[h, g] (raw_g * scale * temp[g])  is lane-local, its factors come
+//      through the scalar cache.
+//   2. the block's largest score a (head, row) goes through LDS (eight waves hold different keys); every wave computes
 //      the same running maximum, weighs its scores, keeps its share of the running sum and leaves the weights in LDS
-//      as bfloat16, [head][key group][row][16 keys].
-//   3. the outputs  O_h^T[lane of v][row] += V_{h / group}^T P_h^T: wave w owns the value lanes 16 w .. 16 w + 15 and
-//      64 + 16 w .. of every head, so a value fragment (A) is read once a key/value head and serves its whole group;
-//      B = weights from LDS.  The k slots of this product hold the keys 4 g + i of two key groups, the order step 2
-//      left them in.
+//      as bfloat16, [head][row][128 keys] with a row's 16-byte pieces XORed by the row (16 rows at one place of the row
+//      would meet in the same banks).
+//   3. the outputs  O_h^T[lane of v][row] += V_{h / group}^T P_h^T: wave w owns the value lanes 16 (w % n) .. of every
+//      head, n = v_dim / 16 rounded up to a power of two; where n < 8 the heads are dealt out among the waves of one n.
+// The keys of the next block and the values of the next key/value head are on their way while this one is multiplied, and
+// page numbers a block earlier still; two barriers a block.
+//
+// What bounds it: vector instructions (the mix alone is H^2 multiply-adds a (row, key) pair) and LDS reads (queries and
+// weights, one 16-byte read a product).  Before, four waves held both value halves and staged keys and values through LDS
+// in two stages a block of 64 keys: 416 to 512 registers a lane, so one wave a SIMD waited out every latency by itself.
+// 1,900 rows from a request's first token on, two key/value heads of 128 lanes: 8 heads 264 -> 48 us, 12 heads 338 -> 75, 16
+// heads 546 -> 139 (the last spills 68 registers); 2,048 rows behind 8,192 keys, 12 heads, 2,609 -> 442.  The general instance:
+// 12 heads on 4 of 64 lanes, 1,000 rows, 143 -> 88 us; 16 on 16 of 32 lanes 324 -> 186.
 //
 // Rows of a tile see different key ranges when a chunk of positions ends inside the tile: the mask is per (row, key).
 #include "api.h"
@@ -33,8 +40,9 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kTileRows = 16;
-constexpr int kKeyBlock = 64;
-constexpr int kVPitch = kKeyBlock + 4;      // a value lane's 64 keys in the stage, padded
+constexpr int kKeyBlock = 64;               // keys a step of the decode kernel
+constexpr int kTileThreads = 512;
+constexpr int kTileKeys = 128;              // keys a step of the tile kernel: 16 a wave
 
 struct TalkArgs {
     const bf16_t *q, *gate;
@@ -51,8 +59,8 @@ struct TalkArgs {
     int chunk;
     int splits;
     float *ws;       // splits > 1: [tile][split] { m [heads][16], l [heads][16], o [16][heads][v_dim] }
-    int gs;          // key/value heads a stage holds
-    int ptab;        // page numbers of a tile's keys that fit into LDS (0: they are read from the table in memory)
+    int page_shift;        // log2 of page_size, -1 where it is no power of two
+    int share_blocks;      // tile kernel: blocks of keys a workgroup takes
 };
 
 __device__ __forceinline__ size_t part_floats(int heads, int v_dim) { return (size_t)kTileRows * heads * (2 + v_dim); }
@@ -83,334 +91,311 @@ __device__ __forceinline__ bool find_tile(const TalkArgs &p, int tile, int *star
     return false;
 }
 
-template <int HMAX>
-__global__ void __launch_bounds__(kThreads)
-talking_tile_kernel(const TalkArgs p) {
-    constexpr int KSMAX = 8;       // k_dim <= 256
-    constexpr int TS = 2;          // v_dim <= 128: two 16-lane pieces a wave
-    constexpr int PRE = 8;         // 16-byte registers a thread holds of the stage in flight
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-    __shared__ float tk[HMAX * HMAX];
-    __shared__ float mx[4][HMAX][kTileRows];
-    __shared__ float al[HMAX][kTileRows];
-    __shared__ __attribute__((aligned(16))) bf16_t ps[HMAX][4][kTileRows][16];
+// Which blocks of 128 keys a tile sees, and how many workgroups share them.
+struct TileKeys {
+    int pos0, plast, kb_start, blocks, per_share, shares;
+};
+__device__ __forceinline__ TileKeys tile_keys(const TalkArgs &p, int first, int nrows) {
+    TileKeys t;
+    t.pos0 = p.row_pos[first];
+    t.plast = t.pos0 + nrows - 1;
+    t.kb_start = (p.chunk > 0 ? t.pos0 - t.pos0 % p.chunk : 0) & ~15;
+    t.blocks = (t.plast - t.kb_start) / kTileKeys + 1;
+    const int even = (t.blocks + p.splits - 1) / p.splits;      // more blocks than the caller's bound: dealt out evenly
+    t.per_share = even > p.share_blocks ? even : p.share_blocks;
+    t.shares = (t.blocks + t.per_share - 1) / t.per_share;
+    return t;
+}
 
-    const int H = p.heads, G = p.kv_heads, D = p.k_dim, DV = p.v_dim, PS = p.page_size;
-    const int group = H / G, KS = D / 32, DVT = DV / 16;
-    const int GS = p.gs, NST = (G + GS - 1) / GS;      // key/value heads a stage, stages of keys (and of values) a block
-    const int QP = H * D + 8, KP = GS * D + 8;
-    bf16_t *qs = (bf16_t *)lds_raw;
-    bf16_t *stage = qs + kTileRows * QP;
-    const size_t stage_elems = (size_t)kKeyBlock * KP > (size_t)GS * DV * kVPitch ? (size_t)kKeyBlock * KP : (size_t)GS * DV * kVPitch;
-    int *ptab = (int *)(stage + ((stage_elems + 7) & ~(size_t)7));
+typedef const __attribute__((address_space(4))) float *scalar_floats;      // read through the scalar cache
+
+// GS > 0: an instance for exactly HMAX heads on GS key/value heads, keys of 128 lanes, values of 80 to 128 and pages of a power
+// of two from 8 on, whose loops carry no conditions and whose key/value heads are unrolled.  GS 0: up to HMAX heads on any
+// number of key/value heads, any widths and pages of multiples of 4.
+template <int HMAX, int GS>
+__global__ void __launch_bounds__(kTileThreads)
+talking_tile_kernel(const TalkArgs p) {
+    constexpr bool EXACT = GS > 0;
+    constexpr int KSM = EXACT ? 4 : 8;         // k_dim <= 256
+    constexpr int NS = kTileKeys / 32;         // products over a block's keys
+    constexpr int UNROLL = EXACT ? GS : 1;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+    const int H = EXACT ? HMAX : p.heads, G = EXACT ? GS : p.kv_heads, D = EXACT ? 128 : p.k_dim, DV = p.v_dim, PS = p.page_size;
+    const int group = H / G, ks_n = D / 32, shift = p.page_shift;
+    const int QP = H * D + 8;
+    bf16_t *qs = (bf16_t *)lds_raw;                         // [16 rows][H][D], + 8 a row
+    bf16_t *ps = qs + kTileRows * QP;                       // [H][16 rows][128 keys]
+    float *mx = (float *)(ps + H * kTileRows * kTileKeys);  // [H][16 rows][8 waves]
     __shared__ int starts[kMaxSegsLds + 1];
     int seg, first, nrows;
     // the last tiles of a prompt see the most keys: they start first, so that the short ones fill the gaps at the end
     const int tile = gridDim.x - 1 - blockIdx.x;
     if (!find_tile(p, tile, starts, seg, first, nrows)) return;
-    const int S = p.splits, split = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int share = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4;
     const size_t out_row = (size_t)H * DV;
     if (p.row_seg[first] < 0) {   // padding rows of a captured step
-        if (split == 0)
-            for (int i = tid; i < nrows * H * DV; i += kThreads) p.out[(size_t)first * out_row + i] = (bf16_t)0.f;
+        if (share == 0)
+            for (int i = tid; i < nrows * H * DV; i += kTileThreads) p.out[(size_t)first * out_row + i] = (bf16_t)0.f;
         return;
     }
-    const int pos0 = p.row_pos[first], plast = pos0 + nrows - 1;
-    const int lo_tile = p.chunk > 0 ? pos0 - pos0 % p.chunk : 0;
-    const int kb_start = lo_tile & ~15;
+    const TileKeys tk = tile_keys(p, first, nrows);
+    if (share >= tk.shares) return;
+    const int plast = tk.plast;
+    const int block0 = share * tk.per_share;
+    const int my_blocks = tk.blocks - block0 < tk.per_share ? tk.blocks - block0 : tk.per_share;
+    const int kb0 = tk.kb_start + kTileKeys * block0;
     const int32_t *tbl = p.tables + (size_t)seg * p.table_stride;
-    const int pos_c = c < nrows ? pos0 + c : -1;
-    const int lo_c = p.chunk > 0 && pos_c >= 0 ? pos_c - pos_c % p.chunk : 0;
-    const int nblk = (plast - kb_start) / kKeyBlock + 1;
-    const int my_blocks = split < nblk ? (nblk - split + S - 1) / S : 0;
-    const int total_stages = my_blocks * 2 * NST;
-    // the pages of the tile's keys: through LDS in one load where they fit, so that a stage's loads wait for no lookup
-    const int page0 = kb_start / PS, npages = plast / PS - page0 + 1;
-    const bool pages_in_lds = npages <= p.ptab;
-    if (pages_in_lds)
-        for (int i = tid; i < npages; i += kThreads) ptab[i] = tbl[page0 + i];
-    auto page_of = [&](int key) __attribute__((always_inline)) { return pages_in_lds ? ptab[key / PS - page0] : tbl[key / PS]; };
+    const int pos_c = c < nrows ? tk.pos0 + c : tk.pos0;        // rows beyond the tile's end: zero queries, never written
+    const int lo_c = p.chunk > 0 ? pos_c - pos_c % p.chunk : 0;
+    const int lo_last = p.chunk > 0 ? plast - plast % p.chunk : 0;
+    // which value lanes this wave owns, and which heads of them (h % HG == hg)
+    const int DVT = DV / 16;
+    const int vt_n = EXACT || DVT > 4 ? 8 : DVT > 2 ? 4 : DVT;
+    const int hg = wave / vt_n, HG = EXACT ? 1 : 8 / vt_n;
+    const bool owns = (wave & (vt_n - 1)) < DVT;
+    const int vt = owns ? wave & (vt_n - 1) : 0;      // a wave without lanes of its own loads the first ones and drops them
+    const bool eights = EXACT || (PS & 7) == 0;       // eight tokens of a value lane lie together; other pages: four and four
+    auto page_of = [&](int key) __attribute__((always_inline)) { return EXACT || shift >= 0 ? key >> shift : key / PS; };
+    auto in_page = [&](int key) __attribute__((always_inline)) { return EXACT || shift >= 0 ? key & (PS - 1) : key % PS; };
+    auto seen = [&](int key) __attribute__((always_inline)) { return key <= plast ? key : plast; };      // beyond it: masked later
 
-    // a stage: block b of this workgroup's blocks, then K of the key/value heads GS at a time, then V likewise
-    bf16x8_t pre[PRE];
-    auto load_stage = [&](int si) __attribute__((always_inline)) {
-        const int b = si / (2 * NST), st = si - b * 2 * NST;
-        const int kb = kb_start + kKeyBlock * (split + S * b);
-        if (st < NST) {
-            const int kvh0 = st * GS;
-            const int key = kb + (tid & 63);
-            const int key_a = key <= plast ? key : plast;      // clamped: masked later
-            const int page = page_of(key_a), off = key_a % PS;
-            const int per_head = D >> 3;                       // at least 4: a step of 4 wraps once at most
-            int l = 0, j = tid >> 6;                           // which head of the stage, which 8 lanes of its keys
+    // the pages of a block's keys: this lane's key of step 1, the lanes' keys of step 3
+    auto key_page = [&](int kb) __attribute__((always_inline)) { return tbl[page_of(seen(kb + 16 * wave + c))]; };
+    int vpage[NS], vpage4[NS];
+    auto value_pages = [&](int kb) __attribute__((always_inline)) {
 #pragma unroll
-            for (int r = 0; r < PRE; r++) {
-                if (l < GS && kvh0 + l < G) pre[r] = *(const bf16x8_t *)(p.k_pages + key_offset(page, G, kvh0 + l, PS, D, off, 8 * j));
-                j += 4;
-                if (j >= per_head) { j -= per_head; l++; }
-            }
-        } else {
-            const int kvh0 = (st - NST) * GS;
-            const int key4 = kb + (tid & 15) * 4;
-            const bool any = key4 <= plast;
-            int page = 0, off = 0;
-            if (any) { page = page_of(key4); off = key4 % PS; }
-            int l = 0, dv = tid >> 4;                          // which head of the stage, which of its value lanes
+        for (int s = 0; s < NS; s++) {
+            vpage[s] = tbl[page_of(seen(kb + 32 * s + 8 * g))];
+            if (!eights) vpage4[s] = tbl[page_of(seen(kb + 32 * s + 8 * g + 4))];
+        }
+    };
+    auto load_keys = [&](bf16x8_t *kf, int kb, int page, int kvh) __attribute__((always_inline)) {
+        const bf16_t *at = p.k_pages + key_offset(page, G, kvh, PS, D, in_page(seen(kb + 16 * wave + c)), 8 * g);
 #pragma unroll
-            for (int r = 0; r < 2 * PRE; r++) {
-                if (l < GS && kvh0 + l < G) {
-                    bf16x4_t v4 = {0, 0, 0, 0};
-                    if (any) v4 = *(const bf16x4_t *)(p.v_pages + (((size_t)page * G + kvh0 + l) * DV + dv) * PS + off);
+        for (int ks = 0; ks < KSM; ks++)
+            if (EXACT || ks < ks_n) kf[ks] = *(const bf16x8_t *)(at + 32 * ks * PS);
+    };
+    auto load_values = [&](bf16x8_t *vf, int kb, int kvh) __attribute__((always_inline)) {
 #pragma unroll
-                    for (int e = 0; e < 4; e++) pre[r >> 1][4 * (r & 1) + e] = key4 + e <= plast ? v4[e] : (bf16_t)0.f;   // slots past the last token hold anything
-                }
-                dv += 16;
-                if (dv >= DV) { dv -= DV; l++; }               // v_dim is a multiple of 16
+        for (int s = 0; s < NS; s++) {
+            const int key = kb + 32 * s + 8 * g;
+            const bf16_t *at = p.v_pages + (((size_t)vpage[s] * G + kvh) * DV + 16 * vt + c) * PS + (key <= plast ? in_page(key) : 0);
+            if (eights) {
+                vf[s] = *(const bf16x8_t *)at;
+            } else {
+                const bf16_t *at4 = p.v_pages + (((size_t)vpage4[s] * G + kvh) * DV + 16 * vt + c) * PS + (key + 4 <= plast ? in_page(key + 4) : 0);
+                const bf16x4_t a4 = *(const bf16x4_t *)at, b4 = *(const bf16x4_t *)at4;
+#pragma unroll
+                for (int e = 0; e < 4; e++) { vf[s][e] = a4[e]; vf[s][4 + e] = b4[e]; }
             }
         }
     };
-    auto store_stage = [&](int si) __attribute__((always_inline)) {
-        const int st = si % (2 * NST);
-        if (st < NST) {
-#pragma unroll
-            for (int r = 0; r < PRE; r++) {
-                const int jj = (tid >> 6) + 4 * r;
-                if (8 * jj < GS * D) *(bf16x8_t *)(stage + (tid & 63) * KP + 8 * jj) = pre[r];
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < 2 * PRE; r++) {
-                const int row = (tid >> 4) + 16 * r;
-                if (row < GS * DV) {
-                    bf16x4_t v4;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v4[e] = pre[r >> 1][4 * (r & 1) + e];
-                    *(bf16x4_t *)(stage + row * kVPitch + (tid & 15) * 4) = v4;
-                }
-            }
-        }
-    };
-    // queries of the tile and the mixing matrix into LDS
+
+    // the first block's keys are on their way while the queries go into LDS
+    bf16x8_t kf[KSM], kn[KSM], vf[NS], vn[NS];
+    int page_now = key_page(kb0);
+    load_keys(kf, kb0, page_now, 0);
     {
         const int per_row = H * D / 8;
-        for (int i = tid; i < kTileRows * per_row; i += kThreads) {
+        for (int i = tid; i < kTileRows * per_row; i += kTileThreads) {
             const int r = i / per_row, e = (i - r * per_row) * 8;
             bf16x8_t v = {0, 0, 0, 0, 0, 0, 0, 0};
             if (r < nrows) v = *(const bf16x8_t *)(p.q + (size_t)(first + r) * H * D + e);
             *(bf16x8_t *)(qs + r * QP + e) = v;
         }
-        for (int i = tid; i < HMAX * HMAX; i += kThreads) {
-            const int h = i / HMAX, gg = i % HMAX;
-            tk[i] = h < H && gg < H ? p.talk[h * H + gg] * (p.scale * p.temp[gg]) : 0.f;
-        }
     }
     __syncthreads();
 
+    // laundered where they are read: the loads stay in the loop instead of filling (and spilling) the scalar registers
+    auto fresh = [](const float *ptr) __attribute__((always_inline)) {
+        uintptr_t v = (uintptr_t)ptr;
+        asm volatile("" : "+s"(v));
+        return (scalar_floats)v;
+    };
     float m_run[HMAX], l_part[HMAX];
-    f32x4_t o[HMAX][TS];
+    f32x4_t o[HMAX];
 #pragma unroll
     for (int h = 0; h < HMAX; h++) {
         m_run[h] = -INFINITY;
         l_part[h] = 0.f;
-#pragma unroll
-        for (int ts = 0; ts < TS; ts++) o[h][ts] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        o[h] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     }
 
-    // One loop over the stages, with one place each where a stage is loaded and stored (the kernel's code has to stay
-    // within the instruction cache): pass -2 loads stage 0, pass -1 stores it and loads stage 1, pass si >= 0 multiplies
-    // from stage si in LDS while stage si + 1 is in flight in `pre`.
-    f32x4_t raw[HMAX];
-    for (int si = -2; si < total_stages; si++) {
-        if (si >= 0) {
-            const int b = si / (2 * NST), st = si - b * 2 * NST;
-            const int kb = kb_start + kKeyBlock * (split + S * b);
-            const int key0 = kb + 16 * wave;
-            const bool active = key0 <= plast;      // wave-uniform
-            if (st < NST) {
-                // ---- 1. raw scores of this wave's 16 keys for the heads of the stage's key/value heads
-                if (st == 0) {
+    for (int b = 0; b < my_blocks; b++) {
+        const int kb = kb0 + kTileKeys * b;
+        const int kb_next = b + 1 < my_blocks ? kb + kTileKeys : kb;
+        value_pages(kb);
+        const int page_next = key_page(kb_next);
+        // ---- 1. raw scores of this wave's 16 keys
+        f32x4_t raw[HMAX];
 #pragma unroll
-                    for (int h = 0; h < HMAX; h++) raw[h] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        for (int h = 0; h < HMAX; h++) raw[h] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll UNROLL
+        for (int kvh = 0; kvh < G; kvh++) {
+            if (kvh + 1 < G) load_keys(kn, kb, page_now, kvh + 1);
+#pragma unroll
+            for (int h = 0; h < HMAX; h++) {
+                if (h % 3 == 0) __builtin_amdgcn_sched_barrier(0);      // registers: LDS reads of three heads ahead, not of all
+                if (h >= kvh * group && h < (kvh + 1) * group) {
+#pragma unroll
+                    for (int ks = 0; ks < KSM; ks++)
+                        if (EXACT || ks < ks_n) {
+                            const bf16x8_t qf = *(const bf16x8_t *)(qs + c * QP + h * D + 32 * ks + 8 * g);
+                            raw[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], qf, raw[h], 0, 0, 0);
+                        }
                 }
-                if (active) {
-                    for (int l = 0; l < GS && st * GS + l < G; l++) {
-                        bf16x8_t kf[KSMAX];
+            }
 #pragma unroll
-                        for (int ks = 0; ks < KSMAX; ks++)
-                            if (ks < KS) kf[ks] = *(const bf16x8_t *)(stage + (16 * wave + c) * KP + l * D + 32 * ks + 8 * g);
-                        const int h_lo = (st * GS + l) * group, h_hi = h_lo + group;
+            for (int ks = 0; ks < KSM; ks++) kf[ks] = kn[ks];
+        }
+        // ---- the mix, lane-local
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4_t s[HMAX];
+        const scalar_floats temp = fresh(p.temp);
 #pragma unroll
-                        for (int h = 0; h < HMAX; h++) {
-                            if (h >= h_lo && h < h_hi) {
+        for (int h = 0; h < HMAX; h++)
+            if (h < H) {
+                const float f = p.scale * temp[h];
 #pragma unroll
-                                for (int ks = 0; ks < KSMAX; ks++)
-                                    if (ks < KS) {
-                                        const bf16x8_t qf = *(const bf16x8_t *)(qs + c * QP + h * D + 32 * ks + 8 * g);
-                                        raw[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], qf, raw[h], 0, 0, 0);
-                                    }
-                            }
-                        }
-                    }
-                }
-                if (st == NST - 1) {
-                    // ---- the mix, lane-local
-                    f32x4_t s[HMAX];
-                    if (active) {
-                        bool see[4];
+                for (int i = 0; i < 4; i++) raw[h][i] *= f;
+            }
 #pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const int key = key0 + 4 * g + i;
-                            see[i] = key >= lo_c && key <= pos_c;
-                        }
+        for (int h = 0; h < HMAX; h++) {
+            s[h] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            if (h < H) {
+                const scalar_floats talk = fresh(p.talk);
 #pragma unroll
-                        for (int h = 0; h < HMAX; h++) {
-                            f32x4_t v = {0.f, 0.f, 0.f, 0.f};
-                            if (h < H) {
+                for (int gg = 0; gg < HMAX; gg++) {
+                    const int at = h * H + gg;
+                    const float t = EXACT ? talk[at] : gg < H ? talk[at < H * H ? at : H * H - 1] : 0.f;
 #pragma unroll
-                                for (int gg = 0; gg < HMAX; gg++) {
-                                    const float t = tk[h * HMAX + gg];
-#pragma unroll
-                                    for (int i = 0; i < 4; i++) v[i] = fmaf(t, raw[gg][i], v[i]);
-                                }
-                            }
-#pragma unroll
-                            for (int i = 0; i < 4; i++) s[h][i] = see[i] ? v[i] : -INFINITY;
-                        }
-                    } else {
-#pragma unroll
-                        for (int h = 0; h < HMAX; h++) s[h] = (f32x4_t){-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-                    }
-                    // ---- 2. the block's largest score a (head, row), through LDS
-#pragma unroll
-                    for (int h = 0; h < HMAX; h++) {
-                        if (h < H) {
-                            float v = fmaxf(fmaxf(s[h][0], s[h][1]), fmaxf(s[h][2], s[h][3]));
-                            v = fmaxf(v, __shfl_xor(v, 16, kWave));
-                            v = fmaxf(v, __shfl_xor(v, 32, kWave));
-                            if (g == 0) mx[wave][h][c] = v;
-                        }
-                    }
-                    __syncthreads();
-#pragma unroll
-                    for (int h = 0; h < HMAX; h++) {
-                        if (h < H) {
-                            const float blk = fmaxf(fmaxf(mx[0][h][c], mx[1][h][c]), fmaxf(mx[2][h][c], mx[3][h][c]));
-                            const float m_new = fmaxf(m_run[h], blk);
-                            const float m_safe = m_new == -INFINITY ? 0.f : m_new;      // a row that has seen no key yet
-                            const float alpha = __expf(m_run[h] - m_safe);
-                            m_run[h] = m_new;
-                            float sum = 0.f;
-                            bf16x4_t w4;
-#pragma unroll
-                            for (int i = 0; i < 4; i++) {
-                                const float e = __expf(s[h][i] - m_safe);
-                                sum += e;
-                                w4[i] = (bf16_t)e;
-                            }
-                            l_part[h] = l_part[h] * alpha + sum;
-                            *(bf16x4_t *)&ps[h][wave][c][4 * g] = w4;
-                            if (wave == 0 && g == 0) al[h][c] = alpha;
-                        }
-                    }
-                    // the barrier below, before the next stage is stored, also publishes ps and al
-                }
-            } else {
-                // ---- 3. outputs: this wave's value lanes of every head of the stage's key/value heads
-                for (int l = 0; l < GS && (st - NST) * GS + l < G; l++) {
-                    const int h_lo = ((st - NST) * GS + l) * group, h_hi = h_lo + group;
-                    const int lrow = l * DV;
-#pragma unroll
-                    for (int ts = 0; ts < TS; ts++) {
-                        const int t = wave + 4 * ts;
-                        if (t < DVT) {
-                            bf16x8_t vf[2];
-#pragma unroll
-                            for (int s2 = 0; s2 < 2; s2++) {
-                                const bf16x4_t a4 = *(const bf16x4_t *)(stage + (lrow + 16 * t + c) * kVPitch + 32 * s2 + 4 * g);
-                                const bf16x4_t b4 = *(const bf16x4_t *)(stage + (lrow + 16 * t + c) * kVPitch + 32 * s2 + 16 + 4 * g);
-#pragma unroll
-                                for (int e = 0; e < 4; e++) { vf[s2][e] = a4[e]; vf[s2][4 + e] = b4[e]; }
-                            }
-#pragma unroll
-                            for (int h = 0; h < HMAX; h++) {
-                                if (h >= h_lo && h < h_hi) {
-                                    const float alpha = al[h][c];
-                                    f32x4_t acc = o[h][ts];
-#pragma unroll
-                                    for (int i = 0; i < 4; i++) acc[i] *= alpha;
-#pragma unroll
-                                    for (int s2 = 0; s2 < 2; s2++) {
-                                        if (kb + 32 * s2 > plast) continue;      // uniform: no key of this half is seen
-                                        const bf16x4_t a4 = *(const bf16x4_t *)&ps[h][2 * s2][c][4 * g];
-                                        const bf16x4_t b4 = *(const bf16x4_t *)&ps[h][2 * s2 + 1][c][4 * g];
-                                        bf16x8_t pf;
-#pragma unroll
-                                        for (int e = 0; e < 4; e++) { pf[e] = a4[e]; pf[4 + e] = b4[e]; }
-                                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[s2], pf, acc, 0, 0, 0);
-                                    }
-                                    o[h][ts] = acc;
-                                }
-                            }
-                        }
-                    }
+                    for (int i = 0; i < 4; i++) s[h][i] = fmaf(t, raw[gg][i], s[h][i]);
                 }
             }
         }
-        __syncthreads();                      // every wave is done with the stage in LDS (and ps, mx, al of its block)
-        if (si + 1 >= 0 && si + 1 < total_stages) store_stage(si + 1);
+        if (kb + kTileKeys - 1 > tk.pos0 || kb < lo_last) {      // uniform: some row does not see all of the block
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int key = kb + 16 * wave + 4 * g + i;
+                const bool see = key >= lo_c && key <= pos_c;
+#pragma unroll
+                for (int h = 0; h < HMAX; h++) s[h][i] = see ? s[h][i] : -INFINITY;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);      // registers: the raw scores' are free from here on
+        load_values(vf, kb, 0);                 // the first values arrive during the softmax
+        // ---- 2. the block's largest score a (head, row), through LDS
+#pragma unroll
+        for (int h = 0; h < HMAX; h++) {
+            if (h < H) {
+                float v = fmaxf(fmaxf(s[h][0], s[h][1]), fmaxf(s[h][2], s[h][3]));
+                v = fmaxf(v, __shfl_xor(v, 16, kWave));
+                v = fmaxf(v, __shfl_xor(v, 32, kWave));
+                mx[(h * kTileRows + c) * 8 + wave] = v;      // the four lanes of a row hold the same
+            }
+        }
+        __syncthreads();      // also: every wave has multiplied the weights of the block before
+#pragma unroll
+        for (int h = 0; h < HMAX; h++) {
+            if (h % 3 == 0) __builtin_amdgcn_sched_barrier(0);
+            if (h < H) {
+                const f32x4_t ma = *(const f32x4_t *)(mx + (h * kTileRows + c) * 8), mb = *(const f32x4_t *)(mx + (h * kTileRows + c) * 8 + 4);
+                const float blk = fmaxf(fmaxf(fmaxf(ma[0], ma[1]), fmaxf(ma[2], ma[3])), fmaxf(fmaxf(mb[0], mb[1]), fmaxf(mb[2], mb[3])));
+                const float m_new = fmaxf(m_run[h], blk);
+                const float m_safe = m_new == -INFINITY ? 0.f : m_new;      // a row that has seen no key yet
+                const float alpha = __expf(m_run[h] - m_safe);
+                m_run[h] = m_new;
+                float sum = 0.f;
+                bf16x4_t w4;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float e = __expf(s[h][i] - m_safe);
+                    sum += e;
+                    w4[i] = (bf16_t)e;
+                }
+                l_part[h] = l_part[h] * alpha + sum;
+#pragma unroll
+                for (int i = 0; i < 4; i++) o[h][i] *= alpha;
+                // keys 16 wave + 4 g ..: half of the 16-byte piece 2 wave + g / 2
+                *(bf16x4_t *)(ps + (h * kTileRows + c) * kTileKeys + 8 * ((2 * wave + (g >> 1)) ^ c) + 4 * (g & 1)) = w4;
+            }
+        }
         __syncthreads();
-        if (si + 2 < total_stages) load_stage(si + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        page_now = page_next;
+        load_keys(kf, kb_next, page_now, 0);    // the next block's first keys arrive during the products
+        // ---- 3. outputs: this wave's value lanes, keys 32 s + 8 g + e in the products' slots
+        if (owns) {
+            const bool ragged = kb + kTileKeys - 1 > plast;      // uniform
+#pragma unroll UNROLL
+            for (int kvh = 0; kvh < G; kvh++) {
+                if (kvh + 1 < G) load_values(vn, kb, kvh + 1);
+                if (ragged) {      // slots past the last token hold anything
+#pragma unroll
+                    for (int s2 = 0; s2 < NS; s2++)
+#pragma unroll
+                        for (int e = 0; e < 8; e++) vf[s2][e] = kb + 32 * s2 + 8 * g + e <= plast ? vf[s2][e] : (bf16_t)0.f;
+                }
+#pragma unroll
+                for (int h = 0; h < HMAX; h++) {
+                    if (h % 3 == 0) __builtin_amdgcn_sched_barrier(0);
+                    if (h >= kvh * group && h < (kvh + 1) * group && (HG == 1 || (h & (HG - 1)) == hg)) {
+#pragma unroll
+                        for (int s2 = 0; s2 < NS; s2++) {
+                            const bf16x8_t pf = *(const bf16x8_t *)(ps + (h * kTileRows + c) * kTileKeys + 8 * ((4 * s2 + g) ^ c));
+                            o[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[s2], pf, o[h], 0, 0, 0);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int s2 = 0; s2 < NS; s2++) vf[s2] = vn[s2];
+            }
+        }
     }
-    // the rows' sums: lanes of one row, then the four waves
+    // the rows' sums: lanes of one row, then the eight waves (nobody reads mx after the last block's second barrier)
 #pragma unroll
     for (int h = 0; h < HMAX; h++) {
         if (h < H) {
             float v = l_part[h];
             v += __shfl_xor(v, 16, kWave);
             v += __shfl_xor(v, 32, kWave);
-            if (g == 0) mx[wave][h][c] = v;
+            if (g == 0) mx[(h * kTileRows + c) * 8 + wave] = v;
         }
     }
     __syncthreads();
-    if (S > 1) {
+    auto row_sum = [&](int h) __attribute__((always_inline)) {
+        const f32x4_t a = *(const f32x4_t *)(mx + (h * kTileRows + c) * 8), b = *(const f32x4_t *)(mx + (h * kTileRows + c) * 8 + 4);
+        return ((a[0] + a[1]) + (a[2] + a[3])) + ((b[0] + b[1]) + (b[2] + b[3]));
+    };
+    if (tk.shares > 1) {
         // this workgroup's share of the tile: maxima and sums [heads][16], unnormalised outputs [16][heads][v_dim]
-        float *part = p.ws + ((size_t)tile * S + split) * part_floats(H, DV);
+        float *part = p.ws + ((size_t)tile * p.splits + share) * part_floats(H, DV);
         float *part_o = part + 2 * kTileRows * H;
 #pragma unroll
         for (int h = 0; h < HMAX; h++) {
             if (h < H) {
                 if (wave == 0 && g == 0) {
                     part[h * kTileRows + c] = m_run[h];
-                    part[(H + h) * kTileRows + c] = (mx[0][h][c] + mx[1][h][c]) + (mx[2][h][c] + mx[3][h][c]);
+                    part[(H + h) * kTileRows + c] = row_sum(h);
                 }
-#pragma unroll
-                for (int ts = 0; ts < TS; ts++) {
-                    const int t = wave + 4 * ts;
-                    if (t < DVT) *(f32x4_t *)(part_o + ((size_t)c * H + h) * DV + 16 * t + 4 * g) = o[h][ts];
-                }
+                if (owns && (HG == 1 || (h & (HG - 1)) == hg)) *(f32x4_t *)(part_o + ((size_t)c * H + h) * DV + 16 * vt + 4 * g) = o[h];
             }
         }
         return;
     }
-    if (c >= nrows) return;
+    if (c >= nrows || !owns) return;
 #pragma unroll
     for (int h = 0; h < HMAX; h++) {
-        if (h < H) {
-            const float l = (mx[0][h][c] + mx[1][h][c]) + (mx[2][h][c] + mx[3][h][c]);
+        if (h < H && (HG == 1 || (h & (HG - 1)) == hg)) {
+            const float l = row_sum(h);
             float f = l > 0.f ? 1.0f / l : 0.f;
             if (p.gate != nullptr) f *= 1.0f / (1.0f + __expf(-(float)p.gate[(size_t)(first + c) * p.gate_stride + h]));
+            bf16x4_t r4;
 #pragma unroll
-            for (int ts = 0; ts < TS; ts++) {
-                const int t = wave + 4 * ts;
-                if (t < DVT) {
-                    bf16x4_t r4;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) r4[i] = (bf16_t)(o[h][ts][i] * f);
-                    *(bf16x4_t *)(p.out + (size_t)(first + c) * out_row + (size_t)h * DV + 16 * t + 4 * g) = r4;
-                }
-            }
+            for (int i = 0; i < 4; i++) r4[i] = (bf16_t)(o[h][i] * f);
+            *(bf16x4_t *)(p.out + (size_t)(first + c) * out_row + (size_t)h * DV + 16 * vt + 4 * g) = r4;
         }
     }
 }
@@ -421,9 +406,11 @@ __global__ void __launch_bounds__(kThreads) talking_merge_kernel(const TalkArgs 
     int seg, first, nrows;
     if (!find_tile(p, blockIdx.x, starts, seg, first, nrows)) return;
     if (p.row_seg[first] < 0) return;      // padding rows: the tile kernel has written zeros
-    const int H = p.heads, DV = p.v_dim, S = p.splits, h = blockIdx.y;
+    const int H = p.heads, DV = p.v_dim, h = blockIdx.y;
+    const int S = tile_keys(p, first, nrows).shares;
+    if (S <= 1) return;                    // one workgroup had the whole tile: it has written the outputs
     const size_t per = part_floats(H, DV);
-    const float *parts = p.ws + (size_t)blockIdx.x * S * per;
+    const float *parts = p.ws + (size_t)blockIdx.x * p.splits * per;
     const int quads = DV / 4;
     for (int i = threadIdx.x; i < nrows * quads; i += kThreads) {
         const int c = i / quads, d4 = (i - c * quads) * 4;
@@ -729,23 +716,22 @@ int launch_decode(const TalkArgs &a, hipStream_t stream) {
     return rc;
 }
 
-template <int HMAX>
-int launch_tiles(const TalkArgs &a, int tiles, size_t lds, hipStream_t stream) {
-    auto kernel = talking_tile_kernel<HMAX>;
-    // the kernel's own arrays (mixing matrix, maxima, factors, weights) come on top of the queries and the stage: beyond
-    // the default 64 KiB of both together the larger amount has to be asked for
-    constexpr size_t own = sizeof(float) * (HMAX * HMAX + 5 * HMAX * kTileRows) + sizeof(bf16_t) * HMAX * 4 * kTileRows * 16 +
-                           sizeof(int) * (kMaxSegsLds + 1);
+size_t tile_lds(int heads, int k_dim) {
+    return ((size_t)kTileRows * (heads * k_dim + 8) + (size_t)heads * kTileRows * kTileKeys) * sizeof(bf16_t) +
+           (size_t)heads * kTileRows * 8 * sizeof(float);
+}
+
+template <int HMAX, int GS>
+int launch_tiles(const TalkArgs &a, int tiles, hipStream_t stream) {
+    auto kernel = talking_tile_kernel<HMAX, GS>;
+    constexpr size_t own = sizeof(int) * (kMaxSegsLds + 1);
+    const size_t lds = tile_lds(a.heads, a.k_dim);
     if (own + lds > 160 * 1024) return 1;
-    if (own + lds > 60 * 1024) {
-        static bool asked = false;
-        if (!asked) {
-            FLLM_REQUIRE(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - (int)own) ==
-                             hipSuccess, "talking_attention: cannot have %zu bytes of LDS", own + lds);
-            asked = true;
-        }
+    if (own + lds > 60 * 1024) {      // beyond the default 64 KiB the larger amount has to be asked for
+        FLLM_REQUIRE(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - (int)own) ==
+                         hipSuccess, "talking_attention: cannot have %zu bytes of LDS", own + lds);
     }
-    hipLaunchKernelGGL(kernel, dim3(tiles, a.splits), dim3(kThreads), lds, stream, a);
+    hipLaunchKernelGGL(kernel, dim3(tiles, a.splits), dim3(kTileThreads), lds, stream, a);
     int rc = fllm_check_launch("talking_attention (matrix cores)");
     if (rc == 0 && a.splits > 1) {
         hipLaunchKernelGGL(talking_merge_kernel, dim3(tiles, a.heads), dim3(kThreads), 0, stream, a);
@@ -771,22 +757,6 @@ int fllm_talking_attention_bf16_fast(const void *q, const void *gate, int gate_s
                                      hipStream_t stream) {
     if (key_chunk != 8 || k_dim % 32 != 0 || k_dim > 256 || v_dim % 16 != 0 || v_dim > 128 || heads > 16 || page_size % 4 != 0)
         return 1;
-    // A stage holds as many key/value heads as a thread's 8 registers of 16 bytes and LDS allow, and the page numbers of
-    // the keys a tile can see lie in LDS where they fit (up to 4,096: 65,536 keys of pages of 16).
-    const int widest = k_dim > v_dim ? k_dim : v_dim;
-    int gs = 256 / widest < kv_heads ? 256 / widest : kv_heads;
-    const long span = chunk > 0 && chunk + 2 * kTileRows < max_context ? chunk + 2 * kTileRows : max_context;
-    int ptab = (int)(span / page_size + 3);
-    if (ptab > 4096) ptab = 0;
-    auto lds_for = [&](int heads_a_stage, int pages) {
-        const size_t k_elems = (size_t)kKeyBlock * (heads_a_stage * k_dim + 8), v_elems = (size_t)heads_a_stage * v_dim * kVPitch;
-        const size_t stage = ((k_elems > v_elems ? k_elems : v_elems) + 7) & ~(size_t)7;
-        return ((size_t)kTileRows * (heads * k_dim + 8) + stage) * sizeof(bf16_t) + (size_t)pages * sizeof(int);
-    };
-    constexpr size_t kLdsRoom = 160 * 1024 - 46 * 1024;      // what the kernel's own arrays leave at 16 heads
-    while (gs > 1 && lds_for(gs, ptab) > kLdsRoom) gs--;
-    if (lds_for(gs, ptab) > kLdsRoom) ptab = 0;
-    const size_t lds = lds_for(gs, ptab);
     if (((uintptr_t)q | (uintptr_t)out | (uintptr_t)k_pages | (uintptr_t)v_pages) & 15) return 1;
     if (splits < 1) splits = 1;
     if (splits > 1) {
@@ -820,16 +790,26 @@ int fllm_talking_attention_bf16_fast(const void *q, const void *gate, int gate_s
     a.chunk = chunk;
     a.splits = splits;
     a.ws = ws;
-    a.gs = gs;
-    a.ptab = ptab;
+    a.page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
+    // the blocks of the longest row tile, dealt out evenly: shorter tiles take fewer workgroups
+    const long span = chunk > 0 && chunk + 2 * kTileRows < max_context ? chunk + 2 * kTileRows : max_context;
+    const long blocks = (span + kTileRows + kTileKeys - 1) / kTileKeys;
+    a.share_blocks = blocks > splits ? (int)((blocks + splits - 1) / splits) : 1;
     if (single_rows && rows == num_segs) {      // a decode step: every request has one row
         const int rc = launch_decode(a, stream);
         if (rc <= 0) return rc;
     }
     // every segment's rows in tiles of 16: at most rows / 16 full tiles and one ragged tile a segment
     const int tiles = rows / kTileRows + num_segs;
-    // the kernel holds every head's scores and outputs of its rows in registers: an instance a head count bracket
-    if (heads <= 8) return launch_tiles<8>(a, tiles, lds, stream);
-    if (heads <= 12) return launch_tiles<12>(a, tiles, lds, stream);
-    return launch_tiles<16>(a, tiles, lds, stream);
+    // The kernel holds every head's scores and outputs of its rows in registers: an instance a bracket of head counts, and
+    // one each for exactly 8, 12 and 16 heads on two key/value heads of 128 lanes: without conditions in
+    // the loops nothing is spilled up to 12 heads, where the general one spills 106 registers (12 heads, 1,000 rows).
+    if (kv_heads == 2 && k_dim == 128 && v_dim > 64 && a.page_shift >= 3) {
+        if (heads == 8) return launch_tiles<8, 2>(a, tiles, stream);
+        if (heads == 12) return launch_tiles<12, 2>(a, tiles, stream);
+        if (heads == 16) return launch_tiles<16, 2>(a, tiles, stream);
+    }
+    if (heads <= 8) return launch_tiles<8, 0>(a, tiles, stream);
+    if (heads <= 12) return launch_tiles<12, 0>(a, tiles, stream);
+    return launch_tiles<16, 0>(a, tiles, stream);
 }

@@ -7,6 +7,8 @@ library cannot be loaded or built, constructing `Ops` raises.
 from __future__ import annotations
 
 import ctypes
+import functools
+import math
 import weakref
 from typing import Dict, NamedTuple, Optional, Sequence, Tuple
 
@@ -249,6 +251,30 @@ def _dense(t: torch.Tensor, name: str, dtype=None, shape=None) -> None:
         raise KernelError(f"{name} must be {dtype}, is {t.dtype}")
     if shape is not None and tuple(t.shape) != tuple(shape):
         raise KernelError(f"{name} must have shape {tuple(shape)}, has {tuple(t.shape)}")
+
+
+@functools.lru_cache(maxsize=256)
+def _talking_shares(tiles: int, least: int, blocks: int, slots: int) -> int:
+    """Workgroups a row tile at most, for tiles that see `least` to `blocks` blocks of keys, evenly spread: a tile of n blocks
+    takes ceil(n / share) workgroups of `share` blocks.  The launch costs its rounds of `slots` workgroups times a share and
+    what a workgroup pays beside it (about one block: queries in, outputs out); sharing at all costs another block (the merge).
+    1,900 rows of 12 heads from a request's first token on: 3 (240 workgroups of up to 5 blocks) 74 us, 2 and 4 (two blocks
+    more, or two rounds) 96 us."""
+    def pieces(n, share):      # sum of ceil(i / share) over i = 1 .. n
+        full, rest = divmod(n, share)
+        return share * full * (full + 1) // 2 + rest * (full + 1)
+    best, best_cost, before = 1, None, None
+    for splits in range(1, min(64, blocks) + 1):
+        share = -(-blocks // splits)
+        if share == before:
+            continue
+        before = share
+        workgroups = tiles * (pieces(blocks, share) - pieces(least - 1, share)) / (blocks - least + 1)
+        cost = max(1, math.ceil(workgroups / slots)) * (share + 1) + (splits > 1)
+        if best_cost is None or cost < best_cost:
+            best, best_cost = splits, cost
+    return best
+
 
 
 class Ops:
@@ -1262,16 +1288,22 @@ class Ops:
         return q_out
 
     TALKING_TILE_ROWS = 16          # rows of one request that a workgroup of the matrix-core kernel takes
-    TALKING_KEY_BLOCK = 64          # keys it walks at a time
-    TALKING_WORKGROUPS = 512        # what a launch should come to: two a compute unit
+    TALKING_TILE_KEYS = 128         # keys it walks at a time
+    TALKING_TILE_SLOTS = 256        # workgroups of it the device holds: registers and LDS leave room for one a compute unit
+    TALKING_KEY_BLOCK = 64          # keys the decode kernel walks at a time
+    TALKING_WORKGROUPS = 512        # what a decode launch should come to: two a compute unit
 
     def talking_attention_splits(self, rows: int, num_segs: int, chunk: Optional[int], max_context: int) -> int:
-        """How many workgroups should share the keys of a row tile of `talking_attention` (1: none): enough to fill the
-        device when the step has few tiles (a decode step has one a request), at most one a block of keys."""
+        """How many workgroups should share the keys of a row tile of `talking_attention` (1: none).  Single rows: enough to
+        fill the device, at most one a block of keys.  Row tiles: see _talking_shares."""
         tiles = rows // self.TALKING_TILE_ROWS + num_segs
         span = max_context if not chunk else min(max_context, chunk + self.TALKING_TILE_ROWS)
-        blocks = -(-(span + self.TALKING_TILE_ROWS) // self.TALKING_KEY_BLOCK)
-        return max(1, min(self.TALKING_WORKGROUPS // max(tiles, 1), blocks, 64))
+        if rows == num_segs:
+            blocks = -(-(span + self.TALKING_TILE_ROWS) // self.TALKING_KEY_BLOCK)
+            return max(1, min(self.TALKING_WORKGROUPS // max(tiles, 1), blocks, 64))
+        blocks = -(-(span + self.TALKING_TILE_ROWS) // self.TALKING_TILE_KEYS)
+        least = 1 if chunk and chunk < max_context else max(1, (max_context - rows // max(num_segs, 1)) // self.TALKING_TILE_KEYS)
+        return _talking_shares(tiles, min(least, blocks), blocks, self.TALKING_TILE_SLOTS)
 
     def talking_attention_workspace(self, rows: int, num_segs: int, heads: int, v_dim: int, splits: int) -> int:
         """float32 elements of workspace that `splits` workgroups a tile need."""

@@ -1,0 +1,47 @@
+"""Row tiles of the attention whose heads talk to each other, at the edges of its blocks of 128 keys: the instances that are built for a
+head count and the general one, shares of a tile's blocks (more blocks than the caller's bound allows for among them), pages that are a power
+of two, a multiple of eight and of four, value widths that leave waves without lanes of their own, chunks that end inside a tile."""
+import pytest
+import torch
+
+from reference_ops import ReferenceOps
+from test_menitar_gpu import BF16_EPS, DEV, Scene, close, run_mixer_kernels
+
+pytestmark = pytest.mark.gpu
+
+# heads, kv heads, key size, value size, chunk, page
+SHAPES = [(8, 2, 128, 128, None, 16), (12, 2, 128, 128, 300, 64), (16, 2, 128, 80, 130, 8), (12, 2, 128, 112, None, 4), (16, 2, 128, 128, 140, 24),
+          (15, 3, 192, 48, None, 12), (16, 16, 160, 16, 200, 16), (7, 7, 96, 128, 129, 32), (8, 4, 256, 96, None, 8)]
+# (held, new): tiles of one row to several, last keys right before, on and behind a block's edge
+SEGMENTS = [(0, 129), (111, 17), (112, 16), (127, 2), (254, 3), (383, 33), (0, 5), (500, 12)]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from fllm_amd.kernels import Ops
+    return Ops()
+
+
+@pytest.mark.parametrize("splits", [1, 2, 4])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_blocks_of_128_keys(ops, shape, splits):
+    H, G, d, dv, chunk, page = shape
+    ref, scale = ReferenceOps(), d ** -0.5
+    loud = [(s, held + new, 8.0) for s, (held, new) in enumerate(SEGMENTS)]      # the slot behind a request's last token
+    sc = Scene(SEGMENTS, H, G, d, dv, page, 32, seed=H + d + dv, dtype=torch.bfloat16, loud=loud)
+    for s, (held, new) in enumerate(SEGMENTS):                                   # and what lies in it for the values
+        at = held + new
+        sc.v_pages[int(sc.tables[s, at // page]), :, :, at % page] = float("nan")
+    t = sc.tensors(DEV)
+    if splits == 4:      # fewer blocks than the rows see: shares still cover all of them
+        sc.max_pos = 64
+    q, got = run_mixer_kernels(ops, t, sc, chunk, scale, torch.bfloat16, splits)
+    torch.cuda.synchronize()
+    # the reference goes on from the queries, keys and values that the store kernel left (its own test holds those)
+    w = {n: v.cpu().double() if v.dtype in (torch.bfloat16, torch.float32) else v.cpu() for n, v in t.items()}
+    want = torch.empty(got.shape, dtype=torch.float64)
+    gate_at = H * d + G * (d + dv)
+    ref.talking_attention(q.cpu().double(), w["qkvg"][:, gate_at:gate_at + H], w["k_pages"], w["v_pages"].nan_to_num(0.0), w["tables"],
+                          w["row_pos"], w["row_seg"], w["seg_start"], w["talk"], w["temp"], want, H, G, d, dv, page, scale, chunk, 8, 600)
+    # weights and the result are rounded to bfloat16 (2^-9 of each), scores of up to about 30 carry float32 sums
+    close(got, want, 3 * BF16_EPS, 3e-2, "attention")
