@@ -45,3 +45,30 @@ def test_blocks_of_128_keys(ops, shape, splits):
                           w["row_pos"], w["row_seg"], w["seg_start"], w["talk"], w["temp"], want, H, G, d, dv, page, scale, chunk, 8, 600)
     # weights and the result are rounded to bfloat16 (2^-9 of each), scores of up to about 30 carry float32 sums
     close(got, want, 3 * BF16_EPS, 3e-2, "attention")
+
+
+# heads, kv heads, key size, value size, chunk, page: the instance for one or two key/value heads of 128 lanes, and beside its rule
+SINGLE = [(12, 2, 128, 128, None, 16), (16, 1, 128, 128, 100, 8), (5, 1, 128, 128, None, 64), (12, 2, 128, 128, 70, 24), (9, 3, 128, 128, None, 16),
+          (16, 8, 64, 128, 130, 16), (6, 2, 128, 112, None, 32)]
+
+
+@pytest.mark.parametrize("splits", [1, 2, 4])
+@pytest.mark.parametrize("shape", SINGLE)
+def test_single_rows(ops, shape, splits):
+    """Contexts around a block of 64 keys and several blocks a workgroup, with what is no number behind the last token."""
+    H, G, d, dv, chunk, page = shape
+    ref, scale = ReferenceOps(), d ** -0.5
+    sc = Scene([(n, 1) for n in (0, 15, 62, 63, 64, 99, 127, 128, 300, 511)], H, G, d, dv, page, 32, seed=H + d + dv, dtype=torch.bfloat16)
+    for s in range(10):
+        at = int(sc.row_pos[s]) + 1
+        sc.v_pages[int(sc.tables[s, at // page]), :, :, at % page] = float("nan")
+        sc.k_pages[int(sc.tables[s, at // page]), :, :, at % page] *= 8.0
+    t = sc.tensors(DEV)
+    q, got = run_mixer_kernels(ops, t, sc, chunk, scale, torch.bfloat16, splits, single_rows=True)
+    torch.cuda.synchronize()
+    w = {n: v.cpu().double() if v.dtype in (torch.bfloat16, torch.float32) else v.cpu() for n, v in t.items()}
+    want = torch.empty(got.shape, dtype=torch.float64)
+    gate_at = H * d + G * (d + dv)
+    ref.talking_attention(q.cpu().double(), w["qkvg"][:, gate_at:gate_at + H], w["k_pages"], w["v_pages"].nan_to_num(0.0), w["tables"],
+                          w["row_pos"], w["row_seg"], w["seg_start"], w["talk"], w["temp"], want, H, G, d, dv, page, scale, chunk, 8, 600)
+    close(got, want, 3 * BF16_EPS, 3e-2, "attention")      # the same roundings as the tiles'
