@@ -53,25 +53,27 @@ int fllm_set_device_workspace(void *workspace, size_t bytes);
 //   fllm_norm_qkv_rope_store  w = [q; k; v]: rotates query and key lanes in pairs (2l, 2l+1), stores the
 //                             queries as bfloat16 [M, heads * head_dim] and keys and values into the pages
 //                             (layouts and row/segment/table arguments as fllm_rope_kv_store)
+// `w_tiles` (may be null), here and below: the tile-major copy of w (fllm_tile_weights; of [gate; up] fllm_tile_weights_gate_up), which
+// steps of up to 16 rows stream instead of w.
 int fllm_fused_decode_supported(int M, int K);
 // out = silu(x gate^T) * (x up^T) for bfloat16 rows x [M, K] (1..64 rows, row stride ldx; fllm_gate_up_swiglu_tiled: to 128), w = [gate; up] ([2 I, K])
 int fllm_gate_up_swiglu(const void *x, int ldx, const void *w_gate_up, const float *bias, void *out, int M, int inter,
                         int K, hipStream_t stream);
 // The gated products with the activation's constants as arguments: a(g') * (u' + offset), a(g) = g * sigmoid(alpha g),
 // g' = min(gate, limit), u' = clamp(up, -limit, limit) (limit <= 0: nothing is clamped).  fllm_norm_gate_up_glu folds the
-// RMSNorm of float32 rows in (1..64 rows); fllm_gate_up_glu takes bfloat16 rows (1..64, or 17..128 with `w_tiles`).
-int fllm_norm_gate_up_glu(const float *x, const float *norm_w, float eps, const void *w_gate_up, const float *bias, void *out,
-                          int M, int inter, int K, float limit, float alpha, float offset, hipStream_t stream);
+// RMSNorm of float32 rows in (1..64 rows); fllm_gate_up_glu takes bfloat16 rows (1..64, or to 128 with `w_tiles`).
+int fllm_norm_gate_up_glu(const float *x, const float *norm_w, float eps, const void *w_gate_up, const void *w_tiles,
+                          const float *bias, void *out, int M, int inter, int K, float limit, float alpha, float offset, hipStream_t stream);
 int fllm_gate_up_glu(const void *x, int ldx, const void *w_gate_up, const void *w_tiles, const float *bias, void *out, int M,
                      int inter, int K, float limit, float alpha, float offset, hipStream_t stream);
 // max(x @ w^T, 0)^2 in bfloat16, the square in float32 before the one rounding: 1..64 bfloat16 rows of `ldx` elements.
-int fllm_linear_relu_squared(const void *x, int ldx, const void *w, void *out, int M, int N, int K, hipStream_t stream);
-int fllm_norm_linear(const float *x, const float *norm_w, float eps, const void *w, const float *bias, void *out, int M,
-                     int N, int K, hipStream_t stream);
-int fllm_norm_gate_up_swiglu(const float *x, const float *norm_w, float eps, const void *w_gate_up, const float *bias,
-                             void *out, int M, int inter, int K, hipStream_t stream);
-int fllm_norm_qkv_rope_store(const float *x, const float *norm_w, float eps, const void *w_qkv, const float *bias,
-                             void *q_out, const int32_t *row_pos, const int32_t *row_seg, const int32_t *tables,
+int fllm_linear_relu_squared(const void *x, int ldx, const void *w, const void *w_tiles, void *out, int M, int N, int K, hipStream_t stream);
+int fllm_norm_linear(const float *x, const float *norm_w, float eps, const void *w, const void *w_tiles, const float *bias, void *out,
+                     int M, int N, int K, hipStream_t stream);
+int fllm_norm_gate_up_swiglu(const float *x, const float *norm_w, float eps, const void *w_gate_up, const void *w_tiles,
+                             const float *bias, void *out, int M, int inter, int K, hipStream_t stream);
+int fllm_norm_qkv_rope_store(const float *x, const float *norm_w, float eps, const void *w_qkv, const void *w_tiles,
+                             const float *bias, void *q_out, const int32_t *row_pos, const int32_t *row_seg, const int32_t *tables,
                              int table_stride, const float *cos_table, const float *sin_table, int rope_dims, void *k_pages,
                              void *v_pages, int M, int heads, int kv_heads, int head_dim, int K, int page_size,
                              int store_kv, hipStream_t stream);
@@ -97,12 +99,12 @@ int fllm_linear_add_normed(const void *x, int ldx, const void *w, const float *b
 // the two products of the feed-forward up to 128 rows):
 // the feed-forward and q/k/v products with their fused prologues and epilogues then beat the library's products and
 // the separate norm, rotary and SwiGLU kernels.
-//   fllm_weight_tiles_supported  1 where the kernels take tiles: N >= 16, K a multiple of 1,024
+//   fllm_weight_tiles_supported  1 where the kernels take tiles: N >= 16, K a multiple of 32 from 256 on
 //   fllm_weight_tiles_elements   bfloat16 elements of the copy: N rounded up to 16, times K
-//   fllm_tile_weights            writes the copy: [tile of 16 rows][k-step of 32][lane][8] (any K in steps of 32; only those that
-//                                are supported serve the products here, the others fllm_experts_stream)
+//   fllm_tile_weights            writes the copy: [tile of 16 rows][k-step of 32][lane][8]
 //   fllm_linear_add_tiled        out += x w^T (+ bias), float32 out, 1..128 rows (beyond 64: w_tiles required, K in steps of 256)
 //   fllm_linear_f32_tiled        out = x w^T (+ bias), float32 out, 1..64 rows (the vocabulary projection); with w_tiles where it can
+//   fllm_linear_store_tiled      the same into a bfloat16 out, 1..16 rows
 //   fllm_tile_weights_gate_up    the copy of [gate; up] ([2 inter][K]) for the SwiGLU epilogue of 17 to 64 rows: tile T holds
 //                                gate rows 8 T .. 8 T + 7 and then the same up rows; fllm_weight_tiles_elements_gate_up elements
 //   fllm_gate_up_swiglu_tiled    fllm_gate_up_swiglu for 17..128 rows with that copy (null: row-major, up to 64 rows)
@@ -111,6 +113,8 @@ size_t fllm_weight_tiles_elements(int N, int K);
 int fllm_tile_weights(const void *w, void *tiles, int N, int K, hipStream_t stream);
 int fllm_linear_add_tiled(const void *x, int ldx, const void *w, const void *w_tiles, const float *bias, float *out, int ldo,
                           int M, int N, int K, hipStream_t stream);
+int fllm_linear_store_tiled(const void *x, int ldx, const void *w, const void *w_tiles, const float *bias, void *out, int ldo, int M,
+                            int N, int K, hipStream_t stream);
 int fllm_linear_f32_tiled(const void *x, int ldx, const void *w, const void *w_tiles, const float *bias, float *out, int ldo,
                           int M, int N, int K, hipStream_t stream);
 size_t fllm_weight_tiles_elements_gate_up(int inter, int K);

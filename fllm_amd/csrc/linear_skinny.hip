@@ -339,7 +339,6 @@ template <int PRO, int EPI, int TM, int WAVES, bool XD, bool WT = false>
 __global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4, 4)))   // 16 waves a CU: 128 registers
 skinny_resident_kernel(SkinnyArgs a, int red_off) {
     static_assert(!XD || PRO == PRO_BF16, "activations straight from global memory: the bfloat16 prologue only");
-    static_assert(!WT || TM != TM_DUALK, "tile-major weights: whole 16-row tiles (or 8 gate and 8 up rows), one slice");
     constexpr int U = 4;                           // k-steps of 32 per block: four 16-byte loads per lane
     constexpr int KB = 32 * U;                     // K elements of one range per block
     constexpr int RB = 4;                          // rows of activations staged at a time (more would spill registers)
@@ -390,9 +389,12 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
             if (TM == TM_GATEUP) row += (r >> 3) * n_out;
             const int kb = kr0 + l_j * KB;
             if (WT) {
-                // tile-major weights (fllm_tile_weights): the 16 rows x 128 columns of a block lie together in the order
-                // the lanes take them, so a load instruction reads 1 KiB in a row instead of 64 bytes of each of 16 rows
-                const bf16_t *wp = a.w_tiles + (size_t)(tile0 + l_item * tstride) * 16 * K + (size_t)((kw0 + l_j * KB) / KB) * (16 * KB) + lane * 8;
+                // tile-major weights (fllm_tile_weights, one slice): the 16 rows x 32 columns of a k-step lie together in the order
+                // the lanes take them, so a load instruction reads 1 KiB in a row instead of 64 bytes of each of 16 rows.
+                // A tile of 8 rows is half of a copied one: 128 bytes of each quarter of the k-steps of both K halves.
+                const int tile = tile0 + l_item * tstride;
+                const int tile16 = TM == TM_DUALK ? tile >> 1 : tile, row16 = TM == TM_DUALK ? (tile & 1) * 8 + (r & 7) : r;
+                const bf16_t *wp = a.w_tiles + (size_t)tile16 * 16 * K + (size_t)((kb - g * 8) / 32) * (16 * 32) + (g * 16 + row16) * 8;
 #pragma unroll
                 for (int u = 0; u < U; u++) buf.w[u] = kb + u * 32 < kr1 ? load_weights<true>(wp + u * (16 * 32)) : zero8();
             } else {
@@ -1276,8 +1278,12 @@ int launch_resident_plan(SkinnyArgs a, const ResidentPlan &p, int ntiles, const 
     return fllm_check_launch("linear_skinny");
 }
 
-// Tile-major weights serve matrices whose eight waves' K ranges are whole blocks of 128 columns.
-bool tiles_fit(int N, int K) { return N >= 16 && K >= 1024 && K % 1024 == 0; }
+// Tile-major weights serve matrices of whole k-steps of 32 columns: a wave's K range is a whole number of them, also where it
+// is no whole number of blocks of 128, and 8-row tiles take half of a copied tile, whole 128-byte lines either way.  What
+// the copies gave where only widths in steps of 1,024 and whole tiles had them before, milliseconds: prompts and answers of
+// models 1,536 wide 10.30 -> 9.57, 11.99 -> 11.57, 8.99 -> 8.51, 16.18 -> 15.61, 13.72 -> 13.11 and 7.69 -> 7.48; two decode steps
+// of the 1B sizes, whose output and down projections run in 8-row tiles, 1.53 -> 1.44.  Below 256 columns a product is its launch.
+bool tiles_fit(int N, int K) { return N >= 16 && K >= 256 && K % 32 == 0; }
 
 // tiles[T][s][lane][8] = w[16 T + lane % 16][32 s + 8 (lane / 16) ...]: tile T of 16 rows, k-step s of 32, and inside it the 16 bytes
 // of each of the 64 lanes of a wave in lane order (four steps are a block of 128 columns); rows past N are zeros
@@ -1304,10 +1310,19 @@ __global__ void __launch_bounds__(256) tile_weights_kernel(const bf16_t *__restr
     }
 }
 
-// Whether a staged launch (activations in LDS) may stream the tile-major copy: one slice, and every wave's K range whole
-// blocks of 128 columns
-bool staged_tiles_fit(const SkinnyArgs &a, const ResidentPlan &p, int n_out) {
-    return a.w_tiles != nullptr && p.S == 1 && tiles_fit(n_out, a.K) && a.K % (p.waves * 128) == 0;
+// Whether a launch may stream the tile-major copy: there is one, and K is not cut into slices
+bool streams_tiles(const SkinnyArgs &a, const ResidentPlan &p, int n_out) { return a.w_tiles != nullptr && p.S == 1 && tiles_fit(n_out, a.K); }
+
+template <int PRO, int EPI, int TM, bool XD>
+int launch_resident_form(const SkinnyArgs &a, const ResidentPlan &p, int ntiles, bool tiled, const Workspace &ws, hipStream_t stream) {
+    if constexpr (!XD) {
+        if (p.waves == 16) {
+            if (tiled) return launch_resident_plan<PRO, EPI, TM, 16, XD, true>(a, p, ntiles, ws, stream);
+            return launch_resident_plan<PRO, EPI, TM, 16, XD, false>(a, p, ntiles, ws, stream);
+        }
+    }
+    if (tiled) return launch_resident_plan<PRO, EPI, TM, 8, XD, true>(a, p, ntiles, ws, stream);
+    return launch_resident_plan<PRO, EPI, TM, 8, XD, false>(a, p, ntiles, ws, stream);
 }
 
 template <int PRO, int EPI>
@@ -1324,12 +1339,7 @@ int launch_resident(const SkinnyArgs &a, hipStream_t stream) {
     if constexpr (EPI == EPI_SWIGLU) {
         const ResidentPlan p = plan_resident(a.M, a.K, tiles8, RT, ws, false);
         if (p.S == 0) return 1;
-        if (fllm_option_resident_tiles() && staged_tiles_fit(a, p, n_out)) {    // the copy of fllm_tile_weights_gate_up
-            if (p.waves == 8) return launch_resident_plan<PRO, EPI, TM_GATEUP, 8, false, true>(a, p, tiles8, ws, stream);
-            return launch_resident_plan<PRO, EPI, TM_GATEUP, 16, false, true>(a, p, tiles8, ws, stream);
-        }
-        if (p.waves == 8) return launch_resident_plan<PRO, EPI, TM_GATEUP, 8>(a, p, tiles8, ws, stream);
-        return launch_resident_plan<PRO, EPI, TM_GATEUP, 16>(a, p, tiles8, ws, stream);
+        return launch_resident_form<PRO, EPI, TM_GATEUP, false>(a, p, tiles8, fllm_option_resident_tiles() && streams_tiles(a, p, n_out), ws, stream);
     } else {
         // bfloat16 activations are read where they lie when a workgroup sees few tiles (it reads each of them once
         // per tile: no dearer than staging for a tile or two, and nothing waits for the staging); with many tiles a
@@ -1345,32 +1355,19 @@ int launch_resident(const SkinnyArgs &a, hipStream_t stream) {
         const int slots = device_cus() * p.per_cu;
         const bool uneven = 2 * tiles16 > slots && tiles16 < 2 * slots && tiles16 % slots != 0;
         const bool dual = a.M <= 8 && p.S == 1 && fllm_option_dual_k() && (uneven || 2 * tiles16 <= device_cus());
+        const bool tiled = streams_tiles(a, p, a.N) && (x_direct || fllm_option_resident_tiles());
+        // q/k/v behind a prepared norm and the vocabulary projection: whole 16-row tiles where there is a copy, rather than
+        // 8-row tiles.  Reading the activations straight from global memory as the output projection does is slower for q/k/v
+        // (4,096 x 6,144 at 1, 8, 16 rows: 14.0, 15.4, 18.3 us against 12.4, 15.0, 18.1 staged).
+        constexpr bool kWhole = (EPI == EPI_QKV && PRO == PRO_SCALED) || (EPI == EPI_STORE_F32 && PRO == PRO_BF16);
         if constexpr (PRO == PRO_BF16) {
-            if constexpr (EPI == EPI_ADD) {     // the output and down projections: their tile-major copy, where there is one
-                if (x_direct && !dual && a.w_tiles != nullptr && tiles_fit(a.N, a.K))
-                    return launch_resident_plan<PRO, EPI, TM_ROWS16, 8, true, true>(a, p, tiles16, ws, stream);
-            }
             if (x_direct) {
-                if (dual) return launch_resident_plan<PRO, EPI, TM_DUALK, 8, true>(a, p, tiles8, ws, stream);
-                return launch_resident_plan<PRO, EPI, TM_ROWS16, 8, true>(a, p, tiles16, ws, stream);
+                if (dual) return launch_resident_form<PRO, EPI, TM_DUALK, true>(a, p, tiles8, tiled, ws, stream);
+                return launch_resident_form<PRO, EPI, TM_ROWS16, true>(a, p, tiles16, tiled, ws, stream);
             }
         }
-        if constexpr ((EPI == EPI_QKV && PRO == PRO_SCALED) || (EPI == EPI_STORE_F32 && PRO == PRO_BF16)) {
-            // q/k/v behind a prepared norm and the vocabulary projection: whole 16-row tiles from the tile-major copy,
-            // where there is one, rather than the matrix (in 8-row tiles where those fill the device better).  Reading
-            // the activations straight from global memory as the output projection does is slower for q/k/v
-            // (4,096 x 6,144 at 1, 8, 16 rows: 14.0, 15.4, 18.3 us against 12.4, 15.0, 18.1 staged).
-            if (!x_direct && fllm_option_resident_tiles() && staged_tiles_fit(a, p, a.N)) {
-                if (p.waves == 8) return launch_resident_plan<PRO, EPI, TM_ROWS16, 8, false, true>(a, p, tiles16, ws, stream);
-                return launch_resident_plan<PRO, EPI, TM_ROWS16, 16, false, true>(a, p, tiles16, ws, stream);
-            }
-        }
-        if (dual) {
-            if (p.waves == 8) return launch_resident_plan<PRO, EPI, TM_DUALK, 8>(a, p, tiles8, ws, stream);
-            return launch_resident_plan<PRO, EPI, TM_DUALK, 16>(a, p, tiles8, ws, stream);
-        }
-        if (p.waves == 8) return launch_resident_plan<PRO, EPI, TM_ROWS16, 8>(a, p, tiles16, ws, stream);
-        return launch_resident_plan<PRO, EPI, TM_ROWS16, 16>(a, p, tiles16, ws, stream);
+        if (dual && !(kWhole && tiled)) return launch_resident_form<PRO, EPI, TM_DUALK, false>(a, p, tiles8, tiled, ws, stream);
+        return launch_resident_form<PRO, EPI, TM_ROWS16, false>(a, p, tiles16, tiled, ws, stream);
     }
 }
 
@@ -1518,7 +1515,7 @@ int fllm_linear_bf16_skinny(const void *x, int ldx, const void *w, const float *
     a.x = x;
     a.ldx = ldx;
     a.w = (const bf16_t *)w;
-    a.w_tiles = M <= 16 && out_mode == 1 ? (const bf16_t *)w_tiles : nullptr;     // the form that streams it
+    a.w_tiles = M <= 16 ? (const bf16_t *)w_tiles : nullptr;      // the kernels of up to 16 rows stream it here
     a.bias = bias;
     a.out = out;
     a.ldo = ldo;
@@ -1530,13 +1527,15 @@ int fllm_linear_bf16_skinny(const void *x, int ldx, const void *w, const float *
     return dispatch<PRO_BF16, EPI_ADD>(a, stream);
 }
 
-extern "C" int fllm_linear_relu_squared(const void *x, int ldx, const void *w, void *out, int M, int N, int K, hipStream_t stream) {
+extern "C" int fllm_linear_relu_squared(const void *x, int ldx, const void *w, const void *w_tiles, void *out, int M, int N, int K,
+                                        hipStream_t stream) {
     FLLM_REQUIRE(M >= 1 && M <= 64 && N > 0 && K > 0 && K % 8 == 0 && ldx >= K && ldx % 8 == 0 && aligned16(x) && aligned16(w),
                  "linear_relu_squared: takes 1..64 rows on 16-byte boundaries and K a multiple of 8 (M=%d N=%d K=%d)", M, N, K);
     SkinnyArgs a = {};
     a.x = x;
     a.ldx = ldx;
     a.w = (const bf16_t *)w;
+    a.w_tiles = M <= 16 ? (const bf16_t *)w_tiles : nullptr;
     a.out = out;
     a.ldo = N;
     a.M = M;
@@ -1553,8 +1552,8 @@ extern "C" int fllm_fused_decode_supported(int M, int K) {
     return (M >= 1 && M <= 64 && K % 8 == 0 && K >= 8 && K <= 65536) ? 1 : 0;
 }
 
-extern "C" int fllm_norm_linear(const float *x, const float *norm_w, float eps, const void *w, const float *bias, void *out,
-                                int M, int N, int K, hipStream_t stream) {
+extern "C" int fllm_norm_linear(const float *x, const float *norm_w, float eps, const void *w, const void *w_tiles, const float *bias,
+                                void *out, int M, int N, int K, hipStream_t stream) {
     FLLM_REQUIRE(fllm_fused_decode_supported(M, K), "norm_linear: takes 1..64 rows and K a multiple of 8 (M=%d K=%d)", M, K);
     FLLM_REQUIRE(aligned16(x) && aligned16(w) && aligned16(norm_w), "norm_linear: operands must be 16-byte aligned");
     FLLM_REQUIRE(eps > 0.f, "norm_linear: eps must be positive");
@@ -1564,6 +1563,7 @@ extern "C" int fllm_norm_linear(const float *x, const float *norm_w, float eps, 
     a.norm_w = norm_w;
     a.eps = eps;
     a.w = (const bf16_t *)w;
+    a.w_tiles = M <= 16 ? (const bf16_t *)w_tiles : nullptr;
     a.bias = bias;
     a.out = out;
     a.ldo = N;
@@ -1575,7 +1575,7 @@ extern "C" int fllm_norm_linear(const float *x, const float *norm_w, float eps, 
     return rc;
 }
 
-extern "C" int fllm_norm_gate_up_swiglu(const float *x, const float *norm_w, float eps, const void *w_gate_up,
+extern "C" int fllm_norm_gate_up_swiglu(const float *x, const float *norm_w, float eps, const void *w_gate_up, const void *w_tiles,
                                         const float *bias, void *out, int M, int inter, int K, hipStream_t stream) {
     FLLM_REQUIRE(fllm_fused_decode_supported(M, K), "norm_gate_up_swiglu: takes 1..64 rows and K a multiple of 8 (M=%d K=%d)", M, K);
     FLLM_REQUIRE(aligned16(x) && aligned16(w_gate_up) && aligned16(norm_w), "norm_gate_up_swiglu: operands must be 16-byte aligned");
@@ -1587,6 +1587,7 @@ extern "C" int fllm_norm_gate_up_swiglu(const float *x, const float *norm_w, flo
     a.norm_w = norm_w;
     a.eps = eps;
     a.w = (const bf16_t *)w_gate_up;
+    a.w_tiles = M <= 16 ? (const bf16_t *)w_tiles : nullptr;
     a.bias = bias;
     a.out = out;
     a.ldo = inter;
@@ -1654,8 +1655,8 @@ SkinnyArgs qkv_args(const void *x, float eps, const void *w_qkv, const float *bi
 }
 }  // namespace
 
-extern "C" int fllm_norm_qkv_rope_store(const float *x, const float *norm_w, float eps, const void *w_qkv, const float *bias,
-                                        void *q_out, const int32_t *row_pos, const int32_t *row_seg, const int32_t *tables,
+extern "C" int fllm_norm_qkv_rope_store(const float *x, const float *norm_w, float eps, const void *w_qkv, const void *w_tiles,
+                                        const float *bias, void *q_out, const int32_t *row_pos, const int32_t *row_seg, const int32_t *tables,
                                         int table_stride, const float *cos_table, const float *sin_table, int rope_dims,
                                         void *k_pages, void *v_pages, int M, int heads, int kv_heads, int head_dim, int K,
                                         int page_size, int store_kv, hipStream_t stream) {
@@ -1668,6 +1669,7 @@ extern "C" int fllm_norm_qkv_rope_store(const float *x, const float *norm_w, flo
     SkinnyArgs a = qkv_args(x, eps, w_qkv, bias, q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table, rope_dims,
                             k_pages, v_pages, M, heads, kv_heads, head_dim, K, page_size, store_kv);
     a.norm_w = norm_w;
+    a.w_tiles = M <= 16 ? (const bf16_t *)w_tiles : nullptr;
     const int rc = dispatch<PRO_NORM_F32, EPI_QKV>(a, stream);
     FLLM_REQUIRE(rc != 1, "norm_qkv_rope_store: shape M=%d K=%d does not fit the staging area", M, K);
     return rc;
@@ -1697,7 +1699,7 @@ extern "C" size_t fllm_weight_tiles_elements_gate_up(int inter, int K) { return 
 
 // The copy for the gate/up product with its SwiGLU epilogue: w is [2 inter][K], gate rows first.
 extern "C" int fllm_tile_weights_gate_up(const void *w, void *tiles, int inter, int K, hipStream_t stream) {
-    FLLM_REQUIRE(tiles_fit(2 * inter, K), "tile_weights_gate_up: takes matrices whose width is a multiple of 1,024 (inter=%d K=%d)", inter, K);
+    FLLM_REQUIRE(tiles_fit(2 * inter, K), "tile_weights_gate_up: takes matrices whose width is a multiple of 32 from 256 on (inter=%d K=%d)", inter, K);
     FLLM_REQUIRE(w != nullptr && tiles != nullptr && aligned16(w) && aligned16(tiles), "tile_weights_gate_up: operands must be there and 16-byte aligned");
     const size_t pieces = fllm_weight_tiles_elements_gate_up(inter, K) / 8;
     const size_t want = (pieces + 255) / 256;
@@ -1779,6 +1781,17 @@ extern "C" int fllm_linear_f32_tiled(const void *x, int ldx, const void *w, cons
     const int rc = fllm_linear_bf16_skinny(x, ldx, w, bias, out, ldo, M, N, K, 1, stream, w_tiles);
     FLLM_REQUIRE(rc != 1, "linear_f32_tiled: shape M=%d K=%d does not fit the staging area", M, K);
     return rc;
+}
+
+// out = x w^T (+ bias) for 1..16 bfloat16 rows and a bfloat16 `out`, as fllm_linear in mode 0, likewise.
+extern "C" int fllm_linear_store_tiled(const void *x, int ldx, const void *w, const void *w_tiles, const float *bias, void *out, int ldo,
+                                       int M, int N, int K, hipStream_t stream) {
+    FLLM_REQUIRE(M >= 1 && M <= 16 && K % 8 == 0 && K >= 8 && ldx % 8 == 0 && ldx >= K && ldo >= N,
+                 "linear_store_tiled: takes 1..16 rows, K and ldx in steps of 8 (M=%d N=%d K=%d ldx=%d ldo=%d)", M, N, K, ldx, ldo);
+    FLLM_REQUIRE(aligned16(x) && aligned16(w) && out != nullptr && (w_tiles == nullptr || aligned16(w_tiles)),
+                 "linear_store_tiled: operands must be there and 16-byte aligned");
+    const int rc = fllm_linear_bf16_skinny(x, ldx, w, bias, out, ldo, M, N, K, 0, stream, w_tiles);
+    return rc == 1 ? fllm_linear(x, ldx, w, bias, out, ldo, M, N, K, FLLM_BF16, 0, stream) : rc;
 }
 
 extern "C" int fllm_linear_add_normed(const void *x, int ldx, const void *w, const float *bias, float *out, int M, int N, int K,
@@ -1873,8 +1886,8 @@ extern "C" int fllm_scaled_qkv_rope_store(const void *xn, const float *ssq, int 
 // g' = min(x gate^T, limit), u' = clamp(x up^T, -limit, limit) (limit <= 0: nothing is clamped); w = [gate; up] ([2 I, K]).
 // fllm_norm_gate_up_glu: x is float32 [M, K] and the RMSNorm with `norm_w` is folded in (1..64 rows).
 // fllm_gate_up_glu: x is bfloat16; 1..64 rows, or 17..128 with the tile-major copy `w_tiles` (null: without).
-extern "C" int fllm_norm_gate_up_glu(const float *x, const float *norm_w, float eps, const void *w_gate_up, const float *bias, void *out,
-                                     int M, int inter, int K, float limit, float alpha, float offset, hipStream_t stream) {
+extern "C" int fllm_norm_gate_up_glu(const float *x, const float *norm_w, float eps, const void *w_gate_up, const void *w_tiles,
+                                     const float *bias, void *out, int M, int inter, int K, float limit, float alpha, float offset, hipStream_t stream) {
     FLLM_REQUIRE(fllm_fused_decode_supported(M, K), "norm_gate_up_glu: takes 1..64 rows and K a multiple of 8 (M=%d K=%d)", M, K);
     FLLM_REQUIRE(aligned16(x) && aligned16(w_gate_up) && aligned16(norm_w), "norm_gate_up_glu: operands must be 16-byte aligned");
     FLLM_REQUIRE(eps > 0.f && inter > 0, "norm_gate_up_glu: bad eps or size");
@@ -1887,6 +1900,7 @@ extern "C" int fllm_norm_gate_up_glu(const float *x, const float *norm_w, float 
     a.norm_w = norm_w;
     a.eps = eps;
     a.w = (const bf16_t *)w_gate_up;
+    a.w_tiles = M <= 16 ? (const bf16_t *)w_tiles : nullptr;
     a.bias = bias;
     a.out = out;
     a.ldo = inter;
@@ -1919,10 +1933,8 @@ extern "C" int fllm_gate_up_glu(const void *x, int ldx, const void *w_gate_up, c
     a.M = M;
     a.N = 2 * inter;
     a.K = K;
-    if (M >= 17 && w_tiles != nullptr) {
-        a.w_tiles = (const bf16_t *)w_tiles;
-        return dispatch_wide<EPI_SWIGLU>(a, stream);
-    }
+    a.w_tiles = (const bf16_t *)w_tiles;
+    if (M >= 17 && w_tiles != nullptr) return dispatch_wide<EPI_SWIGLU>(a, stream);
     const int rc = dispatch<PRO_BF16, EPI_SWIGLU>(a, stream);
     FLLM_REQUIRE(rc != 1, "gate_up_glu: shape M=%d K=%d does not fit", M, K);
     return rc;

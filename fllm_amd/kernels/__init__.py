@@ -51,7 +51,7 @@ assert SAMPLE_ROW_BYTES == 32
 _lib = None
 
 
-ABI_VERSION = 21
+ABI_VERSION = 22
 
 
 def load_library(build_if_missing: bool = True):
@@ -103,12 +103,12 @@ def load_library(build_if_missing: bool = True):
                                  c_void, c_void, c_void, c_float, c_float, c_float, c_void],
         "fllm_attention_sloped": [c_void, c_int, c_void, c_void, c_void, c_int, c_void, c_void, c_void, c_int, c_void, c_int,
                                   c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_void, c_void],
-        "fllm_norm_linear": [c_void, c_void, c_float, c_void, c_void, c_void, c_int, c_int, c_int, c_void],
-        "fllm_norm_gate_up_swiglu": [c_void, c_void, c_float, c_void, c_void, c_void, c_int, c_int, c_int, c_void],
-        "fllm_norm_gate_up_glu": [c_void, c_void, c_float, c_void, c_void, c_void, c_int, c_int, c_int, c_float, c_float, c_float,
+        "fllm_norm_linear": [c_void, c_void, c_float, c_void, c_void, c_void, c_void, c_int, c_int, c_int, c_void],
+        "fllm_norm_gate_up_swiglu": [c_void, c_void, c_float, c_void, c_void, c_void, c_void, c_int, c_int, c_int, c_void],
+        "fllm_norm_gate_up_glu": [c_void, c_void, c_float, c_void, c_void, c_void, c_void, c_int, c_int, c_int, c_float, c_float, c_float,
                                   c_void],
         "fllm_gate_up_glu": [c_void, c_int, c_void, c_void, c_void, c_void, c_int, c_int, c_int, c_float, c_float, c_float, c_void],
-        "fllm_norm_qkv_rope_store": [c_void, c_void, c_float, c_void, c_void, c_void, c_void, c_void, c_void, c_int, c_void,
+        "fllm_norm_qkv_rope_store": [c_void, c_void, c_float, c_void, c_void, c_void, c_void, c_void, c_void, c_void, c_int, c_void,
                                      c_void, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void],
         "fllm_argmax": [c_void, c_void, c_int, c_int, c_void],
         "fllm_gate_up_swiglu": [c_void, c_int, c_void, c_void, c_void, c_int, c_int, c_int, c_void],
@@ -117,6 +117,7 @@ def load_library(build_if_missing: bool = True):
         "fllm_tile_weights_gate_up": [c_void, c_void, c_int, c_int, c_void],
         "fllm_gate_up_swiglu_tiled": [c_void, c_int, c_void, c_void, c_void, c_void, c_int, c_int, c_int, c_void],
         "fllm_linear_add_tiled": [c_void, c_int, c_void, c_void, c_void, c_void, c_int, c_int, c_int, c_int, c_void],
+        "fllm_linear_store_tiled": [c_void, c_int, c_void, c_void, c_void, c_void, c_int, c_int, c_int, c_int, c_void],
         "fllm_linear_f32_tiled": [c_void, c_int, c_void, c_void, c_void, c_void, c_int, c_int, c_int, c_int, c_void],
         "fllm_scaled_gate_up_swiglu": [c_void, c_void, c_int, c_float, c_void, c_void, c_void, c_int, c_int, c_int, c_void, c_void],
         "fllm_scaled_qkv_rope_store": [c_void, c_void, c_int, c_float, c_void, c_void, c_void, c_void, c_void, c_void, c_int, c_void,
@@ -140,7 +141,7 @@ def load_library(build_if_missing: bool = True):
         "fllm_normed_rope_store": [c_void, c_int, c_int, c_void, c_void, c_float, c_void, c_void, c_void, c_void, c_int, c_void, c_void,
                                    c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                    c_void, c_int, c_void, c_void],
-        "fllm_linear_relu_squared": [c_void, c_int, c_void, c_void, c_int, c_int, c_int, c_void],
+        "fllm_linear_relu_squared": [c_void, c_int, c_void, c_void, c_void, c_int, c_int, c_int, c_void],
         "fllm_latent_rope_store": [c_void, c_int, c_int, c_int, c_int, c_void, c_float, c_int, c_int, c_void, c_int, c_int, c_int, c_void,
                                    c_void, c_void, c_int, c_void, c_void, c_int, c_int, c_void, c_int, c_int, c_int, c_int, c_void],
         "fllm_headwise_linear": [c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_void, c_int, c_int, c_int, c_int, c_int, c_int, c_void],
@@ -313,15 +314,15 @@ class Ops:
 
     def tile_for_decode(self, w: torch.Tensor, gate_up: bool = False) -> bool:
         """Keeps beside `w` (bfloat16 [N, K] on the GPU) a copy in the order in which the products of decode steps read
-        it (`fllm_tile_weights`): `linear(..., accumulate=True)`, `linear_add_prepare`, the forms behind a prepared norm
-        and `linear` with float32 logits find it by the matrix's address and use it for steps of up to 64 rows (sums into a
-        float32 `out` and `gate_up_swiglu`: up to 128).  `gate_up`: w is [gate; up] and the copy holds 8 gate rows and the
+        it (`fllm_tile_weights`): `linear`, `linear_add_prepare`, `linear_relu_squared` and the forms behind a norm find it by
+        the matrix's address and use it for steps of up to 16 rows, and where its width is a multiple of 1,024 the sums, the
+        float32 logits and the forms behind a prepared norm for up to 64 (sums into a float32 `out` and `gate_up_swiglu`: up to 128).  `gate_up`: w is [gate; up] and the copy holds 8 gate rows and the
         same 8 up rows a tile (`fllm_tile_weights_gate_up`), for `norm_gate_up_swiglu` and `gate_up_swiglu`.  The copy is
         given up with `w`.  False: nothing was made (another type or place, a shape the kernels do not take tiles of)."""
         if not (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous()):
             return False
         N, K = w.shape
-        if not self.lib.fllm_weight_tiles_supported(N, K) or (gate_up and N % 2 != 0):
+        if not self.lib.fllm_weight_tiles_supported(N, K) or (gate_up and N % 2 != 0) or w.data_ptr() % 16 != 0:
             return False
         key = w.data_ptr()
         kind = (N, K, bool(gate_up))
@@ -338,9 +339,13 @@ class Ops:
         weakref.finalize(w, Ops._tiles.pop, key, None)
         return True
 
-    def _tiles_of(self, w: torch.Tensor, gate_up: bool = False) -> Optional[torch.Tensor]:
+    def _tiles_of(self, w: torch.Tensor, gate_up: bool = False, rows: int = 1) -> Optional[torch.Tensor]:
+        """The copy of `w` that a product of `rows` rows may read, or None: up to 16 rows any, beyond them those whose widths the chunk
+        kernels were measured at beside the GEMM library (steps of 1,024)."""
         held = Ops._tiles.get(w.data_ptr())
-        return held[1] if held is not None and held[0] == (w.shape[0], w.shape[1], bool(gate_up)) else None
+        if held is None or held[0] != (w.shape[0], w.shape[1], bool(gate_up)) or (rows > self.PREPARED_NORM_ROWS and w.shape[1] % 1024 != 0):
+            return None
+        return held[1]
 
     # 17 to 128 rows beside the GEMM library: with the tile-major copies the own products of the feed-forward (gate/up
     # with its SwiGLU epilogue, down with the residual sum) are faster than the library's products and the SwiGLU kernel
@@ -354,7 +359,7 @@ class Ops:
         return (self.library_gemm_from is not None and self.library_gemm_from <= rows <= self.GATE_UP_SWIGLU_TILED_ROWS and bool(Ops._tiles)
                 and (rows <= 64 or (w_gate_up.shape[1] % 256 == 0 and w_down.shape[1] % 256 == 0))
                 and w_gate_up.numel() * w_gate_up.element_size() >= self.OWN_GATE_UP_BYTES
-                and self._tiles_of(w_gate_up, gate_up=True) is not None and self._tiles_of(w_down) is not None)
+                and self._tiles_of(w_gate_up, gate_up=True, rows=rows) is not None and self._tiles_of(w_down, rows=rows) is not None)
 
     def set_fast_kernels(self, on: bool) -> None:
         """Off: bfloat16 calls run the plain kernels (tests compare the two)."""
@@ -463,10 +468,10 @@ class Ops:
             _dense(bias, "bias", torch.float32, (N,))
         ldx = x.stride(0) if M > 1 else K
         ldo = out.stride(0) if M > 1 else N
-        tiles = (self._tiles_of(w) if Ops._tiles and ((mode == OUT_ADD_F32 and M <= self.ADD_KERNEL_ROWS) or (mode == OUT_STORE_F32 and M <= 64))
-                 else None)
-        if tiles is not None and ldx % 8 == 0 and K % 8 == 0 and (M <= 64 or K % 256 == 0):
-            entry = self.lib.fllm_linear_add_tiled if mode == OUT_ADD_F32 else self.lib.fllm_linear_f32_tiled
+        most = self.ADD_KERNEL_ROWS if mode == OUT_ADD_F32 else 64 if mode == OUT_STORE_F32 else self._store_tiled_rows()
+        tiles = self._tiles_of(w, rows=M) if Ops._tiles and M <= most else None
+        if tiles is not None and ldx % 8 == 0 and x.data_ptr() % 16 == 0 and (M <= 64 or K % 256 == 0):
+            entry = (self.lib.fllm_linear_store_tiled, self.lib.fllm_linear_f32_tiled, self.lib.fllm_linear_add_tiled)[mode]
             self._check(entry(_ptr(x), ldx, _ptr(w), _ptr(tiles), _ptr(bias), _ptr(out), ldo, M, N, K, self._stream()))
             return out
         if (self.library_gemm_from is not None and M >= self.library_gemm_from and x.dtype == torch.bfloat16
@@ -484,6 +489,10 @@ class Ops:
         self._check(self.lib.fllm_linear(_ptr(x), ldx, _ptr(w), _ptr(bias), _ptr(out), ldo, M, N, K, _DTYPE_CODE[x.dtype],
                                          mode, self._stream()))
         return out
+
+    def _store_tiled_rows(self) -> int:
+        """Rows up to which a product stored as bfloat16 reads the tile-major copy: those that do not go to the GEMM library."""
+        return min(self.PREPARED_NORM_ROWS, (self.library_gemm_from or 17) - 1)
 
     # ---- products of many rows with the activation in the epilogue ---------------------------------
     def _tiles_take(self, code: int) -> bool:
@@ -542,7 +551,7 @@ class Ops:
         N = w.shape[0]
         M, K = self._fused_operands(x, norm_weight, w, bias, N)
         _dense(out, "out", torch.bfloat16, (M, N))
-        self._check(self.lib.fllm_norm_linear(_ptr(x), _ptr(norm_weight), float(eps), _ptr(w), _ptr(bias), _ptr(out), M, N, K,
+        self._check(self.lib.fllm_norm_linear(_ptr(x), _ptr(norm_weight), float(eps), _ptr(w), self._few_tiles(w, M), _ptr(bias), _ptr(out), M, N, K,
                                               self._stream()))
         return out
 
@@ -563,7 +572,7 @@ class Ops:
             return "resident"
         if (self.fused_decode_rows < rows <= self.CHUNK_ROWS and (self.library_gemm_from is None or rows >= self.library_gemm_from)
                 and self.fused_decode_rows >= self.PREPARED_NORM_ROWS and width % 256 == 0 and Ops._tiles
-                and self._tiles_of(w, gate_up=gate_up) is not None):
+                and self._tiles_of(w, gate_up=gate_up, rows=rows) is not None):
             return "chunks"
         return None
 
@@ -607,8 +616,12 @@ class Ops:
         parts = ctypes.c_int(0)
         self._check(self.lib.fllm_linear_add_normed(_ptr(x), x.stride(0) if M > 1 else K, _ptr(w), _ptr(bias), _ptr(residual), M, N,
                                                     K, _ptr(next_norm_weight), _ptr(xn), _ptr(ssq), ctypes.addressof(parts),
-                                                    _ptr(self._tiles_of(w)) if Ops._tiles else None, self._stream()))
+                                                    _ptr(self._tiles_of(w, rows=M)) if Ops._tiles else None, self._stream()))
         return PreparedNorm(xn, ssq, int(parts.value))
+
+    def _few_tiles(self, w: torch.Tensor, rows: int, gate_up: bool = False):
+        """The tile-major copy for the products of up to 16 rows that take one beside the matrix, or None."""
+        return _ptr(self._tiles_of(w, gate_up=gate_up)) if Ops._tiles and rows <= self.PREPARED_NORM_ROWS else None
 
     def _prepared_operands(self, prepared: PreparedNorm, w, bias, n_rows_w):
         M, K = prepared.x.shape
@@ -624,7 +637,7 @@ class Ops:
     def _chunk_tiles(self, M: int, K: int, w: torch.Tensor, gate_up: bool = False) -> Optional[torch.Tensor]:
         """The tile-major copy that a prepared norm of more than 16 rows needs; up to 16 rows the kernel streams it
         where there is one and the launch it chooses can."""
-        tiles = self._tiles_of(w, gate_up=gate_up) if Ops._tiles else None
+        tiles = self._tiles_of(w, gate_up=gate_up, rows=M) if Ops._tiles else None
         if M <= self.PREPARED_NORM_ROWS:
             return tiles
         _need(tiles is not None and K % 256 == 0,
@@ -645,8 +658,8 @@ class Ops:
             return out
         M, K = self._fused_operands(x, norm_weight, w_gate_up, bias, two_i)
         _dense(out, "out", torch.bfloat16, (M, two_i // 2))
-        self._check(self.lib.fllm_norm_gate_up_swiglu(_ptr(x), _ptr(norm_weight), float(eps), _ptr(w_gate_up), _ptr(bias),
-                                                      _ptr(out), M, two_i // 2, K, self._stream()))
+        self._check(self.lib.fllm_norm_gate_up_swiglu(_ptr(x), _ptr(norm_weight), float(eps), _ptr(w_gate_up), self._few_tiles(w_gate_up, M, True),
+                                                      _ptr(bias), _ptr(out), M, two_i // 2, K, self._stream()))
         return out
 
     GATE_UP_SWIGLU_ROWS = 64          # from the matrix as the checkpoint has it
@@ -675,7 +688,7 @@ class Ops:
             _dense(bias, "bias", torch.float32, (two_i,))
         _dense(out, "out", torch.bfloat16, (M, two_i // 2))
         _need(1 <= M <= self.GATE_UP_SWIGLU_TILED_ROWS and K % 8 == 0, f"gate_up_swiglu takes 1..128 rows and widths in steps of 8, not {M} x {K}")
-        tiles = self._tiles_of(w_gate_up, gate_up=True) if M >= 17 and Ops._tiles else None
+        tiles = self._tiles_of(w_gate_up, gate_up=True, rows=M) if M >= 17 and Ops._tiles else None
         _need(M <= 64 or (tiles is not None and K % 256 == 0 and x.stride(0) % 8 == 0),
               f"gate_up_swiglu takes more than 64 rows only with the tile-major copy of the matrix and widths in steps of 256, not {M} x {K}")
         if tiles is not None and x.stride(0) % 8 == 0:
@@ -694,7 +707,8 @@ class Ops:
         _need(two_i % 2 == 0, "w_gate_up needs an even number of rows")
         M, K = self._fused_operands(x, norm_weight, w_gate_up, bias, two_i)
         _dense(out, "out", torch.bfloat16, (M, two_i // 2))
-        self._check(self.lib.fllm_norm_gate_up_glu(_ptr(x), _ptr(norm_weight), float(eps), _ptr(w_gate_up), _ptr(bias), _ptr(out), M,
+        self._check(self.lib.fllm_norm_gate_up_glu(_ptr(x), _ptr(norm_weight), float(eps), _ptr(w_gate_up),
+                                                   self._few_tiles(w_gate_up, M, True), _ptr(bias), _ptr(out), M,
                                                    two_i // 2, K, float(limit), float(alpha), float(up_offset), self._stream()))
         return out
 
@@ -711,7 +725,7 @@ class Ops:
             _dense(bias, "bias", torch.float32, (two_i,))
         _dense(out, "out", torch.bfloat16, (M, two_i // 2))
         _need(1 <= M <= self.GATE_UP_SWIGLU_TILED_ROWS and K % 8 == 0, f"gate_up_glu takes 1..128 rows and widths in steps of 8, not {M} x {K}")
-        tiles = self._tiles_of(w_gate_up, gate_up=True) if M >= 17 and Ops._tiles else None
+        tiles = self._tiles_of(w_gate_up, gate_up=True, rows=M) if Ops._tiles else None
         _need(M <= 64 or (tiles is not None and K % 256 == 0),
               f"gate_up_glu takes more than 64 rows only with the tile-major copy of the matrix and widths in steps of 256, not {M} x {K}")
         self._check(self.lib.fllm_gate_up_glu(_ptr(x), x.stride(0) if M > 1 else K, _ptr(w_gate_up), _ptr(tiles), _ptr(bias), _ptr(out),
@@ -747,7 +761,7 @@ class Ops:
                 kv_heads, head_dim, K, page_size, 1 if store else 0, _ptr(self._chunk_tiles(M, K, w_qkv)), self._stream()))
             return q_out
         self._check(self.lib.fllm_norm_qkv_rope_store(
-            _ptr(x), _ptr(norm_weight), float(eps), _ptr(w_qkv), _ptr(bias), _ptr(q_out), _ptr(row_pos), _ptr(row_seg),
+            _ptr(x), _ptr(norm_weight), float(eps), _ptr(w_qkv), self._few_tiles(w_qkv, M), _ptr(bias), _ptr(q_out), _ptr(row_pos), _ptr(row_seg),
             _ptr(tables), tables.shape[1], _ptr(cos), _ptr(sin), rope_dims, _ptr(k_pages), _ptr(v_pages), M, heads, kv_heads,
             head_dim, K, page_size, 1 if store else 0, self._stream()))
         return q_out
@@ -1537,7 +1551,8 @@ class Ops:
         _need(x.is_cuda and x.stride(1) == 1, "x must be rows on the GPU")
         _dense(w, "w", torch.bfloat16, (N, K))
         _dense(out, "out", torch.bfloat16, (M, N))
-        self._check(self.lib.fllm_linear_relu_squared(_ptr(x), x.stride(0) if M > 1 else K, _ptr(w), _ptr(out), M, N, K, self._stream()))
+        self._check(self.lib.fllm_linear_relu_squared(_ptr(x), x.stride(0) if M > 1 else K, _ptr(w), self._few_tiles(w, M), _ptr(out), M, N, K,
+                                                      self._stream()))
         return True
 
     def activation(self, x: torch.Tensor, out: torch.Tensor, kind: str = "relu2") -> torch.Tensor:

@@ -1,0 +1,78 @@
+"""Products of up to 16 rows from the tile-major copies of matrices of any width in steps of 32: every epilogue and prologue, tiles of 16 and
+of 8 rows (both halves of a copied tile, a last one that is not whole), K ranges of the waves that are no whole blocks of 128 columns and ranges
+that end early, activations staged and read where they lie.  The copy holds the same numbers and the launch multiplies them in the same
+order, so all forms but two give the same bits as without it; the two that take whole tiles where there is a copy are held against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+BF16 = torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from fllm_amd.kernels import Ops
+    return Ops()
+
+
+def draw(shape, seed, scale=1.0, dtype=BF16):
+    return (torch.randn(*shape, generator=torch.Generator().manual_seed(seed)) * scale).to(dtype).to(DEV)
+
+
+# K: whole steps of 32 in every way eight (and sixteen) waves share them out; N: fewer tiles than half of the compute units, as many as fill
+# them unevenly, more than are read where they lie
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(16, 256), (40, 288), (1000, 544), (1536, 1536), (6150, 1568), (1528, 8960), (16500, 1056), (96, 13312)])
+def test_plain_products(ops, M, N, K):
+    x, w, bias = draw((M, K), M + K), draw((N, K), N + K, K ** -0.5), draw((N,), N, 0.3, torch.float32)
+    start = draw((M, N), 5, 1.0, torch.float32)
+    exact = x.double() @ w.double().T + bias.double()
+
+    def forms():
+        stored = ops.linear(x, w, torch.empty(M, N, dtype=BF16, device=DEV), bias=bias)
+        added = ops.linear(x, w, start.clone(), bias=bias, accumulate=True)
+        squared = torch.empty(M, N, dtype=BF16, device=DEV)
+        assert ops.linear_relu_squared(x, w, squared)
+        return stored, added, squared, ops.linear(x, w, torch.empty(M, N, device=DEV), bias=bias)
+
+    plain = forms()
+    assert ops.tile_for_decode(w)
+    tiled = forms()
+    for a, b in zip(plain[:3], tiled[:3]):
+        assert torch.equal(a, b)
+    # sums of K products of about K^-1/2: float32 rounding errors of K additions, in any order, stay far below this
+    torch.testing.assert_close(tiled[3].double(), exact, rtol=0, atol=2.0 ** -24 * K ** 0.5 * 16)
+    torch.testing.assert_close(tiled[0].double(), exact, rtol=2.0 ** -8, atol=1e-5)
+
+
+@pytest.mark.parametrize("M", [1, 8, 12])
+@pytest.mark.parametrize("N,K", [(48, 256), (1216, 1536), (4600, 2080), (17920, 1536)])
+def test_behind_a_norm(ops, M, N, K):
+    x, nw = draw((M, K), M, 2.0, torch.float32), draw((K,), K, 0.1, torch.float32) + 1
+    w = draw((N, K), N, K ** -0.5)
+
+    def forms():      # of the matrix `w` of the moment
+        wide = ops.norm_linear(x, nw, 1e-5, w, torch.empty(M, N, dtype=BF16, device=DEV))
+        gated = ops.norm_gate_up_glu(x, nw, 1e-5, w, torch.empty(M, N // 2, dtype=BF16, device=DEV), 7.0, 1.7, 1.0)
+        swi = ops.norm_gate_up_swiglu(x, nw, 1e-5, w, torch.empty(M, N // 2, dtype=BF16, device=DEV))
+        glu = ops.gate_up_glu(x.to(BF16), w, torch.empty(M, N // 2, dtype=BF16, device=DEV), 7.0, 1.7, 1.0)
+        return wide, gated, swi, glu
+
+    plain = forms()
+    assert ops.tile_for_decode(w)
+    assert torch.equal(plain[0], forms()[0])
+    w = w.clone()
+    assert ops.tile_for_decode(w, gate_up=True)
+    for a, b in zip(plain, forms()):
+        assert torch.equal(a, b)
+
+
+def test_what_is_read_beside_the_copy_stays_accepted(ops):
+    """Rows that begin off 16 bytes have no 16-byte loads: they take the plain kernel, copy or not; a matrix that does gets no copy."""
+    w = draw((64, 512), 1)
+    assert ops.tile_for_decode(w)
+    x = draw((3 * 512 + 1,), 2)[1:].view(3, 512)
+    out = ops.linear(x, w, torch.empty(3, 64, dtype=BF16, device=DEV))
+    torch.testing.assert_close(out.double(), x.double() @ w.double().T, rtol=2.0 ** -8, atol=1e-4)
+    assert not ops.tile_for_decode(draw((64 * 512 + 1,), 3)[1:].view(64, 512))
