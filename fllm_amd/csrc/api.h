@@ -463,6 +463,11 @@ int fllm_linear_tiles(const void *x, int ldx, const void *w, const float *bias, 
 int fllm_experts_stream(const void *h, int ldh, const int32_t *ids, const float *weights, int rows, int top, const void *w_up,
                         const void *w_down, int E, int inter, int K, int N, int gated, void *act, float *out, float limit, float alpha,
                         float up_offset, hipStream_t stream);
+// The same for experts without a gate beside a shared expert of `shared` lanes that every row uses: out float32 [rows * (top + 1), N], a row's
+// picks times their weights and behind them the shared expert's output; act has rows * shared elements more.  1..16 rows.
+int fllm_experts_stream_shared(const void *h, int ldh, const int32_t *ids, const float *weights, int rows, int top, const void *w_up,
+                               const void *w_down, int E, int inter, int K, int N, const void *w_shared_up, const void *w_shared_down,
+                               int shared, void *act, float *out, hipStream_t stream);
 
 // ---- layer norms and the small passes around them (layer_norms.hip) ----
 // out1[i] = (x[r] - mean) * rsqrt(mean (x[r] - mean)^2 + eps1) * w1, r = rows ? rows[i] : i, and with w2 the same with w2 and eps2 in out2.

@@ -27,11 +27,18 @@ constexpr int kMostPairs = 512;
 // MODE 2: act[pair, c] = relu(w[e][c] . h[pair / top])^2, w [E][N][K]
 // w is tile-major: [16 rows][K / 32] blocks of 64 lanes x 8 values (fllm_tile_weights' order; rows and K whole tiles).
 // G: groups of 16 pairs that share a load of the weights.
-template <int MODE, int G>
+// SHARED (modes 1 and 2): one more expert, which every row uses, is the last row of workgroups: its matrix [shared_n][shared_k] is
+// w_shared, its activations lie behind the pairs'.  A row's outputs are then top + 1 neighbouring rows of `out`, the picks' times
+// out_weights[pair], so that one sum of a row's parts is all that follows: of one layer's launches (2 rows, 8 experts and a shared one of
+// 4,480 lanes at a width of 1,536) two products of 6 to 8 us and a sum of 4 are gone
+// (a prompt and eight decode steps of twelve such layers 15.6 -> 14.5 ms).
+template <int MODE, int G, bool SHARED>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
 expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__restrict__ ids, const float *__restrict__ weights, int pairs,
-                     int top, const bf16_t *__restrict__ w, int E, int N, int K, int k_per, int by_pair, bf16_t *__restrict__ act,
-                     float *__restrict__ out, float limit, float alpha, float up_offset) {
+                     int top, const bf16_t *__restrict__ w, int E, int N, int K, int by_pair, bf16_t *__restrict__ act,
+                     float *__restrict__ out, float limit, float alpha, float up_offset, const bf16_t *__restrict__ w_shared, int shared_n,
+                     int shared_k, const float *__restrict__ out_weights, int out_top) {
+    static_assert(!SHARED || MODE != 0, "a shared expert comes with experts without a gate");
     constexpr int RT = MODE == 1 ? 1 : 2;                  // 16-row weight tiles a workgroup
     constexpr int COLS = MODE == 2 ? 32 : 16;              // output columns a workgroup
     constexpr int U = MODE == 0 && G > 1 ? 3 : 6;          // products a wave asks for at a time (two tiles, two groups: 128 registers)
@@ -46,8 +53,20 @@ expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__res
         return e < 0 ? 0 : (e >= E ? E - 1 : e);           // never outside the stack of experts
     };
     // blockIdx.y names an expert, or (by_pair) a pair: then the first pair of an expert stands for it
-    const int e = by_pair ? expert_of(blockIdx.y) : (int)blockIdx.y;
-    if (wave == 0) {
+    const bool shared = SHARED && blockIdx.y == gridDim.y - 1;
+    const int e = shared ? 0 : by_pair ? expert_of(blockIdx.y) : (int)blockIdx.y;
+    if (shared) {                                          // every row: `pairs` and the pointers become the shared expert's own
+        if (MODE == 1) x += (size_t)pairs * ldx;
+        if (MODE == 2) act += (size_t)pairs * N;
+        pairs = pairs / out_top;
+        if (MODE == 1) ldx = shared_k;
+        w = w_shared;
+        N = shared_n;
+        K = shared_k;
+        top = 1;
+        if ((int)threadIdx.x < pairs) s_pair[threadIdx.x] = (short)threadIdx.x;
+        if (threadIdx.x == 0) s_count = pairs;
+    } else if (wave == 0) {
         int count = 0;
         for (int p0 = 0; p0 < pairs; p0 += kWave) {
             const int p = p0 + lane;
@@ -60,7 +79,8 @@ expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__res
     }
     __syncthreads();
     const int count = s_count;
-    if (count == 0 || (by_pair && s_pair[0] != (int)blockIdx.y)) return;
+    if (count == 0 || (by_pair && !shared && s_pair[0] != (int)blockIdx.y)) return;
+    if (SHARED && c0 >= N) return;                         // the grid covers the wider of the two kinds of experts
 
     const bf16_t *tiles[RT];
 #pragma unroll
@@ -68,6 +88,7 @@ expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__res
         const int c = min(c0 + (MODE == 2 ? 16 * t : 0), N - 16);      // a tile beyond the matrix reads its last one again
         tiles[t] = w + ((size_t)e * (MODE == 0 ? 2 : 1) * N + (MODE == 0 && t == 1 ? N : 0) + c) * K + lane * 8;
     }
+    const int k_per = ((K + kWaves - 1) / kWaves + 31) / 32 * 32;
     const int k_begin = wave * k_per, k_end = min(K, k_begin + k_per);
     for (int g0 = 0; g0 < count; g0 += 16 * G) {
         const bf16_t *src[G];
@@ -127,7 +148,8 @@ expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__res
                     v += red[s][MODE == 2 ? tile : 0][from][at];
                     if (MODE == 0) u += red[s][RT - 1][from][at];
                 }
-                const size_t to = (size_t)s_pair[g0 + 16 * g + n] * N + c0 + m;
+                const int pair = s_pair[g0 + 16 * g + n];
+                const size_t to = (size_t)pair * N + c0 + m;
                 if (MODE == 0) {
                     if (limit > 0.f) {
                         v = fminf(v, limit);
@@ -137,6 +159,9 @@ expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__res
                 } else if (MODE == 2) {
                     v = fmaxf(v, 0.f);
                     act[to] = (bf16_t)(v * v);
+                } else if (SHARED) {
+                    const int row = shared ? pair : pair / out_top, part = shared ? out_top : pair - row * out_top;
+                    out[((size_t)row * (out_top + 1) + part) * N + c0 + m] = shared ? v : v * out_weights[pair];
                 } else {
                     out[to] = v;
                 }
@@ -145,22 +170,28 @@ expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__res
     }
 }
 
-template <int MODE, int G>
+struct Shared {
+    const void *w = nullptr;
+    int n = 0, k = 0;
+    const float *out_weights = nullptr;
+    int top = 1;
+};
+
+template <int MODE, int G, bool SHARED>
 void launch_groups(const void *x, int ldx, const int32_t *ids, const float *weights, long pairs, int top, const void *w, int E, int N, int K,
-            void *act, float *out, float limit, float alpha, float up_offset, hipStream_t stream) {
+                   void *act, float *out, float limit, float alpha, float up_offset, const Shared &sh, hipStream_t stream) {
     const int by_pair = pairs < E;
-    const int cols = MODE == 2 ? 32 : 16;
-    const int k_per = ((K + kWaves - 1) / kWaves + 31) / 32 * 32;
-    hipLaunchKernelGGL((expert_stream_kernel<MODE, G>), dim3((N + cols - 1) / cols, by_pair ? (unsigned)pairs : (unsigned)E), dim3(kThreads), 0,
-                       stream, (const bf16_t *)x, ldx, ids, weights, (int)pairs, top, (const bf16_t *)w, E, N, K, k_per, by_pair,
-                       (bf16_t *)act, out, limit, alpha, up_offset);
+    const int cols = MODE == 2 ? 32 : 16, widest = sh.n > N ? sh.n : N;
+    hipLaunchKernelGGL((expert_stream_kernel<MODE, G, SHARED>), dim3((widest + cols - 1) / cols, (by_pair ? (unsigned)pairs : (unsigned)E) + (SHARED ? 1 : 0)),
+                       dim3(kThreads), 0, stream, (const bf16_t *)x, ldx, ids, weights, (int)pairs, top, (const bf16_t *)w, E, N, K, by_pair,
+                       (bf16_t *)act, out, limit, alpha, up_offset, (const bf16_t *)sh.w, sh.n, sh.k, sh.out_weights, sh.top);
 }
 
-template <int MODE>
+template <int MODE, bool SHARED = false>
 void launch(int groups, const void *x, int ldx, const int32_t *ids, const float *weights, long pairs, int top, const void *w, int E, int N,
-            int K, void *act, float *out, float limit, float alpha, float up_offset, hipStream_t stream) {
-    if (groups == 1) launch_groups<MODE, 1>(x, ldx, ids, weights, pairs, top, w, E, N, K, act, out, limit, alpha, up_offset, stream);
-    else launch_groups<MODE, 2>(x, ldx, ids, weights, pairs, top, w, E, N, K, act, out, limit, alpha, up_offset, stream);
+            int K, void *act, float *out, float limit, float alpha, float up_offset, hipStream_t stream, const Shared &sh = Shared()) {
+    if (groups == 1) launch_groups<MODE, 1, SHARED>(x, ldx, ids, weights, pairs, top, w, E, N, K, act, out, limit, alpha, up_offset, sh, stream);
+    else if constexpr (!SHARED) launch_groups<MODE, 2, SHARED>(x, ldx, ids, weights, pairs, top, w, E, N, K, act, out, limit, alpha, up_offset, sh, stream);
 }
 
 }  // namespace
@@ -192,4 +223,29 @@ extern "C" int fllm_experts_stream(const void *h, int ldh, const int32_t *ids, c
     else launch<2>(groups, h, ldh, ids, nullptr, pairs, top, w_up, E, inter, K, act, nullptr, 0.f, 0.f, 0.f, stream);
     launch<1>(groups, act, inter, ids, nullptr, pairs, 1, w_down, E, N, inter, nullptr, out, 0.f, 0.f, 0.f, stream);
     return fllm_check_launch("experts_stream");
+}
+
+// The same for experts without a gate beside a shared expert (w_shared_up [shared, K], w_shared_down [N, shared], both tile-major) whose
+// output counts once for every row: out float32 [rows * (top + 1), N], row r's picks times their weights and then the shared expert's
+// output; act bfloat16 [rows * top * inter + rows * shared] (scratch).  1..16 rows.
+extern "C" int fllm_experts_stream_shared(const void *h, int ldh, const int32_t *ids, const float *weights, int rows, int top, const void *w_up,
+                                          const void *w_down, int E, int inter, int K, int N, const void *w_shared_up,
+                                          const void *w_shared_down, int shared, void *act, float *out, hipStream_t stream) {
+    FLLM_REQUIRE(rows >= 0 && top > 0 && E > 0 && inter > 0 && K > 0 && N > 0 && shared > 0 && ldh >= K, "experts_stream_shared: bad sizes");
+    FLLM_REQUIRE(h && ids && weights && w_up && w_down && w_shared_up && w_shared_down && act && out, "experts_stream_shared: operands missing");
+    if (!fllm_fast_kernels_enabled()) return 1;
+    // 16 rows meet the shared expert's weights in one pass, and a row's pairs fit into one group of 16 an expert
+    if (rows > 16 || K % 32 != 0 || inter % 32 != 0 || shared % 32 != 0 || K < 32 * kWaves || inter < 32 * kWaves || shared < 32 * kWaves ||
+        N % 16 != 0 || ldh % 8 != 0 || E > 4096)
+        return 1;
+    if ((((uintptr_t)h | (uintptr_t)w_up | (uintptr_t)w_down | (uintptr_t)w_shared_up | (uintptr_t)w_shared_down | (uintptr_t)act) & 15) != 0) return 1;
+    const long pairs = (long)rows * top;
+    if (pairs == 0) return 0;
+    if (pairs > kMostPairs || pairs > 16L * E) return 1;
+    Shared up, down;
+    up.w = w_shared_up, up.n = shared, up.k = K, up.top = top;
+    down.w = w_shared_down, down.n = N, down.k = shared, down.top = top, down.out_weights = weights;
+    launch<2, true>(1, h, ldh, ids, nullptr, pairs, top, w_up, E, inter, K, act, nullptr, 0.f, 0.f, 0.f, stream, up);
+    launch<1, true>(1, act, inter, ids, nullptr, pairs, 1, w_down, E, N, inter, nullptr, out, 0.f, 0.f, 0.f, stream, down);
+    return fllm_check_launch("experts_stream_shared");
 }

@@ -51,7 +51,7 @@ assert SAMPLE_ROW_BYTES == 32
 _lib = None
 
 
-ABI_VERSION = 22
+ABI_VERSION = 23
 
 
 def load_library(build_if_missing: bool = True):
@@ -187,6 +187,8 @@ def load_library(build_if_missing: bool = True):
                                c_void],
         "fllm_gate_up_tiles": [c_void, c_int, c_void, c_void, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_void],
         "fllm_linear_tiles": [c_void, c_int, c_void, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_int, c_void],
+        "fllm_experts_stream_shared": [c_void, c_int, c_void, c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_void, c_void,
+                                       c_int, c_void, c_void, c_void],
         "fllm_experts_stream": [c_void, c_int, c_void, c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_void,
                                 c_void, c_float, c_float, c_float, c_void],
         "fllm_experts_grouped_ungated": [c_void, c_int, c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_void, c_void,
@@ -1097,6 +1099,48 @@ class Ops:
         code = self.lib.fllm_experts_stream(_ptr(h), h.stride(0) if rows > 1 else K, _ptr(ids), _ptr(weights), rows, top, _ptr(up_tiles),
                                             _ptr(down_tiles), E, inter, K, N, 1 if gated else 0, _ptr(act), _ptr(out), float(limit),
                                             float(alpha), float(up_offset), self._stream())
+        if code == 1:
+            return False
+        self._check(code)
+        return True
+
+    STREAM_SHARED_ROWS = 16      # the shared expert's weights meet all rows in one pass
+    STREAM_SHARED_PICKS = 3      # with the shared expert's output four parts a row, what `postnorm_add` sums in registers
+
+    def experts_stream_shared_takes(self, rows: int, top: int, w_up: torch.Tensor, w_down: torch.Tensor, w_shared_up: torch.Tensor,
+                                    w_shared_down: torch.Tensor) -> bool:
+        """Whether `experts_stream_shared` serves a bfloat16 step of `rows` rows with `top` picks each."""
+        if not 1 <= rows <= self.STREAM_SHARED_ROWS or top > self.STREAM_SHARED_PICKS or not Ops._tiles or w_up.dtype != torch.bfloat16:
+            return False
+        E, inter, K = w_up.shape
+        shared = w_shared_up.shape[0]
+        return (rows * top <= 16 * E and all(n % 32 == 0 and n >= 256 for n in (K, inter, shared)) and w_down.shape[1] % 16 == 0
+                and self._expert_tiles_of(w_up) is not None and self._expert_tiles_of(w_down) is not None
+                and self._tiles_of(w_shared_up) is not None and self._tiles_of(w_shared_down) is not None)
+
+    def experts_stream_shared(self, h: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
+                              w_shared_up: torch.Tensor, w_shared_down: torch.Tensor, out: torch.Tensor) -> bool:
+        """`experts_stream` of experts without a gate beside a shared expert (w_shared_up [shared, K], w_shared_down [N, shared]) in the
+        same two launches: out float32 [rows * (top + 1), N], a row's picks times their weights and behind them the shared expert's
+        output.  False: not taken, nothing was written."""
+        rows, K = h.shape
+        top = ids.shape[1]
+        if h.dtype != torch.bfloat16 or not h.is_cuda or not self.experts_stream_shared_takes(rows, top, w_up, w_down, w_shared_up, w_shared_down):
+            return False
+        E, inter, N, shared = w_up.shape[0], w_up.shape[1], w_down.shape[1], w_shared_up.shape[0]
+        _need(h.dim() == 2 and h.stride(1) == 1, "h must be a row-major matrix")
+        _dense(w_up, "w_up", h.dtype, (E, inter, K))
+        _dense(w_down, "w_down", h.dtype, (E, N, inter))
+        _dense(w_shared_up, "w_shared_up", h.dtype, (shared, K))
+        _dense(w_shared_down, "w_shared_down", h.dtype, (N, shared))
+        _dense(ids, "ids", torch.int32, (rows, top))
+        _dense(weights, "weights", torch.float32, (rows, top))
+        _dense(out, "out", torch.float32, (rows * (top + 1), N))
+        act = torch.empty((rows * (top * inter + shared),), dtype=h.dtype, device=h.device)
+        code = self.lib.fllm_experts_stream_shared(_ptr(h), h.stride(0) if rows > 1 else K, _ptr(ids), _ptr(weights), rows, top,
+                                                   _ptr(self._expert_tiles_of(w_up)), _ptr(self._expert_tiles_of(w_down)), E, inter, K, N,
+                                                   _ptr(self._tiles_of(w_shared_up)), _ptr(self._tiles_of(w_shared_down)), shared, _ptr(act),
+                                                   _ptr(out), self._stream())
         if code == 1:
             return False
         self._check(code)

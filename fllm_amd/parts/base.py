@@ -32,7 +32,8 @@ Roles and their interfaces:
                 `branch=t` (float32) and then STORES its output in t instead of adding it to `residual` (which may be
                 None), for arrangements that treat a part's output before it joins the stream (a norm behind the part).
                 t has `branch_parts` rows a token (1 unless the part says otherwise: a token's experts leave their
-                outputs one after the other, and whoever adds the branch sums them in that order).  An arrangement hands
+                outputs one after the other, and whoever adds the branch sums them in that order; `branch_parts_for(rows)`, where
+                a part has it, says how many for a step of that many rows).  An arrangement hands
                 a part without the attribute a zeroed stand-in for the stream, so every part fits.
   block         forward(ctx, residual_f32[R,H], binding) runs norms, mixer and feed-forward.  It is built with
                 mixer=, feed_forward= (None for a layer without one), norms= (by the names the layer's spec

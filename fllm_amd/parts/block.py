@@ -204,7 +204,9 @@ class SandwichBlock(Block):
         return None          # this block's first norm rides on the sum before it only inside the block itself
 
     def _branch(self, part, rows):
-        return self.rt.empty((rows * int(getattr(part, "branch_parts", 1)), self.size), torch.float32)
+        parts_for = getattr(part, "branch_parts_for", None)          # a part may leave more rows a token in steps of few rows
+        parts = parts_for(rows) if parts_for is not None else getattr(part, "branch_parts", 1)
+        return self.rt.empty((rows * int(parts), self.size), torch.float32)
 
     def forward(self, ctx, residual, binding):
         rt, ops = self.rt, self.rt.ops

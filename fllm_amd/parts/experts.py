@@ -97,6 +97,7 @@ class RoutedExperts(FeedForward):
             self.w_shared_up = rt.matrix(weights["shared_up"])
             self.w_shared_down = rt.matrix(weights["shared_down"])
             rt.tile_for_decode(self.w_shared_down)
+            rt.tile_for_decode(self.w_shared_up, priority=1)
 
     @property
     def branch_parts(self) -> int:
@@ -104,9 +105,31 @@ class RoutedExperts(FeedForward):
         other, and whoever adds the branch to the stream sums them in pick order."""
         return self.top if self.weight_on == "input" else 1
 
+    def branch_parts_for(self, rows: int) -> int:
+        """The same for a step of `rows` rows: where picks and a shared expert stream together (decode steps), every pick's
+        weighted output and the shared expert's wait for the sum of whoever adds the branch."""
+        takes = getattr(self.rt.ops, "experts_stream_shared_takes", None)
+        if (self.shared and not self.gated and takes is not None
+                and takes(rows, self.top, self.w_up, self.w_down, self.w_shared_up, self.w_shared_down)):
+            return self.top + 1
+        return self.branch_parts
+
     def forward(self, ctx, h, residual, branch=None):
-        """`branch`: float32 [rows * branch_parts, width], row r's picks at r * top .. or its finished sum at r; None: the sum
-        goes into `residual`."""
+        """`branch`: float32 [rows * branch_parts, width], row r's picks at r * top .. or its finished sum at r, or
+        [rows * branch_parts_for(rows), width]; None: the sum goes into `residual`."""
+        rows = h.shape[0]
+        if branch is not None and self.shared and branch.shape[0] == rows * (self.top + 1):
+            ids, weights = self._route(h)
+            if self.rt.ops.experts_stream_shared(h, ids, weights, self.w_up, self.w_down, self.w_shared_up, self.w_shared_down, branch):
+                return
+            whole = self.rt.empty((rows, self.hidden), torch.float32)      # the plain kernels were asked for
+            self._forward(ctx, h, None, whole, ids, weights)
+            branch.zero_().view(rows, self.top + 1, self.hidden)[:, 0].copy_(whole)
+            return
+        self._forward(ctx, h, residual, branch, *self._route(h))
+
+    def _route(self, h):
+        """The experts that each row picks and their weights."""
         rt, ops = self.rt, self.rt.ops
         rows = h.shape[0]
         ids = rt.empty((rows, self.top), torch.int32)
@@ -119,6 +142,11 @@ class RoutedExperts(FeedForward):
         else:
             ops.route_topk(h, self.w_router, self.top, ids, weights, score=self.score, renormalize=self.renormalize,
                            route_scale=self.route_scale)
+        return ids, weights
+
+    def _forward(self, ctx, h, residual, branch, ids, weights):
+        rt, ops = self.rt, self.rt.ops
+        rows = h.shape[0]
         on_output, stored = None, branch is not None
         if self.weight_on == "output" and branch is not None and not self.shared:
             raise ValueError("experts whose weights lie on their outputs add to the stream themselves: no stored branch")
