@@ -266,6 +266,10 @@ int fllm_logprobs_processed(const float *logits, int rows, int vocab, const int3
 int fllm_sample(const float *logits, float *work, const struct FllmSampleRow *params, int32_t *out, int rows, int vocab,
                 int kinds, hipStream_t stream);
 
+// Zeroes slots `slots` (host memory, `count` of them) of `tensors` tensors: table (device memory) holds an address and the bytes of a
+// slot for each, `largest` is the largest of those sizes.
+int fllm_clear_slots(const uint64_t *table, int tensors, size_t largest, const int32_t *slots, int count, hipStream_t stream);
+
 // ---- parts of other layer designs -------------------------------------------------------------------------------
 // Two RMSNorms of the same float32 rows in one pass: out1 = x * rsqrt(mean(x^2) + eps1) * w1, out2 likewise with w2
 // and eps2 (w2 and out2 null: one norm).  For blocks whose branches read the same residual stream.

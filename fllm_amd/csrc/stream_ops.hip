@@ -215,6 +215,31 @@ postnorm_add_vec_kernel(float *__restrict__ x, const float *__restrict__ branch,
     }
 }
 
+// A request's first step finds the state of its slot at zero in every tensor that keeps one: all tensors and all such requests of a step
+// in one launch (12 requests of a model with 14 tensors were 168 fills of 2 us and their launches:
+// prompts and answers of those 13.11 -> 12.76 ms).  table[i]: where tensor i begins and
+// the bytes of a slot of it.
+constexpr int kSlotsALaunch = 60;      // by value in the kernel's arguments
+constexpr int kClearBytes = 32 * 1024; // of a slot a workgroup
+
+struct ClearTable {
+    const unsigned long long *table;
+    int slots[kSlotsALaunch];
+};
+
+__global__ void __launch_bounds__(256) clear_slots_kernel(const ClearTable p) {
+    const unsigned long long bytes = p.table[2 * blockIdx.y + 1];
+    const unsigned long long from = (unsigned long long)blockIdx.x * kClearBytes;
+    if (from >= bytes) return;
+    unsigned char *at = (unsigned char *)p.table[2 * blockIdx.y] + (unsigned long long)p.slots[blockIdx.z] * bytes + from;
+    const int n = (int)(bytes - from < kClearBytes ? bytes - from : kClearBytes);
+    const int head = min(n, (int)((16 - ((uintptr_t)at & 15)) & 15)), whole = (n - head) / 16;
+    if ((int)threadIdx.x < head) at[threadIdx.x] = 0;
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    for (int i = threadIdx.x; i < whole; i += 256) *(f32x4_t *)(at + head + 16 * i) = zero;
+    for (int i = head + 16 * whole + threadIdx.x; i < n; i += 256) at[i] = 0;
+}
+
 }  // namespace
 
 extern "C" int fllm_postnorm_add(float *x, const void *branch, int branch_dtype, int parts, const float *part_weights, const float *gain,
@@ -320,4 +345,27 @@ extern "C" int fllm_stream_add(float *x, const int32_t *ids, const void *table, 
     else
         FLLM_REQUIRE(false, "stream_add: unknown dtype %d", table_dtype);
     return fllm_check_launch("stream_add");
+}
+
+// Zeroes slots `slots` (host memory, `count` of them) of `tensors` tensors: table (device memory) holds an address and the bytes of a
+// slot for each, `largest` is the largest of those sizes.
+extern "C" int fllm_clear_slots(const uint64_t *table, int tensors, size_t largest, const int32_t *slots, int count, hipStream_t stream) {
+    FLLM_REQUIRE(tensors >= 0 && tensors <= 65535 && count >= 0, "clear_slots: bad sizes");
+    if (tensors == 0 || count == 0 || largest == 0) return 0;
+    FLLM_REQUIRE(table != nullptr && slots != nullptr, "clear_slots: operands missing");
+    const size_t blocks = (largest + kClearBytes - 1) / kClearBytes;
+    FLLM_REQUIRE(blocks <= 0x7fffffff, "clear_slots: slots of %zu bytes are too large", largest);
+    for (int at = 0; at < count; at += kSlotsALaunch) {
+        const int n = count - at < kSlotsALaunch ? count - at : kSlotsALaunch;
+        ClearTable p = {};
+        p.table = (const unsigned long long *)table;
+        for (int i = 0; i < n; i++) {
+            FLLM_REQUIRE(slots[at + i] >= 0, "clear_slots: slot %d", slots[at + i]);
+            p.slots[i] = slots[at + i];
+        }
+        hipLaunchKernelGGL(clear_slots_kernel, dim3((unsigned)blocks, tensors, n), dim3(256), 0, stream, p);
+        const int rc = fllm_check_launch("clear_slots");
+        if (rc != 0) return rc;
+    }
+    return 0;
 }

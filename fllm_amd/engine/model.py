@@ -61,6 +61,7 @@ class Model:
         """Groups cache-owning run entries by what they need; entries that read another entry's
         cache join that entry's group."""
         self.kv_needs: List[Optional[KVNeed]] = []
+        self._slot_table = None                      # where the state tensors lie, for `clear_state`
         self.state_needs: List[object] = []          # per run entry None, a StateNeed, or a dict of named ones
         self.portion_multiple = 1                    # a prompt is cut on multiples of every mixer's own multiple
         for entry in self.spec.run_order:
@@ -150,6 +151,9 @@ class Model:
                                               page_size=page_size, writes=entry.reads_cache_of is None, state=state,
                                               pool_k=None if pools is None else pools[0][idx],
                                               pool_v=None if pools is None else pools[1][idx]))
+        arenas = [arena for _, _, arena in self.state_arenas()]
+        table = getattr(rt.ops, "slot_table", None)
+        self._slot_table = table(arenas) if table is not None and arenas else None      # of tensors that `bindings` hold
         return CacheManager(groups, list(pages_per_group), max_requests, max_step_tokens=max_step_tokens)
 
     def state_arenas(self):
@@ -161,10 +165,19 @@ class Model:
             elif binding.state is not None:
                 yield index, None, binding.state
 
-    def clear_state(self, slot: int) -> None:
-        """Zeros the fixed-size state of every run entry in one request slot (a request's first step)."""
+    def clear_state(self, *slots: int) -> None:
+        """Zeros the fixed-size state of every run entry in the given request slots (requests' first steps)."""
+        if not slots:
+            return
+        if self._slot_table is not None:
+            most = min(arena.shape[0] for _, _, arena in self.state_arenas())
+            if any(not 0 <= s < most for s in slots):
+                raise IndexError(f"slots {slots} of {most}")
+            self.rt.ops.clear_slots(self._slot_table, slots)
+            return
         for _, _, arena in self.state_arenas():
-            arena[slot].zero_()
+            for slot in slots:
+                arena[slot].zero_()
 
     def snapshot_state(self, slot: int):
         """A copy of everything the model keeps in one request slot, for `restore_state`

@@ -255,9 +255,8 @@ class ModelRunner:
                 self.cache.free_request(r)
             raise
         if self.model.has_state:
-            for e in entries:                # a request's first step finds its state slot cleared
-                if self.cache.length(e.req_id) == 0:
-                    self.model.clear_state(self.cache.slot(e.req_id))
+            # a request's first step finds its state slot cleared
+            self.model.clear_state(*(self.cache.slot(e.req_id) for e in entries if self.cache.length(e.req_id) == 0))
         logits = None
         checking = self.model.layer_check is not None and self.model.layer_check.active     # checked steps run eagerly
         if not checking and self.use_graphs and all(len(e.tokens) == 1 for e in entries) and len(entries) <= GRAPH_BUCKETS[-1]:

@@ -51,7 +51,7 @@ assert SAMPLE_ROW_BYTES == 32
 _lib = None
 
 
-ABI_VERSION = 23
+ABI_VERSION = 24
 
 
 def load_library(build_if_missing: bool = True):
@@ -187,6 +187,7 @@ def load_library(build_if_missing: bool = True):
                                c_void],
         "fllm_gate_up_tiles": [c_void, c_int, c_void, c_void, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_void],
         "fllm_linear_tiles": [c_void, c_int, c_void, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_int, c_void],
+        "fllm_clear_slots": [c_void, c_int, ctypes.c_size_t, c_void, c_int, c_void],
         "fllm_experts_stream_shared": [c_void, c_int, c_void, c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_void, c_void,
                                        c_int, c_void, c_void, c_void],
         "fllm_experts_stream": [c_void, c_int, c_void, c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_void,
@@ -908,6 +909,23 @@ class Ops:
         self._check(self.lib.fllm_glu_clamped(_ptr(gate_up), _ptr(out), rows, two_i // 2, float(limit), float(alpha),
                                               float(up_offset), _DTYPE_CODE[gate_up.dtype], self._stream()))
         return out
+
+    @staticmethod
+    def slot_table(tensors: Sequence[torch.Tensor]) -> Tuple[torch.Tensor, int]:
+        """What `clear_slots` reads of tensors [slots, ...]: on the device an address and the bytes of a slot for each, and the
+        largest of those sizes.  It is good as long as the tensors are."""
+        for i, t in enumerate(tensors):
+            _dense(t, f"tensor {i}")
+        sizes = [t[0].numel() * t.element_size() for t in tensors]
+        rows = [[t.data_ptr(), n] for t, n in zip(tensors, sizes)]
+        return torch.tensor(rows, dtype=torch.int64).reshape(-1, 2).to(tensors[0].device), max(sizes)
+
+    def clear_slots(self, table: Tuple[torch.Tensor, int], slots: Sequence[int]) -> None:
+        """Zeroes the given slots of every tensor of a `slot_table`."""
+        addresses, largest = table
+        _dense(addresses, "table", torch.int64)
+        numbers = (ctypes.c_int32 * len(slots))(*slots)
+        self._check(self.lib.fllm_clear_slots(_ptr(addresses), addresses.shape[0], int(largest), numbers, len(slots), self._stream()))
 
     def scale_(self, x: torch.Tensor, scale: float) -> torch.Tensor:
         """x *= scale, float32, in place."""
