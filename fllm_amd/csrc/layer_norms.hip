@@ -192,13 +192,20 @@ gelu_side_kernel(const T *__restrict__ z, const int32_t *__restrict__ ids, const
     }
 }
 
-// One workgroup an output lane d: z = W[d] . x for the R rows of the step (x rounded to T first, as cast_rows gives it), then
-// gelu_side of it.  dims that are multiples of 8 lie side by side in 16-byte loads.
+// One workgroup an output lane d and R rows: z = W[d] . x (x rounded to T first, as cast_rows gives it), then gelu_side of it.
+// widths that are multiples of 8 lie side by side in 16-byte loads.  What bounds it is its launch: up to 32 rows (eight a workgroup)
+// it replaces a cast, a product and a gate of 14 us together, each of them launch too; prompts and answers of 12 such
+// requests 12.70 -> 12.46 ms.
 template <typename T, int R>
 __global__ void __launch_bounds__(kBlock)
 side_gate_kernel(const float *__restrict__ x, const T *__restrict__ w, const int32_t *__restrict__ ids, const T *__restrict__ table, int vocab,
                  int table_width, int offset, T *__restrict__ out, int rows, int width, int dim) {
     __shared__ float part[kWaves][R];
+    const int r0 = blockIdx.y * R;      // R rows a workgroup
+    x += (size_t)r0 * width;
+    ids += r0;
+    out += (size_t)r0 * dim;
+    rows = rows - r0 < R ? rows - r0 : R;
     const int d = blockIdx.x, lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const T *wr = w + (size_t)d * width;
     float acc[R];
@@ -291,15 +298,15 @@ extern "C" int fllm_layernorm_conv(const float *x, const float *w1, float eps1, 
     return fllm_check_launch("layernorm_conv");
 }
 
-// 0: launched; negative: error; 1: declined (more than 8 rows, a width that is no multiple of 8)
+// 0: launched; negative: error; 1: declined (more than 32 rows, a width that is no multiple of 8)
 extern "C" int fllm_side_gate(const float *x, const void *w, const int32_t *ids, const void *table, int vocab, int table_width, int offset, void *out,
                               int rows, int width, int dim, int dtype, hipStream_t stream) {
     FLLM_REQUIRE(rows >= 0 && width > 0 && dim > 0 && vocab > 0 && offset >= 0 && offset + dim <= table_width, "side_gate: bad sizes");
     FLLM_REQUIRE(x && w && ids && table && out, "side_gate: operands missing");
     if (rows == 0) return 0;
-    if (rows > 8 || width % 8 != 0 || (((uintptr_t)x | (uintptr_t)w) & 15) != 0) return 1;
+    if (rows > 32 || width % 8 != 0 || (((uintptr_t)x | (uintptr_t)w) & 15) != 0) return 1;
 #define FLLM_SIDE(T, R)                                                                                                                      \
-    hipLaunchKernelGGL((side_gate_kernel<T, R>), dim3(dim), dim3(kBlock), 0, stream, x, (const T *)w, ids, (const T *)table, vocab, table_width, \
+    hipLaunchKernelGGL((side_gate_kernel<T, R>), dim3(dim, (rows + R - 1) / R), dim3(kBlock), 0, stream, x, (const T *)w, ids, (const T *)table, vocab, table_width, \
                        offset, (T *)out, rows, width, dim)
 #define FLLM_SIDE_R(T)                            \
     do {                                          \

@@ -1761,6 +1761,10 @@ class Ops:
     def side_gate(self, x: torch.Tensor, w: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, offset: int, out: torch.Tensor) -> bool:
         """`gelu_side` of z = W x in one kernel, x the float32 rows of a stream.  False: not taken (more than 8 rows, a width that is no
         multiple of 8), nothing was written."""
+        return x.shape[0] <= 8 and self.side_gate_rows(x, w, ids, table, offset, out)
+
+    def side_gate_rows(self, x: torch.Tensor, w: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, offset: int, out: torch.Tensor) -> bool:
+        """`side_gate` for up to 32 rows, eight a workgroup."""
         rows, width = x.shape
         dim = w.shape[0]
         _dense(x, "x", torch.float32)

@@ -39,7 +39,8 @@ class TokenSide(Part):
         rt, ops = self.rt, self.rt.ops
         rows = x.shape[0]
         g = rt.empty((rows, self.dim))
-        gate = getattr(ops, "side_gate", None)          # steps of few rows: one kernel up to the gated numbers
+        # steps of few rows: one kernel up to the gated numbers
+        gate = getattr(ops, "side_gate" if rows <= 8 else "side_gate_rows", None)
         if gate is None or not gate(x, self.w_gate, ctx.ids, self.table, self.offset, g):
             h = rt.empty((rows, self.size))
             ops.cast_rows(x, h)

@@ -1,4 +1,5 @@
-"""What a request's first step does beside a model's layers: slots of state tensors cleared in one launch."""
+"""What a request's first steps do beside a model's layers: slots of state tensors cleared in one launch; the gate of a token's side input
+for the rows of a busy step."""
 import pytest
 import torch
 
@@ -28,3 +29,21 @@ def test_cleared_slots_and_no_others(ops):
             want = torch.ones_like(t)
             want[slots] = 0
             assert torch.equal(t, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows", [1, 8, 9, 16, 17, 32])
+def test_side_gate_of_more_rows(ops, rows, dtype):
+    """Eight rows a workgroup: a row's numbers are those of its own call, whichever rows it comes with."""
+    g = torch.Generator().manual_seed(rows)
+    width, dim = 520, 24
+    x, w = (torch.randn(rows, width, generator=g) * 3).to(DEV), (torch.randn(dim, width, generator=g) * width ** -0.5).to(dtype).to(DEV)
+    table, ids = torch.randn(31, 3 * dim, generator=g).to(dtype).to(DEV), torch.randint(0, 31, (rows,), generator=g, dtype=torch.int32).to(DEV)
+    got = torch.full((rows, dim), float("nan"), dtype=dtype, device=DEV)
+    assert ops.side_gate_rows(x, w, ids, table, dim, got)
+    alone = torch.empty_like(got)
+    for r in range(rows):
+        assert ops.side_gate(x[r:r + 1], w, ids[r:r + 1], table, dim, alone[r:r + 1])
+    assert torch.equal(got, alone)
+    assert not ops.side_gate_rows(torch.zeros(33, width, device=DEV), w, torch.zeros(33, dtype=torch.int32, device=DEV), table, 0,
+                                  torch.empty(33, dim, dtype=dtype, device=DEV))
