@@ -40,7 +40,8 @@ struct TileParams {
     const float *r1, *r2, *pb;
     int by_heads;                             // 1: a tile is the heads of one key/value head of one row
     int splits;                               // workgroups that share a tile's keys (blockIdx.z); more than one: partial results
-    float *parts;                             // [tile][split][16 * DV sums, 16 maxima, 16 denominators] for the merge kernel
+    float *parts;                             // [tile][split][16 * DV sums, 16 maxima, 16 denominators] in the device workspace
+    int *counters;                            // a tile's finished workgroups, zero between launches
 };
 
 // The hardware's exponential, logarithm and reciprocal (a unit or two in the last place of a float32): these kernels serve the
@@ -56,6 +57,10 @@ __device__ __forceinline__ void split_bf16(const float (&x)[8], bf16x8_t &hi, bf
         lo[e] = (bf16_t)(x[e] - (float)hi[e]);
     }
 }
+
+constexpr int kMostSplits = 32;
+
+__device__ __forceinline__ void publish(float *at, float v) { __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // VARIANT 0: window + pooled blocks, softmax.  VARIANT 1: every key up to the row, sigmoid weights.
 template <int KD, int VT, int VARIANT>
@@ -306,8 +311,8 @@ mixer_tile_kernel(const TileParams p) {
                 acc += sm_o[w][q][d] * f;
             }
             if (part != nullptr) {      // this workgroup's share of the keys: the sums as they are, against its own maximum
-                part[q * DV + d] = acc;
-                if (d == 0) part[16 * DV + q] = m, part[16 * DV + 16 + q] = l;
+                publish(part + q * DV + d, acc);
+                if (d == 0) publish(part + 16 * DV + q, m), publish(part + 16 * DV + 16 + q, l);
                 continue;
             }
             acc = l > 0.f ? acc / l : 0.f;
@@ -315,41 +320,82 @@ mixer_tile_kernel(const TileParams p) {
 #pragma unroll
             for (int w = 0; w < kWavesM; w++) acc += sm_o[w][q][d];
             if (part != nullptr) {
-                part[q * DV + d] = acc;
+                publish(part + q * DV + d, acc);
                 continue;
             }
         }
         const int row = p.by_heads ? row0 : row0 + q, head = p.by_heads ? head0 + q : head0;
         p.out[((size_t)row * p.heads + head) * DV + d] = (bf16_t)acc;
     }
-}
-
-// The shares of a tile's keys put together in the order of the shares: grid (rows, kv_heads), tiles by heads.
-template <int VARIANT>
-__global__ void __launch_bounds__(kThreads)
-mixer_merge_kernel(const float *__restrict__ parts, int splits, const int32_t *__restrict__ row_seg, bf16_t *__restrict__ out, int heads,
-                   int kv_heads, int DV) {
-    const int row = blockIdx.x, kvh = blockIdx.y, G = heads / kv_heads;
-    if (row_seg[row] < 0) return;
-    const int stride = 16 * DV + 32;
-    const float *mine = parts + (size_t)(blockIdx.y * gridDim.x + blockIdx.x) * splits * stride;
-    for (int idx = threadIdx.x; idx < G * DV; idx += kThreads) {
-        const int q = idx / DV, d = idx - q * DV;
-        float acc = 0.f;
-        if (VARIANT == 0) {
-            float m = -INFINITY, l = 0.f;
-            for (int s = 0; s < splits; s++) m = fmaxf(m, mine[(size_t)s * stride + 16 * DV + q]);
-            for (int s = 0; s < splits; s++) {
-                const float ms = mine[(size_t)s * stride + 16 * DV + q];
-                const float f = ms == -INFINITY ? 0.f : expf(ms - m);
-                l += mine[(size_t)s * stride + 16 * DV + 16 + q] * f;
-                acc += mine[(size_t)s * stride + q * DV + d] * f;
-            }
-            acc = l > 0.f ? acc / l : 0.f;
-        } else {
-            for (int s = 0; s < splits; s++) acc += mine[(size_t)s * stride + q * DV + d];
+    if (part == nullptr) return;
+    // ---- the shares meet (tiles by heads): the workgroup that counts last puts them together in the order of the shares, all of
+    // its loads asked for before it waits.  A kernel of its own for this took 8.4 us (softmax) and 6.0 (sigmoid) at 2 rows and 6 shares
+    // (prompts and answers of 2 requests, 72 such launches: 14.46 -> 14.10 ms).
+    __shared__ int s_seen;
+    __shared__ float s_factor[kMostSplits][16], s_sum[kMostSplits][16];
+    const int tile = blockIdx.y * gridDim.x + blockIdx.x, splits = p.splits;
+    parts_published();
+    __syncthreads();
+    if (threadIdx.x == 0) s_seen = __hip_atomic_fetch_add(p.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (s_seen != splits - 1) return;
+    parts_visible();
+    if (threadIdx.x == 0) __hip_atomic_store(p.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // for the next launch
+    constexpr int kStride = 16 * DV + 32, NI = 4, NS = 8;
+    const float *all = p.parts + (size_t)tile * splits * kStride;
+    auto fetch = [](const float *at) __attribute__((always_inline)) { return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    if (VARIANT == 0) {
+        for (int i = threadIdx.x; i < splits * 16; i += kThreads) {
+            const int q = i & 15;
+            if (q < count) s_factor[i >> 4][q] = fetch(all + (size_t)(i >> 4) * kStride + 16 * DV + q), s_sum[i >> 4][q] = fetch(all + (size_t)(i >> 4) * kStride + 16 * DV + 16 + q);
         }
-        out[((size_t)row * heads + kvh * G + q) * DV + d] = (bf16_t)acc;
+    }
+    for (int base = 0; base < count * DV; base += NI * kThreads) {      // every thread the same trips
+        const int idx0 = base + threadIdx.x;
+        float acc[NI], m[NI], l[NI];
+#pragma unroll
+        for (int i = 0; i < NI; i++) acc[i] = l[i] = 0.f, m[i] = -INFINITY;
+        for (int s0 = 0; s0 < splits; s0 += NS) {
+            float v[NI][NS];
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+#pragma unroll
+                for (int s = 0; s < NS; s++) {
+                    const int idx = min(idx0 + i * kThreads, count * DV - 1), at = min(s0 + s, splits - 1);
+                    v[i][s] = fetch(all + (size_t)at * kStride + idx);      // idx = q * DV + d
+                }
+            if (VARIANT == 0 && s0 == 0) {
+                if (base == 0) __syncthreads();                             // the maxima and sums are in LDS
+#pragma unroll
+                for (int i = 0; i < NI; i++) {
+                    const int q = min(idx0 + i * kThreads, count * DV - 1) / DV;
+                    for (int s = 0; s < splits; s++) m[i] = fmaxf(m[i], s_factor[s][q]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const int q = min(idx0 + i * kThreads, count * DV - 1) / DV;
+#pragma unroll
+                for (int s = 0; s < NS; s++) {
+                    if (s0 + s >= splits) break;
+                    if (VARIANT == 0) {
+                        const float ms = s_factor[s0 + s][q], f = ms == -INFINITY ? 0.f : expf(ms - m[i]);
+                        l[i] += s_sum[s0 + s][q] * f;
+                        acc[i] += v[i][s] * f;
+                    } else {
+                        acc[i] += v[i][s];
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int idx = idx0 + i * kThreads;
+            if (idx >= count * DV) break;
+            const int q = idx / DV, d = idx - q * DV;
+            if (VARIANT == 0) acc[i] = l[i] > 0.f ? acc[i] / l[i] : 0.f;
+            p.out[((size_t)row0 * p.heads + head0 + q) * DV + d] = (bf16_t)acc[i];
+        }
     }
 }
 
@@ -375,19 +421,20 @@ int launch_tiles(TileParams &p, int head_dim, int v_dim, int keys_bound, hipStre
     dim3 grid = p.by_heads ? dim3(p.rows, p.kv_heads) : dim3((p.rows + 15) / 16 + p.num_segs, p.heads);
     if (grid.y > 65535) return 1;
     // Steps of single rows have a tile a row and key/value head: with few of them, several workgroups share a tile's keys
-    // (at least 256 keys each, two workgroups a compute unit at most) and a second kernel puts their shares together.
+    // (at least 256 keys each, two workgroups a compute unit at most), and whichever is last puts their shares together.
     p.splits = 1;
     p.parts = nullptr;
     if (p.by_heads) {
         const long tiles = (long)p.rows * p.kv_heads;
-        long splits = std::min<long>(std::min<long>(512 / std::max<long>(tiles, 1), (keys_bound + 255) / 256), 32);
+        long splits = std::min<long>(std::min<long>(512 / std::max<long>(tiles, 1), (keys_bound + 255) / 256), kMostSplits);
         void *base = nullptr;
         size_t bytes = 0;
         if (splits > 1 && fllm_device_workspace(&base, &bytes) && bytes > kWorkspaceCounterBytes) {
             const size_t room = (bytes - kWorkspaceCounterBytes) / sizeof(float), each = (size_t)tiles * (16 * v_dim + 32);
             splits = std::min<long>(splits, (long)(room / each));
-            if (splits > 1) {
+            if (splits > 1) {      // and so there are fewer tiles than 256: a counter each
                 p.splits = (int)splits;
+                p.counters = (int *)base;
                 p.parts = (float *)((char *)base + kWorkspaceCounterBytes);
                 grid.z = (unsigned)splits;
             }
@@ -400,9 +447,6 @@ int launch_tiles(TileParams &p, int head_dim, int v_dim, int keys_bound, hipStre
     case 3: declined = launch_vt<VARIANT, 3>(p, v_dim / 16, grid, stream); break;
     case 4: declined = launch_vt<VARIANT, 4>(p, v_dim / 16, grid, stream); break;
     }
-    if (!declined && p.splits > 1)
-        hipLaunchKernelGGL(mixer_merge_kernel<VARIANT>, dim3(p.rows, p.kv_heads), dim3(kThreads), 0, stream, p.parts, p.splits, p.row_seg, p.out,
-                           p.heads, p.kv_heads, v_dim);
     return declined;
 }
 
