@@ -445,6 +445,12 @@ int fllm_relu_squared(const void *x, void *out, size_t total, int dtype, hipStre
 // Router with corrections and groups, and the up product of experts without a gate (routed_experts.hip).
 int fllm_route_grouped(const void *h, int ldh, const void *w_router, const float *correction, int rows, int K, int E, int top, int groups,
                        int kept, int32_t *ids, float *weights, float route_scale, int dtype, hipStream_t stream);
+// A row's way into routed experts in one kernel, for steps of up to 64 bfloat16 rows: with `branch` (float32 [rows, width]) first x[r] += branch *
+// rsqrt(mean branch^2 + eps) * gain (normalize 0: without that norm), then out = the RMSNorm of x[r] and the router of out's rows: with
+// `correction` as fllm_route_grouped, without as fllm_route_topk.  1: declined (see there), nothing was written.
+int fllm_norm_route(float *x, const float *branch, const float *gain, float eps, int normalize, const float *norm_w, float norm_eps, void *out,
+                    int rows, int width, const void *w_router, const float *correction, int experts, int top, int groups, int kept, int score_mode,
+                    int renormalize, float route_scale, int32_t *ids, float *weights, hipStream_t stream);
 int fllm_experts_up(const void *h, int ldh, const int32_t *ids, int rows, int top, const void *w_up, int E, int inter, int K, void *act,
                     int dtype, hipStream_t stream);
 // Experts without a gate on the matrix cores: pairs grouped by expert, act = relu(W_up[e] h)^2, out = W_down[e] act (float32

@@ -1,0 +1,156 @@
+// A decode step's row on its way into routed experts in one kernel: a branch behind a norm joins the stream (or none does), the norm before
+// the experts, and the router: what postnorm_add (stream_ops.hip) and the routers (routed_experts.hip) do one after the other.
+//
+// One workgroup a row.  What bounds it is its launch and two trips to memory, where the two kernels paid both twice (4.2 and 5.5 us at
+// 2 rows of 1,536 lanes; prompts and answers of models with 12, 6 and 4 such layers a step 14.10 -> 13.87, 11.57 -> 11.42, 8.44 -> 8.31 ms): the row, its branch, the vectors and the first rows of the router are asked for together, the normed row
+// stays in LDS for the router's products, whose sums are added in the order row_score adds them.
+#include "api.h"
+#include "common.h"
+#include "router_picks.h"
+
+namespace {
+
+constexpr int kBlock = 256;
+constexpr int kWaves = kBlock / kWave;
+constexpr int kMostExperts = 64;
+constexpr int kStep = kWave * 8;      // lanes of a row that a wave takes at a time: widths are multiples of it
+
+struct RouteArgs {
+    const bf16_t *w;                  // [experts][width]
+    const float *correction;          // GROUPED: [experts]
+    int experts, top, groups, kept, score_mode, renormalize;
+    float scale;
+    int32_t *ids;
+    float *weights;
+};
+
+// NV pieces of four lanes a thread (width <= NV * 4 * kBlock); BRANCH: x[r] += branch * rsqrt(mean branch^2 + eps) * gain first
+// (`normalize` 0: without the norm); GROUPED: the router with corrections and groups.
+template <int NV, bool BRANCH, bool GROUPED>
+__global__ void __launch_bounds__(kBlock)
+norm_route_kernel(float *__restrict__ x, const float *__restrict__ branch, const float *__restrict__ gain, float eps, int normalize,
+                  const float *__restrict__ norm_w, float norm_eps, bf16_t *__restrict__ out, int width, const RouteArgs p) {
+    constexpr int AHEAD = NV * 4 * kBlock / kStep;      // pieces of a router's row
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    __shared__ float scratch[kWaves];
+    __shared__ float score[kMostExperts], choice[kMostExperts], gsum[kMostExperts], picks[kMostExperts];
+    bf16_t *row = (bf16_t *)smem;                       // [width]
+    const size_t r = blockIdx.x;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int pieces = width / kStep;
+    f32x4_t v[NV], s[NV], w[NV], w2[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int c = min((i * kBlock + (int)threadIdx.x) * 4, width - 4);
+        if (BRANCH) {
+            v[i] = *(const f32x4_t *)(branch + r * width + c);
+            w[i] = *(const f32x4_t *)(gain + c);
+        }
+        s[i] = *(const f32x4_t *)(x + r * width + c);
+        w2[i] = *(const f32x4_t *)(norm_w + c);
+    }
+    bf16x8_t b[AHEAD];                                  // this wave's first expert's row of the router
+    const int first = min(wave, p.experts - 1);
+#pragma unroll
+    for (int j = 0; j < AHEAD; j++) b[j] = *(const bf16x8_t *)(p.w + (size_t)first * width + min(j, pieces - 1) * kStep + lane * 8);
+    auto mine = [&](int i) { return (i * kBlock + (int)threadIdx.x) * 4 < width; };
+    if (BRANCH) {
+        float inv = 1.0f;
+        if (normalize) {
+            float ss = 0.f;
+#pragma unroll
+            for (int i = 0; i < NV; i++)
+                if (mine(i))
+#pragma unroll
+                    for (int e = 0; e < 4; e++) ss = fmaf(v[i][e], v[i][e], ss);
+            inv = 1.0f / sqrtf(block_sum<kWaves>(ss, scratch) / (float)width + eps);
+        }
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            if (!mine(i)) break;
+#pragma unroll
+            for (int e = 0; e < 4; e++) s[i][e] += v[i][e] * inv * w[i][e];
+            *(f32x4_t *)(x + r * width + (i * kBlock + threadIdx.x) * 4) = s[i];
+        }
+    }
+    float ss2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+        if (mine(i))
+#pragma unroll
+            for (int e = 0; e < 4; e++) ss2 = fmaf(s[i][e], s[i][e], ss2);
+    const float inv2 = 1.0f / sqrtf(block_sum<kWaves>(ss2, scratch) / (float)width + norm_eps);
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int c = (i * kBlock + threadIdx.x) * 4;
+        if (!mine(i)) break;
+        bf16x4_t h;
+#pragma unroll
+        for (int e = 0; e < 4; e++) h[e] = (bf16_t)(s[i][e] * inv2 * w2[i][e]);
+        *(bf16x4_t *)(out + r * width + c) = h;
+        *(bf16x4_t *)(row + c) = h;
+    }
+    __syncthreads();
+    for (int e = wave; e < p.experts; e += kWaves) {
+        const float c = GROUPED ? p.correction[e] : 0.f;
+        if (e != wave) {
+#pragma unroll
+            for (int j = 0; j < AHEAD; j++) b[j] = *(const bf16x8_t *)(p.w + (size_t)e * width + min(j, pieces - 1) * kStep + lane * 8);
+        }
+        float z = 0.f;
+#pragma unroll
+        for (int j = 0; j < AHEAD; j++) {
+            if (j >= pieces) break;
+            const bf16x8_t a = *(const bf16x8_t *)(row + j * kStep + lane * 8);
+#pragma unroll
+            for (int k = 0; k < 8; k++) z = fmaf((float)a[k], (float)b[j][k], z);
+        }
+        z = wave_sum(z);
+        if (lane == 0) {
+            const float sigmoid = 1.0f / (1.0f + expf(-z));
+            score[e] = GROUPED || p.score_mode == 0 ? sigmoid : z;
+            if (GROUPED) choice[e] = sigmoid + c;
+        }
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    if (GROUPED) pick_grouped(score, choice, gsum, picks, p.experts, p.top, p.groups, p.kept, p.ids + r * p.top, p.weights + r * p.top, p.scale, lane);
+    else pick_plain(score, picks, p.experts, p.top, p.ids + r * p.top, p.weights + r * p.top, p.score_mode, p.renormalize, p.scale, lane);
+}
+
+template <bool BRANCH, bool GROUPED>
+void launch(float *x, const float *branch, const float *gain, float eps, int normalize, const float *norm_w, float norm_eps, void *out, int rows,
+            int width, const RouteArgs &p, hipStream_t stream) {
+    const size_t smem = (size_t)width * sizeof(bf16_t);
+#define FLLM_NORM_ROUTE(NV)                                                                                                              \
+    hipLaunchKernelGGL((norm_route_kernel<NV, BRANCH, GROUPED>), dim3(rows), dim3(kBlock), smem, stream, x, branch, gain, eps, normalize, norm_w, \
+                       norm_eps, (bf16_t *)out, width, p)
+    if (width <= 4 * kBlock) FLLM_NORM_ROUTE(1);
+    else if (width <= 8 * kBlock) FLLM_NORM_ROUTE(2);
+    else FLLM_NORM_ROUTE(4);
+#undef FLLM_NORM_ROUTE
+}
+
+}  // namespace
+
+// 0: launched; negative: error; 1: declined (a width that is no multiple of 512 or beyond 4,096, more than 64 experts or rows), nothing was written
+extern "C" int fllm_norm_route(float *x, const float *branch, const float *gain, float eps, int normalize, const float *norm_w, float norm_eps,
+                               void *out, int rows, int width, const void *w_router, const float *correction, int experts, int top, int groups,
+                               int kept, int score_mode, int renormalize, float route_scale, int32_t *ids, float *weights, hipStream_t stream) {
+    FLLM_REQUIRE(rows >= 0 && width > 0 && experts > 0 && top > 0 && top <= experts && norm_eps > 0.f, "norm_route: bad sizes");
+    FLLM_REQUIRE(x && norm_w && out && w_router && ids && weights && ((branch == nullptr) == (gain == nullptr)), "norm_route: operands missing");
+    FLLM_REQUIRE(branch == nullptr || !normalize || eps > 0.f, "norm_route: a norm needs an eps");
+    FLLM_REQUIRE(score_mode == 0 || score_mode == 1, "norm_route: unknown score %d", score_mode);
+    if (correction != nullptr)
+        FLLM_REQUIRE(groups > 0 && experts % groups == 0 && kept > 0 && kept <= groups && top <= kept * (experts / groups),
+                     "norm_route: %d experts in %d groups, %d kept, %d picked", experts, groups, kept, top);
+    if (rows == 0) return 0;
+    if (width % kStep != 0 || width > 16 * kBlock || experts > kMostExperts || rows > 64) return 1;
+    if (((uintptr_t)x | (uintptr_t)branch | (uintptr_t)gain | (uintptr_t)norm_w | (uintptr_t)out | (uintptr_t)w_router) & 15) return 1;
+    const RouteArgs p = {(const bf16_t *)w_router, correction, experts, top, groups, kept, score_mode, renormalize, route_scale, ids, weights};
+    if (branch != nullptr && correction != nullptr) launch<true, true>(x, branch, gain, eps, normalize, norm_w, norm_eps, out, rows, width, p, stream);
+    else if (branch != nullptr) launch<true, false>(x, branch, gain, eps, normalize, norm_w, norm_eps, out, rows, width, p, stream);
+    else if (correction != nullptr) launch<false, true>(x, branch, gain, eps, normalize, norm_w, norm_eps, out, rows, width, p, stream);
+    else launch<false, false>(x, branch, gain, eps, normalize, norm_w, norm_eps, out, rows, width, p, stream);
+    return fllm_check_launch("norm_route");
+}

@@ -4,6 +4,7 @@
 // row alone, never on the rest of the batch.
 #include "api.h"
 #include "common.h"
+#include "router_picks.h"
 
 namespace {
 
@@ -78,20 +79,6 @@ __device__ __forceinline__ float row_score(const bf16_t *__restrict__ h, const b
     return wave_sum(acc);
 }
 
-// shuffles that meet among `lanes` (a power of two) neighbouring lanes: the largest value, the lower index among equals
-__device__ __forceinline__ void best_of_lanes(float &best, int &at, int lanes) {
-    for (int o = lanes >> 1; o > 0; o >>= 1) {
-        const float other = __shfl_xor(best, o, kWave);
-        const int other_at = __shfl_xor(at, o, kWave);
-        if (other > best || (other == best && other_at < at)) best = other, at = other_at;
-    }
-}
-__device__ __forceinline__ int lanes_for(int n) {      // the lanes that hold something when lane l holds items l, l + 64, ..
-    int lanes = 1;
-    while (lanes < n && lanes < kWave) lanes *= 2;
-    return lanes;
-}
-
 // Router: z = W h in float32, score = sigmoid(z) (score_mode 0) or the softmax of z over all experts (score_mode 1); the
 // `top` largest scores of a row, ties to the lower index; weights[r, k] = the score of pick k, with `renormalize` divided by
 // the sum of the picks' scores (+ 1e-20), times route_scale.  One workgroup a row; scores through LDS.
@@ -125,41 +112,7 @@ route_kernel(const T *__restrict__ h, int ldh, const T *__restrict__ w, int K, i
     }
     __syncthreads();
     if (wave != 0) return;
-    const int lanes = lanes_for(E);
-    if (score_mode == 1) {   // softmax over all experts: the largest logit, the sum in index order a lane, then across lanes
-        float top_z = -INFINITY;
-        for (int e = lane; e < E; e += kWave) top_z = fmaxf(top_z, score[e]);
-        top_z = wave_max(top_z);
-        float sum = 0.f;
-        for (int e = lane; e < E; e += kWave) sum += expf(score[e] - top_z);
-        sum = wave_sum(sum);
-        for (int e = lane; e < E; e += kWave) score[e] = expf(score[e] - top_z) / sum;
-        __builtin_amdgcn_wave_barrier();
-        __threadfence_block();
-    }
-    float picked = 0.f;
-    // one wave picks: every round the largest score not yet taken, the lowest index among equals
-    for (int k = 0; k < top; k++) {
-        float best = -INFINITY;
-        int at = 0x7fffffff;
-        for (int e = lane; e < E; e += kWave) {
-            const float s = score[e];
-            if (s > best) best = s, at = e;      // ascending e: the first of equals stays
-        }
-        best_of_lanes(best, at, lanes);
-        if (at < 0 || at >= E) at = k;           // scores that compare with nothing (NaN rows): still an expert of the stack
-        picked += best;
-        if (lane == 0) {
-            ids[r * top + k] = at;
-            picks[k] = best;
-            score[at] = -INFINITY;               // scores lie in [0, 1]: nothing real is that small
-        }
-        __builtin_amdgcn_wave_barrier();
-        __threadfence_block();
-    }
-    const float factor = renormalize ? route_scale / (picked + 1e-20f) : route_scale;
-    for (int k = lane; k < top; k += kWave)
-        weights[r * top + k] = (renormalize || route_scale != 1.0f) ? picks[k] * factor : picks[k];
+    pick_plain(score, picks, E, top, ids + r * top, weights + r * top, score_mode, renormalize, route_scale, lane);
 }
 
 // Router with corrections and groups: score = sigmoid(W h); the picks are made by choice = score + correction, and only among
@@ -203,66 +156,7 @@ route_grouped_kernel(const T *__restrict__ h, int ldh, const T *__restrict__ w, 
     }
     __syncthreads();
     if (wave != 0) return;
-    const int lanes = lanes_for(E), group_lanes = lanes_for(groups);
-    const int per = E / groups;
-    if (groups > 1) {
-        for (int g = lane; g < groups; g += kWave) {      // a group counts the sum of its two largest choices (of its one, if it has one)
-            float a = -INFINITY, b = -INFINITY;
-            for (int e = g * per; e < (g + 1) * per; e++) {
-                const float c = choice[e];
-                if (c > a) b = a, a = c;
-                else if (c > b) b = c;
-            }
-            gsum[g] = per > 1 ? a + b : a;
-        }
-        __builtin_amdgcn_wave_barrier();
-        __threadfence_block();
-        for (int k = 0; k < kept; k++) {                  // the best group not yet kept: marked with +inf
-            float best = -INFINITY;
-            int at = 0x7fffffff;
-            for (int g = lane; g < groups; g += kWave) {
-                const float s = gsum[g];
-                if (s != INFINITY && s > best) best = s, at = g;
-            }
-            best_of_lanes(best, at, group_lanes);
-            at = __shfl(at, 0, kWave);
-            if (at < 0 || at >= groups) {                 // sums that compare with nothing: the first group not yet kept
-                at = 0;
-                while (at < groups - 1 && gsum[at] == INFINITY) at++;
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (lane == 0) gsum[at] = INFINITY;
-            __builtin_amdgcn_wave_barrier();
-            __threadfence_block();
-        }
-        for (int e = lane; e < E; e += kWave)
-            if (gsum[e / per] != INFINITY) choice[e] = -INFINITY;
-        __builtin_amdgcn_wave_barrier();
-        __threadfence_block();
-    }
-    float picked = 0.f;
-    for (int k = 0; k < top; k++) {
-        float best = -INFINITY;
-        int at = 0x7fffffff;
-        for (int e = lane; e < E; e += kWave) {
-            const float s = choice[e];
-            if (s > best) best = s, at = e;
-        }
-        best_of_lanes(best, at, lanes);
-        if (at < 0 || at >= E) at = k;
-        const float s = score[at];
-        picked += s;
-        __builtin_amdgcn_wave_barrier();
-        if (lane == 0) {
-            ids[r * top + k] = at;
-            picks[k] = s;
-            choice[at] = -INFINITY;
-        }
-        __builtin_amdgcn_wave_barrier();
-        __threadfence_block();
-    }
-    const float factor = route_scale / (picked + 1e-20f);
-    for (int k = lane; k < top; k += kWave) weights[r * top + k] = picks[k] * factor;
+    pick_grouped(score, choice, gsum, picks, E, top, groups, kept, ids + r * top, weights + r * top, route_scale, lane);
 }
 
 // One (row, pick) pair a workgroup row (blockIdx.y), kCols output columns a workgroup (blockIdx.x), two a wave.

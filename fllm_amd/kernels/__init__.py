@@ -51,7 +51,7 @@ assert SAMPLE_ROW_BYTES == 32
 _lib = None
 
 
-ABI_VERSION = 24
+ABI_VERSION = 25
 
 
 def load_library(build_if_missing: bool = True):
@@ -187,6 +187,8 @@ def load_library(build_if_missing: bool = True):
                                c_void],
         "fllm_gate_up_tiles": [c_void, c_int, c_void, c_void, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_void],
         "fllm_linear_tiles": [c_void, c_int, c_void, c_void, c_void, c_int, c_int, c_int, c_int, c_int, c_int, c_void],
+        "fllm_norm_route": [c_void, c_void, c_void, c_float, c_int, c_void, c_float, c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_int,
+                            c_int, c_int, c_int, c_float, c_void, c_void, c_void],
         "fllm_clear_slots": [c_void, c_int, ctypes.c_size_t, c_void, c_int, c_void],
         "fllm_experts_stream_shared": [c_void, c_int, c_void, c_void, c_int, c_int, c_void, c_void, c_int, c_int, c_int, c_int, c_void, c_void,
                                        c_int, c_void, c_void, c_void],
@@ -994,6 +996,40 @@ class Ops:
                                              _ptr(weights), 1 if score == "softmax" else 0, 1 if renormalize else 0, float(route_scale),
                                              _DTYPE_CODE[h.dtype], self._stream()))
         return ids, weights
+
+    def norm_route(self, x: torch.Tensor, norm_weight: torch.Tensor, norm_eps: float, out: torch.Tensor, w_router: torch.Tensor, top: int,
+                   ids: torch.Tensor, weights: torch.Tensor, branch: Optional[torch.Tensor] = None, gain: Optional[torch.Tensor] = None,
+                   eps: Optional[float] = None, correction: Optional[torch.Tensor] = None, groups: int = 1, kept: int = 1, score: str = "sigmoid",
+                   renormalize: bool = False, route_scale: float = 1.0) -> bool:
+        """One kernel for a step of up to 64 rows: with `branch` first x[r] += branch[r] * rsqrt(mean(branch[r]^2) + eps) * gain (eps None:
+        branch[r] * gain), then out = rmsnorm(x) in bfloat16 and the router of out's rows, with `correction` (and groups) as
+        `route_grouped`, without as `route_topk`.  False: not taken (float32, a width that is no multiple of 512 or beyond 4,096, more
+        than 64 experts or rows), nothing was written."""
+        rows, width = x.shape
+        E = w_router.shape[0]
+        if out.dtype != torch.bfloat16 or w_router.dtype != torch.bfloat16 or rows > 64:
+            return False
+        _need(score in ("sigmoid", "softmax"), f"router score {score!r} unknown")
+        _dense(x, "x", torch.float32)
+        _dense(norm_weight, "norm_weight", torch.float32, (width,))
+        _dense(out, "out", torch.bfloat16, (rows, width))
+        _dense(w_router, "w_router", torch.bfloat16, (E, width))
+        _dense(ids, "ids", torch.int32, (rows, top))
+        _dense(weights, "weights", torch.float32, (rows, top))
+        _need((branch is None) == (gain is None), "a branch comes with its gain")
+        if branch is not None:
+            _dense(branch, "branch", torch.float32, (rows, width))
+            _dense(gain, "gain", torch.float32, (width,))
+        if correction is not None:
+            _dense(correction, "correction", torch.float32, (E,))
+        code = self.lib.fllm_norm_route(_ptr(x), _ptr(branch), _ptr(gain), float(eps or 0.0), 0 if eps is None else 1, _ptr(norm_weight),
+                                        float(norm_eps), _ptr(out), rows, width, _ptr(w_router), _ptr(correction), E, int(top), int(groups),
+                                        int(kept), 1 if score == "softmax" else 0, 1 if renormalize else 0, float(route_scale), _ptr(ids),
+                                        _ptr(weights), self._stream())
+        if code == 1:
+            return False
+        self._check(code)
+        return True
 
     def experts_gate_up(self, h: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, w_gate_up: torch.Tensor, act: torch.Tensor,
                         limit: float = 0.0, alpha: float = 1.0, up_offset: float = 0.0) -> torch.Tensor:

@@ -12,6 +12,18 @@ from ..registry import register_part
 from .base import INIT_NORM, Block
 
 
+def norm_and_route(rt, feed_forward, norm, residual, branch=None, gain=None, eps=None):
+    """(h, {"routed": picks}) where a feed-forward of routed experts has one kernel for the sum of a branch (if there is one), the norm
+    before it and its router; (None, {}): nothing was done."""
+    fused = getattr(feed_forward, "norm_route", None)
+    prologue = getattr(norm, "fused_prologue", lambda: None)() if fused is not None else None
+    if prologue is None or residual.shape[0] > 64:
+        return None, {}
+    h = rt.empty(tuple(residual.shape))
+    routed = fused(residual, prologue, h, branch, gain, eps)
+    return (None, {}) if routed is None else (h, {"routed": routed})
+
+
 class PreNormBlock(Block):
     def __init__(self, spec, weights, rt, mixer=None, feed_forward=None, norms=None):
         super().__init__(spec, weights, rt)
@@ -87,8 +99,10 @@ class PreNormBlock(Block):
         ctx.then_norm = None
         if not taken:
             ctx.prepared = None
-            h = self.feed_forward_norm.forward(ctx, residual)
-            self.feed_forward.forward(ctx, h, residual)
+            h, routed = norm_and_route(self.rt, self.feed_forward, self.feed_forward_norm, residual)
+            if h is None:
+                h = self.feed_forward_norm.forward(ctx, residual)
+            self.feed_forward.forward(ctx, h, residual, **routed)
         return None
 
 
@@ -231,8 +245,12 @@ class SandwichBlock(Block):
         begin = getattr(ff, "begin_from_residual", None) if getattr(ff, "stores_branch", False) else None
         prologue = getattr(self.feed_forward_norm, "fused_prologue", lambda: None)()
         takes_stream = begin is not None and getattr(ff, "begins_from_residual", lambda rows: False)(rows)
-        h = None
-        if prologue is not None and not takes_stream:
+        h, routed = None, {}
+        if not takes_stream and branch.shape[0] == rows:
+            h, routed = norm_and_route(rt, ff, self.feed_forward_norm, residual, branch, self.mixer_gain, self.mixer_eps)
+        if h is not None:
+            pass
+        elif prologue is not None and not takes_stream:
             h = rt.empty((rows, self.size))
             ops.postnorm_add(residual, branch, self.mixer_gain, self.mixer_eps, parts=branch.shape[0] // rows,
                              next_weight=prologue[0], next_eps=prologue[1], next_out=h)
@@ -245,10 +263,10 @@ class SandwichBlock(Block):
             if begun is not None:
                 ff.finish(ctx, begun, None, branch=branch)
             else:
-                ff.forward(ctx, h if h is not None else self.feed_forward_norm.forward(ctx, residual), None, branch=branch)
+                ff.forward(ctx, h if h is not None else self.feed_forward_norm.forward(ctx, residual), None, branch=branch, **routed)
         else:
             branch = torch.zeros((rows, self.size), dtype=torch.float32, device=rt.device)
-            ff.forward(ctx, h if h is not None else self.feed_forward_norm.forward(ctx, residual), branch)
+            ff.forward(ctx, h if h is not None else self.feed_forward_norm.forward(ctx, residual), branch, **routed)
         ops.postnorm_add(residual, branch, self.feed_forward_gain, self.feed_forward_eps, parts=branch.shape[0] // rows)
 
 

@@ -114,19 +114,34 @@ class RoutedExperts(FeedForward):
             return self.top + 1
         return self.branch_parts
 
-    def forward(self, ctx, h, residual, branch=None):
+    def norm_route(self, residual, norm, h, branch=None, gain=None, eps=None):
+        """The norm before this part (`fused_prologue`'s pair) of the stream's rows into `h`, behind the sum of a branch where there is
+        one (as `postnorm_add`), and the router, in one kernel: what `forward` takes as `routed`.  None: nothing was done."""
+        fused = getattr(self.rt.ops, "norm_route", None)
+        if fused is None or self.rt.dtype != torch.bfloat16:
+            return None
+        rows = residual.shape[0]
+        ids, weights = self.rt.empty((rows, self.top), torch.int32), self.rt.empty((rows, self.top), torch.float32)
+        how = (dict(correction=self.correction, groups=self.groups, kept=self.groups_kept) if self.grouped_router
+               else dict(score=self.score, renormalize=self.renormalize))
+        taken = fused(residual, norm[0], norm[1], h, self.w_router, self.top, ids, weights, branch=branch, gain=gain, eps=eps,
+                      route_scale=self.route_scale, **how)
+        return (ids, weights) if taken else None
+
+    def forward(self, ctx, h, residual, branch=None, routed=None):
         """`branch`: float32 [rows * branch_parts, width], row r's picks at r * top .. or its finished sum at r, or
-        [rows * branch_parts_for(rows), width]; None: the sum goes into `residual`."""
+        [rows * branch_parts_for(rows), width]; None: the sum goes into `residual`.  `routed`: the picks, where
+        `norm_route` has made them."""
         rows = h.shape[0]
+        ids, weights = routed if routed is not None else self._route(h)
         if branch is not None and self.shared and branch.shape[0] == rows * (self.top + 1):
-            ids, weights = self._route(h)
             if self.rt.ops.experts_stream_shared(h, ids, weights, self.w_up, self.w_down, self.w_shared_up, self.w_shared_down, branch):
                 return
             whole = self.rt.empty((rows, self.hidden), torch.float32)      # the plain kernels were asked for
             self._forward(ctx, h, None, whole, ids, weights)
             branch.zero_().view(rows, self.top + 1, self.hidden)[:, 0].copy_(whole)
             return
-        self._forward(ctx, h, residual, branch, *self._route(h))
+        self._forward(ctx, h, residual, branch, ids, weights)
 
     def _route(self, h):
         """The experts that each row picks and their weights."""
