@@ -250,6 +250,7 @@ class SquaredReLUMLP(FeedForward):
         self.w_up = rt.matrix(weights["up"])
         self.w_down = rt.matrix(weights["down"])
         rt.tile_for_decode(self.w_down)
+        rt.tile_for_decode(self.w_up, priority=1)
 
     def forward(self, ctx, h, residual, branch=None):
         rt, ops = self.rt, self.rt.ops
