@@ -6,9 +6,11 @@ library cannot be loaded or built, constructing `Ops` raises.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import functools
 import math
+import threading
 import weakref
 from typing import Dict, NamedTuple, Optional, Sequence, Tuple
 
@@ -297,6 +299,8 @@ class Ops:
         if not torch.cuda.is_available():
             raise KernelError("no GPU is visible: the engine runs on gfx950 only")
         self.lib = load_library()
+        # a thread's `copies_together`: .slab = [bytes still to come, memory of the copies being made, elements of it taken]
+        self._copies = threading.local()
         self.library_gemm_from = library_gemm_from
         self.fused_decode_rows = int(fused_decode_rows)
         self._device_workspace(torch.cuda.current_device())
@@ -317,6 +321,29 @@ class Ops:
     # ---- tile-major copies of weights for decode steps --------------------------------------------------
     _tiles: Dict[int, Tuple[tuple, torch.Tensor]] = {}     # address of a weight matrix -> (its shape, its tile-major copy)
 
+    _SLAB_BYTES = 256 << 20
+
+    @contextlib.contextmanager
+    def copies_together(self, nbytes: int):
+        """Copies made inside (about `nbytes` in all) lie in pieces of up to 256 MiB instead of an allocation each, which a model
+        pays for when it is built and again when it goes; a piece is given back with the last matrix whose copy lies in it."""
+        self._copies.slab = [int(nbytes), None, 0]
+        try:
+            yield
+        finally:
+            self._copies.slab = None
+
+    def _room_for_copy(self, elements: int, device) -> torch.Tensor:
+        slab = getattr(self._copies, "slab", None)
+        if slab is None or 2 * elements > Ops._SLAB_BYTES:
+            return torch.empty(elements, dtype=torch.bfloat16, device=device)
+        if slab[1] is None or slab[1].device != device or slab[2] + elements > slab[1].numel():
+            slab[1], slab[2] = torch.empty(max(elements, min(Ops._SLAB_BYTES, slab[0]) // 2), dtype=torch.bfloat16, device=device), 0
+        at = slab[2]
+        slab[0] = max(0, slab[0] - 2 * elements)
+        slab[2] = at + -(-elements // 128) * 128      # on 256 bytes
+        return slab[1][at:at + elements]
+
     def tile_for_decode(self, w: torch.Tensor, gate_up: bool = False) -> bool:
         """Keeps beside `w` (bfloat16 [N, K] on the GPU) a copy in the order in which the products of decode steps read
         it (`fllm_tile_weights`): `linear`, `linear_add_prepare`, `linear_relu_squared` and the forms behind a norm find it by
@@ -335,10 +362,10 @@ class Ops:
             return True
         with torch.cuda.device(w.device):
             if gate_up:
-                tiles = torch.empty(int(self.lib.fllm_weight_tiles_elements_gate_up(N // 2, K)), dtype=torch.bfloat16, device=w.device)
+                tiles = self._room_for_copy(int(self.lib.fllm_weight_tiles_elements_gate_up(N // 2, K)), w.device)
                 self._check(self.lib.fllm_tile_weights_gate_up(_ptr(w), _ptr(tiles), N // 2, K, self._stream()))
             else:
-                tiles = torch.empty(int(self.lib.fllm_weight_tiles_elements(N, K)), dtype=torch.bfloat16, device=w.device)
+                tiles = self._room_for_copy(int(self.lib.fllm_weight_tiles_elements(N, K)), w.device)
                 self._check(self.lib.fllm_tile_weights(_ptr(w), _ptr(tiles), N, K, self._stream()))
         Ops._tiles[key] = (kind, tiles)
         weakref.finalize(w, Ops._tiles.pop, key, None)
@@ -1116,7 +1143,7 @@ class Ops:
         if key in Ops._tiles and Ops._tiles[key][0] == kind:
             return True
         with torch.cuda.device(w.device):
-            tiles = torch.empty(E * N * K, dtype=torch.bfloat16, device=w.device)
+            tiles = self._room_for_copy(E * N * K, w.device)
             self._check(self.lib.fllm_tile_weights(_ptr(w), _ptr(tiles), E * N, K, self._stream()))
         Ops._tiles[key] = (kind, tiles)
         weakref.finalize(w, Ops._tiles.pop, key, None)

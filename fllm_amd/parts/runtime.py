@@ -1,6 +1,7 @@
 """What parts get to work with: the device, the compute precision and the kernel library."""
 from __future__ import annotations
 
+import contextlib
 import weakref
 from typing import Any, Dict
 
@@ -99,15 +100,17 @@ class Runtime:
             free, _ = torch.cuda.mem_get_info(self.device)
             budget, experts_budget = free // 2, free // 8
         made = 0
-        for priority, _, size, make in requests:
-            if budget is not None and size > (min(budget, experts_budget) if priority == EXPERTS else budget):
-                continue
-            if make():
-                made += size
-                if budget is not None:
-                    budget -= size
-                    if priority == EXPERTS:
-                        experts_budget -= size
+        together = getattr(self.ops, "copies_together", None)
+        with together(sum(r[2] for r in requests)) if together is not None else contextlib.nullcontext():
+            for priority, _, size, make in requests:
+                if budget is not None and size > (min(budget, experts_budget) if priority == EXPERTS else budget):
+                    continue
+                if make():
+                    made += size
+                    if budget is not None:
+                        budget -= size
+                        if priority == EXPERTS:
+                            experts_budget -= size
         return made
 
     def forget_host_tensors(self) -> None:

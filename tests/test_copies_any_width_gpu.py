@@ -91,3 +91,23 @@ def test_what_is_read_beside_the_copy_stays_accepted(ops):
     out = ops.linear(x, w, torch.empty(3, 64, dtype=BF16, device=DEV))
     torch.testing.assert_close(out.double(), x.double() @ w.double().T, rtol=2.0 ** -8, atol=1e-4)
     assert not ops.tile_for_decode(draw((64 * 512 + 1,), 3)[1:].view(64, 512))
+
+
+def test_copies_of_a_model_share_their_memory(ops):
+    """Copies made together lie side by side, each on 256 bytes and whole, large ones in memory of their own; each goes with its matrix."""
+    from fllm_amd.kernels import Ops
+    ws = [draw((n, k), n + k) for n, k in ((16, 256), (40, 288), (1000, 544), (17, 1536))]
+    wide = draw((4096, 40000), 7)
+    gone = len(Ops._tiles)
+    with ops.copies_together(sum(2 * w.numel() for w in ws)):
+        for w in ws + [wide]:
+            assert ops.tile_for_decode(w)
+    tiles = [ops._tiles_of(w) for w in ws]
+    assert len({t.untyped_storage().data_ptr() for t in tiles}) < len(ws) and all(t.data_ptr() % 256 == 0 for t in tiles)
+    assert ops._tiles_of(wide).untyped_storage().nbytes() < 2 * wide.numel() + (2 << 20)
+    alone = [w.clone() for w in ws]
+    for w, t, other in zip(ws, tiles, alone):
+        assert ops.tile_for_decode(other) and torch.equal(ops._tiles_of(other), t)
+    assert len(Ops._tiles) == gone + 2 * len(ws) + 1
+    del ws, wide, alone, w, other
+    assert len(Ops._tiles) == gone
