@@ -312,10 +312,12 @@ size_t fllm_talking_attention_workspace(int rows, int num_segs, int heads, int v
 // A branch that is normed on its way into the float32 residual stream: v = the sum of the row's `parts` partial branches
 // (branch: [rows, parts, width] of `branch_dtype`), x[r] += v * rsqrt(mean(v^2) + eps) * gain (normalize 0: x[r] += v * gain).
 // With next_w, next_out[r] = rmsnorm(x[r]) * next_w with next_eps (of `next_dtype`) as well.
+// With next_ssq (float32 [rows]) the norm is prepared instead: next_out[r] = x[r] * next_w, next_ssq[r] = the sum of x[r]^2.
 // part_weights (float32 [rows * parts], or null): partial row k of a token is multiplied by its weight as it is summed.
 int fllm_postnorm_add(float *x, const void *branch, int branch_dtype, int parts, const float *part_weights, const float *gain, float eps,
                       int normalize,
-                      const float *next_w, float next_eps, void *next_out, int next_dtype, int rows, int width, hipStream_t stream);
+                      const float *next_w, float next_eps, void *next_out, int next_dtype, float *next_ssq, int rows, int width,
+                      hipStream_t stream);
 
 // Routed experts, plain kernels.  fllm_route_topk: score = sigmoid(w_router h) in float32 ([E, K] beside rows [rows, K] of
 // `dtype`, row stride ldh); ids[r, k] / weights[r, k] = the expert with the k-th largest score of row r (the lower index

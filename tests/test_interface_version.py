@@ -9,7 +9,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 # version -> the first of the digest of csrc/api.h's declarations (comments and spaces aside).  An entry point that is added, taken away
 # or given other arguments needs a new version in csrc/runtime.hip and kernels/__init__.py, and a line here.
 DECLARATIONS = {20: "1e1b23230576f9ec", 21: "19b0612161b5bb86", 22: "24410fd5ad499510", 23: "40662c18965df9ba", 24: "f920d1abedef5fa6",
-                25: "5d11631c9e87062c"}
+                25: "5d11631c9e87062c", 26: "b420149118ad7001"}
 
 
 def declarations(text: str) -> str:
