@@ -257,7 +257,7 @@ def _dense(t: torch.Tensor, name: str, dtype=None, shape=None) -> None:
         raise KernelError(f"{name} must be contiguous")
     if dtype is not None and t.dtype != dtype:
         raise KernelError(f"{name} must be {dtype}, is {t.dtype}")
-    if shape is not None and tuple(t.shape) != tuple(shape):
+    if shape is not None and t.shape != tuple(shape):      # a torch.Size is a tuple
         raise KernelError(f"{name} must have shape {tuple(shape)}, has {tuple(t.shape)}")
 
 
@@ -375,9 +375,10 @@ class Ops:
         """The copy of `w` that a product of `rows` rows may read, or None: up to 16 rows any, beyond them those whose widths the chunk
         kernels were measured at beside the GEMM library (steps of 1,024)."""
         held = Ops._tiles.get(w.data_ptr())
-        if held is None or held[0] != (w.shape[0], w.shape[1], bool(gate_up)) or (rows > self.PREPARED_NORM_ROWS and w.shape[1] % 1024 != 0):
+        if held is None:
             return None
-        return held[1]
+        kind, tiles = held
+        return tiles if kind == (*w.shape, gate_up) and (rows <= self.PREPARED_NORM_ROWS or kind[1] % 1024 == 0) else None
 
     # 17 to 128 rows beside the GEMM library: with the tile-major copies the own products of the feed-forward (gate/up
     # with its SwiGLU epilogue, down with the residual sum) are faster than the library's products and the SwiGLU kernel
@@ -500,8 +501,9 @@ class Ops:
             _dense(bias, "bias", torch.float32, (N,))
         ldx = x.stride(0) if M > 1 else K
         ldo = out.stride(0) if M > 1 else N
-        most = self.ADD_KERNEL_ROWS if mode == OUT_ADD_F32 else 64 if mode == OUT_STORE_F32 else self._store_tiled_rows()
-        tiles = self._tiles_of(w, rows=M) if Ops._tiles and M <= most else None
+        tiles = None
+        if Ops._tiles and M <= (self.ADD_KERNEL_ROWS if mode == OUT_ADD_F32 else 64 if mode == OUT_STORE_F32 else self._store_tiled_rows()):
+            tiles = self._tiles_of(w, rows=M)
         if tiles is not None and ldx % 8 == 0 and x.data_ptr() % 16 == 0 and (M <= 64 or K % 256 == 0):
             entry = (self.lib.fllm_linear_store_tiled, self.lib.fllm_linear_f32_tiled, self.lib.fllm_linear_add_tiled)[mode]
             self._check(entry(_ptr(x), ldx, _ptr(w), _ptr(tiles), _ptr(bias), _ptr(out), ldo, M, N, K, self._stream()))

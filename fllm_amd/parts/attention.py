@@ -107,6 +107,10 @@ class PagedAttention(Mixer):
             order_k = self._pair_order(self.kv_heads, d0, self.position.dims).to(rt.device)
         elif self.position is not None:
             self.pairing = self.position.pairing
+        # whether the fused store takes these heads (keys and values of one width, keys in chunks of 8, rotated or not), and with it
+        # a norm that the sum before it has prepared
+        self.takes_prepared = (rt.dtype == torch.bfloat16 and self.pairing == 1 and self.head_dim % 4 == 0 and not self.shape_args
+                               and self.qk_norm_eps is None and self.sink is None)
         reorder = lambda t, order: t if order is None or t is None else t.index_select(0, order)
 
         def widen(t, heads, have, want):
@@ -177,12 +181,6 @@ class PagedAttention(Mixer):
                           nh, nkv, d, dims, pairing, binding.page_size, **self.shape_args)
         self._attend_and_project(ctx, qkv[:, : nh * d], residual, binding, branch=branch)
 
-    @property
-    def takes_prepared(self) -> bool:
-        """Whether `forward_from_residual` makes use of a norm that the sum before it has prepared."""
-        return (self.rt.dtype == torch.bfloat16 and self.pairing == 1 and self.head_dim % 4 == 0 and not self.shape_args
-                and self.qk_norm_eps is None and self.sink is None)
-
     def forward_from_residual(self, ctx, residual, norm, binding, branch=None) -> bool:
         """Decode-sized steps in bfloat16: the norm before the mixer, the q/k/v product, rotary and the
         cache store are one kernel.  False: not taken, the block runs norm and `forward`."""
@@ -191,7 +189,7 @@ class PagedAttention(Mixer):
         prologue = getattr(norm, "fused_prologue", lambda: None)()
         form = fused_form(ops, rows, self.hidden, self.w_qkv) if hasattr(ops, "norm_qkv_rope_store") else None
         if prologue is None or form is None or not self.takes_prepared:
-            return False         # the fused store takes keys and values of one width, keys in chunks of 8, and rotates
+            return False
         norm_scale, norm_eps = prologue
         nh, nkv, d = self.heads, self.kv_heads, self.head_dim
         if self.position is not None:
