@@ -442,7 +442,7 @@ polynorm_vec_kernel(const bf16_t *__restrict__ z, int ld, const float *__restric
 }
 
 // ---- q and k normed a head, k and v into the pages ---------------------------------------------------------------------------------
-// One workgroup a row of [q | k | v | ..] (row stride ld); a wave takes a head at a time.  The mean is over `norm_dim` lanes
+// Rows of [q | k | v | ..] (row stride ld), grid (rows, workgroups that share a row's heads); a wave takes a head at a time.  The mean is over `norm_dim` lanes
 // (heads widened with zero lanes keep the mean of their own lanes).
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
@@ -462,9 +462,26 @@ head_norm_kv_store_kernel(T *__restrict__ qkv, int ld, float eps, int norm_dim, 
         off = pos % page_size;
     }
     const int normed = store_kv ? heads + kv_heads : heads;
-    for (int h = wave; h < normed; h += kWaves) {
+    for (int h = blockIdx.y * kWaves + wave; h < normed; h += gridDim.y * kWaves) {
         T *head = row + (size_t)h * head_dim;
         float ss = 0.f;
+        if (head_dim <= 4 * kWave) {       // a head's lanes asked for at once
+            float a[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) a[k] = lane + k * kWave < head_dim ? to_f32<T>(head[lane + k * kWave]) : 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; k++) ss = fmaf(a[k], a[k], ss);
+            const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)norm_dim + eps);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int c = lane + k * kWave;
+                if (c >= head_dim) break;
+                const T y = from_f32<T>(a[k] * inv);
+                if (h < heads) head[c] = y;
+                else k_pages[key_offset_chunked(page, kv_heads, h - heads, page_size, head_dim, off, c, key_chunk)] = y;
+            }
+            continue;
+        }
         for (int c = lane; c < head_dim; c += kWave) {
             const float a = to_f32<T>(head[c]);
             ss = fmaf(a, a, ss);
@@ -479,7 +496,7 @@ head_norm_kv_store_kernel(T *__restrict__ qkv, int ld, float eps, int norm_dim, 
     }
     if (!store_kv) return;
     const T *vrow = row + (size_t)(heads + kv_heads) * head_dim;
-    for (int i = threadIdx.x; i < kv_heads * v_dim; i += kBlock) {
+    for (int i = blockIdx.y * kBlock + threadIdx.x; i < kv_heads * v_dim; i += gridDim.y * kBlock) {
         const int h = i / v_dim, c = i - h * v_dim;
         v_pages[(((size_t)page * kv_heads + h) * v_dim + c) * page_size + off] = vrow[i];
     }
@@ -655,12 +672,16 @@ extern "C" int fllm_head_norm_kv_store(void *qkv, int ld, float eps, int norm_di
                  key_chunk);
     FLLM_REQUIRE(qkv && row_pos && row_seg && tables && (!store_kv || (k_pages && v_pages)), "head_norm_kv_store: operands missing");
     if (rows == 0) return 0;
+    // A head a wave in steps of few rows (a workgroup a row, whose waves take several heads one after the other, runs 7.3 us at 4 rows of
+    // 12 and 2 heads of 128 where this takes 4.3); rows that fill the device by themselves keep a workgroup each (2,000 rows: 13.9 us, and
+    // 15.3 with a head a wave).
+    const dim3 grid(rows, rows > 512 ? 1u : (unsigned)std::min(((store_kv ? heads + kv_heads : heads) + kWaves - 1) / kWaves, 65535));
     if (dtype == FLLM_F32)
-        hipLaunchKernelGGL(head_norm_kv_store_kernel<float>, dim3(rows), dim3(kBlock), 0, stream, (float *)qkv, ld, eps, norm_dim, row_pos,
+        hipLaunchKernelGGL(head_norm_kv_store_kernel<float>, grid, dim3(kBlock), 0, stream, (float *)qkv, ld, eps, norm_dim, row_pos,
                            row_seg, tables, table_stride, (float *)k_pages, (float *)v_pages, heads, kv_heads, head_dim, v_dim, page_size,
                            key_chunk, store_kv);
     else if (dtype == FLLM_BF16)
-        hipLaunchKernelGGL(head_norm_kv_store_kernel<bf16_t>, dim3(rows), dim3(kBlock), 0, stream, (bf16_t *)qkv, ld, eps, norm_dim, row_pos,
+        hipLaunchKernelGGL(head_norm_kv_store_kernel<bf16_t>, grid, dim3(kBlock), 0, stream, (bf16_t *)qkv, ld, eps, norm_dim, row_pos,
                            row_seg, tables, table_stride, (bf16_t *)k_pages, (bf16_t *)v_pages, heads, kv_heads, head_dim, v_dim,
                            page_size, key_chunk, store_kv);
     else
