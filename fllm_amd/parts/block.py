@@ -15,9 +15,9 @@ from .base import INIT_NORM, Block, leave_prepared
 def norm_and_route(rt, feed_forward, norm, residual, branch=None, gain=None, eps=None):
     """(h, {"routed": picks}) where a feed-forward of routed experts has one kernel for the sum of a branch (if there is one), the norm
     before it and its router; (None, {}): nothing was done."""
-    fused = getattr(feed_forward, "norm_route", None)
+    fused = getattr(feed_forward, "norm_route", None) if residual.shape[0] <= 64 else None
     prologue = getattr(norm, "fused_prologue", lambda: None)() if fused is not None else None
-    if prologue is None or residual.shape[0] > 64:
+    if prologue is None:
         return None, {}
     h = rt.empty(tuple(residual.shape))
     routed = fused(residual, prologue, h, branch, gain, eps)
@@ -227,10 +227,11 @@ class SandwichBlock(Block):
         (`ctx.next_norm`): with the feed-forward's normed rows below, prompts and answers of 8 requests of 42 layers, 1,536 wide,
         11.45 -> 11.29 ms.  Beyond 16 rows the products behind a norm take another form."""
         ops, (rows, width) = self.rt.ops, residual.shape
-        after, ctx.prepared = getattr(ctx, "next_norm", None), None
+        ctx.prepared = None
+        prepare = getattr(ops, "postnorm_add_prepare", None) if rows <= 16 and self.rt.dtype == torch.bfloat16 else None
+        after = getattr(ctx, "next_norm", None) if prepare is not None else None
         prologue = getattr(after, "fused_prologue", lambda: None)() if after is not None else None
-        prepare = getattr(ops, "postnorm_add_prepare", None)
-        if prologue is None or prepare is None or self.rt.dtype != torch.bfloat16 or rows > ops.PREPARED_NORM_ROWS or not ops.prepares_norm(rows, width):
+        if prologue is None or not ops.prepares_norm(rows, width):
             ops.postnorm_add(residual, branch, gain, eps, parts=branch.shape[0] // rows)
             return
         leave_prepared(ctx, after, residual, prepare(residual, branch, gain, eps, prologue[0], parts=branch.shape[0] // rows))
