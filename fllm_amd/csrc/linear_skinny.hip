@@ -1351,15 +1351,11 @@ int launch_resident(const SkinnyArgs &a, hipStream_t stream) {
         // tile and two tiles per slot, unevenly: 384 tiles on 512 slots run as long as 512 would.  Also when the 16-row
         // tiles fill no more than half of the compute units (narrow models): twice the workgroups, each with half the
         // weights (128 tiles of 2,048 x 8,192: 12.7 -> 9.4 us at one row; 192 tiles gain nothing, 7.7 -> 8.1 us, and at
-        // 256 tiles it is the other way round, 26.9 -> 32.3 us).  From a tile-major copy the uneven ones run whole tiles all the
-        // same: an 8-row tile takes 128 of each 256 bytes a load, a whole one 1 KiB in a row (13,312 x 1,536 at 1 / 3 / 8 rows 11.6 ->
-        // 10.1 / 12.5 -> 10.4 / 15.0 -> 11.0 us, 4,608 x 1,536 6.5 -> 5.7 / 7.1 -> 6.0 / 8.2 -> 6.3, 6,144 x 1,024 5.8 -> 4.8 / 6.2 -> 5.1 / 6.7 ->
-        // 5.5; the few tiles of 1,536 x 8,960 the other way, 8.5 -> 11.5 / 9.3 -> 11.9 / 11.8 -> 13.1).  Sums into the
-        // stream keep the tiles they have without a copy, so that whether there was memory for one changes no bit of them.
-        const bool tiled = streams_tiles(a, p, a.N) && (x_direct || fllm_option_resident_tiles());
+        // 256 tiles it is the other way round, 26.9 -> 32.3 us)
         const int slots = device_cus() * p.per_cu;
         const bool uneven = 2 * tiles16 > slots && tiles16 < 2 * slots && tiles16 % slots != 0;
-        const bool dual = a.M <= 8 && p.S == 1 && fllm_option_dual_k() && ((uneven && !(tiled && EPI != EPI_ADD)) || 2 * tiles16 <= device_cus());
+        const bool dual = a.M <= 8 && p.S == 1 && fllm_option_dual_k() && (uneven || 2 * tiles16 <= device_cus());
+        const bool tiled = streams_tiles(a, p, a.N) && (x_direct || fllm_option_resident_tiles());
         // q/k/v behind a prepared norm and the vocabulary projection: whole 16-row tiles where there is a copy, rather than
         // 8-row tiles.  Reading the activations straight from global memory as the output projection does is slower for q/k/v
         // (4,096 x 6,144 at 1, 8, 16 rows: 14.0, 15.4, 18.3 us against 12.4, 15.0, 18.1 staged).
