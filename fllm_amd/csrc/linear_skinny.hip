@@ -309,6 +309,8 @@ __device__ __forceinline__ void epilogue(const SkinnyArgs &a, f32x4_t (&s)[RT], 
 //              range): A row r and B column r take K half r / 8, so D[r][c] is a partial sum where
 //              r / 8 == c / 8, and the two are added at the end               (8 outputs a row)
 //   TM_GATEUP  8 gate rows and the 8 up rows that belong to them              (8 outputs a row)
+//   TM_HALVES  16 weight rows that add as TM_DUALK does: the two halves of the wave's range one after the other, each into
+//              sums of its own (16 outputs a row)
 // The smaller tiles are what fills the chip evenly: 16-row tiles of the model's projections come to
 // 1.5 or 3.5 a compute-unit slot.
 //
@@ -317,7 +319,7 @@ __device__ __forceinline__ void epilogue(const SkinnyArgs &a, f32x4_t (&s)[RT], 
 // fit into LDS) it leaves the item's sums in the workspace and counts the item; the workgroup that
 // counts a tile's last item adds the S partial sums in slice order and runs the epilogue, so the
 // result does not depend on which workgroup came last.
-enum { TM_ROWS16 = 0, TM_DUALK = 1, TM_GATEUP = 2 };
+enum { TM_ROWS16 = 0, TM_DUALK = 1, TM_GATEUP = 2, TM_HALVES = 3 };
 
 // A load of weights.  Every weight is read once a step, so the loads from the tile-major copies carry the
 // non-temporal hint: the lines do not push the activations, which every workgroup reads again, out of the caches, and a
@@ -342,7 +344,8 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
     constexpr int U = 4;                           // k-steps of 32 per block: four 16-byte loads per lane
     constexpr int KB = 32 * U;                     // K elements of one range per block
     constexpr int RB = 4;                          // rows of activations staged at a time (more would spill registers)
-    constexpr int NT = TM == TM_ROWS16 ? 16 : 8;   // outputs per row and tile
+    constexpr bool WHOLE = TM == TM_ROWS16 || TM == TM_HALVES;      // 16 weight rows
+    constexpr int NT = WHOLE ? 16 : 8;             // outputs per row and tile
     constexpr int RT = EPI == EPI_SWIGLU ? 2 : 1;
     static_assert((EPI == EPI_SWIGLU) == (TM == TM_GATEUP), "gate/up tiles belong to the SwiGLU epilogue");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -354,7 +357,7 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
     const int ntiles = (n_out + NT - 1) / NT;
     const int pitch = a.slice + 8;
     bf16_t *xs = (bf16_t *)smem;                                  // [M][pitch]
-    f32x4_t *red = (f32x4_t *)(smem + red_off);                   // [WAVES][64]
+    f32x4_t *red = (f32x4_t *)(smem + red_off);                   // [WAVES][64], TM_HALVES: one for each half
     float *ssq_part = (float *)(smem + a.ssq_off);                // [WAVES][16]
 
     const int sl = blockIdx.x % S;
@@ -365,12 +368,14 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
     // the wave's contiguous part of the slice (relative to ks0), in steps of 64, and its blocks (the same number for every wave)
     const int kwlen = ((kcn + WAVES - 1) / WAVES + 63) / 64 * 64;
     const int kw0 = min(kcn, wave * kwlen), kw1 = min(kcn, kw0 + kwlen);
-    const int half = TM == TM_DUALK ? kwlen / 2 : kwlen;          // the K range that one A row covers in an item
-    const int nbw = (half + KB - 1) / KB;
+    const int half = TM == TM_DUALK || TM == TM_HALVES ? kwlen / 2 : kwlen;     // the K range that one A row covers in an item (or half of one)
+    const int nbh = (half + KB - 1) / KB, nbw = TM == TM_HALVES ? 2 * nbh : nbh;
     // this lane's A row and B column: weight row in the tile, activation row, and where its K range starts
-    const int wrow_in_tile = TM == TM_ROWS16 ? r : (r & 7) + (TM == TM_GATEUP ? (r >> 3) * n_out : 0);
     const int kr0 = kw0 + (TM == TM_DUALK ? (r >> 3) * half : 0) + g * 8;      // relative to ks0
     const int kr1 = TM == TM_DUALK ? min(kw1, kw0 + ((r >> 3) + 1) * half) : kw1;
+    // where block j of an item begins, and the end of the range it belongs to
+    auto begin_of = [&](int j) __attribute__((always_inline)) { return kr0 + (TM == TM_HALVES && j >= nbh ? half + (j - nbh) * KB : j * KB); };
+    auto end_of = [&](int j) __attribute__((always_inline)) { return TM == TM_HALVES && j < nbh ? min(kr1, kw0 + half) : kr1; };
     const int row_limit = TM == TM_GATEUP ? n_out : N;            // weight rows past it are clamped (never stored)
 
     // cursor of the loads: (item, block in item) of the next block to ask for
@@ -384,10 +389,10 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
     };
     auto issue = [&](Block &buf) {
         if (l_item < my_items) {
-            int row = (tile0 + l_item * tstride) * NT + (TM == TM_ROWS16 ? r : (r & 7));
+            int row = (tile0 + l_item * tstride) * NT + (WHOLE ? r : (r & 7));
             if (row >= row_limit) row = row_limit - 1;
             if (TM == TM_GATEUP) row += (r >> 3) * n_out;
-            const int kb = kr0 + l_j * KB;
+            const int kb = begin_of(l_j), ke = end_of(l_j);
             if (WT) {
                 // tile-major weights (fllm_tile_weights, one slice): the 16 rows x 32 columns of a k-step lie together in the order
                 // the lanes take them, so a load instruction reads 1 KiB in a row instead of 64 bytes of each of 16 rows.
@@ -396,21 +401,20 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
                 const int tile16 = TM == TM_DUALK ? tile >> 1 : tile, row16 = TM == TM_DUALK ? (tile & 1) * 8 + (r & 7) : r;
                 const bf16_t *wp = a.w_tiles + (size_t)tile16 * 16 * K + (size_t)((kb - g * 8) / 32) * (16 * 32) + (g * 16 + row16) * 8;
 #pragma unroll
-                for (int u = 0; u < U; u++) buf.w[u] = kb + u * 32 < kr1 ? load_weights<true>(wp + u * (16 * 32)) : zero8();
+                for (int u = 0; u < U; u++) buf.w[u] = kb + u * 32 < ke ? load_weights<true>(wp + u * (16 * 32)) : zero8();
             } else {
                 const bf16_t *wp = a.w + (size_t)row * K + ks0 + kb;
 #pragma unroll
-                for (int u = 0; u < U; u++) buf.w[u] = kb + u * 32 < kr1 ? load_weights<false>(wp + u * 32) : zero8();
+                for (int u = 0; u < U; u++) buf.w[u] = kb + u * 32 < ke ? load_weights<false>(wp + u * 32) : zero8();
             }
             if (XD) {
                 const bf16_t *xp = (const bf16_t *)a.x + (size_t)xrow_i * a.ldx + ks0 + kb;
 #pragma unroll
-                for (int u = 0; u < U; u++) buf.x[XD ? u : 0] = (kb + u * 32 < kr1 && xvalid) ? *(const bf16x8_t *)(xp + u * 32) : zero8();
+                for (int u = 0; u < U; u++) buf.x[XD ? u : 0] = (kb + u * 32 < ke && xvalid) ? *(const bf16x8_t *)(xp + u * 32) : zero8();
             }
         }
         if (++l_j == nbw) l_j = 0, l_item++;
     };
-    (void)wrow_in_tile;
     // SCALED: the parts of the sums of squares of this wave's rows (rows wave and wave + WAVES) are asked for before
     // anything else and added up after the staging, when they have long arrived: up to 256 parts a row, four a lane
     f32x4_t ssq_pre[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
@@ -432,7 +436,7 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
     // what the epilogue reads besides the sums: the part that belongs to this lane's row now, the part that belongs
     // to an item when the wave whose turn it is to finish the item starts on it
     const int m_out = TM == TM_DUALK ? (r & 7) : r;
-    const bool owner = TM == TM_ROWS16 ? true : (g < 2 && (TM == TM_GATEUP || r < 8));
+    const bool owner = WHOLE ? true : (g < 2 && (TM == TM_GATEUP || r < 8));
     EpilogueOperands eo;
     load_row_operands<EPI>(a, m_out, eo);
     auto item_operands = [&](int it) {
@@ -515,16 +519,16 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
     // cursor of the products
     int item = 0, j = 0;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-    const bf16_t *xrow = xs + xrow_i * pitch + kr0;
+    const bf16_t *xrow = xs + xrow_i * pitch;
     FLLM_STAMP(a, 1);
 
     auto step = [&](Block &buf) {
         bf16x8_t xf[U];
-        const int kb = kr0 + j * KB;
+        const int kb = begin_of(j), ke = end_of(j);
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (XD) xf[u] = buf.x[XD ? u : 0];
-            else xf[u] = (kb + u * 32 < kr1 && xvalid) ? *(const bf16x8_t *)(xrow + j * KB + u * 32) : zero8();
+            else xf[u] = (kb + u * 32 < ke && xvalid) ? *(const bf16x8_t *)(xrow + kb + u * 32) : zero8();
         }
 #pragma unroll
         for (int u = 0; u < U; u++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(buf.w[u], xf[u], acc, 0, 0, 0);
@@ -535,12 +539,16 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
             FLLM_STAMP(a, 2);
         }
 #endif
+        if (TM == TM_HALVES && j + 1 == nbh) {      // the first half's sums (behind the item before's second barrier: its sums have been read)
+            red[wave * kWave + lane] = acc;
+            acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        }
         if (++j < nbw) return;
         // the item is complete: the waves' sums meet in LDS; one wave (they take turns) adds them up and goes on
         // to the epilogue while the others start the next item
         j = 0;
         if (item == my_items - 1) FLLM_STAMP(a, 3);
-        red[wave * kWave + lane] = acc;
+        red[((TM == TM_HALVES ? WAVES : 0) + wave) * kWave + lane] = acc;
         acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
         __syncthreads();
         const int tile = tile0 + item * tstride;
@@ -555,6 +563,7 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
             for (int wv = 0; wv < WAVES; wv++) {
                 s[0] += red[wv * kWave + lane];
                 if (TM == TM_DUALK) s[0] += red[wv * kWave + lane + 40];
+                if (TM == TM_HALVES) s[0] += red[(WAVES + wv) * kWave + lane];
                 if (TM == TM_GATEUP) s[RT - 1] += red[wv * kWave + lane + 32];
             }
         }
@@ -1252,9 +1261,9 @@ int launch_resident_plan(SkinnyArgs a, const ResidentPlan &p, int ntiles, const 
 #endif
     a.S = p.S;
     a.slice = p.slice;
-    a.ssq_off = (int)(p.stage + p.red);
+    a.ssq_off = (int)(p.stage + (TM == TM_HALVES ? 2 : 1) * p.red);
     if (a.next_x != nullptr) {
-        a.next_nt = TM == TM_ROWS16 ? 16 : 8;
+        a.next_nt = TM == TM_ROWS16 || TM == TM_HALVES ? 16 : 8;
         a.next_tiles = ntiles;
         if (a.next_tiles_out != nullptr) *a.next_tiles_out = ntiles;
     }
@@ -1273,8 +1282,8 @@ int launch_resident_plan(SkinnyArgs a, const ResidentPlan &p, int ntiles, const 
         FLLM_REQUIRE(e == hipSuccess, "linear_skinny: cannot raise the LDS limit: %s", hipGetErrorString(e));
         attribute_set = true;
     }
-    hipLaunchKernelGGL((skinny_resident_kernel<PRO, EPI, TM, WAVES, XD, WT>), dim3(groups * p.S), dim3(WAVES * kWave), p.smem, stream,
-                       a, (int)p.stage);
+    hipLaunchKernelGGL((skinny_resident_kernel<PRO, EPI, TM, WAVES, XD, WT>), dim3(groups * p.S), dim3(WAVES * kWave),
+                       p.smem + (TM == TM_HALVES ? p.red : 0), stream, a, (int)p.stage);
     return fllm_check_launch("linear_skinny");
 }
 
@@ -1351,22 +1360,35 @@ int launch_resident(const SkinnyArgs &a, hipStream_t stream) {
         // tile and two tiles per slot, unevenly: 384 tiles on 512 slots run as long as 512 would.  Also when the 16-row
         // tiles fill no more than half of the compute units (narrow models): twice the workgroups, each with half the
         // weights (128 tiles of 2,048 x 8,192: 12.7 -> 9.4 us at one row; 192 tiles gain nothing, 7.7 -> 8.1 us, and at
-        // 256 tiles it is the other way round, 26.9 -> 32.3 us)
+        // 256 tiles it is the other way round, 26.9 -> 32.3 us).
         const int slots = device_cus() * p.per_cu;
         const bool uneven = 2 * tiles16 > slots && tiles16 < 2 * slots && tiles16 % slots != 0;
         const bool dual = a.M <= 8 && p.S == 1 && fllm_option_dual_k() && (uneven || 2 * tiles16 <= device_cus());
         const bool tiled = streams_tiles(a, p, a.N) && (x_direct || fllm_option_resident_tiles());
-        // q/k/v behind a prepared norm and the vocabulary projection: whole 16-row tiles where there is a copy, rather than
-        // 8-row tiles.  Reading the activations straight from global memory as the output projection does is slower for q/k/v
-        // (4,096 x 6,144 at 1, 8, 16 rows: 14.0, 15.4, 18.3 us against 12.4, 15.0, 18.1 staged).
-        constexpr bool kWhole = (EPI == EPI_QKV && PRO == PRO_SCALED) || (EPI == EPI_STORE_F32 && PRO == PRO_BF16);
+        // From a tile-major copy the uneven ones run whole tiles all the same: an 8-row tile takes 128 of each 256 bytes a load, a whole
+        // one 1 KiB in a row.  They add in the order of the 8-row tiles, so that whether there was memory for a copy changes no
+        // bit; that costs up to 0.3 us beside sums in a whole tile's own order (squared ReLU, 8-row tiles / these / own order at 1 and
+        // 8 rows: 13,312 x 1,536 10.7 / 9.3 / 9.1 and 15.2 / 11.8 / 10.5 us, 4,608 x 1,536 6.5 / 5.8 / 5.6 and 8.6 / 6.8 / 6.6, 6,144 x
+        // 1,024 5.6 / 5.1 / 4.8 and 6.7 / 5.5 / 5.2, 5,120 x 2,048 7.8 / 7.1 / 6.9 and 10.3 / 7.9 / 7.8).
+        // Sums into the stream keep 8-row tiles, whose count is that of the parts of the next norm's sums of squares.
+        constexpr bool kPlainSums = EPI != EPI_ADD;
+        const bool halves = kPlainSums && dual && uneven && tiled && p.waves == 8 && p.per_cu * (p.smem + p.red) <= fllm_plan::kLdsBytes;
+        // q/k/v behind a prepared norm and the vocabulary projection of widths in steps of 1,024: whole 16-row tiles in their own
+        // order where there is a copy, rather than 8-row tiles.  Reading the activations straight from global memory as the
+        // output projection does is slower for q/k/v (4,096 x 6,144 at 1, 8, 16 rows: 14.0, 15.4, 18.3 us against 12.4, 15.0, 18.1 staged).
+        const bool whole = ((EPI == EPI_QKV && PRO == PRO_SCALED) || (EPI == EPI_STORE_F32 && PRO == PRO_BF16)) && tiled && a.K % 1024 == 0;
         if constexpr (PRO == PRO_BF16) {
             if (x_direct) {
+                if constexpr (kPlainSums)
+                    if (halves) return launch_resident_plan<PRO, EPI, TM_HALVES, 8, true, true>(a, p, tiles16, ws, stream);
                 if (dual) return launch_resident_form<PRO, EPI, TM_DUALK, true>(a, p, tiles8, tiled, ws, stream);
                 return launch_resident_form<PRO, EPI, TM_ROWS16, true>(a, p, tiles16, tiled, ws, stream);
             }
         }
-        if (dual && !(kWhole && tiled)) return launch_resident_form<PRO, EPI, TM_DUALK, false>(a, p, tiles8, tiled, ws, stream);
+        if constexpr (kPlainSums) {
+            if (halves && !whole) return launch_resident_plan<PRO, EPI, TM_HALVES, 8, false, true>(a, p, tiles16, ws, stream);
+        }
+        if (dual && !whole) return launch_resident_form<PRO, EPI, TM_DUALK, false>(a, p, tiles8, tiled, ws, stream);
         return launch_resident_form<PRO, EPI, TM_ROWS16, false>(a, p, tiles16, tiled, ws, stream);
     }
 }

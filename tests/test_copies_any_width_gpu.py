@@ -68,6 +68,24 @@ def test_behind_a_norm(ops, M, N, K):
         assert torch.equal(a, b)
 
 
+# 16-row tiles from just beyond a tile for every other slot (of 512) to just short of two a slot; K whose halves are whole blocks of 128
+# columns and not, whose last waves have nothing, and beyond what leaves room for both halves' sums in LDS (3,968) or for eight waves (4,512)
+@pytest.mark.parametrize("M", [1, 8])
+@pytest.mark.parametrize("N,K", [(4112, 256), (6150, 288), (8176, 1024), (8208, 1056), (16360, 544), (4600, 3008), (4600, 3968), (6144, 4512)])
+def test_whole_tiles_of_a_copy_add_as_tiles_of_8_rows(ops, M, N, K):
+    x, w, nw = draw((M, K), M + K), draw((N, K), N + K, K ** -0.5), draw((K,), K, 0.1, torch.float32) + 1
+
+    def forms():
+        squared = torch.empty(M, N, dtype=BF16, device=DEV)
+        assert ops.linear_relu_squared(x, w, squared)
+        return (ops.linear(x, w, torch.empty(M, N, dtype=BF16, device=DEV)), squared,
+                ops.norm_linear(x.float(), nw, 1e-5, w, torch.empty(M, N, dtype=BF16, device=DEV)))
+
+    plain = forms()
+    assert ops.tile_for_decode(w)
+    assert all(torch.equal(a, b) for a, b in zip(plain, forms()))
+
+
 def test_what_is_read_beside_the_copy_stays_accepted(ops):
     """Rows that begin off 16 bytes have no 16-byte loads: they take the plain kernel, copy or not; a matrix that does gets no copy."""
     w = draw((64, 512), 1)

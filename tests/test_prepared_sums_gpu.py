@@ -59,3 +59,33 @@ def test_the_prepared_product_agrees_with_the_norm_in_the_product(ops):
         want = gate * torch.sigmoid(gate) * up
         errors = [(o.double().cpu() - want).abs().max().item() / want.abs().max().item() for o in outs]
         assert errors[1] <= 2 * errors[0] + 2.0 ** -9, errors        # the same roundings: one of the row, one of the result
+
+
+@pytest.mark.parametrize("rows", [1, 8, 9, 16])
+@pytest.mark.parametrize("heads, kv_heads, K", [(12, 2, 1536), (2, 1, 288), (40, 4, 1568)])
+def test_a_copy_changes_no_bit_of_the_rotated_product(ops, rows, heads, kv_heads, K):
+    """q, k and v behind a prepared norm of widths that are no multiple of 1,024, with the tile-major copy of their matrix and without:
+    matrices of few and of unevenly many tiles, whose rows run in tiles of 8."""
+    dim, pages = 128, 4
+    g = torch.Generator().manual_seed(K + rows)
+    w = (torch.randn((heads + 2 * kv_heads) * dim, K, generator=g) * K ** -0.5).to(torch.bfloat16).to(DEV)
+    x, branch = torch.randn(rows, K, generator=g).to(DEV), torch.randn(rows, K, generator=g).to(DEV)
+    gain = torch.ones(K, device=DEV)
+    prepared = ops.postnorm_add_prepare(x, branch, gain, 1e-5, gain)
+    pos = torch.arange(rows, dtype=torch.int32, device=DEV)
+    seg = torch.zeros(rows, dtype=torch.int32, device=DEV)
+    tables = torch.arange(pages, dtype=torch.int32, device=DEV)[None]
+    angles = torch.randn(64, dim // 2, generator=g).to(DEV)
+    cos, sin = angles.cos(), angles.sin()
+
+    def product():
+        q = torch.empty(rows, heads * dim, dtype=torch.bfloat16, device=DEV)
+        k = torch.zeros(pages, kv_heads, dim // 8, 16, 8, dtype=torch.bfloat16, device=DEV)
+        v = torch.zeros(pages, kv_heads, dim, 16, dtype=torch.bfloat16, device=DEV)
+        ops.norm_qkv_rope_store(None, None, 1e-5, w, q, pos, seg, tables, cos, sin, k, v, heads, kv_heads, dim, dim, 16, prepared=prepared)
+        return q, k, v
+
+    plain = product()
+    assert ops.tile_for_decode(w)
+    for a, b in zip(plain, product()):
+        assert torch.equal(a, b)
