@@ -299,7 +299,7 @@ class Ops:
         if not torch.cuda.is_available():
             raise KernelError("no GPU is visible: the engine runs on gfx950 only")
         self.lib = load_library()
-        # a thread's `copies_together`: .slab = [bytes still to come, memory of the copies being made, elements of it taken]
+        # a thread's `copies_together`: .piece = [bytes, memory of the copies being made, elements of it taken]
         self._copies = threading.local()
         self.library_gemm_from = library_gemm_from
         self.fused_decode_rows = int(fused_decode_rows)
@@ -321,28 +321,39 @@ class Ops:
     # ---- tile-major copies of weights for decode steps --------------------------------------------------
     _tiles: Dict[int, Tuple[tuple, torch.Tensor]] = {}     # address of a weight matrix -> (its shape, its tile-major copy)
 
-    _SLAB_BYTES = 256 << 20
-
     @contextlib.contextmanager
     def copies_together(self, nbytes: int):
-        """Copies made inside (about `nbytes` in all) lie in pieces of up to 256 MiB instead of an allocation each, which a model
-        pays for when it is built and again when it goes; a piece is given back with the last matrix whose copy lies in it."""
-        self._copies.slab = [int(nbytes), None, 0]
+        """Copies made inside (`nbytes` in all, `copy_bytes`) lie in one piece of memory instead of an allocation each, which a model
+        pays for when it is built and again when it goes; it is given back with the last matrix whose copy lies in it.  A copy that
+        does not fit into what is left of it has memory of its own."""
+        self._copies.piece = [int(nbytes), None, 0]
         try:
             yield
         finally:
-            self._copies.slab = None
+            self._copies.piece = None
 
     def _room_for_copy(self, elements: int, device) -> torch.Tensor:
-        slab = getattr(self._copies, "slab", None)
-        if slab is None or 2 * elements > Ops._SLAB_BYTES:
+        piece = getattr(self._copies, "piece", None)
+        if piece is not None and piece[1] is None and 2 * elements < piece[0]:
+            try:
+                piece[1] = torch.empty(piece[0] // 2, dtype=torch.bfloat16, device=device)
+            except torch.cuda.OutOfMemoryError:      # not in one piece: each for itself, as long as there is memory
+                self._copies.piece = piece = None
+        if piece is None or piece[1] is None or piece[1].device != device or piece[2] + elements > piece[1].numel():
             return torch.empty(elements, dtype=torch.bfloat16, device=device)
-        if slab[1] is None or slab[1].device != device or slab[2] + elements > slab[1].numel():
-            slab[1], slab[2] = torch.empty(max(elements, min(Ops._SLAB_BYTES, slab[0]) // 2), dtype=torch.bfloat16, device=device), 0
-        at = slab[2]
-        slab[0] = max(0, slab[0] - 2 * elements)
-        slab[2] = at + -(-elements // 128) * 128      # on 256 bytes
-        return slab[1][at:at + elements]
+        at = piece[2]
+        piece[2] = at + elements              # whole tiles of 16 x 32: every copy begins on 1,024 bytes
+        return piece[1][at:at + elements]
+
+    def tile_for_decode_supported(self, w: torch.Tensor, gate_up: bool = False) -> bool:
+        """Whether `tile_for_decode` can keep a copy of this matrix."""
+        return (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.data_ptr() % 16 == 0
+                and bool(self.lib.fllm_weight_tiles_supported(*w.shape)) and not (gate_up and w.shape[0] % 2 != 0))
+
+    def copy_bytes(self, w: torch.Tensor, gate_up: bool = False) -> int:
+        """Bytes of the copy that `tile_for_decode` or `tile_experts` keeps of this matrix or stack: its rows in whole tiles."""
+        rows, K = w.numel() // w.shape[-1], w.shape[-1]
+        return 2 * int(self.lib.fllm_weight_tiles_elements_gate_up(rows // 2, K) if gate_up else self.lib.fllm_weight_tiles_elements(rows, K))
 
     def tile_for_decode(self, w: torch.Tensor, gate_up: bool = False) -> bool:
         """Keeps beside `w` (bfloat16 [N, K] on the GPU) a copy in the order in which the products of decode steps read
@@ -351,25 +362,27 @@ class Ops:
         float32 logits and the forms behind a prepared norm for up to 64 (sums into a float32 `out` and `gate_up_swiglu`: up to 128).  `gate_up`: w is [gate; up] and the copy holds 8 gate rows and the
         same 8 up rows a tile (`fllm_tile_weights_gate_up`), for `norm_gate_up_swiglu` and `gate_up_swiglu`.  The copy is
         given up with `w`.  False: nothing was made (another type or place, a shape the kernels do not take tiles of)."""
-        if not (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous()):
+        if not self.tile_for_decode_supported(w, gate_up):
             return False
         N, K = w.shape
-        if not self.lib.fllm_weight_tiles_supported(N, K) or (gate_up and N % 2 != 0) or w.data_ptr() % 16 != 0:
-            return False
         key = w.data_ptr()
         kind = (N, K, bool(gate_up))
         if key in Ops._tiles and Ops._tiles[key][0] == kind:
             return True
         with torch.cuda.device(w.device):
+            tiles = self._room_for_copy(self.copy_bytes(w, gate_up) // 2, w.device)
             if gate_up:
-                tiles = self._room_for_copy(int(self.lib.fllm_weight_tiles_elements_gate_up(N // 2, K)), w.device)
                 self._check(self.lib.fllm_tile_weights_gate_up(_ptr(w), _ptr(tiles), N // 2, K, self._stream()))
             else:
-                tiles = self._room_for_copy(int(self.lib.fllm_weight_tiles_elements(N, K)), w.device)
                 self._check(self.lib.fllm_tile_weights(_ptr(w), _ptr(tiles), N, K, self._stream()))
         Ops._tiles[key] = (kind, tiles)
         weakref.finalize(w, Ops._tiles.pop, key, None)
         return True
+
+    @staticmethod
+    def forget_copy(w: torch.Tensor) -> None:
+        """Gives the copy of this matrix or stack up, if there is one."""
+        Ops._tiles.pop(w.data_ptr(), None)
 
     def _tiles_of(self, w: torch.Tensor, gate_up: bool = False, rows: int = 1) -> Optional[torch.Tensor]:
         """The copy of `w` that a product of `rows` rows may read, or None: up to 16 rows any, beyond them those whose widths the chunk

@@ -8,6 +8,7 @@ from typing import Any, Dict
 import torch
 
 EXPERTS = 3       # the priority of routed experts' copies, behind every other
+PIECE = 256 << 20     # bytes of copies that lie in one allocation at most (`Ops.copies_together`)
 
 
 class Runtime:
@@ -56,7 +57,8 @@ class Runtime:
         projections), 1 for the layers' other matrices, 2 for the vocabulary projection (once a step), 3 for routed
         experts (`tile_experts`)."""
         tile = getattr(self.ops, "tile_for_decode", None)
-        if tile is not None:
+        supported = getattr(self.ops, "tile_for_decode_supported", None)
+        if tile is not None and (supported is None or supported(w, gate_up)):
             self._ask_for_copy((w,), lambda: tile(w, gate_up=True) if gate_up else tile(w), priority)
 
     def tile_experts(self, *stacks: torch.Tensor) -> None:
@@ -64,13 +66,24 @@ class Runtime:
         them or none, since the kernel that reads the copies takes both products.  They come last (a step reads the
         picked experts of them only) and have a share of their own (`tiles_for_model`)."""
         tile, supported = getattr(self.ops, "tile_experts", None), getattr(self.ops, "tile_experts_supported", None)
-        if tile is not None and all(supported(w) for w in stacks):
-            self._ask_for_copy(stacks, lambda: all([tile(w) for w in stacks]), EXPERTS)
+        if tile is None or not all(supported(w) for w in stacks):
+            return
+
+        def make():
+            try:
+                return all([tile(w) for w in stacks])
+            except torch.cuda.OutOfMemoryError:
+                for w in stacks:
+                    self.ops.forget_copy(w)
+                raise
+
+        self._ask_for_copy(stacks, make, EXPERTS)
 
     def _ask_for_copy(self, matrices, make, priority: int) -> None:
         if not self.decode_weight_tiles or self.dtype != torch.bfloat16 or not all(w.is_cuda for w in matrices):
             return
-        size = sum(w.numel() * w.element_size() for w in matrices)
+        of = getattr(self.ops, "copy_bytes", None)
+        size = sum(of(w) if of is not None else w.numel() * w.element_size() for w in matrices)
         if self._tile_requests is not None:
             self._tile_requests.append((priority, len(self._tile_requests), size, make))
             return
@@ -89,28 +102,39 @@ class Runtime:
         of their priorities, and under "auto" within half of the memory that is free now (the other half is the
         cache's), routed experts within an eighth: their stacks are most of a large routed model, and every byte of a
         copy is one that the cache has no pages for.  A copy that does not fit is left out and smaller ones behind it
-        may still be made, so a model too large for all copies keeps those that every step reads.  Returns the bytes
-        copied."""
+        may still be made, so a model too large for all copies keeps those that every step reads; so is one for which
+        there turns out to be no memory.  Copies that follow each other share allocations of up to `PIECE` bytes, which are
+        exactly theirs.  Returns the bytes copied."""
         requests, self._tile_requests = sorted(self._tile_requests or [], key=lambda r: r[:2]), None
         if not requests:
             return 0
-        budget = experts_budget = None
-        if self.decode_weight_tiles == "auto":
+        auto = self.decode_weight_tiles == "auto"
+        if auto:
             torch.cuda.empty_cache()          # what placing the weights left in the allocator's hands counts as free
             free, _ = torch.cuda.mem_get_info(self.device)
             budget, experts_budget = free // 2, free // 8
-        made = 0
-        together = getattr(self.ops, "copies_together", None)
-        with together(sum(r[2] for r in requests)) if together is not None else contextlib.nullcontext():
-            for priority, _, size, make in requests:
-                if budget is not None and size > (min(budget, experts_budget) if priority == EXPERTS else budget):
+        runs, room = [], 0                    # requests that share an allocation, and what is left of the last one's PIECE
+        for priority, _, size, make in requests:
+            if auto:
+                if size > (min(budget, experts_budget) if priority == EXPERTS else budget):
                     continue
-                if make():
-                    made += size
-                    if budget is not None:
-                        budget -= size
-                        if priority == EXPERTS:
-                            experts_budget -= size
+                budget -= size
+                experts_budget -= size if priority == EXPERTS else 0
+            if not runs or size > room:
+                runs.append([])
+                room = PIECE
+            runs[-1].append((size, make))
+            room -= size
+        made = 0
+        together = getattr(self.ops, "copies_together", lambda nbytes: contextlib.nullcontext())
+        for run in runs:
+            with together(sum(size for size, _ in run)):
+                for size, make in run:
+                    try:
+                        made += size if make() else 0
+                    except torch.cuda.OutOfMemoryError:
+                        if not auto:
+                            raise
         return made
 
     def forget_host_tensors(self) -> None:

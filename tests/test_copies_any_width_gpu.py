@@ -114,3 +114,19 @@ def test_copies_of_a_model_share_their_memory(ops):
     assert len(Ops._tiles) == gone + 2 * len(ws) + 1
     del ws, wide, alone, w, other
     assert len(Ops._tiles) == gone
+
+
+def test_copies_of_a_model_take_no_more_memory_than_theirs(ops):
+    """Matrices of which the next does not fit behind the one before: what is allocated is what was made, and every byte is a copy's."""
+    from fllm_amd.parts.runtime import Runtime
+    rt = Runtime(torch.device(DEV), BF16, ops, 64, decode_weight_tiles=True)
+    ws = [torch.zeros(n, k, dtype=BF16, device=DEV) for n, k in ((6001, 4096), (4096, 28672), (1544, 256), (6144, 4096), (4096, 28640))]
+    rt.collect_tile_requests()
+    for w in ws + [torch.zeros(64, 1000, dtype=BF16, device=DEV)]:      # the last has no copy
+        rt.tile_for_decode(w)
+    before = torch.cuda.memory_allocated()
+    made = rt.tiles_for_model()
+    assert made == sum(ops.copy_bytes(w) for w in ws)
+    # torch's allocator hands out steps of 2 MiB from there on and keeps a remainder of up to 1 MiB with the block
+    assert made <= torch.cuda.memory_allocated() - before <= made + len(ws) * (2 << 20)
+    assert all(ops._tiles_of(w).numel() * 2 == ops.copy_bytes(w) for w in ws)

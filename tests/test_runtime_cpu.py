@@ -1,5 +1,7 @@
 """The copies of matrices that decode steps read (`Runtime.tile_for_decode`): asked for while a model is built, made
 when it is whole, the ones every step reads first, within half of the memory that is free then."""
+import contextlib
+
 import torch
 
 from fllm_amd.parts.runtime import Runtime
@@ -113,3 +115,82 @@ def test_experts_copies_come_last_in_pairs_and_within_an_eighth(monkeypatch):
     rt.tile_experts(Matrix("a", 3), Matrix("b", 3))
     rt.tile_experts(Matrix("c", 3), Matrix("d", 2))
     assert lib.made == ["c", "d"]
+
+
+class LibraryWithPieces(LibraryWithExperts):
+    """Counts the memory of copies: what is made inside `copies_together` lies in that piece as long as it has room."""
+
+    def __init__(self, free=None):
+        super().__init__()
+        self.pieces, self.allocated, self.left, self.free, self.held = [], 0, 0, free, set()
+
+    @contextlib.contextmanager
+    def copies_together(self, nbytes):
+        self.pieces.append(nbytes)
+        self.left = nbytes if self._allocate(nbytes) else 0
+        yield
+        self.left = 0
+
+    def _allocate(self, nbytes):
+        fits = self.free is None or self.allocated + nbytes <= self.free
+        self.allocated += nbytes if fits else 0
+        return fits
+
+    def _copy(self, w):
+        size = w.mib << 20
+        if size <= self.left:
+            self.left -= size
+        elif not self._allocate(size):
+            raise torch.cuda.OutOfMemoryError("no room")
+        self.held.add(w.name)
+        return True
+
+    def tile_for_decode(self, w, gate_up=False):
+        return self._copy(w)
+
+    def tile_experts(self, w):
+        return self._copy(w)
+
+    def forget_copy(self, w):
+        self.held.discard(w.name)
+
+
+def alternating(rt, layers=6):
+    """Matrices of 50 and 235 MiB in turn, the vocabulary's, and a few small ones."""
+    rt.collect_tile_requests()
+    for layer in range(layers):
+        rt.tile_for_decode(Matrix(f"qkv{layer}", 50), priority=1)
+        rt.tile_for_decode(Matrix(f"gate_up{layer}", 235), gate_up=True, priority=1)
+        rt.tile_for_decode(Matrix(f"o{layer}", 8))
+    rt.tile_for_decode(Matrix("vocabulary", 1002), priority=2)
+    return rt.tiles_for_model()
+
+
+def test_copies_take_the_memory_that_the_budget_counts(monkeypatch):
+    """Whatever the sizes and whatever is left out: the pieces hold what is made and nothing else, none beyond 256 MiB but for a single copy."""
+    for free_mib, want in ((1 << 20, 6 * 293 + 1002), (2 * 700, 48 + 50 + 235 + 50 + 235 + 50), (2 * 60, 48), (300, 48 + 50 + 50), (2 * 20, 16)):
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device=None: (free_mib << 20, 1 << 40))
+        lib = LibraryWithPieces()
+        made = alternating(Runtime(torch.device("cpu"), torch.bfloat16, lib, 128, decode_weight_tiles="auto"))
+        assert lib.allocated == sum(lib.pieces) == made == want << 20, (free_mib, lib.pieces)
+        assert made <= free_mib << 19
+        assert all(p <= 256 << 20 or p in (1002 << 20,) for p in lib.pieces)
+    assert len(lib.pieces) == 1                              # small ones share one
+    lib = LibraryWithPieces()
+    build_routed(Runtime(torch.device("cpu"), torch.bfloat16, lib, 128, decode_weight_tiles=True))
+    assert lib.allocated == (540 + 900) << 20
+
+
+def test_a_copy_without_memory_is_left_out(monkeypatch):
+    """More was said to be free than there is: under "auto" the model is built with the copies there was room for, a pair of experts' stacks
+    whole or not at all; where copies were asked for outright the error stands."""
+    import pytest
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device=None: (1 << 40, 1 << 40))
+    lib = LibraryWithPieces(free=500 << 20)
+    made = alternating(Runtime(torch.device("cpu"), torch.bfloat16, lib, 128, decode_weight_tiles="auto"))
+    assert 0 < made == sum(dict(o=8, qkv=50, gate_up=235)[n[:-1]] for n in lib.held) << 20 and lib.allocated <= lib.free
+    lib = LibraryWithPieces(free=(540 + 250) << 20)
+    build_routed(Runtime(torch.device("cpu"), torch.bfloat16, lib, 128, decode_weight_tiles="auto"))
+    assert not any(n.startswith(("up", "down")) for n in lib.held)
+    with pytest.raises(torch.cuda.OutOfMemoryError):
+        alternating(Runtime(torch.device("cpu"), torch.bfloat16, LibraryWithPieces(free=500 << 20), 128, decode_weight_tiles=True))
