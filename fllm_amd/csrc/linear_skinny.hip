@@ -519,7 +519,7 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
     // cursor of the products
     int item = 0, j = 0;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-    const bf16_t *xrow = xs + xrow_i * pitch;
+    const bf16_t *xrow = xs + xrow_i * pitch + kr0;
     FLLM_STAMP(a, 1);
 
     auto step = [&](Block &buf) {
@@ -528,7 +528,7 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (XD) xf[u] = buf.x[XD ? u : 0];
-            else xf[u] = (kb + u * 32 < ke && xvalid) ? *(const bf16x8_t *)(xrow + kb + u * 32) : zero8();
+            else xf[u] = (kb + u * 32 < ke && xvalid) ? *(const bf16x8_t *)(xrow + (kb - kr0) + u * 32) : zero8();
         }
 #pragma unroll
         for (int u = 0; u < U; u++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(buf.w[u], xf[u], acc, 0, 0, 0);
