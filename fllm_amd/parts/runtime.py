@@ -8,7 +8,7 @@ from typing import Any, Dict
 import torch
 
 EXPERTS = 3       # the priority of routed experts' copies, behind every other
-PIECE = 256 << 20     # bytes of copies that lie in one allocation at most (`Ops.copies_together`)
+PIECE = 1 << 30      # bytes of copies that lie in one allocation at most (`Ops.copies_together`): few (decode steps of the 1B sizes 1.433 ms, with 256 MiB 1.438)
 
 
 class Runtime:

@@ -4,7 +4,7 @@ import contextlib
 
 import torch
 
-from fllm_amd.parts.runtime import Runtime
+from fllm_amd.parts.runtime import PIECE, Runtime
 
 
 class Matrix:
@@ -167,14 +167,14 @@ def alternating(rt, layers=6):
 
 
 def test_copies_take_the_memory_that_the_budget_counts(monkeypatch):
-    """Whatever the sizes and whatever is left out: the pieces hold what is made and nothing else, none beyond 256 MiB but for a single copy."""
+    """Whatever the sizes and whatever is left out: the pieces hold what is made and nothing else, none beyond PIECE."""
     for free_mib, want in ((1 << 20, 6 * 293 + 1002), (2 * 700, 48 + 50 + 235 + 50 + 235 + 50), (2 * 60, 48), (300, 48 + 50 + 50), (2 * 20, 16)):
         monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device=None: (free_mib << 20, 1 << 40))
         lib = LibraryWithPieces()
         made = alternating(Runtime(torch.device("cpu"), torch.bfloat16, lib, 128, decode_weight_tiles="auto"))
         assert lib.allocated == sum(lib.pieces) == made == want << 20, (free_mib, lib.pieces)
         assert made <= free_mib << 19
-        assert all(p <= 256 << 20 or p in (1002 << 20,) for p in lib.pieces)
+        assert all(p <= PIECE for p in lib.pieces)
     assert len(lib.pieces) == 1                              # small ones share one
     lib = LibraryWithPieces()
     build_routed(Runtime(torch.device("cpu"), torch.bfloat16, lib, 128, decode_weight_tiles=True))
