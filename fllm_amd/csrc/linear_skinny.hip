@@ -1774,8 +1774,7 @@ extern "C" int fllm_linear_add_tiled(const void *x, int ldx, const void *w, cons
     a.N = N;
     a.K = K;
     const int rc = M <= 16 ? launch_resident<PRO_BF16, EPI_ADD>(a, stream) : dispatch_wide<EPI_ADD>(a, stream);
-    FLLM_REQUIRE(rc != 1, "linear_add_tiled: shape M=%d K=%d does not fit the staging area", M, K);
-    return rc;
+    return rc == 1 ? fllm_linear(x, ldx, w, bias, out, ldo, M, N, K, FLLM_BF16, 2, stream) : rc;      // a shape that does not fit
 }
 
 // out = x w^T (+ bias) for 1..64 bfloat16 rows and a float32 `out` (the vocabulary projection of a decode step), as
@@ -1801,8 +1800,7 @@ extern "C" int fllm_linear_f32_tiled(const void *x, int ldx, const void *w, cons
         return dispatch_wide<EPI_STORE_F32>(a, stream);
     }
     const int rc = fllm_linear_bf16_skinny(x, ldx, w, bias, out, ldo, M, N, K, 1, stream, w_tiles);
-    FLLM_REQUIRE(rc != 1, "linear_f32_tiled: shape M=%d K=%d does not fit the staging area", M, K);
-    return rc;
+    return rc == 1 ? fllm_linear(x, ldx, w, bias, out, ldo, M, N, K, FLLM_BF16, 1, stream) : rc;
 }
 
 // out = x w^T (+ bias) for 1..16 bfloat16 rows and a bfloat16 `out`, as fllm_linear in mode 0, likewise.

@@ -96,6 +96,27 @@ def test_what_is_read_beside_the_copy_stays_accepted(ops):
     assert not ops.tile_for_decode(draw((64 * 512 + 1,), 3)[1:].view(64, 512))
 
 
+@pytest.mark.parametrize("M,K", [(16, 4608), (14, 5376)])
+def test_a_shape_that_fits_no_plan_takes_the_general_kernel(ops, M, K):
+    """More row tiles than there are counters for K slices, and more activations than LDS holds in one: such a matrix is served with a copy
+    as it is without."""
+    N = 262208
+    w = (torch.randint(-8, 9, (N, K), device=DEV, dtype=torch.int8).to(BF16) * 2.0 ** -7)      # sums of whole multiples of 2^-14: exact
+    x = (torch.randint(-8, 9, (M, K), device=DEV).to(BF16) * 2.0 ** -7)
+    ends = torch.cat([torch.arange(3000), torch.arange(N - 3000, N)]).to(DEV)
+    want = x.double() @ w[ends].double().T
+
+    def forms():
+        return (ops.linear(x, w, torch.empty(M, N, device=DEV)), ops.linear(x, w, torch.zeros(M, N, device=DEV), accumulate=True),
+                ops.linear(x, w, torch.empty(M, N, dtype=BF16, device=DEV)))
+
+    plain = forms()
+    assert ops.tile_for_decode(w)
+    for a, b in zip(plain, forms()):
+        assert torch.equal(a, b)
+    assert torch.equal(plain[0][:, ends].double(), want) and torch.equal(plain[1][:, ends].double(), want)
+
+
 def test_copies_of_a_model_share_their_memory(ops):
     """Copies made together lie side by side, each on 256 bytes and whole, large ones in memory of their own; each goes with its matrix."""
     from fllm_amd.kernels import Ops
