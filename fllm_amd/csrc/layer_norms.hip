@@ -298,13 +298,14 @@ extern "C" int fllm_layernorm_conv(const float *x, const float *w1, float eps1, 
     return fllm_check_launch("layernorm_conv");
 }
 
-// 0: launched; negative: error; 1: declined (more than 32 rows, a width that is no multiple of 8)
+// 0: launched; negative: error; 1: declined (more than 32 rows, a width that is no multiple of 8; from 9 rows on, where a plain product would run
+// instead, also the plain kernels asked for)
 extern "C" int fllm_side_gate(const float *x, const void *w, const int32_t *ids, const void *table, int vocab, int table_width, int offset, void *out,
                               int rows, int width, int dim, int dtype, hipStream_t stream) {
     FLLM_REQUIRE(rows >= 0 && width > 0 && dim > 0 && vocab > 0 && offset >= 0 && offset + dim <= table_width, "side_gate: bad sizes");
     FLLM_REQUIRE(x && w && ids && table && out, "side_gate: operands missing");
     if (rows == 0) return 0;
-    if (rows > 32 || width % 8 != 0 || (((uintptr_t)x | (uintptr_t)w) & 15) != 0) return 1;
+    if (rows > (fllm_fast_kernels_enabled() ? 32 : 8) || width % 8 != 0 || (((uintptr_t)x | (uintptr_t)w) & 15) != 0) return 1;
 #define FLLM_SIDE(T, R)                                                                                                                      \
     hipLaunchKernelGGL((side_gate_kernel<T, R>), dim3(dim, (rows + R - 1) / R), dim3(kBlock), 0, stream, x, (const T *)w, ids, (const T *)table, vocab, table_width, \
                        offset, (T *)out, rows, width, dim)

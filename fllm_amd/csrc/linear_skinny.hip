@@ -1762,6 +1762,7 @@ extern "C" int fllm_linear_add_tiled(const void *x, int ldx, const void *w, cons
     FLLM_REQUIRE(M <= 64 || (w_tiles != nullptr && K % 256 == 0), "linear_add_tiled: beyond 64 rows it takes the tile-major copy and K in steps of 256 (M=%d K=%d)", M, K);
     FLLM_REQUIRE(aligned16(x) && aligned16(w) && out != nullptr && (w_tiles == nullptr || aligned16(w_tiles)),
                  "linear_add_tiled: operands must be there and 16-byte aligned");
+    if (!fllm_fast_kernels_enabled()) return fllm_linear(x, ldx, w, bias, out, ldo, M, N, K, FLLM_BF16, 2, stream);
     SkinnyArgs a = {};
     a.x = x;
     a.ldx = ldx;
@@ -1785,6 +1786,7 @@ extern "C" int fllm_linear_f32_tiled(const void *x, int ldx, const void *w, cons
                  "linear_f32_tiled: takes 1..64 rows, K and ldx in steps of 8 (M=%d N=%d K=%d ldx=%d ldo=%d)", M, N, K, ldx, ldo);
     FLLM_REQUIRE(aligned16(x) && aligned16(w) && out != nullptr && (w_tiles == nullptr || aligned16(w_tiles)),
                  "linear_f32_tiled: operands must be there and 16-byte aligned");
+    if (!fllm_fast_kernels_enabled()) return fllm_linear(x, ldx, w, bias, out, ldo, M, N, K, FLLM_BF16, 1, stream);
     if (M > 16) {
         SkinnyArgs a = {};
         a.x = x;
@@ -1810,6 +1812,7 @@ extern "C" int fllm_linear_store_tiled(const void *x, int ldx, const void *w, co
                  "linear_store_tiled: takes 1..16 rows, K and ldx in steps of 8 (M=%d N=%d K=%d ldx=%d ldo=%d)", M, N, K, ldx, ldo);
     FLLM_REQUIRE(aligned16(x) && aligned16(w) && out != nullptr && (w_tiles == nullptr || aligned16(w_tiles)),
                  "linear_store_tiled: operands must be there and 16-byte aligned");
+    if (!fllm_fast_kernels_enabled()) return fllm_linear(x, ldx, w, bias, out, ldo, M, N, K, FLLM_BF16, 0, stream);
     const int rc = fllm_linear_bf16_skinny(x, ldx, w, bias, out, ldo, M, N, K, 0, stream, w_tiles);
     return rc == 1 ? fllm_linear(x, ldx, w, bias, out, ldo, M, N, K, FLLM_BF16, 0, stream) : rc;
 }

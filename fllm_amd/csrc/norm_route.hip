@@ -133,7 +133,8 @@ void launch(float *x, const float *branch, const float *gain, float eps, int nor
 
 }  // namespace
 
-// 0: launched; negative: error; 1: declined (a width that is no multiple of 512 or beyond 4,096, more than 64 experts or rows), nothing was written
+// 0: launched; negative: error; 1: declined (a width that is no multiple of 512 or beyond 4,096, more than 64 experts or rows, the plain kernels
+// asked for), nothing was written
 extern "C" int fllm_norm_route(float *x, const float *branch, const float *gain, float eps, int normalize, const float *norm_w, float norm_eps,
                                void *out, int rows, int width, const void *w_router, const float *correction, int experts, int top, int groups,
                                int kept, int score_mode, int renormalize, float route_scale, int32_t *ids, float *weights, hipStream_t stream) {
@@ -145,7 +146,7 @@ extern "C" int fllm_norm_route(float *x, const float *branch, const float *gain,
         FLLM_REQUIRE(groups > 0 && experts % groups == 0 && kept > 0 && kept <= groups && top <= kept * (experts / groups),
                      "norm_route: %d experts in %d groups, %d kept, %d picked", experts, groups, kept, top);
     if (rows == 0) return 0;
-    if (width % kStep != 0 || width > 16 * kBlock || experts > kMostExperts || rows > 64) return 1;
+    if (!fllm_fast_kernels_enabled() || width % kStep != 0 || width > 16 * kBlock || experts > kMostExperts || rows > 64) return 1;
     if (((uintptr_t)x | (uintptr_t)branch | (uintptr_t)gain | (uintptr_t)norm_w | (uintptr_t)out | (uintptr_t)w_router) & 15) return 1;
     const RouteArgs p = {(const bf16_t *)w_router, correction, experts, top, groups, kept, score_mode, renormalize, route_scale, ids, weights};
     if (branch != nullptr && correction != nullptr) launch<true, true>(x, branch, gain, eps, normalize, norm_w, norm_eps, out, rows, width, p, stream);

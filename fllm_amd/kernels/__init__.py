@@ -408,7 +408,8 @@ class Ops:
                 and self._tiles_of(w_gate_up, gate_up=True, rows=rows) is not None and self._tiles_of(w_down, rows=rows) is not None)
 
     def set_fast_kernels(self, on: bool) -> None:
-        """Off: bfloat16 calls run the plain kernels (tests compare the two)."""
+        """Off: bfloat16 calls run the plain kernels, products also where there is a tile-major copy (tests and the layer check compare the
+        two); only the forms that fold a norm, a rotation or an activation into a product have no plain kernel."""
         self.lib.fllm_set_fast_kernels(1 if on else 0)
 
     def set_option(self, name: str, value: int) -> None:
@@ -1060,7 +1061,7 @@ class Ops:
         """One kernel for a step of up to 64 rows: with `branch` first x[r] += branch[r] * rsqrt(mean(branch[r]^2) + eps) * gain (eps None:
         branch[r] * gain), then out = rmsnorm(x) in bfloat16 and the router of out's rows, with `correction` (and groups) as
         `route_grouped`, without as `route_topk`.  False: not taken (float32, a width that is no multiple of 512 or beyond 4,096, more
-        than 64 experts or rows), nothing was written."""
+        than 64 experts or rows, the plain kernels asked for), nothing was written."""
         rows, width = x.shape
         E = w_router.shape[0]
         if out.dtype != torch.bfloat16 or w_router.dtype != torch.bfloat16 or rows > 64:
@@ -1856,7 +1857,7 @@ class Ops:
         return x.shape[0] <= 8 and self.side_gate_rows(x, w, ids, table, offset, out)
 
     def side_gate_rows(self, x: torch.Tensor, w: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, offset: int, out: torch.Tensor) -> bool:
-        """`side_gate` for up to 32 rows, eight a workgroup."""
+        """`side_gate` for up to 32 rows, eight a workgroup (with the plain kernels asked for up to 8)."""
         rows, width = x.shape
         dim = w.shape[0]
         _dense(x, "x", torch.float32)

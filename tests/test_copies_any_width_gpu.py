@@ -117,6 +117,28 @@ def test_a_shape_that_fits_no_plan_takes_the_general_kernel(ops, M, K):
     assert torch.equal(plain[0][:, ends].double(), want) and torch.equal(plain[1][:, ends].double(), want)
 
 
+@pytest.mark.parametrize("M", [1, 8, 16, 40, 100])
+@pytest.mark.parametrize("N,K", [(1000, 544), (1536, 1536), (6150, 1024)])
+def test_plain_kernels_read_no_copy(M, N, K):
+    """With the matrix-core kernels switched off a matrix with a copy gives the bits of one without: a chain of float32 sums a result."""
+    from fllm_amd.kernels import Ops
+    ops = Ops(library_gemm_from=None)
+    x, w, start = draw((M, K), M + K), draw((N, K), N + K, K ** -0.5), draw((M, N), 5, 1.0, torch.float32)
+
+    def forms():
+        return (ops.linear(x, w, torch.empty(M, N, dtype=BF16, device=DEV)), ops.linear(x, w, torch.empty(M, N, device=DEV)),
+                ops.linear(x, w, start.clone(), accumulate=True))
+
+    ops.set_fast_kernels(False)
+    try:
+        plain = forms()
+        assert ops.tile_for_decode(w)
+        with_copy = forms()
+    finally:
+        ops.set_fast_kernels(True)
+    assert all(torch.equal(a, b) for a, b in zip(plain, with_copy))
+
+
 def test_copies_of_a_model_share_their_memory(ops):
     """Copies made together lie side by side, each on 256 bytes and whole, large ones in memory of their own; each goes with its matrix."""
     from fllm_amd.kernels import Ops

@@ -47,3 +47,16 @@ def test_side_gate_of_more_rows(ops, rows, dtype):
     assert torch.equal(got, alone)
     assert not ops.side_gate_rows(torch.zeros(33, width, device=DEV), w, torch.zeros(33, dtype=torch.int32, device=DEV), table, 0,
                                   torch.empty(33, dim, dtype=dtype, device=DEV))
+
+
+def test_side_gate_of_more_rows_is_left_to_the_plain_product_where_that_is_asked_for(ops):
+    x, w = torch.zeros(9, 64, device=DEV), torch.zeros(8, 64, dtype=torch.bfloat16, device=DEV)
+    ids, table = torch.zeros(9, dtype=torch.int32, device=DEV), torch.zeros(4, 8, dtype=torch.bfloat16, device=DEV)
+    out = torch.empty(9, 8, dtype=torch.bfloat16, device=DEV)
+    ops.set_fast_kernels(False)
+    try:
+        assert not ops.side_gate_rows(x, w, ids, table, 0, out)
+        assert ops.side_gate(x[:8], w, ids[:8], table, 0, out[:8])
+    finally:
+        ops.set_fast_kernels(True)
+    assert ops.side_gate_rows(x, w, ids, table, 0, out)

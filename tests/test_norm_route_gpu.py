@@ -71,3 +71,15 @@ def test_what_it_leaves_to_the_others(ops):
         ids, weights = torch.full((rows, 2), -7, dtype=torch.int32, device=DEV), torch.empty(rows, 2, device=DEV)
         assert not ops.norm_route(x, norm_w, 1e-6, h, w.to(dtype), 2, ids, weights, branch=branch, gain=gain, eps=1e-5)
         assert torch.equal(x, before) and bool((h == 3.0).all()) and bool((ids == -7).all())
+
+
+def test_left_to_the_others_where_plain_kernels_are_asked_for(ops):
+    x, _, _, norm_w, w, _ = operands(2, 512, 4, 3)
+    before, h = x.clone(), torch.zeros(2, 512, dtype=BF16, device=DEV)
+    ids, weights = torch.zeros(2, 1, dtype=torch.int32, device=DEV), torch.zeros(2, 1, device=DEV)
+    ops.set_fast_kernels(False)
+    try:
+        assert not ops.norm_route(x, norm_w, 1e-6, h, w, 1, ids, weights)
+    finally:
+        ops.set_fast_kernels(True)
+    assert torch.equal(x, before) and not h.any() and not weights.any()
