@@ -1551,7 +1551,8 @@ int fllm_linear_bf16_skinny(const void *x, int ldx, const void *w, const float *
 
 extern "C" int fllm_linear_relu_squared(const void *x, int ldx, const void *w, const void *w_tiles, void *out, int M, int N, int K,
                                         hipStream_t stream) {
-    FLLM_REQUIRE(M >= 1 && M <= 64 && N > 0 && K > 0 && K % 8 == 0 && ldx >= K && ldx % 8 == 0 && aligned16(x) && aligned16(w),
+    FLLM_REQUIRE(M >= 1 && M <= 64 && N > 0 && K > 0 && K % 8 == 0 && ldx >= K && ldx % 8 == 0 && aligned16(x) && aligned16(w) &&
+                     aligned16(w_tiles),
                  "linear_relu_squared: takes 1..64 rows on 16-byte boundaries and K a multiple of 8 (M=%d N=%d K=%d)", M, N, K);
     SkinnyArgs a = {};
     a.x = x;
@@ -1577,7 +1578,7 @@ extern "C" int fllm_fused_decode_supported(int M, int K) {
 extern "C" int fllm_norm_linear(const float *x, const float *norm_w, float eps, const void *w, const void *w_tiles, const float *bias,
                                 void *out, int M, int N, int K, hipStream_t stream) {
     FLLM_REQUIRE(fllm_fused_decode_supported(M, K), "norm_linear: takes 1..64 rows and K a multiple of 8 (M=%d K=%d)", M, K);
-    FLLM_REQUIRE(aligned16(x) && aligned16(w) && aligned16(norm_w), "norm_linear: operands must be 16-byte aligned");
+    FLLM_REQUIRE(aligned16(x) && aligned16(w) && aligned16(w_tiles) && aligned16(norm_w), "norm_linear: operands must be 16-byte aligned");
     FLLM_REQUIRE(eps > 0.f, "norm_linear: eps must be positive");
     SkinnyArgs a = {};
     a.x = x;
@@ -1600,7 +1601,8 @@ extern "C" int fllm_norm_linear(const float *x, const float *norm_w, float eps, 
 extern "C" int fllm_norm_gate_up_swiglu(const float *x, const float *norm_w, float eps, const void *w_gate_up, const void *w_tiles,
                                         const float *bias, void *out, int M, int inter, int K, hipStream_t stream) {
     FLLM_REQUIRE(fllm_fused_decode_supported(M, K), "norm_gate_up_swiglu: takes 1..64 rows and K a multiple of 8 (M=%d K=%d)", M, K);
-    FLLM_REQUIRE(aligned16(x) && aligned16(w_gate_up) && aligned16(norm_w), "norm_gate_up_swiglu: operands must be 16-byte aligned");
+    FLLM_REQUIRE(aligned16(x) && aligned16(w_gate_up) && aligned16(w_tiles) && aligned16(norm_w),
+                 "norm_gate_up_swiglu: operands must be 16-byte aligned");
     FLLM_REQUIRE(eps > 0.f && inter > 0, "norm_gate_up_swiglu: bad eps or size");
     SkinnyArgs a = {};
     a.act_alpha = 1.0f;      // silu(gate) * up
@@ -1683,7 +1685,8 @@ extern "C" int fllm_norm_qkv_rope_store(const float *x, const float *norm_w, flo
                                         void *k_pages, void *v_pages, int M, int heads, int kv_heads, int head_dim, int K,
                                         int page_size, int store_kv, hipStream_t stream) {
     FLLM_REQUIRE(fllm_fused_decode_supported(M, K), "norm_qkv_rope_store: takes 1..64 rows and K a multiple of 8 (M=%d K=%d)", M, K);
-    FLLM_REQUIRE(aligned16(x) && aligned16(w_qkv) && aligned16(norm_w), "norm_qkv_rope_store: operands must be 16-byte aligned");
+    FLLM_REQUIRE(aligned16(x) && aligned16(w_qkv) && aligned16(w_tiles) && aligned16(norm_w),
+                 "norm_qkv_rope_store: operands must be 16-byte aligned");
     FLLM_REQUIRE(head_dim % 8 == 0 && rope_dims % 2 == 0 && rope_dims <= head_dim && rope_dims >= 0,
                  "norm_qkv_rope_store: head_dim %d must be a multiple of 8 and rope_dims %d even and no larger", head_dim, rope_dims);
     FLLM_REQUIRE(heads > 0 && kv_heads > 0 && page_size > 0 && table_stride > 0 && eps > 0.f, "norm_qkv_rope_store: bad sizes");
@@ -1908,11 +1911,13 @@ extern "C" int fllm_scaled_qkv_rope_store(const void *xn, const float *ssq, int 
 // The gated products with the activation's constants as arguments: out = a(g') * (u' + offset), a(g) = g * sigmoid(alpha g),
 // g' = min(x gate^T, limit), u' = clamp(x up^T, -limit, limit) (limit <= 0: nothing is clamped); w = [gate; up] ([2 I, K]).
 // fllm_norm_gate_up_glu: x is float32 [M, K] and the RMSNorm with `norm_w` is folded in (1..64 rows).
-// fllm_gate_up_glu: x is bfloat16; 1..64 rows, or 17..128 with the tile-major copy `w_tiles` (null: without).
+// fllm_gate_up_glu: x is bfloat16; 1..64 rows, or to 128 with `w_tiles`.  Both stream the tile-major copy `w_tiles` (null: without) in
+// steps of up to 16 rows, fllm_gate_up_glu from 17 rows on too.
 extern "C" int fllm_norm_gate_up_glu(const float *x, const float *norm_w, float eps, const void *w_gate_up, const void *w_tiles,
                                      const float *bias, void *out, int M, int inter, int K, float limit, float alpha, float offset, hipStream_t stream) {
     FLLM_REQUIRE(fllm_fused_decode_supported(M, K), "norm_gate_up_glu: takes 1..64 rows and K a multiple of 8 (M=%d K=%d)", M, K);
-    FLLM_REQUIRE(aligned16(x) && aligned16(w_gate_up) && aligned16(norm_w), "norm_gate_up_glu: operands must be 16-byte aligned");
+    FLLM_REQUIRE(aligned16(x) && aligned16(w_gate_up) && aligned16(w_tiles) && aligned16(norm_w),
+                 "norm_gate_up_glu: operands must be 16-byte aligned");
     FLLM_REQUIRE(eps > 0.f && inter > 0, "norm_gate_up_glu: bad eps or size");
     SkinnyArgs a = {};
     a.act_limit = limit;

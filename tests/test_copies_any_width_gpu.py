@@ -96,6 +96,30 @@ def test_what_is_read_beside_the_copy_stays_accepted(ops):
     assert not ops.tile_for_decode(draw((64 * 512 + 1,), 3)[1:].view(64, 512))
 
 
+def test_copies_that_begin_off_16_bytes_are_refused(ops):
+    """A lane's load of a copy is 16 bytes: every entry point that takes one says so before it launches anything."""
+    M, K, heads, dim = 4, 512, 2, 64
+    p = lambda t: t.data_ptr()
+    x, xb, nw = torch.zeros(M, K, device=DEV), torch.zeros(M, K, dtype=BF16, device=DEV), torch.ones(K, device=DEV)
+    w, out = torch.zeros(3 * heads * dim, K, dtype=BF16, device=DEV), torch.zeros(M, 3 * heads * dim, device=DEV)
+    rows, table = torch.zeros(M, dtype=torch.int32, device=DEV), torch.zeros(1, dtype=torch.float32, device=DEV)
+    copy = torch.zeros(w.numel() + 8, dtype=BF16, device=DEV)
+    tiles = p(copy) + 8
+    N, lib, stream = w.shape[0], ops.lib, ops._stream()
+    calls = {
+        "norm_linear": lambda: lib.fllm_norm_linear(p(x), p(nw), 1e-5, p(w), tiles, None, p(out), M, N, K, stream),
+        "norm_gate_up_swiglu": lambda: lib.fllm_norm_gate_up_swiglu(p(x), p(nw), 1e-5, p(w), tiles, None, p(out), M, N // 2, K, stream),
+        "norm_gate_up_glu": lambda: lib.fllm_norm_gate_up_glu(p(x), p(nw), 1e-5, p(w), tiles, None, p(out), M, N // 2, K, 7.0, 1.7, 1.0, stream),
+        "gate_up_glu": lambda: lib.fllm_gate_up_glu(p(xb), K, p(w), tiles, None, p(out), M, N // 2, K, 7.0, 1.7, 1.0, stream),
+        "linear_relu_squared": lambda: lib.fllm_linear_relu_squared(p(xb), K, p(w), tiles, p(out), M, N, K, stream),
+        "norm_qkv_rope_store": lambda: lib.fllm_norm_qkv_rope_store(p(x), p(nw), 1e-5, p(w), tiles, None, p(out), p(rows), p(rows), p(rows), 1, p(table),
+                                                                    p(table), 0, None, None, M, heads, heads, dim, K, 16, 0, stream),
+    }
+    for name, call in calls.items():
+        assert call() == -1, name
+        assert b"aligned" in lib.fllm_last_error() or b"boundaries" in lib.fllm_last_error(), name
+
+
 @pytest.mark.parametrize("M,K", [(16, 4608), (14, 5376)])
 def test_a_shape_that_fits_no_plan_takes_the_general_kernel(ops, M, K):
     """More row tiles than there are counters for K slices, and more activations than LDS holds in one: such a matrix is served with a copy
