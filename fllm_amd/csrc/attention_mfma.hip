@@ -989,9 +989,10 @@ int launch_tile32(const AttnArgs &a, int max_context, hipStream_t stream) {
     void *dev_ws = nullptr;
     size_t dev_ws_bytes = 0;
     if (fllm_option_prefill_parts() && fllm_device_workspace(&dev_ws, &dev_ws_bytes) && dev_ws_bytes > kWorkspaceCounterBytes) {
-        p.part_tiles = prefill_part_plan(tiles, a.kv_heads, a.rows, max_context, a.window,
-                                         (dev_ws_bytes - kWorkspaceCounterBytes) / (kPartFloats(D, WAVES * kWave) * sizeof(float)),
-                                         device_slots() * 4 / WAVES, &max_parts);
+        const int slots = device_slots() * 4 / WAVES;
+        p.part_tiles = prefill_part_plan(tiles, a.kv_heads, fllm_plan::rows_of_one_prompt(tiles, a.rows, a.num_segs, a.kv_heads, max_context, slots),
+                                         max_context, a.window,
+                                         (dev_ws_bytes - kWorkspaceCounterBytes) / (kPartFloats(D, WAVES * kWave) * sizeof(float)), slots, &max_parts);
         p.counters = (int *)dev_ws;
         p.parts_ws = (float *)((unsigned char *)dev_ws + kWorkspaceCounterBytes);
     }

@@ -276,14 +276,29 @@ inline bool decode_counters_fit(int rows, int kv_heads, int qtiles) { return (si
 // ---- prompt attention: the key tiles of a row tile shared among workgroups ----
 // what a part of a row tile leaves behind, in floats: every thread of the workgroup its outputs (head_dim / 2), a maximum and a sum
 constexpr size_t part_floats(int head_dim, int threads = 256) { return (size_t)threads * (head_dim / 2 + 2); }
+// The rows of a step as the plan below counts them against its longest context: all of them where they are mostly one prompt's, 0 where
+// others keep the slots busy while the long row tiles run, which are then better whole (shared, their second halves wait behind
+// all other row tiles).  All segments but one may be single rows.  Others are enough
+//   - with a third of the longest prompt's rows, or where there are several a quarter (32 heads on 8 of 128 lanes, us shared / whole: 1,900
+//     and 100 rows 67.9 / 72.5, 1,500 and 500 54.0 / 57.3, 1,450 and 550 59.1 / 55.6, 1,300 and 700 56.5 / 50.9, 500, 650 and 800
+//     42.6 / 39.1, 1,200, 200, 100 and 50 45.4 / 40.1; of 64 lanes 44.2 / 45.4, 35.0 / 36.8, 38.4 / 35.6, 36.6 / 32.6, 27.9 / 25.1, 30.1 / 26.0);
+//   - being single rows, where they take half of the slots and the prompt's row tiles fill the other half by themselves (1,900 rows and
+//     40 / 64 / 100 single ones 85.7 / 74.2, 89.0 / 76.1 and 104 / 87.6; 12 heads on 2, whose row tiles do not, 50.1 / 61.1, 48.2 /
+//     52.4 and 46.8 / 53.2).
+inline int rows_of_one_prompt(int tiles, int rows, int num_segs, int kv_heads, int max_context, int slots) {
+    const long others = num_segs - 1;
+    const bool prompts = (num_segs > 2 ? 4 : 3) * (rows - others - max_context) > max_context;
+    const bool singles = 2 * others * kv_heads > slots && 2 * (tiles - others) * kv_heads >= slots;
+    return prompts || singles ? 0 : rows;
+}
 // The most key tiles one workgroup takes (0: row tiles are not shared) and the most parts a row tile can have.  Row
 // tiles are shared when, one workgroup each, they would leave workgroup slots of the device empty: a part then has
 // about the key tiles that a slot sees in all when every slot is taken, and at least 8, since every part pays for
 // leaving its results and the last one for adding them up.  A step whose rows are as many as its longest context (a
 // prompt from its first token on) has row tiles of every length up to the longest, half of it on average: up to 2,048
 // tokens the long ones are shared in halves (8 to 16 key tiles a part), or the slots of the short ones would idle
-// through the second half of the launch (longer prompts have row tiles enough to keep every slot busy, and so have several
-// prompts in one step: heads of 64, three of 500 to 800 tokens 28.8 us shared and 24.9 whole, seven of 33 to 701 28.7 and 22.9).  `room`: parts that the workspace holds; `by_hand`: key tiles a part when set by hand (> 1).
+// through the second half of the launch (longer prompts have row tiles enough to keep every slot busy).  `rows`: see
+// rows_of_one_prompt.  `room`: parts that the workspace holds; `by_hand`: key tiles a part when set by hand (> 1).
 inline int prefill_part_plan(int tiles, int kv_heads, int rows, int max_context, int window, size_t room, int slots, int by_hand,
                              int *max_parts) {
     *max_parts = 1;
@@ -293,7 +308,7 @@ inline int prefill_part_plan(int tiles, int kv_heads, int rows, int max_context,
     const long most_tiles = ((long)max_context + 63) / 64;        // key tiles of the longest context
     const long per_slot = (groups * most_tiles + slots - 1) / slots;
     long per_part = per_slot > 8 ? per_slot : 8;
-    if (rows + 63 >= max_context && rows <= max_context + 63 && most_tiles <= 32) {       // contexts of every length; measured a gain up to 2,048 tokens only
+    if (rows + 63 >= max_context && most_tiles <= 32) {       // contexts of every length; measured a gain up to 2,048 tokens only
         long half = most_tiles / 2;
         half = half < 8 ? 8 : (half > 16 ? 16 : half);
         if (half < per_part) per_part = half;

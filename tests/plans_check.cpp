@@ -220,6 +220,23 @@ int main() {
                                         "parts %d of %d key tiles for %ld", max_parts, per_part, most_tiles);
                                 REQUIRE((size_t)groups * max_parts <= room, "parts %ld x %d in room %zu", groups, max_parts, room);
                             }
+    // which steps are one prompt's: heads 32 on 8 (row tiles of 32 rows) and 12 on 2 (of 21), 512 slots
+    struct { int longest, more, singles, group, kv_heads; bool one; } steps[] = {
+        {1900, 0, 0, 4, 8, true},     {1900, 40, 0, 4, 8, true},    {1900, 0, 4, 4, 8, true},      {1500, 500, 0, 4, 8, true},
+        {1450, 550, 0, 4, 8, false},  {1024, 1024, 0, 4, 8, false}, {1900, 0, 32, 4, 8, true},     {1900, 0, 40, 4, 8, false},
+        {1900, 0, 100, 4, 8, false},  {1900, 0, 64, 6, 2, true},    {1900, 0, 160, 6, 2, true},    {300, 0, 100, 4, 8, true},
+        {131072, 0, 0, 4, 8, true},   {1 << 30, 1 << 30, 0, 4, 8, false}};
+    for (const auto &t : steps) {
+        const int segs = 1 + (t.more > 0) + t.singles, rows = (int)((unsigned)t.longest + t.more - (t.more == 1 << 30 ? 1 : 0)) + t.singles;
+        const int tiles = rows / (128 / t.group) + 1 + segs;
+        const int got = rows_of_one_prompt(tiles, rows, segs, t.kv_heads, t.longest, 512);
+        REQUIRE(got == (t.one ? rows : 0), "%d + %d rows and %d single ones: %d", t.longest, t.more, t.singles, got);
+        // a step that is not one prompt's is planned by its slots alone
+        int parts = 0, plain = 0;
+        const int a = prefill_part_plan(tiles, t.kv_heads, got, t.longest, 0, (size_t)1 << 20, 512, 0, &parts);
+        const int b = prefill_part_plan(tiles, t.kv_heads, t.one ? rows : 1, t.longest, 0, (size_t)1 << 20, 512, 0, &plain);
+        REQUIRE(a == b && parts == plain, "parts of %d + %d rows and %d single ones", t.longest, t.more, t.singles);
+    }
     printf("plans ok: %ld checks\n", checks);
     return 0;
 }
