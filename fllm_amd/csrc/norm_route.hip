@@ -1,9 +1,16 @@
 // A decode step's row on its way into routed experts in one kernel: a branch behind a norm joins the stream (or none does), the norm before
 // the experts, and the router: what postnorm_add (stream_ops.hip) and the routers (routed_experts.hip) do one after the other.
 //
-// One workgroup a row.  What bounds it is its launch and two trips to memory, where the two kernels paid both twice (4.2 and 5.5 us at
-// 2 rows of 1,536 lanes; prompts and answers of models with 12, 6 and 4 such layers a step 14.10 -> 13.87, 11.57 -> 11.42, 8.44 -> 8.31 ms): the row, its branch, the vectors and the first rows of the router are asked for together, the normed row
-// stays in LDS for the router's products, whose sums are added in the order row_score adds them.
+// One workgroup a row.  What bounds it is its launch and its trips to memory, where the two kernels pay both twice: the row, its
+// branch, the vectors and a wave's first two experts are asked for together, and the normed row stays in LDS for the
+// router's products.  A wave has its SIMD to itself, so it takes two experts at a time (two chains of sums) and asks for the next two
+// before; a chain is added in the order of row_score.  With one expert at a time, asked for when the one before was done, it was slower than
+// the two kernels from 24 experts on.  Microseconds in a graph behind a branch, this and the two kernels, sigmoid scores, at 1 and 64 rows:
+//   8 experts of 1,536 lanes   5.1 / 6.4,   5.5 / 7.1       64 experts of 512     9.6 / 10.0, 10.1 / 10.8
+//   8 of 4,096                 6.7 / 8.2,   7.1 / 9.0       64 of 2,048          12.2 / 14.5, 12.7 / 15.4 (one at a time 18.7, 18.9)
+//   32 of 1,024                7.2 / 8.4,   7.8 / 9.1       64 of 4,096          16.7 / 21.0, 17.8 / 22.2
+// Prompts and answers of models with 12, 6 and 4 such layers a step, 8 experts of 1,536 lanes: 14.10 -> 13.87, 11.57 -> 11.42, 8.44 -> 8.31 ms with
+// one expert at a time.
 #include "api.h"
 #include "common.h"
 #include "router_picks.h"
@@ -49,10 +56,17 @@ norm_route_kernel(float *__restrict__ x, const float *__restrict__ branch, const
         s[i] = *(const f32x4_t *)(x + r * width + c);
         w2[i] = *(const f32x4_t *)(norm_w + c);
     }
-    bf16x8_t b[AHEAD];                                  // this wave's first expert's row of the router
-    const int first = min(wave, p.experts - 1);
+    // this wave's experts' rows of the router, two at work at a time, up to 2,048 lanes the next two on their way
+    constexpr bool DEEP = NV <= 2;
+    bf16x8_t b[2][AHEAD], ahead[2][DEEP ? AHEAD : 1];
+    auto ask = [&](auto &to, int e0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < AHEAD; j++) b[j] = *(const bf16x8_t *)(p.w + (size_t)first * width + min(j, pieces - 1) * kStep + lane * 8);
+        for (int k = 0; k < 2; k++)
+#pragma unroll
+            for (int j = 0; j < AHEAD; j++)
+                to[k][j] = *(const bf16x8_t *)(p.w + (size_t)min(e0 + k * kWaves, p.experts - 1) * width + lane * 8 + min(j, pieces - 1) * kStep);
+    };
+    ask(b, wave);
     auto mine = [&](int i) { return (i * kBlock + (int)threadIdx.x) * 4 < width; };
     if (BRANCH) {
         float inv = 1.0f;
@@ -91,25 +105,39 @@ norm_route_kernel(float *__restrict__ x, const float *__restrict__ branch, const
         *(bf16x4_t *)(row + c) = h;
     }
     __syncthreads();
-    for (int e = wave; e < p.experts; e += kWaves) {
-        const float c = GROUPED ? p.correction[e] : 0.f;
-        if (e != wave) {
+    for (int e0 = wave; e0 < p.experts; e0 += 2 * kWaves) {
+        float c[2] = {0.f, 0.f}, z[2] = {0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < AHEAD; j++) b[j] = *(const bf16x8_t *)(p.w + (size_t)e * width + min(j, pieces - 1) * kStep + lane * 8);
-        }
-        float z = 0.f;
+        for (int k = 0; k < 2; k++)
+            if (GROUPED) c[k] = p.correction[min(e0 + k * kWaves, p.experts - 1)];
+        if constexpr (DEEP) ask(ahead, e0 + 2 * kWaves);
 #pragma unroll
         for (int j = 0; j < AHEAD; j++) {
             if (j >= pieces) break;
             const bf16x8_t a = *(const bf16x8_t *)(row + j * kStep + lane * 8);
 #pragma unroll
-            for (int k = 0; k < 8; k++) z = fmaf((float)a[k], (float)b[j][k], z);
+            for (int i = 0; i < 8; i++)
+#pragma unroll
+                for (int k = 0; k < 2; k++) z[k] = fmaf((float)a[i], (float)b[k][j][i], z[k]);
         }
-        z = wave_sum(z);
-        if (lane == 0) {
-            const float sigmoid = 1.0f / (1.0f + expf(-z));
-            score[e] = GROUPED || p.score_mode == 0 ? sigmoid : z;
-            if (GROUPED) choice[e] = sigmoid + c;
+        if constexpr (DEEP) {
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+#pragma unroll
+                for (int j = 0; j < AHEAD; j++) b[k][j] = ahead[k][j];
+        } else {
+            ask(b, e0 + 2 * kWaves);
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) z[k] = wave_sum(z[k]);
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int e = e0 + k * kWaves;
+            if (lane == 0 && e < p.experts) {
+                const float sigmoid = 1.0f / (1.0f + expf(-z[k]));
+                score[e] = GROUPED || p.score_mode == 0 ? sigmoid : z[k];
+                if (GROUPED) choice[e] = sigmoid + c[k];
+            }
         }
     }
     __syncthreads();

@@ -1,5 +1,5 @@
 """A row's way into routed experts in one kernel against the kernels that it stands for: the stream and the normed row bit for bit behind a
-branch, the picks those of the routers for the row it leaves.  Widths of one to eight steps of 512, one expert, as many as waves, one more and the
+branch, the picks those of the routers for the row it leaves.  Widths of one to eight steps of 512, one expert, as many as waves, one more, an odd pair of a wave's experts and the
 most it takes, both scores, corrections and groups, equal scores, a row that is no number, and what it leaves to the others."""
 import pytest
 import torch
@@ -22,7 +22,8 @@ def operands(rows, width, experts, seed):
                                 (draw(experts, width) * 2 * width ** -0.5).to(BF16), torch.rand(experts, generator=g))]
 
 
-@pytest.mark.parametrize("rows,width,experts,top", [(1, 512, 1, 1), (2, 1536, 8, 2), (5, 1024, 4, 4), (64, 2048, 64, 6), (3, 2560, 6, 3), (7, 4096, 10, 2)])
+@pytest.mark.parametrize("rows,width,experts,top", [(1, 512, 1, 1), (2, 1536, 8, 2), (5, 1024, 4, 4), (64, 2048, 64, 6), (3, 2560, 6, 3), (7, 4096, 10, 2),
+                                                     (4, 512, 9, 2), (2, 1024, 13, 3), (3, 3072, 37, 5)])
 @pytest.mark.parametrize("router", ["sigmoid", "softmax", "grouped"])
 @pytest.mark.parametrize("behind", ["norm", "scale", "nothing"])
 def test_one_kernel_for_sum_norm_and_router(ops, rows, width, experts, top, router, behind):
