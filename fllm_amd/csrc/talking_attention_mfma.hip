@@ -29,7 +29,7 @@
 // weights, one 16-byte read a product).  Before, four waves held both value halves and staged keys and values through LDS
 // in two stages a block of 64 keys: 416 to 512 registers a lane, so one wave a SIMD waited out every latency by itself.
 // 1,900 rows from a request's first token on, two key/value heads of 128 lanes: 8 heads 264 -> 48 us, 12 heads 338 -> 75, 16
-// heads 546 -> 139 (the last spills 68 registers); 2,048 rows behind 8,192 keys, 12 heads, 2,609 -> 442.  The general instance:
+// heads 546 -> 139 (20 and 68 registers spilled at 12 and 16); 2,048 rows behind 8,192 keys, 12 heads, 2,609 -> 442.  The general instance:
 // 12 heads on 4 of 64 lanes, 1,000 rows, 143 -> 88 us; 16 on 16 of 32 lanes 324 -> 186.
 //
 // Rows of a tile see different key ranges when a chunk of positions ends inside the tile: the mask is per (row, key).
@@ -109,7 +109,7 @@ __device__ __forceinline__ TileKeys tile_keys(const TalkArgs &p, int first, int 
 
 typedef const __attribute__((address_space(4))) float *scalar_floats;      // read through the scalar cache
 
-// GS > 0: an instance for exactly HMAX heads on GS key/value heads, keys of 128 lanes, values of 80 to 128 and pages of a power
+// GS > 0 (1, 2 or 4): an instance for exactly HMAX heads on GS key/value heads, keys of 128 lanes, values of 80 to 128 and pages of a power
 // of two from 8 on, whose loops carry no conditions and whose key/value heads are unrolled.  GS 0: up to HMAX heads on any
 // number of key/value heads, any widths and pages of multiples of 4.
 template <int HMAX, int GS>
@@ -456,15 +456,16 @@ constexpr int kDecPPitch = kKeyBlock + 8;
 __device__ __forceinline__ size_t decode_part_floats(int heads, int v_dim) { return (size_t)heads * (2 + v_dim); }
 
 // All of a block's first loads (two key/value heads' keys and values) are asked for before anything waits, and sit behind no
-// condition; a later block's are asked for while the one before is weighed.  Before, every load sat behind a condition and was waited for by itself.
-// With the merge, 12 heads on two key/value heads of 128 lanes, in a graph: one row of 1,900 keys 15.6 -> 10.7 us, 64 rows of 1,000
-// 41.5 -> 20.6, one of 8,000 24.9 -> 15.0 (the general instance, 16 heads on 4 of 64 lanes, 4 rows of 1,000, 16.3 -> 14.1).
-// EXACT: up to two key/value heads, keys and
-// values of 128 lanes in pages of a power of two.
-template <bool EXACT>
+// condition; a later block's are asked for while the one before is weighed.  Before, every load sat behind a condition and was waited for
+// by itself.  With the merge, 12 heads on two key/value heads of 128 lanes, in a graph: one row of 1,900 keys 15.6 -> 10.7 us, 64 rows of
+// 1,000 41.5 -> 20.6, one of 8,000 24.9 -> 15.0 (the general instance, 16 heads on 4 of 64 lanes, 4 rows of 1,000, 16.3 -> 14.1).
+// GX > 0: up to GX key/value heads, keys and values of 128 lanes in pages of a power of two.  General and GX = 4, 12 heads on four: one
+// row of 1,900 keys 15.3 -> 12.4 us, 64 of 1,000 38.3 -> 30.3; GX = 8, 16 heads on eight: 20.9 -> 16.5 and 75.7 -> 55.3.
+template <int GX>
 __global__ void __launch_bounds__(kThreads, 2)
 talking_decode_kernel(const TalkArgs p) {
-    constexpr int HW = kDecHeads, KSM = EXACT ? 4 : 8, TS = 2, GM = EXACT ? 2 : kDecGMax;
+    constexpr bool EXACT = GX > 0;
+    constexpr int HW = kDecHeads, KSM = EXACT ? 4 : 8, TS = 2, GM = EXACT ? GX : kDecGMax;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     const int H = p.heads, G = p.kv_heads, D = EXACT ? 128 : p.k_dim, DV = EXACT ? 128 : p.v_dim, PS = p.page_size;
     const int group = H / G, KS = D / 32, DVT = DV / 16, HP = H | 1, shift = p.page_shift;
@@ -752,8 +753,11 @@ int launch_decode(const TalkArgs &a, hipStream_t stream) {
     const size_t lds = floats * sizeof(float) + ((size_t)H * a.k_dim + (size_t)G * 16 * kDecPPitch) * sizeof(bf16_t);
     if (lds > 60 * 1024) return 1;
     const dim3 grid(a.num_segs, a.splits), block(kThreads);
-    if (G <= 2 && a.k_dim == 128 && a.v_dim == 128 && a.page_shift >= 3) hipLaunchKernelGGL(talking_decode_kernel<true>, grid, block, lds, stream, a);
-    else hipLaunchKernelGGL(talking_decode_kernel<false>, grid, block, lds, stream, a);
+    const bool exact = a.k_dim == 128 && a.v_dim == 128 && a.page_shift >= 3;
+    if (exact && G <= 2) hipLaunchKernelGGL(talking_decode_kernel<2>, grid, block, lds, stream, a);
+    else if (exact && G <= 4) hipLaunchKernelGGL(talking_decode_kernel<4>, grid, block, lds, stream, a);
+    else if (exact) hipLaunchKernelGGL(talking_decode_kernel<kDecGMax>, grid, block, lds, stream, a);
+    else hipLaunchKernelGGL(talking_decode_kernel<0>, grid, block, lds, stream, a);
     int rc = fllm_check_launch("talking_attention (decode rows)");
     if (rc == 0 && a.splits > 1) {
         hipLaunchKernelGGL(talking_decode_merge_kernel, dim3(a.num_segs, H), dim3(kThreads), 0, stream, a);
@@ -784,6 +788,25 @@ int launch_tiles(const TalkArgs &a, int tiles, hipStream_t stream) {
         rc = fllm_check_launch("talking_attention (merge)");
     }
     return rc;
+}
+
+// 2: no instance for exactly these heads
+template <int GS>
+int launch_exact(const TalkArgs &a, int tiles, hipStream_t stream) {
+    switch (a.heads) {
+    case 4: return launch_tiles<4, GS>(a, tiles, stream);
+    case 8: return launch_tiles<8, GS>(a, tiles, stream);
+    case 12: return launch_tiles<12, GS>(a, tiles, stream);
+    case 16: return launch_tiles<16, GS>(a, tiles, stream);
+    }
+    if constexpr (GS <= 2) {
+        switch (a.heads) {
+        case 6: return launch_tiles<6, GS>(a, tiles, stream);
+        case 10: return launch_tiles<10, GS>(a, tiles, stream);
+        case 14: return launch_tiles<14, GS>(a, tiles, stream);
+        }
+    }
+    return 2;
 }
 
 }  // namespace
@@ -848,12 +871,14 @@ int fllm_talking_attention_bf16_fast(const void *q, const void *gate, int gate_s
     // every segment's rows in tiles of 16: at most rows / 16 full tiles and one ragged tile a segment
     const int tiles = rows / kTileRows + num_segs;
     // The kernel holds every head's scores and outputs of its rows in registers: an instance a bracket of head counts, and
-    // one each for exactly 8, 12 and 16 heads on two key/value heads of 128 lanes: without conditions in
-    // the loops nothing is spilled up to 12 heads, where the general one spills 106 registers (12 heads, 1,000 rows).
-    if (kv_heads == 2 && k_dim == 128 && v_dim > 64 && a.page_shift >= 3) {
-        if (heads == 8) return launch_tiles<8, 2>(a, tiles, stream);
-        if (heads == 12) return launch_tiles<12, 2>(a, tiles, stream);
-        if (heads == 16) return launch_tiles<16, 2>(a, tiles, stream);
+    // one each for an even number of heads on 1, 2 or 4 key/value heads of 128 lanes, the counts whose loops unroll without
+    // conditions.  What that is worth, 1,900 rows from a request's first token on, general and exact instance: 4 / 8 / 12 / 16 heads on
+    // one 58 -> 30, 84 -> 47, 187 -> 66, 329 -> 102 us (the last spills 44 registers), on four 78 -> 36, 102 -> 50, 211 -> 82 (35
+    // spilled), 353 -> 161 (126), 6 / 10 / 14 on two 77 -> 40, 169 -> 58, 299 -> 93 (48); 300 rows between 1.5 and 2.3 times.
+    if (k_dim == 128 && v_dim > 64 && a.page_shift >= 3) {
+        const int rc = kv_heads == 1 ? launch_exact<1>(a, tiles, stream) : kv_heads == 2 ? launch_exact<2>(a, tiles, stream)
+                     : kv_heads == 4 ? launch_exact<4>(a, tiles, stream) : 2;
+        if (rc <= 1) return rc;
     }
     if (heads <= 8) return launch_tiles<8, 0>(a, tiles, stream);
     if (heads <= 12) return launch_tiles<12, 0>(a, tiles, stream);

@@ -12,6 +12,9 @@ pytestmark = pytest.mark.gpu
 # heads, kv heads, key size, value size, chunk, page
 SHAPES = [(8, 2, 128, 128, None, 16), (12, 2, 128, 128, 300, 64), (16, 2, 128, 80, 130, 8), (12, 2, 128, 112, None, 4), (16, 2, 128, 128, 140, 24),
           (15, 3, 192, 48, None, 12), (16, 16, 160, 16, 200, 16), (7, 7, 96, 128, 129, 32), (8, 4, 256, 96, None, 8)]
+# every instance built for a head count on 1, 2 or 4 key/value heads of 128 lanes, values of 80 to 128, pages of 8 to 64
+SHAPES += [(H, G, 128, (128, 80, 96, 112)[(H // 2 + G) % 4], (None, 130, 200)[(H + G) % 3], (8, 16, 32, 64)[(H // 2 + G // 2) % 4])
+           for G in (1, 2, 4) for H in range(4, 17, 2) if H % G == 0 and (G, H) not in ((2, 8), (2, 12), (2, 16))]
 # (held, new): tiles of one row to several, last keys right before, on and behind a block's edge
 SEGMENTS = [(0, 129), (111, 17), (112, 16), (127, 2), (254, 3), (383, 33), (0, 5), (500, 12)]
 
@@ -47,9 +50,10 @@ def test_blocks_of_128_keys(ops, shape, splits):
     close(got, want, 3 * BF16_EPS, 3e-2, "attention")
 
 
-# heads, kv heads, key size, value size, chunk, page: the instance for one or two key/value heads of 128 lanes, and beside its rule
+# heads, kv heads, key size, value size, chunk, page: the instances for up to two, four and eight key/value heads of 128 lanes, and beside their rule
 SINGLE = [(12, 2, 128, 128, None, 16), (16, 1, 128, 128, 100, 8), (5, 1, 128, 128, None, 64), (12, 2, 128, 128, 70, 24), (9, 3, 128, 128, None, 16),
-          (16, 8, 64, 128, 130, 16), (6, 2, 128, 112, None, 32)]
+          (16, 8, 64, 128, 130, 16), (6, 2, 128, 112, None, 32), (12, 4, 128, 128, None, 16), (8, 4, 128, 128, 100, 8), (16, 8, 128, 128, None, 64),
+          (12, 6, 128, 128, 130, 16)]
 
 
 @pytest.mark.parametrize("splits", [1, 2, 4])
