@@ -194,8 +194,10 @@ gelu_side_kernel(const T *__restrict__ z, const int32_t *__restrict__ ids, const
 
 // One workgroup an output lane d and R rows: z = W[d] . x (x rounded to T first, as cast_rows gives it), then gelu_side of it.
 // widths that are multiples of 8 lie side by side in 16-byte loads.  What bounds it is its launch: up to 32 rows (eight a workgroup)
-// it replaces a cast, a product and a gate of 14 us together, each of them launch too; prompts and answers of 12 such
-// requests 12.70 -> 12.46 ms.
+// it replaces a cast, a product and a gate, each of them launch too.  Microseconds in a graph, this / those three, at 1, 8, 9, 16, 17 and 32
+// rows: 128 lanes of 1,024 2.5 / 6.6, 5.2 / 6.9, 5.1 / 7.4, 5.2 / 7.8, 5.4 / 9.4, 5.6 / 11.9; 256 of 2,048 2.5 / 7.4, 5.3 / 8.1, 5.5 / 8.7, 5.6 /
+// 9.6, 6.1 / 11.5, 7.2 / 12.0; 128 of 4,096 2.6 / 8.2, 6.6 / 9.7, 6.7 / 11.5, 6.7 / 12.7, 6.8 / 14.1, 7.3 / 12.4.  Prompts and answers of 12
+// such requests 12.70 -> 12.46 ms.
 template <typename T, int R>
 __global__ void __launch_bounds__(kBlock)
 side_gate_kernel(const float *__restrict__ x, const T *__restrict__ w, const int32_t *__restrict__ ids, const T *__restrict__ table, int vocab,
@@ -307,8 +309,8 @@ extern "C" int fllm_side_gate(const float *x, const void *w, const int32_t *ids,
     if (rows == 0) return 0;
     if (rows > (fllm_fast_kernels_enabled() ? 32 : 8) || width % 8 != 0 || (((uintptr_t)x | (uintptr_t)w) & 15) != 0) return 1;
 #define FLLM_SIDE(T, R)                                                                                                                      \
-    hipLaunchKernelGGL((side_gate_kernel<T, R>), dim3(dim, (rows + R - 1) / R), dim3(kBlock), 0, stream, x, (const T *)w, ids, (const T *)table, vocab, table_width, \
-                       offset, (T *)out, rows, width, dim)
+    hipLaunchKernelGGL((side_gate_kernel<T, R>), dim3(dim, (rows + R - 1) / R), dim3(kBlock), 0, stream, x, (const T *)w, ids,                \
+                       (const T *)table, vocab, table_width, offset, (T *)out, rows, width, dim)
 #define FLLM_SIDE_R(T)                            \
     do {                                          \
         if (rows == 1) FLLM_SIDE(T, 1);           \

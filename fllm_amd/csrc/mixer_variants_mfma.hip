@@ -347,7 +347,8 @@ mixer_tile_kernel(const TileParams p) {
     if (VARIANT == 0) {
         for (int i = threadIdx.x; i < splits * 16; i += kThreads) {
             const int q = i & 15;
-            if (q < count) s_factor[i >> 4][q] = fetch(all + (size_t)(i >> 4) * kStride + 16 * DV + q), s_sum[i >> 4][q] = fetch(all + (size_t)(i >> 4) * kStride + 16 * DV + 16 + q);
+            const float *of = all + (size_t)(i >> 4) * kStride + 16 * DV + q;
+            if (q < count) s_factor[i >> 4][q] = fetch(of), s_sum[i >> 4][q] = fetch(of + 16);
         }
     }
     for (int base = 0; base < count * DV; base += NI * kThreads) {      // every thread the same trips

@@ -2,8 +2,8 @@
 // tile-major copies straight into matrix-core operands.
 //
 // What bounds it is the bytes of the picked experts' weights, so everything else is kept out of their way: no list of
-// pairs is made by a kernel of its own (every wave finds its expert's pairs in `ids` itself; one wave for all with a barrier behind it cost prompts and
-// answers of 12 requests 12.40 ms where this takes 12.29), no scaled copies of the rows are
+// pairs is made by a kernel of its own (every wave finds its expert's pairs in `ids` itself; one wave for all with a barrier
+// behind it cost prompts and answers of 12 requests 12.40 ms where this takes 12.29), no scaled copies of the rows are
 // made (an operand is scaled where it is loaded, rounded to bfloat16 as a stored copy would be), and the down product is not cut
 // into planes that a further kernel adds.  A workgroup takes 16 output columns (of gate and of up) or 32 of one expert, its eight waves
 // cut K between them with 6 to 12 KiB asked for at a time each, and they meet in LDS once.  A load of the tile-major copy is

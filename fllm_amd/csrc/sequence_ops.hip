@@ -672,9 +672,10 @@ extern "C" int fllm_head_norm_kv_store(void *qkv, int ld, float eps, int norm_di
                  key_chunk);
     FLLM_REQUIRE(qkv && row_pos && row_seg && tables && (!store_kv || (k_pages && v_pages)), "head_norm_kv_store: operands missing");
     if (rows == 0) return 0;
-    // A head a wave in steps of few rows (a workgroup a row, whose waves take several heads one after the other, runs 7.3 us at 4 rows of
-    // 12 and 2 heads of 128 where this takes 4.3); rows that fill the device by themselves keep a workgroup each (2,000 rows: 13.9 us, and
-    // 15.3 with a head a wave).
+    // A head a wave in steps of few rows; rows that fill the device by themselves keep a workgroup each.  Microseconds in a graph, a head a
+    // wave / a workgroup a row, whose waves take several heads one after the other, at 4, 128, 512, 768, 1,024 and 2,000 rows: 12 and 2 heads
+    // of 128 3.2 / 5.4, 3.5 / 5.7, 5.6 / 6.6, 7.1 / 7.2, 8.6 / 8.2, 13.7 / 11.7; 32 and 8 of 128 3.1 / 10.2, 4.9 / 11.2, 11.0 / 13.5, 15.0 /
+    // 17.6, 18.3 / 20.0, 31.6 / 26.3; 16 and 4 of 64 3.0 / 5.3, 3.4 / 5.8, 6.1 / 6.6, 7.7 / 7.4, 9.4 / 8.3, 15.6 / 12.2.
     const dim3 grid(rows, rows > 512 ? 1u : (unsigned)std::min(((store_kv ? heads + kv_heads : heads) + kWaves - 1) / kWaves, 65535));
     if (dtype == FLLM_F32)
         hipLaunchKernelGGL(head_norm_kv_store_kernel<float>, grid, dim3(kBlock), 0, stream, (float *)qkv, ld, eps, norm_dim, row_pos,

@@ -99,7 +99,7 @@ stream_add_kernel(float *__restrict__ x, const int32_t *__restrict__ ids, const 
 // branch lane by lane: the norm's weight, a layer scale and the constant of the residual sum in one vector.  With
 // `next_w`, the RMSNorm of the new row (its own eps) is written to `next_out` as well, the norm that reads the stream
 // next; with `next_ssq` what the products behind a prepared norm take instead: the row times next_w, and its sum of squares there (a
-// q/k/v product of 8 rows of 1,536 lanes that finds its norm prepared takes 7.2 us, one that norms the stream itself 9.1).
+// q/k/v product of 8 rows of 1,536 lanes that finds its norm prepared takes 6.6 us, one that norms the stream itself 8.6).
 // One workgroup a row, sums in a fixed order: a row gives the same bits whatever else is in the batch.
 template <typename B, typename T>
 __global__ void __launch_bounds__(kBlock)
@@ -222,9 +222,8 @@ postnorm_add_vec_kernel(float *__restrict__ x, const float *__restrict__ branch,
 }
 
 // A request's first step finds the state of its slot at zero in every tensor that keeps one: all tensors and all such requests of a step
-// in one launch (12 requests of a model with 14 tensors were 168 fills of 2 us and their launches:
-// prompts and answers of those 13.11 -> 12.76 ms).  table[i]: where tensor i begins and
-// the bytes of a slot of it.
+// in one launch (12 requests of a model with 14 tensors were 168 fills of 2 us and their launches: prompts and answers of those 13.11 ->
+// 12.76 ms).  table[i]: where tensor i begins and the bytes of a slot of it.
 constexpr int kSlotsALaunch = 60;      // by value in the kernel's arguments
 constexpr int kClearBytes = 32 * 1024; // of a slot a workgroup
 

@@ -284,7 +284,6 @@ def _talking_shares(tiles: int, least: int, blocks: int, slots: int) -> int:
     return best
 
 
-
 class Ops:
     """Launches kernels on the current torch stream of the tensors' device.
 
@@ -359,9 +358,9 @@ class Ops:
         """Keeps beside `w` (bfloat16 [N, K] on the GPU) a copy in the order in which the products of decode steps read
         it (`fllm_tile_weights`): `linear`, `linear_add_prepare`, `linear_relu_squared` and the forms behind a norm find it by
         the matrix's address and use it for steps of up to 16 rows, and where its width is a multiple of 1,024 the sums, the
-        float32 logits and the forms behind a prepared norm for up to 64 (sums into a float32 `out` and `gate_up_swiglu`: up to 128).  `gate_up`: w is [gate; up] and the copy holds 8 gate rows and the
-        same 8 up rows a tile (`fllm_tile_weights_gate_up`), for `norm_gate_up_swiglu` and `gate_up_swiglu`.  The copy is
-        given up with `w`.  False: nothing was made (another type or place, a shape the kernels do not take tiles of)."""
+        float32 logits and the forms behind a prepared norm for up to 64 (sums into a float32 `out` and `gate_up_swiglu`: up
+        to 128).  `gate_up`: w is [gate; up] and the copy holds 8 gate rows and the same 8 up rows a tile
+        (`fllm_tile_weights_gate_up`), for `norm_gate_up_swiglu` and `gate_up_swiglu`.  The copy is given up with `w`.  False: nothing was made (another type or place, a shape the kernels do not take tiles of)."""
         if not self.tile_for_decode_supported(w, gate_up):
             return False
         N, K = w.shape
