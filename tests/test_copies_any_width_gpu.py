@@ -197,3 +197,34 @@ def test_copies_of_a_model_take_no_more_memory_than_theirs(ops):
     # torch's allocator hands out steps of 2 MiB from there on and keeps a remainder of up to 1 MiB with the block
     assert made <= torch.cuda.memory_allocated() - before <= made + len(ws) * (2 << 20)
     assert all(ops._tiles_of(w).numel() * 2 == ops.copy_bytes(w) for w in ws)
+
+
+def test_copies_without_a_piece_lie_by_themselves(ops, monkeypatch):
+    """No memory for the piece that copies were to share: each has its own, with the same contents; one that has none raises and leaves nothing."""
+    import fllm_amd.kernels as kernels
+    ws = [draw((48, 256), 1), draw((32, 512), 2)]
+    total = sum(ops.copy_bytes(w) for w in ws)
+    real, sizes = torch.empty, [total // 2]
+
+    def empty(size, *args, **kwargs):
+        if size in sizes:
+            raise torch.cuda.OutOfMemoryError("no room")
+        return real(size, *args, **kwargs)
+
+    with monkeypatch.context() as m:
+        m.setattr(kernels.torch, "empty", empty)
+        with ops.copies_together(total):
+            assert all(ops.tile_for_decode(w) for w in ws)
+        lone = draw((64, 288), 3)
+        sizes.append(ops.copy_bytes(lone) // 2)
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            ops.tile_for_decode(lone)
+    assert ops._tiles_of(lone) is None
+    tiles = [ops._tiles_of(w) for w in ws]
+    assert tiles[0].untyped_storage().data_ptr() != tiles[1].untyped_storage().data_ptr()
+    again = [w.clone() for w in ws]
+    with ops.copies_together(total):
+        assert all(ops.tile_for_decode(w) for w in again)
+    together = [ops._tiles_of(w) for w in again]
+    assert together[0].untyped_storage().data_ptr() == together[1].untyped_storage().data_ptr()
+    assert all(torch.equal(a, b) for a, b in zip(tiles, together))
