@@ -34,6 +34,9 @@ int fllm_option_x_direct(void);
 // products of 17 to 64 rows: 1 (default) the kernel that suits the shape; 0 activations pass through LDS in chunks wherever
 // that kernel can serve; 2 a K slice of the activations stays in LDS wherever that kernel can serve
 int fllm_option_slab(void);
+// products of many rows on 256-row tiles: 1 (default) a last round of at most 128 tiles runs as tiles of half the rows where that takes less
+// time; 0 never; 2 wherever it can
+int fllm_option_half_tiles(void);
 int fllm_option_wide_waves(void);
 int fllm_option_resident_tiles(void);
 int fllm_option_tile32_rows(void);

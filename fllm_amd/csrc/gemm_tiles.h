@@ -11,9 +11,9 @@
 // 16-byte store); a workgroup asks for its next tile's first steps before it stores the last one.
 //
 // Measured (one MI355X, random operands, weights from memory, launches that follow one another, beside the GEMM library; boxes differ by
-// 5 %): 8,192 x 8,192 x 8,192 720 us (1.53 PFLOP/s, library 703); 2,048 x 28,672 x 4,096 with the SwiGLU in the epilogue 361 to 382 us (1.33 to
-// 1.26; library and a SwiGLU kernel 382 to 422), in a model's prompt step 362; 2,048 x 4,096 x 14,336 as 128-row tiles 197 us (1.22; library
-// 217), as 256-row tiles 257 (half of the compute units).
+// 5 %): 8,192 x 8,192 x 8,192 720 us (1.53 PFLOP/s, library 703); 2,048 x 28,672 x 4,096 with the SwiGLU in the epilogue 346 to 356 us (1.39 to
+// 1.35; library and a SwiGLU kernel 382 to 422), 368 where its last round runs as whole tiles; 2,048 x 4,096 x 14,336 as 128-row tiles 197 us
+// (1.22; library 217), as 256-row tiles 257 (half of the compute units).
 //
 // MFMA operand layout (v_mfma_f32_16x16x32_bf16): A lane l holds A[m = l%16][k = 8*(l/16) .. +7]; B likewise with n = l%16; D lane l holds
 // D[m = 4*(l/16) + i][n = l%16], i = 0..3.  A is W here, B the rows of x.
@@ -35,6 +35,7 @@ struct TileArgs {
     const int32_t *work;    // null: the rows of x as they are
     int max_tiles;
     int top;                // the row of x a pair reads: > 0 pair / top, 0 its slot, -1 the pair
+    int halves;             // the 256-row kernel: whether a last round of at most 128 tiles runs as tiles of half the rows
 };
 
 constexpr int kThreads = 512;
@@ -64,19 +65,28 @@ template <int EPI> __device__ __forceinline__ int tile_column(int r, int h) {
 
 // Which tile a workgroup works on.  The dies (workgroup number modulo 8) take runs of neighbouring tiles, in groups of 8 row tiles, so that
 // what a die's workgroups read at a time fits its L2.
-template <int EPI, bool GROUPED, int BM>
+// HALVES: tiles of 128 rows, two for each of the 256-row tiles of a last round.
+template <int EPI, bool GROUPED, int BM, bool HALVES = false>
 struct Place {
     int total, mt, nt;
     int m0, n0;              // first row (grouped: slot) and column
     int rows;                // rows the tile has
     const bf16_t *w;
+    static constexpr int kRows = HALVES ? 256 : BM;      // that a tile of the order below has
     __device__ __forceinline__ Place(const TileArgs &a) {
-        mt = GROUPED ? __builtin_amdgcn_readfirstlane(a.work[0]) : (a.M + BM - 1) / BM;
+        mt = GROUPED ? __builtin_amdgcn_readfirstlane(a.work[0]) : (a.M + kRows - 1) / kRows;
         nt = (a.N + (EPI == EPI_GLU ? 127 : 255)) / (EPI == EPI_GLU ? 128 : 256);
         total = mt * nt;
         w = a.w;
     }
+    // tiles of the last round that run as halves: their workgroups would take a whole tile's time and leave the others idle
+    __device__ __forceinline__ int in_halves(const TileArgs &a) const { return a.halves && total % 256 <= 128 ? total % 256 : 0; }
     __device__ __forceinline__ void go(const TileArgs &a, int id) {
+        int half = 0;
+        if (HALVES) {                                        // both halves of a tile on the tile's die
+            half = (id / 8) & 1;
+            id = total - in_halves(a) + id / 16 * 8 + id % 8;
+        }
         const int q = total / 8, r = total % 8, die = id % 8;
         id = (die < r ? die * (q + 1) : r * (q + 1) + (die - r) * q) + id / 8;
         const int per = 8 * nt, g = id / per, first = g * 8, tall = min(8, mt - first), in = id - g * per;
@@ -85,11 +95,11 @@ struct Place {
         if (GROUPED) {
             const int32_t *tile = a.work + 1 + 3 * t;
             const int e = __builtin_amdgcn_readfirstlane(tile[0]);
-            m0 = __builtin_amdgcn_readfirstlane(tile[1]);
-            rows = __builtin_amdgcn_readfirstlane(tile[2]);
+            m0 = __builtin_amdgcn_readfirstlane(tile[1]) + half * BM;
+            rows = __builtin_amdgcn_readfirstlane(tile[2]) - half * BM;
             w = a.w + (size_t)e * (EPI == EPI_GLU ? 2 : 1) * a.N * a.K;
         } else {
-            m0 = t * BM;
+            m0 = t * kRows + half * BM;
             rows = a.M - m0;
         }
     }
@@ -173,8 +183,9 @@ __device__ __forceinline__ void tiles256(const TileArgs &a) {
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int wm = w >> 2, wn = w & 3, l16 = lane & 15, lg = lane >> 4;
     Place<EPI, GROUPED, 256> at(a);
+    const int total = at.total - at.in_halves(a);
     int id = blockIdx.x;
-    if (id >= at.total) return;
+    if (id >= total) return;
     const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) bf16_t *)lds;
     const uint32_t mine = __builtin_amdgcn_readfirstlane(base + w * 1024);
     uint32_t off_x[2][2], off_w[2][2];      // bytes from x and from the matrix to what this lane loads of a half tile, in two pieces
@@ -280,7 +291,7 @@ __device__ __forceinline__ void tiles256(const TileArgs &a) {
                 if (GROUPED) asm volatile("" : "+v"(to[i][t]));      // looked up before the next tile's loads are in the way
             }
         id += gridDim.x;
-        const bool more = id < at.total;
+        const bool more = id < total;
         if (more) {
             at.go(a, id);
             offsets();
@@ -301,14 +312,15 @@ __device__ __forceinline__ void tiles256(const TileArgs &a) {
 // 128 x 256 (EPI_GLU: 128 x 128), for launches whose 256-row tiles would leave much of the device idle: an operand read from LDS serves half
 // the products, so LDS and the matrix cores are busy alike.  LDS: three buffers of [x][W half 0][W half 1].  K step k: half 0 reads x of k
 // and asks for W half 1 of k + 2 and W half 0 of k + 3; half 1 reads W half 1 of k and W half 0 of k + 1 and asks for x of k + 3.
-template <int EPI, bool GROUPED>
+template <int EPI, bool GROUPED, bool HALVES = false>
 __device__ __forceinline__ void tiles128(const TileArgs &a) {
     extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int wm = w >> 2, wn = w & 3, l16 = lane & 15, lg = lane >> 4;
-    Place<EPI, GROUPED, 128> at(a);
+    Place<EPI, GROUPED, 128, HALVES> at(a);
     int id = blockIdx.x;
-    if (id >= at.total) return;
+    const int total = HALVES ? (at.in_halves(a) + 7) / 8 * 16 : at.total;      // HALVES: at most one a workgroup
+    if (id >= total || (HALVES && id / 16 * 8 + id % 8 >= at.in_halves(a))) return;
     constexpr uint32_t kSlot = 3 * kHalf;
     const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) bf16_t *)lds;
     const uint32_t mine = __builtin_amdgcn_readfirstlane(base + w * 1024);
@@ -364,6 +376,7 @@ __device__ __forceinline__ void tiles128(const TileArgs &a) {
     };
     const int T = a.K / BK;                 // at least 3
     at.go(a, id);
+    if (HALVES && at.rows <= 0) return;
     offsets();
     first_steps();
     for (;;) {
@@ -409,7 +422,7 @@ __device__ __forceinline__ void tiles128(const TileArgs &a) {
         read_w(s2, 1, w1);
         FLLM_LGKM0; FLLM_SWAP; multiply(acc[1], xs, w1); FLLM_SWAP;
         if (wm == 0) FLLM_SWAP;
-        const Place<EPI, GROUPED, 128> done = at;
+        const Place<EPI, GROUPED, 128, HALVES> done = at;
         int to[4];
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -417,7 +430,7 @@ __device__ __forceinline__ void tiles128(const TileArgs &a) {
             if (GROUPED) asm volatile("" : "+v"(to[t]));
         }
         id += gridDim.x;
-        const bool more = id < at.total;
+        const bool more = !HALVES && id < total;
         if (more) {
             at.go(a, id);
             offsets();
@@ -434,38 +447,44 @@ __device__ __forceinline__ void tiles128(const TileArgs &a) {
 
 // The kernels, products of their own and grouped ones under names of their own in a trace; the modes of the grouped ones are those of
 // the small grouped tiles: 0 gate and up with the activation, 1 float32 sums, 2 the squared ReLU.
-template <int EPI, int ROWS>
+// HALVES: a last round of at most 128 tiles of 256 rows runs as twice as many of 128 rows, which take 0.6 to 0.7 of its time.
+template <int EPI, int ROWS, bool HALVES>
 __global__ void __launch_bounds__(kThreads, 2) tiles_kernel(const TileArgs a) {
     if constexpr (ROWS == 256) tiles256<EPI, false>(a);
-    else tiles128<EPI, false>(a);
+    if constexpr (ROWS == 128 || HALVES) tiles128<EPI, false, HALVES>(a);
 }
-template <int MODE, int ROWS>
+template <int MODE, int ROWS, bool HALVES>
 __global__ void __launch_bounds__(kThreads, 2) large_grouped_tiles_kernel(const TileArgs a) {
     constexpr int EPI = MODE == 0 ? EPI_GLU : MODE == 1 ? EPI_F32 : EPI_RELU2;
     if constexpr (ROWS == 256) tiles256<EPI, true>(a);
-    else tiles128<EPI, true>(a);
+    if constexpr (ROWS == 128 || HALVES) tiles128<EPI, true, HALVES>(a);
 }
-template <int EPI, bool GROUPED, int ROWS>
+template <int EPI, bool GROUPED, int ROWS, bool HALVES>
 auto tiles_entry() -> void (*)(TileArgs) {
-    if constexpr (GROUPED) return large_grouped_tiles_kernel<EPI == EPI_GLU ? 0 : EPI == EPI_F32 ? 1 : 2, ROWS>;
-    else return tiles_kernel<EPI, ROWS>;
+    if constexpr (GROUPED) return large_grouped_tiles_kernel<EPI == EPI_GLU ? 0 : EPI == EPI_F32 ? 1 : 2, ROWS, HALVES>;
+    else return tiles_kernel<EPI, ROWS, HALVES>;
 }
 
-// Launches one of the two on `blocks` workgroups (one a compute unit at most; grouped: as many tiles as there may be).
-template <int EPI, bool GROUPED>
-int launch_tiles(const TileArgs &a, int bm, long tiles, hipStream_t stream) {
+// Launches one of them on one workgroup a compute unit at most (grouped: as many tiles as there may be).
+template <int EPI, bool GROUPED, int ROWS, bool HALVES>
+int launch_entry(const TileArgs &a, unsigned blocks, hipStream_t stream) {
+    constexpr int lds = ROWS == 256 && !HALVES ? kLds256 : kLds128;
+    static_assert(kLds128 >= kLds256, "both kinds of tiles in one launch");
     static bool raised = false;      // more than 64 KiB of LDS has to be asked for once
     if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void *)tiles_entry<EPI, GROUPED, 256>(), hipFuncAttributeMaxDynamicSharedMemorySize, kLds256);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)tiles_entry<EPI, GROUPED, 128>(), hipFuncAttributeMaxDynamicSharedMemorySize, kLds128);
+        const hipError_t e = hipFuncSetAttribute((const void *)tiles_entry<EPI, GROUPED, ROWS, HALVES>(), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         FLLM_REQUIRE(e == hipSuccess, "gemm tiles: cannot raise the LDS limit: %s", hipGetErrorString(e));
         raised = true;
     }
-    const unsigned blocks = (unsigned)(tiles < 256 ? tiles : 256);
-    if (bm == 256) hipLaunchKernelGGL((tiles_entry<EPI, GROUPED, 256>()), dim3(blocks), dim3(kThreads), kLds256, stream, a);
-    else hipLaunchKernelGGL((tiles_entry<EPI, GROUPED, 128>()), dim3(blocks), dim3(kThreads), kLds128, stream, a);
+    hipLaunchKernelGGL((tiles_entry<EPI, GROUPED, ROWS, HALVES>()), dim3(blocks), dim3(kThreads), lds, stream, a);
     return fllm_check_launch("gemm tiles");
+}
+template <int EPI, bool GROUPED>
+int launch_tiles(TileArgs a, int bm, bool halves, long tiles, hipStream_t stream) {
+    a.halves = halves;
+    if (halves) return launch_entry<EPI, GROUPED, 256, true>(a, 256, stream);
+    const unsigned blocks = (unsigned)(tiles < 256 ? tiles : 256);
+    return bm == 256 ? launch_entry<EPI, GROUPED, 256, false>(a, blocks, stream) : launch_entry<EPI, GROUPED, 128, false>(a, blocks, stream);
 }
 
 }  // namespace fllm_tiles

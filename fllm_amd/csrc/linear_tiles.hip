@@ -19,7 +19,10 @@ TileArgs tile_args(const void *x, int ldx, const void *w, void *out, int ldo, in
     a.ldx = ldx, a.ldo = ldo, a.M = M, a.N = N, a.K = K;
     return a;
 }
-long tiles_of(long M, int bm, int N, int cols) { return (M + bm - 1) / bm * ((N + cols - 1) / cols); }
+fllm_plan::TilePlan plan_of(long M, int N, int cols, int K, int force) {
+    const long columns = (N + cols - 1) / cols;
+    return fllm_plan::tile_plan((M + 255) / 256 * columns, (M + 127) / 128 * columns, K, force, fllm_option_half_tiles());
+}
 
 }  // namespace
 
@@ -27,20 +30,18 @@ long tiles_of(long M, int bm, int N, int cols) { return (M + bm - 1) / bm * ((N 
 // asks for that row tile and is declined where K is too short for it or no whole steps, as is any value but 0, 1 and these).
 //
 // The fused product against the library's product and an activation kernel, inside a graph, weights from memory, microseconds at 512 /
-// 1,024 / 2,048 rows: 2 x 14,336 x 4,096 116 -> 104 / 212 -> 191 / 382 -> 361; 2 x 8,192 x 2,048 43 -> 37 / 69 -> 59 / 121 -> 111; 2 x 8,960 x 1,536
-// 45 -> 43 / 79 -> 72 / 137 -> 118; 2 x 4,096 x 1,024 20 -> 18 / 27 -> 21 / 42 -> 35.  Where few rows or half-empty rounds make it slower: activation_joins in plans.h.
+// 1,024 / 2,048 rows: 2 x 14,336 x 4,096 116 -> 104 / 212 -> 185 / 398 -> 352; 2 x 8,192 x 2,048 43 -> 37 / 69 -> 57 / 123 -> 109; 2 x 8,960 x 1,536
+// 45 -> 43 / 82 -> 63 / 137 -> 106; 2 x 4,096 x 1,024 20 -> 18 / 27 -> 21 / 42 -> 35.  Where few rows or half-empty rounds make it slower: activation_joins in plans.h.
 extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up, void *out, int M, int inter, int K, float limit, float alpha,
                                   float up_offset, int force, hipStream_t stream) {
     FLLM_REQUIRE(M >= 0 && inter > 0 && K > 0 && ldx >= K && x && w_gate_up && out, "gate_up_tiles: bad sizes or operands missing");
     if (!fllm_fast_kernels_enabled() || !operands_fit(x, ldx, w_gate_up, out, inter, M, 2L * inter, inter, K)) return 1;
     if (M == 0) return 0;
-    const long t256 = tiles_of(M, 256, inter, 128), t128 = tiles_of(M, 128, inter, 128);
-    const int bm = fllm_plan::row_tile(t256, t128, K, force);
-    const long tiles = bm == 256 ? t256 : t128;
-    if (bm == 0 || (!force && !fllm_plan::activation_joins(M, 2L * inter, K, bm, tiles))) return 1;
+    const fllm_plan::TilePlan plan = plan_of(M, inter, 128, K, force);
+    if (plan.bm == 0 || (!force && !fllm_plan::activation_joins(M, 2L * inter, K, plan.rounds))) return 1;
     TileArgs a = tile_args(x, ldx, w_gate_up, out, inter, M, inter, K);
     a.limit = limit, a.alpha = alpha, a.up_offset = up_offset;
-    return launch_tiles<EPI_GLU, false>(a, bm, tiles, stream);
+    return launch_tiles<EPI_GLU, false>(a, plan.bm, plan.halves, plan.tiles, stream);
 }
 
 // mode 0: out = x w^T (+ bias); 2: out = relu(x w^T)^2; bfloat16.
@@ -56,14 +57,13 @@ extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const fl
                  "linear_tiles: bad sizes or operands missing");
     if (!fllm_fast_kernels_enabled() || (bias && mode != 0) || !operands_fit(x, ldx, w, out, ldo, M, N, N, K)) return 1;
     if (M == 0) return 0;
-    const long t256 = tiles_of(M, 256, N, 256), t128 = tiles_of(M, 128, N, 256);
-    const int bm = fllm_plan::row_tile(t256, t128, K, force);
-    if (bm == 0) return 1;
+    const fllm_plan::TilePlan plan = plan_of(M, N, 256, K, force);
+    if (plan.bm == 0) return 1;
     TileArgs a = tile_args(x, ldx, w, out, ldo, M, N, K);
     a.bias = bias;
-    const long tiles = bm == 256 ? t256 : t128, slots = (tiles + 255) / 256 * 256;
-    if (!force && mode == 2 && !fllm_plan::activation_joins(M, N, K, bm, tiles)) return 1;
-    if (!force && mode == 0 && !bias && (K < 2048 || 10 * tiles < 9 * slots)) return 1;
-    if (mode == 0) return launch_tiles<EPI_STORE, false>(a, bm, tiles, stream);
-    return launch_tiles<EPI_RELU2, false>(a, bm, tiles, stream);
+    const long slots = (plan.tiles + 255) / 256 * 256;
+    if (!force && mode == 2 && !fllm_plan::activation_joins(M, N, K, plan.rounds)) return 1;
+    if (!force && mode == 0 && !bias && (K < 2048 || (!plan.halves && 10 * plan.tiles < 9 * slots))) return 1;
+    if (mode == 0) return launch_tiles<EPI_STORE, false>(a, plan.bm, plan.halves, plan.tiles, stream);
+    return launch_tiles<EPI_RELU2, false>(a, plan.bm, plan.halves, plan.tiles, stream);
 }

@@ -217,6 +217,34 @@ inline int row_tile(long tiles256, long tiles128, int K, int asked = 0) {
     return a <= b ? 256 : 128;
 }
 
+// The row tile and whether a last round of at most 128 tiles of 256 rows runs as halves (twice as many tiles of 128 rows), which leaves no more
+// than half of the compute units idle for 0.6 to 0.7 of a round instead of a whole one; a fuller round would take two of them.  `rounds`: the time
+// in rounds of whole 256-row tiles over the compute units.  Measured without -> with, microseconds: 28,672 columns of 4,096 at 700 / 1,100 / 2,048
+// rows (2, 3, 4 rounds before) 170 -> 150 / 257 -> 239 / 368 -> 352; 17,920 of 1,536 at 1,024 / 2,048 75 -> 63 / 116 -> 106; both products of eight
+// experts of 4,480 of 1,536, 1,900 tokens that pick two 228 -> 209.
+struct TilePlan {
+    int bm = 0;                 // 0: a shape the tiles do not take
+    bool halves = false;
+    long tiles = 0;             // of bm rows
+    double rounds = 0;
+};
+// The time of `tiles` 256-row tiles with the last round in halves where it can be
+inline bool last_round_in_halves(long tiles) { return tiles % 256 != 0 && tiles % 256 <= 128; }
+inline double rounds_with_halves(long tiles) { return (double)(tiles / 256) + (tiles % 256 == 0 ? 0.0 : last_round_in_halves(tiles) ? kShortRound : 1.0); }
+// halves: 0 never, 1 where they take less time, 2 wherever they can be
+inline TilePlan tile_plan(long tiles256, long tiles128, int K, int asked, int halves) {
+    TilePlan p;
+    p.bm = row_tile(tiles256, tiles128, K, asked);
+    if (p.bm == 0) return p;
+    p.tiles = p.bm == 256 ? tiles256 : tiles128;
+    p.rounds = (double)((p.tiles + 255) / 256) * (p.bm == 256 ? 1.0 : kShortRound);
+    const bool asked_other = asked != 0 && asked != 1 && asked != 256;
+    if (halves == 0 || asked_other || !row_tile_takes(256, K) || !last_round_in_halves(tiles256)) return p;
+    if (halves == 2 || (tiles256 > 256 && rounds_with_halves(tiles256) < p.rounds))
+        p.bm = 256, p.halves = true, p.tiles = tiles256, p.rounds = rounds_with_halves(tiles256);
+    return p;
+}
+
 // Whether a product with its activation in the epilogue (gate and up: `columns` counts both; the squared ReLU) goes to the tiles, or to the GEMM
 // library and a kernel for the activation.  A tile costs the same however few of its rows and columns are there and however few of the
 // compute units have one, where the library has smaller tiles and cuts K; against that stands one pass over the product, which
@@ -227,11 +255,13 @@ inline int row_tile(long tiles256, long tiles128, int K, int asked = 0) {
 // the squared ReLU of 4,480 of 1,536 128 19 -> 26, 512 22.9 -> 24.8, then 900 1.21x, of 13,312 of 1,536 128 22 -> 28, then 320 31 -> 26, 512 35 -> 28 (line at
 // 0.29).  Up to K 1,024 the two sides are a few microseconds apart on the device (8,192 of 1,024 128 15.8 -> 20.3, 320 19.5 -> 19.2, 512 21.5 -> 19.9) and a
 // prompt step of such a model waits for the host's launches, of which the tiles save one: 24 -> 18 to 20 at 65 to 512 rows launched one by one.
-inline bool activation_joins(long M, long columns, int K, int bm, long tiles) {
+inline bool activation_joins(long M, long columns, int K, double rounds) {
     if (K <= 1024) return true;
-    const double rounds = (double)((tiles + 255) / 256) * (bm == 256 ? 1.0 : kShortRound);
     const double share = (double)M * (double)columns / (rounds * 256.0 * 65536.0), line = (K - 1024) / 1792.0;
     return share >= (line < 0.65 ? line : 0.65);
+}
+inline bool activation_joins(long M, long columns, int K, int bm, long tiles) {
+    return activation_joins(M, columns, K, (double)((tiles + 255) / 256) * (bm == 256 ? 1.0 : kShortRound));
 }
 
 // ---- decode attention: contexts split over workgroups ----

@@ -253,11 +253,11 @@ int large_row_tile(long pairs, int E, int inter, int K, int N, int up_columns, c
     if ((uint64_t)x_rows * ldx * 2 >= most || (uint64_t)pairs * inter * 2 >= most || (uint64_t)2 * inter * K * 2 >= most || (uint64_t)N * inter * 2 >= most)
         return 0;
     auto cost = [&](int bm) {
-        const long rows = (pairs + (long)E * bm / 2) / bm;
-        const long up = (rows * ((inter + up_columns - 1) / up_columns) + 255) / 256, down = (rows * ((N + 255) / 256) + 255) / 256;
-        return (double)up * K + (double)down * inter;
+        const long rows = (pairs + (long)E * bm / 2 + bm - 1) / bm, up = rows * ((inter + up_columns - 1) / up_columns), down = rows * ((N + 255) / 256);
+        if (bm == 256 && fllm_option_half_tiles()) return fllm_plan::rounds_with_halves(up) * K + fllm_plan::rounds_with_halves(down) * inter;
+        return (bm == 256 ? 1.0 : fllm_plan::kShortRound) * ((double)((up + 255) / 256) * K + (double)((down + 255) / 256) * inter);
     };
-    return cost(256) <= fllm_plan::kShortRound * cost(128) ? 256 : 128;
+    return cost(256) <= cost(128) ? 256 : 128;
 }
 
 // Both products on those tiles, behind group_pairs_kernel and (where the picks' weights scale the rows) scaled_rows_kernel.
@@ -271,11 +271,12 @@ int launch_large(int bm, const void *x, int ldx, int top, const void *w_up, cons
     a.limit = limit, a.alpha = alpha, a.up_offset = up_offset;
     a.work = work, a.max_tiles = (int)max_tiles, a.top = top;
     const int columns = UP == EPI_GLU ? 128 : 256;
-    int rc = launch_tiles<UP, true>(a, bm, max_tiles * ((inter + columns - 1) / columns), stream);
+    const bool halves = bm == 256 && fllm_option_half_tiles() != 0;      // how many tiles there are is known on the device
+    int rc = launch_tiles<UP, true>(a, bm, halves, max_tiles * ((inter + columns - 1) / columns), stream);
     if (rc != 0) return rc;
     a.x = (const bf16_t *)act, a.w = (const bf16_t *)w_down, a.out = out;
     a.ldx = inter, a.ldo = N, a.N = N, a.K = inter, a.top = -1;
-    return launch_tiles<EPI_F32, true>(a, bm, max_tiles * ((N + 255) / 256), stream);
+    return launch_tiles<EPI_F32, true>(a, bm, halves, max_tiles * ((N + 255) / 256), stream);
 }
 
 }  // namespace

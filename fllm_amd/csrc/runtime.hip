@@ -39,6 +39,8 @@ static int g_wide_waves = 0;      // 0: planned
 int fllm_option_wide_waves(void) { return g_wide_waves; }
 static int g_resident_tiles = 1;  // q/k/v of up to 16 rows behind a prepared norm streams its tile-major copy (16-row tiles)
 int fllm_option_resident_tiles(void) { return g_resident_tiles; }
+static int g_half_tiles = 1;      // products of many rows: a last round that is half full at most runs as tiles of half the rows; 0 never, 2 wherever it can
+int fllm_option_half_tiles(void) { return g_half_tiles; }
 static int g_slab = 1;
 int fllm_option_slab(void) { return g_slab; }
 static int g_fused_merge = 1;
@@ -55,6 +57,10 @@ extern "C" int fllm_set_option(const char *name, int value) {
     }
     if (strcmp(name, "attention.prefill_parts") == 0) {
         g_prefill_parts = value > 0 ? value : 0;
+        return 0;
+    }
+    if (strcmp(name, "linear.half_tiles") == 0) {
+        g_half_tiles = value < 0 ? 0 : (value > 2 ? 2 : value);
         return 0;
     }
     if (strcmp(name, "linear.slab") == 0) {
