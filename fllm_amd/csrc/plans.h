@@ -278,6 +278,11 @@ inline void decode_split_plan(int rows, int kv_heads, int qtiles, int max_contex
         if (base < 512) want = (512 + base - 1) / base;
         const long most = (span + unit - 1) / unit;
         if (want > most) want = most;
+        // Heads of 128 lanes, contexts of two rounds at most: whole.  The second round's keys are on their way before the first's are multiplied, where a
+        // second part has to be handed over (us split / whole at 300 and 500 keys: 12 heads on 2, eight rows 8.3 / 7.0 and 8.7 / 8.1, one row
+        // 7.1 / 6.2 and 7.4 / 6.8; 32 on 8, eight rows 8.0 / 7.2 and 8.4 / 8.6, forty 13.6 / 13.2 and 19.5 / 18.6).  Of 64 lanes a round is 512 keys,
+        // and the two are even (700 and 1,000 keys, eight rows 7.8 / 7.1 and 8.1 / 8.6; 16 rows of 48 to 798 8.1 / 8.2).
+        if (unit == 256 && max_context <= 2 * unit) want = 1;
     } else if (max_context > 2048 && base < 256) {
         want = (256 + base - 1) / base;
         const long most = (span + 2047) / 2048;
