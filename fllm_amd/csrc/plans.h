@@ -66,15 +66,36 @@ inline ResidentPlan plan_resident(int M, int K, int ntiles, int rt, size_t ws_by
     return best;
 }
 
+// The most tiles that one compute unit has where `groups` workgroups take `ntiles` in turn and workgroups i and i + cus meet on one unit:
+// the first unit's, since a workgroup has no more tiles than the ones before it
+inline int busiest_unit(int ntiles, int groups, int cus) {
+    return (ntiles + groups - 1) / groups + (groups > cus ? (ntiles - cus + groups - 1) / groups : 0);
+}
 // workgroups of a resident launch: one per slot of the device and slice, no more than there are tiles
 inline int resident_groups(const ResidentPlan &p, int ntiles, int cus) {
     int groups = cus * p.per_cu / p.S;
     if (groups < 1) groups = 1;
     if (groups > ntiles) groups = ntiles;
+    const int most = groups;
     // no more workgroups than give every one the same number of tiles: 1,792 tiles on 512 slots are 448 workgroups of 4
     // tiles, not 256 of 4 beside 256 of 3 that wait for them (gate/up of the 8B sizes at 8 rows: 40.2 -> 39.6 us)
     const int rounds = (ntiles + groups - 1) / groups;
     groups = (ntiles + rounds - 1) / rounds;
+    // Two workgroups a compute unit: where that gives some units two such workgroups and others one, as many more as take more than an eighth
+    // off what the busiest unit streams (to three tiles from four, to five from six).  1,120 tiles are 432 workgroups of 3 and 2 tiles,
+    // where 374 of 3 left 138 units half of what the others had; all 512 slots were slower than the fewest that do.  Microseconds at one and
+    // eight rows, by gate/up tiles and K: 1,120 of 1,536 14.7 -> 13.3 and 17.3 -> 15.9, of 4,096 29.0 -> 27.3 and 32.0 -> 29.5; 600 of 2,048
+    // 11.9 -> 10.8 and 14.9 -> 13.3; 1,280 of 1,024 12.5 -> 11.9 and 15.8 -> 15.1.  An eighth and less is even: seven tiles from eight 42.4 -> 42.0
+    // (1,700 of 4,096) and 40.3 -> 41.9 (1,792 of 4,096), nine from ten 30.7 -> 31.7 (2,300 of 2,048).
+    if (p.S == 1 && p.per_cu == 2 && groups > cus) {
+        const int old = busiest_unit(ntiles, groups, cus);
+        int few = groups, least = old;
+        for (int g = groups + 1; g <= most; g++) {
+            const int n = busiest_unit(ntiles, g, cus);
+            if (n < least) few = g, least = n;
+        }
+        if (8 * (old - least) > old) groups = few;
+    }
     return groups;       // the grid is groups * S
 }
 
