@@ -394,12 +394,12 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
             if (TM == TM_GATEUP) row += (r >> 3) * n_out;
             const int kb = begin_of(l_j), ke = end_of(l_j);
             if (WT) {
-                // tile-major weights (fllm_tile_weights, one slice): the 16 rows x 32 columns of a k-step lie together in the order
+                // tile-major weights (fllm_tile_weights): the 16 rows x 32 columns of a k-step lie together in the order
                 // the lanes take them, so a load instruction reads 1 KiB in a row instead of 64 bytes of each of 16 rows.
                 // A tile of 8 rows is half of a copied one: 128 bytes of each quarter of the k-steps of both K halves.
                 const int tile = tile0 + l_item * tstride;
                 const int tile16 = TM == TM_DUALK ? tile >> 1 : tile, row16 = TM == TM_DUALK ? (tile & 1) * 8 + (r & 7) : r;
-                const bf16_t *wp = a.w_tiles + (size_t)tile16 * 16 * K + (size_t)((kb - g * 8) / 32) * (16 * 32) + (g * 16 + row16) * 8;
+                const bf16_t *wp = a.w_tiles + (size_t)tile16 * 16 * K + (size_t)((ks0 + kb - g * 8) / 32) * (16 * 32) + (g * 16 + row16) * 8;
 #pragma unroll
                 for (int u = 0; u < U; u++) buf.w[u] = kb + u * 32 < ke ? load_weights<true>(wp + u * (16 * 32)) : zero8();
             } else {
@@ -440,7 +440,7 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
     EpilogueOperands eo;
     load_row_operands<EPI>(a, m_out, eo);
     auto item_operands = [&](int it) {
-        if (S == 1 && it < my_items && wave == (it & (WAVES - 1)) && owner)
+        if (it < my_items && wave == (it & (WAVES - 1)) && owner)
             load_item_operands<EPI>(a, m_out, (tile0 + it * tstride) * NT + g * 4, n_out, eo);
     };
     item_operands(0);
@@ -577,19 +577,17 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
                     for (int wv = 0; wv < WAVES; wv++) ss += ssq_part[wv * 16 + m];
                 }
                 if (S > 1) {
-                    float *part = a.ws + ((size_t)(tile * S + sl) * RT * kWave + lane) * 4;
+                    const __amdgpu_buffer_rsrc_t wsb = workspace_buffer(a.ws);
+                    const unsigned int part = (unsigned int)(((tile * S + sl) * RT * kWave + lane) * 16);      // tiles are counted in 64 KiB: below 2 GiB
                     if (owner && m < M) {
 #pragma unroll
-                        for (int t = 0; t < RT; t++)
-#pragma unroll
-                            for (int i = 0; i < 4; i++)
-                                __hip_atomic_store(part + t * kWave * 4 + i, s[t][i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        for (int t = 0; t < RT; t++) hand_over(wsb, part + t * kWave * 16, s[t]);
                         if (PRO != PRO_BF16 && g == 0)
                             __hip_atomic_store(a.ws_ssq + (size_t)(tile * S + sl) * 16 + m, ss, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     }
-                    // Every access to the workspace goes to the device's point of coherence by itself (agent-scope
-                    // atomics), so no cache has to be written back or dropped: it is enough that the wave's partial
-                    // sums have arrived there before the item is counted.
+                    // Every access to the workspace goes to the device's point of coherence by itself (past the caches, or
+                    // agent-scope atomics), so no cache has to be written back or dropped: it is enough that the wave's
+                    // partial sums have arrived there before the item is counted.
                     parts_published();
                     int seen = 0;
                     if (lane == 0) seen = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -603,32 +601,28 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
                     ss = 0.f;
                     // four slices at a time: their loads are all asked for before the first is added (in slice order)
                     for (int s0 = 0; s0 < S; s0 += 4) {
-                        float pv[4][RT][4], ps[4];
+                        f32x4_t pv[4][RT];
+                        float ps[4];
 #pragma unroll
                         for (int j = 0; j < 4; j++) {
                             const bool live = s0 + j < S;
-                            const float *src = a.ws + ((size_t)(tile * S + (live ? s0 + j : s0)) * RT * kWave + lane) * 4;
+                            const unsigned int src = (unsigned int)(((tile * S + (live ? s0 + j : s0)) * RT * kWave + lane) * 16);
 #pragma unroll
-                            for (int t = 0; t < RT; t++)
-#pragma unroll
-                                for (int i = 0; i < 4; i++)
-                                    pv[j][t][i] = live ? __hip_atomic_load(src + t * kWave * 4 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
+                            for (int t = 0; t < RT; t++) pv[j][t] = take_over(wsb, src + t * kWave * 16);
                             ps[j] = (PRO != PRO_BF16 && live)
                                         ? __hip_atomic_load(a.ws_ssq + (size_t)(tile * S + s0 + j) * 16 + m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
                                         : 0.f;
                         }
 #pragma unroll
                         for (int j = 0; j < 4; j++) {
+                            if (s0 + j >= S) continue;
 #pragma unroll
-                            for (int t = 0; t < RT; t++)
-#pragma unroll
-                                for (int i = 0; i < 4; i++) s[t][i] += pv[j][t][i];
+                            for (int t = 0; t < RT; t++) s[t] += pv[j][t];
                             ss += ps[j];
                         }
                     }
                 }
                 if (!owner || m >= M || nb >= n_out) break;
-                if (S > 1) eo.have = false;     // the tile was finished by whoever came last: nothing was asked for ahead
                 epilogue<PRO, EPI, RT>(a, s, ss, m, nb, n_out, eo);
             } while (false);
         }
@@ -1319,8 +1313,10 @@ __global__ void __launch_bounds__(256) tile_weights_kernel(const bf16_t *__restr
     }
 }
 
-// Whether a launch may stream the tile-major copy: there is one, and K is not cut into slices
-bool streams_tiles(const SkinnyArgs &a, const ResidentPlan &p, int n_out) { return a.w_tiles != nullptr && p.S == 1 && tiles_fit(n_out, a.K); }
+// Whether a launch may stream the tile-major copy: there is one, and K is not cut into slices to stage them (`stage` is 0 where nothing is)
+bool streams_tiles(const SkinnyArgs &a, const ResidentPlan &p, int n_out) {
+    return a.w_tiles != nullptr && (p.S == 1 || p.stage == 0) && tiles_fit(n_out, a.K);
+}
 
 template <int PRO, int EPI, int TM, bool XD>
 int launch_resident_form(const SkinnyArgs &a, const ResidentPlan &p, int ntiles, bool tiled, const Workspace &ws, hipStream_t stream) {
@@ -1356,6 +1352,7 @@ int launch_resident(const SkinnyArgs &a, hipStream_t stream) {
         const bool x_direct = PRO == PRO_BF16 && fllm_option_x_direct() && a.ldx % 8 == 0 && tiles16 <= 4 * device_cus();
         ResidentPlan p = plan_resident(a.M, a.K, tiles16, RT, ws, x_direct);
         if (p.S == 0) return 1;
+        if (x_direct) fllm_plan::slice_direct(p, a.M, a.K, tiles16, RT, ws.bytes, ws.base != nullptr, device_cus());
         // 8-row tiles (two K halves a product) when the rows allow it and the 16-row tiles come to between half a
         // tile and two tiles per slot, unevenly: 384 tiles on 512 slots run as long as 512 would.  Also when the 16-row
         // tiles fill no more than half of the compute units (narrow models): twice the workgroups, each with half the
