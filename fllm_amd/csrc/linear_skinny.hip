@@ -142,11 +142,20 @@ struct EpilogueOperands {
 };
 
 template <int EPI>
-__device__ __forceinline__ void load_row_operands(const SkinnyArgs &a, int m, EpilogueOperands &e) {
+__device__ __forceinline__ void load_row_place(const SkinnyArgs &a, int m, EpilogueOperands &e) {
     if (EPI != EPI_QKV || m >= a.M) return;
     e.seg = a.row_seg[m];
     e.pos = a.row_pos[m];
+}
+template <int EPI>
+__device__ __forceinline__ void load_row_page(const SkinnyArgs &a, int m, EpilogueOperands &e) {
+    if (EPI != EPI_QKV || m >= a.M) return;
     if (e.seg >= 0 && a.store_kv) e.page = a.tables[(size_t)e.seg * a.table_stride + e.pos / a.page_size];
+}
+template <int EPI>
+__device__ __forceinline__ void load_row_operands(const SkinnyArgs &a, int m, EpilogueOperands &e) {
+    load_row_place<EPI>(a, m, e);
+    load_row_page<EPI>(a, m, e);
 }
 
 template <int EPI>
@@ -431,14 +440,15 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
 #endif
     constexpr int NB = XD ? 2 : FLLM_BLOCKS_IN_FLIGHT;      // blocks of weights a wave has asked for ahead of its products
     Block bl[NB];
+    const int m_out = TM == TM_DUALK ? (r & 7) : r;
+    EpilogueOperands eo;
+    load_row_place<EPI>(a, m_out, eo);      // ahead of the weights: loads come back in their order, and the page waits for these
 #pragma unroll
     for (int i = 0; i < NB; i++) issue(bl[i]);      // in flight while the activations are staged
     // what the epilogue reads besides the sums: the part that belongs to this lane's row now, the part that belongs
     // to an item when the wave whose turn it is to finish the item starts on it
-    const int m_out = TM == TM_DUALK ? (r & 7) : r;
     const bool owner = WHOLE ? true : (g < 2 && (TM == TM_GATEUP || r < 8));
-    EpilogueOperands eo;
-    load_row_operands<EPI>(a, m_out, eo);
+    load_row_page<EPI>(a, m_out, eo);
     auto item_operands = [&](int it) {
         if (it < my_items && wave == (it & (WAVES - 1)) && owner)
             load_item_operands<EPI>(a, m_out, (tile0 + it * tstride) * NT + g * 4, n_out, eo);
@@ -458,21 +468,39 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
             if (lane == 0) ssq_part[wave * 16 + m] = t;
         }
     }
-    for (int cw = kw0; cw < (XD ? 0 : kw1); cw += kWave * 8) {   // the same trips for every lane: the sums below are over the wave
-        const int c0 = cw + lane * 8;
-        const bool in = c0 < kw1;
-        if (PRO != PRO_NORM_F32) {
-            const bf16_t *x = (const bf16_t *)a.x + ks0 + c0;
-            for (int m0 = 0; m0 < M; m0 += 4) {
-                bf16x8_t v[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (in && m0 + i < M) v[i] = *(const bf16x8_t *)(x + (size_t)(m0 + i) * a.ldx);
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (in && m0 + i < M) *(bf16x8_t *)(xs + (m0 + i) * pitch + c0) = v[i];
+    if constexpr (!XD && PRO != PRO_NORM_F32) {
+        // Ranges of 256 and 128 columns take two and four rows a load instruction, four instructions are on their way at a time: a trip to L2 takes
+        // eight or sixteen rows where one row an instruction was four.  Microseconds at 16 rows behind a prepared norm: q/k/v 3,072 x 2,048
+        // 8.8 -> 7.7, 2,048 x 1,536 8.1 -> 7.3, gate/up 2 x 8,192 x 2,048 17.1 -> 15.8, 2 x 8,960 x 1,536 15.6 -> 14.1; the vocabulary 24,576 x 1,536 at 8
+        // rows 16.7 -> 15.7.  Eight instructions were no faster there and slower for ranges of 512 (6,144 x 4,096 at 8 rows 12.2 -> 12.8).
+        constexpr int RX = 4;
+        const int at = kwlen <= 128 ? 4 : kwlen <= 256 ? 5 : 6, rows_at = kWave >> at;      // lanes a row (its logarithm), rows an instruction
+        const int own = lane >> at, col = (lane & ((1 << at) - 1)) * 8;
+        for (int cw = kw0; cw < kw1; cw += 8 << at) {
+            const int c0 = cw + col;
+            const bool in = c0 < kw1;
+            const bf16_t *x = (const bf16_t *)a.x + ks0 + (in ? c0 : kw0);
+            if (M <= rows_at) {
+                if (in && own < M) *(bf16x8_t *)(xs + own * pitch + c0) = *(const bf16x8_t *)(x + (size_t)own * a.ldx);
+                continue;
             }
-        } else {
+            for (int m0 = 0; m0 < M; m0 += RX * rows_at) {
+                bf16x8_t v[RX];
+#pragma unroll
+                for (int i = 0; i < RX; i++)
+                    if (m0 + i * rows_at < M) v[i] = *(const bf16x8_t *)(x + (size_t)min(m0 + i * rows_at + own, M - 1) * a.ldx);
+#pragma unroll
+                for (int i = 0; i < RX; i++) {
+                    const int m = m0 + i * rows_at + own;
+                    if (in && m < M) *(bf16x8_t *)(xs + m * pitch + c0) = v[i];
+                }
+            }
+        }
+    }
+    if constexpr (PRO == PRO_NORM_F32)
+        for (int cw = kw0; cw < kw1; cw += kWave * 8) {   // the same trips for every lane: the sums below are over the wave
+            const int c0 = cw + lane * 8;
+            const bool in = c0 < kw1;
             const float *x = (const float *)a.x + ks0 + c0;
             f32x4_t w0 = {0.f, 0.f, 0.f, 0.f}, w1 = w0;
             if (in) w0 = *(const f32x4_t *)(a.norm_w + ks0 + c0), w1 = *(const f32x4_t *)(a.norm_w + ks0 + c0 + 4);
@@ -486,24 +514,33 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
                         xv[i][1] = *(const f32x4_t *)(x + (size_t)(m0 + i) * a.ldx + 4);
                     }
                 }
+                float ss[RB];
 #pragma unroll
                 for (int i = 0; i < RB; i++) {
-                    if (m0 + i >= M) break;
                     bf16x8_t v;
-                    float ss = 0.f;
+                    ss[i] = 0.f;
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        ss += xv[i][0][e] * xv[i][0][e] + xv[i][1][e] * xv[i][1][e];
+                        ss[i] += xv[i][0][e] * xv[i][0][e] + xv[i][1][e] * xv[i][1][e];
                         v[e] = (bf16_t)(xv[i][0][e] * w0[e]);
                         v[4 + e] = (bf16_t)(xv[i][1][e] * w1[e]);
                     }
-                    if (in) *(bf16x8_t *)(xs + (m0 + i) * pitch + c0) = v;
-                    ss = wave_sum(ss);
-                    if (lane == 0) ssq_part[wave * 16 + m0 + i] += ss;
+                    if (in && m0 + i < M) *(bf16x8_t *)(xs + (m0 + i) * pitch + c0) = v;
                 }
+                // The rows' sums side by side: each is six dependent trips through LDS.  Microseconds one by one -> side by side at 4 / 8 / 16
+                // rows: 3,072 x 2,048 7.0 -> 6.6 / 8.7 -> 7.8 / 12.1 -> 10.1, gate/up of 2 x 8,192 x 2,048 15.9 -> 14.7 / 17.6 -> 17.4 / 21.2 -> 20.8.
+                if (M == 1) ss[0] = wave_sum(ss[0]);
+                else
+#pragma unroll
+                    for (int o = kWave / 2; o > 0; o >>= 1)
+#pragma unroll
+                        for (int i = 0; i < RB; i++) ss[i] += __shfl_xor(ss[i], o, kWave);
+                if (lane == 0)
+#pragma unroll
+                    for (int i = 0; i < RB; i++)
+                        if (m0 + i < M) ssq_part[wave * 16 + m0 + i] += ss[i];
             }
         }
-    }
     if (PRO == PRO_SCALED && ssq_quick && sl == 0) {
 #pragma unroll
         for (int k = 0; k < 2; k++) {
@@ -621,6 +658,10 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
                             ss += ps[j];
                         }
                     }
+                    // Parts of slices that are not there have been asked for and not used: without this wait the compiler, which takes their
+                    // registers for a block's activations, waits for all loads ahead of reading those from LDS, sliced or not
+                    // (14,336 x 2 x 4,096 at one row 42.5 -> 44.3 us).
+                    __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0)
                 }
                 if (!owner || m >= M || nb >= n_out) break;
                 epilogue<PRO, EPI, RT>(a, s, ss, m, nb, n_out, eo);
