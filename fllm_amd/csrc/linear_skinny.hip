@@ -790,6 +790,12 @@ skinny_wide_kernel(SkinnyArgs a) {
 #pragma unroll
         for (int i = 0; i < SQ; i++) sq[PRO == PRO_SCALED ? i : 0] = *(const f32x4_t *)(sq0 + 4 * i < sq1 ? sq_parts + sq0 + 4 * i : (const float *)zeros);
     }
+    // segment, position and page of this lane's rows: the same for every item.  The pages wait for the rest, which is asked for first of all.
+    EpilogueOperands rows[DEEP ? MT : 1];
+    if (DEEP) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) load_row_place<EPI>(a, mt * 16 + r, rows[mt]);
+    }
     bf16x8_t wa[KS], wb[KS], xa[XL], xb[XL];
     const int second = nchunks > 1 ? 1 : 0;
     load_x(xa, 0);
@@ -798,6 +804,10 @@ skinny_wide_kernel(SkinnyArgs a) {
     issue_w(wa);
     issue_w(wb);
     __builtin_amdgcn_sched_barrier(0);
+    if (DEEP) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) load_row_page<EPI>(a, mt * 16 + r, rows[mt]);
+    }
     if (PRO == PRO_SCALED) {
         // A row's sum of squares arrives in parts (up to a few hundred).  Four neighbouring threads share a row: each adds
         // a quarter of the parts in index order, and the quarters are added in order: the same sum for a row whatever the
@@ -834,11 +844,6 @@ skinny_wide_kernel(SkinnyArgs a) {
     store_x(xa, 0);
     __syncthreads();
 
-    EpilogueOperands rows[DEEP ? MT : 1];       // segment, position and page of this lane's rows: the same for every item
-    if (DEEP) {
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) load_row_operands<EPI>(a, mt * 16 + r, rows[mt]);
-    }
     f32x4_t acc[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) acc[mt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
@@ -1454,8 +1459,8 @@ int launch_wide(SkinnyArgs a, hipStream_t stream) {
     // prepared norm has four threads a row)
     const fllm_plan::ChunkPlan p =
         MT > 4 ? fllm_plan::plan_chunks(a.K, ntiles, MT, RT, bytes, have_ws, device_cus(), fllm_option_linear_slices(), 8)
-        : tiled ? fllm_plan::plan_chunks_balanced(a.K, ntiles, MT, RT, bytes, have_ws, device_cus(), fllm_option_linear_slices(),
-                                                  fllm_option_wide_waves())
+        : tiled ? fllm_plan::plan_chunks_even(a.K, ntiles, MT, RT, bytes, have_ws, device_cus(), fllm_option_linear_slices(),
+                                              fllm_option_wide_waves())
                 : fllm_plan::plan_chunks(a.K, ntiles, MT, RT, bytes, have_ws, device_cus(), fllm_option_linear_slices(), 4);
     a.S = p.S;
     a.slice = p.slice;
@@ -1475,6 +1480,7 @@ int launch_wide(SkinnyArgs a, hipStream_t stream) {
     } else {
         if constexpr (kHasTiles) {
             if (tiled) {
+                if (p.waves == 6) return launch_wide_kernel<MT, EPI, true, 6, PRO>(a, p.grid, stream);
                 if (p.waves == 7) return launch_wide_kernel<MT, EPI, true, 7, PRO>(a, p.grid, stream);
                 if (p.waves == 8) return launch_wide_kernel<MT, EPI, true, 8, PRO>(a, p.grid, stream);
                 return launch_wide_kernel<MT, EPI, true, 4, PRO>(a, p.grid, stream);

@@ -76,7 +76,7 @@ extern "C" int fllm_set_option(const char *name, int value) {
         return 0;
     }
     if (strcmp(name, "linear.wide_waves") == 0) {
-        g_wide_waves = (value == 4 || value == 7 || value == 8) ? value : 0;
+        g_wide_waves = value == 4 || (value >= 6 && value <= 8) ? value : 0;
         return 0;
     }
     if (strcmp(name, "linear.x_direct") == 0) {
