@@ -99,8 +99,8 @@ __device__ __forceinline__ void softmax_step(f32x4_t (&s)[NS], float &m_run, flo
     for (int t = 0; t < NS; t++)
 #pragma unroll
         for (int i = 0; i < 4; i++) tmax = fmaxf(tmax, s[t][i]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+    tmax = max_16_apart(tmax);
+    tmax = max_32_apart(tmax);
     const float m_new = fmaxf(m_run, tmax);
     alpha = (m_run == -INFINITY) ? 0.f : fast_exp2(m_run - m_new);
     float psum = 0.f;
@@ -112,8 +112,8 @@ __device__ __forceinline__ void softmax_step(f32x4_t (&s)[NS], float &m_run, flo
             s[t][i] = p;
             psum += p;
         }
-    psum += __shfl_xor(psum, 16, kWave);
-    psum += __shfl_xor(psum, 32, kWave);
+    psum = sum_16_apart(psum);
+    psum = sum_32_apart(psum);
     l_run = l_run * alpha + psum;
     m_run = m_new;
 }
@@ -501,7 +501,7 @@ attn_tile32_kernel(AttnArgs p) {
         for (int rb = 0; rb < 2; rb++)
 #pragma unroll
             for (int i = 0; i < 16; i++) tmax = fmaxf(tmax, s[rb][i]);
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+        tmax = max_32_apart(tmax);
         // The reference point of the exponents follows the maximum only when that has grown by more than 2^8 in the
         // exponent's units: until then the probabilities are at most 256 times their final size, which float32 sums and
         // bfloat16 operands hold as well, and the outputs need no rescaling (with it at every new maximum, short
@@ -518,7 +518,7 @@ attn_tile32_kernel(AttnArgs p) {
                 s[rb][i] = pv;
                 psum += pv;
             }
-        psum += __shfl_xor(psum, 32, kWave);
+        psum = sum_32_apart(psum);
         l_run = l_run * alpha + psum;
         m_run = m_new;
         if (__any(alpha != 1.0f)) {   // once the maximum has settled the outputs need no rescaling

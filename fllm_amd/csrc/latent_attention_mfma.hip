@@ -122,8 +122,8 @@ latent_rows_kernel(const LatentParams p) {
             s[i] = key >= lo && key <= pos ? (st[0][i] + st[1][i]) * p.scale_log2 : -INFINITY;
             m_blk = fmaxf(m_blk, s[i]);
         }
-        m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 16, kWave));
-        m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 32, kWave));
+        m_blk = max_16_apart(m_blk);
+        m_blk = max_32_apart(m_blk);
         if (g == 0) sm_m[wave * 16 + c] = m_blk;
         __syncthreads();
         float m_new = m_run;
@@ -163,8 +163,8 @@ latent_rows_kernel(const LatentParams p) {
             }
         }
     }
-    l_run += __shfl_xor(l_run, 16, kWave);
-    l_run += __shfl_xor(l_run, 32, kWave);
+    l_run = sum_16_apart(l_run);
+    l_run = sum_32_apart(l_run);
     if (g == 0) sm_l[wave * 16 + c] = l_run;
     __syncthreads();
     float l = 0.f;

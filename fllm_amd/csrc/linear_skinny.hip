@@ -527,14 +527,8 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
                     }
                     if (in && m0 + i < M) *(bf16x8_t *)(xs + (m0 + i) * pitch + c0) = v;
                 }
-                // The rows' sums side by side: each is six dependent trips through LDS.  Microseconds one by one -> side by side at 4 / 8 / 16
-                // rows: 3,072 x 2,048 7.0 -> 6.6 / 8.7 -> 7.8 / 12.1 -> 10.1, gate/up of 2 x 8,192 x 2,048 15.9 -> 14.7 / 17.6 -> 17.4 / 21.2 -> 20.8.
-                if (M == 1) ss[0] = wave_sum(ss[0]);
-                else
 #pragma unroll
-                    for (int o = kWave / 2; o > 0; o >>= 1)
-#pragma unroll
-                        for (int i = 0; i < RB; i++) ss[i] += __shfl_xor(ss[i], o, kWave);
+                for (int i = 0; i < RB; i++) ss[i] = wave_sum(ss[i]);
                 if (lane == 0)
 #pragma unroll
                     for (int i = 0; i < RB; i++)

@@ -293,8 +293,8 @@ masked_rows_kernel(const MaskedParams p) {
             for (int b = 0; b < 2; b++)
 #pragma unroll
                 for (int e = 0; e < 8; e++) m_blk = fmaxf(m_blk, s[b][e]);
-            m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 16, kWave));
-            m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 32, kWave));
+            m_blk = max_16_apart(m_blk);
+            m_blk = max_32_apart(m_blk);
             m_new = fmaxf(m_run, m_blk);
         }
         if (!fixed && __any(m_new > m_run)) {      // the outputs are rescaled only when some row's maximum moved
@@ -316,8 +316,8 @@ masked_rows_kernel(const MaskedParams p) {
             }
         }
     }
-    l_run += __shfl_xor(l_run, 16, kWave);
-    l_run += __shfl_xor(l_run, 32, kWave);
+    l_run = sum_16_apart(l_run);
+    l_run = sum_32_apart(l_run);
     if (!valid) return;
     if (p.zero_sink) l_run += fast_exp2(-m_run);
     if (p.sinks != nullptr) l_run += fast_exp2(p.sinks[head] * kLog2e - m_run);
@@ -411,8 +411,8 @@ masked_heads_kernel(const MaskedParams p) {
                 if (base + g * 8 + e > pos)
 #pragma unroll
                     for (int t = 0; t < NV * VT; t++) va[t][e] = (bf16_t)0.f;
-        m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 16, kWave));
-        m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 32, kWave));
+        m_blk = max_16_apart(m_blk);
+        m_blk = max_32_apart(m_blk);
         const float m_new = fmaxf(m_run, m_blk);
         const float alpha = m_run == -INFINITY ? 0.f : fast_exp2(m_run - m_new);
         bf16x8_t hi, lo8;
@@ -425,8 +425,8 @@ masked_heads_kernel(const MaskedParams p) {
             o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[t], lo8, o[t], 0, 0, 0);
         }
     }
-    l_run += __shfl_xor(l_run, 16, kWave);
-    l_run += __shfl_xor(l_run, 32, kWave);
+    l_run = sum_16_apart(l_run);
+    l_run = sum_32_apart(l_run);
     if (g == 0) sm_m[wave][qi] = m_run, sm_l[wave][qi] = l_run;
     float *part = p.parts + (((size_t)row * gridDim.y + blockIdx.y) * p.splits + blockIdx.z) * (16 * W + 32);
 #pragma unroll

@@ -151,8 +151,8 @@ mixer_tile_kernel(const TileParams p) {
                     s[j][i] = visible(g * 8 + j * 4 + i) ? s[j][i] * sc : -INFINITY;
                     m_blk = fmaxf(m_blk, s[j][i]);
                 }
-            m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 16, kWave));
-            m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 32, kWave));
+            m_blk = max_16_apart(m_blk);
+            m_blk = max_32_apart(m_blk);
             const float m_new = fmaxf(m_run, m_blk);
             const float alpha = m_run == -INFINITY ? 0.f : fast_exp(m_run - m_new);
             float sum = 0.f;
@@ -287,8 +287,8 @@ mixer_tile_kernel(const TileParams p) {
     }
     // ---- the waves meet
     if (VARIANT == 0) {
-        l_run += __shfl_xor(l_run, 16, kWave);
-        l_run += __shfl_xor(l_run, 32, kWave);
+        l_run = sum_16_apart(l_run);
+        l_run = sum_32_apart(l_run);
         if (g == 0) sm_m[wave][qi] = m_run, sm_l[wave][qi] = l_run;
     }
 #pragma unroll

@@ -258,9 +258,9 @@ linear_attention_rows_kernel(const T *__restrict__ q, const T *__restrict__ k, c
         }
 #pragma unroll
         for (int e = 0; e < 4; e++) {      // the eight row groups of a wave: lanes 8, 16 and 32 apart hold the same columns
-            acc[e] += __shfl_xor(acc[e], 8, kWave);
-            acc[e] += __shfl_xor(acc[e], 16, kWave);
-            acc[e] += __shfl_xor(acc[e], 32, kWave);
+            acc[e] += along_row<8>(acc[e]);
+            acc[e] = sum_16_apart(acc[e]);
+            acc[e] = sum_32_apart(acc[e]);
         }
         if ((tid & (kWave - 1)) < 8) part[tid / kWave][j4] = acc;
         __syncthreads();

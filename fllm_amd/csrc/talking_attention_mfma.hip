@@ -291,8 +291,8 @@ talking_tile_kernel(const TalkArgs p) {
         for (int h = 0; h < HMAX; h++) {
             if (h < H) {
                 float v = fmaxf(fmaxf(s[h][0], s[h][1]), fmaxf(s[h][2], s[h][3]));
-                v = fmaxf(v, __shfl_xor(v, 16, kWave));
-                v = fmaxf(v, __shfl_xor(v, 32, kWave));
+                v = max_16_apart(v);
+                v = max_32_apart(v);
                 mx[(h * kTileRows + c) * 8 + wave] = v;      // the four lanes of a row hold the same
             }
         }
@@ -359,8 +359,8 @@ talking_tile_kernel(const TalkArgs p) {
     for (int h = 0; h < HMAX; h++) {
         if (h < H) {
             float v = l_part[h];
-            v += __shfl_xor(v, 16, kWave);
-            v += __shfl_xor(v, 32, kWave);
+            v = sum_16_apart(v);
+            v = sum_32_apart(v);
             if (g == 0) mx[(h * kTileRows + c) * 8 + wave] = v;
         }
     }
@@ -591,9 +591,7 @@ talking_decode_kernel(const TalkArgs p) {
                 mx[j] = sc[j];
             }
 #pragma unroll
-            for (int d = 32; d >= 1; d >>= 1)
-#pragma unroll
-                for (int j = 0; j < HW; j++) mx[j] = fmaxf(mx[j], __shfl_xor(mx[j], d, kWave));
+            for (int j = 0; j < HW; j++) mx[j] = wave_max(mx[j]);
             float alpha[HW];
 #pragma unroll
             for (int j = 0; j < HW; j++) {
@@ -609,9 +607,7 @@ talking_decode_kernel(const TalkArgs p) {
                 }
             }
 #pragma unroll
-            for (int d = 32; d >= 1; d >>= 1)
-#pragma unroll
-                for (int j = 0; j < HW; j++) sum[j] += __shfl_xor(sum[j], d, kWave);
+            for (int j = 0; j < HW; j++) sum[j] = wave_sum(sum[j]);
 #pragma unroll
             for (int j = 0; j < HW; j++) l_run[j] = l_run[j] * alpha[j] + sum[j];
         }
