@@ -16,7 +16,7 @@ def test_every_lane_counts_once(width):
     x = torch.diag(value).cuda()
     weight = (torch.rand(width, generator=gen) + 0.5).cuda()
     out = torch.full((width, width), float("nan"), device="cuda")
-    ops.rmsnorm(x, weight, 0.0, out)
+    ops.rmsnorm(x, weight, 1e-30, out)
     want = torch.diag(weight.double() * width ** 0.5)
     assert ((out.double() - want).abs() <= 2.0 ** -21 * want).all()
 
@@ -34,5 +34,5 @@ def test_every_lane_counts_once_in_a_product(rows, K):
         x = torch.zeros((rows, K), device="cuda")
         for r in range(rows):
             x[r, places[(at + r) % len(places)]] = 1.0
-        ops.norm_linear(x, torch.ones(K, device="cuda"), 0.0, w, out)
+        ops.norm_linear(x, torch.ones(K, device="cuda"), 1e-30, w, out)
         assert (out.float() - K ** 0.5).abs().max() <= 2.0 ** -8 * K ** 0.5
