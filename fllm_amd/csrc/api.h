@@ -16,7 +16,7 @@ int fllm_abi_version(void);
 void fllm_set_fast_kernels(int on);
 // Switches a kernel variant (for measurements and tests): "attention.tile32" 0/1; "linear.slices" n
 // (0: chosen by shape); "linear.dual_k" 0/1; "linear.x_direct" 0/1; "attention.fused_merge" 0/1;
-// "attention.prefill_parts" 0/1; "linear.slab" 0/1/2; "linear.wide_waves" 0 (planned)/4/6/7/8; "linear.resident_tiles" 0/1;
+// "attention.prefill_parts" 0/1; "linear.slab" 0/1/2; "linear.wide_waves" 0 (planned)/4/6/7/8; "linear.tile_slices" 0 (never)/1 (planned)/2 to 8; "linear.resident_tiles" 0/1;
 // "attention.tile32_rows" 0 (chosen by the launch)/128/256.  0 on success.
 int fllm_set_option(const char *name, int value);
 
@@ -462,7 +462,8 @@ int fllm_experts_grouped_ungated(const void *h, int ldh, const int32_t *ids, int
                                  hipStream_t stream);
 
 // Products of many bfloat16 rows on 256- and 128-row tiles (gemm_tiles.h).  0: launched, 1: declined (sizes that are no multiples of the
-// tiles' pieces, or with `force` 0 shapes that the general path is faster at).  fllm_linear_tiles: mode 0 stores, 2 the squared ReLU.
+// tiles' pieces, or with `force` 0 shapes that the general path is faster at).  fllm_linear_tiles: mode 0 stores, 1 stores
+// float32 (K in slices alone: declined otherwise), 2 the squared ReLU.
 int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up, void *out, int M, int inter, int K, float limit, float alpha,
                        float up_offset, int force, hipStream_t stream);
 int fllm_linear_tiles(const void *x, int ldx, const void *w, const float *bias, void *out, int ldo, int M, int N, int K, int mode, int force,

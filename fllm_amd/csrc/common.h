@@ -42,6 +42,7 @@ int fllm_option_resident_tiles(void);
 int fllm_option_tile32_rows(void);
 // 1: decode-shaped products of up to 8 rows use 8-row weight tiles with two K halves a product (default); 0: 16-row tiles
 int fllm_option_dual_k(void);
+int fllm_option_tile_slices(void);
 
 // The device workspace of the current device (fllm_set_device_workspace): its first kWorkspaceCounterBytes are
 // counters that every kernel leaves at zero, the rest is for partial results of the kernel that is running.
@@ -83,6 +84,24 @@ __device__ __forceinline__ void parts_visible() { __builtin_amdgcn_fence(__ATOMI
             return -1;                     \
         }                                  \
     } while (0)
+
+// Partial sums that workgroups hand to each other go through the device workspace in 16-byte pieces that pass by the
+// caches of the compute units and of their die on both ways (the sc0 sc1 forms of the buffer instructions: written
+// through to memory, read from memory), as device-scope atomics do for single words.  The workspace is one buffer
+// for these instructions; offsets are in bytes from its base.
+typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
+constexpr int kThroughCaches = 17;        // cache policy bits sc0 (1) and sc1 (16)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t workspace_buffer(float *base) {
+    return __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00020000);      // raw buffer, offsets up to 2 GiB
+}
+__device__ __forceinline__ void hand_over(__amdgpu_buffer_rsrc_t ws, unsigned int byte_offset, f32x4_t v) {
+    u32x4_t bits = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+    __builtin_amdgcn_raw_buffer_store_b128(bits, ws, byte_offset, 0, kThroughCaches);
+}
+__device__ __forceinline__ f32x4_t take_over(__amdgpu_buffer_rsrc_t ws, unsigned int byte_offset) {
+    const u32x4_t bits = __builtin_amdgcn_raw_buffer_load_b128(ws, byte_offset, 0, kThroughCaches);
+    return (f32x4_t){__uint_as_float(bits[0]), __uint_as_float(bits[1]), __uint_as_float(bits[2]), __uint_as_float(bits[3])};
+}
 
 // Where a key's value lies in the pages.  Inside a page the keys of a key/value head are stored chunk by chunk:
 // [kv_head][head_dim / 8][token][8], so that the 8 neighbouring values (16 bytes in bfloat16) of all tokens of the page lie

@@ -22,7 +22,7 @@
 
 namespace fllm_tiles {
 
-enum { EPI_STORE = 0, EPI_GLU = 1, EPI_RELU2 = 2, EPI_F32 = 3 };      // EPI_F32: grouped products alone
+enum { EPI_STORE = 0, EPI_GLU = 1, EPI_RELU2 = 2, EPI_F32 = 3 };      // EPI_F32: grouped and sliced products alone
 
 struct TileArgs {
     const bf16_t *x;        // rows, row stride ldx (a multiple of 8)
@@ -35,6 +35,10 @@ struct TileArgs {
     const int32_t *work;    // null: the rows of x as they are
     int max_tiles;
     int top;                // the row of x a pair reads: > 0 pair / top, 0 its slot, -1 the pair
+    // K cut into slices, a workgroup each (128-row tiles): the tiles' parts [tile][slice][128 x 256 floats] and a counter a tile, zero between launches
+    int slices;
+    float *parts;
+    int *counters;
     int halves;             // the 256-row kernel: whether a last round of at most 128 tiles runs as tiles of half the rows
 };
 
@@ -309,17 +313,49 @@ __device__ __forceinline__ void tiles256(const TileArgs &a) {
 #undef FLLM_STEP
 }
 
+// The slices of a 128-row tile meet: every workgroup leaves its sums in the device workspace and counts the tile, the one that counts last goes on
+// with the sum of all in slice order (so it does not matter which one that is), the others are done: false.  Nobody waits for another.
+__device__ __forceinline__ bool meet_slices(const TileArgs &a, int tile, int slice, f32x4_t (&acc)[2][4][2], int *seen) {
+    const __amdgpu_buffer_rsrc_t parts = workspace_buffer(a.parts);
+    const unsigned int part = 128 * 256 * 4, mine = threadIdx.x * 16;      // bytes; 256 workgroups at most: 32 MiB
+    const unsigned int first = (unsigned int)tile * a.slices * part + mine;
+#pragma unroll
+    for (int p = 0; p < 16; p++) hand_over(parts, first + slice * part + p * kThreads * 16, acc[p >> 3][(p >> 1) & 3][p & 1]);
+    parts_published();
+    __syncthreads();
+    if (threadIdx.x == 0) *seen = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (*seen != a.slices - 1) return false;
+    parts_visible();
+    if (threadIdx.x == 0) __hip_atomic_store(a.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // for the next launch
+    f32x4_t sum[16];
+    for (int s = 0; s < a.slices; s++) {
+        f32x4_t v[16];
+#pragma unroll
+        for (int p = 0; p < 16; p++) v[p] = take_over(parts, first + s * part + p * kThreads * 16);
+#pragma unroll
+        for (int p = 0; p < 16; p++) sum[p] = s == 0 ? v[p] : sum[p] + v[p];
+    }
+#pragma unroll
+    for (int p = 0; p < 16; p++) acc[p >> 3][(p >> 1) & 3][p & 1] = sum[p];
+    return true;
+}
+
 // 128 x 256 (EPI_GLU: 128 x 128), for launches whose 256-row tiles would leave much of the device idle: an operand read from LDS serves half
 // the products, so LDS and the matrix cores are busy alike.  LDS: three buffers of [x][W half 0][W half 1].  K step k: half 0 reads x of k
 // and asks for W half 1 of k + 2 and W half 0 of k + 3; half 1 reads W half 1 of k and W half 0 of k + 1 and asks for x of k + 3.
-template <int EPI, bool GROUPED, bool HALVES = false>
+// SLICED: workgroup number b takes slice b / tiles of tile b % tiles; see meet_slices.
+template <int EPI, bool GROUPED, bool HALVES = false, bool SLICED = false>
 __device__ __forceinline__ void tiles128(const TileArgs &a) {
     extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int wm = w >> 2, wn = w & 3, l16 = lane & 15, lg = lane >> 4;
     Place<EPI, GROUPED, 128, HALVES> at(a);
-    int id = blockIdx.x;
+    const int slice = SLICED ? blockIdx.x / at.total : 0;
+    int id = SLICED ? blockIdx.x % at.total : blockIdx.x;
+    const int tile = id;
     const int total = HALVES ? (at.in_halves(a) + 7) / 8 * 16 : at.total;      // HALVES: at most one a workgroup
+    const int first_step = SLICED ? (int)((long)(a.K / BK) * slice / a.slices) : 0;
     if (id >= total || (HALVES && id / 16 * 8 + id % 8 >= at.in_halves(a))) return;
     constexpr uint32_t kSlot = 3 * kHalf;
     const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) bf16_t *)lds;
@@ -340,11 +376,11 @@ __device__ __forceinline__ void tiles128(const TileArgs &a) {
     };
     auto ask_x = [&](uint32_t slot, int k) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) to_lds(a.x + k * BK, off_x[j], mine + slot + j * 8192);
+        for (int j = 0; j < 2; j++) to_lds(a.x + (first_step + k) * BK, off_x[j], mine + slot + j * 8192);
     };
     auto ask_w = [&](uint32_t slot, int h, int k) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) to_lds(at.w + k * BK, off_w[h][j], mine + slot + (1 + h) * kHalf + j * 8192);
+        for (int j = 0; j < 2; j++) to_lds(at.w + (first_step + k) * BK, off_w[h][j], mine + slot + (1 + h) * kHalf + j * 8192);
     };
     uint32_t rx[2], rw[2];
 #pragma unroll
@@ -374,7 +410,7 @@ __device__ __forceinline__ void tiles128(const TileArgs &a) {
         ask_w(kSlot, 0, 1); ask_x(kSlot, 1); ask_w(kSlot, 1, 1);
         ask_w(2 * kSlot, 0, 2); ask_x(2 * kSlot, 2);
     };
-    const int T = a.K / BK;                 // at least 3
+    const int T = SLICED ? (int)((long)(a.K / BK) * (slice + 1) / a.slices) - first_step : a.K / BK;      // at least 3
     at.go(a, id);
     if (HALVES && at.rows <= 0) return;
     offsets();
@@ -422,6 +458,8 @@ __device__ __forceinline__ void tiles128(const TileArgs &a) {
         read_w(s2, 1, w1);
         FLLM_LGKM0; FLLM_SWAP; multiply(acc[1], xs, w1); FLLM_SWAP;
         if (wm == 0) FLLM_SWAP;
+        if constexpr (SLICED)
+            if (!meet_slices(a, tile, slice, acc, (int *)lds)) return;
         const Place<EPI, GROUPED, 128, HALVES> done = at;
         int to[4];
 #pragma unroll
@@ -430,7 +468,7 @@ __device__ __forceinline__ void tiles128(const TileArgs &a) {
             if (GROUPED) asm volatile("" : "+v"(to[t]));
         }
         id += gridDim.x;
-        const bool more = !HALVES && id < total;
+        const bool more = !HALVES && !SLICED && id < total;
         if (more) {
             at.go(a, id);
             offsets();
@@ -463,6 +501,23 @@ template <int EPI, bool GROUPED, int ROWS, bool HALVES>
 auto tiles_entry() -> void (*)(TileArgs) {
     if constexpr (GROUPED) return large_grouped_tiles_kernel<EPI == EPI_GLU ? 0 : EPI == EPI_F32 ? 1 : 2, ROWS, HALVES>;
     else return tiles_kernel<EPI, ROWS, HALVES>;
+}
+
+template <int EPI>
+__global__ void __launch_bounds__(kThreads, 2) sliced_tiles_kernel(const TileArgs a) {
+    tiles128<EPI, false, false, true>(a);
+}
+// `tiles` 128-row tiles in a.slices slices: tiles * slices workgroups, no more than compute units
+template <int EPI>
+int launch_sliced(const TileArgs &a, long tiles, hipStream_t stream) {
+    static bool raised = false;
+    if (!raised) {
+        const hipError_t e = hipFuncSetAttribute((const void *)sliced_tiles_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds128);
+        FLLM_REQUIRE(e == hipSuccess, "gemm tiles: cannot raise the LDS limit: %s", hipGetErrorString(e));
+        raised = true;
+    }
+    hipLaunchKernelGGL(sliced_tiles_kernel<EPI>, dim3((unsigned)(tiles * a.slices)), dim3(kThreads), kLds128, stream, a);
+    return fllm_check_launch("sliced gemm tiles");
 }
 
 // Launches one of them on one workgroup a compute unit at most (grouped: as many tiles as there may be).

@@ -32,24 +32,6 @@ namespace {
 // issues every load and no load sits behind a branch.
 __device__ uint4 kZeros = {0u, 0u, 0u, 0u};     // not const: in the same address space as the tensors it stands in for
 
-// Partial sums that workgroups hand to each other go through the device workspace in 16-byte pieces that pass by the
-// caches of the compute units and of their die on both ways (the sc0 sc1 forms of the buffer instructions: written
-// through to memory, read from memory), as device-scope atomics do for single words.  The workspace is one buffer
-// for these instructions; offsets are in bytes from its base.
-typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
-constexpr int kThroughCaches = 17;        // cache policy bits sc0 (1) and sc1 (16)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t workspace_buffer(float *base) {
-    return __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00020000);      // raw buffer, offsets up to 2 GiB
-}
-__device__ __forceinline__ void hand_over(__amdgpu_buffer_rsrc_t ws, unsigned int byte_offset, f32x4_t v) {
-    u32x4_t bits = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
-    __builtin_amdgcn_raw_buffer_store_b128(bits, ws, byte_offset, 0, kThroughCaches);
-}
-__device__ __forceinline__ f32x4_t take_over(__amdgpu_buffer_rsrc_t ws, unsigned int byte_offset) {
-    const u32x4_t bits = __builtin_amdgcn_raw_buffer_load_b128(ws, byte_offset, 0, kThroughCaches);
-    return (f32x4_t){__uint_as_float(bits[0]), __uint_as_float(bits[1]), __uint_as_float(bits[2]), __uint_as_float(bits[3])};
-}
-
 constexpr int kWideRows = 128;            // the most rows of the kernel that passes the activations through LDS in chunks
 enum { PRO_BF16 = 0, PRO_NORM_F32 = 1, PRO_SCALED = 2 };
 enum { EPI_STORE = 0, EPI_STORE_F32 = 1, EPI_ADD = 2, EPI_QKV = 3, EPI_SWIGLU = 4 };

@@ -44,7 +44,7 @@ extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up,
     return launch_tiles<EPI_GLU, false>(a, plan.bm, plan.halves, plan.tiles, stream);
 }
 
-// mode 0: out = x w^T (+ bias); 2: out = relu(x w^T)^2; bfloat16.
+// mode 0: out = x w^T (+ bias); 2: out = relu(x w^T)^2; bfloat16.  1: float32, where K is cut into slices (tile_slices in plans.h).
 //
 // The squared ReLU against the library's product and a kernel of its own (13,312 x 1,536): 37 -> 28 us at 512 rows, 95 -> 79 at 2,048; fewer rows
 // as above.  A bias (2,048 x 1,536; the general path is linear_tiled_mfma_kernel): 32 -> 23 us at 136 rows, 34 -> 24 at 2,048.  Without either
@@ -53,14 +53,27 @@ extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up,
 // 2,048 rows 59 -> 55; 6,144 x 4,096 at 2,048 rows (192 of 256 rows) 80 -> 77, at 1,900 76 -> 78.  Hence nine tenths of the last round.
 extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const float *bias, void *out, int ldo, int M, int N, int K, int mode,
                                  int force, hipStream_t stream) {
-    FLLM_REQUIRE(M >= 0 && N > 0 && K > 0 && ldx >= K && ldo >= N && x && w && out && (mode == 0 || mode == 2),
+    FLLM_REQUIRE(M >= 0 && N > 0 && K > 0 && ldx >= K && ldo >= N && x && w && out && mode >= 0 && mode <= 2,
                  "linear_tiles: bad sizes or operands missing");
     if (!fllm_fast_kernels_enabled() || (bias && mode != 0) || !operands_fit(x, ldx, w, out, ldo, M, N, N, K)) return 1;
     if (M == 0) return 0;
-    const fllm_plan::TilePlan plan = plan_of(M, N, 256, K, force);
-    if (plan.bm == 0) return 1;
     TileArgs a = tile_args(x, ldx, w, out, ldo, M, N, K);
     a.bias = bias;
+    if (!force && mode != 2 && !bias) {
+        void *base = nullptr;
+        size_t bytes = 0;
+        const bool have_ws = fllm_device_workspace(&base, &bytes);
+        const long tiles = (long)((M + 127) / 128) * ((N + 255) / 256);
+        a.slices = fllm_plan::tile_slices(tiles, K, bytes, have_ws, fllm_option_tile_slices());
+        if (a.slices > 1) {
+            a.counters = (int *)base;
+            a.parts = (float *)((unsigned char *)base + fllm_plan::kCounterBytes);
+            return mode == 1 ? launch_sliced<EPI_F32>(a, tiles, stream) : launch_sliced<EPI_STORE>(a, tiles, stream);
+        }
+    }
+    if (mode == 1) return 1;
+    const fllm_plan::TilePlan plan = plan_of(M, N, 256, K, force);
+    if (plan.bm == 0) return 1;
     const long slots = (plan.tiles + 255) / 256 * 256;
     if (!force && mode == 2 && !fllm_plan::activation_joins(M, N, K, plan.rounds)) return 1;
     if (!force && mode == 0 && !bias && (K < 2048 || (!plan.halves && 10 * plan.tiles < 9 * slots))) return 1;

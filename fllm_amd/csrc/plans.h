@@ -287,6 +287,25 @@ inline TilePlan tile_plan(long tiles256, long tiles128, int K, int asked, int ha
     return p;
 }
 
+// K slices of a product whose 128-row tiles leave half of the compute units or more without one, a workgroup a slice; 1: whole.  What it costs is a
+// tile's sums on their way through memory, some 10 us for two to four slices; what it is measured against is the GEMM library, which has smaller
+// tiles.  Hence 32 steps of 64 columns a slice at least, K of 8,192 at least (4,096 x 4,096 at 1,024 rows 42.5 -> 43.7 us), and four fifths of the device
+// taken (2,048 x 8,192 at 1,500 rows, two slices of 96 tiles 61.3 -> 61.8, at 405 rows, 128 workgroups 31.3 -> 37.2).  Microseconds library -> slices:
+// 2,048 x 8,192 at 1,024 / 1,735 / 2,048 rows 51 -> 45 / 72 -> 66 / 75 -> 69; 1,536 x 13,312 at 700 / 1,500 / 1,735 65 -> 50 / 99 -> 73 / 89 -> 77 (float32 results
+// 98 -> 79); 1,536 x 8,960 at 1,500 / 1,735 66 -> 55 / 62 -> 57; 4,096 x 14,336 at 257 / 405 / 1,024 75 -> 58 / 86 -> 69 / 139 -> 117.
+// `asked`: 0 never, 1 planned, more: as many as that and K allow.
+inline size_t tile_slices_need(long tiles128, int slices) { return kCounterBytes + (size_t)tiles128 * slices * 128 * 256 * kF32; }
+inline int tile_slices(long tiles128, int K, size_t ws_bytes, bool have_ws, int asked) {
+    if (asked == 0 || !have_ws || K % 64 != 0 || tiles128 < 1 || tiles128 > 128 || (asked == 1 && K < 8192)) return 1;
+    const int least = asked > 1 ? 3 : 32;      // steps a slice; the kernel needs three
+    long s = asked > 1 ? asked : 256 / tiles128;
+    if (s > 256 / tiles128) s = 256 / tiles128;
+    if (s > K / 64 / least) s = K / 64 / least;
+    if (s > 8) s = 8;
+    if (s < 2 || tile_slices_need(tiles128, (int)s) > ws_bytes) return 1;
+    return asked > 1 || 10 * s * tiles128 >= 8 * 256 ? (int)s : 1;
+}
+
 // Whether a product with its activation in the epilogue (gate and up: `columns` counts both; the squared ReLU) goes to the tiles, or to the GEMM
 // library and a kernel for the activation.  A tile costs the same however few of its rows and columns are there and however few of the
 // compute units have one, where the library has smaller tiles and cuts K; against that stands one pass over the product, which

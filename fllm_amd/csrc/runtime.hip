@@ -35,6 +35,8 @@ static int g_x_direct = 1;
 int fllm_option_x_direct(void) { return g_x_direct; }
 static int g_tile32_rows = 0;     // 0: chosen by the launch; 128 or 256
 int fllm_option_tile32_rows(void) { return g_tile32_rows; }
+static int g_tile_slices = 1;     // 0: never, 1: planned, 2 and more: that many wherever K has steps enough
+int fllm_option_tile_slices(void) { return g_tile_slices; }
 static int g_wide_waves = 0;      // 0: planned
 int fllm_option_wide_waves(void) { return g_wide_waves; }
 static int g_resident_tiles = 1;  // q/k/v of up to 16 rows behind a prepared norm streams its tile-major copy (16-row tiles)
@@ -73,6 +75,10 @@ extern "C" int fllm_set_option(const char *name, int value) {
     }
     if (strcmp(name, "linear.resident_tiles") == 0) {
         g_resident_tiles = value != 0;
+        return 0;
+    }
+    if (strcmp(name, "linear.tile_slices") == 0) {
+        g_tile_slices = value < 0 ? 0 : value;
         return 0;
     }
     if (strcmp(name, "linear.wide_waves") == 0) {

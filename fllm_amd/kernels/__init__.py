@@ -523,8 +523,8 @@ class Ops:
             return out
         if (self.library_gemm_from is not None and M >= self.library_gemm_from and x.dtype == torch.bfloat16
                 and bias is None):
-            if mode == OUT_STORE and M > 64 and self._tiles_take(self.lib.fllm_linear_tiles(
-                    _ptr(x), ldx, _ptr(w), None, _ptr(out), ldo, M, N, K, 0, 0, self._stream())):
+            if mode != OUT_ADD_F32 and M > 64 and self._tiles_take(self.lib.fllm_linear_tiles(
+                    _ptr(x), ldx, _ptr(w), None, _ptr(out), ldo, M, N, K, 0 if mode == OUT_STORE else 1, 0, self._stream())):
                 return out
             if mode == OUT_STORE:
                 torch.matmul(x, w.t(), out=out)
