@@ -38,8 +38,8 @@ int fllm_linear(const void *x, int ldx, const void *w, const float *bias, void *
                 int dtype, int out_mode, hipStream_t stream);
 
 // Device memory for kernels that meet across workgroups: the decode-shaped products (1..16 rows), whose K
-// dimension is cut into slices over workgroups when the activations of all of K do not fit into LDS, and
-// decode attention over split contexts, and prompt attention of few rows over long contexts (the keys of a row
+// dimension is cut into slices over workgroups when the activations of all of K do not fit into LDS or its
+// tiles are few, products of many rows whose tiles are few (128 KiB a tile and slice), decode attention over split contexts, and prompt attention of few rows over long contexts (the keys of a row
 // tile go to several workgroups: 66 KiB a part for heads of 128).  Its first 64 KiB are counters, which must be zero when it is handed
 // over and are zero again after every launch; partial sums follow.  One per device (the current one);
 // work that would need more than it holds runs another way.  Launches on different streams of one device

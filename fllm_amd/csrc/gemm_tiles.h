@@ -313,33 +313,8 @@ __device__ __forceinline__ void tiles256(const TileArgs &a) {
 #undef FLLM_STEP
 }
 
-// The slices of a 128-row tile meet: every workgroup leaves its sums in the device workspace and counts the tile, the one that counts last goes on
-// with the sum of all in slice order (so it does not matter which one that is), the others are done: false.  Nobody waits for another.
-__device__ __forceinline__ bool meet_slices(const TileArgs &a, int tile, int slice, f32x4_t (&acc)[2][4][2], int *seen) {
-    const __amdgpu_buffer_rsrc_t parts = workspace_buffer(a.parts);
-    const unsigned int part = 128 * 256 * 4, mine = threadIdx.x * 16;      // bytes; 256 workgroups at most: 32 MiB
-    const unsigned int first = (unsigned int)tile * a.slices * part + mine;
-#pragma unroll
-    for (int p = 0; p < 16; p++) hand_over(parts, first + slice * part + p * kThreads * 16, acc[p >> 3][(p >> 1) & 3][p & 1]);
-    parts_published();
-    __syncthreads();
-    if (threadIdx.x == 0) *seen = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (*seen != a.slices - 1) return false;
-    parts_visible();
-    if (threadIdx.x == 0) __hip_atomic_store(a.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // for the next launch
-    f32x4_t sum[16];
-    for (int s = 0; s < a.slices; s++) {
-        f32x4_t v[16];
-#pragma unroll
-        for (int p = 0; p < 16; p++) v[p] = take_over(parts, first + s * part + p * kThreads * 16);
-#pragma unroll
-        for (int p = 0; p < 16; p++) sum[p] = s == 0 ? v[p] : sum[p] + v[p];
-    }
-#pragma unroll
-    for (int p = 0; p < 16; p++) acc[p >> 3][(p >> 1) & 3][p & 1] = sum[p];
-    return true;
-}
+// The slices of a 128-row tile meet (below): whether this workgroup goes on with the sums of all.
+__device__ __forceinline__ bool meet_slices(const TileArgs &a, int tile, int slice, f32x4_t (&acc)[2][4][2], int *seen);
 
 // 128 x 256 (EPI_GLU: 128 x 128), for launches whose 256-row tiles would leave much of the device idle: an operand read from LDS serves half
 // the products, so LDS and the matrix cores are busy alike.  LDS: three buffers of [x][W half 0][W half 1].  K step k: half 0 reads x of k
@@ -503,6 +478,36 @@ auto tiles_entry() -> void (*)(TileArgs) {
     else return tiles_kernel<EPI, ROWS, HALVES>;
 }
 
+// The slices of a 128-row tile meet: every workgroup leaves its sums in the device workspace and counts the tile, the one that counts last goes on
+// with the sum of all in slice order (so it does not matter which one that is), the others are done: false.  Nobody waits for another.
+__device__ __forceinline__ bool meet_slices(const TileArgs &a, int tile, int slice, f32x4_t (&acc)[2][4][2], int *seen) {
+    const __amdgpu_buffer_rsrc_t parts = workspace_buffer(a.parts);
+    const unsigned int part = 128 * 256 * 4, mine = threadIdx.x * 16;      // bytes; 256 workgroups at most: 32 MiB
+    const unsigned int first = (unsigned int)tile * a.slices * part + mine;
+#pragma unroll
+    for (int p = 0; p < 16; p++) hand_over(parts, first + slice * part + p * kThreads * 16, acc[p >> 3][(p >> 1) & 3][p & 1]);
+    parts_published();
+    __syncthreads();
+    if (threadIdx.x == 0) *seen = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (*seen != a.slices - 1) return false;
+    parts_visible();
+    if (threadIdx.x == 0) __hip_atomic_store(a.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // for the next launch
+    f32x4_t sum[16];
+    for (int s = 0; s < a.slices; s++) {
+        f32x4_t v[16];
+#pragma unroll
+        for (int p = 0; p < 16; p++) v[p] = take_over(parts, first + s * part + p * kThreads * 16);
+#pragma unroll
+        for (int p = 0; p < 16; p++) sum[p] = s == 0 ? v[p] : sum[p] + v[p];
+    }
+#pragma unroll
+    for (int p = 0; p < 16; p++) acc[p >> 3][(p >> 1) & 3][p & 1] = sum[p];
+    return true;
+}
+
+// What bounds it is what bounds the 128-row tiles, 0.88 us a step of K, and then the sums' way through memory: 2,048 x 2,048 x 8,192 in two slices of 128
+// tiles 69 us (1.0 PFLOP/s; library 75), 13 of them before the first and behind the last step; 1,735 x 1,536 x 13,312 in three of 84 77 (89).
 template <int EPI>
 __global__ void __launch_bounds__(kThreads, 2) sliced_tiles_kernel(const TileArgs a) {
     tiles128<EPI, false, false, true>(a);

@@ -306,8 +306,8 @@ __device__ __forceinline__ void epilogue(const SkinnyArgs &a, f32x4_t (&s)[RT], 
 // 1.5 or 3.5 a compute-unit slot.
 //
 // At the end of an item the waves' sums meet in LDS; one wave (they take turns) adds them in wave
-// order.  With S = 1 it runs the epilogue.  With S > 1 (only when the activations of all of K do not
-// fit into LDS) it leaves the item's sums in the workspace and counts the item; the workgroup that
+// order.  With S = 1 it runs the epilogue.  With S > 1 (when the activations of all of K do not fit
+// into LDS, and see slice_direct in plans.h) it leaves the item's sums in the workspace and counts the item; the workgroup that
 // counts a tile's last item adds the S partial sums in slice order and runs the epilogue, so the
 // result does not depend on which workgroup came last.
 enum { TM_ROWS16 = 0, TM_DUALK = 1, TM_GATEUP = 2, TM_HALVES = 3 };
