@@ -125,9 +125,10 @@ inline ChunkPlan plan_chunks(int K, int ntiles, int mt, int rt, size_t ws_bytes,
     // K slices: as many as fill the chip with the row groups there are, each at least two chunks long.  Up to 48 rows a
     // workgroup has enough on its way for a compute unit of its own, and more slices only cost their sums' way through
     // memory (40 rows, with one workgroup a unit and with two: 4,096 x 4,096 13.3 and 16.2 us, 4,096 x 14,336 28.0 and
-    // 29.6).  49 to 64 rows keep two; one is faster for sums into the stream (64 rows: 16.1 and 18.4, 30.3 and 32.7), their
-    // other epilogues were not measured with it.
-    const int fill = mt <= 3 ? cus : slots;
+    // 29.6).  49 to 64 rows keep two, but where one still leaves four slices and a tile is 16 rows (64 rows, sums into the
+    // stream: 4,096 x 4,096 17.0 and 19.8, 4,096 x 14,336 30.5 and 32.8; two slices instead of four 8,192 x 8,192 35.5 and
+    // 34.3, 8,192 x 28,672 91.5 and 90.3).
+    const int fill = mt <= 3 || (mt == 4 && rt == 1 && 4 * ngroups <= cus) ? cus : slots;
     int S = 1;
     while (S < 8 && ngroups * S * 2 <= fill && (K + 2 * S - 1) / (2 * S) >= 512) S *= 2;
     if (forced > 0) S = forced;
