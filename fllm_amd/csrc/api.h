@@ -463,7 +463,7 @@ int fllm_experts_grouped_ungated(const void *h, int ldh, const int32_t *ids, int
 
 // Products of many bfloat16 rows on 256- and 128-row tiles (gemm_tiles.h).  0: launched, 1: declined (sizes that are no multiples of the
 // tiles' pieces, or with `force` 0 shapes that the general path is faster at).  fllm_linear_tiles: mode 0 stores, 1 stores
-// float32 (K in slices alone: declined otherwise), 2 the squared ReLU.
+// float32 (K in slices alone: declined otherwise), 2 the squared ReLU; rows that share memory (ldx < K) and empty products are declined.
 int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up, void *out, int M, int inter, int K, float limit, float alpha,
                        float up_offset, int force, hipStream_t stream);
 int fllm_linear_tiles(const void *x, int ldx, const void *w, const float *bias, void *out, int ldo, int M, int N, int K, int mode, int force,

@@ -53,8 +53,9 @@ extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up,
 // 2,048 rows 59 -> 55; 6,144 x 4,096 at 2,048 rows (192 of 256 rows) 80 -> 77, at 1,900 76 -> 78.  Hence nine tenths of the last round.
 extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const float *bias, void *out, int ldo, int M, int N, int K, int mode,
                                  int force, hipStream_t stream) {
-    FLLM_REQUIRE(M >= 0 && N > 0 && K > 0 && ldx >= K && ldo >= N && x && w && out && mode >= 0 && mode <= 2,
-                 "linear_tiles: bad sizes or operands missing");
+    FLLM_REQUIRE(M >= 0 && N >= 0 && K >= 0 && mode >= 0 && mode <= 2, "linear_tiles: bad sizes");
+    // rows that share memory, products without columns or steps: the general path's
+    if (N == 0 || K == 0 || ldx < K || ldo < N || !x || !w || !out) return 1;
     if (!fllm_fast_kernels_enabled() || (bias && mode != 0) || !operands_fit(x, ldx, w, out, ldo, M, N, N, K)) return 1;
     if (M == 0) return 0;
     TileArgs a = tile_args(x, ldx, w, out, ldo, M, N, K);
