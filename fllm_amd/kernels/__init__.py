@@ -422,18 +422,22 @@ class Ops:
     _streams = {}            # device index -> the stream on which this process launches the kernels of that device
 
     @staticmethod
+    def _current_stream() -> Tuple[int, int]:
+        """(device, the current stream's handle)."""
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None:               # the handle without a Stream object around it (a launch asks for it every time)
+            device = torch.cuda.current_device()
+            return device, raw(device)
+        stream = torch.cuda.current_stream()
+        return stream.device_index, stream.cuda_stream
+
+    @staticmethod
     def _stream() -> int:
         """The current stream.  Kernels of one device meet in that device's workspace (counters that each launch leaves
         at zero, partial results behind them), so launches on one device must not overlap: all of them go to one stream
         (a stream that is capturing a graph stands for the stream the graph will be replayed on).  A launch on a second
         stream of the same device is refused."""
-        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-        if raw is not None:               # the handle without a Stream object around it (a launch asks for it every time)
-            device = torch.cuda.current_device()
-            handle = raw(device)
-        else:
-            stream = torch.cuda.current_stream()
-            handle, device = stream.cuda_stream, stream.device_index
+        device, handle = Ops._current_stream()
         seen = Ops._streams.get(device)
         if seen is None:
             if not torch.cuda.is_current_stream_capturing():
@@ -442,6 +446,13 @@ class Ops:
             raise KernelError(f"kernels of device {device} were launched on stream {seen:#x} before and are now asked for on "
                               f"stream {handle:#x}: they share the device workspace and must stay on one stream")
         return handle
+
+    @staticmethod
+    def _on_the_kernels_stream() -> bool:
+        """Whether `_stream` would hand out the current stream without refusing it or making it the device's."""
+        device, handle = Ops._current_stream()
+        seen = Ops._streams.get(device)
+        return seen is not None and (handle == seen or torch.cuda.is_current_stream_capturing())
 
     def random_fill(self, out: torch.Tensor, key, kind: int) -> torch.Tensor:
         """Fills `out` with the random tensor of `key` (two 32-bit words): kind 0 normal numbers of deviation 0.02, kind 1
@@ -493,7 +504,9 @@ class Ops:
 
     def linear(self, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor] = None,
                accumulate: bool = False) -> torch.Tensor:
-        """out = x @ w.T (+ bias); `accumulate` adds into a float32 `out` instead of storing."""
+        """out = x @ w.T (+ bias); `accumulate` adds into a float32 `out` instead of storing.  Launches of one device share its
+        workspace and stay on one stream (`_stream`); what goes to the GEMM library whole (up to 64 rows stored, float32 results of
+        more) runs on any."""
         _need(x.dim() == 2 and w.dim() == 2 and out.dim() == 2, "linear takes matrices")
         M, K = x.shape
         N = w.shape[0]
@@ -523,7 +536,8 @@ class Ops:
             return out
         if (self.library_gemm_from is not None and M >= self.library_gemm_from and x.dtype == torch.bfloat16
                 and bias is None):
-            if mode != OUT_ADD_F32 and M > 64 and self._tiles_take(self.lib.fllm_linear_tiles(
+            # float32 results: on another stream than the kernels' the library's, as it needs no workspace
+            if mode != OUT_ADD_F32 and M > 64 and (mode == OUT_STORE or self._on_the_kernels_stream()) and self._tiles_take(self.lib.fllm_linear_tiles(
                     _ptr(x), ldx, _ptr(w), None, _ptr(out), ldo, M, N, K, 0 if mode == OUT_STORE else 1, 0, self._stream())):
                 return out
             if mode == OUT_STORE:

@@ -1,5 +1,6 @@
 """Products of more than 64 bfloat16 rows whose operands the tile products do not take, through `Ops.linear`: rows that share memory (one row for all,
-windows that overlap), products without a step or a column, with the kernels for matrix cores on and off.  Float32 sums of K = 512 products of
+windows that overlap), products without a step or a column, with the kernels for matrix cores on and off; and float32 results on a stream
+that is not the kernels'.  Float32 sums of K = 512 products of
 bfloat16 operands that are exact in float64: K 2^-24 of the largest value, below 2^-14; bfloat16 results one rounding more, 2^-9."""
 import pytest
 import torch
@@ -35,3 +36,26 @@ def test_operands_of_the_library(ops, dtype, fast):
     ops.linear(torch.empty(M, 0, dtype=torch.bfloat16, device="cuda"), torch.empty(N, 0, dtype=torch.bfloat16, device="cuda"), nothing)
     assert (nothing == 0).all()
     ops.linear(FORMS["rows"](g), torch.empty(0, K, dtype=torch.bfloat16, device="cuda"), torch.empty(M, 0, dtype=dtype, device="cuda"))
+
+
+def test_float32_results_on_another_stream(ops):
+    """The library has no workspace to share: such a product runs on any stream, also of a shape whose K the tiles cut on their own stream; nothing
+    is asked of the device's stream for it."""
+    from fllm_amd.kernels import Ops
+    g = torch.Generator().manual_seed(4)
+    x, w = torch.randn(1024, 8192, generator=g).bfloat16().cuda(), (torch.randn(2048, 8192, generator=g) * 8192 ** -0.5).bfloat16().cuda()
+    want = x.double() @ w.double().t()
+    ops._stream()
+    claimed, other = dict(Ops._streams), torch.cuda.Stream()
+    outs = [torch.full((1024, 2048), float("nan"), device="cuda") for _ in range(2)]
+    ops.linear(x, w, outs[0])
+    other.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(other):
+        ops.linear(x, w, outs[1])
+    torch.cuda.synchronize()
+    assert Ops._streams == claimed
+    for out in outs:
+        assert (out.double() - want).abs().max() <= 2.0 ** -10 * want.abs().max()
+    library = torch.empty_like(outs[1])
+    torch.mm(x, w.t(), out_dtype=torch.float32, out=library)
+    assert torch.equal(outs[1], library)
