@@ -50,7 +50,8 @@ extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up,
 // as above.  A bias (2,048 x 1,536; the general path is linear_tiled_mfma_kernel): 32 -> 23 us at 136 rows, 34 -> 24 at 2,048.  Without either
 // the library has kernels for every tile of the device's time, and these tiles are ahead only where they fill whole rounds over the compute
 // units: 4,096 x 14,336 at 2,048 rows (256 tiles) 207 -> 188 us, at 1,900 (240) 191 -> 182, at 1,536 (192) 167 -> 177; 4,096 x 4,096 at
-// 2,048 rows 59 -> 55; 6,144 x 4,096 at 2,048 rows (192 of 256 rows) 80 -> 77, at 1,900 76 -> 78.  Hence nine tenths of the last round.
+// 2,048 rows 59 -> 55; 6,144 x 4,096 at 2,048 rows (192 of 256 rows) 80 -> 77, at 1,900 76 -> 78.  Hence nine
+// tenths of the rounds, and what that means where a last round runs as halves: plain_takes_tiles in plans.h.
 extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const float *bias, void *out, int ldo, int M, int N, int K, int mode,
                                  int force, hipStream_t stream) {
     FLLM_REQUIRE(M >= 0 && N >= 0 && K >= 0 && mode >= 0 && mode <= 2, "linear_tiles: bad sizes");
@@ -75,9 +76,8 @@ extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const fl
     if (mode == 1) return 1;
     const fllm_plan::TilePlan plan = plan_of(M, N, 256, K, force);
     if (plan.bm == 0) return 1;
-    const long slots = (plan.tiles + 255) / 256 * 256;
     if (!force && mode == 2 && !fllm_plan::activation_joins(M, N, K, plan.rounds)) return 1;
-    if (!force && mode == 0 && !bias && (K < 2048 || (!plan.halves && 10 * plan.tiles < 9 * slots))) return 1;
+    if (!force && mode == 0 && !bias && !fllm_plan::plain_takes_tiles(M, N, K, plan)) return 1;
     if (mode == 0) return launch_tiles<EPI_STORE, false>(a, plan.bm, plan.halves, plan.tiles, stream);
     return launch_tiles<EPI_RELU2, false>(a, plan.bm, plan.halves, plan.tiles, stream);
 }

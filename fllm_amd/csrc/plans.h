@@ -288,6 +288,19 @@ inline TilePlan tile_plan(long tiles256, long tiles128, int K, int asked, int ha
     return p;
 }
 
+// Whether a plain product (neither bias nor activation) goes to the tiles, or to the GEMM library: K of 2,048 at least and nine tenths of the rounds
+// filled, in tiles (whole rounds) or, where a last round runs as halves, in outputs: such a round is short because half of the device is enough for it,
+// and what its tiles do for rows that are not there counts all the more.  Microseconds library / halves by share, one MI355X, weights from memory:
+// 0.90 and more 16,384 x 2,048 at 1,500 rows 86.7 / 84.6, x 3,072 at 1,536 124.8 / 122.7, 24,576 x 4,096 at 1,024 166.8 / 154.7, 8,192 x 8,192 at
+// 3,072 293 / 283, 57,344 x 8,192 at 1,280 907 / 827; 0.80 to 0.87 16,384 x 2,048 at 2,304 128 / 138, x 4,096 at 2,304 234 / 239, 13,824 x 5,120 at 2,560
+// 279 / 286, but 6,144 x 4,096 at 3,840 149 / 144; below 28,672 x 4,096 at 513 125 / 139, 10,240 x 8,192 at 1,537 and 2,048 238 / 247 and 269 / 269,
+// 16,384 x 2,048 at 1,100 69 / 77.  (Where the library takes one of its slow kernels the tiles are up to 1.9 times as fast at any share.)
+inline bool plain_takes_tiles(long M, long N, int K, const TilePlan &p) {
+    if (p.bm == 0 || K < 2048) return false;
+    if (p.halves) return (double)M * (double)N >= 0.9 * p.rounds * 256.0 * 65536.0;
+    return 10 * p.tiles >= 9 * ((p.tiles + 255) / 256 * 256);
+}
+
 // K slices of a product whose 128-row tiles leave half of the compute units or more without one, a workgroup a slice; 1: whole.  What it costs is a
 // tile's sums on their way through memory, some 10 us for two to four slices; what it is measured against is the GEMM library, which has smaller
 // tiles.  Hence 32 steps of 64 columns a slice at least, K of 8,192 at least (4,096 x 4,096 at 1,024 rows 42.5 -> 43.7 us), and four fifths of the device

@@ -162,6 +162,17 @@ int main() {
         const int bm = row_tile(t256, t128, m.K);
         REQUIRE(activation_joins(m.rows, m.columns, m.K, bm, bm == 256 ? t256 : t128) == m.joins, "%d columns of %d, %ld rows", m.columns, m.K, m.rows);
     }
+    // A plain product leaves the library where the tiles were measured ahead, and stays where they were behind.
+    struct { int columns, K; long rows; bool tiles; } plain[] = {
+        {16384, 2048, 1536, true}, {16384, 2048, 1500, true}, {24576, 4096, 1024, true}, {8192, 8192, 3072, true}, {57344, 8192, 1280, true},
+        {6144, 4096, 4096, true}, {6144, 4096, 2560, true}, {4096, 14336, 2048, true}, {6144, 4096, 2048, false}, {16384, 2048, 1100, false}, {16384, 2048, 1280, false},
+        {16384, 2048, 2304, false}, {16384, 4096, 2304, false}, {28672, 4096, 513, false}, {24576, 4096, 513, true} /* 128-row tiles */, {24576, 4096, 768, false},
+        {10240, 8192, 1537, false}, {10240, 8192, 2048, false}, {13824, 5120, 2560, false}, {28672, 1536, 2304, false}};
+    for (auto &m : plain) {
+        const long cols = (m.columns + 255) / 256;
+        const TilePlan p = tile_plan((m.rows + 255) / 256 * cols, (m.rows + 127) / 128 * cols, m.K, 0, 1);
+        REQUIRE(plain_takes_tiles(m.rows, m.columns, m.K, p) == m.tiles, "%d columns of %d, %ld rows", m.columns, m.K, m.rows);
+    }
     // ---- decode attention ----
     for (int head_dim : {32, 64, 128}) {      // a wave's 64 keys; one row of one head group, and the part that tips the choice
         const int unit = decode_unit(head_dim), last = 16 * unit - 31;

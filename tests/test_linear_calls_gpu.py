@@ -59,3 +59,12 @@ def test_float32_results_on_another_stream(ops):
     library = torch.empty_like(outs[1])
     torch.mm(x, w.t(), out_dtype=torch.float32, out=library)
     assert torch.equal(outs[1], library)
+
+
+@pytest.mark.parametrize("rows,columns,K,taken", [(1100, 16384, 2048, 1), (513, 28672, 4096, 1), (1537, 10240, 8192, 1), (1536, 16384, 2048, 0), (1024, 24576, 4096, 0)])
+def test_plain_products_leave_the_library_where_they_fill_their_rounds(ops, rows, columns, K, taken):
+    """All of them have a last round of half tiles; the first three fill 0.54 to 0.66 of their rounds and are the library's (1: declined)."""
+    x, w = torch.zeros(rows, K, dtype=torch.bfloat16, device="cuda"), torch.zeros(columns, K, dtype=torch.bfloat16, device="cuda")
+    out = torch.ones(rows, columns, dtype=torch.bfloat16, device="cuda")
+    assert ops.lib.fllm_linear_tiles(x.data_ptr(), K, w.data_ptr(), None, out.data_ptr(), columns, rows, columns, K, 0, 0, ops._stream()) == taken
+    assert (out == taken).all()
