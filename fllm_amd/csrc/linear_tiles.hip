@@ -38,7 +38,7 @@ extern "C" int fllm_gate_up_tiles(const void *x, int ldx, const void *w_gate_up,
     if (!fllm_fast_kernels_enabled() || !operands_fit(x, ldx, w_gate_up, out, inter, M, 2L * inter, inter, K)) return 1;
     if (M == 0) return 0;
     const fllm_plan::TilePlan plan = plan_of(M, inter, 128, K, force);
-    if (plan.bm == 0 || (!force && !fllm_plan::activation_joins(M, 2L * inter, K, plan.rounds))) return 1;
+    if (plan.bm == 0 || (!force && !fllm_plan::activation_joins(M, 2L * inter, K, plan))) return 1;
     TileArgs a = tile_args(x, ldx, w_gate_up, out, inter, M, inter, K);
     a.limit = limit, a.alpha = alpha, a.up_offset = up_offset;
     return launch_tiles<EPI_GLU, false>(a, plan.bm, plan.halves, plan.tiles, stream);
@@ -76,7 +76,7 @@ extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const fl
     if (mode == 1) return 1;
     const fllm_plan::TilePlan plan = plan_of(M, N, 256, K, force);
     if (plan.bm == 0) return 1;
-    if (!force && mode == 2 && !fllm_plan::activation_joins(M, N, K, plan.rounds)) return 1;
+    if (!force && mode == 2 && !fllm_plan::activation_joins(M, N, K, plan)) return 1;
     if (!force && mode == 0 && !bias && !fllm_plan::plain_takes_tiles(M, N, K, plan)) return 1;
     if (mode == 0) return launch_tiles<EPI_STORE, false>(a, plan.bm, plan.halves, plan.tiles, stream);
     return launch_tiles<EPI_RELU2, false>(a, plan.bm, plan.halves, plan.tiles, stream);

@@ -326,17 +326,17 @@ inline int tile_slices(long tiles128, int K, size_t ws_bytes, bool have_ws, int 
 // weighs less the longer K is.  share: what the rounds of the tiles do for this product, 1 where every compute unit has whole 256-row
 // tiles all the time.  Measured inside a graph, weights from memory, microseconds library and kernel -> tiles at rows: 28,672 columns of
 // 4,096 65 60 -> 67, 160 65 -> 68, 320 85 -> 97, 640 0.92x, then 420 1.08x, 512 114 -> 100, 900 1.10x (line at 0.65); 16,384 of 2,048 128 24 -> 34, 256 33 -> 34,
-// 513 0.92x, 1,030 0.94x, then 420 1.18x, 512 43 -> 38, 768 1.08x (line at 0.57); 17,920 of 1,536 128 25.5 -> 29.6, then 192 29.3 -> 27.5, 320 34 -> 28;
+// 513 0.92x, then 420 1.18x, 512 43 -> 38, 768 1.08x (line at 0.57); 17,920 of 1,536 128 25.5 -> 29.6, then 192 29.3 -> 27.5, 320 34 -> 28;
 // the squared ReLU of 4,480 of 1,536 128 19 -> 26, 512 22.9 -> 24.8, then 900 1.21x, of 13,312 of 1,536 128 22 -> 28, then 320 31 -> 26, 512 35 -> 28 (line at
 // 0.29).  Up to K 1,024 the two sides are a few microseconds apart on the device (8,192 of 1,024 128 15.8 -> 20.3, 320 19.5 -> 19.2, 512 21.5 -> 19.9) and a
 // prompt step of such a model waits for the host's launches, of which the tiles save one: 24 -> 18 to 20 at 65 to 512 rows launched one by one.
-inline bool activation_joins(long M, long columns, int K, double rounds) {
+// Where a last round runs as halves the line is no lower than 0.68: 28,672 of 4,096 620 148 -> 150 (0.65), 640 144 -> 149 (0.67), then 645 159 -> 147
+// (0.68), 700 162 -> 150; 16,384 of 4,096 1,085 140 -> 145 (0.65), 1,120 142 -> 146, then 1,280 150 -> 152, 2,304 257 -> 243; 24,576 of 4,096 768 155 -> 150;
+// 16,384 of 2,048 1,030 82 -> 80 and 1,280 88 -> 86 (above its line of 0.57).
+inline bool activation_joins(long M, long columns, int K, const TilePlan &p) {
     if (K <= 1024) return true;
-    const double share = (double)M * (double)columns / (rounds * 256.0 * 65536.0), line = (K - 1024) / 1792.0;
-    return share >= (line < 0.65 ? line : 0.65);
-}
-inline bool activation_joins(long M, long columns, int K, int bm, long tiles) {
-    return activation_joins(M, columns, K, (double)((tiles + 255) / 256) * (bm == 256 ? 1.0 : kShortRound));
+    const double share = (double)M * (double)columns / (p.rounds * 256.0 * 65536.0), line = (K - 1024) / 1792.0, most = p.halves ? 0.68 : 0.65;
+    return share >= (line < most ? line : most);
 }
 
 // ---- decode attention: contexts split over workgroups ----
