@@ -118,17 +118,23 @@ inline size_t chunk_workspace_need(int ntiles, int S, int mt, int rt) {
     return kCounterBytes + (size_t)ntiles * S * mt * rt * kWaveLanes * 4 * kF32;
 }
 // `waves`: row tiles (waves) of a workgroup; a compute unit holds eight waves of this kernel, two workgroups of four or
-// one of five to eight
-inline ChunkPlan plan_chunks(int K, int ntiles, int mt, int rt, size_t ws_bytes, bool have_ws, int cus, int forced, int waves = 4) {
+// one of five to eight.  `copy`: whether the weights come from their tile-major copy
+inline ChunkPlan plan_chunks(int K, int ntiles, int mt, int rt, size_t ws_bytes, bool have_ws, int cus, int forced, int waves = 4,
+                             bool copy = false) {
     const int ngroups = (ntiles + waves - 1) / waves;
     const int slots = 8 / waves * cus;
     // K slices: as many as fill the chip with the row groups there are, each at least two chunks long.  Up to 48 rows a
     // workgroup has enough on its way for a compute unit of its own, and more slices only cost their sums' way through
     // memory (40 rows, with one workgroup a unit and with two: 4,096 x 4,096 13.3 and 16.2 us, 4,096 x 14,336 28.0 and
-    // 29.6).  49 to 64 rows keep two, but where one still leaves four slices and a tile is 16 rows (64 rows, sums into the
-    // stream: 4,096 x 4,096 17.0 and 19.8, 4,096 x 14,336 30.5 and 32.8; two slices instead of four 8,192 x 8,192 35.5 and
-    // 34.3, 8,192 x 28,672 91.5 and 90.3).
-    const int fill = mt <= 3 || (mt == 4 && rt == 1 && 4 * ngroups <= cus) ? cus : slots;
+    // 29.6).  49 to 64 rows keep two, but where one still leaves four slices and a tile is 16 rows: from a tile-major copy up to K of 16,384, where
+    // the loads of one workgroup begin to be too few; and where eight slices of one a unit would hold all tiles but one, they keep eight.
+    // Microseconds at 49 and 64 rows, eight slices / four of workgroups of four waves: stored with a bias 4,096 x 4,096 18.9 / 15.7 and 18.8 / 15.5,
+    // float32 results 16.5 / 14.0 and 16.7 / 14.1; sums that prepare a norm 4,096 x 8,192 25.3 / 25.0 and 25.8 / 25.1, x 14,336 38.1 / 34.3 and 37.9 / 33.3, 2,560 x
+    // 8,192 24.2 / 21.7 and 24.9 / 21.8, 3,600 x 24,576 54.3 / 54.9 and 54.2 / 52.6; with a copy 4,096 x 8,192 23.4 / 22.0 and 24.1 / 22.0, x 14,336 31.7 / 30.3
+    // and 32.1 / 29.6, but x 16,384 32.9 / 36.0 and 33.2 / 36.7, x 28,672 47.9 / 49.4 and 48.5 / 49.1; of 129 tiles (2,064 columns) x 8,192 19.8 / 20.8 and
+    // 19.9 / 21.1, x 24,576 41.1 / 45.1 and 41.5 / 45.3.  Two slices instead of four (64 rows): 8,192 x 8,192 35.5 and 34.3, 8,192 x 28,672 91.5 and 90.3.
+    const bool four = mt == 4 && rt == 1 && (K < 16384 || !copy) && 4 * ngroups <= cus && ntiles > cus / 8 * waves + 1;
+    const int fill = mt <= 3 || four ? cus : slots;
     int S = 1;
     while (S < 8 && ngroups * S * 2 <= fill && (K + 2 * S - 1) / (2 * S) >= 512) S *= 2;
     if (forced > 0) S = forced;
@@ -163,18 +169,18 @@ inline long chunk_plan_cost(const ChunkPlan &p, int ntiles, int cus) {
     const long together = p.grid <= cus ? 1 : 8 / p.waves;       // workgroups of a compute unit
     return rounds * together * p.waves * (long)p.slice;
 }
-// The number of waves (four, seven or eight) whose plan leaves the least to the busiest compute unit; on a tie four,
+// From a copy: the number of waves (four, seven or eight) whose plan leaves the least to the busiest compute unit; on a tie four,
 // but see below.
 // 1,792 tiles over 256 compute units are seven a unit: workgroups of seven waves take a tile each in one round, where
 // four or eight waves leave an eighth of the device idle in the last round.
 inline ChunkPlan plan_chunks_balanced(int K, int ntiles, int mt, int rt, size_t ws_bytes, bool have_ws, int cus, int forced,
                                       int forced_waves) {
     if (forced_waves == 4 || forced_waves == 7 || forced_waves == 8)
-        return plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, forced_waves);
-    ChunkPlan best = plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, 4);
+        return plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, forced_waves, true);
+    ChunkPlan best = plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, 4, true);
     long best_cost = chunk_plan_cost(best, ntiles, cus);
     for (int waves = 7; waves <= 8; waves++) {
-        const ChunkPlan p = plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, waves);
+        const ChunkPlan p = plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, waves, true);
         const long cost = chunk_plan_cost(p, ntiles, cus);
         // a tie between four and eight waves, no slices either way, three or four row tiles of activations: eight waves
         // share one copy of a chunk in LDS where two workgroups of four hold one each (the vocabulary projection at
@@ -188,10 +194,10 @@ inline ChunkPlan plan_chunks_balanced(int K, int ntiles, int mt, int rt, size_t 
 // Six waves where they leave less still: 384 tiles in four slices are 256 workgroups of six, where seven waves make 220 and leave 36 units idle
 // (q/k/v of 6,144 x 4,096 at 17 / 40 rows 18.2 -> 17.3 / 21.2 -> 20.3 us, of 10,240 x 8,192 37.4 -> 37.2 / 42.8 -> 41.3).
 inline ChunkPlan plan_chunks_even(int K, int ntiles, int mt, int rt, size_t ws_bytes, bool have_ws, int cus, int forced, int forced_waves) {
-    if (forced_waves == 6) return plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, 6);
+    if (forced_waves == 6) return plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, 6, true);
     const ChunkPlan best = plan_chunks_balanced(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, forced_waves);
     if (forced_waves == 4 || forced_waves == 7 || forced_waves == 8) return best;
-    const ChunkPlan six = plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, 6);
+    const ChunkPlan six = plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, 6, true);
     return chunk_plan_cost(six, ntiles, cus) < chunk_plan_cost(best, ntiles, cus) ? six : best;
 }
 

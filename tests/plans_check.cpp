@@ -134,6 +134,15 @@ int main() {
                                 }
                             }
                 }
+    // 49 to 64 rows, tiles of 16: slices for one workgroup a compute unit where that is four of them, but for one tile over
+    struct { int tiles, K, mt, rt; bool copy; int slices; } sums[] = {
+        {256, 4096, 4, 1, false, 4}, {256, 4096, 4, 1, true, 4}, {256, 14336, 4, 1, true, 4}, {256, 16384, 4, 1, true, 8}, {256, 16384, 4, 1, false, 4},
+        {130, 8192, 4, 1, false, 4}, {129, 8192, 4, 1, false, 8}, {129, 8192, 4, 1, true, 8}, {128, 8192, 4, 1, false, 8}, {257, 4096, 4, 1, false, 4},
+        {257, 2048, 4, 1, false, 4}, {256, 4096, 4, 2, false, 8}, {256, 4096, 3, 1, false, 4}, {129, 8192, 3, 1, false, 4}};
+    for (auto &t : sums) {
+        const ChunkPlan c = plan_chunks(t.K, t.tiles, t.mt, t.rt, (size_t)192 << 20, true, 256, 0, 4, t.copy);
+        REQUIRE(c.S == t.slices, "%d tiles of %d, %d row tiles, copy %d: %d slices", t.tiles, t.K, t.mt, t.copy, c.S);
+    }
     // ---- products of many rows on tiles ----
     // What a tile walks: 256 rows steps 0 1 .. in pairs, the last four apart, 128 rows the last three apart; a K that is not taken
     // would be cut short or read past its end, also where a caller asks for the tile.
