@@ -27,6 +27,16 @@ int main() {
                     int most = 0;
                     for (int n : unit) most = n > most ? n : most;
                     const bool shared = S == 1 && per_cu == 2;
+                    // the fewest workgroups, each number tried, that leave the busiest unit the least, where that is an eighth and more
+                    int few = even, least = busiest_unit(tiles, even, cus);
+                    for (int g = even + 1; g <= slots; g++)
+                        if (busiest_unit(tiles, g, cus) < least) few = g, least = busiest_unit(tiles, g, cus);
+                    const int before = busiest_unit(tiles, even, cus);
+                    const int wanted = shared && even > cus && 8 * (before - least) > before ? few : even;
+                    if (groups != wanted) {
+                        fprintf(stderr, "FAILED cus %d per %d S %d tiles %d: %d groups, not %d\n", cus, per_cu, S, tiles, groups, wanted);
+                        return 1;
+                    }
                     if (groups < 1 || groups > slots || busiest_unit(tiles, groups, cus) > busiest_unit(tiles, even, cus) || (!shared && groups != even) ||
                         (shared && most != busiest_unit(tiles, groups, cus))) {
                         fprintf(stderr, "FAILED cus %d per %d S %d tiles %d: %d groups, busiest %d\n", cus, per_cu, S, tiles, groups, most);
