@@ -15,9 +15,10 @@ int fllm_abi_version(void);
 // 0: bfloat16 calls use the plain kernels only (for comparing them with the MFMA kernels); default 1
 void fllm_set_fast_kernels(int on);
 // Switches a kernel variant (for measurements and tests): "attention.tile32" 0/1; "linear.slices" n
-// (0: chosen by shape); "linear.dual_k" 0/1; "linear.x_direct" 0/1; "attention.fused_merge" 0/1;
-// "attention.prefill_parts" 0/1; "linear.slab" 0/1/2; "linear.wide_waves" 0 (planned)/4/6/7/8; "linear.tile_slices" 0 (never)/1 (planned)/2 to 8; "linear.resident_tiles" 0/1;
-// "attention.tile32_rows" 0 (chosen by the launch)/128/256.  0 on success.
+// (0: chosen by shape; 1 also keeps K whole where products of 9 to 16 rows read their activations where they lie); "linear.dual_k" 0/1;
+// "linear.x_direct" 0/1; "attention.fused_merge" 0/1; "attention.prefill_parts" 0/1; "linear.slab" 0/1/2; "linear.wide_waves" 0
+// (planned)/4/6/7/8; "linear.half_tiles" 0 (never)/1 (planned)/2 (wherever a last round can be halved); "linear.tile_slices" 0 (never)/1
+// (planned)/2 to 8; "linear.resident_tiles" 0/1; "attention.tile32_rows" 0 (chosen by the launch)/128/256.  0 on success.
 int fllm_set_option(const char *name, int value);
 
 // out[r, :] = scale * table[ids[r], :]            out: float32 [rows, width]

@@ -1374,7 +1374,7 @@ int launch_resident(const SkinnyArgs &a, hipStream_t stream) {
         const bool x_direct = PRO == PRO_BF16 && fllm_option_x_direct() && a.ldx % 8 == 0 && tiles16 <= 4 * device_cus();
         ResidentPlan p = plan_resident(a.M, a.K, tiles16, RT, ws, x_direct);
         if (p.S == 0) return 1;
-        if (x_direct) fllm_plan::slice_direct(p, a.M, a.K, tiles16, RT, ws.bytes, ws.base != nullptr, device_cus());
+        if (x_direct) fllm_plan::slice_direct(p, a.M, a.K, tiles16, RT, ws.bytes, ws.base != nullptr, device_cus(), fllm_option_linear_slices());
         // 8-row tiles (two K halves a product) when the rows allow it and the 16-row tiles come to between half a
         // tile and two tiles per slot, unevenly: 384 tiles on 512 slots run as long as 512 would.  Also when the 16-row
         // tiles fill no more than half of the compute units (narrow models): twice the workgroups, each with half the

@@ -70,9 +70,9 @@ inline ResidentPlan plan_resident(int M, int K, int ntiles, int rt, size_t ws_by
 // two slices, whose workgroups fill the device.  What it costs is the tile's way through memory, about 1 us.  Microseconds at 9 / 16 rows whole ->
 // sliced: 2,048 x 8,192 11.8 -> 10.2 / 14.7 -> 11.3, 1,536 x 13,312 17.6 -> 12.8 / 21.7 -> 14.8, 1,536 x 4,480 8.0 -> 7.6 / 9.8 -> 8.4, 2,048 x 4,224 7.9 -> 7.7 /
 // 9.5 -> 8.5, 768 x 8,192 11.1 -> 8.6 / 13.6 -> 10.0; not so 1,024 x 4,096 6.9 -> 7.4 / 8.6 -> 8.1 and 2,048 x 2,048 5.5 -> 6.8 / 6.1 -> 7.1.  Four slices were
-// slower than two (2,048 x 8,192 at 16 rows 12.5 where two took 11.4).
-inline void slice_direct(ResidentPlan &p, int M, int K, int ntiles, int rt, size_t ws_bytes, bool have_ws, int cus) {
-    if (M <= 8 || K <= 4096 || 2 * ntiles > cus) return;
+// slower than two (2,048 x 8,192 at 16 rows 12.5 where two took 11.4).  `forced`: 1 keeps K whole, others leave the choice here.
+inline void slice_direct(ResidentPlan &p, int M, int K, int ntiles, int rt, size_t ws_bytes, bool have_ws, int cus, int forced) {
+    if (forced == 1 || M <= 8 || K <= 4096 || 2 * ntiles > cus) return;
     if (!have_ws || resident_workspace_need(ntiles, 2, rt) > ws_bytes || (size_t)ntiles * sizeof(int) > kCounterBytes) return;
     p.S = 2;
     p.slice = (K + 255) / 256 * 128;
