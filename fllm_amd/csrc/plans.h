@@ -298,6 +298,20 @@ inline TilePlan tile_plan(long tiles256, long tiles128, int K, int asked, int ha
     return p;
 }
 
+// The row tile of both products of `pairs` (row, pick) pairs grouped by expert, `up` and `down` column tiles wide, with K_up and K_down steps: of 256
+// and 128 the one whose two products take fewer rounds over the compute units, weighted with their K; how many row tiles the experts fill is known on
+// the device alone, so half a tile an expert is assumed on top of the pairs.  On a tie (a round that could be halves) 128: tiles of 256 cost their
+// halves' order and more rows that are not there (microseconds of 256 / 128, both products, tokens that pick two: 4 x 1,024 x 1,024 at 512 and 1,024
+// 43.5 / 42.1 and 46.2 / 45.1, 8 x 2,048 x 1,024 at 512 67.2 / 65.6).
+inline int grouped_row_tile(long pairs, long experts, long up, long down, int K_up, int K_down, int halves) {
+    auto cost = [&](int bm) {
+        const long rows = (pairs + experts * bm / 2 + bm - 1) / bm;
+        if (bm == 256 && halves) return rounds_with_halves(rows * up) * K_up + rounds_with_halves(rows * down) * K_down;
+        return (bm == 256 ? 1.0 : kShortRound) * ((double)((rows * up + 255) / 256) * K_up + (double)((rows * down + 255) / 256) * K_down);
+    };
+    return cost(256) < cost(128) ? 256 : 128;
+}
+
 // Whether a plain product (neither bias nor activation) goes to the tiles, or to the GEMM library: K of 2,048 at least and nine tenths of the rounds
 // filled, in tiles (whole rounds) or, where a last round runs as halves, in outputs: such a round is short because half of the device is enough for it,
 // and what its tiles do for rows that are not there counts all the more.  Microseconds library / halves by share, one MI355X, weights from memory:

@@ -243,8 +243,7 @@ int down_slices(long pairs, int E, int N, int inter) {
 }
 
 // The row tile of gemm_tiles.h for both products of a step's pairs, 0 where the tiles above serve: steps of few pairs an expert, sizes that are
-// no whole pieces.  Of 256 and 128 the one whose two products take fewer rounds over the compute units, weighted with their K; how many
-// row tiles the experts fill is known on the device alone, so half a tile an expert is assumed on top of the pairs.
+// no whole pieces.
 int large_row_tile(long pairs, int E, int inter, int K, int N, int up_columns, const void *x, int ldx, long x_rows, const void *out) {
     using namespace fllm_tiles;
     if (pairs / E < kLargeTilePairs || K % 128 != 0 || inter % 128 != 0 || K < 256 || inter < 256 || N % 8 != 0) return 0;
@@ -252,12 +251,7 @@ int large_row_tile(long pairs, int E, int inter, int K, int N, int up_columns, c
     const uint64_t most = 1ull << 32;      // byte offsets of 32 bits
     if ((uint64_t)x_rows * ldx * 2 >= most || (uint64_t)pairs * inter * 2 >= most || (uint64_t)2 * inter * K * 2 >= most || (uint64_t)N * inter * 2 >= most)
         return 0;
-    auto cost = [&](int bm) {
-        const long rows = (pairs + (long)E * bm / 2 + bm - 1) / bm, up = rows * ((inter + up_columns - 1) / up_columns), down = rows * ((N + 255) / 256);
-        if (bm == 256 && fllm_option_half_tiles()) return fllm_plan::rounds_with_halves(up) * K + fllm_plan::rounds_with_halves(down) * inter;
-        return (bm == 256 ? 1.0 : fllm_plan::kShortRound) * ((double)((up + 255) / 256) * K + (double)((down + 255) / 256) * inter);
-    };
-    return cost(256) <= cost(128) ? 256 : 128;
+    return fllm_plan::grouped_row_tile(pairs, E, (inter + up_columns - 1) / up_columns, (N + 255) / 256, K, inter, fllm_option_half_tiles());
 }
 
 // Both products on those tiles, behind group_pairs_kernel and (where the picks' weights scale the rows) scaled_rows_kernel.

@@ -185,6 +185,14 @@ int main() {
         const TilePlan p = tile_plan((m.rows + 255) / 256 * cols, (m.rows + 127) / 128 * cols, m.K, 0, 1);
         REQUIRE(plain_takes_tiles(m.rows, m.columns, m.K, p) == m.tiles, "%d columns of %d, %ld rows", m.columns, m.K, m.rows);
     }
+    // experts' row tiles where both were measured: experts x inner width x width, tokens that pick two
+    struct { int experts, inter, width, tokens, rows; } grouped[] = {
+        {4, 1024, 1024, 512, 128}, {4, 1024, 1024, 1024, 128}, {4, 1024, 1024, 1500, 128}, {8, 2048, 1024, 512, 128}, {4, 1024, 1024, 2048, 256},
+        {8, 2048, 1024, 1024, 256}, {8, 4480, 1536, 1900, 256}, {16, 1408, 2048, 1024, 256}, {16, 1408, 2048, 512, 128}, {8, 7168, 2048, 1900, 256}};
+    for (auto &m : grouped) {
+        const int got = grouped_row_tile(2L * m.tokens, m.experts, (m.inter + 127) / 128, (m.width + 255) / 256, m.width, m.inter, 1);
+        REQUIRE(got == m.rows, "%d experts of %d x %d, %d tokens: tiles of %d rows", m.experts, m.inter, m.width, m.tokens, got);
+    }
     // ---- decode attention ----
     for (int head_dim : {32, 64, 128}) {      // a wave's 64 keys; one row of one head group, and the part that tips the choice
         const int unit = decode_unit(head_dim), last = 16 * unit - 31;
