@@ -57,13 +57,17 @@ int main() {
                     // ---- up to 16 rows ----
                     for (int M : {1, 3, 8, 9, 16})
                         for (int rt = 1; rt <= 2; rt++)
-                            for (int forced : {0, 2, 4, 8})
+                            for (int forced : {0, 1, 2, 4, 8})
                                 for (int xd = 0; xd < 2; xd++) {
                                     const int nt = rt == 2 ? 8 : 16;
                                     const int ntiles = (int)ceil_div(rt == 2 ? N / 2 : N, nt);
                                     if (ntiles == 0) continue;
-                                    const ResidentPlan p = plan_resident(M, K, ntiles, rt, ws_bytes, have_ws, xd != 0, forced);
+                                    ResidentPlan p = plan_resident(M, K, ntiles, rt, ws_bytes, have_ws, xd != 0, forced);
                                     if (p.S == 0) continue;      // declined: the caller says so
+                                    if (xd) {
+                                        slice_direct(p, M, K, ntiles, rt, ws_bytes, have_ws, cus, forced);
+                                        REQUIRE(p.S == 1 || (p.S == 2 && forced != 1 && M > 8 && 2 * ntiles <= cus && p.stage == 0), "direct slices %d", p.S);
+                                    }
                                     slices_cover(K, p.S, p.slice, "resident");
                                     REQUIRE(p.slice % 128 == 0, "resident slice %d", p.slice);
                                     REQUIRE(p.smem * p.per_cu <= kLdsBytes, "resident LDS %zu x %d", p.smem, p.per_cu);
@@ -91,10 +95,15 @@ int main() {
                                 const int nt = rt == 2 ? 8 : 16;
                                 const int ntiles = (int)ceil_div(rt == 2 ? N / 2 : N, nt);
                                 if (ntiles == 0) continue;
-                              for (int waves : {0, 4, 7, 8}) {
-                                const ChunkPlan c = plan_chunks_balanced(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, waves);
-                                REQUIRE(c.waves == 4 || c.waves == 7 || c.waves == 8, "chunks waves %d", c.waves);
-                                REQUIRE(waves == 0 || c.waves == waves, "chunks waves %d forced %d", c.waves, waves);
+                              for (int waves : {-1, 0, 4, 6, 7, 8}) {      // -1: without a copy
+                                const ChunkPlan c = waves < 0 ? plan_chunks(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, 4)
+                                                              : plan_chunks_even(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, waves);
+                                REQUIRE(c.waves == 4 || (waves >= 0 && c.waves >= 6 && c.waves <= 8), "chunks waves %d", c.waves);
+                                REQUIRE(waves <= 0 || c.waves == waves, "chunks waves %d forced %d", c.waves, waves);
+                                if (waves == 0)
+                                    REQUIRE(chunk_plan_cost(c, ntiles, cus) <=
+                                                chunk_plan_cost(plan_chunks_balanced(K, ntiles, mt, rt, ws_bytes, have_ws, cus, forced, 0), ntiles, cus),
+                                            "chunks: %d waves leave more than four, seven or eight", c.waves);
                                 REQUIRE(c.grid / c.S <= (int)ceil_div(ntiles, c.waves), "chunks grid %d beyond the row groups", c.grid);
                                 slices_cover(K, c.S, c.slice, "chunks");
                                 REQUIRE(c.grid >= 1 && c.grid % c.S == 0, "chunks grid %d S %d", c.grid, c.S);
@@ -134,6 +143,16 @@ int main() {
                                 }
                             }
                 }
+    // six waves where they leave the least: q/k/v of 6,144 x 4,096 in four slices; and not where seven do
+    const ChunkPlan six = plan_chunks_even(4096, 384, 3, 1, (size_t)192 << 20, true, 256, 0, 0);
+    REQUIRE(six.waves == 6 && six.S == 4 && six.grid == 256, "%d waves, %d slices, %d workgroups", six.waves, six.S, six.grid);
+    REQUIRE(plan_chunks_even(4096, 1792, 3, 1, (size_t)192 << 20, true, 256, 0, 0).waves == 7, "1,792 tiles");
+    // two slices of products of 9 to 16 rows: K beyond 4,096, tiles for half of the compute units at most
+    for (auto &t : {std::vector<int>{9, 4104, 128, 2}, {16, 8192, 1, 2}, {16, 4096, 128, 1}, {8, 8192, 128, 1}, {16, 8192, 129, 1}}) {
+        ResidentPlan p = plan_resident(t[0], t[1], t[2], 1, (size_t)192 << 20, true, true, 0);
+        slice_direct(p, t[0], t[1], t[2], 1, (size_t)192 << 20, true, 256, 0);
+        REQUIRE(p.S == t[3], "%d rows, %d tiles of %d: %d slices", t[0], t[2], t[1], p.S);
+    }
     // 49 to 64 rows, tiles of 16: slices for one workgroup a compute unit where that is four of them, but for one tile over
     struct { int tiles, K, mt, rt; bool copy; int slices; } sums[] = {
         {256, 4096, 4, 1, false, 4}, {256, 4096, 4, 1, true, 4}, {256, 14336, 4, 1, true, 4}, {256, 16384, 4, 1, true, 8}, {256, 16384, 4, 1, false, 4},

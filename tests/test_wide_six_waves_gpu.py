@@ -1,5 +1,6 @@
 """Products of 17 to 64 rows by workgroups of six waves: with the same K slices they add what workgroups of four add, in the same order, so no bit differs;
-row groups that six divides, that end short, and fewer tiles than waves.  The plan takes six where they leave the least to the busiest compute unit."""
+row groups that six divides, that end short, and fewer tiles than waves.  Left to the plan, 384 tiles of K 4,096 run as four slices of six waves, and another
+shape as the plan likes."""
 import pytest
 import torch
 
@@ -16,7 +17,7 @@ def ops():
 
 
 @pytest.mark.parametrize("M", [17, 32, 48, 64])
-@pytest.mark.parametrize("heads,kv,d,slices", [(4, 1, 32, 1), (6, 3, 64, 2), (32, 8, 64, 4), (3, 1, 64, 0)])
+@pytest.mark.parametrize("heads,kv,d,slices", [(4, 1, 32, 1), (6, 3, 64, 2), (32, 8, 64, 4), (3, 1, 64, 1)])
 def test_six_waves_add_as_four(ops, M, heads, kv, d, slices):
     from fllm_amd.kernels import PreparedNorm
     K, page, pages = 2048, 16, 64
@@ -31,7 +32,7 @@ def test_six_waves_add_as_four(ops, M, heads, kv, d, slices):
     cos, sin = torch.randn((64, d // 2), generator=gen).cuda(), torch.randn((64, d // 2), generator=gen).cuda()
     stream = torch.randn((M, N), generator=gen).cuda()
     assert ops.tile_for_decode(w)
-    ops.set_option("linear.slices", slices or 1)
+    ops.set_option("linear.slices", slices)
     made = []
     for waves in (4, 6):
         ops.set_option("linear.wide_waves", waves)
@@ -50,3 +51,23 @@ def test_six_waves_add_as_four(ops, M, heads, kv, d, slices):
     c, s = cos[pos.long()].double()[:, None], sin[pos.long()].double()[:, None]
     turned = torch.stack((y[..., 0] * c - y[..., 1] * s, y[..., 1] * c + y[..., 0] * s), -1).reshape(M, heads * d)
     assert (made[1][0].double() - turned).abs().max() <= 2.0 ** -8 * turned.abs().max()
+
+
+@pytest.mark.parametrize("M", [17, 40, 64])
+@pytest.mark.parametrize("N,K,slices,waves", [(6144, 4096, 4, 6), (1000, 3072, None, None)])
+def test_as_planned(ops, M, N, K, slices, waves):
+    gen = torch.Generator().manual_seed(M + N)
+    w = (torch.randn((N, K), generator=gen) * K ** -0.5).to(torch.bfloat16).cuda()
+    x, stream = torch.randn((M, K), generator=gen).to(torch.bfloat16).cuda(), torch.randn((M, N), generator=gen).cuda()
+    assert ops.tile_for_decode(w)
+    planned = stream.clone()
+    ops.linear(x, w, planned, accumulate=True)
+    want = stream.double() + x.double() @ w.double().t()
+    assert (planned.double() - want).abs().max() <= 2.0 ** -11 * want.abs().max()
+    if slices:
+        ops.set_option("linear.slices", slices)
+        ops.set_option("linear.wide_waves", waves)
+        asked = stream.clone()
+        ops.linear(x, w, asked, accumulate=True)
+        assert torch.equal(planned, asked)
+    ops.forget_copy(w)
