@@ -23,7 +23,8 @@ def host_form(source: str) -> str:
     assert "asm" not in source and source.count('#include "common.h"') == 1
     kernels = source.split("// The kernels, products of their own")
     assert len(kernels) == 2
-    return kernels[0].replace('#include "common.h"', "").replace("#pragma once", "") + "\n}  // namespace fllm_tiles\n"
+    meeting = re.search(r"^__device__ __forceinline__ bool meet_slices\(.*?^\}$", kernels[1], re.S | re.M).group(0)
+    return kernels[0].replace('#include "common.h"', "").replace("#pragma once", "") + "\n" + meeting + "\n}  // namespace fllm_tiles\n"
 
 
 def test_half_tiles_are_read_after_they_arrive_and_before_they_are_asked_for_again(tmp_path):
