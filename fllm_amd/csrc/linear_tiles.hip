@@ -66,7 +66,7 @@ extern "C" int fllm_linear_tiles(const void *x, int ldx, const void *w, const fl
         size_t bytes = 0;
         const bool have_ws = fllm_device_workspace(&base, &bytes);
         const long tiles = (long)((M + 127) / 128) * ((N + 255) / 256);
-        a.slices = fllm_plan::tile_slices(tiles, K, bytes, have_ws, fllm_option_tile_slices());
+        a.slices = fllm_plan::tile_slices(M, tiles, K, bytes, have_ws, fllm_option_tile_slices());
         if (a.slices > 1) {
             a.counters = (int *)base;
             a.parts = (float *)((unsigned char *)base + fllm_plan::kCounterBytes);

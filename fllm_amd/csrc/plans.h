@@ -331,10 +331,16 @@ inline bool plain_takes_tiles(long M, long N, int K, const TilePlan &p) {
 // taken (2,048 x 8,192 at 1,500 rows, two slices of 96 tiles 61.3 -> 61.8, at 405 rows, 128 workgroups 31.3 -> 37.2).  Microseconds library -> slices:
 // 2,048 x 8,192 at 1,024 / 1,735 / 2,048 rows 51 -> 45 / 72 -> 66 / 75 -> 69; 1,536 x 13,312 at 700 / 1,500 / 1,735 65 -> 50 / 99 -> 73 / 89 -> 77 (float32 results
 // 98 -> 79); 1,536 x 8,960 at 1,500 / 1,735 66 -> 55 / 62 -> 57; 4,096 x 14,336 at 257 / 405 / 1,024 75 -> 58 / 86 -> 69 / 139 -> 117.
+// Few rows: the tiles' own time is then the weights' way from memory, and the library's kernels for such rows are as good up to longer K.  Up to 128 rows
+// K of 18,432 at least (65 rows: 16,384 x 8,192 64.5 -> 81.0, 8,192 x 16,384 64.7 -> 85.3, 28,672 x 12,288 154 -> 169, but 16,384 x 10,240 81 -> 75; from
+// there on 8,192 x 18,432 135 -> 74, x 28,672 187 -> 102, 20,480 x 20,480 204 -> 157, 16,384 x 24,576 186 -> 192), up to 200 rows 10,240 (8,192 x 8,192 at
+// 140 / 180 / 200 rows 49.8 -> 53.9 / 48.6 -> 52.7 / 53.7 -> 52.7, x 8,960 at 140 52 -> 55; 4,096 x 14,336 at 150 58 -> 51, 8,192 x 12,288 at 140 71 -> 63,
+// 6,144 x 10,240 at 150 89 -> 52, 5,120 x 12,288 at 129 49 -> 53).
 // `asked`: 0 never, 1 planned, more: as many as that and K allow.
 inline size_t tile_slices_need(long tiles128, int slices) { return kCounterBytes + (size_t)tiles128 * slices * 128 * 256 * kF32; }
-inline int tile_slices(long tiles128, int K, size_t ws_bytes, bool have_ws, int asked) {
-    if (asked == 0 || !have_ws || K % 64 != 0 || tiles128 < 1 || tiles128 > 128 || (asked == 1 && K < 8192)) return 1;
+inline int tile_slices_from(long rows) { return rows > 200 ? 8192 : rows > 128 ? 10240 : 18432; }
+inline int tile_slices(long rows, long tiles128, int K, size_t ws_bytes, bool have_ws, int asked) {
+    if (asked == 0 || !have_ws || K % 64 != 0 || tiles128 < 1 || tiles128 > 128 || (asked == 1 && K < tile_slices_from(rows))) return 1;
     const int least = asked > 1 ? 3 : 32;      // steps a slice; the kernel needs three
     long s = asked > 1 ? asked : 256 / tiles128;
     if (s > 256 / tiles128) s = 256 / tiles128;
