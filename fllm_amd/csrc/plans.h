@@ -70,7 +70,8 @@ inline ResidentPlan plan_resident(int M, int K, int ntiles, int rt, size_t ws_by
 // two slices, whose workgroups fill the device.  What it costs is the tile's way through memory, about 1 us.  Microseconds at 9 / 16 rows whole ->
 // sliced: 2,048 x 8,192 11.8 -> 10.2 / 14.7 -> 11.3, 1,536 x 13,312 17.6 -> 12.8 / 21.7 -> 14.8, 1,536 x 4,480 8.0 -> 7.6 / 9.8 -> 8.4, 2,048 x 4,224 7.9 -> 7.7 /
 // 9.5 -> 8.5, 768 x 8,192 11.1 -> 8.6 / 13.6 -> 10.0; not so 1,024 x 4,096 6.9 -> 7.4 / 8.6 -> 8.1 and 2,048 x 2,048 5.5 -> 6.8 / 6.1 -> 7.1.  Four slices were
-// slower than two (2,048 x 8,192 at 16 rows 12.5 where two took 11.4).  `forced`: 1 keeps K whole, others leave the choice here.
+// slower than two (2,048 x 8,192 at 16 rows 12.5 where two took 11.4).  Over 16 to 2,048 columns of K 4,104 to 28,672, with a copy and without, stored
+// and added, at 9 and 16 rows: 0.56 to 0.96 of the time whole (220 products; 16 x 28,672 the most).  `forced`: 1 keeps K whole, others leave the choice here.
 inline void slice_direct(ResidentPlan &p, int M, int K, int ntiles, int rt, size_t ws_bytes, bool have_ws, int cus, int forced) {
     if (forced == 1 || M <= 8 || K <= 4096 || 2 * ntiles > cus) return;
     if (!have_ws || resident_workspace_need(ntiles, 2, rt) > ws_bytes || (size_t)ntiles * sizeof(int) > kCounterBytes) return;
@@ -260,7 +261,8 @@ inline SlabPlan plan_slab(int M, int n_tiles, int K, int mt, int rt, bool norm, 
 // K that the tiles can walk: in steps of 64, two steps a trip and four at least (256 rows), three at least (128 rows).
 inline bool row_tile_takes(int bm, int K) { return bm == 256 ? K % 128 == 0 && K >= 256 : bm == 128 && K % 64 == 0 && K >= 192; }
 // 256 or 128: the row tile whose rounds over the 256 compute units take less; 0: shapes they do not take.  A round of 128-row tiles takes
-// kShortRound of one of 256-row tiles (measured 0.54 to 0.64: 28,672 columns of 4,096 57 against 89 us, 16,384 of 2,048 30 against 53).
+// kShortRound of one of 256-row tiles (measured 0.54 to 0.64: 28,672 columns of 4,096 57 against 89 us, 16,384 of 2,048 30 against 53; over
+// several rounds 0.63 to 0.67).
 // `asked`: 256 or 128 where a caller wants that one, 0 or 1 where it leaves the choice here.
 constexpr double kShortRound = 0.62;
 inline int row_tile(long tiles256, long tiles128, int K, int asked = 0) {
@@ -271,10 +273,12 @@ inline int row_tile(long tiles256, long tiles128, int K, int asked = 0) {
 }
 
 // The row tile and whether a last round of at most 128 tiles of 256 rows runs as halves (twice as many tiles of 128 rows), which leaves no more
-// than half of the compute units idle for 0.6 to 0.7 of a round instead of a whole one; a fuller round would take two of them.  `rounds`: the time
-// in rounds of whole 256-row tiles over the compute units.  Measured without -> with, microseconds: 28,672 columns of 4,096 at 700 / 1,100 / 2,048
-// rows (2, 3, 4 rounds before) 170 -> 150 / 257 -> 239 / 368 -> 352; 17,920 of 1,536 at 1,024 / 2,048 75 -> 63 / 116 -> 106; both products of eight
-// experts of 4,480 of 1,536, 1,900 tokens that pick two 228 -> 209.
+// than half of the compute units idle, for 0.73 to 0.85 of a round instead of a whole one (28,672 columns of 4,096 at 768 rows 0.74, 16,384 of 2,048 at
+// 1,280 0.73, 57,344 of 8,192 at 1,024 0.85); a fuller round would take two of them.  `rounds`: the time in rounds of whole 256-row tiles over the
+// compute units, a round of halves counted as kShortRound like one of 128-row tiles alone: where halves are planned by that they were ahead of whole
+// rounds and of 128-row tiles at all 38 shapes measured.  Without -> with, microseconds: 28,672 columns of 4,096 at 700 / 1,200 / 2,048 rows (2, 3, 4
+// rounds before) 167 -> 150 / 259 -> 238 / 368 -> 352; 17,920 of 1,536 at 1,024 / 2,048 75 -> 63 / 116 -> 106; both products of eight experts of 4,480
+// of 1,536, 1,900 tokens that pick two 228 -> 209.
 struct TilePlan {
     int bm = 0;                 // 0: a shape the tiles do not take
     bool halves = false;
@@ -331,6 +335,8 @@ inline bool plain_takes_tiles(long M, long N, int K, const TilePlan &p) {
 // taken (2,048 x 8,192 at 1,500 rows, two slices of 96 tiles 61.3 -> 61.8, at 405 rows, 128 workgroups 31.3 -> 37.2).  Microseconds library -> slices:
 // 2,048 x 8,192 at 1,024 / 1,735 / 2,048 rows 51 -> 45 / 72 -> 66 / 75 -> 69; 1,536 x 13,312 at 700 / 1,500 / 1,735 65 -> 50 / 99 -> 73 / 89 -> 77 (float32 results
 // 98 -> 79); 1,536 x 8,960 at 1,500 / 1,735 66 -> 55 / 62 -> 57; 4,096 x 14,336 at 257 / 405 / 1,024 75 -> 58 / 86 -> 69 / 139 -> 117.
+// Over 512 to 8,192 columns of K 8,192 to 16,384 at 225 to 2,048 rows 0.45 to 1.0 (1,280 x 12,288 at 1,700 92 -> 62; float32 results of K 8,192 up to 1.07,
+// 1,280 columns at 1,300 rows 42 -> 45), of K 28,672 0.27 to 0.7.
 // Few rows: the tiles' own time is then the weights' way from memory, and the library's kernels for such rows are as good up to longer K.  Up to 128 rows
 // K of 18,432 at least (65 rows: 16,384 x 8,192 64.5 -> 81.0, 8,192 x 16,384 64.7 -> 85.3, 28,672 x 12,288 154 -> 169, but 16,384 x 10,240 81 -> 75; from
 // there on 8,192 x 18,432 135 -> 74, x 28,672 187 -> 102, 20,480 x 20,480 204 -> 157, 16,384 x 24,576 186 -> 192), up to 200 rows 10,240 (8,192 x 8,192 at
