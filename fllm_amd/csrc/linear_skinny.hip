@@ -46,6 +46,9 @@ struct SkinnyArgs {
     const float *bias;
     void *out;
     int ldo;
+    // gated epilogue: g' * sigmoid(act_alpha g') * (u' + act_offset), g' = min(g, act_limit), u' = clamp(u, +-act_limit)
+    // (act_limit <= 0: nothing is clamped).  SwiGLU is alpha 1, offset 0, no limit.
+    float act_limit, act_alpha, act_offset;
     int M, N, K;
     int S, slice;  // K is cut into S slices of `slice` elements (a multiple of 128); a workgroup stages one slice
     int ssq_off;   // byte offset of the sums of squares in LDS (behind the staging / reduction area)
@@ -68,9 +71,6 @@ struct SkinnyArgs {
     // SCALED prologue
     const float *ssq_in;   // [M, ssq_count]
     int ssq_count;
-    // gated epilogue: g' * sigmoid(act_alpha g') * (u' + act_offset), g' = min(g, act_limit), u' = clamp(u, +-act_limit)
-    // (act_limit <= 0: nothing is clamped).  SwiGLU is alpha 1, offset 0, no limit.
-    float act_limit, act_alpha, act_offset;
     int relu_squared;          // STORE epilogue: max(sum, 0)^2 instead of the sum
 #ifdef FLLM_TIMELINE
     unsigned long long *timeline;   // measurement builds only: [workgroup][8] times of the 100 MHz clock
@@ -310,6 +310,12 @@ __device__ __forceinline__ void epilogue(const SkinnyArgs &a, f32x4_t (&s)[RT], 
 // into LDS, and see slice_direct in plans.h) it leaves the item's sums in the workspace and counts the item; the workgroup that
 // counts a tile's last item adds the S partial sums in slice order and runs the epilogue, so the
 // result does not depend on which workgroup came last.
+//
+// Between a launch and its first load of weights lies nothing that can be had before: what the addresses need are the kernel's
+// first arguments, which arrive in registers with the wave (-amdgpu-kernarg-preload-count), the divisions are the host's (tstride workgroups a
+// slice, which have `items` tiles each and the first `more` of them one more), and what the epilogue needs is asked for behind
+// the weights.  Arguments out of memory, the grid's size out of another line of it and three divisions were 0.5 to 0.8 us of every
+// launch: two decode steps of the 1B sizes 1.424 -> 1.355 ms, of four at 8 rows of the 8B sizes 12.95 -> 12.75.
 enum { TM_ROWS16 = 0, TM_DUALK = 1, TM_GATEUP = 2, TM_HALVES = 3 };
 
 // A load of weights.  Every weight is read once a step, so the loads from the tile-major copies carry the
@@ -330,7 +336,8 @@ __device__ __forceinline__ bf16x8_t load_weights(const bf16_t *p) {
 
 template <int PRO, int EPI, int TM, int WAVES, bool XD, bool WT = false>
 __global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4, 4)))   // 16 waves a CU: 128 registers
-skinny_resident_kernel(SkinnyArgs a, int red_off) {
+skinny_resident_kernel(const bf16_t *w, const void *x0, int K, int slice, int M, int N, int S, int tstride, int items, int more, int ldx,
+                       SkinnyArgs a, int red_off) {
     static_assert(!XD || PRO == PRO_BF16, "activations straight from global memory: the bfloat16 prologue only");
     constexpr int U = 4;                           // k-steps of 32 per block: four 16-byte loads per lane
     constexpr int KB = 32 * U;                     // K elements of one range per block
@@ -342,20 +349,19 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int r = lane & 15, g = lane >> 4;
-    const int M = a.M, N = a.N, K = a.K, S = a.S;
     FLLM_STAMP(a, 0);
+    a.M = M, a.N = N, a.K = K;      // the epilogue reads these, too
     const int n_out = EPI == EPI_SWIGLU ? N / 2 : N;
-    const int ntiles = (n_out + NT - 1) / NT;
-    const int pitch = a.slice + 8;
+    const int pitch = slice + 8;
     bf16_t *xs = (bf16_t *)smem;                                  // [M][pitch]
     f32x4_t *red = (f32x4_t *)(smem + red_off);                   // [WAVES][64], TM_HALVES: one for each half
     float *ssq_part = (float *)(smem + a.ssq_off);                // [WAVES][16]
 
-    const int sl = blockIdx.x % S;
-    const int tile0 = blockIdx.x / S, tstride = gridDim.x / S;
-    const int ks0 = sl * a.slice;
-    const int kcn = min(K, ks0 + a.slice) - ks0;                  // a multiple of 8
-    const int my_items = tile0 < ntiles ? (ntiles - tile0 + tstride - 1) / tstride : 0;
+    int sl = 0, tile0 = blockIdx.x;
+    if (S > 1) tile0 /= S, sl = blockIdx.x - tile0 * S;
+    const int ks0 = sl * slice;
+    const int kcn = min(K, ks0 + slice) - ks0;                    // a multiple of 8
+    const int my_items = items + (tile0 < more ? 1 : 0);
     // the wave's contiguous part of the slice (relative to ks0), in steps of 64, and its blocks (the same number for every wave)
     const int kwlen = ((kcn + WAVES - 1) / WAVES + 63) / 64 * 64;
     const int kw0 = min(kcn, wave * kwlen), kw1 = min(kcn, kw0 + kwlen);
@@ -390,24 +396,34 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
                 // A tile of 8 rows is half of a copied one: 128 bytes of each quarter of the k-steps of both K halves.
                 const int tile = tile0 + l_item * tstride;
                 const int tile16 = TM == TM_DUALK ? tile >> 1 : tile, row16 = TM == TM_DUALK ? (tile & 1) * 8 + (r & 7) : r;
-                const bf16_t *wp = a.w_tiles + (size_t)tile16 * 16 * K + (size_t)((ks0 + kb - g * 8) / 32) * (16 * 32) + (g * 16 + row16) * 8;
+                const bf16_t *wp = w + (size_t)tile16 * 16 * K + (size_t)((ks0 + kb - g * 8) / 32) * (16 * 32) + (g * 16 + row16) * 8;
 #pragma unroll
                 for (int u = 0; u < U; u++) buf.w[u] = kb + u * 32 < ke ? load_weights<true>(wp + u * (16 * 32)) : zero8();
             } else {
-                const bf16_t *wp = a.w + (size_t)row * K + ks0 + kb;
+                const bf16_t *wp = w + (size_t)row * K + ks0 + kb;
 #pragma unroll
                 for (int u = 0; u < U; u++) buf.w[u] = kb + u * 32 < ke ? load_weights<false>(wp + u * 32) : zero8();
             }
             if (XD) {
-                const bf16_t *xp = (const bf16_t *)a.x + (size_t)xrow_i * a.ldx + ks0 + kb;
+                const bf16_t *xp = (const bf16_t *)x0 + (size_t)xrow_i * ldx + ks0 + kb;
 #pragma unroll
                 for (int u = 0; u < U; u++) buf.x[XD ? u : 0] = (kb + u * 32 < ke && xvalid) ? *(const bf16x8_t *)(xp + u * 32) : zero8();
             }
         }
         if (++l_j == nbw) l_j = 0, l_item++;
     };
-    // SCALED: the parts of the sums of squares of this wave's rows (rows wave and wave + WAVES) are asked for before
-    // anything else and added up after the staging, when they have long arrived: up to 256 parts a row, four a lane
+#ifndef FLLM_BLOCKS_IN_FLIGHT
+#define FLLM_BLOCKS_IN_FLIGHT 2
+#endif
+    constexpr int NB = XD ? 2 : FLLM_BLOCKS_IN_FLIGHT;      // blocks of weights a wave has asked for ahead of its products
+    Block bl[NB];
+    const int m_out = TM == TM_DUALK ? (r & 7) : r;
+    EpilogueOperands eo;
+#pragma unroll
+    for (int i = 0; i < NB; i++) issue(bl[i]);      // in flight while the activations are staged
+    load_row_place<EPI>(a, m_out, eo);
+    // SCALED: the parts of the sums of squares of this wave's rows (rows wave and wave + WAVES) are asked for behind
+    // the first weights and added up after the staging, when they have long arrived: up to 256 parts a row, four a lane
     f32x4_t ssq_pre[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     const bool ssq_quick = PRO == PRO_SCALED && a.ssq_count <= 4 * kWave && (a.ssq_count & 3) == 0 && ((uintptr_t)a.ssq_in & 15) == 0;
     if (PRO == PRO_SCALED && ssq_quick && sl == 0) {
@@ -417,25 +433,13 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
             if (m < M && lane * 4 < a.ssq_count) ssq_pre[k] = *(const f32x4_t *)(a.ssq_in + (size_t)m * a.ssq_count + lane * 4);
         }
     }
-#ifndef FLLM_BLOCKS_IN_FLIGHT
-#define FLLM_BLOCKS_IN_FLIGHT 2
-#endif
-    constexpr int NB = XD ? 2 : FLLM_BLOCKS_IN_FLIGHT;      // blocks of weights a wave has asked for ahead of its products
-    Block bl[NB];
-    const int m_out = TM == TM_DUALK ? (r & 7) : r;
-    EpilogueOperands eo;
-    load_row_place<EPI>(a, m_out, eo);      // ahead of the weights: loads come back in their order, and the page waits for these
-#pragma unroll
-    for (int i = 0; i < NB; i++) issue(bl[i]);      // in flight while the activations are staged
     // what the epilogue reads besides the sums: the part that belongs to this lane's row now, the part that belongs
     // to an item when the wave whose turn it is to finish the item starts on it
     const bool owner = WHOLE ? true : (g < 2 && (TM == TM_GATEUP || r < 8));
-    load_row_page<EPI>(a, m_out, eo);
     auto item_operands = [&](int it) {
         if (it < my_items && wave == (it & (WAVES - 1)) && owner)
             load_item_operands<EPI>(a, m_out, (tile0 + it * tstride) * NT + g * 4, n_out, eo);
     };
-    item_operands(0);
 
     // the wave's own columns kw0 .. kw1 of every row
     if (PRO != PRO_BF16 && lane < 16) ssq_part[wave * 16 + lane] = 0.f;
@@ -461,16 +465,16 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
         for (int cw = kw0; cw < kw1; cw += 8 << at) {
             const int c0 = cw + col;
             const bool in = c0 < kw1;
-            const bf16_t *x = (const bf16_t *)a.x + ks0 + (in ? c0 : kw0);
+            const bf16_t *x = (const bf16_t *)x0 + ks0 + (in ? c0 : kw0);
             if (M <= rows_at) {
-                if (in && own < M) *(bf16x8_t *)(xs + own * pitch + c0) = *(const bf16x8_t *)(x + (size_t)own * a.ldx);
+                if (in && own < M) *(bf16x8_t *)(xs + own * pitch + c0) = *(const bf16x8_t *)(x + (size_t)own * ldx);
                 continue;
             }
             for (int m0 = 0; m0 < M; m0 += RX * rows_at) {
                 bf16x8_t v[RX];
 #pragma unroll
                 for (int i = 0; i < RX; i++)
-                    if (m0 + i * rows_at < M) v[i] = *(const bf16x8_t *)(x + (size_t)min(m0 + i * rows_at + own, M - 1) * a.ldx);
+                    if (m0 + i * rows_at < M) v[i] = *(const bf16x8_t *)(x + (size_t)min(m0 + i * rows_at + own, M - 1) * ldx);
 #pragma unroll
                 for (int i = 0; i < RX; i++) {
                     const int m = m0 + i * rows_at + own;
@@ -483,7 +487,7 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
         for (int cw = kw0; cw < kw1; cw += kWave * 8) {   // the same trips for every lane: the sums below are over the wave
             const int c0 = cw + lane * 8;
             const bool in = c0 < kw1;
-            const float *x = (const float *)a.x + ks0 + c0;
+            const float *x = (const float *)x0 + ks0 + c0;
             f32x4_t w0 = {0.f, 0.f, 0.f, 0.f}, w1 = w0;
             if (in) w0 = *(const f32x4_t *)(a.norm_w + ks0 + c0), w1 = *(const f32x4_t *)(a.norm_w + ks0 + c0 + 4);
             for (int m0 = 0; m0 < M; m0 += RB) {   // the loads of RB rows are in flight together
@@ -492,8 +496,8 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
                 for (int i = 0; i < RB; i++) {
                     xv[i][0] = xv[i][1] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
                     if (in && m0 + i < M) {
-                        xv[i][0] = *(const f32x4_t *)(x + (size_t)(m0 + i) * a.ldx);
-                        xv[i][1] = *(const f32x4_t *)(x + (size_t)(m0 + i) * a.ldx + 4);
+                        xv[i][0] = *(const f32x4_t *)(x + (size_t)(m0 + i) * ldx);
+                        xv[i][1] = *(const f32x4_t *)(x + (size_t)(m0 + i) * ldx + 4);
                     }
                 }
                 auto row = [&](int i) {      // rounds a row on its way to LDS; what this lane adds to its sum of squares
@@ -540,6 +544,8 @@ skinny_resident_kernel(SkinnyArgs a, int red_off) {
         }
     }
     __builtin_amdgcn_wave_barrier();   // the wave reads what its own lanes wrote: LDS keeps a wave's accesses in order
+    load_row_page<EPI>(a, m_out, eo);
+    item_operands(0);
 
     // cursor of the products
     int item = 0, j = 0;
@@ -1311,7 +1317,8 @@ int launch_resident_plan(SkinnyArgs a, const ResidentPlan &p, int ntiles, const 
         attribute_set = true;
     }
     hipLaunchKernelGGL((skinny_resident_kernel<PRO, EPI, TM, WAVES, XD, WT>), dim3(groups * p.S), dim3(WAVES * kWave),
-                       p.smem + (TM == TM_HALVES ? p.red : 0), stream, a, (int)p.stage);
+                       p.smem + (TM == TM_HALVES ? p.red : 0), stream, WT ? a.w_tiles : a.w, a.x, a.K, p.slice, a.M, a.N, p.S, groups,
+                       ntiles / groups, ntiles % groups, a.ldx, a, (int)p.stage);
     return fllm_check_launch("linear_skinny");
 }
 

@@ -20,8 +20,11 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(_HERE), "csrc")
 LIB_NAME = "libfllm_kernels.so"
 ARCH = "gfx950"
+# kernarg-preload: a kernel's first arguments (up to 14 words of scalars and pointers, ahead of the first struct) are in registers when a
+# wave starts, instead of behind a load that misses the caches after every kernel that streams weights (0.3 us a launch in such a chain)
 HIPCC_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC",
-               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument"]
+               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=16",
+               "-Wno-unused-command-line-argument"]
 # flags of single sources: the random-weights generator must round every product and every sum on its own
 SOURCE_FLAGS = {"random_fill.hip": ["-ffp-contract=off"]}
 
