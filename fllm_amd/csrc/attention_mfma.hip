@@ -82,7 +82,7 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // smallest and the last row the largest.
 __device__ __forceinline__ int first_key(int pos, int window, int chunk) {
     int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
-    if (chunk > 0 && pos >= 0) lo = max(lo, pos - pos % chunk);
+    if (chunk > 0 && pos >= chunk) lo = max(lo, pos - pos % chunk);      // (the first chunk begins at 0: most rows need no division)
     return lo;
 }
 
@@ -663,32 +663,34 @@ __device__ __forceinline__ void store2(bf16_t *to, float a, float b) {
 // spilled at 128, and 133 left a compute unit one workgroup of eight waves.
 template <int D, int WAVES, int PM>
 __global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(D >= 128 ? 2 : 3)))
-attn_decode_kernel(AttnArgs p, int qtiles) {
+attn_decode_kernel(const int32_t *row_seg, const int32_t *row_pos, const int32_t *tables, int table_stride, int G, int nkv, int qtiles,
+                   int keys_per_split, int window, int chunk, int ps_shift, AttnArgs p) {
     constexpr int KD = D / 32, DT = D / 16;
     constexpr int OP = D + 2;
+    typedef const __attribute__((address_space(4))) int32_t *constant_t;      // the same for every lane: a scalar load
     // sm_m[WAVES][16], sm_l[WAVES][16], sm_o[WAVES][gq][OP]; outputs are read in pairs, so the area begins on 16 bytes behind the kernel's own
     extern __shared__ __attribute__((aligned(16))) float dsm[];
     const int row = blockIdx.x;
-    const int qtile = blockIdx.y % qtiles, kvh = blockIdx.y / qtiles;
     const int split = blockIdx.z;
-    const int G = p.heads / p.kv_heads;
+    // One trip to memory for the row's place, with the other arguments on the same trip; the next one is for the pages.
+    const int seg = ((constant_t)(uintptr_t)row_seg)[row], pos = ((constant_t)(uintptr_t)row_pos)[row];
+    asm volatile("" ::"s"(p.q), "s"(p.q_stride), "s"(p.kp), "s"(p.vp), "s"(p.out), "s"(p.counters), "s"(p.sinks));
+    int qtile = 0, kvh = blockIdx.y;
+    if (qtiles > 1) kvh /= qtiles, qtile = blockIdx.y - kvh * qtiles;
     const int gq = min(G - qtile * 16, 16);   // query heads of this workgroup
     float *sm_m = dsm, *sm_l = dsm + WAVES * 16, *sm_o = dsm + 2 * WAVES * 16;
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int c = lane & 15, g = lane >> 4;
     const int hg = qtile * 16 + c;
-    const int seg = p.row_seg[row];
     const int head = kvh * G + (hg < G ? hg : 0);        // lanes without a head of their own: computed, never stored
-    const int n = seg >= 0 ? p.row_pos[row] + 1 : 0;
-    const int lo = first_key(n - 1, p.window, p.chunk);
-    const int ps = p.page_size, psh = p.ps_shift, pmask = ps - 1, nkv = p.kv_heads;
+    const int n = seg >= 0 ? pos + 1 : 0;
+    const int lo = first_key(n - 1, window, chunk);
+    const int psh = PM == 0 ? 3 : PM == 1 ? 4 : ps_shift, ps = 1 << psh, pmask = ps - 1;
     const int first = (lo / 32) * 32;
-    const int begin = first + split * p.keys_per_split;
-    const int end = min(begin + p.keys_per_split, n);
-    // the splits that hold keys of this row; the others have nothing to add and leave at once
-    const int live_splits = p.counters ? max(1, (n - first + p.keys_per_split - 1) / p.keys_per_split) : p.splits;
-    if (p.counters && split >= live_splits) return;
-    const int32_t *tbl = p.tables + (size_t)(seg >= 0 ? seg : 0) * p.table_stride;
+    const int begin = first + split * keys_per_split;
+    const int end = min(begin + keys_per_split, n);
+    if (p.counters && split > 0 && begin >= n) return;      // a split without keys of this row has nothing to add and leaves at once
+    const int32_t *tbl = tables + (size_t)(seg >= 0 ? seg : 0) * table_stride;
 
     // A wave takes 64 neighbouring keys at a time, two blocks of 32, each two score tiles of 16.  Row c of a tile at key t is
     // key t + c, so that a load of the tile's keys (chunks 4 kk + g of 16 neighbouring tokens) is 1 KiB in a row where a page
@@ -697,8 +699,7 @@ attn_decode_kernel(AttnArgs p, int qtiles) {
     // The keys of the wave's next 64 are asked for as soon as these are multiplied, the values likewise, into the same
     // registers.  Every lane loads, so that no load sits behind a branch: a block without keys loads its neighbour's again,
     // a lane without a key of its own reads page 0.
-    typedef const __attribute__((address_space(4))) int32_t *constant_t;
-    const constant_t ctbl = (constant_t)(uintptr_t)tbl;      // a page that is the same for every lane: a scalar load
+    const constant_t ctbl = (constant_t)(uintptr_t)tbl;
     struct Pages {
         int k[4], v[2];       // pages of 16 tokens or more: k for the values as well
     };
@@ -817,6 +818,8 @@ attn_decode_kernel(AttnArgs p, int qtiles) {
         scores();
         add_values();
     }
+    // the splits that hold keys of this row
+    const int live_splits = p.counters ? max(1, (n - first + keys_per_split - 1) / keys_per_split) : p.splits;
     // the waves saw different keys: merge their statistics and outputs, two neighbouring outputs a thread
     if (g == 0) {
         sm_m[wave * 16 + c] = m_run;
@@ -1037,9 +1040,13 @@ int launch(const AttnArgs &a, int uniform_rows, int max_context, void *workspace
             attribute_set = true;
         }
         const dim3 grid(a.rows, a.kv_heads * qtiles, p.splits);
-        if (a.page_size >= 32) hipLaunchKernelGGL((attn_decode_kernel<D, WAVES, 2>), grid, dim3(WAVES * kWave), smem, stream, p, qtiles);
-        else if (a.page_size == 16) hipLaunchKernelGGL((attn_decode_kernel<D, WAVES, 1>), grid, dim3(WAVES * kWave), smem, stream, p, qtiles);
-        else hipLaunchKernelGGL((attn_decode_kernel<D, WAVES, 0>), grid, dim3(WAVES * kWave), smem, stream, p, qtiles);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(WAVES * kWave), smem, stream, p.row_seg, p.row_pos, p.tables, p.table_stride, G, p.kv_heads, qtiles,
+                               p.keys_per_split, p.window, p.chunk, p.ps_shift, p);
+        };
+        if (a.page_size >= 32) go(attn_decode_kernel<D, WAVES, 2>);
+        else if (a.page_size == 16) go(attn_decode_kernel<D, WAVES, 1>);
+        else go(attn_decode_kernel<D, WAVES, 0>);
         if (p.splits > 1 && !p.counters)
             hipLaunchKernelGGL(attn_merge_kernel<D>, dim3(a.rows, a.heads), dim3(kWave), 0, stream, p.ws_ml, p.ws_o, a.out,
                                a.heads, p.splits, p.sinks);
