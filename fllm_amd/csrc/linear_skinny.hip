@@ -693,12 +693,16 @@ skinny_resident_kernel(const bf16_t *w, const void *x0, int K, int slice, int M,
 // 2 x 14,336 x 4,096 47.7 -> 44.6, of 2 x 8,192 x 2,048 22.8 -> 16.5.  The parts of a group of slices have to be asked for ahead of a
 // barrier for the compiler, which otherwise fetches and awaits them two at a time: 4,096 x 4,096 at 40 / 64 / 128 rows 13.6 -> 13.3 / 20.3 ->
 // 18.3 / 30.7 -> 28.5, 2,048 x 8,192 15.5 -> 15.0 / 19.5 -> 17.3 / 35.7 -> 32.0.
+// As in the resident kernel, nothing that the first loads need has to be fetched: 40 rows of the 8B sizes, arguments fetched and now, q/k/v 20.9 -> 19.1
+// us, output and down 20.5 -> 20.1, gate/up 43.4 -> 43.15; a step 4.18 -> 4.08 ms.  The parts of the sums of squares behind the weights
+// were slower in gate/up (44.9).
 // WT: the weights come from their tile-major copy (fllm_tile_weights, fllm_tile_weights_gate_up), K a multiple of 256.
 // PRO_SCALED: the rows are what the product before prepared for an RMSNorm (fllm_linear_add_normed); the row's scale,
 // from the parts of its sum of squares, multiplies the finished sums.
 template <int MT, int EPI, bool WT = false, int WAVES = 4, int PRO = PRO_BF16>
 __global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
-skinny_wide_kernel(SkinnyArgs a) {
+skinny_wide_kernel(const bf16_t *w, const bf16_t *x, const float *ssq_in, int K, int slice, int M, int N, int slices_stride, int items_more, int ldx,
+                   int ssq_count, SkinnyArgs a) {
     static_assert(PRO == PRO_BF16 || PRO == PRO_SCALED, "rows arrive in bfloat16");
     constexpr int THREADS = WAVES * kWave;
     constexpr int KC = 256;                        // columns per chunk
@@ -713,18 +717,18 @@ skinny_wide_kernel(SkinnyArgs a) {
     __shared__ __attribute__((aligned(16))) bf16_t xs[2][ROWS * XP];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int r = lane & 15, g = lane >> 4;
-    const int M = a.M, N = a.N, K = a.K, S = a.S;
+    a.M = M, a.N = N, a.K = K;      // the epilogue reads these, too
     const int n_out = EPI == EPI_SWIGLU ? N / 2 : N;
     const int ntiles = (n_out + NT - 1) / NT;
-    const int ngroups = (ntiles + WAVES - 1) / WAVES;
-    const int sl = blockIdx.x % S;
-    const int rg0 = blockIdx.x / S, rstride = gridDim.x / S;
-    const int ks0 = sl * a.slice;
-    const int kcn = min(K, ks0 + a.slice) - ks0;                  // columns of this slice, a multiple of 8
+    const int S = slices_stride >> 16, rstride = slices_stride & 0xffff;      // two numbers a register (launch_wide_kernel): 14 are there
+    const int items = items_more >> 16, more = items_more & 0xffff;
+    int sl = 0, rg0 = blockIdx.x;
+    if (S > 1) rg0 /= S, sl = blockIdx.x - rg0 * S;
+    const int ks0 = sl * slice;
+    const int kcn = min(K, ks0 + slice) - ks0;                    // columns of this slice, a multiple of 8
     const int nchunks = (kcn + KC - 1) / KC;
-    const int my_items = rg0 < ngroups ? (ngroups - rg0 + rstride - 1) / rstride : 0;
+    const int my_items = items + (rg0 < more ? 1 : 0);
     const int total = my_items * nchunks;                         // chunk steps of this workgroup, the same for every wave
-    const bf16_t *x = (const bf16_t *)a.x;
 
     // weights: cursor (item, chunk) of the next chunk to ask for
     int w_item = 0, w_chunk = 0;
@@ -742,11 +746,11 @@ skinny_wide_kernel(SkinnyArgs a) {
         const int kb = w_chunk * KC + g * 8;
         if (WT) {
             // a chunk is two blocks of 128 columns of the tile, each 4 KiB in the order the lanes take it
-            const bf16_t *wp = a.w_tiles + (size_t)min(tile, ntiles - 1) * 16 * K + (size_t)((ks0 + w_chunk * KC) >> 7) * 2048 + lane * 8;
+            const bf16_t *wp = w + (size_t)min(tile, ntiles - 1) * 16 * K + (size_t)((ks0 + w_chunk * KC) >> 7) * 2048 + lane * 8;
 #pragma unroll
             for (int u = 0; u < KS; u++) buf[u] = load_weights<true>(live ? wp + (u >> 2) * 2048 + (u & 3) * 512 : zeros);
         } else {
-            const bf16_t *wp = a.w + (size_t)row * K + ks0;
+            const bf16_t *wp = w + (size_t)row * K + ks0;
 #pragma unroll
             for (int u = 0; u < KS; u++) buf[u] = load_weights<false>(live ? wp + min(kb + u * 32, kcn - 8) : zeros);
         }
@@ -758,7 +762,7 @@ skinny_wide_kernel(SkinnyArgs a) {
         for (int i = 0; i < XL; i++) {
             const int idx = threadIdx.x + i * THREADS;
             const int m = idx / (KC / 8), c = (idx - m * (KC / 8)) * 8 + chunk * KC;
-            xr[i] = *(const bf16x8_t *)((m < M && c < kcn && idx < XPIECES) ? x + (size_t)m * a.ldx + ks0 + c : zeros);
+            xr[i] = *(const bf16x8_t *)((m < M && c < kcn && idx < XPIECES) ? x + (size_t)m * ldx + ks0 + c : zeros);
         }
     };
     auto store_x = [&](const bf16x8_t (&xr)[XL], int buffer) {
@@ -771,24 +775,18 @@ skinny_wide_kernel(SkinnyArgs a) {
     };
 
     // Loads come back in the order they were asked for, so what is waited for first is asked for first: the parts of the
-    // sums of squares, two chunks of activations, two of weights.
+    // sums of squares, two chunks of activations, two of weights, none of which wants an argument that is not in a register yet.
     __shared__ float ssq_rows[PRO == PRO_SCALED ? ROWS : 1];
     constexpr int SQ = 16;                       // pieces of four parts asked for in one go
     f32x4_t sq[PRO == PRO_SCALED ? SQ : 1];
     const int sq_m = threadIdx.x >> 2, sq_q = threadIdx.x & 3;
-    const int per = (a.ssq_count + 3) / 4;
-    const int sq0 = min(sq_q * per, a.ssq_count), sq1 = min(sq0 + per, a.ssq_count);
-    const float *sq_parts = PRO == PRO_SCALED ? a.ssq_in + (size_t)min(sq_m, M - 1) * a.ssq_count : nullptr;
-    const bool sq_pieces = (per & 3) == 0 && (a.ssq_count & 3) == 0 && ((uintptr_t)a.ssq_in & 15) == 0;
+    const int per = (ssq_count + 3) / 4;
+    const int sq0 = min(sq_q * per, ssq_count), sq1 = min(sq0 + per, ssq_count);
+    const float *sq_parts = PRO == PRO_SCALED ? ssq_in + (size_t)min(sq_m, M - 1) * ssq_count : nullptr;
+    const bool sq_pieces = (per & 3) == 0 && (ssq_count & 3) == 0 && ((uintptr_t)ssq_in & 15) == 0;
     if (PRO == PRO_SCALED && sq_pieces) {
 #pragma unroll
         for (int i = 0; i < SQ; i++) sq[PRO == PRO_SCALED ? i : 0] = *(const f32x4_t *)(sq0 + 4 * i < sq1 ? sq_parts + sq0 + 4 * i : (const float *)zeros);
-    }
-    // segment, position and page of this lane's rows: the same for every item.  The pages wait for the rest, which is asked for first of all.
-    EpilogueOperands rows[DEEP ? MT : 1];
-    if (DEEP) {
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) load_row_place<EPI>(a, mt * 16 + r, rows[mt]);
     }
     bf16x8_t wa[KS], wb[KS], xa[XL], xb[XL];
     const int second = nchunks > 1 ? 1 : 0;
@@ -798,9 +796,11 @@ skinny_wide_kernel(SkinnyArgs a) {
     issue_w(wa);
     issue_w(wb);
     __builtin_amdgcn_sched_barrier(0);
+    // segment and position of this lane's rows: the same for every item.  The pages wait for them, behind the first chunk.
+    EpilogueOperands rows[DEEP ? MT : 1];
     if (DEEP) {
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) load_row_page<EPI>(a, mt * 16 + r, rows[mt]);
+        for (int mt = 0; mt < MT; mt++) load_row_place<EPI>(a, mt * 16 + r, rows[mt]);
     }
     if (PRO == PRO_SCALED) {
         // A row's sum of squares arrives in parts (up to a few hundred).  Four neighbouring threads share a row: each adds
@@ -863,6 +863,10 @@ skinny_wide_kernel(SkinnyArgs a) {
         }
         issue_w(buf);      // the chunk two ahead takes this one's registers
         store_x(DEEP ? next : now, (q + 1) & 1);
+        if (DEEP && EPI == EPI_QKV && q == 0) {
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) load_row_page<EPI>(a, mt * 16 + r, rows[mt]);
+        }
         __syncthreads();   // the next chunk is in LDS; everybody has read the one before it
         chunk = next_chunk;
         if (chunk != 0 || item >= my_items) return;      // (a step behind the last item multiplies zeros and ends nothing)
@@ -1433,7 +1437,13 @@ int launch_resident(const SkinnyArgs &a, hipStream_t stream) {
 
 template <int MT, int EPI, bool WT, int WAVES, int PRO>
 int launch_wide_kernel(const SkinnyArgs &a, int grid, hipStream_t stream) {
-    hipLaunchKernelGGL((skinny_wide_kernel<MT, EPI, WT, WAVES, PRO>), dim3(grid), dim3(WAVES * kWave), 0, stream, a);
+    constexpr int kOutputs = EPI == EPI_SWIGLU ? 8 : 16;      // of a tile
+    const int n_out = EPI == EPI_SWIGLU ? a.N / 2 : a.N, groups = ((n_out + kOutputs - 1) / kOutputs + WAVES - 1) / WAVES, per_slice = grid / a.S;
+    const int items = groups / per_slice;
+    FLLM_REQUIRE(per_slice <= 0xffff && items <= 0x7fff && a.S <= 0x7fff, "linear_wide: too many workgroups or tiles");
+    hipLaunchKernelGGL((skinny_wide_kernel<MT, EPI, WT, WAVES, PRO>), dim3(grid), dim3(WAVES * kWave), 0, stream, WT ? a.w_tiles : a.w,
+                       (const bf16_t *)a.x, a.ssq_in, a.K, a.slice, a.M, a.N, a.S << 16 | per_slice, items << 16 | groups % per_slice, a.ldx,
+                       a.ssq_count, a);
     return fllm_check_launch("linear_wide");
 }
 
