@@ -161,16 +161,19 @@ __device__ __forceinline__ void load_item_operands(const SkinnyArgs &a, int m, i
     }
 }
 
+// The row scale of the norm from the row's sum of squares: a root and two divisions, some 0.2 us where they stand between the last
+// sum and its store, so whoever knows the sum of squares first works it out while the weights are on their way.
+__device__ __forceinline__ float row_scale(const SkinnyArgs &a, float ss) { return 1.0f / sqrtf(ss / (float)a.K + a.eps); }
+
 // What happens to the finished sums of one output group: row scale of the norm, bias, then the store.
-// ss: the row's sum of squares (norm prologue).
+// scale: the row's scale (norm prologues).
 template <int PRO, int EPI, int RT>
-__device__ __forceinline__ void epilogue(const SkinnyArgs &a, f32x4_t (&s)[RT], float ss, int m, int nb, int n_out,
+__device__ __forceinline__ void epilogue(const SkinnyArgs &a, f32x4_t (&s)[RT], float scale, int m, int nb, int n_out,
                                          const EpilogueOperands &e) {
-    const int N = a.N, K = a.K;
+    const int N = a.N;
     if (PRO != PRO_BF16) {
-        const float inv = 1.0f / sqrtf(ss / (float)K + a.eps);
 #pragma unroll
-        for (int t = 0; t < RT; t++) s[t] *= inv;
+        for (int t = 0; t < RT; t++) s[t] *= scale;
     }
     if (a.bias) {
 #pragma unroll
@@ -197,8 +200,8 @@ __device__ __forceinline__ void epilogue(const SkinnyArgs &a, f32x4_t (&s)[RT], 
             const f32x4_t w = e.have ? e.next_w : *(const f32x4_t *)(a.next_w + nb);
             *(bf16x4_t *)(a.next_x + (size_t)m * a.N + nb) = pack4(sum * w);
             float sq = sum[0] * sum[0] + sum[1] * sum[1] + sum[2] * sum[2] + sum[3] * sum[3];
-            sq += __shfl_xor(sq, 16, kWave);
-            if (a.next_nt == 16) sq += __shfl_xor(sq, 32, kWave);
+            sq = sum_16_apart(sq);
+            if (a.next_nt == 16) sq = sum_32_apart(sq);
             if ((threadIdx.x & (kWave - 1)) < 16) a.next_ssq[(size_t)m * a.next_tiles + nb / a.next_nt] = sq;
         }
     } else if (EPI == EPI_STORE && whole && ((uintptr_t)a.out & 7) == 0) {
@@ -347,7 +350,7 @@ skinny_resident_kernel(const bf16_t *w, const void *x0, int K, int slice, int M,
     constexpr int RT = EPI == EPI_SWIGLU ? 2 : 1;
     static_assert((EPI == EPI_SWIGLU) == (TM == TM_GATEUP), "gate/up tiles belong to the SwiGLU epilogue");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int r = lane & 15, g = lane >> 4;
     FLLM_STAMP(a, 0);
     a.M = M, a.N = N, a.K = K;      // the epilogue reads these, too
@@ -363,10 +366,10 @@ skinny_resident_kernel(const bf16_t *w, const void *x0, int K, int slice, int M,
     const int kcn = min(K, ks0 + slice) - ks0;                    // a multiple of 8
     const int my_items = items + (tile0 < more ? 1 : 0);
     // the wave's contiguous part of the slice (relative to ks0), in steps of 64, and its blocks (the same number for every wave)
-    const int kwlen = ((kcn + WAVES - 1) / WAVES + 63) / 64 * 64;
+    const int kwlen = (int)((((unsigned)kcn + WAVES - 1) / WAVES + 63) / 64 * 64);
     const int kw0 = min(kcn, wave * kwlen), kw1 = min(kcn, kw0 + kwlen);
-    const int half = TM == TM_DUALK || TM == TM_HALVES ? kwlen / 2 : kwlen;     // the K range that one A row covers in an item (or half of one)
-    const int nbh = (half + KB - 1) / KB, nbw = TM == TM_HALVES ? 2 * nbh : nbh;
+    const int half = TM == TM_DUALK || TM == TM_HALVES ? kwlen >> 1 : kwlen;     // the K range that one A row covers in an item (or half of one)
+    const int nbh = (int)(((unsigned)half + KB - 1) / KB), nbw = TM == TM_HALVES ? 2 * nbh : nbh;
     // this lane's A row and B column: weight row in the tile, activation row, and where its K range starts
     const int kr0 = kw0 + (TM == TM_DUALK ? (r >> 3) * half : 0) + g * 8;      // relative to ks0
     const int kr1 = TM == TM_DUALK ? min(kw1, kw0 + ((r >> 3) + 1) * half) : kw1;
@@ -396,7 +399,7 @@ skinny_resident_kernel(const bf16_t *w, const void *x0, int K, int slice, int M,
                 // A tile of 8 rows is half of a copied one: 128 bytes of each quarter of the k-steps of both K halves.
                 const int tile = tile0 + l_item * tstride;
                 const int tile16 = TM == TM_DUALK ? tile >> 1 : tile, row16 = TM == TM_DUALK ? (tile & 1) * 8 + (r & 7) : r;
-                const bf16_t *wp = w + (size_t)tile16 * 16 * K + (size_t)((ks0 + kb - g * 8) / 32) * (16 * 32) + (g * 16 + row16) * 8;
+                const bf16_t *wp = w + (size_t)tile16 * 16 * K + (size_t)((unsigned)(ks0 + kb - g * 8) / 32) * (16 * 32) + (g * 16 + row16) * 8;
 #pragma unroll
                 for (int u = 0; u < U; u++) buf.w[u] = kb + u * 32 < ke ? load_weights<true>(wp + u * (16 * 32)) : zero8();
             } else {
@@ -442,18 +445,10 @@ skinny_resident_kernel(const bf16_t *w, const void *x0, int K, int slice, int M,
     };
 
     // the wave's own columns kw0 .. kw1 of every row
-    if (PRO != PRO_BF16 && lane < 16) ssq_part[wave * 16 + lane] = 0.f;
+    // sums of squares: a wave's parts of all rows; behind a prepared norm and with all of K here the rows' scales, which one wave a row has (the
+    // others leave the place alone)
+    if ((PRO == PRO_NORM_F32 || (PRO == PRO_SCALED && S > 1)) && lane < 16) ssq_part[wave * 16 + lane] = 0.f;
     __builtin_amdgcn_wave_barrier();
-    if (PRO == PRO_SCALED && sl == 0 && !ssq_quick) {
-        // the rows' sums of squares arrive in parts: wave w adds those of rows w, w + WAVES, ..., lane by lane in
-        // index order and then across the lanes, which no other row or wave changes
-        for (int m = wave; m < M; m += WAVES) {
-            float t = 0.f;
-            for (int i = lane; i < a.ssq_count; i += kWave) t += a.ssq_in[(size_t)m * a.ssq_count + i];
-            t = wave_sum(t);
-            if (lane == 0) ssq_part[wave * 16 + m] = t;
-        }
-    }
     if constexpr (!XD && PRO != PRO_NORM_F32) {
         // Ranges of 256 and 128 columns take two and four rows a load instruction, four instructions are on their way at a time: a trip to L2 takes
         // eight or sixteen rows where one row an instruction was four.  Microseconds at 16 rows behind a prepared norm: q/k/v 3,072 x 2,048
@@ -533,15 +528,20 @@ skinny_resident_kernel(const bf16_t *w, const void *x0, int K, int slice, int M,
                 }
             }
         }
-    if (PRO == PRO_SCALED && ssq_quick && sl == 0) {
+    if (PRO == PRO_SCALED && sl == 0) {
+        // the rows' sums of squares arrive in parts: wave w adds those of rows w and w + WAVES, lane by lane in
+        // index order and then across the lanes, which no other row or wave changes
+        float t[2];
 #pragma unroll
         for (int k = 0; k < 2; k++) {
-            const int m = wave + k * WAVES;
-            if (m < M) {      // the same for all lanes of the wave
-                const float t = wave_sum((ssq_pre[k][0] + ssq_pre[k][1]) + (ssq_pre[k][2] + ssq_pre[k][3]));
-                if (lane == 0) ssq_part[wave * 16 + m] = t;
-            }
+            t[k] = (ssq_pre[k][0] + ssq_pre[k][1]) + (ssq_pre[k][2] + ssq_pre[k][3]);
+            if (!ssq_quick && wave + k * WAVES < M)
+                for (int i = lane; i < a.ssq_count; i += kWave) t[k] += a.ssq_in[(size_t)(wave + k * WAVES) * a.ssq_count + i];
+            t[k] = wave_sum(t[k]);
         }
+        const int m = wave + lane * WAVES;
+        const float mine = lane == 0 ? t[0] : t[1];
+        if (lane < 2 && m < M) ssq_part[(S > 1 ? wave * 16 : 0) + m] = S > 1 ? mine : row_scale(a, mine);
     }
     __builtin_amdgcn_wave_barrier();   // the wave reads what its own lanes wrote: LDS keeps a wave's accesses in order
     load_row_page<EPI>(a, m_out, eo);
@@ -598,12 +598,18 @@ skinny_resident_kernel(const bf16_t *w, const void *x0, int K, int slice, int M,
                 if (TM == TM_GATEUP) s[RT - 1] += red[wv * kWave + lane + 32];
             }
         }
+        if (PRO == PRO_NORM_F32 && item == 0 && wave == 1 && lane < 16 && S == 1) {      // beside the first finisher: the rows' scales, for all items
+            float ss = 0.f;
+#pragma unroll
+            for (int wv = 0; wv < WAVES; wv++) ss += ssq_part[wv * 16 + lane];
+            ssq_part[lane] = row_scale(a, ss);
+        }
         __syncthreads();      // the sums have been read: the next item may overwrite them
         if (finisher) {
             do {
                 const int m = m_out, nb = tile * NT + g * 4;
                 float ss = 0.f;
-                if (PRO != PRO_BF16) {
+                if (PRO != PRO_BF16 && S > 1) {
 #pragma unroll
                     for (int wv = 0; wv < WAVES; wv++) ss += ssq_part[wv * 16 + m];
                 }
@@ -658,7 +664,7 @@ skinny_resident_kernel(const bf16_t *w, const void *x0, int K, int slice, int M,
                     __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0)
                 }
                 if (!owner || m >= M || nb >= n_out) break;
-                epilogue<PRO, EPI, RT>(a, s, ss, m, nb, n_out, eo);
+                epilogue<PRO, EPI, RT>(a, s, PRO == PRO_BF16 ? 1.f : S > 1 ? row_scale(a, ss) : ssq_part[m], m, nb, n_out, eo);
             } while (false);
         }
         item++;
@@ -776,7 +782,7 @@ skinny_wide_kernel(const bf16_t *w, const bf16_t *x, const float *ssq_in, int K,
 
     // Loads come back in the order they were asked for, so what is waited for first is asked for first: the parts of the
     // sums of squares, two chunks of activations, two of weights, none of which wants an argument that is not in a register yet.
-    __shared__ float ssq_rows[PRO == PRO_SCALED ? ROWS : 1];
+    __shared__ float scales[PRO == PRO_SCALED ? ROWS : 1];
     constexpr int SQ = 16;                       // pieces of four parts asked for in one go
     f32x4_t sq[PRO == PRO_SCALED ? SQ : 1];
     const int sq_m = threadIdx.x >> 2, sq_q = threadIdx.x & 3;
@@ -832,7 +838,7 @@ skinny_wide_kernel(const bf16_t *w, const bf16_t *x, const float *ssq_in, int K,
             const float pair = (sq_q & 1) ? t1 + t : t + t1;          // quarter 2 k, then quarter 2 k + 1
             const float other = __shfl_xor(pair, 2, kWave);
             const float sum = (sq_q & 2) ? other + pair : pair + other;
-            if (sq_q == 0 && sq_m < M) ssq_rows[sq_m] = sum;
+            if (sq_q == 0 && sq_m < M) scales[sq_m] = row_scale(a, sum);
         }
     }
     store_x(xa, 0);
@@ -884,7 +890,7 @@ skinny_wide_kernel(const bf16_t *w, const bf16_t *x, const float *ssq_in, int K,
             sums[0] = acc[mt];
             if (EPI == EPI_SWIGLU) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) sums[RT - 1][i] = __shfl(acc[mt][i], (lane + 32) & 63, kWave);
+                for (int i = 0; i < 4; i++) sums[RT - 1][i] = lanes_32_apart(acc[mt][i]).b;
             }
             acc[mt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
         };
@@ -905,7 +911,7 @@ skinny_wide_kernel(const bf16_t *w, const bf16_t *x, const float *ssq_in, int K,
             if (!owner || m >= M || nb >= n_out) return;
             EpilogueOperands own;
             if (!DEEP) load_row_operands<EPI>(a, m, own);
-            epilogue<PRO, EPI, RT>(a, sums, PRO == PRO_SCALED ? ssq_rows[m] : 0.f, m, nb, n_out, DEEP ? eo[DEEP ? mt : 0] : own);
+            epilogue<PRO, EPI, RT>(a, sums, PRO == PRO_SCALED ? scales[m] : 1.f, m, nb, n_out, DEEP ? eo[DEEP ? mt : 0] : own);
         };
         if (S == 1) {
             ask();
@@ -1135,7 +1141,7 @@ skinny_slab_kernel(SkinnyArgs a, int cells_off) {
         EpilogueOperands eo;
         load_row_operands<EPI>(a, m, eo);
         load_item_operands<EPI>(a, m, nb, n_out, eo);
-        epilogue<PRO, EPI, RT>(a, s, ss, m, nb, n_out, eo);
+        epilogue<PRO, EPI, RT>(a, s, PRO == PRO_BF16 ? 1.f : row_scale(a, ss), m, nb, n_out, eo);
     };
     auto look = [&]() __attribute__((always_inline)) {
         if (counted_tile < 0) return;
@@ -1221,7 +1227,7 @@ skinny_slab_kernel(SkinnyArgs a, int cells_off) {
             s[mt][0] = acc[mt];
             if (EPI == EPI_SWIGLU) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) s[mt][RT - 1][i] = __shfl(acc[mt][i], (lane + 32) & 63, kWave);
+                for (int i = 0; i < 4; i++) s[mt][RT - 1][i] = lanes_32_apart(acc[mt][i]).b;
             }
             acc[mt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
             ss[mt] = 0.f;
