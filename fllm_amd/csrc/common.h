@@ -184,6 +184,23 @@ template <int NW> __device__ __forceinline__ float block_sum(float v, float *scr
     for (int i = 0; i < NW; i++) total += scratch[i];
     return total;
 }
+// The same over a place that nothing has used yet: one meeting instead of two.
+template <int NW> __device__ __forceinline__ float block_sum_once(float v, float *scratch /* NW floats, this sum's own */) {
+    v = wave_sum(v);
+    if ((threadIdx.x & (kWave - 1)) == 0) scratch[threadIdx.x / kWave] = v;
+    __syncthreads();
+    float total = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; i++) total += scratch[i];
+    return total;
+}
+// Arguments that no register holds at the start of a wave, asked for here: behind the first loads, whose trip to memory theirs then shares.
+// Left to itself the compiler fetches an argument just ahead of its use, which is a trip of its own (0.3 to 0.5 us, the line is cold).
+template <typename... A> __device__ __forceinline__ void fetch_arguments(A... a) {
+    __builtin_amdgcn_sched_barrier(0);      // no load of before moves behind the wait
+    const int done[] = {([](auto one) { asm volatile("" ::"s"(one)); return 0; }(a))...};
+    (void)done;
+}
 template <int NW> __device__ __forceinline__ float block_max(float v, float *scratch) {
     v = wave_max(v);
     __syncthreads();

@@ -74,61 +74,72 @@ layernorm_kernel(const float *__restrict__ x, const int32_t *__restrict__ rows, 
 // thread loops over channels behind the sums and all it reads is on its way at once.  The first norm's value is rounded to T before
 // the convolution, as layernorm_kernel's output is.  A thread owns a channel of the state: it reads the old entries before it
 // writes any.
-template <typename T, int N>
+template <typename T, int N, int TAPS>
 __global__ void __launch_bounds__(kBlock)
-layernorm_conv_kernel(const float *__restrict__ x, const float *__restrict__ w1, float eps1, const float *__restrict__ conv, int taps,
-                      T *__restrict__ state, const int32_t *__restrict__ row_seg, const int32_t *__restrict__ slots, T *__restrict__ out1,
-                      const float *__restrict__ w2, float eps2, T *__restrict__ out2, int width) {
-    __shared__ float scratch[kWaves];
+layernorm_conv_kernel(const float *__restrict__ x, const int32_t *__restrict__ row_seg, const int32_t *__restrict__ slots,
+                      const float *__restrict__ w1, const float *__restrict__ w2 /* null: one norm */, const float *__restrict__ conv, int width, int taps_,
+                      T *__restrict__ state, T *__restrict__ out1, T *__restrict__ out2, float eps1, float eps2) {
+    __shared__ float scratch[2][kWaves];
     const int r = blockIdx.x, c = blockIdx.y * kBlock + threadIdx.x;
     const bool mine = c < width;
-    T *d1 = out1 + (size_t)r * width, *d2 = out2 == nullptr ? nullptr : out2 + (size_t)r * width;
-    const int seg = row_seg[r];
-    if (seg < 0) {      // padding row
-        if (mine) d1[c] = from_f32<T>(0.f);
-        if (mine && d2 != nullptr) d2[c] = from_f32<T>(0.f);
-        return;
-    }
-    const int keep = taps - 1;
-    T *old = state + (size_t)slots[seg] * keep * width;
-    const float *wc = conv + (size_t)c * taps;
-    T held[kMaxKeep];
-#pragma unroll
-    for (int i = 0; i < kMaxKeep; i++)
-        if (i < keep && mine) held[i] = old[(size_t)i * width + c];
-    const float *src = x + (size_t)r * width;
-    const float own = mine ? src[c] : 0.f, a1 = mine ? w1[c] : 0.f, a2 = mine && d2 != nullptr ? w2[c] : 0.f;
+    // Three trips to memory: the row's segment with everything that needs no place in the state, the segment's slot, the slot's entries,
+    // the last beside the sums over the row.  No load sits behind a condition (1,536 lanes at 16 rows 4.1 -> 3.2 us at best).
+    const int seg = row_seg[r], at_c = min(c, width - 1), taps = TAPS > 0 ? TAPS : taps_, keep = taps - 1;
+    const float *src = x + (size_t)r * width, *wc = conv + (size_t)at_c * taps;
+    const float own = src[at_c], a1 = w1[at_c], a2 = (w2 != nullptr ? w2 : w1)[at_c];
     float v[N];
+#pragma unroll
+    for (int j = 0; j < N; j++) v[j] = src[min((int)threadIdx.x + j * kBlock, width - 1)];
+    constexpr int KEEP = TAPS > 0 ? TAPS - 1 : kMaxKeep;      // at most
+    float factor[KEEP + 1];
+    if constexpr (TAPS == 4) {
+        *(f32x4_t *)factor = *(const f32x4_t *)wc;
+    } else {
+#pragma unroll
+        for (int i = 0; i <= KEEP; i++)
+            if (i < taps) factor[i] = wc[i];
+    }
+    fetch_arguments(state, out1, out2, eps1, eps2);
+    T *d1 = out1 + (size_t)r * width, *d2 = out2 == nullptr ? nullptr : out2 + (size_t)r * width;
+    // a padding row goes the whole way (a return here would be a wait ahead of the first loads) and stores zeros, no state
+    const bool padding = seg < 0;
+    const int slot = slots[max(seg, 0)];
+    T *old = state + (size_t)(padding ? 0 : slot) * keep * width;
+    T held[KEEP];
+#pragma unroll
+    for (int i = 0; i < KEEP; i++)
+        if (i < keep) held[i] = old[(size_t)i * width + at_c];
     float sum = 0.f;
 #pragma unroll
     for (int j = 0; j < N; j++) {
-        const int at = threadIdx.x + j * kBlock;
-        v[j] = at < width ? src[at] : 0.f;
+        if ((int)threadIdx.x + j * kBlock >= width) v[j] = 0.f;
         sum += v[j];
     }
-    const float mean = block_sum<kWaves>(sum, scratch) / (float)width;
+    const float mean = block_sum_once<kWaves>(sum, scratch[0]) / (float)width;
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < N; j++) {
         v[j] -= mean;
         if (threadIdx.x + j * kBlock < width) ss = fmaf(v[j], v[j], ss);
     }
-    const float var = block_sum<kWaves>(ss, scratch) / (float)width;
+    const float var = block_sum_once<kWaves>(ss, scratch[1]) / (float)width;
     if (!mine) return;
     const float inv1 = 1.0f / sqrtf(var + eps1), inv2 = 1.0f / sqrtf(var + eps2);
     const T h = from_f32<T>((own - mean) * (inv1 * a1));
     const float now = to_f32<T>(h);
     float acc = 0.f;
 #pragma unroll
-    for (int i = 0; i < kMaxKeep; i++) {      // oldest input first; entry i moves to i - 1
+    for (int i = 0; i < KEEP; i++) {      // oldest input first; entry i moves to i - 1
         if (i >= keep) break;
-        acc = fmaf(wc[i], to_f32<T>(held[i]), acc);
-        if (i > 0) old[(size_t)(i - 1) * width + c] = held[i];
+        acc = fmaf(factor[i], to_f32<T>(held[i]), acc);
+        if (i > 0 && !padding) old[(size_t)(i - 1) * width + c] = held[i];
     }
-    if (keep > 0) old[(size_t)(keep - 1) * width + c] = h;
-    acc = fmaf(wc[keep], now, acc);
-    d1[c] = from_f32<T>(now + acc);
-    if (d2 != nullptr) d2[c] = from_f32<T>((own - mean) * (inv2 * a2));
+    if (keep > 0 && !padding) old[(size_t)(keep - 1) * width + c] = h;
+#pragma unroll
+    for (int i = 0; i <= KEEP; i++)
+        if (i == keep) acc = fmaf(factor[i], now, acc);
+    d1[c] = from_f32<T>(padding ? 0.f : now + acc);
+    if (d2 != nullptr) d2[c] = from_f32<T>(padding ? 0.f : (own - mean) * (inv2 * a2));
 }
 
 __global__ void __launch_bounds__(kBlock)
@@ -200,8 +211,8 @@ gelu_side_kernel(const T *__restrict__ z, const int32_t *__restrict__ ids, const
 // such requests 12.70 -> 12.46 ms.
 template <typename T, int R>
 __global__ void __launch_bounds__(kBlock)
-side_gate_kernel(const float *__restrict__ x, const T *__restrict__ w, const int32_t *__restrict__ ids, const T *__restrict__ table, int vocab,
-                 int table_width, int offset, T *__restrict__ out, int rows, int width, int dim) {
+side_gate_kernel(const float *__restrict__ x, const T *__restrict__ w, const int32_t *__restrict__ ids, int rows, int width,
+                 const T *__restrict__ table, int vocab, int table_width, int offset, int dim, T *__restrict__ out) {
     __shared__ float part[kWaves][R];
     const int r0 = blockIdx.y * R;      // R rows a workgroup
     x += (size_t)r0 * width;
@@ -210,40 +221,45 @@ side_gate_kernel(const float *__restrict__ x, const T *__restrict__ w, const int
     rows = rows - r0 < R ? rows - r0 : R;
     const int d = blockIdx.x, lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const T *wr = w + (size_t)d * width;
+    // the row that this thread ends, if it has one: its token ahead of the products, its entry of the table beside their sums
+    const int r = threadIdx.x;
+    int id = ids[min(r, rows - 1)];
+    const int own = min((int)threadIdx.x, rows - 1);      // the row that this thread ends, if it has one: its token, behind it its table's row
+    const int own_id = ids[own];
     float acc[R];
 #pragma unroll
     for (int r = 0; r < R; r++) acc[r] = 0.f;
     for (int c0 = threadIdx.x * 8; c0 < width; c0 += kBlock * 8) {
+        // all rows' pieces are asked for before the first is used: left alone the compiler awaits row after row, eight trips to L2 (128 lanes of
+        // 1,536 at 16 rows 4.6 -> 3.6 us at best)
         float wv[8];
+        f32x4_t xv[R][2];
         load8(wr + c0, wv);
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const float *xr = x + (size_t)(r < rows ? r : 0) * width + c0;
-            const f32x4_t a = *(const f32x4_t *)xr, b = *(const f32x4_t *)(xr + 4);
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[r] = fmaf(wv[e], to_f32<T>(from_f32<T>(a[e])), acc[r]);
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[r] = fmaf(wv[4 + e], to_f32<T>(from_f32<T>(b[e])), acc[r]);
+            xv[r][0] = *(const f32x4_t *)xr, xv[r][1] = *(const f32x4_t *)(xr + 4);
         }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[r] = fmaf(wv[e], to_f32<T>(from_f32<T>(xv[r][e / 4][e % 4])), acc[r]);
     }
+    id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);      // ids are validated on the host; never read outside the table
+    const T entry = table[(size_t)id * table_width + offset + d];
+    fetch_arguments(out);
 #pragma unroll
     for (int r = 0; r < R; r++) {
         acc[r] = wave_sum(acc[r]);
         if (lane == 0) part[wave][r] = acc[r];
-    }
-    const int r = threadIdx.x;
-    float e = 0.f;
-    if (r < rows) {
-        int id = ids[r];
-        id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);      // ids are validated on the host; never read outside the table
-        e = to_f32<T>(table[(size_t)id * table_width + offset + d]);
     }
     __syncthreads();
     if (r >= rows) return;
     float z = 0.f;
 #pragma unroll
     for (int w = 0; w < kWaves; w++) z += part[w][r];
-    out[(size_t)r * dim + d] = from_f32<T>(gelu_tanh(z) * e);
+    out[(size_t)r * dim + d] = from_f32<T>(gelu_tanh(z) * to_f32<T>(entry));
 }
 
 int small_grid(size_t total) {
@@ -283,14 +299,17 @@ extern "C" int fllm_layernorm_conv(const float *x, const float *w1, float eps1, 
                      (w2 == nullptr || eps2 > 0.f), "layernorm_conv: operands missing");
     if (rows == 0) return 0;
     const dim3 grid(rows, (width + kBlock - 1) / kBlock);
-#define FLLM_LNC(T, N)                                                                                                                       \
-    hipLaunchKernelGGL((layernorm_conv_kernel<T, N>), grid, dim3(kBlock), 0, stream, x, w1, eps1, conv, taps, (T *)state, row_seg, slots,      \
-                       (T *)out1, w2, eps2, (T *)out2, width)
-#define FLLM_LNC_N(T)                                       \
-    do {                                                    \
-        if (width <= 4 * kBlock) FLLM_LNC(T, 4);            \
-        else if (width <= 8 * kBlock) FLLM_LNC(T, 8);       \
-        else FLLM_LNC(T, 32);                               \
+#define FLLM_LNC(T, N, TAPS)                                                                                                                  \
+    hipLaunchKernelGGL((layernorm_conv_kernel<T, N, TAPS>), grid, dim3(kBlock), 0, stream, x, row_seg, slots, w1, w2, conv, width, taps,       \
+                       (T *)state, (T *)out1, (T *)out2, eps1, eps2)
+    // four taps are one 16-byte load; any other number is a load each, behind a question each
+#define FLLM_LNC_N(T)                                                                      \
+    do {                                                                                   \
+        const bool four = taps == 4 && ((uintptr_t)conv & 15) == 0;                        \
+        if (four && width <= 8 * kBlock) FLLM_LNC(T, 8, 4);                                \
+        else if (width <= 4 * kBlock) FLLM_LNC(T, 4, 0);                                   \
+        else if (width <= 8 * kBlock) FLLM_LNC(T, 8, 0);                                   \
+        else FLLM_LNC(T, 32, 0);                                                           \
     } while (0)
     if (out_dtype == FLLM_F32) FLLM_LNC_N(float);
     else if (out_dtype == FLLM_BF16) FLLM_LNC_N(bf16_t);
@@ -309,8 +328,8 @@ extern "C" int fllm_side_gate(const float *x, const void *w, const int32_t *ids,
     if (rows == 0) return 0;
     if (rows > (fllm_fast_kernels_enabled() ? 32 : 8) || width % 8 != 0 || (((uintptr_t)x | (uintptr_t)w) & 15) != 0) return 1;
 #define FLLM_SIDE(T, R)                                                                                                                      \
-    hipLaunchKernelGGL((side_gate_kernel<T, R>), dim3(dim, (rows + R - 1) / R), dim3(kBlock), 0, stream, x, (const T *)w, ids,                \
-                       (const T *)table, vocab, table_width, offset, (T *)out, rows, width, dim)
+    hipLaunchKernelGGL((side_gate_kernel<T, R>), dim3(dim, (rows + R - 1) / R), dim3(kBlock), 0, stream, x, (const T *)w, ids, rows, width,   \
+                       (const T *)table, vocab, table_width, offset, dim, (T *)out)
 #define FLLM_SIDE_R(T)                            \
     do {                                          \
         if (rows == 1) FLLM_SIDE(T, 1);           \

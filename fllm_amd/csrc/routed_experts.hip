@@ -93,7 +93,7 @@ route_kernel(const T *__restrict__ h, int ldh, const T *__restrict__ w, int K, i
     float *picks = score + E;  // top: the picks' scores, until their sum is known
     const size_t r = blockIdx.x;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const int waves = blockDim.x / kWave;
+    constexpr int waves = kRouteBlock / kWave;
     auto keep = [&](int e, float z) {
         if (lane == 0) score[e] = score_mode == 0 ? 1.0f / (1.0f + expf(-z)) : z;
     };
@@ -105,7 +105,7 @@ route_kernel(const T *__restrict__ h, int ldh, const T *__restrict__ w, int K, i
         }
     }
     if (!done) {
-        for (int c = threadIdx.x; c < K; c += blockDim.x) xs[c] = to_f32<T>(h[r * ldh + c]);
+        for (int c = threadIdx.x; c < K; c += kRouteBlock) xs[c] = to_f32<T>(h[r * ldh + c]);
         __syncthreads();
         const bool vec = sizeof(T) == 2 && K % 8 == 0 && ((uintptr_t)w & 15) == 0;
         for (int e = wave; e < E; e += waves) keep(e, row_dot<T>(xs, w + (size_t)e * K, K, lane, vec));
@@ -131,7 +131,7 @@ route_grouped_kernel(const T *__restrict__ h, int ldh, const T *__restrict__ w, 
     float *picks = gsum + groups;   // top
     const size_t r = blockIdx.x;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const int waves = blockDim.x / kWave;
+    constexpr int waves = kRouteBlock / kWave;
     auto keep = [&](int e, float z, float c) {
         if (lane != 0) return;
         const float s = 1.0f / (1.0f + expf(-z));
@@ -149,7 +149,7 @@ route_grouped_kernel(const T *__restrict__ h, int ldh, const T *__restrict__ w, 
         }
     }
     if (!done) {
-        for (int c = threadIdx.x; c < K; c += blockDim.x) xs[c] = to_f32<T>(h[r * ldh + c]);
+        for (int c = threadIdx.x; c < K; c += kRouteBlock) xs[c] = to_f32<T>(h[r * ldh + c]);
         __syncthreads();
         const bool vec = sizeof(T) == 2 && K % 8 == 0 && ((uintptr_t)w & 15) == 0;
         for (int e = wave; e < E; e += waves) keep(e, row_dot<T>(xs, w + (size_t)e * K, K, lane, vec), correction[e]);

@@ -17,11 +17,55 @@ __device__ __forceinline__ int lanes_for(int n) {      // the lanes that hold so
     return lanes;
 }
 
+// Up to 64 experts the picks are made in registers, an expert a lane: a round is the wave's largest score by lane swaps and the first lane that
+// holds it, some 100 cycles, where shuffles and a pass through LDS were 500 (two of 8 experts in four groups, two kept: 1 us of a launch).
+__device__ __forceinline__ int first_lane_with(bool yes) {      // -1: none
+    const unsigned long long lanes = __ballot(yes);
+    return lanes ? __builtin_ctzll(lanes) : -1;
+}
+__device__ __forceinline__ float value_of_lane(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
+
+// `top` rounds over what the lanes hold: the largest `choice`, the lower lane among equals, taken out; the lanes' picks (of lane k the k-th), the
+// sum of their scores in order.  A round whose choices compare with nothing picks expert k: still one of the stack.
+struct LanePicks {
+    int id;
+    float score, sum;
+};
+__device__ __forceinline__ LanePicks pick_lanes(float choice, float score, int top, int lane, bool score_is_choice) {
+    LanePicks out = {0, 0.f, 0.f};
+    float left = choice > -INFINITY ? choice : -INFINITY;      // NaN: compares with nothing
+    for (int k = 0; k < top; k++) {
+        const float best = wave_max(left);
+        int at = first_lane_with(left == best && left > -INFINITY);
+        const float s = at < 0 && score_is_choice ? -INFINITY : value_of_lane(score, at < 0 ? k : at);
+        if (at < 0) at = k;
+        out.sum += s;
+        if (lane == k) out.id = at, out.score = s;
+        if (lane == at) left = -INFINITY;
+    }
+    return out;
+}
+
 // score[E]: sigmoid scores (score_mode 0) or logits whose softmax over all experts is the score (1).  ids[top] and weights[top]: the
 // `top` largest, the lower index among equals; weights with `renormalize` divided by the sum of the picks' scores (+ 1e-20), times
 // route_scale.  picks[top] is scratch.
 __device__ __forceinline__ void pick_plain(float *score, float *picks, int E, int top, int32_t *ids, float *weights, int score_mode,
                                            int renormalize, float route_scale, int lane) {
+    if (E <= kWave) {
+        float s = lane < E ? score[lane] : -INFINITY;
+        if (score_mode == 1) {
+            const float top_z = wave_max(s);
+            const float sum = wave_sum(lane < E ? expf(s - top_z) : 0.f);
+            s = lane < E ? expf(s - top_z) / sum : -INFINITY;
+        }
+        const LanePicks got = pick_lanes(s, s, top, lane, true);
+        const float factor = renormalize ? route_scale / (got.sum + 1e-20f) : route_scale;
+        if (lane < top) {
+            ids[lane] = got.id;
+            weights[lane] = (renormalize || route_scale != 1.0f) ? got.score * factor : got.score;
+        }
+        return;
+    }
     const int lanes = lanes_for(E);
     if (score_mode == 1) {   // softmax over all experts: the largest logit, the sum in index order a lane, then across lanes
         float top_z = -INFINITY;
@@ -64,8 +108,41 @@ __device__ __forceinline__ void pick_plain(float *score, float *picks, int E, in
 // picks divided by their sum (+ 1e-20), times route_scale.  gsum[groups] and picks[top] are scratch.
 __device__ __forceinline__ void pick_grouped(const float *score, float *choice, float *gsum, float *picks, int E, int top, int groups,
                                              int kept, int32_t *ids, float *weights, float route_scale, int lane) {
-    const int lanes = lanes_for(E), group_lanes = lanes_for(groups);
     const int per = E / groups;
+    if (E <= kWave) {
+        const int g = lane / per;      // this lane's expert's group, and this lane's group below
+        float c = lane < E ? choice[lane] : -INFINITY;
+        const float s = lane < E ? score[lane] : 0.f;
+        if (groups > 1) {
+            float a = -INFINITY, b = -INFINITY;
+            for (int i = 0; i < per; i++) {
+                const float v = lane < groups ? choice[lane * per + i] : -INFINITY;
+                if (v > a) b = a, a = v;
+                else if (v > b) b = v;
+            }
+            float sum = per > 1 ? a + b : a;
+            for (int k = 0; k < kept; k++) {      // the best group not yet kept: marked with +inf
+                const float left = lane < groups && sum != INFINITY && sum > -INFINITY ? sum : -INFINITY;
+                const float best = wave_max(left);
+                int at = first_lane_with(left == best && left > -INFINITY);
+                if (at < 0) {                     // sums that compare with nothing: the first group not yet kept
+                    at = first_lane_with(lane < groups && sum != INFINITY);
+                    if (at < 0) at = groups - 1;
+                }
+                if (lane == at) sum = INFINITY;
+            }
+            const unsigned long long keeps = __ballot(lane < groups && sum == INFINITY);
+            if (((keeps >> (g & 63)) & 1) == 0) c = -INFINITY;
+        }
+        const LanePicks got = pick_lanes(c, s, top, lane, false);
+        const float factor = route_scale / (got.sum + 1e-20f);
+        if (lane < top) {
+            ids[lane] = got.id;
+            weights[lane] = got.score * factor;
+        }
+        return;
+    }
+    const int lanes = lanes_for(E), group_lanes = lanes_for(groups);
     if (groups > 1) {
         for (int g = lane; g < groups; g += kWave) {      // a group counts the sum of its two largest choices (of its one, if it has one)
             float a = -INFINITY, b = -INFINITY;

@@ -89,50 +89,75 @@ short_conv_state_kernel(const T *__restrict__ x, T *__restrict__ state, const in
 // thread loops over channels and all it reads is on its way at once.  The normed value is rounded to T before it is used, as
 // the norm kernel's output would be, so that a token gives the same bits whether it came alone or in a portion.  A thread
 // owns a channel of the state: it reads the old entries before it writes any.
-template <typename T>
+// N > 0: the row (at most N * kBlock values) is asked for in one go; 0: any width.
+// Three trips to memory: the row's segment with everything that needs no place in the state, the segment's slot, the slot's entries, the
+// last beside the sum over the row; no load behind a condition (1,536 lanes at 4 rows 3.6 -> 1.8 us at best).
+template <typename T, int N, int TAPS>
 __global__ void __launch_bounds__(kBlock)
-norm_short_conv_kernel(const float *__restrict__ x, const float *__restrict__ norm_w, float eps, const float *__restrict__ w,
-                       T *__restrict__ state, const int32_t *__restrict__ row_seg, const int32_t *__restrict__ slots,
-                       T *__restrict__ out, int width, int taps) {
+norm_short_conv_kernel(const float *__restrict__ x, const int32_t *__restrict__ row_seg, const int32_t *__restrict__ slots,
+                       const float *__restrict__ norm_w, const float *__restrict__ w, T *__restrict__ state, int width, int taps_,
+                       T *__restrict__ out, float eps) {
     __shared__ float scratch[kWaves];
     const int r = blockIdx.x;
-    const int c = blockIdx.y * kBlock + threadIdx.x;
-    const int seg = row_seg[r];
-    if (seg < 0) {   // padding row
-        if (c < width) out[(size_t)r * width + c] = from_f32<T>(0.f);
-        return;
+    const int c = blockIdx.y * kBlock + threadIdx.x, at_c = min(c, width - 1);
+    const int seg = row_seg[r], taps = TAPS > 0 ? TAPS : taps_, keep = taps - 1;
+    const float *src = x + (size_t)r * width, *wc = w + (size_t)at_c * taps;
+    const float own = src[at_c], own_w = norm_w[at_c];
+    float a[N > 0 ? N : 4];
+    if constexpr (N > 0) {
+#pragma unroll
+        for (int j = 0; j < N; j++) a[j] = src[min((int)threadIdx.x + j * kBlock, width - 1)];
     }
-    const float *src = x + (size_t)r * width;
+    constexpr int KEEP = TAPS > 0 ? TAPS - 1 : kMaxKeep;      // at most
+    float factor[KEEP + 1];
+    if constexpr (TAPS == 4) {
+        *(f32x4_t *)factor = *(const f32x4_t *)wc;
+    } else {
+#pragma unroll
+        for (int i = 0; i <= KEEP; i++)
+            if (i < taps) factor[i] = wc[i];
+    }
+    fetch_arguments(out, eps);
+    // a padding row goes the whole way (a return here would be a wait ahead of the first loads) and stores zeros, no state
+    const bool padding = seg < 0;
+    const int slot = slots[max(seg, 0)];
+    T *mine = state + (size_t)(padding ? 0 : slot) * keep * width;
+    T held[KEEP];
+#pragma unroll
+    for (int i = 0; i < KEEP; i++)
+        if (i < keep) held[i] = mine[(size_t)i * width + at_c];
     float ss = 0.f;
-    for (int i0 = threadIdx.x; i0 < width; i0 += 4 * kBlock) {      // four loads on their way at once, summed in the row's order
-        float a[4];
+    if constexpr (N > 0) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) a[j] = i0 + j * kBlock < width ? src[i0 + j * kBlock] : 0.f;
+        for (int j = 0; j < N; j++) {
+            if ((int)threadIdx.x + j * kBlock >= width) a[j] = 0.f;
+            ss = fmaf(a[j], a[j], ss);
+        }
+    } else {
+        for (int i0 = threadIdx.x; i0 < width; i0 += 4 * kBlock) {      // four loads on their way at once, summed in the row's order
 #pragma unroll
-        for (int j = 0; j < 4; j++) ss = fmaf(a[j], a[j], ss);
+            for (int j = 0; j < 4; j++) a[j] = i0 + j * kBlock < width ? src[i0 + j * kBlock] : 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; j++) ss = fmaf(a[j], a[j], ss);
+        }
     }
-    ss = block_sum<kWaves>(ss, scratch);
+    ss = block_sum_once<kWaves>(ss, scratch);
     if (c >= width) return;
     const float inv = 1.0f / sqrtf(ss / (float)width + eps);
-    const int keep = taps - 1;
-    T *mine = state + (size_t)slots[seg] * keep * width;
-    const float *wc = w + (size_t)c * taps;
-    T held[kMaxKeep];
-#pragma unroll
-    for (int i = 0; i < kMaxKeep; i++)
-        if (i < keep) held[i] = mine[(size_t)i * width + c];
-    const T h = from_f32<T>(src[c] * (inv * norm_w[c]));
+    const T h = from_f32<T>(own * (inv * own_w));
     const float now = to_f32<T>(h);
     float acc = 0.f;
 #pragma unroll
-    for (int i = 0; i < kMaxKeep; i++) {      // oldest input first; entry i moves to i - 1
+    for (int i = 0; i < KEEP; i++) {      // oldest input first; entry i moves to i - 1
         if (i >= keep) break;
-        acc = fmaf(wc[i], to_f32<T>(held[i]), acc);
-        if (i > 0) mine[(size_t)(i - 1) * width + c] = held[i];
+        acc = fmaf(factor[i], to_f32<T>(held[i]), acc);
+        if (i > 0 && !padding) mine[(size_t)(i - 1) * width + c] = held[i];
     }
-    if (keep > 0) mine[(size_t)(keep - 1) * width + c] = h;
-    acc = fmaf(wc[taps - 1], now, acc);
-    out[(size_t)r * width + c] = from_f32<T>(now + acc);
+    if (keep > 0 && !padding) mine[(size_t)(keep - 1) * width + c] = h;
+#pragma unroll
+    for (int i = 0; i <= KEEP; i++)
+        if (i == keep) acc = fmaf(factor[i], now, acc);
+    out[(size_t)r * width + c] = from_f32<T>(padding ? 0.f : now + acc);
 }
 
 // ---- linear attention, one token after the other ----------------------------------------------------------------------------
@@ -310,8 +335,9 @@ gated_norm_kernel(const X *__restrict__ x, const float *__restrict__ w, float ep
 }
 
 // The same for bfloat16 rows out, widths in steps of 4 and everything on 16 (rows in float32) or 8 bytes: a thread holds NV pieces of four
-// lanes of the row, the weight and the gate, asked for at once (1,536 lanes at 4 rows: 7.4 us in two rounds lane by lane, 4.7 like this).
-template <int NV, typename X>
+// lanes of the row, the weight and the gate, asked for at once (1,536 lanes at 4 rows: 7.4 us in two rounds lane by lane, 4.7 like this; no load behind a
+// condition, which the compiler awaits before the next: 16 rows 3.1 -> 2.2 at best).
+template <int NV, typename X, bool NORMED>
 __global__ void __launch_bounds__(kBlock)
 gated_norm_vec_kernel(const X *__restrict__ x, const float *__restrict__ w, float eps, const bf16_t *__restrict__ gate, int gate_ld,
                       bf16_t *__restrict__ out, int width) {
@@ -323,8 +349,7 @@ gated_norm_vec_kernel(const X *__restrict__ x, const float *__restrict__ w, floa
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-        const int c = (i * kBlock + threadIdx.x) * 4;
-        if (c >= width) break;
+        const int c = min((i * kBlock + (int)threadIdx.x) * 4, width - 4);
         if constexpr (sizeof(X) == 4) {
             const f32x4_t a = *(const f32x4_t *)(x + r * width + c);
 #pragma unroll
@@ -335,17 +360,17 @@ gated_norm_vec_kernel(const X *__restrict__ x, const float *__restrict__ w, floa
             for (int e = 0; e < 4; e++) v[i][e] = (float)a[e];
         }
         g[i] = *(const bf16x4_t *)(gate + r * gate_ld + c);
-        if (w != nullptr) weight[i] = *(const f32x4_t *)(w + c);
+        if (NORMED) weight[i] = *(const f32x4_t *)(w + c);
     }
     float inv = 1.0f;
-    if (w != nullptr) {
+    if (NORMED) {
 #pragma unroll
         for (int i = 0; i < NV; i++) {
             if ((i * kBlock + threadIdx.x) * 4 >= width) break;
 #pragma unroll
             for (int e = 0; e < 4; e++) ss = fmaf(v[i][e], v[i][e], ss);
         }
-        inv = 1.0f / sqrtf(block_sum<kWaves>(ss, scratch) / (float)width + eps);
+        inv = 1.0f / sqrtf(block_sum_once<kWaves>(ss, scratch) / (float)width + eps);
     }
 #pragma unroll
     for (int i = 0; i < NV; i++) {
@@ -355,7 +380,7 @@ gated_norm_vec_kernel(const X *__restrict__ x, const float *__restrict__ w, floa
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             float a = v[i][e] * inv;
-            if (w != nullptr) a *= weight[i][e];
+            if (NORMED) a *= weight[i][e];
             o[e] = (bf16_t)(a * sigmoid_f((float)g[i][e]));
         }
         *(bf16x4_t *)(out + r * width + c) = o;
@@ -534,14 +559,23 @@ extern "C" int fllm_norm_short_conv(const float *x, const float *norm_w, float e
     FLLM_REQUIRE(rows >= 0 && width > 0 && taps >= 1 && taps - 1 <= kMaxKeep && eps > 0.f, "norm_short_conv: bad sizes");
     FLLM_REQUIRE(x && norm_w && w && out && row_seg && slots && (state || taps == 1), "norm_short_conv: operands missing");
     if (rows == 0) return 0;
-    if (dtype == FLLM_F32)
-        hipLaunchKernelGGL(norm_short_conv_kernel<float>, dim3(rows, (width + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, x, norm_w, eps, w, (float *)state, row_seg,
-                           slots, (float *)out, width, taps);
-    else if (dtype == FLLM_BF16)
-        hipLaunchKernelGGL(norm_short_conv_kernel<bf16_t>, dim3(rows, (width + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, x, norm_w, eps, w, (bf16_t *)state, row_seg,
-                           slots, (bf16_t *)out, width, taps);
-    else
-        FLLM_REQUIRE(false, "norm_short_conv: unknown dtype %d", dtype);
+    const dim3 grid(rows, (width + kBlock - 1) / kBlock);
+#define FLLM_NSC(T, N, TAPS)                                                                                                             \
+    hipLaunchKernelGGL((norm_short_conv_kernel<T, N, TAPS>), grid, dim3(kBlock), 0, stream, x, row_seg, slots, norm_w, w, (T *)state, width, \
+                       taps, (T *)out, eps)
+    // four taps are one 16-byte load; any other number is a load each, behind a question each
+#define FLLM_NSC_N(T)                                                      \
+    do {                                                                   \
+        const bool four = taps == 4 && ((uintptr_t)w & 15) == 0;           \
+        if (four && width <= 8 * kBlock) FLLM_NSC(T, 8, 4);                \
+        else if (width <= 8 * kBlock) FLLM_NSC(T, 8, 0);                   \
+        else FLLM_NSC(T, 0, 0);                                            \
+    } while (0)
+    if (dtype == FLLM_F32) FLLM_NSC_N(float);
+    else if (dtype == FLLM_BF16) FLLM_NSC_N(bf16_t);
+    else FLLM_REQUIRE(false, "norm_short_conv: unknown dtype %d", dtype);
+#undef FLLM_NSC_N
+#undef FLLM_NSC
     return fllm_check_launch("norm_short_conv");
 }
 
@@ -610,9 +644,14 @@ extern "C" int fllm_gated_norm(const void *x, int x_dtype, const float *w, float
     const uintptr_t bases = (uintptr_t)x | (uintptr_t)w;
     if (dtype == FLLM_BF16 && width % 4 == 0 && width <= 8 * 4 * kBlock && gate_ld % 4 == 0 && (bases & 15) == 0 &&
         (((uintptr_t)gate | (uintptr_t)out) & 7) == 0) {
-#define FLLM_GATED_VEC(NV, X)                                                                                                          \
-    hipLaunchKernelGGL((gated_norm_vec_kernel<NV, X>), dim3(rows), dim3(kBlock), 0, stream, (const X *)x, w, eps, (const bf16_t *)gate, gate_ld, \
-                       (bf16_t *)out, width)
+#define FLLM_GATED_FORM(NV, X, NORMED)                                                                                                 \
+    hipLaunchKernelGGL((gated_norm_vec_kernel<NV, X, NORMED>), dim3(rows), dim3(kBlock), 0, stream, (const X *)x, w, eps, (const bf16_t *)gate, \
+                       gate_ld, (bf16_t *)out, width)
+#define FLLM_GATED_VEC(NV, X)                              \
+    do {                                                   \
+        if (w != nullptr) FLLM_GATED_FORM(NV, X, true);    \
+        else FLLM_GATED_FORM(NV, X, false);                \
+    } while (0)
 #define FLLM_GATED_ROW(X)                              \
     do {                                               \
         if (pieces <= 2) FLLM_GATED_VEC(2, X);         \
@@ -625,6 +664,7 @@ extern "C" int fllm_gated_norm(const void *x, int x_dtype, const float *w, float
         else FLLM_REQUIRE(false, "gated_norm: unknown dtypes %d, %d", x_dtype, dtype);
 #undef FLLM_GATED_ROW
 #undef FLLM_GATED_VEC
+#undef FLLM_GATED_FORM
         return fllm_check_launch("gated_norm");
     }
 #define FLLM_GATED(X, T) hipLaunchKernelGGL((gated_norm_kernel<X, T>), dim3(rows), dim3(kBlock), 0, stream, (const X *)x, w, eps, \

@@ -146,34 +146,39 @@ postnorm_add_kernel(float *__restrict__ x, const B *__restrict__ branch, int par
 
 // The same for P float32 branches a row and widths in steps of 4: a thread holds NV pieces of four lanes of everything the row needs, asked
 // for at once, so that a row costs one wait for memory and two sums over the workgroup (two branches of 1,536 lanes at 8 rows: 9.1 us
-// lane by lane, 4.8 like this).
+// lane by lane, 4.8 like this).  What addresses and sums need are the first 14 words of the arguments, which arrive with the wave, and no
+// load sits behind a condition: a thread without lanes of its own reads the row's last ones again, an operand that is not there another one.  With conditions
+// the compiler awaited a piece before it asked for the next (one branch of 1,536 lanes at 4 and 8 rows 2.8 -> 2.0 and 3.2 -> 2.4 us at best, two at 16 rows 3.4 -> 2.4).
 template <int NV, int P, typename T>
 __global__ void __launch_bounds__(kBlock)
-postnorm_add_vec_kernel(float *__restrict__ x, const float *__restrict__ branch, const float *__restrict__ part_weights,
-                        const float *__restrict__ gain, float eps, int normalize, const float *__restrict__ next_w, float next_eps,
-                        T *__restrict__ next_out, float *__restrict__ next_ssq, int width) {
-    __shared__ float scratch[kWaves];
+postnorm_add_vec_kernel(float *__restrict__ x, const float *__restrict__ branch, const float *__restrict__ gain, const float *__restrict__ next_w,
+                        const float *__restrict__ part_weights, int width, int normalize, float eps, float next_eps,
+                        T *__restrict__ next_out, float *__restrict__ next_ssq) {
+    __shared__ float scratch[2][kWaves];
     const size_t r = blockIdx.x;
     f32x4_t v[NV], s[NV], w[NV], w2[NV], more[NV][P];
     float pw[P];
     float ss = 0.f;
+    auto mine = [&](int i) { return (i * kBlock + (int)threadIdx.x) * 4 < width; };
+    const float *after = next_w != nullptr ? next_w : gain, *scales = part_weights != nullptr ? part_weights + r * P : gain;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-        const int c = (i * kBlock + threadIdx.x) * 4;
-        if (c >= width) break;
+        const int c = min((i * kBlock + (int)threadIdx.x) * 4, width - 4);
         v[i] = *(const f32x4_t *)(branch + r * P * width + c);
 #pragma unroll
         for (int k = 1; k < P; k++) more[i][k] = *(const f32x4_t *)(branch + (r * P + k) * width + c);
         s[i] = *(const f32x4_t *)(x + r * width + c);
         w[i] = *(const f32x4_t *)(gain + c);
-        if (next_w != nullptr) w2[i] = *(const f32x4_t *)(next_w + c);
+        w2[i] = *(const f32x4_t *)(after + c);
     }
 #pragma unroll
-    for (int k = 0; k < P; k++) pw[k] = part_weights == nullptr ? 1.0f : part_weights[r * P + k];
+    for (int k = 0; k < P; k++) pw[k] = scales[k];      // (a row has four lanes at least)
+    fetch_arguments(next_out, next_ssq);
+#pragma unroll
+    for (int k = 0; k < P; k++) pw[k] = part_weights == nullptr ? 1.0f : pw[k];
     // the row's branches in index order: x * 1 + y is x + y
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-        if ((i * kBlock + threadIdx.x) * 4 >= width) break;
         v[i] *= pw[0];
 #pragma unroll
         for (int k = 1; k < P; k++)
@@ -183,33 +188,31 @@ postnorm_add_vec_kernel(float *__restrict__ x, const float *__restrict__ branch,
     float inv = 1.0f;
     if (normalize) {
 #pragma unroll
-        for (int i = 0; i < NV; i++) {
-            if ((i * kBlock + threadIdx.x) * 4 >= width) break;
+        for (int i = 0; i < NV; i++)
+            if (mine(i))
 #pragma unroll
-            for (int e = 0; e < 4; e++) ss = fmaf(v[i][e], v[i][e], ss);
-        }
-        inv = 1.0f / sqrtf(block_sum<kWaves>(ss, scratch) / (float)width + eps);
+                for (int e = 0; e < 4; e++) ss = fmaf(v[i][e], v[i][e], ss);
+        inv = 1.0f / sqrtf(block_sum_once<kWaves>(ss, scratch[0]) / (float)width + eps);
     }
     float ss2 = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-        const int c = (i * kBlock + threadIdx.x) * 4;
-        if (c >= width) break;
+        if (!mine(i)) break;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             s[i][e] += v[i][e] * inv * w[i][e];
             ss2 = fmaf(s[i][e], s[i][e], ss2);
         }
-        *(f32x4_t *)(x + r * width + c) = s[i];
+        *(f32x4_t *)(x + r * width + (i * kBlock + threadIdx.x) * 4) = s[i];
     }
     if (next_w == nullptr) return;
-    ss2 = block_sum<kWaves>(ss2, scratch);
+    ss2 = block_sum_once<kWaves>(ss2, scratch[1]);
     if (next_ssq != nullptr && threadIdx.x == 0) next_ssq[r] = ss2;
     const float inv2 = next_ssq != nullptr ? 1.0f : 1.0f / sqrtf(ss2 / (float)width + next_eps);
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         const int c = (i * kBlock + threadIdx.x) * 4;
-        if (c >= width) break;
+        if (!mine(i)) break;
         if constexpr (sizeof(T) == 2) {
             bf16x4_t b;
 #pragma unroll
@@ -260,8 +263,8 @@ extern "C" int fllm_postnorm_add(float *x, const void *branch, int branch_dtype,
     if (branch_dtype == FLLM_F32 && parts <= 4 && width % 4 == 0 && width <= (parts == 1 ? 8 : 4) * 4 * kBlock && (bases & 15) == 0 &&
         (next_dtype == FLLM_F32 || next_dtype == FLLM_BF16)) {
 #define FLLM_POSTNORM_VEC(NV, P, T)                                                                                                       \
-    hipLaunchKernelGGL((postnorm_add_vec_kernel<NV, P, T>), dim3(rows), dim3(kBlock), 0, stream, x, (const float *)branch, part_weights, gain, \
-                       eps, normalize, next_w, next_eps, (T *)next_out, next_ssq, width)
+    hipLaunchKernelGGL((postnorm_add_vec_kernel<NV, P, T>), dim3(rows), dim3(kBlock), 0, stream, x, (const float *)branch, gain, next_w, part_weights, \
+                       width, normalize, eps, next_eps, (T *)next_out, next_ssq)
 #define FLLM_POSTNORM_PARTS(NV, T)                     \
     do {                                               \
         if (parts == 1) FLLM_POSTNORM_VEC(NV, 1, T);   \
