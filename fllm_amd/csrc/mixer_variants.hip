@@ -646,31 +646,61 @@ __global__ void __launch_bounds__(kBlock) relu_squared_vec_kernel(const bf16_t *
 // 13.0 us in a decode step of two rows; like this 5.5.  TURNS false, no rotation: a kernel of its own, so that a row neither waits for nor
 // holds what a rotation needs (a step of one row of 12 + 2 heads of 128 6.1 us with the question asked in the kernel, 4.8 like this).
 // norm_mode as in normed_rope_store_kernel; rope_dims / 2 a multiple of 8.
+// A row waits for its segment and position beside everything that does not depend on them (the lanes, their weights, the values), then for the page and
+// the angles: two trips to memory.  What the first of them needs are the first 14 words of the arguments, which arrive with the wave (heads and key/value heads share
+// one, the head's lanes and the mode another, the values' and the turning lanes a third), and no load sits behind a condition (12 + 2 heads of 128 at 2 rows
+// 3.3 -> 2.4 us at best; 1,900 rows 11.7 -> 11.0).
 template <bool TURNS>
 __global__ void __launch_bounds__(kBlock)
-normed_rope_store_vec_kernel(const bf16_t *__restrict__ qkv, int ld, int norm_mode, const float *__restrict__ q_weight,
-                             const float *__restrict__ k_weight, float eps, bf16_t *__restrict__ q_out, const int32_t *__restrict__ row_pos,
-                             const int32_t *__restrict__ row_seg, const int32_t *__restrict__ tables, int table_stride,
-                             const float *__restrict__ cos_table, const float *__restrict__ sin_table, bf16_t *__restrict__ k_pages,
-                             bf16_t *__restrict__ v_pages, int heads, int kv_heads, int k_dim, int v_dim, int rope_dims, int page_size,
-                             int store_kv, int values_from_keys, const bf16_t *__restrict__ blend, int blend_ld,
-                             const float *__restrict__ blend_amount, int lanes) {
+normed_rope_store_vec_kernel(const bf16_t *__restrict__ qkv, const int32_t *__restrict__ row_pos, const int32_t *__restrict__ row_seg,
+                             const float *__restrict__ q_weight, const float *__restrict__ k_weight, int ld, int all_heads, int head_lanes, int value_rope,
+                             const float *__restrict__ cos_table, const float *__restrict__ sin_table, const int32_t *__restrict__ tables,
+                             int table_stride, int page_size, float eps, bf16_t *__restrict__ q_out, bf16_t *__restrict__ k_pages,
+                             bf16_t *__restrict__ v_pages, const bf16_t *__restrict__ blend, int blend_ld, const float *__restrict__ blend_amount) {
+    typedef const __attribute__((address_space(4))) int32_t *constant_t;      // the same for every lane: a scalar load
     __shared__ float scratch[2 * kWaves];
     const size_t r = blockIdx.x;
-    const int seg = row_seg[r], pos = row_pos[r];
+    const int seg = ((constant_t)(uintptr_t)row_seg)[r], pos = ((constant_t)(uintptr_t)row_pos)[r];
+    const int heads = all_heads & 0xffff, kv_heads = (int)((unsigned)all_heads >> 16), all = heads + kv_heads;
+    const int k_dim = head_lanes & 0xffff, lanes = (head_lanes >> 16) & 0xff, norm_mode = (head_lanes >> 24) & 3;
+    const int v_dim = value_rope & 0xffff, rope_dims = (int)((unsigned)value_rope >> 16);
+    const bool store_kv = (head_lanes >> 26) & 1, values_from_keys = (head_lanes >> 27) & 1;
     const bf16_t *row = qkv + r * ld;
-    const int each = kBlock / lanes, c = (threadIdx.x % lanes) * 8, half = rope_dims / 2;
-    const bool turns = TURNS && c < rope_dims;
-    const int pc = c < half ? c + half : c - half;              // the lanes that these turn with
-    const int all = heads + kv_heads;
+    const int each = kBlock / lanes, c = (int)(threadIdx.x & (lanes - 1)) * 8, half = rope_dims / 2;
+    const bool there = c < k_dim, turns = TURNS && c < rope_dims;
+    const int at = min(c, k_dim - 8);                           // a thread without lanes of its own reads the head's last ones
+    const int pc = turns ? (c < half ? c + half : c - half) : at;      // the lanes that these turn with
+    const int last = store_kv ? all : heads;
     float inv_q = 1.f, inv_k = 1.f;
+    // a head's lanes, the ones they turn with and the weights of both
+    bf16x8_t v, p;
+    f32x4_t w[2], wp[2];
+    auto fetch = [&](int h) __attribute__((always_inline)) {
+        const bool is_q = h < heads;
+        const bf16_t *head = row + (size_t)h * k_dim;
+        const float *weight = (is_q ? q_weight : k_weight) + (norm_mode == 2 ? (size_t)(is_q ? h : h - heads) * k_dim : 0);
+        v = *(const bf16x8_t *)(head + at);
+        if (TURNS) p = *(const bf16x8_t *)(head + pc);
+        if (norm_mode == 0) return;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            w[j] = *(const f32x4_t *)(weight + at + 4 * j);
+            if (TURNS) wp[j] = *(const f32x4_t *)(weight + pc + 4 * j);
+        }
+    };
+    const int h0 = threadIdx.x / lanes, value_lanes = kv_heads * v_dim;
+    fetch(min(h0, last - 1));
+    const bf16_t *values = row + (size_t)(values_from_keys ? heads : all) * k_dim;
+    bf16x8_t value = {};
+    if (store_kv) value = *(const bf16x8_t *)(values + min((int)threadIdx.x * 8, value_lanes - 8));
+    fetch_arguments(cos_table, sin_table, tables, table_stride, page_size, eps, q_out, k_pages, v_pages, blend, blend_ld, blend_amount);
     if (norm_mode == 2) {                                       // one norm over all of q, one over all of k
         float sq = 0.f, sk = 0.f;
         for (int e0 = threadIdx.x * 8; e0 < all * k_dim; e0 += kBlock * 8) {
-            const bf16x8_t v = *(const bf16x8_t *)(row + e0);
+            const bf16x8_t u = *(const bf16x8_t *)(row + e0);
             float ss = 0.f;
 #pragma unroll
-            for (int e = 0; e < 8; e++) ss = fmaf((float)v[e], (float)v[e], ss);
+            for (int e = 0; e < 8; e++) ss = fmaf((float)u[e], (float)u[e], ss);
             if (e0 < heads * k_dim) sq += ss;
             else sk += ss;
         }
@@ -685,34 +715,32 @@ normed_rope_store_vec_kernel(const bf16_t *__restrict__ qkv, int ld, int norm_mo
         inv_k = 1.0f / sqrtf(sk / (float)(kv_heads * k_dim) + eps);
     }
     if (seg < 0) return;                                        // padding row: its queries are never read
-    const int off = pos % page_size;
-    const int page = store_kv ? tables[(size_t)seg * table_stride + pos / page_size] : 0;
-    const float *cs = cos_table + (size_t)pos * half, *sn = sin_table + (size_t)pos * half;
-    // the lanes of a head stay together: the shuffles below reach active lanes
-    for (int h = threadIdx.x / lanes; h < (store_kv ? all : heads); h += each) {
-        const bool is_q = h < heads, there = c < k_dim;
-        bf16x8_t v = {}, p = {};
-        f32x4_t w[2], wp[2], cv[2], sv[2];
-        if (there) {
-            const bf16_t *head = row + (size_t)h * k_dim;
-            const float *weight = (is_q ? q_weight : k_weight) + (norm_mode == 2 ? (size_t)(is_q ? h : h - heads) * k_dim : 0);
-            v = *(const bf16x8_t *)(head + c);
-            if (turns) p = *(const bf16x8_t *)(head + pc);
+    const int page_at = pos / page_size, off = pos - page_at * page_size;
+    const int page = store_kv ? ((constant_t)(uintptr_t)tables)[(size_t)seg * table_stride + page_at] : 0;
+    f32x4_t cv[2], sv[2];      // the angles are the same for every head
+    if (TURNS) {
+        const size_t angle = (size_t)pos * half + (turns ? (c < half ? c : pc) : 0);
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                if (norm_mode != 0) w[j] = *(const f32x4_t *)(weight + c + 4 * j);
-                if (!turns) continue;
-                if (norm_mode != 0) wp[j] = *(const f32x4_t *)(weight + pc + 4 * j);
-                cv[j] = *(const f32x4_t *)(cs + (c < half ? c : pc) + 4 * j);
-                sv[j] = *(const f32x4_t *)(sn + (c < half ? c : pc) + 4 * j);
-            }
-        }
+        for (int j = 0; j < 2; j++) cv[j] = *(const f32x4_t *)(cos_table + angle + 4 * j), sv[j] = *(const f32x4_t *)(sin_table + angle + 4 * j);
+    }
+    // the lanes of a head stay together: what meets below reaches active lanes
+    for (int h = h0; h < last; h += each) {
+        const bool is_q = h < heads;
+        if (h != h0) fetch(h);
         float inv = is_q ? inv_q : inv_k;
         if (norm_mode == 1) {
             float ss = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; e++) ss = fmaf((float)v[e], (float)v[e], ss);
-            for (int o = lanes / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, kWave);
+            if (!there) ss = 0.f;
+            if (lanes == 16) {                                  // heads of 128: the same order without shuffles
+                ss += along_row<8>(ss);
+                ss += along_row<4>(ss);
+                ss += along_row<2>(ss);
+                ss += along_row<1>(ss);
+            } else {
+                for (int o = lanes / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, kWave);
+            }
             inv = 1.0f / sqrtf(ss / (float)k_dim + eps);
         }
         if (!there) continue;
@@ -731,18 +759,18 @@ normed_rope_store_vec_kernel(const bf16_t *__restrict__ qkv, int ld, int norm_mo
         else *(bf16x8_t *)(k_pages + key_offset(page, kv_heads, h - heads, page_size, k_dim, off, c)) = o8;
     }
     if (!store_kv) return;
-    const bf16_t *values = row + (size_t)(values_from_keys ? heads : all) * k_dim;
     const float a = blend != nullptr ? blend_amount[0] : 0.f;
-    for (int e0 = threadIdx.x * 8; e0 < kv_heads * v_dim; e0 += kBlock * 8) {
-        bf16x8_t v = *(const bf16x8_t *)(values + e0);
+    for (int e0 = threadIdx.x * 8; e0 < value_lanes; e0 += kBlock * 8) {
+        if (e0 >= kBlock * 8) value = *(const bf16x8_t *)(values + e0);
+        bf16x8_t u = value;
         if (blend != nullptr) {
             const bf16x8_t b = *(const bf16x8_t *)(blend + r * blend_ld + e0);
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = (bf16_t)((1.0f - a) * (float)v[e] + a * (float)b[e]);
+            for (int e = 0; e < 8; e++) u[e] = (bf16_t)((1.0f - a) * (float)u[e] + a * (float)b[e]);
         }
         bf16_t *dst = v_pages + ((size_t)page * kv_heads * v_dim + e0) * page_size + off;      // a head's values lie behind the head's before
 #pragma unroll
-        for (int e = 0; e < 8; e++) dst[(size_t)e * page_size] = v[e];
+        for (int e = 0; e < 8; e++) dst[(size_t)e * page_size] = u[e];
     }
 }
 
@@ -771,14 +799,14 @@ int fllm_launch_normed_rope_store(const void *qkv, int ld, int norm_mode, const 
                             (rope_dims > 0 ? (uintptr_t)cos_table | (uintptr_t)sin_table : 0) | (store_kv ? (uintptr_t)k_pages : 0);
     // whole pieces of 8 lanes everywhere, on 16 bytes (values are stored one by one); a head's threads in one wave
     if (dtype == FLLM_BF16 && rope_dims % 16 == 0 && key_chunk == 8 && k_dim % 8 == 0 && k_dim <= 8 * kWave && v_dim % 8 == 0 && ld % 8 == 0 &&
-        blend_ld % 8 == 0 && (bases & 15) == 0) {
+        blend_ld % 8 == 0 && (bases & 15) == 0 && heads <= 0xffff && kv_heads <= 0x7fff && v_dim <= 0xffff) {
         int lanes = 1;
         while (lanes < k_dim / 8) lanes *= 2;
         const auto kernel = rope_dims > 0 ? normed_rope_store_vec_kernel<true> : normed_rope_store_vec_kernel<false>;
-        hipLaunchKernelGGL(kernel, dim3(rows), dim3(kBlock), 0, stream, (const bf16_t *)qkv, ld, norm_mode, q_weight, k_weight, eps,
-                           (bf16_t *)q_out, row_pos, row_seg, tables, table_stride, cos_table, sin_table, (bf16_t *)k_pages,
-                           (bf16_t *)v_pages, heads, kv_heads, k_dim, v_dim, rope_dims, page_size, store_kv, values_from_keys,
-                           (const bf16_t *)blend, blend_ld, blend_amount, lanes);
+        const int head_lanes = k_dim | lanes << 16 | norm_mode << 24 | (store_kv ? 1 << 26 : 0) | (values_from_keys ? 1 << 27 : 0);
+        hipLaunchKernelGGL(kernel, dim3(rows), dim3(kBlock), 0, stream, (const bf16_t *)qkv, row_pos, row_seg, q_weight, k_weight, ld,
+                           heads | kv_heads << 16, head_lanes, v_dim | rope_dims << 16, cos_table, sin_table, tables, table_stride, page_size, eps,
+                           (bf16_t *)q_out, (bf16_t *)k_pages, (bf16_t *)v_pages, (const bf16_t *)blend, blend_ld, blend_amount);
         return fllm_check_launch("normed_rope_store");
     }
     if (dtype == FLLM_F32)

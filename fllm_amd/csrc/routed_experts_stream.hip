@@ -35,8 +35,8 @@ constexpr int kMostPairs = 512;
 // (a prompt and eight decode steps of twelve such layers 15.6 -> 14.5 ms).
 template <int MODE, int G, bool SHARED>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
-expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__restrict__ ids, const float *__restrict__ weights, int pairs,
-                     int top, const bf16_t *__restrict__ w, int E, int N, int K, int by_pair, bf16_t *__restrict__ act,
+expert_stream_kernel(const bf16_t *__restrict__ x, const int32_t *__restrict__ ids, const bf16_t *__restrict__ w, int ldx, int pairs, int top, int E,
+                     int N, int K, int by_pair, const float *__restrict__ weights, bf16_t *__restrict__ act,
                      float *__restrict__ out, float limit, float alpha, float up_offset, const bf16_t *__restrict__ w_shared, int shared_n,
                      int shared_k, const float *__restrict__ out_weights, int out_top) {
     static_assert(!SHARED || MODE != 0, "a shared expert comes with experts without a gate");
@@ -48,13 +48,13 @@ expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__res
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int l16 = lane & 15, lg = lane >> 4;
     const int c0 = blockIdx.x * COLS;
-    auto expert_of = [&](int p) {
-        const int e = ids[p];
-        return e < 0 ? 0 : (e >= E ? E - 1 : e);           // never outside the stack of experts
-    };
+    typedef const __attribute__((address_space(4))) int32_t *constant_t;      // the same for every lane: a scalar load
+    auto in_stack = [&](int e) { return e < 0 ? 0 : (e >= E ? E - 1 : e); };      // never outside the stack of experts
     // blockIdx.y names an expert, or (by_pair) a pair: then the first pair of an expert stands for it
-    const bool shared = SHARED && blockIdx.y == gridDim.y - 1;
-    const int e = shared ? 0 : by_pair ? expert_of(blockIdx.y) : (int)blockIdx.y;
+    const bool shared = SHARED && (int)blockIdx.y == (by_pair ? pairs : E);
+    const int first_id = ids[min(lane, pairs - 1)];        // of the first 64 pairs, on its way with the workgroup's own
+    const int own_id = ((constant_t)(uintptr_t)ids)[by_pair && !shared ? (int)blockIdx.y : 0];
+    const int e = shared ? 0 : by_pair ? in_stack(own_id) : (int)blockIdx.y;
     if (shared) {                                          // every row: `pairs` and the pointers become the shared expert's own
         if (MODE == 1) x += (size_t)pairs * ldx;
         if (MODE == 2) act += (size_t)pairs * N;
@@ -66,6 +66,18 @@ expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__res
         top = 1;
     }
     if (SHARED && c0 >= N) return;                         // the grid covers the wider of the two kinds of experts
+    const bf16_t *tiles[RT];
+#pragma unroll
+    for (int t = 0; t < RT; t++) {
+        const int c = min(c0 + (MODE == 2 ? 16 * t : 0), N - 16);      // a tile beyond the matrix reads its last one again
+        tiles[t] = w + ((size_t)e * (MODE == 0 ? 2 : 1) * N + (MODE == 0 && t == 1 ? N : 0) + c) * K + lane * 8;
+    }
+    const int k_per = ((K + kWaves - 1) / kWaves + 31) / 32 * 32;
+    const int k_begin = wave * k_per, k_end = min(K, k_begin + k_per);
+    // Ahead of the first weights lies one trip to memory, for the pairs' experts; the arguments that are not among the first 14 words (those arrive with
+    // the wave) ride on it.  It was three, an argument line, the workgroup's own pair and the list: 4,480 lanes at a width of 1,536, 2 rows
+    // with a shared expert 16.5 -> 15.2 and 14.2 -> 13.2 us, 8 rows 33.9 -> 32.3 and 19.5 -> 18.5.  Asking for the first weights ahead of the list as well spilled registers.
+    fetch_arguments(weights, act, out, limit, alpha, up_offset, out_weights, out_top);
     short *s_pair = s_pairs[wave];
     int count = 0;
     if (shared) {
@@ -74,7 +86,7 @@ expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__res
     } else {
         for (int p0 = 0; p0 < pairs; p0 += kWave) {
             const int p = p0 + lane;
-            const bool mine = p < pairs && expert_of(p) == e;
+            const bool mine = p < pairs && in_stack(p0 == 0 ? first_id : ids[min(p, pairs - 1)]) == e;
             const unsigned long long mask = __ballot(mine);
             if (mine) s_pair[count + __popcll(mask & ((1ull << lane) - 1))] = (short)p;
             count += __popcll(mask);
@@ -84,14 +96,6 @@ expert_stream_kernel(const bf16_t *__restrict__ x, int ldx, const int32_t *__res
     __threadfence_block();
     if (count == 0 || (by_pair && !shared && s_pair[0] != (int)blockIdx.y)) return;      // the same for all waves
 
-    const bf16_t *tiles[RT];
-#pragma unroll
-    for (int t = 0; t < RT; t++) {
-        const int c = min(c0 + (MODE == 2 ? 16 * t : 0), N - 16);      // a tile beyond the matrix reads its last one again
-        tiles[t] = w + ((size_t)e * (MODE == 0 ? 2 : 1) * N + (MODE == 0 && t == 1 ? N : 0) + c) * K + lane * 8;
-    }
-    const int k_per = ((K + kWaves - 1) / kWaves + 31) / 32 * 32;
-    const int k_begin = wave * k_per, k_end = min(K, k_begin + k_per);
     for (int g0 = 0; g0 < count; g0 += 16 * G) {
         const bf16_t *src[G];
         float scale[G];
@@ -185,7 +189,7 @@ void launch_groups(const void *x, int ldx, const int32_t *ids, const float *weig
     const int by_pair = pairs < E;
     const int cols = MODE == 2 ? 32 : 16, widest = sh.n > N ? sh.n : N;
     hipLaunchKernelGGL((expert_stream_kernel<MODE, G, SHARED>), dim3((widest + cols - 1) / cols, (by_pair ? (unsigned)pairs : (unsigned)E) + (SHARED ? 1 : 0)),
-                       dim3(kThreads), 0, stream, (const bf16_t *)x, ldx, ids, weights, (int)pairs, top, (const bf16_t *)w, E, N, K, by_pair,
+                       dim3(kThreads), 0, stream, (const bf16_t *)x, ids, (const bf16_t *)w, ldx, (int)pairs, top, E, N, K, by_pair, weights,
                        (bf16_t *)act, out, limit, alpha, up_offset, (const bf16_t *)sh.w, sh.n, sh.k, sh.out_weights, sh.top);
 }
 
