@@ -463,11 +463,21 @@ __device__ __forceinline__ size_t decode_part_floats(int heads, int v_dim) { ret
 // row of 1,900 keys 15.3 -> 12.4 us, 64 of 1,000 38.3 -> 30.3; GX = 8, 16 heads on eight: 20.9 -> 16.5 and 75.7 -> 55.3.
 template <int GX>
 __global__ void __launch_bounds__(kThreads, 2)
-talking_decode_kernel(const TalkArgs p) {
+talking_decode_kernel(const bf16_t *__restrict__ q, const int32_t *__restrict__ row_seg, const int32_t *__restrict__ row_pos,
+                      const int32_t *__restrict__ tables, const float *__restrict__ talk, const float *__restrict__ temp, int table_stride,
+                      int all_heads /* heads | kv_heads << 16 */, const TalkArgs p) {
     constexpr bool EXACT = GX > 0;
+    typedef const __attribute__((address_space(4))) int32_t *constant_t;      // the same for every lane: a scalar load
     constexpr int HW = kDecHeads, KSM = EXACT ? 4 : 8, TS = 2, GM = EXACT ? GX : kDecGMax;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-    const int H = p.heads, G = p.kv_heads, D = EXACT ? 128 : p.k_dim, DV = EXACT ? 128 : p.v_dim, PS = p.page_size;
+    const int H = all_heads & 0xffff, G = (int)((unsigned)all_heads >> 16), D = EXACT ? 128 : p.k_dim, DV = EXACT ? 128 : p.v_dim, PS = p.page_size;
+    // One trip to memory for the row's place, the other arguments and the first pieces of the queries and of the mix; then the pages, then keys and values.
+    // The first 14 words of the arguments are in registers when a wave starts.  (12 heads on two of 128, one row of 1,900 keys 7.05 -> 6.8 us)
+    const int row_of = blockIdx.x;      // every segment has one row: its first row is its own number, no lookup to wait for
+    const int placed = ((constant_t)(uintptr_t)row_seg)[row_of], pos = ((constant_t)(uintptr_t)row_pos)[row_of];
+    const bf16x8_t q_first = *(const bf16x8_t *)(q + (size_t)row_of * H * D + 8 * min((int)threadIdx.x, H * D / 8 - 1));
+    const float talk_first = talk[min((int)threadIdx.x, H * H - 1)], temp_first = temp[threadIdx.x % H];
+    fetch_arguments(p.k_pages, p.v_pages, p.page_size, p.page_shift, p.chunk, p.splits, p.scale, p.ws);
     const int group = H / G, KS = D / 32, DVT = DV / 16, HP = H | 1, shift = p.page_shift;
     float *tk = (float *)lds_raw;                       // [H][H]
     float *rawl = tk + H * H;                           // [64 keys][HP]
@@ -478,19 +488,16 @@ talking_decode_kernel(const TalkArgs p) {
     const int seg = blockIdx.x, split = blockIdx.y, S = p.splits;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4;
-    const int r = seg;      // every segment has one row: its first row is its own number, no lookup to wait for
+    const int r = row_of;
     const size_t out_row = (size_t)H * DV;
-    if (p.row_seg[r] < 0) {   // padding rows of a captured step
-        if (split == 0)
-            for (int i = tid; i < H * DV; i += kThreads) p.out[(size_t)r * out_row + i] = (bf16_t)0.f;
-        return;
-    }
-    const int pos = p.row_pos[r];
-    const int lo = p.chunk > 0 ? pos - pos % p.chunk : 0;
+    const bool padding = placed < 0;      // of a captured step: zeros out, no keys (a return here would be a wait ahead of the loads)
+    if (padding && split == 0)
+        for (int i = tid; i < H * DV; i += kThreads) p.out[(size_t)r * out_row + i] = (bf16_t)0.f;
+    const int lo = p.chunk > 0 && pos >= p.chunk ? pos - pos % p.chunk : 0;
     const int kb_start = lo & ~15;
-    const int32_t *tbl = p.tables + (size_t)seg * p.table_stride;
+    const int32_t *tbl = tables + (size_t)seg * table_stride;
     const int nblk = (pos - kb_start) / kKeyBlock + 1;
-    const int my_blocks = split < nblk ? (nblk - split + S - 1) / S : 0;
+    const int my_blocks = !padding && split < nblk ? (nblk - split + S - 1) / S : 0;
     auto page_of = [&](int key) __attribute__((always_inline)) { return EXACT || shift >= 0 ? key >> shift : key / PS; };
     auto in_page = [&](int key) __attribute__((always_inline)) { return EXACT || shift >= 0 ? key & (PS - 1) : key % PS; };
     auto seen = [&](int key) __attribute__((always_inline)) { return key <= pos ? key : pos; };      // beyond it: masked in step 2
@@ -524,13 +531,15 @@ talking_decode_kernel(const TalkArgs p) {
     };
     const int second = G > 1 ? 1 : 0;
     if (my_blocks > 0) pages(block_at(0));
-    for (int i = tid; i < H * D / 8; i += kThreads) *(bf16x8_t *)(qs + 8 * i) = *(const bf16x8_t *)(p.q + (size_t)r * H * D + 8 * i);
-    for (int i = tid; i < H * H; i += kThreads) tk[i] = p.talk[i] * (p.scale * p.temp[i % H]);
     if (my_blocks > 0) {
         load_keys(kf, block_at(0), kpage, 0);
         load_keys(kn, block_at(0), kpage, second);
         load_values(vf, block_at(0), vpage, 0);
     }
+    if (tid < H * D / 8) *(bf16x8_t *)(qs + 8 * tid) = q_first;
+    if (tid < H * H) tk[tid] = talk_first * (p.scale * temp_first);
+    for (int i = tid + kThreads; i < H * D / 8; i += kThreads) *(bf16x8_t *)(qs + 8 * i) = *(const bf16x8_t *)(q + (size_t)r * H * D + 8 * i);
+    for (int i = tid + kThreads; i < H * H; i += kThreads) tk[i] = talk[i] * (p.scale * temp[i % H]);
     __syncthreads();
 
     float m_run[HW], l_run[HW];
@@ -661,7 +670,7 @@ talking_decode_kernel(const TalkArgs p) {
     __syncthreads();
     float *part = S > 1 ? p.ws + ((size_t)seg * S + split) * decode_part_floats(H, DV) : nullptr;
     if (S > 1 && tid < 2 * H) part[tid] = mlv[tid];
-    if (c >= group) return;
+    if (c >= group || padding) return;
 #pragma unroll
     for (int kvh = 0; kvh < GM; kvh++) {
         if (kvh < G) {
@@ -687,35 +696,46 @@ talking_decode_kernel(const TalkArgs p) {
 }
 
 // The shares of a decode row's workgroups into its output, a workgroup a (request, head): eight groups of 32 threads take
-// every eighth share each (a thread four value lanes), then the eight partial merges meet in LDS.
-__global__ void __launch_bounds__(kThreads) talking_decode_merge_kernel(const TalkArgs p) {
+// every eighth share each (a thread four value lanes), then the eight partial merges meet in LDS.  A group asks for four of its shares at a
+// time, behind no condition: a share a trip to memory were four trips for 31 shares (3.6 -> 2.7 us at best).
+__global__ void __launch_bounds__(kThreads)
+talking_decode_merge_kernel(const float *__restrict__ ws, const int32_t *__restrict__ row_seg, const bf16_t *__restrict__ gate, bf16_t *__restrict__ out,
+                            int H, int DV, int S, int gate_stride) {
     __shared__ float gm[8], gl[8];
     __shared__ __attribute__((aligned(16))) float go[8][128];
-    const int seg = blockIdx.x, h = blockIdx.y, H = p.heads, DV = p.v_dim, S = p.splits;
+    const int seg = blockIdx.x, h = blockIdx.y;
     const int r = seg;
-    if (p.row_seg[r] < 0) return;      // a padding row: the decode kernel has written zeros
+    const bool padding = ((const __attribute__((address_space(4))) int32_t *)(uintptr_t)row_seg)[r] < 0;
     const size_t per = decode_part_floats(H, DV);
-    const float *parts = p.ws + (size_t)seg * S * per;
+    const float *parts = ws + (size_t)seg * S * per;
     const int sg = threadIdx.x >> 5, d4 = 4 * (threadIdx.x & 31);
     float m = -INFINITY, l = 0.f;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-    for (int s = sg; s < S; s += 8) {
-        const float *part = parts + s * per;
-        const float ms = part[h], ls = part[H + h];
-        f32x4_t o4 = {0.f, 0.f, 0.f, 0.f};
-        if (d4 < DV) o4 = *(const f32x4_t *)(part + 2 * H + (size_t)h * DV + d4);
-        if (ms == -INFINITY) continue;      // a share that saw no key
-        const float m_new = fmaxf(m, ms);
-        const float a = __expf(m - m_new), w = __expf(ms - m_new);      // m = -inf: a = 0
-        l = l * a + ls * w;
+    constexpr int AT = 4;      // shares of a group on their way together
+    for (int s0 = sg; s0 < S; s0 += 8 * AT) {
+        float ms[AT], ls[AT];
+        f32x4_t o4[AT];
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[e] = acc[e] * a + o4[e] * w;
-        m = m_new;
+        for (int i = 0; i < AT; i++) {
+            const float *part = parts + min(s0 + 8 * i, S - 1) * per;
+            ms[i] = part[h], ls[i] = part[H + h];
+            o4[i] = *(const f32x4_t *)(part + 2 * H + (size_t)h * DV + min(d4, DV - 4));
+        }
+#pragma unroll
+        for (int i = 0; i < AT; i++) {
+            if (s0 + 8 * i >= S || ms[i] == -INFINITY) continue;      // no share, or one that saw no key
+            const float m_new = fmaxf(m, ms[i]);
+            const float a = __expf(m - m_new), w = __expf(ms[i] - m_new);      // m = -inf: a = 0
+            l = l * a + ls[i] * w;
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[e] = acc[e] * a + o4[i][e] * w;
+            m = m_new;
+        }
     }
     if ((threadIdx.x & 31) == 0) { gm[sg] = m; gl[sg] = l; }
     if (d4 < DV) *(f32x4_t *)&go[sg][d4] = acc;
     __syncthreads();
-    if (sg != 0 || d4 >= DV) return;
+    if (sg != 0 || d4 >= DV || padding) return;      // a padding row: the decode kernel has written zeros
     float mt = -INFINITY;
 #pragma unroll
     for (int k = 0; k < 8; k++) mt = fmaxf(mt, gm[k]);
@@ -732,11 +752,11 @@ __global__ void __launch_bounds__(kThreads) talking_decode_merge_kernel(const Ta
         }
     }
     float f = lt > 0.f ? 1.0f / lt : 0.f;
-    if (p.gate != nullptr) f *= 1.0f / (1.0f + __expf(-(float)p.gate[(size_t)r * p.gate_stride + h]));
+    if (gate != nullptr) f *= 1.0f / (1.0f + __expf(-(float)gate[(size_t)r * gate_stride + h]));
     bf16x4_t r4;
 #pragma unroll
     for (int e = 0; e < 4; e++) r4[e] = (bf16_t)(tot[e] * f);
-    *(bf16x4_t *)(p.out + (size_t)r * H * DV + (size_t)h * DV + d4) = r4;
+    *(bf16x4_t *)(out + (size_t)r * H * DV + (size_t)h * DV + d4) = r4;
 }
 
 // 1: not taken
@@ -750,13 +770,17 @@ int launch_decode(const TalkArgs &a, hipStream_t stream) {
     if (lds > 60 * 1024) return 1;
     const dim3 grid(a.num_segs, a.splits), block(kThreads);
     const bool exact = a.k_dim == 128 && a.v_dim == 128 && a.page_shift >= 3;
-    if (exact && G <= 2) hipLaunchKernelGGL(talking_decode_kernel<2>, grid, block, lds, stream, a);
-    else if (exact && G <= 4) hipLaunchKernelGGL(talking_decode_kernel<4>, grid, block, lds, stream, a);
-    else if (exact) hipLaunchKernelGGL(talking_decode_kernel<kDecGMax>, grid, block, lds, stream, a);
-    else hipLaunchKernelGGL(talking_decode_kernel<0>, grid, block, lds, stream, a);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, lds, stream, a.q, a.row_seg, a.row_pos, a.tables, a.talk, a.temp, a.table_stride, H | G << 16, a);
+    };
+    if (exact && G <= 2) go(talking_decode_kernel<2>);
+    else if (exact && G <= 4) go(talking_decode_kernel<4>);
+    else if (exact) go(talking_decode_kernel<kDecGMax>);
+    else go(talking_decode_kernel<0>);
     int rc = fllm_check_launch("talking_attention (decode rows)");
     if (rc == 0 && a.splits > 1) {
-        hipLaunchKernelGGL(talking_decode_merge_kernel, dim3(a.num_segs, H), dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL(talking_decode_merge_kernel, dim3(a.num_segs, H), dim3(kThreads), 0, stream, a.ws, a.row_seg, a.gate, a.out, H,
+                           a.v_dim, a.splits, a.gate_stride);
         rc = fllm_check_launch("talking_attention (decode merge)");
     }
     return rc;
