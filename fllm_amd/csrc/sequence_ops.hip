@@ -222,31 +222,35 @@ linear_attention_kernel(const T *__restrict__ q, const T *__restrict__ k, const 
 // workgroup a (segment, head, slice of 32 value lanes), thread (g, j4) owns rows g, g + 32, .. of the four columns at 4 * j4.
 // The state is read once, 16 bytes a thread and 128 bytes a row, and written once behind the segment's last token, which is
 // all a decode step does; the sum over the rows is taken over the lanes of a wave and then over the four waves, in an order
-// that no size of the batch changes.
+// that no size of the batch changes.  Ahead of the state and the rows lie two trips to memory, the segment's rows and slot (with the arguments that
+// are not in registers) and whether it is a padding one; they were four (1,536 lanes in heads of 128 at 4 rows 4.3 -> 3.9 us at best).
 constexpr int kRowsVB = 32;
 template <typename T, int RP>
 __global__ void __launch_bounds__(kBlock)
-linear_attention_rows_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v, int ld,
+linear_attention_rows_kernel(const int32_t *__restrict__ seg_start, const int32_t *__restrict__ slots, const int32_t *__restrict__ row_seg,
+                             const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v, int ld, int dims /* dim | vdim << 16 */,
                              const float *__restrict__ decay_hi, const float *__restrict__ decay_lo, float *__restrict__ state,
-                             const int32_t *__restrict__ row_seg, const int32_t *__restrict__ seg_start,
-                             const int32_t *__restrict__ slots, float *__restrict__ out, int heads, int dim, int vdim,
-                             int activation) {
+                             float *__restrict__ out, int heads, int activation) {
     constexpr int G = kBlock / (kRowsVB / 4);      // 32 groups of rows
     __shared__ float qs[G * RP], ks[G * RP];
     __shared__ f32x4_t part[kWaves][kRowsVB / 4];
     const int seg = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * kRowsVB;
-    const int r0 = seg_start[seg], n = seg_start[seg + 1] - r0;
+    typedef const __attribute__((address_space(4))) int32_t *constant_t;      // the same for every lane: a scalar load
+    const int dim = dims & 0xffff, vdim = (int)((unsigned)dims >> 16);
+    const int r0 = ((constant_t)(uintptr_t)seg_start)[seg], r1 = ((constant_t)(uintptr_t)seg_start)[seg + 1], slot = ((constant_t)(uintptr_t)slots)[seg];
+    fetch_arguments(decay_hi, decay_lo, state, out, heads, activation);
+    const int n = r1 - r0;
     if (n <= 0) return;
     const int tid = threadIdx.x, j4 = tid & 7, g = tid >> 3;
     const int col = j0 + 4 * j4;
     const bool live = col < vdim;
     const size_t out_ld = (size_t)heads * vdim;
-    if (row_seg[r0] < 0) {   // padding rows: no state is touched
+    if (((constant_t)(uintptr_t)row_seg)[r0] < 0) {   // padding rows: no state is touched
         if (g == 0 && live)
             for (int t = 0; t < n; t++) *(f32x4_t *)(out + (size_t)(r0 + t) * out_ld + (size_t)h * vdim + col) = f32x4_t{0.f, 0.f, 0.f, 0.f};
         return;
     }
-    float *mine = state + ((size_t)slots[seg] * heads + h) * dim * vdim;
+    float *mine = state + ((size_t)slot * heads + h) * dim * vdim;
     f32x4_t S[RP];
 #pragma unroll
     for (int p = 0; p < RP; p++) {
@@ -598,11 +602,11 @@ extern "C" int fllm_linear_attention(const void *q, const void *k, const void *v
         FLLM_REQUIRE(form != 2, "linear_attention: heads of %d and %d lanes are not the chunked kernel's", dim, vdim);
     }
     // values in groups of four lanes: the state passes through registers
-    if (vdim % 4 == 0 && dim <= 256) {
+    if (vdim % 4 == 0 && vdim <= 0xffff && dim <= 256) {
         const dim3 grid(num_segs, heads, (vdim + kRowsVB - 1) / kRowsVB);
 #define FLLM_ROWS(T, RP)                                                                                                          \
-    hipLaunchKernelGGL((linear_attention_rows_kernel<T, RP>), grid, dim3(kBlock), 0, stream, (const T *)q, (const T *)k,          \
-                       (const T *)v, ld, decay_hi, decay_lo, state, row_seg, seg_start, slots, out, heads, dim, vdim, activation)
+    hipLaunchKernelGGL((linear_attention_rows_kernel<T, RP>), grid, dim3(kBlock), 0, stream, seg_start, slots, row_seg,           \
+                       (const T *)q, (const T *)k, (const T *)v, ld, dim | vdim << 16, decay_hi, decay_lo, state, out, heads, activation)
 #define FLLM_ROWS_OF(T)                                                                                                           \
     do {                                                                                                                          \
         if (dim <= 32) FLLM_ROWS(T, 1);                                                                                           \
