@@ -63,26 +63,37 @@ constexpr int kMostSplits = 32;
 __device__ __forceinline__ void publish(float *at, float v) { __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // VARIANT 0: window + pooled blocks, softmax.  VARIANT 1: every key up to the row, sigmoid weights.
-template <int KD, int VT, int VARIANT>
+// What bounds a step of single rows is its chain of trips to memory: the row's place with the arguments that are not in registers when a wave starts
+// (the first 14 words are), its pages, its keys and values (of the pooled blocks as well: both are asked for before a score is known), and the
+// hand-over of the shares: windows of 1,024 with pooled blocks, 2 rows of 12 heads on two of 128 13.9 -> 12.5 us, sigmoid weights 10.3 -> 9.9.
+// Pages of a power of two have instances of their own: divisions by the page size, or the question at each address, cost more than they
+// save (2,000 rows 57 us with divisions, 63 with the question, 55 like this).
+template <int KD, int VT, int VARIANT, bool POW2>
 __global__ void __launch_bounds__(kThreads)
-mixer_tile_kernel(const TileParams p) {
+mixer_tile_kernel(const int32_t *__restrict__ row_seg, const int32_t *__restrict__ row_pos, const int32_t *__restrict__ tables,
+                  const bf16_t *__restrict__ q, int table_stride, int heads, int kv_heads, int q_stride, int by_heads, int page_shift,
+                  const TileParams p) {
+    typedef const __attribute__((address_space(4))) int32_t *constant_t;      // the same for every lane: a scalar load
     constexpr int D = KD * 32, DV = VT * 16;
     __shared__ float sm_o[kWavesM][16][DV + 1];
     __shared__ float sm_m[kWavesM][16], sm_l[kWavesM][16];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int qi = lane & 15, g = lane >> 4;
-    const int G = p.heads / p.kv_heads;
     // ---- which queries this tile holds
-    int seg = -1, row0 = 0, count = 0, kvh = 0, head0 = 0;
-    if (p.by_heads) {
+    int seg = -1, row0 = 0, count = 0, kvh = 0, head0 = 0, pos_here = 0;
+    if (by_heads) {
         row0 = blockIdx.x;
-        seg = p.row_seg[row0];
+        seg = ((constant_t)(uintptr_t)row_seg)[row0], pos_here = ((constant_t)(uintptr_t)row_pos)[row0];
+        fetch_arguments(p.k_pages, p.v_pages, p.page_size, p.scale, p.window, p.pool, p.slots, p.splits, p.parts, p.counters, p.out, p.rows, pos_here);
+    }
+    const int G = heads / kv_heads;
+    if (by_heads) {
         kvh = blockIdx.y;
         head0 = kvh * G;
         count = G;
         if (seg < 0) {      // padding row: zeros
             if (blockIdx.z == 0)
-                for (int i = threadIdx.x; i < G * DV; i += kThreads) p.out[((size_t)row0 * p.heads + head0) * DV + i] = (bf16_t)0.f;
+                for (int i = threadIdx.x; i < G * DV; i += kThreads) p.out[((size_t)row0 * heads + head0) * DV + i] = (bf16_t)0.f;
             return;
         }
     } else {
@@ -103,16 +114,18 @@ mixer_tile_kernel(const TileParams p) {
         kvh = head0 / G;
     }
     const bool valid = qi < count;
-    const int my_row = p.by_heads ? row0 : row0 + (valid ? qi : 0);
-    const int my_head = p.by_heads ? head0 + (valid ? qi : 0) : head0;
-    const int my_pos = p.row_pos[my_row];
-    const int pos_min = p.row_pos[row0], pos_max = p.by_heads ? pos_min : p.row_pos[row0 + count - 1];
-    const int32_t *tbl = p.tables + (size_t)seg * p.table_stride;
+    const int my_row = by_heads ? row0 : row0 + (valid ? qi : 0);
+    const int my_head = by_heads ? head0 + (valid ? qi : 0) : head0;
+    const int my_pos = by_heads ? pos_here : row_pos[my_row];
+    const int pos_min = by_heads ? pos_here : row_pos[row0], pos_max = by_heads ? pos_here : row_pos[row0 + count - 1];
+    const int32_t *tbl = tables + (size_t)seg * table_stride;
     const int ps = p.page_size;
+    auto page_of = [&](int key) __attribute__((always_inline)) { return POW2 ? key >> page_shift : key / ps; };
+    auto in_page = [&](int key) __attribute__((always_inline)) { return POW2 ? key & (ps - 1) : key % ps; };
     // ---- Q^T as the B operand: column = the lane's query, k = g * 8 + e of every 32 lanes of a head
     bf16x8_t qf[KD];
     {
-        const bf16_t *qrow = p.q + (size_t)my_row * p.q_stride + (size_t)my_head * D;
+        const bf16_t *qrow = q + (size_t)my_row * q_stride + (size_t)my_head * D;
 #pragma unroll
         for (int kk = 0; kk < KD; kk++) {
             qf[kk] = *(const bf16x8_t *)(qrow + kk * 32 + g * 8);
@@ -192,19 +205,39 @@ mixer_tile_kernel(const TileParams p) {
         const int nb_max = lo_max / p.pool;
         for (int base = 0; base < nb_max; base += 32, turn++) {
             if ((turn & (kWavesM - 1)) != wave || (turn / kWavesM) % p.splits != (int)blockIdx.z) continue;
+            // where a block's mean lies: the page of its last token, and its place there
+            auto mean_of = [&](int b) __attribute__((always_inline)) {
+                const int end = min(b, nb_max - 1) * p.pool + p.pool - 1;
+                return ((size_t)tbl[page_of(end)] * kv_heads + kvh) * p.slots + (p.slots > 1 ? in_page(end) / p.pool : 0);
+            };
+            size_t kat[2], vat[8];
+#pragma unroll
+            for (int j = 0; j < 2; j++) kat[j] = mean_of(base + (qi >> 2) * 8 + j * 4 + (qi & 3)) * D;
+            // A = V^T: row = a value lane, k = the blocks base + g * 8 + e, each in a page and slot of its own
+#pragma unroll
+            for (int e = 0; e < 8; e++) vat[e] = mean_of(base + g * 8 + e) * DV;
+            f32x4_t kx[2][KD][2];
+            float vx[VT][8];
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int kk = 0; kk < KD; kk++)
+#pragma unroll
+                    for (int i = 0; i < 2; i++) kx[j][kk][i] = *(const f32x4_t *)(p.pool_k + kat[j] + kk * 32 + g * 8 + 4 * i);
+#pragma unroll
+            for (int t = 0; t < VT; t++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) vx[t][e] = p.pool_v[vat[e] + t * 16 + qi];
+            __builtin_amdgcn_sched_barrier(0);      // all of them before the first product
             f32x4_t s[2];
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 s[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-                int b = base + (qi >> 2) * 8 + j * 4 + (qi & 3);
-                b = b < nb_max ? b : nb_max - 1;
-                const int end = b * p.pool + p.pool - 1;
-                const float *kr = p.pool_k + (((size_t)tbl[end / ps] * p.kv_heads + kvh) * p.slots + (end % ps) / p.pool) * D;
 #pragma unroll
                 for (int kk = 0; kk < KD; kk++) {
                     float x[8];
-                    *(f32x4_t *)x = *(const f32x4_t *)(kr + kk * 32 + g * 8);
-                    *(f32x4_t *)(x + 4) = *(const f32x4_t *)(kr + kk * 32 + g * 8 + 4);
+                    *(f32x4_t *)x = kx[j][kk][0];
+                    *(f32x4_t *)(x + 4) = kx[j][kk][1];
                     bf16x8_t hi, lo;
                     split_bf16(x, hi, lo);
                     s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, qf[kk], s[j], 0, 0, 0);
@@ -214,22 +247,10 @@ mixer_tile_kernel(const TileParams p) {
             weigh_and_add(
                 s, [&](int slot) { return valid && base + slot < nb_q; }, [&](int) { return 0.f; },
                 [&](const bf16x8_t &p_hi, const bf16x8_t &p_lo) {
-                    // A = V^T: row = a value lane, k = the blocks base + g * 8 + e, each in a page and slot of its own
-                    size_t at[8];
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        int b = base + g * 8 + e;
-                        b = b < nb_max ? b : nb_max - 1;
-                        const int end = b * p.pool + p.pool - 1;
-                        at[e] = (((size_t)tbl[end / ps] * p.kv_heads + kvh) * p.slots + (end % ps) / p.pool) * DV;
-                    }
 #pragma unroll
                     for (int t = 0; t < VT; t++) {
-                        float x[8];
-#pragma unroll
-                        for (int e = 0; e < 8; e++) x[e] = p.pool_v[at[e] + t * 16 + qi];
                         bf16x8_t hi, lo;
-                        split_bf16(x, hi, lo);
+                        split_bf16(vx[t], hi, lo);
                         o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, p_hi, o[t], 0, 0, 0);
                         o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, p_lo, o[t], 0, 0, 0);
                         o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, p_hi, o[t], 0, 0, 0);
@@ -252,13 +273,13 @@ mixer_tile_kernel(const TileParams p) {
                 for (int j = 0; j < 2; j++) {
                     int key = base + (qi >> 2) * 8 + j * 4 + (qi & 3);
                     key = key <= pos_max ? key : pos_max;
-                    const bf16_t *kr = p.k_pages + key_offset(tbl[key / ps], p.kv_heads, kvh, ps, D, key % ps, g * 8);
+                    const bf16_t *kr = p.k_pages + key_offset(tbl[page_of(key)], kv_heads, kvh, ps, D, in_page(key), g * 8);
 #pragma unroll
                     for (int kk = 0; kk < KD; kk++) ka[half][j][kk] = *(const bf16x8_t *)(kr + (size_t)kk * 4 * ps * 8);      // 32 lanes on: four chunks of 8
                 }
                 int key = base + g * 8;                  // eight tokens side by side in one page (pages hold multiples of 16)
                 key = key <= pos_max ? key : pos_max & ~7;
-                const bf16_t *vr = p.v_pages + (((size_t)tbl[key / ps] * p.kv_heads + kvh) * DV + qi) * ps + key % ps;
+                const bf16_t *vr = p.v_pages + (((size_t)tbl[page_of(key)] * kv_heads + kvh) * DV + qi) * ps + in_page(key);
 #pragma unroll
                 for (int t = 0; t < VT; t++) va[half][t] = *(const bf16x8_t *)(vr + (size_t)t * 16 * ps);
             }
@@ -296,7 +317,7 @@ mixer_tile_kernel(const TileParams p) {
 #pragma unroll
         for (int i = 0; i < 4; i++) sm_o[wave][qi][t * 16 + g * 4 + i] = o[t][i];
     __syncthreads();
-    float *part = p.splits > 1 ? p.parts + ((size_t)(blockIdx.y * gridDim.x + blockIdx.x) * p.splits + blockIdx.z) * (16 * DV + 32) : nullptr;
+    float *part = p.splits > 1 ? p.parts + ((size_t)(blockIdx.y * p.rows + blockIdx.x) * p.splits + blockIdx.z) * (16 * DV + 32) : nullptr;
     for (int idx = threadIdx.x; idx < count * DV; idx += kThreads) {
         const int q = idx / DV, d = idx - q * DV;
         float acc = 0.f, l = 0.f;
@@ -324,8 +345,8 @@ mixer_tile_kernel(const TileParams p) {
                 continue;
             }
         }
-        const int row = p.by_heads ? row0 : row0 + q, head = p.by_heads ? head0 + q : head0;
-        p.out[((size_t)row * p.heads + head) * DV + d] = (bf16_t)acc;
+        const int row = by_heads ? row0 : row0 + q, head = by_heads ? head0 + q : head0;
+        p.out[((size_t)row * heads + head) * DV + d] = (bf16_t)acc;
     }
     if (part == nullptr) return;
     // ---- the shares meet (tiles by heads): the workgroup that counts last puts them together in the order of the shares, all of
@@ -333,7 +354,7 @@ mixer_tile_kernel(const TileParams p) {
     // (prompts and answers of 2 requests, 72 such launches: 14.46 -> 14.10 ms).
     __shared__ int s_seen;
     __shared__ float s_factor[kMostSplits][16], s_sum[kMostSplits][16];
-    const int tile = blockIdx.y * gridDim.x + blockIdx.x, splits = p.splits;
+    const int tile = blockIdx.y * p.rows + blockIdx.x, splits = p.splits;
     parts_published();
     __syncthreads();
     if (threadIdx.x == 0) s_seen = __hip_atomic_fetch_add(p.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -395,18 +416,24 @@ mixer_tile_kernel(const TileParams p) {
             if (idx >= count * DV) break;
             const int q = idx / DV, d = idx - q * DV;
             if (VARIANT == 0) acc[i] = l[i] > 0.f ? acc[i] / l[i] : 0.f;
-            p.out[((size_t)row0 * p.heads + head0 + q) * DV + d] = (bf16_t)acc[i];
+            p.out[((size_t)row0 * heads + head0 + q) * DV + d] = (bf16_t)acc[i];
         }
     }
 }
 
 template <int VARIANT, int KD>
 int launch_vt(const TileParams &p, int vt, dim3 grid, hipStream_t stream) {
+    int shift = -1;
+    if ((p.page_size & (p.page_size - 1)) == 0) shift = __builtin_ctz((unsigned)p.page_size);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, p.row_seg, p.row_pos, p.tables, p.q, p.table_stride, p.heads, p.kv_heads,
+                           p.q_stride, p.by_heads, shift, p);
+    };
     switch (vt) {
-    case 2: hipLaunchKernelGGL((mixer_tile_kernel<KD, 2, VARIANT>), grid, dim3(kThreads), 0, stream, p); return 0;
-    case 4: hipLaunchKernelGGL((mixer_tile_kernel<KD, 4, VARIANT>), grid, dim3(kThreads), 0, stream, p); return 0;
-    case 6: hipLaunchKernelGGL((mixer_tile_kernel<KD, 6, VARIANT>), grid, dim3(kThreads), 0, stream, p); return 0;
-    case 8: hipLaunchKernelGGL((mixer_tile_kernel<KD, 8, VARIANT>), grid, dim3(kThreads), 0, stream, p); return 0;
+    case 2: shift >= 0 ? go(mixer_tile_kernel<KD, 2, VARIANT, true>) : go(mixer_tile_kernel<KD, 2, VARIANT, false>); return 0;
+    case 4: shift >= 0 ? go(mixer_tile_kernel<KD, 4, VARIANT, true>) : go(mixer_tile_kernel<KD, 4, VARIANT, false>); return 0;
+    case 6: shift >= 0 ? go(mixer_tile_kernel<KD, 6, VARIANT, true>) : go(mixer_tile_kernel<KD, 6, VARIANT, false>); return 0;
+    case 8: shift >= 0 ? go(mixer_tile_kernel<KD, 8, VARIANT, true>) : go(mixer_tile_kernel<KD, 8, VARIANT, false>); return 0;
     }
     return 1;
 }
