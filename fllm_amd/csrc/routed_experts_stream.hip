@@ -6,7 +6,7 @@
 // behind it cost prompts and answers of 12 requests 12.40 ms where this takes 12.29), no scaled copies of the rows are
 // made (an operand is scaled where it is loaded, rounded to bfloat16 as a stored copy would be), and the down product is not cut
 // into planes that a further kernel adds.  A workgroup takes 16 output columns (of gate and of up) or 32 of one expert, its eight waves
-// cut K between them with 6 to 12 KiB asked for at a time each, and they meet in LDS once.  A load of the tile-major copy is
+// cut K between them with 6 KiB asked for at a time each, and they meet in LDS once.  A load of the tile-major copy is
 // 1 KiB in a row, whole cache lines that carry the non-temporal hint; the same kernel reading the rows as the checkpoint has them
 // (64 bytes of each of 16) runs at 4.4 instead of 5.9 TB/s, and through LDS in whole rows, a tile at a time, at 4.0.
 // A load of an expert's weights serves up to 32 pairs from registers.
@@ -42,7 +42,11 @@ expert_stream_kernel(const bf16_t *__restrict__ x, const int32_t *__restrict__ i
     static_assert(!SHARED || MODE != 0, "a shared expert comes with experts without a gate");
     constexpr int RT = MODE == 1 ? 1 : 2;                  // 16-row weight tiles a workgroup
     constexpr int COLS = MODE == 2 ? 32 : 16;              // output columns a workgroup
-    constexpr int U = MODE == 0 && G > 1 ? 3 : 6;          // products a wave asks for at a time (two tiles, two groups: 128 registers)
+    // Products a wave asks for at a time.  Two tiles of one group: three, so that 64 to 75 registers hold three or four workgroups a compute unit where
+    // six left two: how many workgroups are there to ask while others' sums meet counts for more than how much each asks for (4,480
+    // lanes at 1,536: 2 rows with a shared expert 15.2 -> 13.1 us, 8 rows 32.3 -> 31.1, 16 rows 34.7 -> 32.2; two products 30.4 and 32.6).  One tile: six (four: 18.5
+    // and 18.4, 20.2 and 20.4, with a shared expert 13.2 and 13.7; nine 21.4, 22.8, 13.2).  Two groups: 128 registers.
+    constexpr int U = G > 1 ? (MODE == 0 ? 3 : 6) : MODE == 1 ? 6 : 3;
     __shared__ __attribute__((aligned(16))) f32x4_t red[kWaves][RT][kWave];
     __shared__ short s_pairs[kWaves][kMostPairs];          // a wave's own list: no barrier before the first loads
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
