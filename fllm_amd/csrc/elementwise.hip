@@ -25,10 +25,14 @@ embed_kernel(const int32_t *__restrict__ ids, const T *__restrict__ table, float
 // gives the same bits whatever else is in the batch.  With `branch` the kernel first adds it to
 // the row (x += branch, in float32, written back): residual add and the next norm in one pass.
 // Rows of up to 256 * 4 * VEC values stay in registers between the two uses.
-template <typename T, typename B, int VEC>
+// All that a row needs is asked for before the first of it is used, behind no condition (a thread without values of its own reads the row's last
+// ones again): behind conditions a piece was awaited, added and stored before the next was asked for, and the weights came behind the
+// sum.  WIDE: everything lies on 8 bytes (rows of the branch and of the output in bfloat16 too): four values are one load or store.
+// 2,048 rows of 4,096 values with a branch in bfloat16 18.8 -> 17.0 us (101 MB), 405 rows 7.4 -> 5.8; of 2,048 values 9.5 -> 9.1.
+template <typename T, typename B, int VEC, bool WIDE>
 __global__ void __launch_bounds__(kBlock)
-rmsnorm_kernel(float *__restrict__ x, const B *__restrict__ branch, const int32_t *__restrict__ rows,
-               const float *__restrict__ weight, T *__restrict__ out, int width, float eps) {
+rmsnorm_kernel(float *__restrict__ x, const B *__restrict__ branch, const float *__restrict__ weight, const int32_t *__restrict__ rows,
+               int width, float eps, T *__restrict__ out) {
     __shared__ float scratch[kWaves];
     const int i = blockIdx.x;
     const int r = rows ? rows[i] : i;
@@ -36,31 +40,56 @@ rmsnorm_kernel(float *__restrict__ x, const B *__restrict__ branch, const int32_
     const B *br = branch ? branch + (size_t)r * width : nullptr;
     T *dst = out + (size_t)i * width;
     if constexpr (VEC > 0) {   // width is a multiple of 4 and at most 1024 * VEC
-        f32x4_t v[VEC > 0 ? VEC : 1];
+        typedef __attribute__((ext_vector_type(4))) B b4_t;
+        typedef __attribute__((ext_vector_type(4))) T t4_t;
+        f32x4_t v[VEC > 0 ? VEC : 1], w[VEC > 0 ? VEC : 1];
+        b4_t add[VEC > 0 ? VEC : 1];
         float ss = 0.f;
+        auto mine = [&](int j) { return ((int)threadIdx.x + j * kBlock) * 4 < width; };
 #pragma unroll
         for (int j = 0; j < VEC; j++) {
-            const int c = (threadIdx.x + j * kBlock) * 4;
-            if (c < width) {
-                v[j] = *(const f32x4_t *)(src + c);
-                if (br) {
+            const int c = min(((int)threadIdx.x + j * kBlock) * 4, width - 4);
+            v[j] = *(const f32x4_t *)(src + c);
+            w[j] = *(const f32x4_t *)(weight + c);
+        }
+        if (br) {
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[j][e] += to_f32<B>(br[c + e]);
-                    *(f32x4_t *)(src + c) = v[j];
+            for (int j = 0; j < VEC; j++) {
+                const int c = min(((int)threadIdx.x + j * kBlock) * 4, width - 4);
+                if constexpr (WIDE) {
+                    add[j] = *(const b4_t *)(br + c);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) add[j][e] = br[c + e];
                 }
+            }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int e = 0; e < 4; e++) ss += v[j][e] * v[j][e];
+            for (int j = 0; j < VEC; j++) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[j][e] += to_f32<B>(add[j][e]);
+                if (mine(j)) *(f32x4_t *)(src + ((int)threadIdx.x + j * kBlock) * 4) = v[j];
             }
         }
-        ss = block_sum<kWaves>(ss, scratch);
+#pragma unroll
+        for (int j = 0; j < VEC; j++)
+            if (mine(j))
+#pragma unroll
+                for (int e = 0; e < 4; e++) ss += v[j][e] * v[j][e];
+        ss = block_sum_once<kWaves>(ss, scratch);
         const float inv = 1.0f / sqrtf(ss / (float)width + eps);
 #pragma unroll
         for (int j = 0; j < VEC; j++) {
-            const int c = (threadIdx.x + j * kBlock) * 4;
-            if (c < width) {
-                const f32x4_t w = *(const f32x4_t *)(weight + c);
+            const int c = ((int)threadIdx.x + j * kBlock) * 4;
+            if (!mine(j)) break;
+            t4_t o;
 #pragma unroll
-                for (int e = 0; e < 4; e++) dst[c + e] = from_f32<T>(v[j][e] * (inv * w[e]));
+            for (int e = 0; e < 4; e++) o[e] = from_f32<T>(v[j][e] * (inv * w[j][e]));
+            if constexpr (WIDE) {
+                *(t4_t *)(dst + c) = o;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) dst[c + e] = o[e];
             }
         }
     } else {
@@ -217,13 +246,21 @@ template <typename T, typename B>
 void launch_rmsnorm(float *x, const B *branch, const int32_t *rows, const float *weight, T *out, int count, int width,
                     float eps, hipStream_t stream) {
     const bool vec = width % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)weight & 15) == 0;
-#define FLLM_NORM(V) hipLaunchKernelGGL((rmsnorm_kernel<T, B, V>), dim3(count), dim3(kBlock), 0, stream, x, branch, rows, weight, out, width, eps)
+    const bool wide = (((uintptr_t)branch | (uintptr_t)out) & 15) == 0;
+#define FLLM_NORM_FORM(V, WIDE) \
+    hipLaunchKernelGGL((rmsnorm_kernel<T, B, V, WIDE>), dim3(count), dim3(kBlock), 0, stream, x, branch, weight, rows, width, eps, out)
+#define FLLM_NORM(V)                               \
+    do {                                           \
+        if (wide) FLLM_NORM_FORM(V, true);         \
+        else FLLM_NORM_FORM(V, false);             \
+    } while (0)
     if (vec && width <= 1024) FLLM_NORM(1);
     else if (vec && width <= 2048) FLLM_NORM(2);
     else if (vec && width <= 4096) FLLM_NORM(4);
     else if (vec && width <= 8192) FLLM_NORM(8);
-    else FLLM_NORM(0);
+    else FLLM_NORM_FORM(0, false);
 #undef FLLM_NORM
+#undef FLLM_NORM_FORM
 }
 
 template <typename B>
@@ -307,7 +344,7 @@ extern "C" int fllm_add_residual(float *residual, const void *branch, int rows, 
 // share 8 rows (a read and a write of the same buffer cannot overlap inside a thread, so many short threads beat few
 // long ones); where the rows are 8 consecutive tokens of one request that start at a multiple of 8 (a prompt portion), their values go
 // into the transposed page as one 16-byte store per head lane instead of eight 2-byte ones.
-template <int RB>
+template <int RB, int U>
 __global__ void __launch_bounds__(kBlock)
 rope_kv_store_vec_kernel(bf16_t *__restrict__ qkv, const int32_t *__restrict__ row_pos, const int32_t *__restrict__ row_seg,
                          const int32_t *__restrict__ tables, int table_stride, const float *__restrict__ cos_table,
@@ -322,18 +359,19 @@ rope_kv_store_vec_kernel(bf16_t *__restrict__ qkv, const int32_t *__restrict__ r
     const int per_head_v = v_dim / 8;
     // position (-1: padding row), page and slot of the workgroup's rows
     __shared__ int s_pos[RB], s_page[RB], s_off[RB], s_run;
-    if ((int)threadIdx.x < nrows) {
-        const int r = r0 + threadIdx.x;
+    if ((int)threadIdx.x < kWave) {      // one wave: a lane a row, so that the rows are asked for together
+        const int i = min((int)threadIdx.x, nrows - 1), r = r0 + i;
         const int seg = row_seg[r], pos = row_pos[r];
-        s_pos[threadIdx.x] = seg < 0 ? -1 : pos;
-        s_page[threadIdx.x] = (store_kv && seg >= 0) ? tables[(size_t)seg * table_stride + pos / page_size] : 0;
-        s_off[threadIdx.x] = pos % page_size;
-    }
-    if (threadIdx.x == 0) {
-        const int seg0 = row_seg[r0], pos0 = row_pos[r0];
-        bool run = RB == 8 && store_kv && nrows == RB && seg0 >= 0 && (pos0 & (RB - 1)) == 0 && page_size % RB == 0;
-        for (int i = 1; i < RB && run; i++) run = row_seg[r0 + i] == seg0 && row_pos[r0 + i] == pos0 + i;
-        s_run = run;
+        const int seg0 = __builtin_amdgcn_readfirstlane(seg), pos0 = __builtin_amdgcn_readfirstlane(pos);
+        const bool follows = seg == seg0 && pos == pos0 + i;
+        const bool run = RB == 8 && store_kv && nrows == RB && seg0 >= 0 && (pos0 & (RB - 1)) == 0 && page_size % RB == 0 && __all(follows);
+        const int page = (store_kv && seg >= 0) ? tables[(size_t)seg * table_stride + pos / page_size] : 0;
+        if ((int)threadIdx.x < nrows) {
+            s_pos[i] = seg < 0 ? -1 : pos;
+            s_page[i] = page;
+            s_off[i] = pos % page_size;
+        }
+        if (threadIdx.x == 0) s_run = run;
     }
     __syncthreads();
     const bool run = s_run != 0;
@@ -341,25 +379,40 @@ rope_kv_store_vec_kernel(bf16_t *__restrict__ qkv, const int32_t *__restrict__ r
     // queries and keys: every (row, 16-byte chunk) is a piece of work of its own, so that a thread has several in flight
     const int per_row = rot_heads * per_head;
     const int first = blockIdx.y * kBlock + threadIdx.x, stride = gridDim.y * kBlock;   // the workgroups of a row group share its pieces
-    for (int it = first; it < nrows * per_row; it += stride) {
-        const int i = RB == 1 ? 0 : it / per_row, t = it - i * per_row;
-        const int pos = s_pos[i];
-        if (pos < 0) continue;   // padding row
-        const int h = t / per_head, c = (t - h * per_head) * 8;
-        bf16_t *row = qkv + (size_t)(r0 + i) * row_elems;
-        bf16x8_t v = *(const bf16x8_t *)(row + (size_t)h * head_dim + c);
-        if (c < rope_dims) {   // rope_dims is a multiple of 8: the chunk is rotated as a whole
-            const f32x4_t c4 = *(const f32x4_t *)(cos_table + (size_t)pos * half + c / 2);
-            const f32x4_t s4 = *(const f32x4_t *)(sin_table + (size_t)pos * half + c / 2);
+    // U pieces of a thread on their way together
+    for (int it0 = first; it0 < nrows * per_row; it0 += U * stride) {
+        bf16x8_t v[U];
+        f32x4_t c4[U], s4[U];
+        int row_of[U], head_of[U], lane_of[U];
 #pragma unroll
-            for (int p = 0; p < 4; p++) {
-                const float a = (float)v[2 * p], b = (float)v[2 * p + 1];
-                v[2 * p] = (bf16_t)(a * c4[p] - b * s4[p]);
-                v[2 * p + 1] = (bf16_t)(b * c4[p] + a * s4[p]);
+        for (int u = 0; u < U; u++) {
+            const int it = min(it0 + u * stride, nrows * per_row - 1);
+            const int i = RB == 1 ? 0 : it / per_row, t = it - i * per_row;
+            const int h = t / per_head, c = (t - h * per_head) * 8;
+            row_of[u] = i, head_of[u] = h, lane_of[u] = c;
+            v[u] = *(const bf16x8_t *)(qkv + (size_t)(r0 + i) * row_elems + (size_t)h * head_dim + c);
+            if (rope_dims > 0) {
+                const size_t angle = (size_t)max(s_pos[i], 0) * half + (c < rope_dims ? c / 2 : 0);
+                c4[u] = *(const f32x4_t *)(cos_table + angle);
+                s4[u] = *(const f32x4_t *)(sin_table + angle);
             }
         }
-        if (h < heads) *(bf16x8_t *)(row + (size_t)h * head_dim + c) = v;
-        else *(bf16x8_t *)(k_pages + key_offset(s_page[i], kv_heads, h - heads, page_size, head_dim, s_off[i], c)) = v;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = row_of[u], h = head_of[u], c = lane_of[u];
+            if (it0 + u * stride >= nrows * per_row || s_pos[i] < 0) continue;   // no such piece, or a padding row
+            if (c < rope_dims) {   // rope_dims is a multiple of 8: the chunk is rotated as a whole
+#pragma unroll
+                for (int p = 0; p < 4; p++) {
+                    const float a = (float)v[u][2 * p], b = (float)v[u][2 * p + 1];
+                    v[u][2 * p] = (bf16_t)fmaf(a, c4[u][p], -(b * s4[u][p]));      // which product is rounded is the same in every instance
+                    v[u][2 * p + 1] = (bf16_t)fmaf(a, s4[u][p], b * c4[u][p]);
+                }
+            }
+            if (h < heads) *(bf16x8_t *)(qkv + (size_t)(r0 + i) * row_elems + (size_t)h * head_dim + c) = v[u];
+            else *(bf16x8_t *)(k_pages + key_offset(s_page[i], kv_heads, h - heads, page_size, head_dim, s_off[i], c)) = v[u];
+        }
     }
     if (!store_kv) return;
     if (!run) {
@@ -410,13 +463,19 @@ extern "C" int fllm_rope_kv_store(void *qkv, const int32_t *row_pos, const int32
              ((uintptr_t)cos_table & 15) == 0 && ((uintptr_t)sin_table & 15) == 0 && (!store_kv || ((((uintptr_t)k_pages | (uintptr_t)v_pages) & 15) == 0)))
     {
         // prompt portions: 8 rows a workgroup, so that runs of 8 tokens store their values 16 bytes at a time; few rows
-        // (decode steps): a workgroup a row
-        if (rows >= 256)
-            hipLaunchKernelGGL(rope_kv_store_vec_kernel<8>, dim3((rows + 7) / 8, 4), dim3(kBlock), 0, stream, (bf16_t *)qkv, row_pos,
+        // (decode steps): a workgroup a row.  Threads with more than three pieces (8 rows of 40 heads of 128 lanes are five a thread) ask for four together:
+        // 2,048 rows of those 17.4 -> 15.1 us; where there are fewer (32 + 8 heads of 64, 12 + 2 of 128) the pieces that are not there
+        // cost as much as the trips (13.1 -> 13.5, 7.7 -> 8.0).
+        const bool many = (long)(store_kv ? heads + kv_heads : heads) * (head_dim / 8) * 8 > 3 * 4 * kBlock;
+        auto portion = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((rows + 7) / 8, 4), dim3(kBlock), 0, stream, (bf16_t *)qkv, row_pos,
                                row_seg, tables, table_stride, cos_table, sin_table, (bf16_t *)k_pages, (bf16_t *)v_pages, rows,
                                heads, kv_heads, head_dim, v_dim, rope_dims, page_size, store_kv);
+        };
+        if (rows >= 256 && many) portion(rope_kv_store_vec_kernel<8, 4>);
+        else if (rows >= 256) portion(rope_kv_store_vec_kernel<8, 1>);
         else
-            hipLaunchKernelGGL(rope_kv_store_vec_kernel<1>, dim3(rows), dim3(kBlock), 0, stream, (bf16_t *)qkv, row_pos, row_seg,
+            hipLaunchKernelGGL((rope_kv_store_vec_kernel<1, 1>), dim3(rows), dim3(kBlock), 0, stream, (bf16_t *)qkv, row_pos, row_seg,
                                tables, table_stride, cos_table, sin_table, (bf16_t *)k_pages, (bf16_t *)v_pages, rows, heads,
                                kv_heads, head_dim, v_dim, rope_dims, page_size, store_kv);
     }
