@@ -14,8 +14,10 @@ constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / kWave;
 constexpr int kMaxKeep = 15;
 constexpr int kMaxPer = 8;      // heads of up to 512 lanes
+constexpr int kStepTaps = 4;    // conv_qkv_step_kernel: at most
 
-// grid (rows, heads in fours): a wave takes one head of q, k or v of one row; conv_tail_kernel moves the state on behind this kernel.
+// grid (rows, heads in fours): a wave takes one head of q, k or v of one row.  `update` (steps of one row a segment): the wave,
+// which alone reads its channels of the state, moves them on; otherwise conv_tail_kernel does behind this kernel.
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
 conv_qkv_store_kernel(const T *__restrict__ joint, int ld, const float *__restrict__ conv, int taps, const float *__restrict__ bias,
@@ -24,7 +26,7 @@ conv_qkv_store_kernel(const T *__restrict__ joint, int ld, const float *__restri
                       const int32_t *__restrict__ seg_start, const int32_t *__restrict__ slots, const int32_t *__restrict__ tables,
                       int table_stride, const float *__restrict__ cos_table, const float *__restrict__ sin_table, T *__restrict__ k_pages,
                       T *__restrict__ v_pages, int heads, int kv_heads, int k_dim, int v_dim, int rope_dims, int pairing, int page_size,
-                      int key_chunk, int store_kv) {
+                      int key_chunk, int store_kv, int update) {
     extern __shared__ float smem[];
     const int r = blockIdx.x;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -52,11 +54,25 @@ conv_qkv_store_kernel(const T *__restrict__ joint, int ld, const float *__restri
         const float b = bias != nullptr ? bias[ch] : 0.f;
         const T now = joint[(size_t)r * ld + ch];
         float acc = 0.f;
-        for (int d = keep; d >= 1; d--) {
-            if (pos - d < 0) continue;
-            const int at = t - d;
-            const float u = at >= 0 ? to_f32<T>(joint[(size_t)(r - d) * ld + ch]) : to_f32<T>(mine[(size_t)(keep + at) * channels + ch]);
-            acc = fmaf(w[keep - d], u + b, acc);
+        if (update) {
+            T held[kMaxKeep];
+#pragma unroll
+            for (int i = 0; i < kMaxKeep; i++)
+                if (i < keep) held[i] = mine[(size_t)i * channels + ch];
+#pragma unroll
+            for (int i = 0; i < kMaxKeep; i++) {      // oldest first; entry i moves to i - 1
+                if (i >= keep) break;
+                if (pos - (keep - i) >= 0) acc = fmaf(w[i], to_f32<T>(held[i]) + b, acc);
+                if (i > 0) mine[(size_t)(i - 1) * channels + ch] = held[i];
+            }
+            if (keep > 0) mine[(size_t)(keep - 1) * channels + ch] = now;
+        } else {
+            for (int d = keep; d >= 1; d--) {
+                if (pos - d < 0) continue;
+                const int at = t - d;
+                const float u = at >= 0 ? to_f32<T>(joint[(size_t)(r - d) * ld + ch]) : to_f32<T>(mine[(size_t)(keep + at) * channels + ch]);
+                acc = fmaf(w[keep - d], u + b, acc);
+            }
         }
         acc = fmaf(w[keep], to_f32<T>(now) + b, acc);
         y[j] = acc;
@@ -117,8 +133,10 @@ conv_qkv_store_kernel(const T *__restrict__ joint, int ld, const float *__restri
 // arguments, some of them two or three numbers, are in registers when a wave starts; the other arguments ride along), then the state's entries, the page, weights
 // and angles.  No load sits behind a condition: a lane beyond the head reads its last channel again.  A trip a question, as
 // the form for portions has it, took 8.5 us at 16 rows of 12 + 2 heads of 128, this 4.3 (7.6 and 2.8 at best).
-// N pieces of 64 lanes a head (at most); TAPS 4: four taps are one 16-byte load; 0: any number.
-template <typename T, int N, int TAPS>
+// N pieces of 64 lanes a head (at most), up to four taps; FOUR: four of them, one 16-byte load.  Of fewer the last ones are read again: behind a
+// question each (is there an i-th) every 16-bit entry was awaited before the next was asked for (three taps in bfloat16, 16 rows of 6 + 2 heads of
+// 192 12.9 us, of 4 + 2 of 64 6.0; without 5.6 and 3.3, by the form for portions 7.0 and 4.3).
+template <typename T, int N, bool FOUR>
 __global__ void __launch_bounds__(kBlock)
 conv_qkv_step_kernel(const T *__restrict__ joint, const int32_t *__restrict__ row_seg, const int32_t *__restrict__ row_pos,
                      const int32_t *__restrict__ slots, const float *__restrict__ conv, int ld, int all_heads /* heads | kv_heads << 16 */,
@@ -127,14 +145,14 @@ conv_qkv_step_kernel(const T *__restrict__ joint, const int32_t *__restrict__ ro
                      T *__restrict__ q_out, const int32_t *__restrict__ tables, int table_stride, const float *__restrict__ cos_table,
                      const float *__restrict__ sin_table, T *__restrict__ k_pages, T *__restrict__ v_pages, int page_size, int key_chunk) {
     typedef const __attribute__((address_space(4))) int32_t *constant_t;      // the same for every lane: a scalar load
-    constexpr int KEEP = TAPS > 0 ? TAPS - 1 : kMaxKeep;                      // at most
+    constexpr int KEEP = kStepTaps - 1;
     extern __shared__ float smem[];
     const int r = blockIdx.x;
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int unit = blockIdx.y * kWaves + wave;
     const int seg = ((constant_t)(uintptr_t)row_seg)[r], pos = ((constant_t)(uintptr_t)row_pos)[r], slot_here = ((constant_t)(uintptr_t)slots)[r];
     const int heads = all_heads & 0xffff, kv_heads = (int)((unsigned)all_heads >> 16), k_dim = dims & 0xffff, v_dim = (int)((unsigned)dims >> 16);
-    const int taps = TAPS > 0 ? TAPS : form & 0xff, keep = taps - 1, rope_dims = (form >> 8) & 0xffff;
+    const int taps = FOUR ? kStepTaps : form & 0xff, keep = taps - 1, rope_dims = (form >> 8) & 0xffff;
     const bool pairing = (form >> 24) & 1, store_kv = (form >> 25) & 1;
     if (unit >= heads + (store_kv ? 2 * kv_heads : 0)) return;      // no such head (no barrier below)
     const int kind = unit < heads ? 0 : (unit < heads + kv_heads ? 1 : 2);
@@ -143,36 +161,34 @@ conv_qkv_step_kernel(const T *__restrict__ joint, const int32_t *__restrict__ ro
     const int nq = heads * k_dim, nk = kv_heads * k_dim;
     const int channels = nq + (store_kv ? nk + kv_heads * v_dim : 0);
     const int base = kind == 0 ? h * k_dim : (kind == 1 ? nq + h * k_dim : nq + nk + h * v_dim);
-    constexpr bool LATE = N > 2 && TAPS == 0;      // any number of taps of a wide head: a piece at a time, all of them are too many registers
-    T now[N], held[LATE ? 1 : N][KEEP > 0 ? KEEP : 1];
-    float w[LATE ? 1 : N][KEEP + 1];
+    T now[N], held[N][KEEP];
+    float w[N][kStepTaps];
     T *mine = nullptr;
+    const T *kept = joint + (size_t)r * ld;       // one tap: read, never used
     auto lane_of = [&](int j) __attribute__((always_inline)) { return min(lane + j * kWave, dim - 1); };
     auto ask_taps = [&](int j, int ch) __attribute__((always_inline)) {
-        if constexpr (TAPS == 4) {
+        if constexpr (FOUR) {
             *(f32x4_t *)w[j] = *(const f32x4_t *)(conv + (size_t)ch * 4);
         } else {
 #pragma unroll
-            for (int i = 0; i <= KEEP; i++)
-                if (i < taps) w[j][i] = conv[(size_t)ch * taps + i];
+            for (int i = 0; i < kStepTaps; i++) w[j][i] = conv[(size_t)ch * taps + min(i, keep)];
         }
     };
     auto ask_state = [&](int j, int ch) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < KEEP; i++)
-            if (i < keep) held[j][i] = mine[(size_t)i * channels + ch];
+        for (int i = 0; i < KEEP; i++) held[j][i] = kept[(size_t)(FOUR ? i : max(min(i, keep - 1), 0)) * channels + ch];
     };
 #pragma unroll
     for (int j = 0; j < N; j++) {
         const int ch = base + lane_of(j);
         now[j] = joint[(size_t)r * ld + ch];
-        if constexpr (!LATE) ask_taps(j, ch);
+        ask_taps(j, ch);
     }
     fetch_arguments(state, bias, q_weight, k_weight, eps, q_out, tables, table_stride, cos_table, sin_table, k_pages, v_pages, page_size, key_chunk, pos, slot_here);
     const bool padding = seg < 0;      // goes the whole way and stores nothing (a return here would be a wait ahead of the first loads)
     // a segment of one row has its row's number
     const int slot = padding ? 0 : seg == r ? slot_here : ((constant_t)(uintptr_t)slots)[seg];
-    if (keep > 0) mine = state + (size_t)slot * keep * channels;
+    if (keep > 0) kept = mine = state + (size_t)slot * keep * channels;
     const int page_at = padding ? 0 : pos / page_size, off = padding ? 0 : pos - page_at * page_size;
     const int page = kind > 0 ? ((constant_t)(uintptr_t)tables)[(size_t)(padding ? 0 : seg) * table_stride + page_at] : 0;
     const float *weight = kind == 0 ? q_weight : (kind == 1 ? k_weight : nullptr);
@@ -183,7 +199,7 @@ conv_qkv_step_kernel(const T *__restrict__ joint, const int32_t *__restrict__ ro
 #pragma unroll
     for (int j = 0; j < N; j++) {
         const int c = lane_of(j), ch = base + c;
-        if constexpr (!LATE) ask_state(j, ch);
+        ask_state(j, ch);
         b[j] = 0.f, weigh[j] = 1.f, cv[j] = sv[j] = 0.f;
         if (bias != nullptr) b[j] = bias[ch];
         if (weight != nullptr) weigh[j] = weight[c];
@@ -198,19 +214,17 @@ conv_qkv_step_kernel(const T *__restrict__ joint, const int32_t *__restrict__ ro
     for (int j = 0; j < N; j++) {
         const int c = lane + j * kWave, ch = base + c;
         const bool here = c < dim;
-        if constexpr (LATE) ask_taps(0, base + lane_of(j)), ask_state(0, base + lane_of(j));
-        constexpr int ONE = LATE ? 0 : 1;
         float acc = 0.f;
 #pragma unroll
         for (int i = 0; i < KEEP; i++) {      // oldest first; entry i moves to i - 1
             if (i >= keep) break;
-            if (pos - (keep - i) >= 0) acc = fmaf(w[ONE * j][i], to_f32<T>(held[ONE * j][i]) + b[j], acc);
-            if (i > 0 && here && !padding) mine[(size_t)(i - 1) * channels + ch] = held[ONE * j][i];
+            if (pos - (keep - i) >= 0) acc = fmaf(w[j][i], to_f32<T>(held[j][i]) + b[j], acc);
+            if (i > 0 && here && !padding) mine[(size_t)(i - 1) * channels + ch] = held[j][i];
         }
         if (keep > 0 && here && !padding) mine[(size_t)(keep - 1) * channels + ch] = now[j];
 #pragma unroll
         for (int i = 0; i <= KEEP; i++)
-            if (i == keep) acc = fmaf(w[ONE * j][i], to_f32<T>(now[j]) + b[j], acc);
+            if (i == keep) acc = fmaf(w[j][i], to_f32<T>(now[j]) + b[j], acc);
         y[j] = acc;
         if (here) ss = fmaf(acc, acc, ss);
     }
@@ -311,28 +325,29 @@ extern "C" int fllm_conv_qkv_store(const void *joint, int ld, const float *conv,
     const int blocks = (channels + kBlock - 1) / kBlock;
     FLLM_REQUIRE(groups <= 65535 && blocks <= 65535, "conv_qkv_store: too many heads");
     const size_t smem = rope_dims > 0 ? (size_t)kWaves * k_dim * sizeof(float) : 0;
-    // the step form takes sizes two in a word; sizes beyond that (no model has them) go the portions' way, which serves every step
-    const bool packs = heads <= 0xffff && kv_heads <= 0x7fff && table_stride > 0;
-#define FLLM_STEP(T, N, TAPS)                                                                                                               \
-    hipLaunchKernelGGL((conv_qkv_step_kernel<T, N, TAPS>), dim3(rows, groups), dim3(kBlock), smem, stream, (const T *)joint, row_seg, row_pos, \
+    // The step form takes up to four taps, and sizes two in a word.  More taps go the portions' way, a tap a load as it comes: all at once are
+    // more loads than a wave's trips cost (eight taps in bfloat16, 16 rows of 12 + 2 heads of 128 8.3 us, 12.3 in the step form; 16 taps 12.3, 19.7).
+    const bool step = single_rows && taps <= kStepTaps && heads <= 0xffff && kv_heads <= 0x7fff;
+#define FLLM_STEP(T, N, FOUR)                                                                                                               \
+    hipLaunchKernelGGL((conv_qkv_step_kernel<T, N, FOUR>), dim3(rows, groups), dim3(kBlock), smem, stream, (const T *)joint, row_seg, row_pos, \
                        slots, conv, ld, heads | kv_heads << 16, k_dim | v_dim << 16,                                                        \
                        taps | rope_dims << 8 | pairing << 24 | (store_kv ? 1 << 25 : 0), (T *)state, bias, q_weight, k_weight, eps,            \
                        (T *)q_out, tables, table_stride, cos_table, sin_table, (T *)k_pages, (T *)v_pages, page_size, key_chunk)
 #define FLLM_CONV(T)                                                                                                                        \
     do {                                                                                                                                    \
-        if (single_rows && packs) {                                                                                                         \
+        if (step) {                                                                                                                         \
             const bool four = taps == 4 && ((uintptr_t)conv & 15) == 0, narrow = k_dim <= 2 * kWave && v_dim <= 2 * kWave;                   \
-            if (four && narrow) FLLM_STEP(T, 2, 4);                                                                                         \
-            else if (four) FLLM_STEP(T, kMaxPer, 4);                                                                                        \
-            else if (narrow) FLLM_STEP(T, 2, 0);                                                                                            \
-            else FLLM_STEP(T, kMaxPer, 0);                                                                                                  \
+            if (four && narrow) FLLM_STEP(T, 2, true);                                                                                      \
+            else if (four) FLLM_STEP(T, kMaxPer, true);                                                                                     \
+            else if (narrow) FLLM_STEP(T, 2, false);                                                                                        \
+            else FLLM_STEP(T, kMaxPer, false);                                                                                              \
             break;                                                                                                                          \
         }                                                                                                                                   \
         hipLaunchKernelGGL(conv_qkv_store_kernel<T>, dim3(rows, groups), dim3(kBlock), smem, stream, (const T *)joint, ld, conv, taps, bias, \
                            (T *)state, q_weight, k_weight, eps, (T *)q_out, row_pos, row_seg, seg_start, slots, tables, table_stride,       \
                            cos_table, sin_table, (T *)k_pages, (T *)v_pages, heads, kv_heads, k_dim, v_dim, rope_dims, pairing, page_size,  \
-                           key_chunk, store_kv);                                                                                            \
-        if (taps > 1)                                                                                                                       \
+                           key_chunk, store_kv, single_rows);                                                                               \
+        if (taps > 1 && !single_rows)                                                                                                       \
             hipLaunchKernelGGL(conv_tail_kernel<T>, dim3(num_segs, blocks), dim3(kBlock), 0, stream, (const T *)joint, ld, (T *)state,       \
                                row_seg, seg_start, slots, channels, taps);                                                                  \
     } while (0)

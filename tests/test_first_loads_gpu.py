@@ -68,11 +68,12 @@ def test_picks_of_equals_and_of_rows_that_compare_with_nothing(ops, experts, top
         assert ids2[r].cpu().tolist() == picks(choice.tolist(), top)
 
 
-@pytest.mark.parametrize("taps", [4, 5])
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 5, 16])
 @pytest.mark.parametrize("H,G,d,dv,rope,pairing", [(2, 1, 128, 128, 128, 0), (3, 1, 136, 64, 64, 1), (1, 1, 512, 512, 16, 0), (2, 2, 8, 130, 0, 0)])
 @pytest.mark.parametrize("dtype", [F32, BF16])
 def test_convolved_heads_of_single_rows(ops, H, G, d, dv, rope, pairing, taps, dtype):
-    """Four taps on 16 bytes are one load, any others a load each; heads of up to 128 lanes and wider ones have instances of their own."""
+    """Four taps on 16 bytes are one load, up to four others a load each, more go the form for portions; heads of up to 128 lanes and wider
+    ones have instances of their own."""
     g = torch.Generator().manual_seed(d + taps)
     rows, page, channels = 5, 16, H * d + G * (d + dv)
     joint = torch.randn(rows, channels, generator=g).to(dtype).to(DEV)

@@ -1,0 +1,48 @@
+"""What the compiled kernels of decode steps are held to where nothing in their results shows it: loads that wait for nothing between them."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from fllm_amd.kernels import build
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def kernels(source, pattern, tmp_path):
+    """(name, text up to the next kernel, the pattern's groups) of every kernel of a source whose name the pattern matches."""
+    try:
+        hipcc = build._hipcc()
+    except RuntimeError as e:
+        pytest.skip(str(e))
+    listing = tmp_path / "listing.s"
+    run = subprocess.run([hipcc, *build.HIPCC_FLAGS, "--cuda-device-only", "-S", os.path.join(ROOT, "fllm_amd", "csrc", source), "-o", str(listing)],
+                         capture_output=True, text=True, timeout=600)
+    assert run.returncode == 0, run.stderr
+    parts = re.split(r"^(_Z\w+):.*$", listing.read_text(), flags=re.M)
+    found = [(name, text, re.search(pattern, name)) for name, text in zip(parts[1::2], parts[2::2])]
+    return [(name, text, match.groups()) for name, text, match in found if match]
+
+
+def longest_run(text):
+    """The most 16-bit loads in a row without a wait for loads between them."""
+    longest = run = 0
+    for line in text.splitlines():
+        line = line.strip()
+        if line.startswith("global_load_ushort"):
+            run += 1
+            longest = max(longest, run)
+        elif line.startswith("s_waitcnt") and "vmcnt" in line:
+            run = 0
+    return longest
+
+
+@pytest.mark.parametrize("source,pattern,instances", [("conv_store.hip", r"20conv_qkv_step_kernelIDF16bLi(\d+)E", 4)])
+def test_entries_of_the_state_are_asked_for_together(tmp_path, source, pattern, instances):
+    """bfloat16 entries, three of every piece of a row that a wave has: behind a question each they are awaited one by one."""
+    found = kernels(source, pattern, tmp_path)
+    assert len(found) == instances
+    for name, text, groups in found:
+        want = 3 * int(groups[0]) if groups else 3
+        assert longest_run(text) >= want, name
