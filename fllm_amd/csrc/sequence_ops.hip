@@ -59,6 +59,7 @@ short_conv_kernel(const T *__restrict__ x, const float *__restrict__ w, const T 
 // One workgroup a segment and block of channels, after the rows have been computed: the state becomes the last taps - 1 inputs of the sequence.
 // A thread owns a channel: it reads what it keeps of the old entries before it writes any.
 constexpr int kMaxKeep = 15;
+constexpr int kStepTaps = 4;      // norm_short_conv_kernel: at most
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
 short_conv_state_kernel(const T *__restrict__ x, T *__restrict__ state, const int32_t *__restrict__ row_seg,
@@ -89,10 +90,11 @@ short_conv_state_kernel(const T *__restrict__ x, T *__restrict__ state, const in
 // thread loops over channels and all it reads is on its way at once.  The normed value is rounded to T before it is used, as
 // the norm kernel's output would be, so that a token gives the same bits whether it came alone or in a portion.  A thread
 // owns a channel of the state: it reads the old entries before it writes any.
-// N > 0: the row (at most N * kBlock values) is asked for in one go; 0: any width.
+// N > 0: the row (at most N * kBlock values) is asked for in one go; 0: any width.  Up to four taps; FOUR: four of them, one 16-byte load.  Of fewer
+// the last ones are read again: behind a question each (is there an i-th) every 16-bit entry was awaited before the next was asked for.
 // Three trips to memory: the row's segment with everything that needs no place in the state, the segment's slot, the slot's entries, the
 // last beside the sum over the row; no load behind a condition (1,536 lanes at 4 rows 3.6 -> 1.8 us at best).
-template <typename T, int N, int TAPS>
+template <typename T, int N, bool FOUR>
 __global__ void __launch_bounds__(kBlock)
 norm_short_conv_kernel(const float *__restrict__ x, const int32_t *__restrict__ row_seg, const int32_t *__restrict__ slots,
                        const float *__restrict__ norm_w, const float *__restrict__ w, T *__restrict__ state, int width, int taps_,
@@ -100,7 +102,7 @@ norm_short_conv_kernel(const float *__restrict__ x, const int32_t *__restrict__ 
     __shared__ float scratch[kWaves];
     const int r = blockIdx.x;
     const int c = blockIdx.y * kBlock + threadIdx.x, at_c = min(c, width - 1);
-    const int seg = row_seg[r], taps = TAPS > 0 ? TAPS : taps_, keep = taps - 1;
+    const int seg = row_seg[r], taps = FOUR ? kStepTaps : taps_, keep = taps - 1;
     const float *src = x + (size_t)r * width, *wc = w + (size_t)at_c * taps;
     const float own = src[at_c], own_w = norm_w[at_c];
     float a[N > 0 ? N : 4];
@@ -108,24 +110,23 @@ norm_short_conv_kernel(const float *__restrict__ x, const int32_t *__restrict__ 
 #pragma unroll
         for (int j = 0; j < N; j++) a[j] = src[min((int)threadIdx.x + j * kBlock, width - 1)];
     }
-    constexpr int KEEP = TAPS > 0 ? TAPS - 1 : kMaxKeep;      // at most
-    float factor[KEEP + 1];
-    if constexpr (TAPS == 4) {
+    constexpr int KEEP = kStepTaps - 1;
+    float factor[kStepTaps];
+    if constexpr (FOUR) {
         *(f32x4_t *)factor = *(const f32x4_t *)wc;
     } else {
 #pragma unroll
-        for (int i = 0; i <= KEEP; i++)
-            if (i < taps) factor[i] = wc[i];
+        for (int i = 0; i < kStepTaps; i++) factor[i] = wc[min(i, keep)];
     }
     fetch_arguments(out, eps);
     // a padding row goes the whole way (a return here would be a wait ahead of the first loads) and stores zeros, no state
     const bool padding = seg < 0;
     const int slot = slots[max(seg, 0)];
     T *mine = state + (size_t)(padding ? 0 : slot) * keep * width;
+    const T *kept = keep > 0 ? mine : (const T *)src;      // one tap: read, never used
     T held[KEEP];
 #pragma unroll
-    for (int i = 0; i < KEEP; i++)
-        if (i < keep) held[i] = mine[(size_t)i * width + at_c];
+    for (int i = 0; i < KEEP; i++) held[i] = kept[(size_t)(FOUR ? i : max(min(i, keep - 1), 0)) * width + at_c];
     float ss = 0.f;
     if constexpr (N > 0) {
 #pragma unroll
@@ -158,6 +159,54 @@ norm_short_conv_kernel(const float *__restrict__ x, const int32_t *__restrict__ 
     for (int i = 0; i <= KEEP; i++)
         if (i == keep) acc = fmaf(factor[i], now, acc);
     out[(size_t)r * width + c] = from_f32<T>(padding ? 0.f : now + acc);
+}
+
+// More than four taps, as they come: all of them ahead of the sum were more loads than the trips they spared (eight taps: 64 rows of 8,192 lanes
+// 18.3 us, 12.3 like this, of 256 lanes 4.8 and 4.25).
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+norm_short_conv_taps_kernel(const float *__restrict__ x, const float *__restrict__ norm_w, float eps, const float *__restrict__ w,
+                            T *__restrict__ state, const int32_t *__restrict__ row_seg, const int32_t *__restrict__ slots,
+                            T *__restrict__ out, int width, int taps) {
+    __shared__ float scratch[kWaves];
+    const int r = blockIdx.x;
+    const int c = blockIdx.y * kBlock + threadIdx.x;
+    const int seg = row_seg[r];
+    if (seg < 0) {   // padding row
+        if (c < width) out[(size_t)r * width + c] = from_f32<T>(0.f);
+        return;
+    }
+    const float *src = x + (size_t)r * width;
+    float ss = 0.f;
+    for (int i0 = threadIdx.x; i0 < width; i0 += 4 * kBlock) {      // four loads on their way at once, summed in the row's order
+        float a[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) a[j] = i0 + j * kBlock < width ? src[i0 + j * kBlock] : 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; j++) ss = fmaf(a[j], a[j], ss);
+    }
+    ss = block_sum<kWaves>(ss, scratch);
+    if (c >= width) return;
+    const float inv = 1.0f / sqrtf(ss / (float)width + eps);
+    const int keep = taps - 1;
+    T *mine = state + (size_t)slots[seg] * keep * width;
+    const float *wc = w + (size_t)c * taps;
+    T held[kMaxKeep];
+#pragma unroll
+    for (int i = 0; i < kMaxKeep; i++)
+        if (i < keep) held[i] = mine[(size_t)i * width + c];
+    const T h = from_f32<T>(src[c] * (inv * norm_w[c]));
+    const float now = to_f32<T>(h);
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < kMaxKeep; i++) {      // oldest input first; entry i moves to i - 1
+        if (i >= keep) break;
+        acc = fmaf(wc[i], to_f32<T>(held[i]), acc);
+        if (i > 0) mine[(size_t)(i - 1) * width + c] = held[i];
+    }
+    if (keep > 0) mine[(size_t)(keep - 1) * width + c] = h;
+    acc = fmaf(wc[taps - 1], now, acc);
+    out[(size_t)r * width + c] = from_f32<T>(now + acc);
 }
 
 // ---- linear attention, one token after the other ----------------------------------------------------------------------------
@@ -564,16 +613,20 @@ extern "C" int fllm_norm_short_conv(const float *x, const float *norm_w, float e
     FLLM_REQUIRE(x && norm_w && w && out && row_seg && slots && (state || taps == 1), "norm_short_conv: operands missing");
     if (rows == 0) return 0;
     const dim3 grid(rows, (width + kBlock - 1) / kBlock);
-#define FLLM_NSC(T, N, TAPS)                                                                                                             \
-    hipLaunchKernelGGL((norm_short_conv_kernel<T, N, TAPS>), grid, dim3(kBlock), 0, stream, x, row_seg, slots, norm_w, w, (T *)state, width, \
+#define FLLM_NSC(T, N, FOUR)                                                                                                             \
+    hipLaunchKernelGGL((norm_short_conv_kernel<T, N, FOUR>), grid, dim3(kBlock), 0, stream, x, row_seg, slots, norm_w, w, (T *)state, width, \
                        taps, (T *)out, eps)
-    // four taps are one 16-byte load; any other number is a load each, behind a question each
-#define FLLM_NSC_N(T)                                                      \
-    do {                                                                   \
-        const bool four = taps == 4 && ((uintptr_t)w & 15) == 0;           \
-        if (four && width <= 8 * kBlock) FLLM_NSC(T, 8, 4);                \
-        else if (width <= 8 * kBlock) FLLM_NSC(T, 8, 0);                   \
-        else FLLM_NSC(T, 0, 0);                                            \
+    // four taps are one 16-byte load, up to three a load each
+#define FLLM_NSC_N(T)                                                                                                                    \
+    do {                                                                                                                                 \
+        const bool four = taps == 4 && ((uintptr_t)w & 15) == 0;                                                                         \
+        if (taps > kStepTaps)                                                                                                            \
+            hipLaunchKernelGGL(norm_short_conv_taps_kernel<T>, grid, dim3(kBlock), 0, stream, x, norm_w, eps, w, (T *)state, row_seg,     \
+                               slots, (T *)out, width, taps);                                                                            \
+        else if (four && width <= 8 * kBlock) FLLM_NSC(T, 8, true);                                                                      \
+        else if (four) FLLM_NSC(T, 0, true);                                                                                             \
+        else if (width <= 8 * kBlock) FLLM_NSC(T, 8, false);                                                                             \
+        else FLLM_NSC(T, 0, false);                                                                                                      \
     } while (0)
     if (dtype == FLLM_F32) FLLM_NSC_N(float);
     else if (dtype == FLLM_BF16) FLLM_NSC_N(bf16_t);

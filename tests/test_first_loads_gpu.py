@@ -118,6 +118,32 @@ def test_norms_with_four_taps(ops, width, dtype):
     assert not any(o[2].any() for o in results[0][:3]) and all(torch.equal(s[[0, 2]], state[[0, 2]]) for s in results[0][3:])
 
 
+@pytest.mark.parametrize("width,taps", [(40, 1), (40, 3), (1020, 4), (2048, 2), (2052, 3), (2052, 4), (5000, 1)])
+@pytest.mark.parametrize("dtype", [F32, BF16])
+def test_norms_with_few_taps_and_with_more(ops, width, taps, dtype):
+    """Up to four taps and more of them are kernels of their own, rows of up to 2,048 lanes and wider ones instances: taps of zero ahead of the
+    others leave the bits as they are, whatever the entries that they meet."""
+    g = torch.Generator().manual_seed(width + taps)
+    rows, ahead = 3, 6 - taps
+    x, w1, w2 = torch.randn(rows, width, generator=g).to(DEV), torch.rand(width, generator=g).to(DEV), torch.rand(width, generator=g).to(DEV)
+    conv, state = torch.randn(width, taps, generator=g).to(DEV), torch.randn(4, taps - 1, width, generator=g).to(dtype).to(DEV)
+    conv6, state6 = torch.cat([torch.zeros(width, ahead, device=DEV), conv], 1), torch.cat([torch.randn(4, ahead, width, generator=g).to(dtype).to(DEV), state], 1)
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    row_seg, slots = i32(0, 1, -1), i32(3, 1, 0)
+    results = []
+    for w, st in ((conv, state), (conv6, state6)):
+        a, b = st.clone(), st.clone()
+        outs = [torch.full((rows, width), 7.0, dtype=dtype, device=DEV) for _ in range(4)]
+        ops.norm_short_conv(x, w1, 1e-5, w, a if w.shape[1] > 1 else None, row_seg, slots, outs[0])
+        assert ops.layernorm_conv(x, w1, 1e-5, w, b if w.shape[1] > 1 else None, row_seg, slots, outs[1], w2, 1e-3, outs[2])
+        assert ops.layernorm_conv(x, w1, 1e-5, w, st.clone() if w.shape[1] > 1 else None, row_seg, slots, outs[3])      # one norm
+        results.append(outs + [t[:, t.shape[1] - (taps - 1):] for t in (a, b)])
+    for one, other in zip(*results):
+        assert torch.equal(one, other)
+    assert torch.equal(results[0][1], results[0][3]) and not any(o[2].any() for o in results[0][:4])
+    assert all(torch.equal(t[[0, 2]], state[[0, 2]]) for t in results[0][4:])
+
+
 @pytest.mark.parametrize("width", [4, 1024, 1028, 2044, 4096, 8192])
 @pytest.mark.parametrize("branch", [F32, BF16])
 @pytest.mark.parametrize("out", [F32, BF16])
