@@ -16,6 +16,7 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / kWave;
 constexpr int kMaxKeep = 15;
+constexpr int kStepTaps = 4;      // layernorm_conv_kernel: at most
 
 // N > 0: the row (at most N * kBlock values) stays in registers between the mean, the deviations and the output; 0: any width
 template <typename T, int N>
@@ -74,7 +75,9 @@ layernorm_kernel(const float *__restrict__ x, const int32_t *__restrict__ rows, 
 // thread loops over channels behind the sums and all it reads is on its way at once.  The first norm's value is rounded to T before
 // the convolution, as layernorm_kernel's output is.  A thread owns a channel of the state: it reads the old entries before it
 // writes any.
-template <typename T, int N, int TAPS>
+// Up to four taps; FOUR: four of them, one 16-byte load.  Of fewer the last ones are read again: behind a question each (is there an i-th) every
+// 16-bit entry was awaited before the next was asked for.
+template <typename T, int N, bool FOUR>
 __global__ void __launch_bounds__(kBlock)
 layernorm_conv_kernel(const float *__restrict__ x, const int32_t *__restrict__ row_seg, const int32_t *__restrict__ slots,
                       const float *__restrict__ w1, const float *__restrict__ w2 /* null: one norm */, const float *__restrict__ conv, int width, int taps_,
@@ -84,20 +87,19 @@ layernorm_conv_kernel(const float *__restrict__ x, const int32_t *__restrict__ r
     const bool mine = c < width;
     // Three trips to memory: the row's segment with everything that needs no place in the state, the segment's slot, the slot's entries,
     // the last beside the sums over the row.  No load sits behind a condition (1,536 lanes at 16 rows 4.1 -> 3.2 us at best).
-    const int seg = row_seg[r], at_c = min(c, width - 1), taps = TAPS > 0 ? TAPS : taps_, keep = taps - 1;
+    const int seg = row_seg[r], at_c = min(c, width - 1), taps = FOUR ? kStepTaps : taps_, keep = taps - 1;
     const float *src = x + (size_t)r * width, *wc = conv + (size_t)at_c * taps;
     const float own = src[at_c], a1 = w1[at_c], a2 = (w2 != nullptr ? w2 : w1)[at_c];
     float v[N];
 #pragma unroll
     for (int j = 0; j < N; j++) v[j] = src[min((int)threadIdx.x + j * kBlock, width - 1)];
-    constexpr int KEEP = TAPS > 0 ? TAPS - 1 : kMaxKeep;      // at most
-    float factor[KEEP + 1];
-    if constexpr (TAPS == 4) {
+    constexpr int KEEP = kStepTaps - 1;
+    float factor[kStepTaps];
+    if constexpr (FOUR) {
         *(f32x4_t *)factor = *(const f32x4_t *)wc;
     } else {
 #pragma unroll
-        for (int i = 0; i <= KEEP; i++)
-            if (i < taps) factor[i] = wc[i];
+        for (int i = 0; i < kStepTaps; i++) factor[i] = wc[min(i, keep)];
     }
     fetch_arguments(state, out1, out2, eps1, eps2);
     T *d1 = out1 + (size_t)r * width, *d2 = out2 == nullptr ? nullptr : out2 + (size_t)r * width;
@@ -105,10 +107,10 @@ layernorm_conv_kernel(const float *__restrict__ x, const int32_t *__restrict__ r
     const bool padding = seg < 0;
     const int slot = slots[max(seg, 0)];
     T *old = state + (size_t)(padding ? 0 : slot) * keep * width;
+    const T *kept = keep > 0 ? old : (const T *)src;      // one tap: read, never used
     T held[KEEP];
 #pragma unroll
-    for (int i = 0; i < KEEP; i++)
-        if (i < keep) held[i] = old[(size_t)i * width + at_c];
+    for (int i = 0; i < KEEP; i++) held[i] = kept[(size_t)(FOUR ? i : max(min(i, keep - 1), 0)) * width + at_c];
     float sum = 0.f;
 #pragma unroll
     for (int j = 0; j < N; j++) {
@@ -140,6 +142,65 @@ layernorm_conv_kernel(const float *__restrict__ x, const int32_t *__restrict__ r
         if (i == keep) acc = fmaf(factor[i], now, acc);
     d1[c] = from_f32<T>(padding ? 0.f : now + acc);
     if (d2 != nullptr) d2[c] = from_f32<T>(padding ? 0.f : (own - mean) * (inv2 * a2));
+}
+
+// More than four taps, as they come: all of them ahead of the sums were more loads than the trips they spared (eight taps: 64 rows of 8,192 lanes
+// 20.3 us, 14.4 like this, of 256 lanes 5.1 and 4.7).
+template <typename T, int N>
+__global__ void __launch_bounds__(kBlock)
+layernorm_conv_taps_kernel(const float *__restrict__ x, const float *__restrict__ w1, float eps1, const float *__restrict__ conv, int taps,
+                           T *__restrict__ state, const int32_t *__restrict__ row_seg, const int32_t *__restrict__ slots, T *__restrict__ out1,
+                           const float *__restrict__ w2, float eps2, T *__restrict__ out2, int width) {
+    __shared__ float scratch[kWaves];
+    const int r = blockIdx.x, c = blockIdx.y * kBlock + threadIdx.x;
+    const bool mine = c < width;
+    T *d1 = out1 + (size_t)r * width, *d2 = out2 == nullptr ? nullptr : out2 + (size_t)r * width;
+    const int seg = row_seg[r];
+    if (seg < 0) {      // padding row
+        if (mine) d1[c] = from_f32<T>(0.f);
+        if (mine && d2 != nullptr) d2[c] = from_f32<T>(0.f);
+        return;
+    }
+    const int keep = taps - 1;
+    T *old = state + (size_t)slots[seg] * keep * width;
+    const float *wc = conv + (size_t)c * taps;
+    T held[kMaxKeep];
+#pragma unroll
+    for (int i = 0; i < kMaxKeep; i++)
+        if (i < keep && mine) held[i] = old[(size_t)i * width + c];
+    const float *src = x + (size_t)r * width;
+    const float own = mine ? src[c] : 0.f, a1 = mine ? w1[c] : 0.f, a2 = mine && d2 != nullptr ? w2[c] : 0.f;
+    float v[N];
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        const int at = threadIdx.x + j * kBlock;
+        v[j] = at < width ? src[at] : 0.f;
+        sum += v[j];
+    }
+    const float mean = block_sum<kWaves>(sum, scratch) / (float)width;
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        v[j] -= mean;
+        if (threadIdx.x + j * kBlock < width) ss = fmaf(v[j], v[j], ss);
+    }
+    const float var = block_sum<kWaves>(ss, scratch) / (float)width;
+    if (!mine) return;
+    const float inv1 = 1.0f / sqrtf(var + eps1), inv2 = 1.0f / sqrtf(var + eps2);
+    const T h = from_f32<T>((own - mean) * (inv1 * a1));
+    const float now = to_f32<T>(h);
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < kMaxKeep; i++) {      // oldest input first; entry i moves to i - 1
+        if (i >= keep) break;
+        acc = fmaf(wc[i], to_f32<T>(held[i]), acc);
+        if (i > 0) old[(size_t)(i - 1) * width + c] = held[i];
+    }
+    if (keep > 0) old[(size_t)(keep - 1) * width + c] = h;
+    acc = fmaf(wc[keep], now, acc);
+    d1[c] = from_f32<T>(now + acc);
+    if (d2 != nullptr) d2[c] = from_f32<T>((own - mean) * (inv2 * a2));
 }
 
 __global__ void __launch_bounds__(kBlock)
@@ -299,22 +360,29 @@ extern "C" int fllm_layernorm_conv(const float *x, const float *w1, float eps1, 
                      (w2 == nullptr || eps2 > 0.f), "layernorm_conv: operands missing");
     if (rows == 0) return 0;
     const dim3 grid(rows, (width + kBlock - 1) / kBlock);
-#define FLLM_LNC(T, N, TAPS)                                                                                                                  \
-    hipLaunchKernelGGL((layernorm_conv_kernel<T, N, TAPS>), grid, dim3(kBlock), 0, stream, x, row_seg, slots, w1, w2, conv, width, taps,       \
+#define FLLM_LNC(T, N, FOUR)                                                                                                                 \
+    hipLaunchKernelGGL((layernorm_conv_kernel<T, N, FOUR>), grid, dim3(kBlock), 0, stream, x, row_seg, slots, w1, w2, conv, width, taps,      \
                        (T *)state, (T *)out1, (T *)out2, eps1, eps2)
-    // four taps are one 16-byte load; any other number is a load each, behind a question each
+#define FLLM_LNC_TAPS(T, N)                                                                                                                  \
+    hipLaunchKernelGGL((layernorm_conv_taps_kernel<T, N>), grid, dim3(kBlock), 0, stream, x, w1, eps1, conv, taps, (T *)state, row_seg, slots, \
+                       (T *)out1, w2, eps2, (T *)out2, width)
+    // four taps are one 16-byte load, up to three a load each
 #define FLLM_LNC_N(T)                                                                      \
     do {                                                                                   \
         const bool four = taps == 4 && ((uintptr_t)conv & 15) == 0;                        \
-        if (four && width <= 8 * kBlock) FLLM_LNC(T, 8, 4);                                \
-        else if (width <= 4 * kBlock) FLLM_LNC(T, 4, 0);                                   \
-        else if (width <= 8 * kBlock) FLLM_LNC(T, 8, 0);                                   \
-        else FLLM_LNC(T, 32, 0);                                                           \
+        if (taps > kStepTaps && width <= 4 * kBlock) FLLM_LNC_TAPS(T, 4);                  \
+        else if (taps > kStepTaps && width <= 8 * kBlock) FLLM_LNC_TAPS(T, 8);             \
+        else if (taps > kStepTaps) FLLM_LNC_TAPS(T, 32);                                   \
+        else if (four && width <= 8 * kBlock) FLLM_LNC(T, 8, true);                        \
+        else if (four) FLLM_LNC(T, 32, true);                                              \
+        else if (width <= 8 * kBlock) FLLM_LNC(T, 8, false);                               \
+        else FLLM_LNC(T, 32, false);                                                       \
     } while (0)
     if (out_dtype == FLLM_F32) FLLM_LNC_N(float);
     else if (out_dtype == FLLM_BF16) FLLM_LNC_N(bf16_t);
     else FLLM_REQUIRE(false, "layernorm_conv: unknown dtype %d", out_dtype);
 #undef FLLM_LNC_N
+#undef FLLM_LNC_TAPS
 #undef FLLM_LNC
     return fllm_check_launch("layernorm_conv");
 }

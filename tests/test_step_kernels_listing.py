@@ -39,7 +39,8 @@ def longest_run(text):
 
 
 @pytest.mark.parametrize("source,pattern,instances", [("conv_store.hip", r"20conv_qkv_step_kernelIDF16bLi(\d+)E", 4),
-                                                      ("sequence_ops.hip", r"22norm_short_conv_kernelIDF16b", 4)])
+                                                      ("sequence_ops.hip", r"22norm_short_conv_kernelIDF16b", 4),
+                                                      ("layer_norms.hip", r"21layernorm_conv_kernelIDF16b", 4)])
 def test_entries_of_the_state_are_asked_for_together(tmp_path, source, pattern, instances):
     """bfloat16 entries, three of every piece of a row that a wave has: behind a question each they are awaited one by one."""
     found = kernels(source, pattern, tmp_path)
