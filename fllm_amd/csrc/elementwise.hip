@@ -344,6 +344,8 @@ extern "C" int fllm_add_residual(float *residual, const void *branch, int rows, 
 // share 8 rows (a read and a write of the same buffer cannot overlap inside a thread, so many short threads beat few
 // long ones); where the rows are 8 consecutive tokens of one request that start at a multiple of 8 (a prompt portion), their values go
 // into the transposed page as one 16-byte store per head lane instead of eight 2-byte ones.
+// One row a workgroup (RB 1) is placed by one thread, and a piece asks for its angles if it turns: in the form for portions, where a wave places the rows
+// and every piece reads angles, 16 rows of 32 + 8 heads of 128 were 4.47 us instead of 4.23, of 64 + 8 with 64 lanes turning 5.44 instead of 5.00.
 template <int RB, int U>
 __global__ void __launch_bounds__(kBlock)
 rope_kv_store_vec_kernel(bf16_t *__restrict__ qkv, const int32_t *__restrict__ row_pos, const int32_t *__restrict__ row_seg,
@@ -359,7 +361,15 @@ rope_kv_store_vec_kernel(bf16_t *__restrict__ qkv, const int32_t *__restrict__ r
     const int per_head_v = v_dim / 8;
     // position (-1: padding row), page and slot of the workgroup's rows
     __shared__ int s_pos[RB], s_page[RB], s_off[RB], s_run;
-    if ((int)threadIdx.x < kWave) {      // one wave: a lane a row, so that the rows are asked for together
+    if constexpr (RB == 1) {
+        if (threadIdx.x == 0) {
+            const int seg = row_seg[r0], pos = row_pos[r0];
+            s_pos[0] = seg < 0 ? -1 : pos;
+            s_page[0] = (store_kv && seg >= 0) ? tables[(size_t)seg * table_stride + pos / page_size] : 0;
+            s_off[0] = pos % page_size;
+            s_run = 0;
+        }
+    } else if ((int)threadIdx.x < kWave) {      // one wave: a lane a row, so that the rows are asked for together
         const int i = min((int)threadIdx.x, nrows - 1), r = r0 + i;
         const int seg = row_seg[r], pos = row_pos[r];
         const int seg0 = __builtin_amdgcn_readfirstlane(seg), pos0 = __builtin_amdgcn_readfirstlane(pos);
@@ -379,39 +389,54 @@ rope_kv_store_vec_kernel(bf16_t *__restrict__ qkv, const int32_t *__restrict__ r
     // queries and keys: every (row, 16-byte chunk) is a piece of work of its own, so that a thread has several in flight
     const int per_row = rot_heads * per_head;
     const int first = blockIdx.y * kBlock + threadIdx.x, stride = gridDim.y * kBlock;   // the workgroups of a row group share its pieces
-    // U pieces of a thread on their way together
-    for (int it0 = first; it0 < nrows * per_row; it0 += U * stride) {
-        bf16x8_t v[U];
-        f32x4_t c4[U], s4[U];
-        int row_of[U], head_of[U], lane_of[U];
+    auto rotate = [&](bf16x8_t &v, const f32x4_t &c4, const f32x4_t &s4) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int it = min(it0 + u * stride, nrows * per_row - 1);
-            const int i = RB == 1 ? 0 : it / per_row, t = it - i * per_row;
-            const int h = t / per_head, c = (t - h * per_head) * 8;
-            row_of[u] = i, head_of[u] = h, lane_of[u] = c;
-            v[u] = *(const bf16x8_t *)(qkv + (size_t)(r0 + i) * row_elems + (size_t)h * head_dim + c);
-            if (rope_dims > 0) {
-                const size_t angle = (size_t)max(s_pos[i], 0) * half + (c < rope_dims ? c / 2 : 0);
-                c4[u] = *(const f32x4_t *)(cos_table + angle);
-                s4[u] = *(const f32x4_t *)(sin_table + angle);
-            }
+        for (int p = 0; p < 4; p++) {
+            const float a = (float)v[2 * p], b = (float)v[2 * p + 1];
+            v[2 * p] = (bf16_t)fmaf(a, c4[p], -(b * s4[p]));      // which product is rounded is the same in every instance
+            v[2 * p + 1] = (bf16_t)fmaf(a, s4[p], b * c4[p]);
         }
-        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto store = [&](const bf16x8_t &v, int i, int h, int c) __attribute__((always_inline)) {
+        if (h < heads) *(bf16x8_t *)(qkv + (size_t)(r0 + i) * row_elems + (size_t)h * head_dim + c) = v;
+        else *(bf16x8_t *)(k_pages + key_offset(s_page[i], kv_heads, h - heads, page_size, head_dim, s_off[i], c)) = v;
+    };
+    if constexpr (RB == 1) {
+        const int pos = s_pos[0];
+        if (pos < 0) return;   // padding row
+        for (int it = first; it < per_row; it += stride) {
+            const int h = it / per_head, c = (it - h * per_head) * 8;
+            bf16x8_t v = *(const bf16x8_t *)(qkv + (size_t)r0 * row_elems + (size_t)h * head_dim + c);
+            if (c < rope_dims)   // rope_dims is a multiple of 8: the chunk is rotated as a whole
+                rotate(v, *(const f32x4_t *)(cos_table + (size_t)pos * half + c / 2), *(const f32x4_t *)(sin_table + (size_t)pos * half + c / 2));
+            store(v, 0, h, c);
+        }
+    } else {
+        // U pieces of a thread on their way together
+        for (int it0 = first; it0 < nrows * per_row; it0 += U * stride) {
+            bf16x8_t v[U];
+            f32x4_t c4[U], s4[U];
+            int row_of[U], head_of[U], lane_of[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int i = row_of[u], h = head_of[u], c = lane_of[u];
-            if (it0 + u * stride >= nrows * per_row || s_pos[i] < 0) continue;   // no such piece, or a padding row
-            if (c < rope_dims) {   // rope_dims is a multiple of 8: the chunk is rotated as a whole
-#pragma unroll
-                for (int p = 0; p < 4; p++) {
-                    const float a = (float)v[u][2 * p], b = (float)v[u][2 * p + 1];
-                    v[u][2 * p] = (bf16_t)fmaf(a, c4[u][p], -(b * s4[u][p]));      // which product is rounded is the same in every instance
-                    v[u][2 * p + 1] = (bf16_t)fmaf(a, s4[u][p], b * c4[u][p]);
+            for (int u = 0; u < U; u++) {
+                const int it = min(it0 + u * stride, nrows * per_row - 1);
+                const int i = it / per_row, t = it - i * per_row;
+                const int h = t / per_head, c = (t - h * per_head) * 8;
+                row_of[u] = i, head_of[u] = h, lane_of[u] = c;
+                v[u] = *(const bf16x8_t *)(qkv + (size_t)(r0 + i) * row_elems + (size_t)h * head_dim + c);
+                if (rope_dims > 0) {
+                    const size_t angle = (size_t)max(s_pos[i], 0) * half + (c < rope_dims ? c / 2 : 0);
+                    c4[u] = *(const f32x4_t *)(cos_table + angle);
+                    s4[u] = *(const f32x4_t *)(sin_table + angle);
                 }
             }
-            if (h < heads) *(bf16x8_t *)(qkv + (size_t)(r0 + i) * row_elems + (size_t)h * head_dim + c) = v[u];
-            else *(bf16x8_t *)(k_pages + key_offset(s_page[i], kv_heads, h - heads, page_size, head_dim, s_off[i], c)) = v[u];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (it0 + u * stride >= nrows * per_row || s_pos[row_of[u]] < 0) continue;   // no such piece, or a padding row
+                if (lane_of[u] < rope_dims) rotate(v[u], c4[u], s4[u]);   // rope_dims is a multiple of 8: the chunk is rotated as a whole
+                store(v[u], row_of[u], head_of[u], lane_of[u]);
+            }
         }
     }
     if (!store_kv) return;
