@@ -13,6 +13,7 @@
 // Weights stay float32: P goes into the product as the sum of two bfloat16 numbers (its rounding and what the rounding
 // lost), two products a tile.  The means of blocks are float32 in memory and go in the same way, for keys and for values.
 #include <algorithm>
+#include <type_traits>
 
 #include "api.h"
 #include "common.h"
@@ -68,15 +69,20 @@ __device__ __forceinline__ void publish(float *at, float v) { __hip_atomic_store
 // hand-over of the shares: windows of 1,024 with pooled blocks, 2 rows of 12 heads on two of 128 13.9 -> 12.5 us, sigmoid weights 10.3 -> 9.9.
 // Pages of a power of two have instances of their own: divisions by the page size, or the question at each address, cost more than they
 // save (2,000 rows 57 us with divisions, 63 with the question, 55 like this).
-template <int KD, int VT, int VARIANT, bool POW2>
+// BY_HEADS: tiles of single rows.  Tiles of 16 rows have instances of their own, which ask for a pooled block's keys and values as they come: a prompt
+// has enough workgroups to cover the trips, and what all of them at once hold in registers cost it a wave a SIMD (1,900 rows of 12 heads on two, windows of
+// 1,024, keys and values of 64 and 96 lanes 47.5 us, 49.2 all at once, 44.4 like this; 128 and 64 43.6, 44.8, 40.9; with pages of 48 tokens
+// 44.1, 48.7, 44.0).
+template <int KD, int VT, int VARIANT, bool POW2, bool BY_HEADS>
 __global__ void __launch_bounds__(kThreads)
 mixer_tile_kernel(const int32_t *__restrict__ row_seg, const int32_t *__restrict__ row_pos, const int32_t *__restrict__ tables,
-                  const bf16_t *__restrict__ q, int table_stride, int heads, int kv_heads, int q_stride, int by_heads, int page_shift,
+                  const bf16_t *__restrict__ q, int table_stride, int heads, int kv_heads, int q_stride, int page_shift,
                   const TileParams p) {
     typedef const __attribute__((address_space(4))) int32_t *constant_t;      // the same for every lane: a scalar load
     constexpr int D = KD * 32, DV = VT * 16;
     __shared__ float sm_o[kWavesM][16][DV + 1];
     __shared__ float sm_m[kWavesM][16], sm_l[kWavesM][16];
+    constexpr bool by_heads = BY_HEADS;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int qi = lane & 15, g = lane >> 4;
     // ---- which queries this tile holds
@@ -210,28 +216,37 @@ mixer_tile_kernel(const int32_t *__restrict__ row_seg, const int32_t *__restrict
                 const int end = min(b, nb_max - 1) * p.pool + p.pool - 1;
                 return ((size_t)tbl[page_of(end)] * kv_heads + kvh) * p.slots + (p.slots > 1 ? in_page(end) / p.pool : 0);
             };
-            size_t kat[2], vat[8];
-#pragma unroll
-            for (int j = 0; j < 2; j++) kat[j] = mean_of(base + (qi >> 2) * 8 + j * 4 + (qi & 3)) * D;
             // A = V^T: row = a value lane, k = the blocks base + g * 8 + e, each in a page and slot of its own
-#pragma unroll
-            for (int e = 0; e < 8; e++) vat[e] = mean_of(base + g * 8 + e) * DV;
+            size_t vat[8];
             f32x4_t kx[2][KD][2];
             float vx[VT][8];
-#pragma unroll
-            for (int j = 0; j < 2; j++)
+            auto ask_keys = [&](int j) __attribute__((always_inline)) {
+                const float *kr = p.pool_k + mean_of(base + (qi >> 2) * 8 + j * 4 + (qi & 3)) * D;
 #pragma unroll
                 for (int kk = 0; kk < KD; kk++)
 #pragma unroll
-                    for (int i = 0; i < 2; i++) kx[j][kk][i] = *(const f32x4_t *)(p.pool_k + kat[j] + kk * 32 + g * 8 + 4 * i);
+                    for (int i = 0; i < 2; i++) kx[j][kk][i] = *(const f32x4_t *)(kr + kk * 32 + g * 8 + 4 * i);
+            };
+            auto places = [&]() __attribute__((always_inline)) {
 #pragma unroll
-            for (int t = 0; t < VT; t++)
+                for (int e = 0; e < 8; e++) vat[e] = mean_of(base + g * 8 + e) * DV;
+            };
+            auto ask_values = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
                 for (int e = 0; e < 8; e++) vx[t][e] = p.pool_v[vat[e] + t * 16 + qi];
-            __builtin_amdgcn_sched_barrier(0);      // all of them before the first product
+            };
+            if constexpr (by_heads) {
+                places();
+#pragma unroll
+                for (int j = 0; j < 2; j++) ask_keys(j);
+#pragma unroll
+                for (int t = 0; t < VT; t++) ask_values(t);
+                __builtin_amdgcn_sched_barrier(0);      // all of them before the first product
+            }
             f32x4_t s[2];
 #pragma unroll
             for (int j = 0; j < 2; j++) {
+                if constexpr (!by_heads) ask_keys(j);
                 s[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int kk = 0; kk < KD; kk++) {
@@ -247,8 +262,10 @@ mixer_tile_kernel(const int32_t *__restrict__ row_seg, const int32_t *__restrict
             weigh_and_add(
                 s, [&](int slot) { return valid && base + slot < nb_q; }, [&](int) { return 0.f; },
                 [&](const bf16x8_t &p_hi, const bf16x8_t &p_lo) {
+                    if constexpr (!by_heads) places();
 #pragma unroll
                     for (int t = 0; t < VT; t++) {
+                        if constexpr (!by_heads) ask_values(t);
                         bf16x8_t hi, lo;
                         split_bf16(vx[t], hi, lo);
                         o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, p_hi, o[t], 0, 0, 0);
@@ -427,15 +444,20 @@ int launch_vt(const TileParams &p, int vt, dim3 grid, hipStream_t stream) {
     if ((p.page_size & (p.page_size - 1)) == 0) shift = __builtin_ctz((unsigned)p.page_size);
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, p.row_seg, p.row_pos, p.tables, p.q, p.table_stride, p.heads, p.kv_heads,
-                           p.q_stride, p.by_heads, shift, p);
+                           p.q_stride, shift, p);
     };
-    switch (vt) {
-    case 2: shift >= 0 ? go(mixer_tile_kernel<KD, 2, VARIANT, true>) : go(mixer_tile_kernel<KD, 2, VARIANT, false>); return 0;
-    case 4: shift >= 0 ? go(mixer_tile_kernel<KD, 4, VARIANT, true>) : go(mixer_tile_kernel<KD, 4, VARIANT, false>); return 0;
-    case 6: shift >= 0 ? go(mixer_tile_kernel<KD, 6, VARIANT, true>) : go(mixer_tile_kernel<KD, 6, VARIANT, false>); return 0;
-    case 8: shift >= 0 ? go(mixer_tile_kernel<KD, 8, VARIANT, true>) : go(mixer_tile_kernel<KD, 8, VARIANT, false>); return 0;
-    }
-    return 1;
+    auto of = [&](auto pow2, auto by_heads) {
+        constexpr bool P = decltype(pow2)::value, B = decltype(by_heads)::value;
+        switch (vt) {
+        case 2: go(mixer_tile_kernel<KD, 2, VARIANT, P, B>); return 0;
+        case 4: go(mixer_tile_kernel<KD, 4, VARIANT, P, B>); return 0;
+        case 6: go(mixer_tile_kernel<KD, 6, VARIANT, P, B>); return 0;
+        case 8: go(mixer_tile_kernel<KD, 8, VARIANT, P, B>); return 0;
+        }
+        return 1;
+    };
+    if (p.by_heads) return shift >= 0 ? of(std::true_type{}, std::true_type{}) : of(std::false_type{}, std::true_type{});
+    return shift >= 0 ? of(std::true_type{}, std::false_type{}) : of(std::false_type{}, std::false_type{});
 }
 
 template <int VARIANT>

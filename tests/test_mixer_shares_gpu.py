@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from reference_ops import ReferenceOps
-from test_dumizen_gpu import BF16_EPS, DEV, Scene, close, fill_pools, gen, pooled_attend
+from test_dumizen_gpu import BF16_EPS, DEV, SEGMENTS, SINGLE_ROWS, Scene, close, fill_pools, gen, pooled_attend
 
 pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
@@ -52,3 +52,29 @@ def test_shares_of_single_rows(ops, H, G, d, dv, contexts):
     t["row_seg"][1] = -1                                                               # a padding row of a captured step
     padded = pooled_attend(ops, t, q.to(DEV, BF16), sc, H, G, d, dv, 0.3, window, pool, BF16)
     assert torch.equal(padded[0], first[0][0]) and torch.equal(padded[2:], first[0][2:]) and not padded[1].any()
+
+
+@pytest.mark.parametrize("rows", ["mixed", "single"])
+@pytest.mark.parametrize("H,G,d,dv,page,pool", [(4, 1, 32, 64, 48, 8), (8, 2, 64, 96, 48, 20), (9, 3, 96, 96, 48, 16), (12, 2, 128, 128, 80, 32)])
+def test_pages_that_are_no_power_of_two(ops, H, G, d, dv, page, pool, rows):
+    """Pages of a power of two have instances of their own; these are the others, with blocks that divide the pages and blocks that do not."""
+    ref, window = ReferenceOps(), 70
+    sc = Scene(SINGLE_ROWS if rows == "single" else SEGMENTS, G, d, dv, page, seed=H + d, pool=pool)
+    g = gen(3)
+    q = torch.randn(sc.rows, H * d, generator=g).to(BF16).float()
+    r1, r2, pb = torch.rand(H, generator=g) + 0.2, torch.rand(H, generator=g) * 0.5 + 0.05, torch.randn(H, generator=g) - 1.0
+    want_t = sc.to("cpu", torch.float64)
+    want_t["k_pages"], want_t["v_pages"] = want_t["k_pages"].to(BF16).double(), want_t["v_pages"].to(BF16).double()
+    fill_pools(ref, sc, want_t, G, d, dv, pool)
+    t = sc.to(DEV, BF16)
+    t["pool_k"], t["pool_v"] = want_t["pool_k"].float().to(DEV), want_t["pool_v"].float().to(DEV)
+    outs = []
+    for o, tensors, on, kind in ((ref, want_t, "cpu", torch.float64), (ops, t, DEV, BF16)):
+        pooled = pooled_attend(o, tensors, q.to(on, kind), sc, H, G, d, dv, 0.3, window, pool, kind)
+        weighed = torch.empty(sc.rows, H * dv, dtype=kind, device=on)
+        o.sigmoid_attention(q.to(on, kind), tensors["k_pages"], tensors["v_pages"], tensors["tables"], tensors["row_pos"], tensors["row_seg"],
+                            tensors["seg_start"], weighed, H, G, d, dv, page, 0.2, 4.0, r1.to(on), r2.to(on), pb.to(on), 0.4, 8, sc.key_chunk,
+                            max_context=sc.max_pos)
+        outs.append((pooled, weighed))
+    close(outs[1][0], outs[0][0], 2 * BF16_EPS, 5e-3, "pooled windows")                # the bounds of the attentions' own tests
+    close(outs[1][1], outs[0][1], 2 * BF16_EPS, 4e-3 * outs[0][1].abs().max().item(), "sigmoid weights")

@@ -1,4 +1,5 @@
-"""What the compiled kernels of decode steps are held to where nothing in their results shows it: loads that wait for nothing between them."""
+"""What the compiled kernels of decode steps and prompts are held to where nothing in their results shows it: loads that wait for nothing between
+them, registers that leave a compute unit its waves."""
 import os
 import re
 import subprocess
@@ -48,3 +49,16 @@ def test_entries_of_the_state_are_asked_for_together(tmp_path, source, pattern, 
     for name, text, groups in found:
         want = 3 * int(groups[0]) if groups else 3
         assert longest_run(text) >= want, name
+
+
+# waves a SIMD of prompts' tiles of windows with pooled blocks, (key lanes / 32, value lanes / 16): where asking for a block's keys and values at
+# once costs one of them
+TILE_WAVES = {(2, 6): 3, (3, 2): 4, (3, 4): 3, (3, 6): 3, (4, 2): 4, (4, 4): 3}
+
+
+def test_waves_of_prompts_with_pooled_blocks(tmp_path):
+    found = kernels("mixer_variants_mfma.hip", r"17mixer_tile_kernelILi(\d)ELi(\d)ELi0ELb[01]ELb0E", tmp_path)
+    assert len(found) == 32
+    for name, text, (kd, vt) in found:
+        waves = int(re.search(r"^; Occupancy: (\d+)", text, re.M).group(1))
+        assert waves >= TILE_WAVES.get((int(kd), int(vt)), 2), (name, waves)
