@@ -6,7 +6,7 @@
 // behind it cost prompts and answers of 12 requests 12.40 ms where this takes 12.29), no scaled copies of the rows are
 // made (an operand is scaled where it is loaded, rounded to bfloat16 as a stored copy would be), and the down product is not cut
 // into planes that a further kernel adds.  A workgroup takes 16 output columns (of gate and of up) or 32 of one expert, its eight waves
-// cut K between them with 6 KiB asked for at a time each, and they meet in LDS once.  A load of the tile-major copy is
+// cut K between them with 4 to 12 KiB asked for at a time each, and they meet in LDS once.  A load of the tile-major copy is
 // 1 KiB in a row, whole cache lines that carry the non-temporal hint; the same kernel reading the rows as the checkpoint has them
 // (64 bytes of each of 16) runs at 4.4 instead of 5.9 TB/s, and through LDS in whole rows, a tile at a time, at 4.0.
 // A load of an expert's weights serves up to 32 pairs from registers.
@@ -33,7 +33,8 @@ constexpr int kMostPairs = 512;
 // out_weights[pair], so that one sum of a row's parts is all that follows: of one layer's launches (2 rows, 8 experts and a shared one of
 // 4,480 lanes at a width of 1,536) two products of 6 to 8 us and a sum of 4 are gone
 // (a prompt and eight decode steps of twelve such layers 15.6 -> 14.5 ms).
-template <int MODE, int G, bool SHARED>
+// U: products a wave asks for at a time (launch_groups).
+template <int MODE, int G, bool SHARED, int U>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
 expert_stream_kernel(const bf16_t *__restrict__ x, const int32_t *__restrict__ ids, const bf16_t *__restrict__ w, int ldx, int pairs, int top, int E,
                      int N, int K, int by_pair, const float *__restrict__ weights, bf16_t *__restrict__ act,
@@ -42,11 +43,6 @@ expert_stream_kernel(const bf16_t *__restrict__ x, const int32_t *__restrict__ i
     static_assert(!SHARED || MODE != 0, "a shared expert comes with experts without a gate");
     constexpr int RT = MODE == 1 ? 1 : 2;                  // 16-row weight tiles a workgroup
     constexpr int COLS = MODE == 2 ? 32 : 16;              // output columns a workgroup
-    // Products a wave asks for at a time.  Two tiles of one group: three, so that 64 to 75 registers hold three or four workgroups a compute unit where
-    // six left two: how many workgroups are there to ask while others' sums meet counts for more than how much each asks for (4,480
-    // lanes at 1,536: 2 rows with a shared expert 15.2 -> 13.1 us, 8 rows 32.3 -> 31.1, 16 rows 34.7 -> 32.2; two products 30.4 and 32.6).  One tile: six (four: 18.5
-    // and 18.4, 20.2 and 20.4, with a shared expert 13.2 and 13.7; nine 21.4, 22.8, 13.2).  Two groups: 128 registers.
-    constexpr int U = G > 1 ? (MODE == 0 ? 3 : 6) : MODE == 1 ? 6 : 3;
     __shared__ __attribute__((aligned(16))) f32x4_t red[kWaves][RT][kWave];
     __shared__ short s_pairs[kWaves][kMostPairs];          // a wave's own list: no barrier before the first loads
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -192,9 +188,29 @@ void launch_groups(const void *x, int ldx, const int32_t *ids, const float *weig
                    void *act, float *out, float limit, float alpha, float up_offset, const Shared &sh, hipStream_t stream) {
     const int by_pair = pairs < E;
     const int cols = MODE == 2 ? 32 : 16, widest = sh.n > N ? sh.n : N;
-    hipLaunchKernelGGL((expert_stream_kernel<MODE, G, SHARED>), dim3((widest + cols - 1) / cols, (by_pair ? (unsigned)pairs : (unsigned)E) + (SHARED ? 1 : 0)),
-                       dim3(kThreads), 0, stream, (const bf16_t *)x, ids, (const bf16_t *)w, ldx, (int)pairs, top, E, N, K, by_pair, weights,
-                       (bf16_t *)act, out, limit, alpha, up_offset, (const bf16_t *)sh.w, sh.n, sh.k, sh.out_weights, sh.top);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((widest + cols - 1) / cols, (by_pair ? (unsigned)pairs : (unsigned)E) + (SHARED ? 1 : 0)), dim3(kThreads), 0, stream,
+                           (const bf16_t *)x, ids, (const bf16_t *)w, ldx, (int)pairs, top, E, N, K, by_pair, weights, (bf16_t *)act, out, limit, alpha,
+                           up_offset, (const bf16_t *)sh.w, sh.n, sh.k, sh.out_weights, sh.top);
+    };
+    // Products a wave asks for at a time.  Two tiles of one group: two or three, so that 64 to 75 registers hold three or four workgroups a compute
+    // unit where six left two: how many workgroups are there to ask while others' sums meet counts for more than how much each asks for.  Which of the
+    // two: three, unless a wave has few products and a third of them would be asked for twice.  Microseconds of both products with two, three, four, six:
+    //   gated experts of 2,048 lanes    width 1,024 (4 products a wave), 1 row 11.7, 12.3, 11.6, 11.4;  8 rows 21.2, 23.2, 22.0, 22.4
+    //                                   width 2,048 (8), 1 row 14.7, 14.8, 14.8, 15.5;  8 rows 38.6, 39.2, 38.8, 41.5
+    //   gated experts of 4,480 lanes    width 1,024, 1 row 19.0, 20.1, 19.8, 19.9;  8 rows 37.8, 40.5, 41.4, 41.3
+    //                                   width 1,536 (6), 1 row 23.4, 23.1, 24.9, 24.1;  8 rows 53.7, 53.3, 57.7, 55.4
+    //                                   width 4,096 (16), 1 row 43.3, 43.2, 42.5, 42.9;  8 rows 134.0, 132.3, 134.0, 131.9
+    //   4,480 lanes beside a shared expert, width 1,536, 2 rows 26.1, 26.2, 26.4, 28.8;  16 rows 49.2, 49.4, 49.7, 53.1
+    // One tile: six (4,480 lanes at 1,536, the down product alone, four: 18.5 and 18.4, 20.2 and 20.4, with a shared expert 13.2 and 13.7; nine 21.4, 22.8,
+    // 13.2).  Two groups: 128 registers.
+    if constexpr (G == 1 && MODE != 1) {
+        const int each = ((K + kWaves - 1) / kWaves + 31) / 32;
+        if (each % 3 != 0 && each <= 8) go(expert_stream_kernel<MODE, G, SHARED, 2>);
+        else go(expert_stream_kernel<MODE, G, SHARED, 3>);
+    } else {
+        go(expert_stream_kernel<MODE, G, SHARED, MODE == 0 ? 3 : 6>);
+    }
 }
 
 template <int MODE, bool SHARED = false>

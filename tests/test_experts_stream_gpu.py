@@ -20,7 +20,8 @@ def ops():
 @pytest.mark.parametrize("spread", ["random", "one expert"])
 @pytest.mark.parametrize("gated,weighted,limit,alpha,offset", [(True, True, 0.0, 1.0, 0.0), (True, False, 1.5, 1.702, 1.0), (False, False, 0.0, 1.0, 0.0)])
 @pytest.mark.parametrize("rows,width,inter,experts,top", [(1, 256, 256, 8, 2), (3, 288, 320, 9, 1), (8, 1536, 480, 8, 2), (17, 512, 288, 3, 2),
-                                                          (64, 256, 256, 8, 2), (40, 272 + 16, 256, 5, 2), (128, 256, 288, 32, 4)])
+                                                          (64, 256, 256, 8, 2), (40, 272 + 16, 256, 5, 2), (128, 256, 288, 32, 4), (2, 1024, 256, 8, 2),
+                                                          (9, 1312, 256, 8, 2), (3, 2560, 288, 8, 2)])
 def test_the_picked_experts_stream_from_their_copies(ops, rows, width, inter, experts, top, gated, weighted, limit, alpha, offset, spread):
     ref = ReferenceOps()
     g = torch.Generator().manual_seed(rows * 31 + width)
