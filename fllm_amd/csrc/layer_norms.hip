@@ -285,8 +285,6 @@ side_gate_kernel(const float *__restrict__ x, const T *__restrict__ w, const int
     // the row that this thread ends, if it has one: its token ahead of the products, its entry of the table beside their sums
     const int r = threadIdx.x;
     int id = ids[min(r, rows - 1)];
-    const int own = min((int)threadIdx.x, rows - 1);      // the row that this thread ends, if it has one: its token, behind it its table's row
-    const int own_id = ids[own];
     float acc[R];
 #pragma unroll
     for (int r = 0; r < R; r++) acc[r] = 0.f;
