@@ -36,22 +36,26 @@ constexpr int kWideRows = 128;            // the most rows of the kernel that pa
 enum { PRO_BF16 = 0, PRO_NORM_F32 = 1, PRO_SCALED = 2 };
 enum { EPI_STORE = 0, EPI_STORE_F32 = 1, EPI_ADD = 2, EPI_QKV = 3, EPI_SWIGLU = 4 };
 
+// The gated epilogue's constants fill what would be padding: g' * sigmoid(act_alpha g') * (u' + act_offset), g' = min(g, act_limit), u' = clamp(u,
+// +-act_limit) (act_limit <= 0: nothing is clamped).  SwiGLU is alpha 1, offset 0, no limit.  Behind everything else they were a trip to memory of their own
+// at the end of a tile of up to 16 rows (gate/up of 2 x 4,480 x 1,536 9.7 -> 9.4 us); ahead of M they moved what follows to other lines, and the compiler asked for
+// the slab kernel's parts one by one (2 x 14,336 x 4,096 behind a norm at 48 rows 130 -> 182 us).
 struct SkinnyArgs {
     const void *x;
     int ldx;
+    float act_limit;
     const float *norm_w;
     float eps;
+    float act_alpha;
     const bf16_t *w;
     const bf16_t *w_tiles;   // the same matrix tile by tile (fllm_tile_weights), or null
     const float *bias;
     void *out;
     int ldo;
-    // gated epilogue: g' * sigmoid(act_alpha g') * (u' + act_offset), g' = min(g, act_limit), u' = clamp(u, +-act_limit)
-    // (act_limit <= 0: nothing is clamped).  SwiGLU is alpha 1, offset 0, no limit.
-    float act_limit, act_alpha, act_offset;
     int M, N, K;
     int S, slice;  // K is cut into S slices of `slice` elements (a multiple of 128); a workgroup stages one slice
     int ssq_off;   // byte offset of the sums of squares in LDS (behind the staging / reduction area)
+    float act_offset;
     float *ws;     // S > 1: partial sums [tile][slice][RT][64 lanes][4], then sums of squares [tile][slice][16]
     float *ws_ssq;
     int *counters; // S > 1: items of a tile counted so far (zero between launches)
@@ -1006,7 +1010,7 @@ skinny_wide_kernel(const bf16_t *w, const bf16_t *x, const float *ssq_in, int K,
 // runs the epilogue, so the result does not depend on who came last.
 template <int PRO, int EPI, int MT>
 __global__ void __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
-skinny_slab_kernel(SkinnyArgs a, int cells_off) {
+skinny_slab_kernel(SkinnyArgs a, int cells_off, float act_limit, float act_alpha, float act_offset /* again: fetched where they are used */) {
     constexpr int WAVES = 8, THREADS = WAVES * kWave;
     constexpr int KC = 256;                        // columns per chunk of weights
     constexpr int KS = KC / 32;                    // MFMA k-steps per chunk
@@ -1017,6 +1021,7 @@ skinny_slab_kernel(SkinnyArgs a, int cells_off) {
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int r = lane & 15, g = lane >> 4;
     const int M = a.M, N = a.N, K = a.K, S = a.S;
+    a.act_limit = act_limit, a.act_alpha = act_alpha, a.act_offset = act_offset;
     const int n_out = EPI == EPI_SWIGLU ? N / 2 : N;
     const int ntiles = (n_out + NT - 1) / NT;
     const int ngroups = (ntiles + WAVES - 1) / WAVES;
@@ -1227,7 +1232,7 @@ skinny_slab_kernel(SkinnyArgs a, int cells_off) {
             s[mt][0] = acc[mt];
             if (EPI == EPI_SWIGLU) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) s[mt][RT - 1][i] = lanes_32_apart(acc[mt][i]).b;
+                for (int i = 0; i < 4; i++) s[mt][RT - 1][i] = __shfl(acc[mt][i], (lane + 32) & 63, kWave);
             }
             acc[mt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
             ss[mt] = 0.f;
@@ -1530,7 +1535,8 @@ int launch_slab(SkinnyArgs a, hipStream_t stream) {
         FLLM_REQUIRE(e == hipSuccess, "linear_skinny: cannot raise the LDS limit: %s", hipGetErrorString(e));
         attribute_set = true;
     }
-    hipLaunchKernelGGL((skinny_slab_kernel<PRO, EPI, MT>), dim3(p.grid), dim3(8 * kWave), p.smem, stream, a, (int)p.cells_off);
+    hipLaunchKernelGGL((skinny_slab_kernel<PRO, EPI, MT>), dim3(p.grid), dim3(8 * kWave), p.smem, stream, a, (int)p.cells_off, a.act_limit,
+                       a.act_alpha, a.act_offset);
     return fllm_check_launch("linear_slab");
 }
 
