@@ -28,7 +28,8 @@ embed_kernel(const int32_t *__restrict__ ids, const T *__restrict__ table, float
 // All that a row needs is asked for before the first of it is used, behind no condition (a thread without values of its own reads the row's last
 // ones again): behind conditions a piece was awaited, added and stored before the next was asked for, and the weights came behind the
 // sum.  WIDE: everything lies on 8 bytes (rows of the branch and of the output in bfloat16 too): four values are one load or store.
-// 2,048 rows of 4,096 values with a branch in bfloat16 18.8 -> 17.0 us (101 MB), 405 rows 7.4 -> 5.8; of 2,048 values 9.5 -> 9.1.
+// 2,048 rows of 4,096 values with a branch in bfloat16 18.8 -> 17.0 us (101 MB), 405 rows 7.4 -> 5.8; of 2,048 values 9.5 -> 9.1; of
+// 8,192, where registers leave four waves a SIMD, 49.0 -> 39.0, 16 rows 5.7 -> 3.7.
 template <typename T, typename B, int VEC, bool WIDE>
 __global__ void __launch_bounds__(kBlock)
 rmsnorm_kernel(float *__restrict__ x, const B *__restrict__ branch, const float *__restrict__ weight, const int32_t *__restrict__ rows,

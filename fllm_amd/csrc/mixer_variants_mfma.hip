@@ -71,8 +71,8 @@ __device__ __forceinline__ void publish(float *at, float v) { __hip_atomic_store
 // save (2,000 rows 57 us with divisions, 63 with the question, 55 like this).
 // BY_HEADS: tiles of single rows.  Tiles of 16 rows have instances of their own, which ask for a pooled block's keys and values as they come: a prompt
 // has enough workgroups to cover the trips, and what all of them at once hold in registers cost it a wave a SIMD (1,900 rows of 12 heads on two, windows of
-// 1,024, keys and values of 64 and 96 lanes 47.5 us, 49.2 all at once, 44.4 like this; 128 and 64 43.6, 44.8, 40.9; with pages of 48 tokens
-// 44.1, 48.7, 44.0).
+// 1,024, keys and values of 64 and 96 lanes 47.5 us with one kernel that asks as they come, 48.6 with one that asks for all at once, 44.2 like this; 128 and 64
+// 43.5, 45.3, 39.9, with pages of 48 tokens 44.0, 48.8, 44.2).
 template <int KD, int VT, int VARIANT, bool POW2, bool BY_HEADS>
 __global__ void __launch_bounds__(kThreads)
 mixer_tile_kernel(const int32_t *__restrict__ row_seg, const int32_t *__restrict__ row_pos, const int32_t *__restrict__ tables,

@@ -149,8 +149,8 @@ norm_route_kernel(float *__restrict__ x, const float *__restrict__ branch, const
             }
         }
     };
-    // up to eight experts are a pass of the four waves: nothing is asked for ahead, which the pass would wait for (with the picks in registers, 8 experts of 1,536 lanes: grouped scores at 2 rows 6.6 -> 5.0 us, plain at 4 rows
-    // 4.8 -> 3.8)
+    // up to eight experts are a pass of the four waves: nothing is asked for ahead, which the pass would wait for (with the picks in registers, 8 experts of
+    // 1,536 lanes: grouped scores at 2 rows 6.6 -> 5.0 us, plain at 4 rows 4.8 -> 3.8)
     if (experts <= 2 * kWaves) two(wave, std::true_type{});
     else
         for (int e0 = wave; e0 < experts; e0 += 2 * kWaves) two(e0, std::false_type{});
