@@ -14,7 +14,7 @@ constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / kWave;
 constexpr int kMaxKeep = 15;
 constexpr int kMaxPer = 8;      // heads of up to 512 lanes
-constexpr int kStepTaps = 4;    // conv_qkv_step_kernel: at most
+constexpr int kStepTaps = 4;    // conv_qkv_step_kernel, but for narrow float32 heads: at most
 
 // grid (rows, heads in fours): a wave takes one head of q, k or v of one row.  `update` (steps of one row a segment): the wave,
 // which alone reads its channels of the state, moves them on; otherwise conv_tail_kernel does behind this kernel.
@@ -133,10 +133,11 @@ conv_qkv_store_kernel(const T *__restrict__ joint, int ld, const float *__restri
 // arguments, some of them two or three numbers, are in registers when a wave starts; the other arguments ride along), then the state's entries, the page, weights
 // and angles.  No load sits behind a condition: a lane beyond the head reads its last channel again.  A trip a question, as
 // the form for portions has it, took 8.5 us at 16 rows of 12 + 2 heads of 128, this 4.3 (7.6 and 2.8 at best).
-// N pieces of 64 lanes a head (at most), up to four taps; FOUR: four of them, one 16-byte load.  Of fewer the last ones are read again: behind a
-// question each (is there an i-th) every 16-bit entry was awaited before the next was asked for (three taps in bfloat16, 16 rows of 6 + 2 heads of
-// 192 12.9 us, of 4 + 2 of 64 6.0; without 5.6 and 3.3, by the form for portions 7.0 and 4.3).
-template <typename T, int N, bool FOUR>
+// N pieces of 64 lanes a head (at most), MOST taps (at most); FOUR: four of them, one 16-byte load.  Of fewer than four the last ones are read again: behind
+// a question each (is there an i-th) every 16-bit entry was awaited before the next was asked for (three taps in bfloat16, 16 rows of 6 + 2 heads of
+// 192 12.9 us, of 4 + 2 of 64 6.0; without 5.6 and 3.3, by the form for portions 7.0 and 4.3).  Of more than four (float32, where a load has a register of
+// its own) each is behind its question: reading the last ones again were too many loads.
+template <typename T, int N, int MOST, bool FOUR>
 __global__ void __launch_bounds__(kBlock)
 conv_qkv_step_kernel(const T *__restrict__ joint, const int32_t *__restrict__ row_seg, const int32_t *__restrict__ row_pos,
                      const int32_t *__restrict__ slots, const float *__restrict__ conv, int ld, int all_heads /* heads | kv_heads << 16 */,
@@ -145,7 +146,8 @@ conv_qkv_step_kernel(const T *__restrict__ joint, const int32_t *__restrict__ ro
                      T *__restrict__ q_out, const int32_t *__restrict__ tables, int table_stride, const float *__restrict__ cos_table,
                      const float *__restrict__ sin_table, T *__restrict__ k_pages, T *__restrict__ v_pages, int page_size, int key_chunk) {
     typedef const __attribute__((address_space(4))) int32_t *constant_t;      // the same for every lane: a scalar load
-    constexpr int KEEP = kStepTaps - 1;
+    static_assert(!FOUR || MOST == kStepTaps, "four taps are four");
+    constexpr int KEEP = MOST - 1;
     extern __shared__ float smem[];
     const int r = blockIdx.x;
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -162,7 +164,7 @@ conv_qkv_step_kernel(const T *__restrict__ joint, const int32_t *__restrict__ ro
     const int channels = nq + (store_kv ? nk + kv_heads * v_dim : 0);
     const int base = kind == 0 ? h * k_dim : (kind == 1 ? nq + h * k_dim : nq + nk + h * v_dim);
     T now[N], held[N][KEEP];
-    float w[N][kStepTaps];
+    float w[N][MOST];
     T *mine = nullptr;
     const T *kept = joint + (size_t)r * ld;       // one tap: read, never used
     auto lane_of = [&](int j) __attribute__((always_inline)) { return min(lane + j * kWave, dim - 1); };
@@ -171,12 +173,18 @@ conv_qkv_step_kernel(const T *__restrict__ joint, const int32_t *__restrict__ ro
             *(f32x4_t *)w[j] = *(const f32x4_t *)(conv + (size_t)ch * 4);
         } else {
 #pragma unroll
-            for (int i = 0; i < kStepTaps; i++) w[j][i] = conv[(size_t)ch * taps + min(i, keep)];
+            for (int i = 0; i < MOST; i++) {
+                if constexpr (MOST == kStepTaps) w[j][i] = conv[(size_t)ch * taps + min(i, keep)];
+                else if (i < taps) w[j][i] = conv[(size_t)ch * taps + i];
+            }
         }
     };
     auto ask_state = [&](int j, int ch) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < KEEP; i++) held[j][i] = kept[(size_t)(FOUR ? i : max(min(i, keep - 1), 0)) * channels + ch];
+        for (int i = 0; i < KEEP; i++) {
+            if constexpr (MOST == kStepTaps) held[j][i] = kept[(size_t)(FOUR ? i : max(min(i, keep - 1), 0)) * channels + ch];
+            else if (i < keep) held[j][i] = kept[(size_t)i * channels + ch];
+        }
     };
 #pragma unroll
     for (int j = 0; j < N; j++) {
@@ -326,21 +334,24 @@ extern "C" int fllm_conv_qkv_store(const void *joint, int ld, const float *conv,
     FLLM_REQUIRE(groups <= 65535 && blocks <= 65535, "conv_qkv_store: too many heads");
     const size_t smem = rope_dims > 0 ? (size_t)kWaves * k_dim * sizeof(float) : 0;
     // The step form takes up to four taps, and sizes two in a word.  More taps go the portions' way, a tap a load as it comes: all at once are
-    // more loads than a wave's trips cost (eight taps in bfloat16, 16 rows of 12 + 2 heads of 128 8.3 us, 12.3 in the step form; 16 taps 12.3, 19.7).
-    const bool step = single_rows && taps <= kStepTaps && heads <= 0xffff && kv_heads <= 0x7fff;
-#define FLLM_STEP(T, N, FOUR)                                                                                                               \
-    hipLaunchKernelGGL((conv_qkv_step_kernel<T, N, FOUR>), dim3(rows, groups), dim3(kBlock), smem, stream, (const T *)joint, row_seg, row_pos, \
+    // more loads than a wave's trips cost (eight taps in bfloat16, 16 rows of 12 + 2 heads of 128 8.3 us, 12.3 in the step form; 16 taps 12.3, 19.7), but in
+    // float32 for heads of up to 128 lanes (7.6, 5.8; heads of 64 behind a kernel that streams 5.8, 5.1; heads of 256 11.9, 16.4).
+    const bool narrow = k_dim <= 2 * kWave && v_dim <= 2 * kWave;
+    const bool step = single_rows && (taps <= kStepTaps || (dtype == FLLM_F32 && narrow)) && heads <= 0xffff && kv_heads <= 0x7fff;
+#define FLLM_STEP(T, N, MOST, FOUR)                                                                                                         \
+    hipLaunchKernelGGL((conv_qkv_step_kernel<T, N, MOST, FOUR>), dim3(rows, groups), dim3(kBlock), smem, stream, (const T *)joint, row_seg, row_pos, \
                        slots, conv, ld, heads | kv_heads << 16, k_dim | v_dim << 16,                                                        \
                        taps | rope_dims << 8 | pairing << 24 | (store_kv ? 1 << 25 : 0), (T *)state, bias, q_weight, k_weight, eps,            \
                        (T *)q_out, tables, table_stride, cos_table, sin_table, (T *)k_pages, (T *)v_pages, page_size, key_chunk)
-#define FLLM_CONV(T)                                                                                                                        \
+#define FLLM_CONV(T, MORE_TAPS)                                                                                                             \
     do {                                                                                                                                    \
         if (step) {                                                                                                                         \
-            const bool four = taps == 4 && ((uintptr_t)conv & 15) == 0, narrow = k_dim <= 2 * kWave && v_dim <= 2 * kWave;                   \
-            if (four && narrow) FLLM_STEP(T, 2, true);                                                                                      \
-            else if (four) FLLM_STEP(T, kMaxPer, true);                                                                                     \
-            else if (narrow) FLLM_STEP(T, 2, false);                                                                                        \
-            else FLLM_STEP(T, kMaxPer, false);                                                                                              \
+            const bool four = taps == 4 && ((uintptr_t)conv & 15) == 0;                                                                     \
+            if (taps > kStepTaps) MORE_TAPS;                                                                                                \
+            else if (four && narrow) FLLM_STEP(T, 2, kStepTaps, true);                                                                      \
+            else if (four) FLLM_STEP(T, kMaxPer, kStepTaps, true);                                                                          \
+            else if (narrow) FLLM_STEP(T, 2, kStepTaps, false);                                                                             \
+            else FLLM_STEP(T, kMaxPer, kStepTaps, false);                                                                                   \
             break;                                                                                                                          \
         }                                                                                                                                   \
         hipLaunchKernelGGL(conv_qkv_store_kernel<T>, dim3(rows, groups), dim3(kBlock), smem, stream, (const T *)joint, ld, conv, taps, bias, \
@@ -351,8 +362,8 @@ extern "C" int fllm_conv_qkv_store(const void *joint, int ld, const float *conv,
             hipLaunchKernelGGL(conv_tail_kernel<T>, dim3(num_segs, blocks), dim3(kBlock), 0, stream, (const T *)joint, ld, (T *)state,       \
                                row_seg, seg_start, slots, channels, taps);                                                                  \
     } while (0)
-    if (dtype == FLLM_F32) FLLM_CONV(float);
-    else if (dtype == FLLM_BF16) FLLM_CONV(bf16_t);
+    if (dtype == FLLM_F32) FLLM_CONV(float, FLLM_STEP(float, 2, kMaxKeep + 1, false));
+    else if (dtype == FLLM_BF16) FLLM_CONV(bf16_t, (void)0);
     else FLLM_REQUIRE(false, "conv_qkv_store: unknown dtype %d", dtype);
 #undef FLLM_CONV
 #undef FLLM_STEP
